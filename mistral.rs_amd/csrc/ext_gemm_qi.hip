@@ -5,14 +5,13 @@
 // (d_w d_x) <integer dot> - (dmin_w d_x) <integer min term>.  Rounds 1-3 ran prompts in a different arithmetic (weights and activations rounded to bf16);
 // this kernel computes the reference's integers EXACTLY on v_mfma_f32_32x32x16_f16 and combines them in the f32 order of the decode engine ("ORD-U",
 // dec_core2.cuh / oracle orc_gemv_engine), so a token's logits and KV pages do not depend on whether it was part of a prompt or decoded:
-//   * the 6-bit sub-block scale is folded INTO the weight operand as an exact small integer in f16: Q4_K  sc q <= 945;  Q6_K  two operands
+//   * the 6-bit sub-block scale is folded INTO the weight operand as an exact small integer in f16: Q4_K  sc (q - 8);  Q6_K  two operands
 //     sl (q - 32) and sh (q - 32) with sc = 16 sh + sl, |.| <= 480 / 256.  The activation operand is the Q8_K quant as f16.  Every product and every partial
 //     sum of a superblock is an integer below 2^24, so the f32 accumulator of the matrix core holds the EXACT sum (tests/test_gemm_qi.py holds
 //     v_mfma_f32_32x32x16_f16 to that on adversarial operands); no per-sub-block scale multiply is left on the vector ALU;
-//   * Q4_K: the operand is sc q (<= 945); the first and the second eight runs of a superblock go to two accumulators (<= 15.5 M each), (float)isum = XA + XB is
-//     one rounding of the exact integer -- what (float)int gives; msum = sum_j m_j bsum_j is one more MFMA per superblock (K = the 16 run sums of the Q8_K
-//     block, mins duplicated per run);
-//   * Q5_K (round 5): the operand is sc (q - 16) (|.| <= 1008: one packed fma for sc q, one packed add for - 16 sc), two accumulators like Q4_K (<= 16.5 M each), and the
+//   * Q4_K (gemm_qi_wide_kernel): the operand is sc (q - 8), the 8 sum_j sc_j bsum_j the offset leaves out and msum = sum_j m_j bsum_j are one more MFMA each per superblock
+//     (K = the 16 run sums of the Q8_K block, scales / mins duplicated per run); (float)isum = X + 8 S is one rounding of the exact integer -- what (float)int gives;
+//   * Q5_K (round 5): the operand is sc (q - 16) (|.| <= 1008: one packed fma for sc q, one packed add for - 16 sc), two accumulators (<= 16.5 M each), and the
 //     16 sum_j sc_j bsum_j the offset leaves out is one more MFMA (S); isum = XA + XB + 16 S is formed in int32 (a superblock's sum reaches 64 M: two f32 additions
 //     would round twice) and converted once; the mins' M as for Q4_K;
 //   * per superblock and output ONE f32 term T (the decode engine's expression), terms added left to right inside each of the row's four runs of
@@ -20,7 +19,7 @@
 // Operands: weights in an MFMA-order copy made at load time (mrs_gemm_qi_repack: per 32-row panel and superblock, every lane's 16 bytes of a piece
 // contiguous: one buffer_load_dwordx4 per lane and piece, straight into registers); activations from mrs_qi_quantize (engine-order RmsNorm + the candle
 // Q8_K quantizer of dec_core2.cuh, then f16 in the operand's k order, slab-major [superblock][token][256]).
-// Tiling: workgroup 512 threads = 8 waves (two per SIMD: one wave's MFMAs run under the other's operand build and fix-up), tile 128 weight rows x 128
+// Tiling (Q5_K, Q6_K; Q4_K: gemm_qi_wide_kernel below): workgroup 512 threads = 8 waves (two per SIMD: one wave's MFMAs run under the other's operand build and fix-up), tile 128 weight rows x 128
 // tokens, wave 32 x 64 = 1 x 2 MFMA tiles; per superblock the 128 tokens' f16 quants (64 KiB) are staged in LDS (16-byte chunks XOR-swizzled by the token
 // index: conflict-free ds_read_b128 fragments), double buffered: superblock s + 1 arrives by LDS-DMA (global_load_lds) while s is multiplied.
 #include "dec_core2.cuh"
@@ -36,6 +35,7 @@ using namespace mrs::dec2;
 typedef _Float16 h2 __attribute__((ext_vector_type(2)));
 typedef _Float16 h8 __attribute__((ext_vector_type(8)));
 typedef float f16v __attribute__((ext_vector_type(16)));
+typedef float f32v __attribute__((ext_vector_type(32)));
 typedef float f2 __attribute__((ext_vector_type(2)));
 
 constexpr int REC_Q4K = 4096 + 512 + 128, REC_Q6K = 8192 + 512 + 128, REC_Q5K = REC_Q6K;  // Q5_K: the 5-bit values as bytes, like Q6_K's 6-bit ones
@@ -200,9 +200,19 @@ struct GemmArgs {
   const _Float16 *qf; const float *yd; const _Float16 *bsf;
   float *out; int ldo; int accumulate;  // out[t * ldo + n] (+)= row sum
   float *part; int ksplit;              // ksplit = 4: workgroup z multiplies run z of the row's superblocks only and writes its sum to part[z][t][n]; the reduce kernel combines
-  const int *win;                       // device {begin, end}: only the operand rows [begin, end) take part (one expert's routes of a grouped MoE prompt GEMM: the bounds
-                                        // come from launch_moe_dispatch on the device, the grid is sized for the worst case and tiles past `end` leave); nullptr = all T rows
+  const int *bounds; int experts;       // expert e multiplies the operand rows [bounds[e], bounds[e + 1]) by the weights at w + e * w_bytes (a grouped MoE prompt GEMM: the
+                                        // bounds come from launch_moe_dispatch on the device, the grid is sized for the worst case and tiles past it leave); nullptr = all T rows
 };
+// (expert, first row, end) of token tile yt of a launch over the experts' windows; false: past the last tile
+__device__ __forceinline__ bool expert_tile(const int *bounds, int experts, int tile, int &yt, int &e, int &tbeg, int &tend) {
+  for (e = 0; e < experts; ++e) {
+    tbeg = __builtin_amdgcn_readfirstlane(bounds[e]); tend = __builtin_amdgcn_readfirstlane(bounds[e + 1]);
+    const int nt = (tend - tbeg + tile - 1) / tile;
+    if (yt < nt) return true;
+    yt -= nt;
+  }
+  return false;
+}
 constexpr int TN = 128, TT = 128;                   // workgroup tile: weight rows x tokens
 constexpr int GT = 512;                             // 8 waves: 4 (32-row panels) x 2 (64-token halves); two waves per SIMD overlap each other's MFMA and VALU phases
 constexpr int LDS_ACT = TT * 512, LDS_YD = TT * 4, LDS_BS = TT * 32;
@@ -230,13 +240,15 @@ __global__ void __launch_bounds__(GT) gemm_qi_kernel(const GemmArgs a) {
   const int tid = tid_opaque(), lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int nn = lane & 31, hf = lane >> 5;
   const int n0 = blockIdx.x * TN;
-  const int tbeg = a.win ? __builtin_amdgcn_readfirstlane(a.win[0]) : 0, tend = a.win ? __builtin_amdgcn_readfirstlane(a.win[1]) : a.T;
-  const int t0 = tbeg + blockIdx.y * TT;
+  int tbeg = 0, tend = a.T, yt = blockIdx.y, ex = 0;
+  if (a.bounds && !expert_tile(a.bounds, a.experts, TT, yt, ex, tbeg, tend)) return;
+  const uint8_t *wbase = a.w + (size_t)ex * a.w_bytes;
+  const int t0 = tbeg + yt * TT;
   if (t0 >= tend) return;  // workgroup-uniform
   const int wn = wave & 3, wt = wave >> 2;  // the wave's 32-row panel / 64-token half of the tile
   const int S = a.K / 256, Cs = (S + 3) / 4;
-  const __amdgpu_buffer_rsrc_t rw = __builtin_amdgcn_make_buffer_rsrc((void *)a.w, (short)0, (int)a.w_bytes, 0x00020000);
-  constexpr int REC = rec_bytes_qi(TYPE), NPC = TYPE == T_Q4_K ? 4 : 8;
+  const __amdgpu_buffer_rsrc_t rw = __builtin_amdgcn_make_buffer_rsrc((void *)wbase, (short)0, (int)a.w_bytes, 0x00020000);
+  constexpr int REC = rec_bytes_qi(TYPE), NPC = 8;
   struct WRegs { v4u q[NPC]; v4u hs; unsigned hd; };
   const unsigned panel = (unsigned)((n0 + wn * 32) >> 5);
   auto load_w = [&](WRegs &wr, int sb) {
@@ -318,80 +330,7 @@ __global__ void __launch_bounds__(GT) gemm_qi_kernel(const GemmArgs a) {
     };
     const bool cfirst = (sb % Cs) == 0;
     const f2 keep2 = cfirst ? f2{0.f, 0.f} : f2{1.f, 1.f};  // the first term of a run of superblocks starts its sum (0 * run + t), the others add (1 * run + t: exact)
-    if constexpr (TYPE == T_Q4_K) {
-      // operand = sc q as an exact integer in f16 from ONE packed fma per pair of weights: (1024 + q) sc - 1024 sc for a nibble at bits 3:0 of a half-word,
-      // (1024 + 16 q) (sc / 16) - 64 sc for one at bits 7:4 (1024 sc, 64 sc and sc / 16 are exact in f16; 1032 sc, which q - 8 would need, is not).  With the
-      // unsigned q a superblock's sum can reach 30.9 M > 2^24, so runs 0 .. 7 and 8 .. 15 go to two accumulators (<= 15.5 M each, exact) and
-      // (float)isum = XA + XB is one rounding of the exact integer.
-      unsigned mg = 0x64006400u;
-      MRS_OPAQUE_TID(mg);  // keeps the constant in a VGPR: v_and_or_b32 takes one literal
-      auto lo4 = [&](unsigned v, h2 sc, h2 off) -> h2 { return pkfma(as_h2((v & 0x000F000Fu) | mg), sc, off); };
-      auto hi4 = [&](unsigned v, h2 sc16, h2 off) -> h2 { return pkfma(as_h2((v & 0x00F000F0u) | mg), sc16, off); };
-      const unsigned s01[2] = {wr.hs.x, wr.hs.y};
-      // Activation fragments are read ONE GROUP AHEAD (round 6): the code used to ask for a group's four fragments and wait for them (s_waitcnt lgkmcnt(0)) right in front
-      // of its MFMAs -- 8 exposed LDS round trips per superblock and wave with two waves per SIMD to hide them (MFMA pipes 25 % busy, profiles/round4_pmc.md).  Group (c, h)
-      // = runs 4 c + h (low nibbles) and 4 c + 2 + h (high) for both token tiles; scheduling barriers keep the read of group g + 1 in front of the operand build of group g.
-      h8 fr[2][4];
-      auto read_group = [&](int gi, h8 (&f)[4]) {
-        const int c = gi >> 1, h = gi & 1;
-        f[0] = act_frag(0, 4 * c + h); f[1] = act_frag(0, 4 * c + 2 + h); f[2] = act_frag(1, 4 * c + h); f[3] = act_frag(1, 4 * c + 2 + h);
-      };
-      read_group(0, fr[0]);
-#pragma unroll
-      for (int gi = 0; gi < 8; ++gi) {
-        const int c = gi >> 1, h = gi & 1;
-        if (gi + 1 < 8) read_group(gi + 1, fr[(gi + 1) & 1]);
-        __builtin_amdgcn_sched_barrier(0);
-        const float sa = (float)byte_of(s01[c >> 1], 2 * (c & 1)), sb2 = (float)byte_of(s01[c >> 1], 2 * (c & 1) + 1);
-        const h2 sl = h2{(_Float16)sa, (_Float16)sa}, ol = h2{(_Float16)(-1024.0f * sa), (_Float16)(-1024.0f * sa)};
-        const h2 sh = h2{(_Float16)(sb2 * 0.0625f), (_Float16)(sb2 * 0.0625f)}, oh = h2{(_Float16)(-64.0f * sb2), (_Float16)(-64.0f * sb2)};
-        const unsigned d0 = h == 0 ? wr.q[c].x : wr.q[c].z, d1 = h == 0 ? wr.q[c].y : wr.q[c].w;
-        const unsigned e0 = d0 >> 8, e1 = d1 >> 8;
-        const h8 wlo = mk_h8(lo4(d0, sl, ol), lo4(e0, sl, ol), lo4(d1, sl, ol), lo4(e1, sl, ol));
-        const h8 whi = mk_h8(hi4(d0, sh, oh), hi4(e0, sh, oh), hi4(d1, sh, oh), hi4(e1, sh, oh));
-        const h8 (&f)[4] = fr[gi & 1];
-        if (c < 2) {
-          X[0] = __builtin_amdgcn_mfma_f32_32x32x16_f16(f[0], wlo, X[0], 0, 0, 0);
-          X[1] = __builtin_amdgcn_mfma_f32_32x32x16_f16(f[2], wlo, X[1], 0, 0, 0);
-          X[0] = __builtin_amdgcn_mfma_f32_32x32x16_f16(f[1], whi, X[0], 0, 0, 0);
-          X[1] = __builtin_amdgcn_mfma_f32_32x32x16_f16(f[3], whi, X[1], 0, 0, 0);
-        } else {
-          X2[0] = __builtin_amdgcn_mfma_f32_32x32x16_f16(f[0], wlo, X2[0], 0, 0, 0);
-          X2[1] = __builtin_amdgcn_mfma_f32_32x32x16_f16(f[2], wlo, X2[1], 0, 0, 0);
-          X2[0] = __builtin_amdgcn_mfma_f32_32x32x16_f16(f[1], whi, X2[0], 0, 0, 0);
-          X2[1] = __builtin_amdgcn_mfma_f32_32x32x16_f16(f[3], whi, X2[1], 0, 0, 0);
-        }
-        __builtin_amdgcn_sched_barrier(0);
-      }
-      // M = sum_run m_{run / 2} bsum_run: operand slot (hf, jj) <-> run 8 hf + jj -> sub-block 4 hf + jj / 2
-      const unsigned mw = hf ? wr.hs.w : wr.hs.z;
-      h8 wm;
-#pragma unroll
-      for (int k = 0; k < 4; ++k) { const _Float16 mk = (_Float16)(float)byte_of(mw, k); wm[2 * k] = mk; wm[2 * k + 1] = mk; }
-      const float d = half_bits_to_float((uint16_t)(wr.hd & 0xffff)), dmin = half_bits_to_float((uint16_t)(wr.hd >> 16));
-#pragma unroll
-      for (int tt = 0; tt < 2; ++tt) {
-        const h8 bsf = *(const h8 *)(bs_s + (trow + 32 * tt) * 32 + hf * 16);
-        f16v zero;
-#pragma unroll
-        for (int v = 0; v < 16; ++v) zero[v] = 0.f;
-        const f16v M = __builtin_amdgcn_mfma_f32_32x32x16_f16(bsf, wm, zero, 0, 0, 0);
-#pragma unroll
-        for (int q4 = 0; q4 < 4; ++q4) {  // outputs in pairs
-          const float4 y4 = *(const float4 *)(yd_s + wt * 64 + tt * 32 + 8 * q4 + 4 * hf);
-#pragma unroll
-          for (int k = 0; k < 4; k += 2) {
-            const int v = 4 * q4 + k;
-            const f2 yd2 = k == 0 ? f2{y4.x, y4.y} : f2{y4.z, y4.w};
-            const f2 If = f2{X[tt][v], X[tt][v + 1]} + f2{X2[tt][v], X2[tt][v + 1]};  // (float)isum: one rounding of the exact integer
-            const f2 mm = (f2{dmin, dmin} * yd2) * f2{M[v], M[v + 1]};
-            const f2 t = __builtin_elementwise_fma(f2{d, d} * yd2, If, -mm);
-            const f2 r = __builtin_elementwise_fma(f2{run[tt][v], run[tt][v + 1]}, keep2, t);  // run * 1 + t, or (first superblock of a run) run * 0 + t
-            run[tt][v] = r[0]; run[tt][v + 1] = r[1];
-          }
-        }
-      }
-    } else if constexpr (TYPE == T_Q5_K) {
+    if constexpr (TYPE == T_Q5_K) {
       // operand = sc (q - 16), |.| <= 1008: (1024 + q) sc - 1024 sc = sc q exactly (one packed fma; 1024 sc <= 64512 is an f16 value), then - 16 sc (1040 sc is not an
       // f16 value for sc = 63, so the offset takes a second packed add).  Runs 0 .. 7 and 8 .. 15 go to two accumulators (<= 128 x 1008 x 128 = 16.5 M < 2^24 each,
       // exact); the 16 sc_j bsum terms the offset leaves out are one more MFMA (S, like the mins' M); isum = XA + XB + 16 S is added as int32 and converted once --
@@ -519,6 +458,214 @@ __global__ void __launch_bounds__(GT) gemm_qi_kernel(const GemmArgs a) {
     }
 }
 
+// ------------------------------------------------------------------------------------------------ Q4_K, all prompt lengths
+// What bounds this product is the vector ALU beside the matrix cores: building a run's f16 operand costs ~12 instructions per 32 weight rows, the f32 term 4 per output and
+// superblock, one matrix instruction covers 1024 outputs x 16 values and hides about five of them (measured: 4.3 cycles per vector, ~9 issue cycles per matrix instruction
+// of a SIMD, 32 cycles of matrix pipe; at full matrix rate the card also drops to ~1.5 GHz).  So:
+//   * the operand is sc (q - 8), |.| <= 504: a superblock's sum stays below 504 x 128 x 256 = 16.5 M < 2^24, ONE exact accumulator; the 8 sum_j sc_j bsum_j that the
+//     offset leaves out are a matrix instruction over the run sums (S, like the mins' M), and isum = X + 8 S is one rounding of the exact integer: fma(8, S, X);
+//   * nibbles go to bits 7:4 of a half-word: 64 + q is one v_and_or (0x5400 = 64, 1/16 per mantissa step), sc (q - 8) = (64 + q) sc - 72 sc exactly (9 sc < 2^11);
+//   * d yd and dmin yd of a tile are one v_mfma_f32_32x32x1_2b (two outer products, each rounded once) instead of 32 multiplies;
+//   * reads, operand build and the next superblock's LDS-DMA stand one by one behind the matrix instructions of the step before; small workgroups (4 waves, 32 weight rows
+//     each, NT token tiles) leave two (NT = 2) or three (NT = 1) workgroups per CU, so that one's barriers and latencies run under another's arithmetic;
+//   * the projections that share their input are segments of ONE launch, the experts of a sparse-MoE prompt (windows of the expert-sorted rows) token tiles of one launch.
+// NT = 4 (128 tokens per wave, the operand built once per four matrix instructions) needs 255 registers and the earlier runs' sums in memory: 343 us against 199 us for
+// 28672 x 4096 x 512 tokens.
+struct QiSeg { const uint8_t *w; unsigned w_bytes; int N; float *out; int ldo; };
+struct WideArgs {
+  QiSeg s0, s1, s2; int x1, x2;  // segment of a workgroup: blockIdx.x < x1: s0, < x2: s1, else s2 (x1 = x2 = gridDim.x for a single one)
+  int K, T;
+  const _Float16 *qf; const float *yd; const _Float16 *bsf;
+  int accumulate, ksplit; float *part; int part_n;  // ksplit = 4: workgroup z multiplies run z only, plane z of part [4][T][part_n] takes its sums
+  const int *bounds; int experts;                   // as in GemmArgs
+};
+template <int NT> constexpr int wide_meta = 512 + NT * 32 * 32;     // block scales [32 NT] f32, run sums [32 NT][16] f16
+template <int NT> constexpr int wide_buf = NT * 32 * 512 + wide_meta<NT>;  // + quants; two buffers, each a multiple of 512 (the fragments' exclusive or)
+constexpr int WIDE_ROWS = 128;                                                      // weight rows of a workgroup: four waves
+#ifndef MRS_BLDS16
+// buffer load to LDS, 16 / 4 bytes per lane: LDS destination = wave-uniform base + lane * size
+#define MRS_BLDS16(rsrc, lbase, voff) __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, (__attribute__((address_space(3))) void *)(lbase), 16, voff, 0, 0, 0)
+#define MRS_BLDS4(rsrc, lbase, voff) __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, (__attribute__((address_space(3))) void *)(lbase), 4, voff, 0, 0, 0)
+#define MRS_LDS_BASE(p) ((unsigned)(size_t)(__attribute__((address_space(3))) char *)(p))
+#define MRS_LDS_H8(p, addr, off) (*(const __attribute__((address_space(3))) h8 *)(size_t)((addr) + (off)))
+#endif
+template <int NT>
+__global__ void __launch_bounds__(256, NT == 1 ? 3 : 2) gemm_qi_wide_kernel(const WideArgs a) {
+  extern __shared__ __attribute__((aligned(16))) char smem[];
+  constexpr int TT_ = NT * 32, ACT_ = TT_ * 512, YD_ = wide_meta<NT> - TT_ * 32;
+  const int tid = tid_opaque(), lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int nn = lane & 31, hf = lane >> 5;
+  const int bx = blockIdx.x, seg = bx >= a.x2 ? 2 : bx >= a.x1 ? 1 : 0;
+  const QiSeg sg = seg == 2 ? a.s2 : seg == 1 ? a.s1 : a.s0;
+  const int coff = seg == 2 ? a.s0.N + a.s1.N : seg == 1 ? a.s0.N : 0;
+  int tbeg = 0, tend = a.T, yt = blockIdx.y, ex = 0;
+  if (a.bounds && !expert_tile(a.bounds, a.experts, TT_, yt, ex, tbeg, tend)) return;
+  const uint8_t *wbase = sg.w + (size_t)ex * sg.w_bytes;
+  const int t0 = tbeg + yt * TT_;
+  if (t0 >= tend) return;
+  const int S = a.K / 256, Cs = (S + 3) / 4;
+  const __amdgpu_buffer_rsrc_t rw = __builtin_amdgcn_make_buffer_rsrc((void *)wbase, (short)0, (int)sg.w_bytes, 0x00020000);
+  const unsigned panel = (unsigned)((bx - (seg == 2 ? a.x2 : seg == 1 ? a.x1 : 0)) * 4 + wave);
+  // six loads per superblock: a piece of the next one is requested when this one's has been multiplied (panels past N, superblocks past the end: out of range -> zeros)
+  auto rec_of = [&](int sb) { return (panel * (unsigned)S + (unsigned)sb) * (unsigned)REC_Q4K; };
+  auto load_q = [&](unsigned rec, int c) { return __builtin_amdgcn_raw_buffer_load_b128(rw, rec + (unsigned)(c * 64 + lane) * 16u, 0, 0); };
+  auto load_hs = [&](unsigned rec) { return __builtin_amdgcn_raw_buffer_load_b128(rw, rec + 4096u + (unsigned)nn * 16u, 0, 0); };
+  auto load_hd = [&](unsigned rec) { return __builtin_amdgcn_raw_buffer_load_b32(rw, rec + 4608u + (unsigned)nn * 4u, 0, 0); };
+  // LDS-DMA of superblock sb's rows (8 NT per wave), as in gemm_qi_kernel: chunk ch of row tr at position ch ^ (tr & 31).  Rows past the window hold
+  // whatever follows it in the operand buffer (their outputs are not stored), rows past the buffer zeros.  it = sb - sb_begin
+  const __amdgpu_buffer_rsrc_t rq = __builtin_amdgcn_make_buffer_rsrc((void *)a.qf, (short)0, (int)((size_t)S * a.T * 512), 0x00020000);
+  const __amdgpu_buffer_rsrc_t ry = __builtin_amdgcn_make_buffer_rsrc((void *)a.yd, (short)0, (int)((size_t)S * a.T * 4), 0x00020000);
+  const __amdgpu_buffer_rsrc_t rb = __builtin_amdgcn_make_buffer_rsrc((void *)a.bsf, (short)0, (int)((size_t)S * a.T * 32), 0x00020000);
+  const unsigned dma_row = (unsigned)(hf * 512), dma_ch = (unsigned)((lane & 31) ^ hf) << 4;
+  auto stage_q = [&](int sb, int it, int i) {  // rows 2 i, 2 i + 1 of the wave's 8 NT: 1 KiB
+    MRS_BLDS16(rq, smem + (it & 1) * wide_buf<NT> + (wave * 4 * NT + i) * 1024, dma_row + (dma_ch ^ (unsigned)(((wave * 8 * NT + 2 * i) & 31) << 4)) +
+               ((unsigned)sb * (unsigned)a.T + (unsigned)(t0 + wave * 8 * NT + 2 * i)) * 512u);
+  };
+  auto stage_meta = [&](int sb, int it) {
+    char *meta = smem + (it & 1) * wide_buf<NT> + ACT_;
+    const unsigned row = (unsigned)sb * (unsigned)a.T + (unsigned)t0;
+    if (wave < (NT + 1) / 2 && (NT > 1 || lane < 32)) MRS_BLDS4(ry, meta + wave * 256, (row + (unsigned)(wave * 64 + lane)) * 4u);
+    if (wave < NT) MRS_BLDS16(rb, meta + YD_ + wave * 1024, (row + (unsigned)wave * 32u) * 32u + (unsigned)lane * 16u);
+  };
+  const int n = (int)panel * 32 + nn;
+  float run[NT][16], pend[NT][16];
+#pragma unroll
+  for (int tt = 0; tt < NT; ++tt)
+#pragma unroll
+    for (int v = 0; v < 16; ++v) { run[tt][v] = 0.f; pend[tt][v] = 0.f; }
+  const int sb_begin = a.ksplit > 1 ? (int)blockIdx.z * Cs : 0, sb_end = a.ksplit > 1 ? min(S, sb_begin + Cs) : S;
+  // outputs through bounded buffers that begin at the tile's first row: a lane holds column n, rows 32 tt + 8 (v / 4) + 4 hf + v % 4; a buffer ends behind the window's
+  // last row, columns past N are pushed out of it
+  const bool split = a.ksplit > 1;
+  const int ldo = (split ? a.part_n : sg.ldo) * 4;
+  char *obase = split ? (char *)(a.part + coff) + ((size_t)blockIdx.z * a.T + t0) * ldo : (char *)sg.out + (size_t)t0 * ldo;
+  const __amdgpu_buffer_rsrc_t ro = __builtin_amdgcn_make_buffer_rsrc((void *)obase, (short)0, min(tend - t0, TT_) * ldo - (split ? coff * 4 : 0), 0x00020000);
+  const unsigned vo = (unsigned)(4 * hf * ldo + n * 4) | (n < sg.N ? 0u : 0x80000000u);
+  auto at = [&](int tt, int v) -> unsigned { return vo + (unsigned)((tt * 32 + 8 * (v >> 2) + (v & 3)) * ldo); };
+  auto ld32 = [&](__amdgpu_buffer_rsrc_t r, unsigned off) { return __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(r, off, 0, 0)); };
+  auto st32 = [&](float v, __amdgpu_buffer_rsrc_t r, unsigned off) { __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(v), r, off, 0, 0); };
+  if (sb_begin >= sb_end) {  // a run without superblocks contributes +0 (only with ksplit: S >= 1)
+#pragma unroll
+    for (int tt = 0; tt < NT; ++tt)
+#pragma unroll
+      for (int v = 0; v < 16; ++v) st32(0.f, ro, at(tt, v));
+    return;
+  }
+#pragma unroll
+  for (int i = 0; i < 4 * NT; ++i) stage_q(sb_begin, 0, i);
+  stage_meta(sb_begin, 0);
+  v4u wq[4], hs_next;
+  unsigned hd_next;
+#pragma unroll
+  for (int c = 0; c < 4; ++c) wq[c] = load_q(rec_of(sb_begin), c);
+  hs_next = load_hs(rec_of(sb_begin)); hd_next = load_hd(rec_of(sb_begin));
+  const f16v zero = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+  unsigned mg = 0x54005400u;
+  MRS_OPAQUE_TID(mg);  // keeps the constant in a VGPR: v_and_or_b32 takes one literal
+  auto nib = [&](unsigned v) -> h2 { return as_h2((v & 0x00F000F0u) | mg); };  // 64 + the nibbles at bits 7:4 of the half-words
+  for (int sb = sb_begin; sb < sb_end; ++sb) {
+    const int it = sb - sb_begin;
+    const bool more = sb + 1 < sb_end;
+    const v4u hs = hs_next;
+    const unsigned hd = hd_next, rec_next = more ? rec_of(sb + 1) : 0xF0000000u;
+    h2 sc2[2], of2[2];  // scale of the low / high nibbles' sub-block, - 72 times it
+    auto scales = [&](int c, int hi) {
+      const float f = (float)byte_of(c < 2 ? hs.x : hs.y, 2 * (c & 1) + hi);
+      sc2[hi] = __builtin_bit_cast(h2, __builtin_amdgcn_cvt_pkrtz(f, f));  // an integer below 64: exact
+      of2[hi] = sc2[hi] * h2{(_Float16)-72.0f, (_Float16)-72.0f};
+    };
+    // step k = run 4 c + h (low nibbles) or 4 c + 2 + h (high nibbles) of piece c, in the order (c, h, hi)
+    auto run_of = [](int k) { return 4 * (k >> 2) + 2 * (k & 1) + ((k >> 1) & 1); };
+    auto pair_of = [&](int k, int p) -> h2 {  // operand slots 2 p, 2 p + 1
+      const int c = k >> 2, h = (k >> 1) & 1, hi = k & 1;
+      const unsigned d = h == 0 ? (p < 2 ? wq[c].x : wq[c].y) : (p < 2 ? wq[c].z : wq[c].w);
+      return pkfma(nib(hi ? ((p & 1) ? d >> 8 : d) : ((p & 1) ? d >> 4 : d << 4)), sc2[hi], of2[hi]);
+    };
+    h8 fr[2][NT];
+    h2 w[2][4];
+    scales(0, 0); scales(0, 1);
+#pragma unroll
+    for (int p = 0; p < 4; ++p) w[0][p] = pair_of(0, p);
+    __builtin_amdgcn_sched_barrier(0);
+    MRS_WAIT_VMCNT0();  // this wave's DMA pieces of superblock sb have landed
+    __syncthreads();    // everyone's have, and every wave has finished reading the other buffer
+    hs_next = load_hs(rec_next); hd_next = load_hd(rec_next);
+    // fragment of run r, token tile tt: chunk (2 r + hf) ^ nn of row 32 tt + nn
+    unsigned abase = MRS_LDS_BASE(smem) + (unsigned)((it & 1) * wide_buf<NT> + nn * 512 + ((nn ^ hf) << 4));
+    MRS_OPAQUE_TID(abase);  // one register: the run's offset is one exclusive or on it
+    auto frag = [&](int r, int tt) -> h8 { return MRS_LDS_H8(smem, abase ^ (unsigned)(32 * r), tt * 16384); };
+    f16v X[NT];
+#pragma unroll
+    for (int tt = 0; tt < NT; ++tt) X[tt] = zero;
+    // behind each matrix instruction of a step stand one read and a share of the operand build of the next step, behind the step's first one a piece of the next
+    // superblock's DMA: the wave's own vector and memory instructions run under its matrix instructions (scheduling barriers keep the order)
+#pragma unroll
+    for (int tt = 0; tt < NT; ++tt) fr[0][tt] = frag(run_of(0), tt);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int k = 0; k < 16; ++k) {
+      const h8 wk = mk_h8(w[k & 1][0], w[k & 1][1], w[k & 1][2], w[k & 1][3]);
+#pragma unroll
+      for (int tt = 0; tt < NT; ++tt) {
+        X[tt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(fr[k & 1][tt], wk, X[tt], 0, 0, 0);
+        if (k + 1 < 16) {
+          fr[(k + 1) & 1][tt] = frag(run_of(k + 1), tt);
+          if (tt == 0 && ((k + 1) & 3) == 0) scales((k + 1) >> 2, 0);  // the high nibbles' first step comes one later
+          if (tt == 0 && ((k + 1) & 3) == 1) scales((k + 1) >> 2, 1);
+#pragma unroll
+          for (int p = tt * 4 / NT; p < (tt + 1) * 4 / NT; ++p) w[(k + 1) & 1][p] = pair_of(k + 1, p);
+        }
+        if (tt == 0 && more && (k + 1) % (4 / NT) == 0) stage_q(sb + 1, it + 1, (k + 1) / (4 / NT) - 1);
+        if (tt == NT - 1 && more && k == 0) stage_meta(sb + 1, it + 1);
+        if (tt == NT - 1 && (k & 3) == 2) wq[k >> 2] = load_q(rec_next, k >> 2);  // step k + 1, the piece's last, has been built
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+    const float *yd_s = (const float *)(smem + (it & 1) * wide_buf<NT> + ACT_);
+    const char *bs_s = (const char *)yd_s + YD_;
+    // M = sum_run m_{run / 2} bsum_run, S = sum_run sc_{run / 2} bsum_run: operand slot (hf, jj) <-> run 8 hf + jj -> sub-block 4 hf + jj / 2
+    const unsigned mw = hf ? hs.w : hs.z, sw = hf ? hs.y : hs.x;
+    h8 wm, wsc;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      const _Float16 mk = (_Float16)(float)byte_of(mw, k), sk = (_Float16)(float)byte_of(sw, k);
+      wm[2 * k] = mk; wm[2 * k + 1] = mk; wsc[2 * k] = sk; wsc[2 * k + 1] = sk;
+    }
+    // d yd and dmin yd of the tile's outputs, each product rounded once: one matrix instruction of two 32 x 32 outer products (lane halves = blocks)
+    const float dd = half_bits_to_float((uint16_t)(hf ? hd >> 16 : hd & 0xffff));
+    const float keep = (sb % Cs) == 0 ? 0.f : 1.f;  // the first term of a run of superblocks starts its sum (0 * run + t), the others add (1 * run + t: exact)
+    const f32v zero32 = {0.f};
+#pragma unroll
+    for (int tt = 0; tt < NT; ++tt) {
+      const h8 bsf = *(const h8 *)(bs_s + (tt * 32 + nn) * 32 + hf * 16);
+      const f32v dy = __builtin_amdgcn_mfma_f32_32x32x1f32(yd_s[tt * 32 + nn], dd, zero32, 0, 0, 0);
+      const f16v Sx = __builtin_amdgcn_mfma_f32_32x32x16_f16(bsf, wsc, zero, 0, 0, 0);
+      const f16v M = __builtin_amdgcn_mfma_f32_32x32x16_f16(bsf, wm, zero, 0, 0, 0);
+#pragma unroll
+      for (int v = 0; v < 16; ++v) {
+        const float If = fmaf(8.0f, Sx[v], X[tt][v]);  // (float)isum: one rounding of the exact integer
+        const float t = fmaf(dy[v], If, -(dy[16 + v] * M[v]));
+        run[tt][v] = fmaf(run[tt][v], keep, t);
+      }
+      __builtin_amdgcn_sched_barrier(0);  // one token tile at a time: the sums of all of them would not fit the registers
+    }
+    if ((sb + 1) % Cs == 0 || sb + 1 == sb_end) {  // a run of superblocks ends: its sum joins the row's left-to-right combination
+      const bool first = sb < Cs;
+#pragma unroll
+      for (int tt = 0; tt < NT; ++tt)
+#pragma unroll
+        for (int v = 0; v < 16; ++v) pend[tt][v] = first ? run[tt][v] : pend[tt][v] + run[tt][v];
+    }
+  }
+#pragma unroll
+  for (int tt = 0; tt < NT; ++tt)
+#pragma unroll
+    for (int v = 0; v < 16; ++v) {
+      if (split) st32(run[tt][v], ro, at(tt, v));  // one run per workgroup: combined by gemm_qi_reduce_kernel
+      else st32(a.accumulate ? ld32(ro, at(tt, v)) + pend[tt][v] : pend[tt][v], ro, at(tt, v));
+    }
+}
+
 // ------------------------------------------------------------------------------------------------ Q8_0 weights x Q8_0 activation rows (round 6)
 // The decode engine's Q8_0 term (dec_core2.cuh Tile<T_Q8_0>, oracle term_q8_0): per 32-value block the exact integer dot, p_b = ((float)isum_b dw_b) dx_b, the
 // superblock's T = p_0 + p_1 + ... + p_7 left to right; superblock terms and runs combine as for the K-quants.  One v_mfma_i32_32x32x32_i8 IS one block of 32 tokens x 32
@@ -533,12 +680,14 @@ __global__ void __launch_bounds__(GT) gemm_q80_kernel(const GemmArgs a) {
   const int tid = tid_opaque(), lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int nn = lane & 31, hf = lane >> 5;
   const int n0 = blockIdx.x * TN;
-  const int tbeg = a.win ? a.win[0] : 0, tend = a.win ? a.win[1] : a.T;  // the launch's token rows [tbeg, tend) of the operand buffers (one expert's routes; all rows when dense)
-  const int t0 = tbeg + blockIdx.y * TT;
+  int tbeg = 0, tend = a.T, yt = blockIdx.y, ex = 0;  // the workgroup's token rows [tbeg, tend) of the operand buffers (one expert's routes; all rows when dense)
+  if (a.bounds && !expert_tile(a.bounds, a.experts, TT, yt, ex, tbeg, tend)) return;
+  const uint8_t *wbase = a.w + (size_t)ex * a.w_bytes;
+  const int t0 = tbeg + yt * TT;
   if (t0 >= tend) return;
   const int wn = wave & 3, wt = wave >> 2;
   const int S = a.K / 256, Cs = (S + 3) / 4;
-  const __amdgpu_buffer_rsrc_t rw = __builtin_amdgcn_make_buffer_rsrc((void *)a.w, (short)0, (int)a.w_bytes, 0x00020000);
+  const __amdgpu_buffer_rsrc_t rw = __builtin_amdgcn_make_buffer_rsrc((void *)wbase, (short)0, (int)a.w_bytes, 0x00020000);
   constexpr int REC = REC_Q6K;
   struct WRegs { v4u q[8]; v4u hs; };
   const unsigned panel = (unsigned)((n0 + wn * 32) >> 5);
@@ -662,10 +811,11 @@ __global__ void __launch_bounds__(GT) gemm_q80_kernel(const GemmArgs a) {
     }
 }
 // out[t][n] (+)= ((c0 + c1) + c2) + c3 of the four run sums (the row combination of ORD-U)
-__global__ void __launch_bounds__(256) gemm_qi_reduce_kernel(const float *__restrict__ part, float *__restrict__ out, int T, int N, int ldo, int accumulate) {
-  const size_t i = ((size_t)blockIdx.x * 256 + threadIdx.x) * 4, tot = (size_t)T * N;
-  if (i >= tot) return;
-  const float4 c0 = *(const float4 *)(part + i), c1 = *(const float4 *)(part + tot + i), c2 = *(const float4 *)(part + 2 * tot + i), c3 = *(const float4 *)(part + 3 * tot + i);
+__global__ void __launch_bounds__(256) gemm_qi_reduce_kernel(const float *__restrict__ part, float *__restrict__ out, int T, int N, int ldo, int accumulate, int part_n) {
+  const size_t i = ((size_t)blockIdx.x * 256 + threadIdx.x) * 4, tot = (size_t)T * part_n;  // `part`: the tensor's first column of the launch's [4][T][part_n] sums
+  if (i >= (size_t)T * N) return;
+  const float *pp = part + (i / N) * part_n + i % N;
+  const float4 c0 = *(const float4 *)pp, c1 = *(const float4 *)(pp + tot), c2 = *(const float4 *)(pp + 2 * tot), c3 = *(const float4 *)(pp + 3 * tot);
   float4 r = make_float4(((c0.x + c1.x) + c2.x) + c3.x, ((c0.y + c1.y) + c2.y) + c3.y, ((c0.z + c1.z) + c2.z) + c3.z, ((c0.w + c1.w) + c2.w) + c3.w);
   const size_t t = i / N, n = i % N;  // N % 4 == 0: the four values share a row
   float4 *o = (float4 *)(out + t * ldo + n);
@@ -734,37 +884,72 @@ extern "C" int mrs_gemm_qi_ws(const void *w_qi, int type, int N, int K, const vo
 extern "C" int mrs_gemm_qi(const void *w_qi, int type, int N, int K, const void *act, int T, float *out, int ldo, int accumulate, void *stream) {
   return mrs_gemm_qi_ws(w_qi, type, N, K, act, T, out, ldo, accumulate, nullptr, 0, stream);
 }
-// mrs_gemm_qi_win: the grouped form (MoE prompts): `act` holds T_total operand rows, only rows [win[0], win[1]) (device ints) are multiplied and only those rows of `out`
-// are written; `max_rows` (host) bounds end - begin and sizes the grid.  No split launch (the expert GEMMs fill the chip).
-static int gemm_qi_launch(const void *w_qi, int type, int N, int K, const void *act, int T, const int *win, int max_rows, float *out, int ldo, int accumulate, void *workspace,
-                          size_t workspace_bytes, void *stream);
+// mrs_gemm_qi_multi: up to three tensors of one type that multiply the same operand rows, in one launch where the kernel takes segments.  bounds != NULL (device
+// [experts + 1]): every tensor is a stack of `experts` tensors and expert e multiplies (and writes) the rows [bounds[e], bounds[e + 1]); max_rows (host) bounds one expert's rows.
+extern "C" int mrs_gemm_qi_multi(int type, int nt, const void *const *w_qi, const int *N, int K, const void *act, int T, float *const *out, const int *ldo, int accumulate,
+                                 const int *bounds, int experts, int max_rows, void *workspace, size_t workspace_bytes, void *stream);
 extern "C" int mrs_gemm_qi_win(const void *w_qi, int type, int N, int K, const void *act, int T_total, const int *win, int max_rows, float *out, int ldo, int accumulate, void *stream) {
   if (!win || max_rows <= 0 || max_rows > T_total) return -1;
-  return gemm_qi_launch(w_qi, type, N, K, act, T_total, win, max_rows, out, ldo, accumulate, nullptr, 0, stream);
+  return mrs_gemm_qi_multi(type, 1, &w_qi, &N, K, act, T_total, &out, &ldo, accumulate, win, 1, max_rows, nullptr, 0, stream);
 }
 extern "C" int mrs_gemm_qi_ws(const void *w_qi, int type, int N, int K, const void *act, int T, float *out, int ldo, int accumulate, void *workspace, size_t workspace_bytes,
                               void *stream) {
-  return gemm_qi_launch(w_qi, type, N, K, act, T, nullptr, T, out, ldo, accumulate, workspace, workspace_bytes, stream);
+  return mrs_gemm_qi_multi(type, 1, &w_qi, &N, K, act, T, &out, &ldo, accumulate, nullptr, 0, 0, workspace, workspace_bytes, stream);
 }
-static int gemm_qi_launch(const void *w_qi, int type, int N, int K, const void *act, int T, const int *win, int max_rows, float *out, int ldo, int accumulate, void *workspace,
-                          size_t workspace_bytes, void *stream) {
-  if (!w_qi || !act || !out || !qi::qi_type(type) || N <= 0 || T <= 0 || K <= 0 || K % 256) return -1;
-  qi::GemmArgs a{};
-  a.w = (const uint8_t *)w_qi; a.w_bytes = (unsigned)qi::qi_tensor_bytes(type, N, K); a.type = type; a.N = N; a.K = K; a.T = T;
+template <int NT>
+static void wide_launch(const qi::WideArgs &a, dim3 grid, hipStream_t s) {
+  auto kern = qi::gemm_qi_wide_kernel<NT>;
+  lds_attr_once((const void *)kern, 158 * 1024);
+  hipLaunchKernelGGL(kern, grid, dim3(256), 2 * qi::wide_buf<NT>, s, a);
+}
+extern "C" int mrs_gemm_qi_multi(int type, int nt, const void *const *w_qi, const int *N, int K, const void *act, int T, float *const *out, const int *ldo, int accumulate,
+                                 const int *bounds, int experts, int max_rows, void *workspace, size_t workspace_bytes, void *stream) {
+  if (!w_qi || !N || !act || !out || !ldo || nt < 1 || nt > 3 || !qi::qi_type(type) || T <= 0 || K <= 0 || K % 256 || (bounds && (experts <= 0 || max_rows <= 0))) return -1;
+  int n_all = 0;
+  bool mult4 = true;
+  for (int i = 0; i < nt; ++i) {
+    if (!w_qi[i] || !out[i] || N[i] <= 0) return -1;
+    if (qi::qi_tensor_bytes(type, N[i], K) >= 0xffffff00ull) return -2;
+    n_all += N[i]; mult4 = mult4 && N[i] % 4 == 0;
+  }
+  if ((size_t)(K / 256) * T * 512 >= 0x7fffffffull) return -2;
+  hipStream_t s = (hipStream_t)stream;
   _Float16 *qf, *bsf; float *yd;
   qi_split((void *)act, T, K, &qf, &yd, &bsf);
-  if ((size_t)(K / 256) * T * 512 >= 0x7fffffffull || qi::qi_tensor_bytes(type, N, K) >= 0xffffff00ull) return -2;
-  a.qf = qf; a.yd = yd; a.bsf = bsf; a.out = out; a.ldo = ldo; a.accumulate = accumulate; a.win = win;
-  dim3 grid((N + qi::TN - 1) / qi::TN, (max_rows + qi::TT - 1) / qi::TT);
-  // few workgroups (o_proj / down_proj of a 512-token prompt: 128): one workgroup per run of superblocks, then the reduce -- the same additions in the same order
-  static const int split_max = [] { const char *e = getenv("MRS_GEMM_QI_SPLIT_BELOW"); return e ? atoi(e) : 200; }();
-  a.ksplit = 1; a.part = nullptr;
-  if (!win && (int)(grid.x * grid.y) < split_max && K / 256 >= 4 && N % 4 == 0 && workspace && workspace_bytes >= (size_t)4 * T * N * 4) { a.ksplit = 4; a.part = (float *)workspace; grid.z = 4; }
-  if (type == T_Q8_0) { auto kern = qi::gemm_q80_kernel; lds_attr_once((const void *)kern, 158 * 1024); hipLaunchKernelGGL(kern, grid, dim3(qi::GT), qi::L8_TOTAL, (hipStream_t)stream, a); }
-  else if (type == T_Q4_K) { auto kern = qi::gemm_qi_kernel<T_Q4_K>; lds_attr_once((const void *)kern, 158 * 1024); hipLaunchKernelGGL(kern, grid, dim3(qi::GT), qi::LDS_TOTAL, (hipStream_t)stream, a); }
-  else if (type == T_Q5_K) { auto kern = qi::gemm_qi_kernel<T_Q5_K>; lds_attr_once((const void *)kern, 158 * 1024); hipLaunchKernelGGL(kern, grid, dim3(qi::GT), qi::LDS_TOTAL, (hipStream_t)stream, a); }
-  else { auto kern = qi::gemm_qi_kernel<T_Q6_K>; lds_attr_once((const void *)kern, 158 * 1024); hipLaunchKernelGGL(kern, grid, dim3(qi::GT), qi::LDS_TOTAL, (hipStream_t)stream, a); }
-  if (a.ksplit > 1) hipLaunchKernelGGL(qi::gemm_qi_reduce_kernel, dim3((unsigned)(((size_t)T * N / 4 + 255) / 256)), dim3(256), 0, (hipStream_t)stream, a.part, out, T, N, ldo, accumulate);
+  const bool split_ok = !bounds && K / 256 >= 4 && mult4 && workspace && workspace_bytes >= (size_t)4 * T * n_all * 4;
+  auto reduce = [&](const float *part, int i, int part_n) {
+    hipLaunchKernelGGL(qi::gemm_qi_reduce_kernel, dim3((unsigned)(((size_t)T * N[i] / 4 + 255) / 256)), dim3(256), 0, s, part, out[i], T, N[i], ldo[i], accumulate, part_n);
+  };
+  if (type == T_Q4_K) {
+    // token tiles per wave: 32 rows fill one; from 33 rows on two waste no more and build each operand once for both (measured, 28672 x 4096: 28 us against 38 us at 20
+    // rows, 37 / 37 at 37, 221 / 199 at 512)
+    const int NT = (bounds ? T / experts : T) <= 32 ? 1 : 2, tl = 32 * NT;
+    qi::WideArgs a{};
+    qi::QiSeg *sg[3] = {&a.s0, &a.s1, &a.s2};
+    int gx = 0, x[3] = {0, 0, 0};
+    for (int i = 0; i < nt; ++i) { *sg[i] = qi::QiSeg{(const uint8_t *)w_qi[i], (unsigned)qi::qi_tensor_bytes(type, N[i], K), N[i], out[i], ldo[i]}; gx += (N[i] + qi::WIDE_ROWS - 1) / qi::WIDE_ROWS; x[i] = gx; }
+    a.x1 = x[0]; a.x2 = nt > 1 ? x[1] : gx;
+    a.K = K; a.T = T; a.qf = qf; a.yd = yd; a.bsf = bsf; a.accumulate = accumulate; a.part = (float *)workspace; a.part_n = n_all; a.bounds = bounds; a.experts = experts; a.ksplit = 1;
+    dim3 grid(gx, bounds ? T / tl + experts : (T + tl - 1) / tl);
+    // two workgroups fit a CU: below 512 they are cut by runs of superblocks (4096 x 14336 at 512 tokens, 256 workgroups: 119 us whole, 102 us cut; at 1024 tokens 185 / 192)
+    if (split_ok && (int)(grid.x * grid.y) < 512) { a.ksplit = 4; grid.z = 4; }
+    if (NT == 2) wide_launch<2>(a, grid, s); else wide_launch<1>(a, grid, s);
+    for (int i = 0, c = 0; i < nt && a.ksplit > 1; c += N[i++]) reduce(a.part + c, i, n_all);
+    return 0;
+  }
+  for (int i = 0; i < nt; ++i) {
+    qi::GemmArgs a{};
+    a.w = (const uint8_t *)w_qi[i]; a.w_bytes = (unsigned)qi::qi_tensor_bytes(type, N[i], K); a.type = type; a.N = N[i]; a.K = K; a.T = T;
+    a.qf = qf; a.yd = yd; a.bsf = bsf; a.out = out[i]; a.ldo = ldo[i]; a.accumulate = accumulate; a.bounds = bounds; a.experts = experts;
+    dim3 grid((N[i] + qi::TN - 1) / qi::TN, bounds ? T / qi::TT + experts : (T + qi::TT - 1) / qi::TT);
+    // few workgroups (o_proj / down_proj of a 512-token prompt: 128): one workgroup per run of superblocks, then the reduce -- the same additions in the same order
+    a.ksplit = 1; a.part = nullptr;
+    if (split_ok && (int)(grid.x * grid.y) < 200) { a.ksplit = 4; a.part = (float *)workspace; grid.z = 4; }
+    if (type == T_Q8_0) { auto kern = qi::gemm_q80_kernel; lds_attr_once((const void *)kern, 158 * 1024); hipLaunchKernelGGL(kern, grid, dim3(qi::GT), qi::L8_TOTAL, s, a); }
+    else if (type == T_Q5_K) { auto kern = qi::gemm_qi_kernel<T_Q5_K>; lds_attr_once((const void *)kern, 158 * 1024); hipLaunchKernelGGL(kern, grid, dim3(qi::GT), qi::LDS_TOTAL, s, a); }
+    else { auto kern = qi::gemm_qi_kernel<T_Q6_K>; lds_attr_once((const void *)kern, 158 * 1024); hipLaunchKernelGGL(kern, grid, dim3(qi::GT), qi::LDS_TOTAL, s, a); }
+    if (a.ksplit > 1) reduce(a.part, i, N[i]);
+  }
   return 0;
 }
 

@@ -548,6 +548,11 @@ class Llama {
   // prompts longer than this use the 256-row-tile GEMM over bf16 slabs (its L1-bypassing A loads beat the 128-row f32 kernel even when
   // half of the tile rows are empty: TTFT 16.3 -> 10.1 ms at T = 128, 19.5 -> 8.3 ms at T = 64, 18.5 -> 7.7 ms at T = 32)
   static int prefill_big_min() { static int v = -1; if (v < 0) { const char *e = getenv("MRS_PREFILL_BIG_MIN"); v = e ? atoi(e) : 16; } return v; }
+  // run sums of the exact prompt GEMMs' split launches: q / k / v and o_proj / down_proj at any length, gate / up of short prompts (above 128 tokens they fill the chip)
+  static size_t qi_split_bytes(const mrs_llama_config &c, int T) {
+    const int nq = c.num_heads * c.head_dim, nkv = c.num_kv_heads * c.head_dim;
+    return mrs_gemm_qi_workspace_bytes(T, std::max(std::max(c.hidden_size, nq + 2 * nkv), T <= 128 && c.num_experts == 0 ? 2 * c.intermediate_size : 0));
+  }
   static size_t prefill_workspace_bytes(const mrs_llama_config &c, int T) {
     const size_t t = (size_t)T, d = c.hidden_size, nq = (size_t)c.num_heads * c.head_dim, nkv = (size_t)c.num_kv_heads * c.head_dim;
     const size_t ff = c.intermediate_size;
@@ -557,7 +562,7 @@ class Llama {
     b += align(t * nkv * 4) * 2;      // k, v
     b += align(t * ff * 4) * 3;       // gate, up, act
     b += align((pad_to((int)d, MATRIX_ROW_PADDING) / 32) * 36);  // Q8_1 scratch of the last-token lm_head GEMV
-    b += align(mrs_qi_act_bytes(T, (int)std::max(std::max(d, nq), ff))) + align(mrs_gemm_qi_workspace_bytes(T, (int)std::max(d, nq)));  // exact prompt path: Q8_K operands of T rows (f16 quants, scales, run sums) + run sums of split launches
+    b += align(mrs_qi_act_bytes(T, (int)std::max(std::max(d, nq), ff))) + align(qi_split_bytes(c, T));  // exact prompt path: Q8_K operands of T rows (f16 quants, scales, run sums) + run sums of split launches
     if (T > prefill_big_min()) b += align(t * std::max(std::max(d, nq), ff) * 2) + align(mrs_gemm_q_bf16_workspace_bytes(T)) + align(t * ff * 2);  // bf16 activations + split-K partials + act(gate)*up slabs of the fused gate/up GEMM
     if (c.num_experts > 0) {  // MoE FFN of the prompt: routes = T * top_k rows in expert-sorted order
       const size_t tk = (size_t)std::max(1, (int)c.num_experts_per_tok), r = t * tk, E = (size_t)c.num_experts;
@@ -661,15 +666,12 @@ class Llama {
     const int tg = bl.gate_exps.dtype, td = bl.down_exps.dtype;
     if (mrs_qi_quantize_for(tg, h, nullptr, d, bl.post_attention_layernorm, cfg.rms_eps, T, d, qact, nullptr, s)) return fail("prefill (exact): activation quantizer refused K=%d", d);
     if (mrs_qi_gather_rows(tg, qact, T, m.qact_g, R, d, m.sorted, tk, m.inv, s)) return fail("prefill (exact): operand gather refused");
-    const size_t pg = mrs_gemm_qi_repack_bytes(tg, ff, d), pd = mrs_gemm_qi_repack_bytes(td, d, ff);  // bytes of one expert's panels
-    for (int e = 0; e < E; ++e) {
-      if (mrs_gemm_qi_win((const char *)bl.gate_exps.qi + (size_t)e * pg, tg, ff, d, m.qact_g, R, m.bounds + e, T, g, ff, 0, s) ||
-          mrs_gemm_qi_win((const char *)bl.up_exps.qi + (size_t)e * pg, tg, ff, d, m.qact_g, R, m.bounds + e, T, u, ff, 0, s))
-        return fail("prefill (exact): expert gate / up GEMM refused (ggml dtype %d)", tg);
-    }
+    const void *wgu[2] = {bl.gate_exps.qi, bl.up_exps.qi}, *wd[1] = {bl.down_exps.qi};
+    const int ngu[2] = {ff, ff}, nd[1] = {d};
+    float *ogu[2] = {g, u}, *od[1] = {m.y};
+    if (mrs_gemm_qi_multi(tg, 2, wgu, ngu, d, m.qact_g, R, ogu, ngu, 0, m.bounds, E, T, nullptr, 0, s)) return fail("prefill (exact): expert gate / up GEMM refused (ggml dtype %d)", tg);
     if (mrs_qi_quantize_for(td, g, u, ff, nullptr, 0.f, R, ff, m.qact_r, act, s)) return fail("prefill (exact): activation quantizer refused K=%d", ff);
-    for (int e = 0; e < E; ++e)
-      if (mrs_gemm_qi_win((const char *)bl.down_exps.qi + (size_t)e * pd, td, d, ff, m.qact_r, R, m.bounds + e, T, m.y, d, 0, s)) return fail("prefill (exact): expert down GEMM refused (ggml dtype %d)", td);
+    if (mrs_gemm_qi_multi(td, 1, wd, nd, ff, m.qact_r, R, od, nd, 0, m.bounds, E, T, nullptr, 0, s)) return fail("prefill (exact): expert down GEMM refused (ggml dtype %d)", td);
     if (mrs_moe_fold_exact(h, rs, m.y, m.inv, m.w, T, d, tk, s)) return fail("prefill (exact): moe fold refused");
     return all_reduce(h, (size_t)T * d, s) ? fail("prefill (exact): moe all-reduce failed: %s", g_last_error.c_str()) : 0;
   }
@@ -679,10 +681,13 @@ class Llama {
     const int bs = cfg.block_size, kvh = cfg.num_kv_heads, kvd = cfg.kv_f16 ? 0 : 1;
     const int eff_max = std::min(cfg.max_blocks_per_seq * bs, cfg.max_context_len);
     const int64_t st = (int64_t)(intptr_t)s;
-    auto lin = [&](const GgufMatMul &m, int N, int K, float *out, int acc) -> int {
-      const QTensor *w = m.get_qtensor();
-      return mrs_gemm_qi_ws(w->qi, w->dtype, N, K, qact, T, out, N, acc, N <= std::max(d, nq) ? qws : nullptr, qws_bytes, s) ? fail("prefill (exact): mrs_gemm_qi refused ggml dtype %d (N=%d K=%d)", w->dtype, N, K) : 0;
+    auto lins = [&](int nt, const GgufMatMul *const *m, const int *N, int K, float *const *out, int acc) -> int {  // tensors of one type
+      const void *w[3];
+      for (int i = 0; i < nt; ++i) w[i] = m[i]->get_qtensor()->qi;
+      const int ty = m[0]->get_qtensor()->dtype;
+      return mrs_gemm_qi_multi(ty, nt, w, N, K, qact, T, out, N, acc, nullptr, 0, 0, qws, qws_bytes, s) ? fail("prefill (exact): mrs_gemm_qi_multi refused ggml dtype %d (N=%d K=%d)", ty, N[0], K) : 0;
     };
+    auto lin = [&](const GgufMatMul &m, int N, int K, float *out, int acc) -> int { const GgufMatMul *p = &m; return lins(1, &p, &N, K, &out, acc); };
     // o_proj / down_proj: h <- h + W . x;  tensor parallel: h <- h * (1 / world) + W_shard . x on every rank (the decode step's RESID epilogue, two roundings), then ONE
     // sum all-reduce of h (distributed/layers.rs:965-975) -- the same sums as the decode step whenever the all-reduce adds the ranks in the same order (world 2: always;
     // the peer-mailbox route: rank order for every message it takes)
@@ -706,8 +711,14 @@ class Llama {
         if (done[i]) continue;
         const int ty = m[i]->get_qtensor()->dtype, mode = ty == Q8_0 ? 1 : 0;
         if (mrs_qi_quantize_for(ty, x, x2, ldx, nw, cfg.rms_eps, T, K, qact, xtmp, s)) return fail("prefill (exact): activation quantizer refused K=%d (ggml dtype %d)", K, ty);
-        for (size_t j = i; j < m.size(); ++j)
-          if (!done[j] && ((m[j]->get_qtensor()->dtype == Q8_0) ? 1 : 0) == mode) { if (lin(*m[j], n[j], K, o[j], acc)) return -1; done[j] = true; }
+        for (size_t j = i; j < m.size(); ++j) {
+          const int tj = m[j]->get_qtensor()->dtype;
+          if (done[j] || (tj == Q8_0 ? 1 : 0) != mode) continue;
+          const GgufMatMul *mm[3]; int nn[3]; float *oo[3]; int c = 0;
+          for (size_t l = j; l < m.size(); ++l)
+            if (!done[l] && m[l]->get_qtensor()->dtype == tj) { mm[c] = m[l]; nn[c] = n[l]; oo[c] = o[l]; ++c; done[l] = true; }
+          if (lins(c, mm, nn, K, oo, acc)) return -1;
+        }
       }
       return 0;
     };
@@ -749,7 +760,7 @@ class Llama {
     float *g = (float *)take(t * ff * 4), *u = (float *)take(t * ff * 4), *act = (float *)take(t * ff * 4);
     if (prefill_exact_ok()) {
       void *qact = take(mrs_qi_act_bytes(T, std::max(std::max(d, nq), ff)));
-      const size_t qws_bytes = mrs_gemm_qi_workspace_bytes(T, std::max(d, nq));
+      const size_t qws_bytes = qi_split_bytes(cfg, T);
       void *qws = take(qws_bytes);
       MoeExactBufs mx{};
       if (cfg.num_experts > 0) {  // routes = T * top_k rows in expert-sorted order; g / u / act become [routes][ff]

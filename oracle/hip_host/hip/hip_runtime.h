@@ -266,6 +266,23 @@ static hiphost_f32x16 mfma_32x32x2_f32(float a, float b, hiphost_f32x16 c) {
 }
 }  // namespace hiphost
 #define __builtin_amdgcn_mfma_f32_32x32x2f32(A, B, C, CBSZ, ABID, BLGP) hiphost::mfma_32x32x2_f32((A), (B), (C))
+// v_mfma_f32_32x32x1_2b_f32: two blocks of outer products, D_b = C_b + a_b b_b: lane l holds a_b[l % 32] and b_b[l % 32] of block b = l / 32; registers 16 b .. 16 b + 15
+// are block b in the layout of every 32 x 32 MFMA
+typedef float hiphost_f32x32 __attribute__((ext_vector_type(32)));
+namespace hiphost {
+static hiphost_f32x32 mfma_32x32x1_f32(float a, float b, hiphost_f32x32 c) {
+  const int tid = linear_tid(), w = tid / WAVE, lane = tid & (WAVE - 1), base = w * WAVE;
+  mfma_af[tid] = a; mfma_bf[tid] = b;
+  wave_barrier(w, 0);
+  const int col = lane & 31, hi = lane >> 5;
+  hiphost_f32x32 d = c;
+  for (int k = 0; k < 2; ++k)
+    for (int i = 0; i < 16; ++i) d[16 * k + i] = fmaf(mfma_af[base + 32 * k + 8 * (i / 4) + 4 * hi + (i % 4)], mfma_bf[base + 32 * k + col], c[16 * k + i]);
+  wave_barrier(w, 0);
+  return d;
+}
+}  // namespace hiphost
+#define __builtin_amdgcn_mfma_f32_32x32x1f32(A, B, C, CBSZ, ABID, BLGP) hiphost::mfma_32x32x1_f32((A), (B), (C))
 // v_mfma_i32_32x32x32_i8: D = A (32 x 32 int8) * B (32 x 32 int8) + C, exact in int32.  Lane l holds A[l % 32][16 * (l / 32) + j] and
 // B[16 * (l / 32) + j][l % 32] (j = 0..15, 16 consecutive bytes); C / D as every 32 x 32 MFMA (the layout of the accumulators is dtype-independent).
 // Which 16 k a lane half holds does not change the result as long as A and B agree -- they do by symmetry.
@@ -335,6 +352,12 @@ static inline short hiphost_raw_buffer_load_b16(__amdgpu_buffer_rsrc_t r, unsign
   if (o + 2 <= r.bytes) memcpy(&v, r.base + o, 2);
   return v;
 }
+static inline void hiphost_raw_buffer_store_b32(unsigned v, __amdgpu_buffer_rsrc_t r, unsigned voff) {
+  if ((unsigned long long)voff + 4 <= r.bytes) memcpy((char *)r.base + voff, &v, 4);
+}
+#define __builtin_amdgcn_raw_buffer_store_b32(V, R, VOFF, SOFF, AUX) hiphost_raw_buffer_store_b32((V), (R), (VOFF))
+typedef _Float16 hiphost_h2 __attribute__((ext_vector_type(2)));
+#define __builtin_amdgcn_cvt_pkrtz(A, B) (hiphost_h2{(_Float16)(A), (_Float16)(B)}) /* used on values that f16 holds exactly */
 #define __builtin_amdgcn_raw_buffer_load_b32(R, VOFF, SOFF, AUX) hiphost_raw_buffer_load_b32((R), (VOFF), (SOFF))
 typedef unsigned hiphost_v2u __attribute__((ext_vector_type(2)));
 static inline hiphost_v2u hiphost_raw_buffer_load_b64(__amdgpu_buffer_rsrc_t r, unsigned voff, unsigned soff) {
@@ -366,6 +389,14 @@ namespace hiphost { inline unsigned long long fake_realtime() { static thread_lo
 // LDS-DMA (global_load_lds): LDS destination = wave-uniform base + lane * size, source address per lane; synchronous here
 #define MRS_GLDS16(gptr, lbase) memcpy((char *)(lbase) + (hiphost::linear_tid() & 63) * 16, (const void *)(gptr), 16)
 #define MRS_GLDS4(gptr, lbase) memcpy((char *)(lbase) + (hiphost::linear_tid() & 63) * 4, (const void *)(gptr), 4)
+#define MRS_BLDS16(RSRC, LBASE, VOFF) hiphost_buffer_load_lds((RSRC), (char *)(LBASE) + (hiphost::linear_tid() & 63) * 16, 16, (VOFF))
+#define MRS_BLDS4(RSRC, LBASE, VOFF) hiphost_buffer_load_lds((RSRC), (char *)(LBASE) + (hiphost::linear_tid() & 63) * 4, 4, (VOFF))
+static inline void hiphost_buffer_load_lds(__amdgpu_buffer_rsrc_t r, char *dst, unsigned n, unsigned voff) {
+  const unsigned long long o = voff;
+  if (o + n <= r.bytes) memcpy(dst, r.base + o, n); else memset(dst, 0, n);
+}
+#define MRS_LDS_BASE(P) 0u
+#define MRS_LDS_H8(P, ADDR, OFF) (*(const h8 *)((P) + (ADDR) + (OFF)))
 #define MRS_WAIT_VMCNT0() ((void)0)                                     /* product code: s_waitcnt vmcnt(0) */
 #define __builtin_amdgcn_fence(ORDER, SCOPE) ((void)0)                  /* one workgroup runs at a time: nothing to order */
 #define __builtin_amdgcn_s_sleep(N) ((void)0)

@@ -154,3 +154,57 @@ def test_mfma_f16_accumulates_small_integers_exactly(dev):
             assert np.array_equal(got, ref)
     got, ref = run(np.full((16, 32, 16), 504), np.full((16, 32, 16), -128))  # |sum| = 16.5 M, the largest a Q4_K superblock can reach
     assert np.array_equal(got, ref) and ref[0, 0] == -16515072
+
+
+def run_multi(O, be, tname, ns, k, T, bounds=None, ws=False, acc=False, seed=0):
+    """mrs_gemm_qi_multi: several tensors on the same operand rows; with `bounds` every tensor is a stack whose expert e takes the rows bounds[e] .. bounds[e + 1] - 1."""
+    t = getattr(O, tname)
+    rng = np.random.default_rng(seed)
+    E = len(bounds) - 1 if bounds is not None else 1
+    x = rng.standard_normal((T, k)).astype(np.float32)
+    act = be.buf(np.zeros(be.sym("mrs_qi_act_bytes", [CI, CI], C.c_size_t)(T, k), np.uint8))
+    xb = be.buf(x)
+    assert be.sym("mrs_qi_quantize_for", [CI, VP, VP, CI, VP, C.c_float, CI, CI, VP, VP, VP], CI)(t, xb.ptr, None, k, None, 1e-5, T, k, act.ptr, None, be.stream) == 0
+    keep, packed, base, outs = [act, xb], [], [], []
+    for n in ns:
+        p = O.quantize(t, (rng.standard_normal((E * n, k)) * 0.05).astype(np.float32)).reshape(E * n, -1)
+        nb = be.sym("mrs_gemm_qi_repack_bytes", [CI, C.c_longlong, C.c_longlong], C.c_size_t)(t, E * n, k)
+        src, wq = be.buf(np.ascontiguousarray(p).reshape(-1)), be.buf(np.full(nb, 0xA5, np.uint8))
+        assert be.sym("mrs_gemm_qi_repack", [VP, CI, C.c_longlong, C.c_longlong, VP, VP], CI)(src.ptr, t, E * n, k, wq.ptr, be.stream) == 0
+        b = rng.standard_normal((T, n)).astype(np.float32)
+        o = be.buf(b.copy())
+        keep += [src, wq]; packed.append(p); base.append(b); outs.append((wq, o))
+    bb = be.buf(np.asarray(bounds, np.int32)) if bounds is not None else None
+    w = be.buf(np.zeros(4 * T * sum(ns), np.float32)) if ws else None
+    ptrs = lambda i: (VP * len(ns))(*[o[i].ptr for o in outs])  # noqa: E731
+    ints = (CI * len(ns))(*ns)
+    rc = be.sym("mrs_gemm_qi_multi", [CI, CI, VP, VP, CI, VP, CI, VP, VP, CI, VP, CI, CI, VP, C.c_size_t, VP], CI)(
+        t, len(ns), ptrs(0), ints, k, act.ptr, T, ptrs(1), ints, int(acc), bb.ptr if bb else None, E, T, w.ptr if ws else None, 4 * T * sum(ns) * 4 if ws else 0, be.stream)
+    assert rc == 0, rc
+    for n, p, b, (_, o) in zip(ns, packed, base, outs):
+        want = b.copy()
+        for e in range(E):
+            lo, hi = (bounds[e], bounds[e + 1]) if bounds is not None else (0, T)
+            for r in range(lo, hi):
+                want[r] = O.gemv_engine(t, p[e * n:(e + 1) * n], n, k, x[r])[0] + (b[r] if acc else 0)
+        got = o.numpy()
+        assert np.array_equal(got, want), (tname, n, int((got != want).sum()))
+
+
+# segments of 1 .. 3 tensors with ragged row counts; one / two token tiles per wave with remainders; windows that are empty, one row, a tile and a tile + 1; runs of superblocks
+# that are empty (5 superblocks: 2, 2, 1, 0) and whole launches cut by runs
+MULTI = [("Q4_K", (40,), 512, 70, None, False, False), ("Q4_K", (130, 33, 64), 1280, 33, None, False, True), ("Q4_K", (128, 36), 1280, 65, None, True, True),
+         ("Q4_K", (64, 32), 1024, 5, None, True, False), ("Q4_K", (32, 64), 512, 130, (0, 0, 64, 129, 130), False, False), ("Q4_K", (64,), 768, 40, (0, 33, 34, 34, 40), False, False),
+         ("Q6_K", (40, 64), 512, 9, None, False, False), ("Q6_K", (64,), 512, 20, (0, 0, 1, 20), False, False), ("Q8_0", (40, 64), 512, 9, None, False, False),
+         ("Q8_0", (64,), 512, 20, (0, 0, 1, 20), False, False), ("Q5_K", (64,), 512, 20, (0, 7, 7, 20), False, False)]
+
+
+@pytest.mark.parametrize("case", MULTI)
+def test_gemm_qi_multi_host_emulation(oracle, case):
+    run_multi(oracle, HostBackend(), *case, seed=3)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("case", MULTI + [("Q4_K", (1024, 256, 256), 4096, 200, None, True, True), ("Q4_K", (512,), 1024, 400, (0, 100, 100, 333, 400), False, False)])
+def test_gemm_qi_multi_gpu(oracle, dev, case):
+    run_multi(oracle, GpuBackend(dev), *case, seed=4)
