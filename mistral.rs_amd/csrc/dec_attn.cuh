@@ -44,7 +44,8 @@ __device__ __forceinline__ void attn_load_block(const AttnArgs &a, size_t base, 
 // The online-softmax update of one block for the G query heads in q_s (G * 128 floats of wave-private LDS; p_s: G * 32): scores by fma chains over the lane's 64
 // dims + the other half, block max / sum trees, fast_exp, (WITH_V) o = o * alpha + P.V by fma chains.  `first` = first block of the split (l = o = 0: no correction).
 // EVERY engine attention path (decode split kernel, prompt kernel) goes through this function: same bits.
-template <int G, class CT, bool WITH_V>
+// TAIL = false: only the sequence's last block is cleared past the context (a wave-uniform branch; 64 selects per other block less)
+template <int G, class CT, bool WITH_V, bool TAIL = true>
 __device__ __forceinline__ void attn_block_update(const AttnArgs &a, const int4 (&kr)[8], const int4 (&vr)[8], const float *q_s, float *p_s, int b, bool first, int ctx,
                                                   int lo, float (&m)[G], float (&l)[G], float (&o0)[G], float (&o1)[G]) {
   constexpr int HD = 128, BS = 32;
@@ -89,14 +90,17 @@ __device__ __forceinline__ void attn_block_update(const AttnArgs &a, const int4 
   }
   if (!WITH_V) return;
   MRS_WAVE_SYNC();
+  const bool cut = TAIL || (b + 1) * BS > ctx;
 #pragma unroll
   for (int r = 0; r < 2; ++r) {
 #pragma unroll
     for (int c = 0; c < 4; ++c) {
       float vf[8];
       unpack16<CT>(vr[r * 4 + c], vf);
+      if (cut) {
 #pragma unroll
-      for (int j = 0; j < 8; ++j) vf[j] = (b * BS + c * 8 + j < ctx) ? vf[j] : 0.f;  // stale slots may hold NaNs
+        for (int j = 0; j < 8; ++j) vf[j] = (b * BS + c * 8 + j < ctx) ? vf[j] : 0.f;  // stale slots may hold NaNs
+      }
 #pragma unroll
       for (int g = 0; g < G; ++g) {
         const float4 pa = *(const float4 *)(p_s + g * BS + c * 8);
@@ -113,7 +117,8 @@ __device__ __forceinline__ void attn_block_update(const AttnArgs &a, const int4 
 
 // q_s: G * 128 floats, p_s: G * 32 floats of wave-private LDS; the item covers query heads [head0, head0 + G) of kv head kvh
 // blocks [b0, b1) of the sequence; sink(g, o0, o1, m, l) receives the un-normalised partial of query head head0 + g (o0 / o1: dims lane / lane + 64)
-template <int G, class CT, class Sink>
+// ONE: splits of a single block (b1 = b0 + 1), without the registers of a second one
+template <int G, class CT, bool ONE = false, class Sink>
 __device__ __forceinline__ void attn_split_core(const AttnArgs &a, int kvh, int head0, int seq, int b0, int b1, float *q_s, float *p_s, Sink sink, int first_page = -1) {
   constexpr int HD = 128;
   const int lane = lane_opaque();
@@ -134,12 +139,27 @@ __device__ __forceinline__ void attn_split_core(const AttnArgs &a, int kvh, int 
   float m[G], l[G], o0[G], o1[G];
 #pragma unroll
   for (int g = 0; g < G; ++g) { m[g] = -FLT_MAX; l[g] = 0.f; o0[g] = 0.f; o1[g] = 0.f; }
-  for (int b = b0; b < b1; ++b) {
-    if (b > b0) {
-      const size_t base = (size_t)bt[b] * a.kv_block_stride + (size_t)kvh * a.kv_head_stride;
-      attn_load_block<true>(a, base, kr, vr);
-    }
-    attn_block_update<G, CT, true>(a, kr, vr, q_s, p_s, b, b == b0, ctx, lo, m, l, o0, o1);
+  if constexpr (ONE) {
+    attn_block_update<G, CT, true, false>(a, kr, vr, q_s, p_s, b0, true, ctx, lo, m, l, o0, o1);
+#pragma unroll
+    for (int g = 0; g < G; ++g) sink(g, o0[g], o1[g], m[g], l[g]);
+    return;
+  }
+  // The next block's K / V are in flight while a block is worked on (its page index was read one block earlier): a split of several blocks -- contexts above 2048 tokens --
+  // used to pay a memory latency per block (four at 7000 tokens: a Llama-3-8B step of 2644 us, 2591 us with the merge's partials requested ahead as well)
+  int4 kn[8], vn[8];
+  unsigned page = b0 + 1 < b1 ? bt[b0 + 1] : 0;
+  auto request = [&](int b, int4 (&k)[8], int4 (&v)[8]) {
+    const size_t base = (size_t)page * a.kv_block_stride + (size_t)kvh * a.kv_head_stride;
+    if (b + 1 < b1) page = bt[b + 1];
+    attn_load_block<true>(a, base, k, v);
+  };
+  for (int b = b0; b < b1; b += 2) {
+    if (b + 1 < b1) request(b + 1, kn, vn);
+    attn_block_update<G, CT, true, false>(a, kr, vr, q_s, p_s, b, b == b0, ctx, lo, m, l, o0, o1);
+    if (b + 1 >= b1) break;
+    if (b + 2 < b1) request(b + 2, kr, vr);
+    attn_block_update<G, CT, true, false>(a, kn, vn, q_s, p_s, b + 1, false, ctx, lo, m, l, o0, o1);
   }
 #pragma unroll
   for (int g = 0; g < G; ++g) sink(g, o0[g], o1[g], m[g], l[g]);

@@ -126,7 +126,7 @@ struct Attn2Args {
 };
 // merge of one (sequence, kv head): wave w <-> query heads (2w, 2w + 1) of the group (G == 1: wave 0, one head in lanes 0..31), lane = 4 consecutive
 // dims, sequential over the splits.  AGENT: the partials were published by other workgroups of the SAME launch (sc1 loads); else plain loads.
-template <int G, bool AGENT>
+template <int G, bool AGENT, int MB>
 __device__ __forceinline__ void attn2_merge(const Attn2Args &a, int kvh, int seq, int ns, int wave, int lane, int ncols) {
   constexpr int HD = 128, NP = (G + 1) / 2;
   const AttnArgs &t = a.t;
@@ -138,11 +138,10 @@ __device__ __forceinline__ void attn2_merge(const Attn2Args &a, int kvh, int seq
   auto ldw = [&](const float *p) { if constexpr (AGENT) return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); else return *p; };
   const float mA = lane < ns ? ldw(t.part_m + pA + lane) : -FLT_MAX, lA = lane < ns ? ldw(t.part_l + pA + lane) : 0.f;
   const float mB = lane < ns ? ldw(t.part_m + pB + lane) : -FLT_MAX, lB = lane < ns ? ldw(t.part_l + pB + lane) : 0.f;
-  // one descriptor for both heads' partials (wave-uniform); the lanes of head B add its distance.  The partial outputs of up to 16 splits are
-  // requested before anything is consumed
+  // one descriptor for both heads' partials (wave-uniform); the lanes of head B add its distance.  The partial outputs of 2 MB splits are
+  // in flight at a time
   const __amdgpu_buffer_rsrc_t ro = __builtin_amdgcn_make_buffer_rsrc((void *)(t.part_o + pA * HD), (short)0, (int)((pB - pA + ns) * HD * 4), 0x00020000);
   const unsigned off0 = (unsigned)(lane & 31) * 16u + (hsel ? (unsigned)((pB - pA) * HD * 4) : 0u);
-  constexpr int MB = 16;
   constexpr int AUX = AGENT ? 16 : 0;
   v4u r[MB];
 #pragma unroll
@@ -161,14 +160,23 @@ __device__ __forceinline__ void attn2_merge(const Attn2Args &a, int kvh, int seq
     const float t0 = o.x * wj, t1 = o.y * wj, t2 = o.z * wj, t3 = o.w * wj;
     acc.x = acc.x + t0; acc.y = acc.y + t1; acc.z = acc.z + t2; acc.w = acc.w + t3;
   };
-  for (int j0 = 0; j0 < ns; j0 += MB) {
-    if (j0 > 0) {
+  // the next MB partials are in flight while MB are added up: the merge is the launch's serial tail, and every batch used to pay a memory latency of its own
+  v4u rn[MB];
+  auto request = [&](int j0, v4u (&x)[MB]) {
 #pragma unroll
-      for (int i = 0; i < MB; ++i) r[i] = __builtin_amdgcn_raw_buffer_load_b128(ro, off0 + (unsigned)(j0 + i) * 512u, 0, AUX);
-    }
+    for (int i = 0; i < MB; ++i) x[i] = __builtin_amdgcn_raw_buffer_load_b128(ro, off0 + (unsigned)(j0 + i) * 512u, 0, AUX);
+  };
+  auto add = [&](int j0, v4u (&x)[MB]) {
 #pragma unroll
     for (int i = 0; i < MB; ++i)
-      if (j0 + i < ns) step(j0 + i, r[i]);  // wave-uniform
+      if (j0 + i < ns) step(j0 + i, x[i]);  // wave-uniform
+  };
+  for (int j0 = 0; j0 < ns; j0 += 2 * MB) {
+    if (j0 + MB < ns) request(j0 + MB, rn);
+    add(j0, r);
+    if (j0 + MB >= ns) break;
+    if (j0 + 2 * MB < ns) request(j0 + 2 * MB, r);
+    add(j0 + MB, rn);
   }
   const float inv = 1.0f / s_all;
   const float4 v = make_float4(acc.x * inv, acc.y * inv, acc.z * inv, acc.w * inv);
@@ -183,7 +191,8 @@ __device__ __forceinline__ void attn2_merge(const Attn2Args &a, int kvh, int seq
 // Round 5 geometry: grid (kv heads, sequences, splits), G waves per workgroup: wave g = query head head0 + g of ONE split (round 4: 4 splits per workgroup, every wave
 // all G heads: 56 workgroups of 329 VGPRs at a 512-token context).  The per-head arithmetic is the same function (attn_split_core<1>): same bits; the G waves read the
 // same 16 KB of K / V (L1 / L2 hits), every wave's serial chain is 1 / G as long, and a 512-token context fills 8 x 24 = 192 CUs.
-template <int G, class CT, bool TICKET>
+// ONE: splits of one block (contexts up to 2048 tokens); registers for four waves per SIMD, where a batch's many small splits are what fills the chip
+template <int G, class CT, bool TICKET, bool ONE>
 __global__ void __launch_bounds__(64 * G) dec_attn2_kernel(const Attn2Args a) {
   constexpr int HD = 128;
   __shared__ __attribute__((aligned(16))) float q_s[G][HD + 32];
@@ -218,7 +227,7 @@ __global__ void __launch_bounds__(64 * G) dec_attn2_kernel(const Attn2Args a) {
     if (b1 * 32 <= lo_w) {  // every block of the split lies before the sliding window: the partial a fully masked pass would give, without reading K / V
       publish(0, 0.f, 0.f, -FLT_MAX, 0.f);
     } else {
-      attn_split_core<1, CT>(t, kvh, head0 + wave, seq, b0, b1, q_s[wave], q_s[wave] + HD, publish, (int)blk_first);
+      attn_split_core<1, CT, ONE>(t, kvh, head0 + wave, seq, b0, b1, q_s[wave], q_s[wave] + HD, publish, (int)blk_first);
     }
   }
   if constexpr (TICKET) {
@@ -237,7 +246,7 @@ __global__ void __launch_bounds__(64 * G) dec_attn2_kernel(const Attn2Args a) {
     __syncthreads();
     if (!last_s) return;
     if (tid == 0) __hip_atomic_store(tk, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);  // every other workgroup of this (seq, kv head) has already drawn
-    attn2_merge<G, true>(a, kvh, seq, ns, wave, lane, gridDim.y);
+    attn2_merge<G, true, ONE ? 8 : 16>(a, kvh, seq, ns, wave, lane, gridDim.y);
   }
 }
 // the merge as its own launch: grid (kv heads, sequences), (G + 1) / 2 waves
@@ -245,7 +254,7 @@ template <int G>
 __global__ void __launch_bounds__(64 * ((G + 1) / 2)) dec_attn2_merge_kernel(const Attn2Args a) {
   const int tid = tid_opaque(), lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int nblk = ((int)a.t.context_lens[blockIdx.y] + 31) / 32;
-  attn2_merge<G, false>(a, blockIdx.x, blockIdx.y, (nblk + a.t.bpw - 1) / a.t.bpw, wave, lane, gridDim.y);
+  attn2_merge<G, false, 16>(a, blockIdx.x, blockIdx.y, (nblk + a.t.bpw - 1) / a.t.bpw, wave, lane, gridDim.y);
 }
 
 
@@ -553,9 +562,10 @@ extern "C" int mrs_dec_attention(float *out_f32, void *img_out, unsigned *ticket
   const dim3 mgrid(num_kv_heads, num_seqs);
 #define MRS_A2(GG, CT)                                                                                                   \
   do {                                                                                                                   \
-    if (one_launch) hipLaunchKernelGGL((dec_attn2_kernel<GG, CT, true>), grid, dim3(64 * GG), 0, s, a);                      \
+    if (one_launch && t.bpw == 1) hipLaunchKernelGGL((dec_attn2_kernel<GG, CT, true, true>), grid, dim3(64 * GG), 0, s, a);  \
+    else if (one_launch) hipLaunchKernelGGL((dec_attn2_kernel<GG, CT, true, false>), grid, dim3(64 * GG), 0, s, a);          \
     else {                                                                                                               \
-      hipLaunchKernelGGL((dec_attn2_kernel<GG, CT, false>), grid, dim3(64 * GG), 0, s, a);                                   \
+      hipLaunchKernelGGL((dec_attn2_kernel<GG, CT, false, false>), grid, dim3(64 * GG), 0, s, a);                            \
       hipLaunchKernelGGL((dec_attn2_merge_kernel<GG>), mgrid, dim3(64 * ((GG + 1) / 2)), 0, s, a);                       \
     }                                                                                                                    \
   } while (0)
