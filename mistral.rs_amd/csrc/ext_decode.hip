@@ -463,6 +463,24 @@ __global__ void __launch_bounds__(64) sample_advance_kernel(const SampleArgs a) 
   if (c == 0) *a.step_counter = step + 1;
 }
 
+// The decode state of b sequences from the host's token ids and positions, which travel in the launch's arguments: one launch without a synchronisation, where four
+// copies from pageable memory and a read-back of the block table cost a scheduler step about 0.2 ms.  The slot rule is sample_advance_kernel's.
+constexpr int STATE_MAX = 64;  // sequences of a launch (a model is made for up to 8)
+struct StateArgs {
+  int32_t ids[STATE_MAX], pos[STATE_MAX];
+  int32_t *input_ids, *positions; uint32_t *context_lens; int64_t *slot_mapping; const uint32_t *block_tables;
+  int b, max_blocks, block_size;
+};
+__global__ void __launch_bounds__(64) set_state_kernel(const StateArgs a) {
+  const int c = threadIdx.x;
+  if (c >= a.b) return;
+  const int pos = a.pos[c], blk = pos / a.block_size;
+  a.input_ids[c] = a.ids[c];
+  a.positions[c] = pos;
+  a.context_lens[c] = (uint32_t)pos + 1;
+  a.slot_mapping[c] = blk < a.max_blocks ? (int64_t)a.block_tables[(size_t)c * a.max_blocks + blk] * a.block_size + pos % a.block_size : (int64_t)-1;
+}
+
 // round 6, batch 1: sample_advance_kernel + the NEXT step's embedding gather in one launch (the captured decode graph then opens with layer 0's qkv: the step is two
 // launches shorter -- argmax_partial_kernel lives in lm_head's epilogue, mrs_dec_proj_argmax, and embedding_kernel here).  a.scratch[0] holds the packed maximum.
 struct EmbedNext { const uint8_t *table; int type; float *h; int K; };
@@ -809,6 +827,19 @@ extern "C" int mrs_quantize_rows_q8_1(const float *x, void *y, int K, int stride
 }
 
 // batch 1, the maximum already in scratch[0] (mrs_dec_proj_argmax): next id, state advance and h_next = embedding row of the next id (mrs_embedding's values)
+// ids / pos: HOST arrays [b]; the rest device buffers of at least b entries (block_tables [b][max_blocks])
+extern "C" int mrs_set_state(const int32_t *ids, const int32_t *pos, int b, int32_t *input_ids, int32_t *positions, uint32_t *context_lens, int64_t *slot_mapping,
+                             const uint32_t *block_tables, int max_blocks, int block_size, void *stream) {
+  if (!ids || !pos || b <= 0 || b > STATE_MAX || !input_ids || !positions || !context_lens || !slot_mapping || !block_tables || max_blocks <= 0 || block_size <= 0) return -1;
+  for (int c = 0; c < b; ++c)
+    if (pos[c] < 0) return -1;
+  StateArgs a{};
+  for (int c = 0; c < b; ++c) { a.ids[c] = ids[c]; a.pos[c] = pos[c]; }
+  a.input_ids = input_ids; a.positions = positions; a.context_lens = context_lens; a.slot_mapping = slot_mapping; a.block_tables = block_tables;
+  a.b = b; a.max_blocks = max_blocks; a.block_size = block_size;
+  hipLaunchKernelGGL(set_state_kernel, dim3(1), dim3(64), 0, (hipStream_t)stream, a);
+  return 0;
+}
 extern "C" int mrs_sample_advance_embed(int32_t *next_ids, int32_t *tokens_out, int tokens_out_stride, int32_t *step_counter, int32_t *positions, uint32_t *context_lens,
                                         int64_t *slot_mapping, const uint32_t *block_tables, int max_blocks, int block_size, void *scratch, const void *table, int type,
                                         float *h_next, int K, void *stream) {

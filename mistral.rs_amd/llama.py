@@ -174,6 +174,7 @@ class Llama:
         want = os.environ.get("MRS_PREFILL_BF16_SHADOW", "auto")
         self._bf16_shadow_wanted = (want == "1" or (want == "auto" and shadow_bytes <= float(os.environ.get("MRS_BF16_SHADOW_MAX_GB", "24")) * 2 ** 30)) \
             and not cfg.num_experts and device.type == "cuda"
+        L.mrs_set_state.argtypes = [C.c_void_p, C.c_void_p, C.c_int] + [C.c_void_p] * 5 + [C.c_int, C.c_int, C.c_void_p]
         L.mrs_dequantize.argtypes = [C.c_void_p, C.c_int, C.c_longlong, C.c_int, C.c_void_p, C.c_int, C.c_void_p]
         L.mrs_llama_set_bf16_tensor.argtypes = [C.c_void_p, C.c_char_p, C.c_void_p]
         L.mrs_last_error.restype = C.c_char_p
@@ -230,6 +231,7 @@ class Llama:
         self._chk(L.mrs_llama_set_buffers(self._h, C.byref(b)))
         self._graph = None
         self._replays_left = None
+        self._state_pos = None  # positions of the last set_state() while the device state is still that
         self._graph_chained = False  # the captured step is the chained one (mrs_llama_decode_step_chained): it expects the hidden-state buffer to hold embedding(input_ids)
         self._need_embed = True      # ... which is stale whenever the host changed input_ids or ran an eager step since the last replay
 
@@ -389,12 +391,17 @@ class Llama:
         pos = np.asarray(positions, dtype=np.int64)
         if pos.max() >= cfg.max_context_len:
             raise ValueError("position beyond max_context_len")
-        bt = self.block_tables[:b].cpu().numpy()
-        slots = bt[np.arange(b), pos // cfg.block_size].astype(np.int64) * cfg.block_size + pos % cfg.block_size
-        self.input_ids[:b] = torch.tensor(np.asarray(token_ids, dtype=np.int32), device=self.device)
-        self.positions[:b] = torch.tensor(pos.astype(np.int32), device=self.device)
-        self.context_lens[:b] = torch.tensor((pos + 1).astype(np.int32), device=self.device)
-        self.slot_mapping[:b] = torch.tensor(slots, device=self.device)
+        if pos.min() < 0:
+            raise ValueError("negative position")
+        if b > cfg.max_batch:
+            raise ValueError(f"{b} sequences, the model was made for {cfg.max_batch}")
+        ids = np.ascontiguousarray(token_ids, dtype=np.int32)
+        pos = np.ascontiguousarray(np.broadcast_to(pos, (b,)), dtype=np.int32)
+        self._chk(self._L.mrs_set_state(ids.ctypes.data, pos.ctypes.data, b, self.input_ids.data_ptr(), self.positions.data_ptr(), self.context_lens.data_ptr(),
+                                        self.slot_mapping.data_ptr(), self.block_tables.data_ptr(), self.block_tables.shape[1], cfg.block_size, self._stream()))
+        # what replay() would read back, unless `positions` is written to in between (an inference tensor does not count its writes: read it back)
+        self._state_pos = None if self.positions.is_inference() else pos
+        self._state_version = None if self._state_pos is None else self.positions._version
         self._replays_left = None  # recomputed from the device state at the next replay()
         self._need_embed = True
 
@@ -420,6 +427,7 @@ class Llama:
     def decode_step(self, b: int = 1) -> None:
         self._set_mode()
         self._need_embed = True
+        self._state_pos = None  # the step advances the positions
         self._chk(self._L.mrs_llama_decode_step(self._h, b, self._stream()))
 
     def _chained_ok(self, b: int) -> bool:
@@ -470,10 +478,13 @@ class Llama:
         # the captured step advances device-side state; refuse to run it past the buffers it indexes (tokens_out, block table, RoPE tables)
         if self._replays_left is None:  # one read-back per set_state(): replays that stay inside the context window and the token buffer
             b = getattr(self, "_graph_batch", None) or self.positions.numel()  # only the sequences of the captured batch count (stale entries of earlier, larger batches do not)
-            self._replays_left = int(min(self.cfg.max_context_len - 1 - int(self.positions[:b].max().item()), self.tokens_out.shape[1] - int(self.step_counter.item())))
+            known = self._state_pos is not None and len(self._state_pos) >= b and self._state_version == self.positions._version
+            last = int(self._state_pos[:b].max()) if known else int(self.positions[:b].max().item())
+            self._replays_left = int(min(self.cfg.max_context_len - 1 - last, self.tokens_out.shape[1] - int(self.step_counter.item())))
         if self._replays_left <= 0:
             raise ValueError("replay(): the decode graph would run past max_new_tokens / max_context_len; set_state() to a new position first")
         self._replays_left -= 1
+        self._state_pos = None
         if self._graph_chained and self._need_embed:
             self._embed_state(self._graph_batch)  # eager, on the current stream, ahead of the graph: the chained step starts from embedding(input_ids)
             self._need_embed = False

@@ -508,3 +508,31 @@ def test_engine_mixtral_moe_vs_cpu_path_oracle(oracle, dev, request):
     from oracle import llama_ref
     cfg, w, m, cos, sin = _mk(oracle, dev, types, "bf16", experts=4)
     _vs_exact(m, cfg, w, cos, sin, "bf16", steps, "moe", check=steps >= 10, factor=1.1)  # 24 positions of a 4-expert toy: 1.046 x on the restatement
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("max_batch,b", [(1, 1), (8, 3), (8, 8)])
+def test_set_state_writes_the_decode_state(dev, max_batch, b):
+    """set_state(): ids, positions, context lengths and slots by the block table -- also a permuted one -- and nothing behind the b sequences; what it refuses."""
+    import torch
+    from mistralrs_amd.llama import Llama, LlamaConfig
+    cfg = LlamaConfig(hidden_size=256, intermediate_size=256, num_layers=1, num_heads=2, num_kv_heads=1, vocab_size=512, max_batch=max_batch, max_context_len=320)
+    m = Llama(cfg, dev, max_new_tokens=8)
+    rng = np.random.default_rng(b)
+    table = rng.permutation(m.block_tables.numel()).astype(np.int32).reshape(m.block_tables.shape)
+    m.block_tables.copy_(torch.from_numpy(table))
+    for t in (m.input_ids, m.positions, m.context_lens, m.slot_mapping):
+        t.fill_(-7)
+    ids, pos = rng.integers(0, 512, b).tolist(), rng.integers(0, 320, b)
+    pos[0] = 319
+    m.set_state(ids, pos.tolist())
+    assert m.input_ids[:b].tolist() == ids and m.positions[:b].tolist() == pos.tolist() and m.context_lens[:b].tolist() == (pos + 1).tolist()
+    assert m.slot_mapping[:b].tolist() == (table[np.arange(b), pos // 32].astype(np.int64) * 32 + pos % 32).tolist()
+    assert all((t[b:] == -7).all() for t in (m.input_ids, m.positions, m.context_lens, m.slot_mapping))
+    m.set_state(ids, [5])  # one position for all
+    assert m.positions[:b].tolist() == [5] * b
+    for bad in (320, -1):
+        with pytest.raises(ValueError):
+            m.set_state([1], [bad])
+    with pytest.raises(ValueError):
+        m.set_state([1] * (max_batch + 1), [0] * (max_batch + 1))
