@@ -9,19 +9,17 @@
 //     sl (q - 32) and sh (q - 32) with sc = 16 sh + sl, |.| <= 480 / 256.  The activation operand is the Q8_K quant as f16.  Every product and every partial
 //     sum of a superblock is an integer below 2^24, so the f32 accumulator of the matrix core holds the EXACT sum (tests/test_gemm_qi.py holds
 //     v_mfma_f32_32x32x16_f16 to that on adversarial operands); no per-sub-block scale multiply is left on the vector ALU;
-//   * Q4_K (gemm_qi_wide_kernel): the operand is sc (q - 8), the 8 sum_j sc_j bsum_j the offset leaves out and msum = sum_j m_j bsum_j are one more MFMA each per superblock
+//   * Q4_K: the operand is sc (q - 8), the 8 sum_j sc_j bsum_j the offset leaves out and msum = sum_j m_j bsum_j are one more MFMA each per superblock
 //     (K = the 16 run sums of the Q8_K block, scales / mins duplicated per run); (float)isum = X + 8 S is one rounding of the exact integer -- what (float)int gives;
-//   * Q5_K (round 5): the operand is sc (q - 16) (|.| <= 1008: one packed fma for sc q, one packed add for - 16 sc), two accumulators (<= 16.5 M each), and the
-//     16 sum_j sc_j bsum_j the offset leaves out is one more MFMA (S); isum = XA + XB + 16 S is formed in int32 (a superblock's sum reaches 64 M: two f32 additions
-//     would round twice) and converted once; the mins' M as for Q4_K;
+//   * Q5_K: the operand is sc (q - 16) (|.| <= 1008), two accumulators (<= 16.5 M each), and the 16 sum_j sc_j bsum_j the offset leaves out is one more MFMA (S);
+//     isum = XA + XB + 16 S is formed in int32 (a superblock's sum reaches 64 M: two f32 additions would round twice) and converted once; the mins' M as for Q4_K;
+//   * Q8_0: blocks of 32 int8 are one v_mfma_i32_32x32x32_i8 each, the block term in the engine's f32 expression;
 //   * per superblock and output ONE f32 term T (the decode engine's expression), terms added left to right inside each of the row's four runs of
 //     superblocks, the four run sums left to right (dec_core2.cuh header).
 // Operands: weights in an MFMA-order copy made at load time (mrs_gemm_qi_repack: per 32-row panel and superblock, every lane's 16 bytes of a piece
 // contiguous: one buffer_load_dwordx4 per lane and piece, straight into registers); activations from mrs_qi_quantize (engine-order RmsNorm + the candle
 // Q8_K quantizer of dec_core2.cuh, then f16 in the operand's k order, slab-major [superblock][token][256]).
-// Tiling (Q5_K, Q6_K; Q4_K: gemm_qi_wide_kernel below): workgroup 512 threads = 8 waves (two per SIMD: one wave's MFMAs run under the other's operand build and fix-up), tile 128 weight rows x 128
-// tokens, wave 32 x 64 = 1 x 2 MFMA tiles; per superblock the 128 tokens' f16 quants (64 KiB) are staged in LDS (16-byte chunks XOR-swizzled by the token
-// index: conflict-free ds_read_b128 fragments), double buffered: superblock s + 1 arrives by LDS-DMA (global_load_lds) while s is multiplied.
+// One kernel, gemm_qi_wide_kernel<type, token tiles of a wave>, multiplies all four types at all prompt lengths.
 #include "dec_core2.cuh"
 #include <stdio.h>
 #include <stdlib.h>
@@ -36,7 +34,8 @@ typedef _Float16 h2 __attribute__((ext_vector_type(2)));
 typedef _Float16 h8 __attribute__((ext_vector_type(8)));
 typedef float f16v __attribute__((ext_vector_type(16)));
 typedef float f32v __attribute__((ext_vector_type(32)));
-typedef float f2 __attribute__((ext_vector_type(2)));
+typedef int i4v __attribute__((ext_vector_type(4)));
+typedef int i16v __attribute__((ext_vector_type(16)));
 
 constexpr int REC_Q4K = 4096 + 512 + 128, REC_Q6K = 8192 + 512 + 128, REC_Q5K = REC_Q6K;  // Q5_K: the 5-bit values as bytes, like Q6_K's 6-bit ones
 __host__ __device__ constexpr int rec_bytes_qi(int type) { return type == T_Q4_K ? REC_Q4K : REC_Q6K; }
@@ -195,14 +194,6 @@ __global__ void __launch_bounds__(NT) qi_quantize_kernel(const QuantArgs a) {
 }
 
 // ------------------------------------------------------------------------------------------------ the GEMM
-struct GemmArgs {
-  const uint8_t *w; unsigned w_bytes; int type, N, K, T;
-  const _Float16 *qf; const float *yd; const _Float16 *bsf;
-  float *out; int ldo; int accumulate;  // out[t * ldo + n] (+)= row sum
-  float *part; int ksplit;              // ksplit = 4: workgroup z multiplies run z of the row's superblocks only and writes its sum to part[z][t][n]; the reduce kernel combines
-  const int *bounds; int experts;       // expert e multiplies the operand rows [bounds[e], bounds[e + 1]) by the weights at w + e * w_bytes (a grouped MoE prompt GEMM: the
-                                        // bounds come from launch_moe_dispatch on the device, the grid is sized for the worst case and tiles past it leave); nullptr = all T rows
-};
 // (expert, first row, end) of token tile yt of a launch over the experts' windows; false: past the last tile
 __device__ __forceinline__ bool expert_tile(const int *bounds, int experts, int tile, int &yt, int &e, int &tbeg, int &tend) {
   for (e = 0; e < experts; ++e) {
@@ -213,17 +204,6 @@ __device__ __forceinline__ bool expert_tile(const int *bounds, int experts, int 
   }
   return false;
 }
-constexpr int TN = 128, TT = 128;                   // workgroup tile: weight rows x tokens
-constexpr int GT = 512;                             // 8 waves: 4 (32-row panels) x 2 (64-token halves); two waves per SIMD overlap each other's MFMA and VALU phases
-constexpr int LDS_ACT = TT * 512, LDS_YD = TT * 4, LDS_BS = TT * 32;
-constexpr int LDS_BUF = LDS_ACT + LDS_YD + LDS_BS;  // one superblock of the tile's tokens; two buffers: the next superblock arrives by LDS-DMA during the MFMAs
-constexpr int LDS_TOTAL = 2 * LDS_BUF;
-
-// async global -> LDS copy, 16 / 4 bytes per lane: LDS destination = wave-uniform base + lane * size (the hardware's rule), source address per lane
-#ifndef MRS_GLDS16
-#define MRS_GLDS16(gptr, lbase) __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void *)(gptr), (__attribute__((address_space(3))) void *)(lbase), 16, 0, 0)
-#define MRS_GLDS4(gptr, lbase) __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void *)(gptr), (__attribute__((address_space(3))) void *)(lbase), 4, 0, 0)
-#endif
 #ifndef MRS_WAIT_VMCNT0
 #define MRS_WAIT_VMCNT0() asm volatile("s_waitcnt vmcnt(0)" ::: "memory")
 #endif
@@ -231,244 +211,22 @@ constexpr int LDS_TOTAL = 2 * LDS_BUF;
 __device__ __forceinline__ h2 as_h2(unsigned v) { return __builtin_bit_cast(h2, v); }
 __device__ __forceinline__ h8 mk_h8(h2 a, h2 b, h2 c, h2 d) { h8 r; r[0] = a[0]; r[1] = a[1]; r[2] = b[0]; r[3] = b[1]; r[4] = c[0]; r[5] = c[1]; r[6] = d[0]; r[7] = d[1]; return r; }
 __device__ __forceinline__ h2 pkfma(h2 x, h2 s, h2 c) { return __builtin_elementwise_fma(x, s, c); }
-// two bytes of a small unsigned integer -> (1024 + b0, 1024 + b1) as f16 (0x6400 = 1024: one unit per mantissa step up to 2047)
-__device__ __forceinline__ h2 magic(unsigned v, unsigned mask) { return as_h2((v & mask) | 0x64006400u); }
 
-template <int TYPE>
-__global__ void __launch_bounds__(GT) gemm_qi_kernel(const GemmArgs a) {
-  extern __shared__ __attribute__((aligned(16))) char smem[];
-  const int tid = tid_opaque(), lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int nn = lane & 31, hf = lane >> 5;
-  const int n0 = blockIdx.x * TN;
-  int tbeg = 0, tend = a.T, yt = blockIdx.y, ex = 0;
-  if (a.bounds && !expert_tile(a.bounds, a.experts, TT, yt, ex, tbeg, tend)) return;
-  const uint8_t *wbase = a.w + (size_t)ex * a.w_bytes;
-  const int t0 = tbeg + yt * TT;
-  if (t0 >= tend) return;  // workgroup-uniform
-  const int wn = wave & 3, wt = wave >> 2;  // the wave's 32-row panel / 64-token half of the tile
-  const int S = a.K / 256, Cs = (S + 3) / 4;
-  const __amdgpu_buffer_rsrc_t rw = __builtin_amdgcn_make_buffer_rsrc((void *)wbase, (short)0, (int)a.w_bytes, 0x00020000);
-  constexpr int REC = rec_bytes_qi(TYPE), NPC = 8;
-  struct WRegs { v4u q[NPC]; v4u hs; unsigned hd; };
-  const unsigned panel = (unsigned)((n0 + wn * 32) >> 5);
-  auto load_w = [&](WRegs &wr, int sb) {
-    const unsigned rec = (panel * (unsigned)S + (unsigned)sb) * (unsigned)REC;  // panels past N: out of range -> zeros
-#pragma unroll
-    for (int c = 0; c < NPC; ++c) wr.q[c] = __builtin_amdgcn_raw_buffer_load_b128(rw, rec + (unsigned)(c * 64 + lane) * 16u, 0, 0);
-    wr.hs = __builtin_amdgcn_raw_buffer_load_b128(rw, rec + (unsigned)(NPC * 1024) + (unsigned)nn * 16u, 0, 0);
-    wr.hd = __builtin_amdgcn_raw_buffer_load_b32(rw, rec + (unsigned)(NPC * 1024 + 512) + (unsigned)nn * 4u, 0, 0);
-  };
-  // stage superblock sb of the tile's tokens into buffer `buf` by LDS-DMA.  acts: 128 rows x 32 chunks of 16 B, chunk ch of row tr at position ch ^ (tr & 31);
-  // a DMA instruction fills 1 KiB = 2 rows lane by lane, so lane l of the instruction for rows (2 i, 2 i + 1) fetches chunk (l & 31) ^ (tr & 31) of row
-  // tr = 2 i + (l >> 5).  Rows past T re-read the last token (their outputs are never stored).
-  const int tlast = tend - 1 - t0;  // last existing row of the tile
-  auto stage = [&](int sb, int buf) {
-    char *base = smem + buf * LDS_BUF;
-    const char *gq = (const char *)a.qf + ((size_t)sb * a.T + t0) * 512;
-#pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      const int pair = wave * 8 + i;  // rows 2 pair, 2 pair + 1
-      const int tr = 2 * pair + hf, trc = min(tr, tlast);
-      MRS_GLDS16(gq + (size_t)trc * 512 + (((lane & 31) ^ (tr & 31)) << 4), base + pair * 1024);
-    }
-    if (wave < 2) {  // yd: 128 floats = 2 instructions of 64 x 4 B
-      const int tr = wave * 64 + lane;
-      MRS_GLDS4((const char *)a.yd + ((size_t)sb * a.T + t0 + min(tr, tlast)) * 4, base + LDS_ACT + wave * 256);
-    } else if (wave < 6) {  // run sums: 128 rows x 32 B = 4 instructions of 1 KiB
-      const int i = wave - 2, tr = i * 32 + (lane >> 1);
-      MRS_GLDS16((const char *)a.bsf + ((size_t)sb * a.T + t0 + min(tr, tlast)) * 32 + (lane & 1) * 16, base + LDS_ACT + LDS_YD + i * 1024);
-    }
-  };
-  f16v run[2], pend[2];
-#pragma unroll
-  for (int tt = 0; tt < 2; ++tt)
-#pragma unroll
-    for (int v = 0; v < 16; ++v) { run[tt][v] = 0.f; pend[tt][v] = 0.f; }
-  WRegs wr, wnx;
-  const int sb_first = a.ksplit > 1 ? (int)blockIdx.z * ((a.K / 256 + 3) / 4) : 0;
-  if (sb_first < a.K / 256) { load_w(wr, sb_first); stage(sb_first, sb_first & 1); }
-  const int trow = wt * 64 + nn;  // + 32 tt: the token row whose fragment this lane supplies
-  // fragment of run r for this lane: chunk (2 r + hf) ^ (row & 31) of its token row; row & 31 == nn for both token tiles, so the 16 offsets are computed once
-  int aoff[16];
-#pragma unroll
-  for (int r = 0; r < 16; ++r) aoff[r] = trow * 512 + (((2 * r + hf) ^ nn) << 4);
-  const int sb_begin = a.ksplit > 1 ? (int)blockIdx.z * Cs : 0, sb_end = a.ksplit > 1 ? min(S, sb_begin + Cs) : S;
-  if (sb_begin >= sb_end) {
-    if (a.ksplit > 1) {  // a run without superblocks contributes +0
-      const int n = n0 + wn * 32 + nn;
-#pragma unroll
-      for (int tt = 0; tt < 2; ++tt)
-#pragma unroll
-        for (int v = 0; v < 16; ++v) {
-          const int t = t0 + wt * 64 + tt * 32 + 8 * (v >> 2) + 4 * hf + (v & 3);
-          if (n < a.N && t < tend) a.part[((size_t)blockIdx.z * a.T + t) * a.N + n] = 0.f;
-        }
-    }
-    return;
-  }
-  for (int sb = sb_begin; sb < sb_end; ++sb) {
-    const int buf = sb & 1;
-    MRS_WAIT_VMCNT0();  // this wave's DMA pieces of superblock sb (and the weights of sb) have landed
-    __syncthreads();    // everyone's have, and every wave has finished reading the other buffer
-    if (sb + 1 < sb_end) { stage(sb + 1, buf ^ 1); load_w(wnx, sb + 1); }
-    const char *act_s = smem + buf * LDS_BUF;
-    const float *yd_s = (const float *)(act_s + LDS_ACT);
-    const char *bs_s = act_s + LDS_ACT + LDS_YD;
-    f16v X[2], X2[2];
-#pragma unroll
-    for (int tt = 0; tt < 2; ++tt)
-#pragma unroll
-      for (int v = 0; v < 16; ++v) { X[tt][v] = 0.f; X2[tt][v] = 0.f; }
-    // Q5_K: the 16 fragment offsets are recomputed per superblock from an opaque copy of the lane's row (kept as loop invariants -- aoff[] -- they are what tips this
-    // branch over 256 registers: 6 spilled dwords)
-    constexpr bool RECOMP = TYPE == T_Q5_K;
-    int nnv = nn;
-    if constexpr (RECOMP) MRS_OPAQUE_TID(nnv);
-    auto act_frag = [&](int tt, int run_i) -> h8 {
-      if constexpr (RECOMP) return *(const h8 *)(act_s + trow * 512 + (((2 * run_i + hf) ^ nnv) << 4) + tt * (32 * 512));
-      else return *(const h8 *)(act_s + aoff[run_i] + tt * (32 * 512));
-    };
-    const bool cfirst = (sb % Cs) == 0;
-    const f2 keep2 = cfirst ? f2{0.f, 0.f} : f2{1.f, 1.f};  // the first term of a run of superblocks starts its sum (0 * run + t), the others add (1 * run + t: exact)
-    if constexpr (TYPE == T_Q5_K) {
-      // operand = sc (q - 16), |.| <= 1008: (1024 + q) sc - 1024 sc = sc q exactly (one packed fma; 1024 sc <= 64512 is an f16 value), then - 16 sc (1040 sc is not an
-      // f16 value for sc = 63, so the offset takes a second packed add).  Runs 0 .. 7 and 8 .. 15 go to two accumulators (<= 128 x 1008 x 128 = 16.5 M < 2^24 each,
-      // exact); the 16 sc_j bsum terms the offset leaves out are one more MFMA (S, like the mins' M); isum = XA + XB + 16 S is added as int32 and converted once --
-      // what the CPU path's (float)int is.
-      unsigned mg = 0x64006400u;
-      MRS_OPAQUE_TID(mg);
-      auto b2 = [&](unsigned v) -> h2 { return as_h2((v & 0x00FF00FFu) | mg); };  // (1024 + u0, 1024 + u1)
-#pragma unroll
-      for (int g = 0; g < 8; ++g) {
-        const float scf = (float)byte_of(g < 4 ? wr.hs.x : wr.hs.y, g & 3);
-        const h2 sc = h2{(_Float16)scf, (_Float16)scf}, off = h2{(_Float16)(-1024.0f * scf), (_Float16)(-1024.0f * scf)}, o16 = h2{(_Float16)(-16.0f * scf), (_Float16)(-16.0f * scf)};
-        auto opnd = [&](unsigned v) -> h2 { return pkfma(b2(v), sc, off) + o16; };
-#pragma unroll
-        for (int h = 0; h < 2; ++h) {  // run 2 g + h
-          const unsigned d0 = h == 0 ? wr.q[g].x : wr.q[g].z, d1 = h == 0 ? wr.q[g].y : wr.q[g].w;
-          const h8 w = mk_h8(opnd(d0), opnd(d0 >> 8), opnd(d1), opnd(d1 >> 8));
-#pragma unroll
-          for (int tt = 0; tt < 2; ++tt) {
-            const h8 af = act_frag(tt, 2 * g + h);
-            if (g < 4) X[tt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(af, w, X[tt], 0, 0, 0);
-            else X2[tt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(af, w, X2[tt], 0, 0, 0);
-          }
-        }
-      }
-      // M = sum_run m_{run / 2} bsum_run, S = sum_run sc_{run / 2} bsum_run: operand slot (hf, jj) <-> run 8 hf + jj -> sub-block 4 hf + jj / 2
-      const unsigned mw = hf ? wr.hs.w : wr.hs.z, sw = hf ? wr.hs.y : wr.hs.x;
-      h8 wm, ws;
-#pragma unroll
-      for (int k = 0; k < 4; ++k) {
-        const _Float16 mk = (_Float16)(float)byte_of(mw, k), sk = (_Float16)(float)byte_of(sw, k);
-        wm[2 * k] = mk; wm[2 * k + 1] = mk; ws[2 * k] = sk; ws[2 * k + 1] = sk;
-      }
-      const float d = half_bits_to_float((uint16_t)(wr.hd & 0xffff)), dmin = half_bits_to_float((uint16_t)(wr.hd >> 16));
-#pragma unroll
-      for (int tt = 0; tt < 2; ++tt) {
-        const h8 bsf = *(const h8 *)(bs_s + (trow + 32 * tt) * 32 + hf * 16);
-        f16v zero;
-#pragma unroll
-        for (int v = 0; v < 16; ++v) zero[v] = 0.f;
-        const f16v M = __builtin_amdgcn_mfma_f32_32x32x16_f16(bsf, wm, zero, 0, 0, 0);
-        const f16v Sx = __builtin_amdgcn_mfma_f32_32x32x16_f16(bsf, ws, zero, 0, 0, 0);
-#pragma unroll
-        for (int q4 = 0; q4 < 4; ++q4) {
-          const float4 y4 = *(const float4 *)(yd_s + wt * 64 + tt * 32 + 8 * q4 + 4 * hf);
-#pragma unroll
-          for (int k = 0; k < 4; k += 2) {
-            const int v = 4 * q4 + k;
-            const f2 yd2 = k == 0 ? f2{y4.x, y4.y} : f2{y4.z, y4.w};
-            const int i0 = ((int)X[tt][v] + (int)X2[tt][v]) + 16 * (int)Sx[v], i1 = ((int)X[tt][v + 1] + (int)X2[tt][v + 1]) + 16 * (int)Sx[v + 1];
-            const f2 If = f2{(float)i0, (float)i1};  // (float)isum
-            const f2 mm = (f2{dmin, dmin} * yd2) * f2{M[v], M[v + 1]};
-            const f2 t = __builtin_elementwise_fma(f2{d, d} * yd2, If, -mm);
-            const f2 r = __builtin_elementwise_fma(f2{run[tt][v], run[tt][v + 1]}, keep2, t);
-            run[tt][v] = r[0]; run[tt][v + 1] = r[1];
-          }
-        }
-      }
-    } else {  // Q6_K
-      unsigned mg = 0x64006400u;
-      MRS_OPAQUE_TID(mg);
-      auto b2 = [&](unsigned v) -> h2 { return as_h2((v & 0x00FF00FFu) | mg); };  // (1024 + u0, 1024 + u1)
-#pragma unroll
-      for (int g = 0; g < 8; ++g) {
-#pragma unroll
-        for (int h = 0; h < 2; ++h) {  // run 2 g + h
-          const unsigned d0 = h == 0 ? wr.q[g].x : wr.q[g].z, d1 = h == 0 ? wr.q[g].y : wr.q[g].w;
-          const int r = 2 * g + h;
-          const unsigned scw = r < 4 ? wr.hs.x : r < 8 ? wr.hs.y : r < 12 ? wr.hs.z : wr.hs.w;
-          const int sc = sbyte_of(scw, r & 3), sli = sc & 15, shi = sc >> 4;  // sc = 16 shi + sli
-          const float slf = (float)sli, shf = (float)shi;
-          // (1024 + u) s - 1056 s = (u - 32) s = (q - 32) s in one fma: 1056 s is an f16 value for |s| <= 15 (a multiple of 8 below 16384)
-          const h2 sl = h2{(_Float16)slf, (_Float16)slf}, sh = h2{(_Float16)shf, (_Float16)shf};
-          const h2 ol = h2{(_Float16)(-1056.0f * slf), (_Float16)(-1056.0f * slf)}, oh = h2{(_Float16)(-1056.0f * shf), (_Float16)(-1056.0f * shf)};
-          const h2 p0 = b2(d0), p1 = b2(d0 >> 8), p2 = b2(d1), p3 = b2(d1 >> 8);
-          const h8 wl = mk_h8(pkfma(p0, sl, ol), pkfma(p1, sl, ol), pkfma(p2, sl, ol), pkfma(p3, sl, ol));
-          const h8 wh = mk_h8(pkfma(p0, sh, oh), pkfma(p1, sh, oh), pkfma(p2, sh, oh), pkfma(p3, sh, oh));
-#pragma unroll
-          for (int tt = 0; tt < 2; ++tt) {
-            const h8 af = act_frag(tt, r);
-            X[tt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(af, wl, X[tt], 0, 0, 0);
-            X2[tt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(af, wh, X2[tt], 0, 0, 0);
-          }
-        }
-      }
-      const float d = half_bits_to_float((uint16_t)(wr.hd & 0xffff));
-#pragma unroll
-      for (int tt = 0; tt < 2; ++tt)
-#pragma unroll
-        for (int q4 = 0; q4 < 4; ++q4) {
-          const float4 y4 = *(const float4 *)(yd_s + wt * 64 + tt * 32 + 8 * q4 + 4 * hf);
-#pragma unroll
-          for (int k = 0; k < 4; k += 2) {
-            const int v = 4 * q4 + k;
-            const f2 yd2 = k == 0 ? f2{y4.x, y4.y} : f2{y4.z, y4.w};
-            const f2 If = __builtin_elementwise_fma(f2{16.0f, 16.0f}, f2{X2[tt][v], X2[tt][v + 1]}, f2{X[tt][v], X[tt][v + 1]});  // (float)isum
-            const f2 t = (f2{d, d} * yd2) * If;
-            const f2 r = __builtin_elementwise_fma(f2{run[tt][v], run[tt][v + 1]}, keep2, t);
-            run[tt][v] = r[0]; run[tt][v + 1] = r[1];
-          }
-        }
-    }
-    if ((sb + 1) % Cs == 0 || sb + 1 == sb_end) {  // a run of superblocks ends: its sum joins the row's left-to-right combination
-      const bool first = sb < Cs;
-#pragma unroll
-      for (int tt = 0; tt < 2; ++tt)
-#pragma unroll
-        for (int v = 0; v < 16; ++v) pend[tt][v] = first ? run[tt][v] : pend[tt][v] + run[tt][v];
-    }
-    if (sb + 1 < sb_end) wr = wnx;
-  }
-  // store: lane holds column n, rows t = 8 (v / 4) + 4 hf + v % 4 of each MFMA tile
-  const int n = n0 + wn * 32 + nn;
-#pragma unroll
-  for (int tt = 0; tt < 2; ++tt)
-#pragma unroll
-    for (int v = 0; v < 16; ++v) {
-      const int t = t0 + wt * 64 + tt * 32 + 8 * (v >> 2) + 4 * hf + (v & 3);
-      if (n < a.N && t < tend) {
-        if (a.ksplit > 1) a.part[((size_t)blockIdx.z * a.T + t) * a.N + n] = run[tt][v];  // one run per workgroup: its sum, combined by gemm_qi_reduce_kernel
-        else {
-          float *o = a.out + (size_t)t * a.ldo + n;
-          *o = a.accumulate ? *o + pend[tt][v] : pend[tt][v];
-        }
-      }
-    }
-}
-
-// ------------------------------------------------------------------------------------------------ Q4_K, all prompt lengths
+// ------------------------------------------------------------------------------------------------ the kernel
 // What bounds this product is the vector ALU beside the matrix cores: building a run's f16 operand costs ~12 instructions per 32 weight rows, the f32 term 4 per output and
 // superblock, one matrix instruction covers 1024 outputs x 16 values and hides about five of them (measured: 4.3 cycles per vector, ~9 issue cycles per matrix instruction
 // of a SIMD, 32 cycles of matrix pipe; at full matrix rate the card also drops to ~1.5 GHz).  So:
-//   * the operand is sc (q - 8), |.| <= 504: a superblock's sum stays below 504 x 128 x 256 = 16.5 M < 2^24, ONE exact accumulator; the 8 sum_j sc_j bsum_j that the
+//   * Q4_K's operand is sc (q - 8), |.| <= 504: a superblock's sum stays below 504 x 128 x 256 = 16.5 M < 2^24, ONE exact accumulator; the 8 sum_j sc_j bsum_j that the
 //     offset leaves out are a matrix instruction over the run sums (S, like the mins' M), and isum = X + 8 S is one rounding of the exact integer: fma(8, S, X);
-//   * nibbles go to bits 7:4 of a half-word: 64 + q is one v_and_or (0x5400 = 64, 1/16 per mantissa step), sc (q - 8) = (64 + q) sc - 72 sc exactly (9 sc < 2^11);
+//   * its nibbles go to bits 7:4 of a half-word: 64 + q is one v_and_or (0x5400 = 64, 1/16 per mantissa step), sc (q - 8) = (64 + q) sc - 72 sc exactly (9 sc < 2^11);
 //   * d yd and dmin yd of a tile are one v_mfma_f32_32x32x1_2b (two outer products, each rounded once) instead of 32 multiplies;
 //   * reads, operand build and the next superblock's LDS-DMA stand one by one behind the matrix instructions of the step before; small workgroups (4 waves, 32 weight rows
 //     each, NT token tiles) leave two (NT = 2) or three (NT = 1) workgroups per CU, so that one's barriers and latencies run under another's arithmetic;
 //   * the projections that share their input are segments of ONE launch, the experts of a sparse-MoE prompt (windows of the expert-sorted rows) token tiles of one launch.
+//   * Q6_K takes two matrix instructions per run (sl, sh), so its vector work hides better under them; Q8_0's bound is the four f32 instructions per output and block that the
+//     engine's order of terms asks for.
+// Against 512-thread workgroups of 128 x 128 tiles (one per CU, their phases in lockstep), 4096 x 14336 (down) and 2 x 14336 x 4096 (gate / up) weights:
+//   Q6_K  down  512 tokens 170 -> 129 us, 1999 tokens 628 -> 457;   Q8_0  gate / up  700 tokens 402 -> 348, q / k / v 700 tokens three launches -> one of 95 us.
 // NT = 4 (128 tokens per wave, the operand built once per four matrix instructions) needs 255 registers and the earlier runs' sums in memory: 343 us against 199 us for
 // 28672 x 4096 x 512 tokens.
 struct QiSeg { const uint8_t *w; unsigned w_bytes; int N; float *out; int ldo; };
@@ -477,22 +235,26 @@ struct WideArgs {
   int K, T;
   const _Float16 *qf; const float *yd; const _Float16 *bsf;
   int accumulate, ksplit; float *part; int part_n;  // ksplit = 4: workgroup z multiplies run z only, plane z of part [4][T][part_n] takes its sums
-  const int *bounds; int experts;                   // as in GemmArgs
+  const int *bounds; int experts;       // expert e multiplies the operand rows [bounds[e], bounds[e + 1]) by the weights at w + e * w_bytes (a grouped MoE prompt GEMM: the
+                                        // bounds come from launch_moe_dispatch on the device, the grid is sized for the worst case and tiles past it leave); nullptr = all T rows
 };
-template <int NT> constexpr int wide_meta = 512 + NT * 32 * 32;     // block scales [32 NT] f32, run sums [32 NT][16] f16
-template <int NT> constexpr int wide_buf = NT * 32 * 512 + wide_meta<NT>;  // + quants; two buffers, each a multiple of 512 (the fragments' exclusive or)
+// LDS of a superblock of a workgroup's tokens, two buffers: K-quants: f16 quants [32 NT][512], block scales [32 NT] f32 (512 bytes), run sums [32 NT][16] f16;  Q8_0: int8
+// quants [32 NT][256], scales [8 blocks][32 NT] f32.  A buffer is a multiple of a token's row (the fragments' exclusive or)
+template <int TYPE> constexpr int wide_row = TYPE == T_Q8_0 ? 256 : 512;
+template <int TYPE, int NT> constexpr int wide_buf = NT * 32 * wide_row<TYPE> + (TYPE == T_Q8_0 ? 0 : 512) + NT * 32 * 32;
 constexpr int WIDE_ROWS = 128;                                                      // weight rows of a workgroup: four waves
 #ifndef MRS_BLDS16
 // buffer load to LDS, 16 / 4 bytes per lane: LDS destination = wave-uniform base + lane * size
 #define MRS_BLDS16(rsrc, lbase, voff) __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, (__attribute__((address_space(3))) void *)(lbase), 16, voff, 0, 0, 0)
 #define MRS_BLDS4(rsrc, lbase, voff) __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, (__attribute__((address_space(3))) void *)(lbase), 4, voff, 0, 0, 0)
 #define MRS_LDS_BASE(p) ((unsigned)(size_t)(__attribute__((address_space(3))) char *)(p))
-#define MRS_LDS_H8(p, addr, off) (*(const __attribute__((address_space(3))) h8 *)(size_t)((addr) + (off)))
+#define MRS_LDS_FRAG(type, p, addr, off) (*(const __attribute__((address_space(3))) type *)(size_t)((addr) + (off)))
 #endif
-template <int NT>
-__global__ void __launch_bounds__(256, NT == 1 ? 3 : 2) gemm_qi_wide_kernel(const WideArgs a) {
+template <int TYPE, int NT>
+__global__ void __launch_bounds__(256, NT == 1 && TYPE != T_Q5_K ? 3 : 2) gemm_qi_wide_kernel(const WideArgs a) {
   extern __shared__ __attribute__((aligned(16))) char smem[];
-  constexpr int TT_ = NT * 32, ACT_ = TT_ * 512, YD_ = wide_meta<NT> - TT_ * 32;
+  constexpr int TT_ = NT * 32, ROWB = wide_row<TYPE>, ACT_ = TT_ * ROWB, BUF_ = wide_buf<TYPE, NT>, YD_ = 512;
+  constexpr int NPC = TYPE == T_Q4_K ? 4 : 8;  // 1-KiB pieces of a record
   const int tid = tid_opaque(), lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int nn = lane & 31, hf = lane >> 5;
   const int bx = blockIdx.x, seg = bx >= a.x2 ? 2 : bx >= a.x1 ? 1 : 0;
@@ -506,26 +268,35 @@ __global__ void __launch_bounds__(256, NT == 1 ? 3 : 2) gemm_qi_wide_kernel(cons
   const int S = a.K / 256, Cs = (S + 3) / 4;
   const __amdgpu_buffer_rsrc_t rw = __builtin_amdgcn_make_buffer_rsrc((void *)wbase, (short)0, (int)sg.w_bytes, 0x00020000);
   const unsigned panel = (unsigned)((bx - (seg == 2 ? a.x2 : seg == 1 ? a.x1 : 0)) * 4 + wave);
-  // six loads per superblock: a piece of the next one is requested when this one's has been multiplied (panels past N, superblocks past the end: out of range -> zeros)
-  auto rec_of = [&](int sb) { return (panel * (unsigned)S + (unsigned)sb) * (unsigned)REC_Q4K; };
+  // a piece of the next superblock is requested when this one's has been multiplied (panels past N, superblocks past the end: out of range -> zeros)
+  auto rec_of = [&](int sb) { return (panel * (unsigned)S + (unsigned)sb) * (unsigned)rec_bytes_qi(TYPE); };
   auto load_q = [&](unsigned rec, int c) { return __builtin_amdgcn_raw_buffer_load_b128(rw, rec + (unsigned)(c * 64 + lane) * 16u, 0, 0); };
-  auto load_hs = [&](unsigned rec) { return __builtin_amdgcn_raw_buffer_load_b128(rw, rec + 4096u + (unsigned)nn * 16u, 0, 0); };
-  auto load_hd = [&](unsigned rec) { return __builtin_amdgcn_raw_buffer_load_b32(rw, rec + 4608u + (unsigned)nn * 4u, 0, 0); };
-  // LDS-DMA of superblock sb's rows (8 NT per wave), as in gemm_qi_kernel: chunk ch of row tr at position ch ^ (tr & 31).  Rows past the window hold
-  // whatever follows it in the operand buffer (their outputs are not stored), rows past the buffer zeros.  it = sb - sb_begin
-  const __amdgpu_buffer_rsrc_t rq = __builtin_amdgcn_make_buffer_rsrc((void *)a.qf, (short)0, (int)((size_t)S * a.T * 512), 0x00020000);
+  auto load_hs = [&](unsigned rec) { return __builtin_amdgcn_raw_buffer_load_b128(rw, rec + (unsigned)(NPC * 1024) + (unsigned)nn * 16u, 0, 0); };
+  auto load_hd = [&](unsigned rec) { return __builtin_amdgcn_raw_buffer_load_b32(rw, rec + (unsigned)(NPC * 1024 + 512) + (unsigned)nn * 4u, 0, 0); };
+  // LDS-DMA of superblock sb's rows (8 NT per wave): 16-byte chunk ch of row tr at position ch ^ (tr % chunks of a row), so that the fragments' reads hit every bank.  An
+  // instruction fills 1 KiB = RPI rows.  Rows past the window hold whatever follows it in the operand buffer (their outputs are not stored), rows past the buffer zeros.
+  // it = sb - sb_begin
+  constexpr int CPR = ROWB / 16, RPI = 1024 / ROWB, NSTAGE = 8 * NT / RPI;
+  const __amdgpu_buffer_rsrc_t rq = __builtin_amdgcn_make_buffer_rsrc((void *)a.qf, (short)0, (int)((size_t)S * a.T * ROWB), 0x00020000);
   const __amdgpu_buffer_rsrc_t ry = __builtin_amdgcn_make_buffer_rsrc((void *)a.yd, (short)0, (int)((size_t)S * a.T * 4), 0x00020000);
   const __amdgpu_buffer_rsrc_t rb = __builtin_amdgcn_make_buffer_rsrc((void *)a.bsf, (short)0, (int)((size_t)S * a.T * 32), 0x00020000);
-  const unsigned dma_row = (unsigned)(hf * 512), dma_ch = (unsigned)((lane & 31) ^ hf) << 4;
-  auto stage_q = [&](int sb, int it, int i) {  // rows 2 i, 2 i + 1 of the wave's 8 NT: 1 KiB
-    MRS_BLDS16(rq, smem + (it & 1) * wide_buf<NT> + (wave * 4 * NT + i) * 1024, dma_row + (dma_ch ^ (unsigned)(((wave * 8 * NT + 2 * i) & 31) << 4)) +
-               ((unsigned)sb * (unsigned)a.T + (unsigned)(t0 + wave * 8 * NT + 2 * i)) * 512u);
+  const unsigned dma_row = (unsigned)(lane / CPR * ROWB), dma_ch = (unsigned)((lane % CPR) ^ (lane / CPR)) << 4;
+  constexpr unsigned DEAD = 0xF0000000u;  // past every buffer: a request that is only there to keep the code without branches (they let hipcc move matrix instructions together)
+  auto stage_q = [&](int sb, int it, int i, bool live = true) {  // rows RPI i .. of the wave's 8 NT
+    const int row = wave * 8 * NT + RPI * i;
+    MRS_BLDS16(rq, smem + (it & 1) * BUF_ + row * ROWB, dma_row + (dma_ch ^ (unsigned)((row % CPR) << 4)) + (live ? ((unsigned)sb * (unsigned)a.T + (unsigned)(t0 + row)) * (unsigned)ROWB : DEAD));
   };
-  auto stage_meta = [&](int sb, int it) {
-    char *meta = smem + (it & 1) * wide_buf<NT> + ACT_;
-    const unsigned row = (unsigned)sb * (unsigned)a.T + (unsigned)t0;
-    if (wave < (NT + 1) / 2 && (NT > 1 || lane < 32)) MRS_BLDS4(ry, meta + wave * 256, (row + (unsigned)(wave * 64 + lane)) * 4u);
-    if (wave < NT) MRS_BLDS16(rb, meta + YD_ + wave * 1024, (row + (unsigned)wave * 32u) * 32u + (unsigned)lane * 16u);
+  auto stage_meta = [&](int sb, int it, bool live = true) {
+    char *meta = smem + (it & 1) * BUF_ + ACT_;
+    if constexpr (TYPE == T_Q8_0) {
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+        if (NT > 1 || lane < 32) MRS_BLDS4(rb, meta + (2 * wave + i) * TT_ * 4, live ? (((unsigned)sb * 8u + (unsigned)(2 * wave + i)) * (unsigned)a.T + (unsigned)(t0 + lane)) * 4u : DEAD);
+    } else {
+      const unsigned row = (unsigned)sb * (unsigned)a.T + (unsigned)t0;
+      if (wave < (NT + 1) / 2 && (NT > 1 || lane < 32)) MRS_BLDS4(ry, meta + wave * 256, live ? (row + (unsigned)(wave * 64 + lane)) * 4u : DEAD);
+      if (wave < NT) MRS_BLDS16(rb, meta + YD_ + wave * 1024, live ? (row + (unsigned)wave * 32u) * 32u + (unsigned)lane * 16u : DEAD);
+    }
   };
   const int n = (int)panel * 32 + nn;
   float run[NT][16], pend[NT][16];
@@ -552,51 +323,123 @@ __global__ void __launch_bounds__(256, NT == 1 ? 3 : 2) gemm_qi_wide_kernel(cons
     return;
   }
 #pragma unroll
-  for (int i = 0; i < 4 * NT; ++i) stage_q(sb_begin, 0, i);
+  for (int i = 0; i < NSTAGE; ++i) stage_q(sb_begin, 0, i);
   stage_meta(sb_begin, 0);
-  v4u wq[4], hs_next;
+  v4u wq[NPC], hs_next;
   unsigned hd_next;
 #pragma unroll
-  for (int c = 0; c < 4; ++c) wq[c] = load_q(rec_of(sb_begin), c);
+  for (int c = 0; c < NPC; ++c) wq[c] = load_q(rec_of(sb_begin), c);
   hs_next = load_hs(rec_of(sb_begin)); hd_next = load_hd(rec_of(sb_begin));
   const f16v zero = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-  unsigned mg = 0x54005400u;
+  unsigned mg = TYPE == T_Q6_K ? 0x64006400u : 0x54005400u;
   MRS_OPAQUE_TID(mg);  // keeps the constant in a VGPR: v_and_or_b32 takes one literal
-  auto nib = [&](unsigned v) -> h2 { return as_h2((v & 0x00F000F0u) | mg); };  // 64 + the nibbles at bits 7:4 of the half-words
   for (int sb = sb_begin; sb < sb_end; ++sb) {
     const int it = sb - sb_begin;
     const bool more = sb + 1 < sb_end;
     const v4u hs = hs_next;
-    const unsigned hd = hd_next, rec_next = more ? rec_of(sb + 1) : 0xF0000000u;
-    h2 sc2[2], of2[2];  // scale of the low / high nibbles' sub-block, - 72 times it
-    auto scales = [&](int c, int hi) {
-      const float f = (float)byte_of(c < 2 ? hs.x : hs.y, 2 * (c & 1) + hi);
-      sc2[hi] = __builtin_bit_cast(h2, __builtin_amdgcn_cvt_pkrtz(f, f));  // an integer below 64: exact
-      of2[hi] = sc2[hi] * h2{(_Float16)-72.0f, (_Float16)-72.0f};
-    };
-    // step k = run 4 c + h (low nibbles) or 4 c + 2 + h (high nibbles) of piece c, in the order (c, h, hi)
-    auto run_of = [](int k) { return 4 * (k >> 2) + 2 * (k & 1) + ((k >> 1) & 1); };
-    auto pair_of = [&](int k, int p) -> h2 {  // operand slots 2 p, 2 p + 1
-      const int c = k >> 2, h = (k >> 1) & 1, hi = k & 1;
-      const unsigned d = h == 0 ? (p < 2 ? wq[c].x : wq[c].y) : (p < 2 ? wq[c].z : wq[c].w);
-      return pkfma(nib(hi ? ((p & 1) ? d >> 8 : d) : ((p & 1) ? d >> 4 : d << 4)), sc2[hi], of2[hi]);
-    };
-    h8 fr[2][NT];
-    h2 w[2][4];
-    scales(0, 0); scales(0, 1);
+    const unsigned hd = hd_next, rec_next = more ? rec_of(sb + 1) : DEAD;
+    const char *meta_s = smem + (it & 1) * BUF_ + ACT_;
+    unsigned abase = MRS_LDS_BASE(smem) + (unsigned)((it & 1) * BUF_ + nn * ROWB + (((nn % CPR) ^ hf) << 4));
+    MRS_OPAQUE_TID(abase);  // one register: a fragment's offset is one exclusive or on it
+    if constexpr (TYPE == T_Q8_0) {
+      // one v_mfma_i32_32x32x32_i8 IS one block of 32 tokens x 32 rows (int32: exact); p_b = ((float)isum_b dw_b) dx_b, T = p_0 + .. + p_7 left to right: four vector
+      // instructions per output and block, which is what bounds this format
+      MRS_WAIT_VMCNT0();
+      __syncthreads();
+      stage_meta(sb + 1, it + 1, more);
+      auto frag8 = [&](int b, int tt) -> i4v { return MRS_LDS_FRAG(i4v, smem, abase ^ (unsigned)(32 * b), tt * (32 * ROWB)); };
+      const i16v izero = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
+      i4v af[2][NT];
+      float Tt[NT][16];
 #pragma unroll
-    for (int p = 0; p < 4; ++p) w[0][p] = pair_of(0, p);
+      for (int tt = 0; tt < NT; ++tt) af[0][tt] = frag8(0, tt);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int b = 0; b < 8; ++b) {
+        i16v is[NT];
+        if (b + 1 < 8) {
+#pragma unroll
+          for (int tt = 0; tt < NT; ++tt) af[(b + 1) & 1][tt] = frag8(b + 1, tt);
+        }
+#pragma unroll
+        for (int tt = 0; tt < NT; ++tt) is[tt] = __builtin_amdgcn_mfma_i32_32x32x32_i8(af[b & 1][tt], __builtin_bit_cast(i4v, wq[b]), izero, 0, 0, 0);
+        wq[b] = load_q(rec_next, b);
+        if (b < NSTAGE) stage_q(sb + 1, it + 1, b, more);
+        const unsigned hw = b < 2 ? hs.x : b < 4 ? hs.y : b < 6 ? hs.z : hs.w;
+        const float dwb = half_bits_to_float((uint16_t)((b & 1) ? (hw >> 16) : (hw & 0xffffu)));
+#pragma unroll
+        for (int tt = 0; tt < NT; ++tt) {
+          __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+          for (int q4 = 0; q4 < 4; ++q4) {
+            const float4 y4 = *(const float4 *)(meta_s + (b * TT_ + tt * 32 + 8 * q4 + 4 * hf) * 4);
+            const float yy[4] = {y4.x, y4.y, y4.z, y4.w};
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+              const int v = 4 * q4 + k;
+              const float p = ((float)is[tt][v] * dwb) * yy[k];
+              Tt[tt][v] = b == 0 ? p : Tt[tt][v] + p;
+            }
+          }
+        }
+        __builtin_amdgcn_sched_barrier(0);  // one block at a time: more results in flight do not fit the registers
+      }
+      hs_next = load_hs(rec_next);
+#pragma unroll
+      for (int tt = 0; tt < NT; ++tt)
+#pragma unroll
+        for (int v = 0; v < 16; ++v) run[tt][v] = (sb % Cs) == 0 ? Tt[tt][v] : run[tt][v] + Tt[tt][v];
+    } else {
+    // ---- the weight operand of a run (16 values of 32 rows x 16 / 8 of the K order per lane) as exact small integers in f16, from packed integer and f16 instructions:
+    //   Q4_K  sc (q - 8) = (64 + q) sc - 72 sc      (q at bits 7:4 of a half-word: 0x5400 = 64, one unit per 16 mantissa steps; 9 sc < 2^11)
+    //   Q5_K  sc (q - 16) = (64 + q) sc - 80 sc     (q at bits 8:4)
+    //   Q6_K  sl (q - 32), sh (q - 32) with sc = 16 sh + sl: (1024 + u) s - 1056 s (0x6400 = 1024, one unit per mantissa step; 1056 s is an f16 value for |s| <= 15)
+    h2 sc2[2], of2[2];  // Q4_K: of the low / high nibbles' sub-block;  Q5_K: [0];  Q6_K: sl, sh
+    auto scales = [&](int k) {  // of step k and, where they share one, the steps behind it
+      auto put = [&](int i, float f, float c) {
+        sc2[i] = __builtin_bit_cast(h2, __builtin_amdgcn_cvt_pkrtz(f, f));  // a small integer: exact
+        of2[i] = sc2[i] * h2{(_Float16)c, (_Float16)c};
+      };
+      if constexpr (TYPE == T_Q4_K) {
+        if ((k & 3) < 2) { const int c = k >> 2, hi = k & 1; put(hi, (float)byte_of(c < 2 ? hs.x : hs.y, 2 * (c & 1) + hi), -72.0f); }  // the high nibbles' first step comes one later
+      } else if constexpr (TYPE == T_Q5_K) {
+        if ((k & 1) == 0) { const int g = k >> 1; put(0, (float)byte_of(g < 4 ? hs.x : hs.y, g & 3), -80.0f); }
+      } else {
+        const int sc = sbyte_of(k < 4 ? hs.x : k < 8 ? hs.y : k < 12 ? hs.z : hs.w, k & 3);
+        put(0, (float)(sc & 15), -1056.0f); put(1, (float)(sc >> 4), -1056.0f);
+      }
+    };
+    // step k: Q4_K: run 4 c + h (low nibbles) or 4 c + 2 + h (high nibbles) of piece c, in the order (c, h, hi);  else run k = half k % 2 of piece k / 2
+    auto run_of = [](int k) { return TYPE == T_Q4_K ? 4 * (k >> 2) + 2 * (k & 1) + ((k >> 1) & 1) : k; };
+    auto pair_of = [&](int k, int p, h2 &w, h2 &w2) {  // operand slots 2 p, 2 p + 1
+      const int c = TYPE == T_Q4_K ? k >> 2 : k >> 1, h = TYPE == T_Q4_K ? (k >> 1) & 1 : k & 1, hi = k & 1;
+      const unsigned d = h == 0 ? (p < 2 ? wq[c].x : wq[c].y) : (p < 2 ? wq[c].z : wq[c].w);
+      if constexpr (TYPE == T_Q4_K) w = pkfma(as_h2(((hi ? ((p & 1) ? d >> 8 : d) : ((p & 1) ? d >> 4 : d << 4)) & 0x00F000F0u) | mg), sc2[hi], of2[hi]);
+      else if constexpr (TYPE == T_Q5_K) w = pkfma(as_h2((((p & 1) ? d >> 4 : d << 4) & 0x01F001F0u) | mg), sc2[0], of2[0]);
+      else {
+        const h2 u = as_h2((((p & 1) ? d >> 8 : d) & 0x00FF00FFu) | mg);
+        w = pkfma(u, sc2[0], of2[0]); w2 = pkfma(u, sc2[1], of2[1]);
+      }
+    };
+    constexpr int NW2 = TYPE == T_Q6_K ? 4 : 1;
+    h8 fr[2][NT];
+    h2 w[2][4], w2[2][NW2];
+    scales(0);
+    if (TYPE == T_Q4_K) scales(1);
+#pragma unroll
+    for (int p = 0; p < 4; ++p) pair_of(0, p, w[0][p], w2[0][p % NW2]);
     __builtin_amdgcn_sched_barrier(0);
     MRS_WAIT_VMCNT0();  // this wave's DMA pieces of superblock sb have landed
     __syncthreads();    // everyone's have, and every wave has finished reading the other buffer
+    stage_meta(sb + 1, it + 1, more);
     hs_next = load_hs(rec_next); hd_next = load_hd(rec_next);
-    // fragment of run r, token tile tt: chunk (2 r + hf) ^ nn of row 32 tt + nn
-    unsigned abase = MRS_LDS_BASE(smem) + (unsigned)((it & 1) * wide_buf<NT> + nn * 512 + ((nn ^ hf) << 4));
-    MRS_OPAQUE_TID(abase);  // one register: the run's offset is one exclusive or on it
-    auto frag = [&](int r, int tt) -> h8 { return MRS_LDS_H8(smem, abase ^ (unsigned)(32 * r), tt * 16384); };
-    f16v X[NT];
+    auto frag = [&](int r, int tt) -> h8 { return MRS_LDS_FRAG(h8, smem, abase ^ (unsigned)(32 * r), tt * (32 * ROWB)); };
+    constexpr int NX = TYPE == T_Q4_K ? 1 : 2;  // accumulators: Q5_K: runs 0 .. 7 | 8 .. 15 (|.| <= 16.5 M each);  Q6_K: the sl | sh operands
+    f16v X[NX][NT];
 #pragma unroll
-    for (int tt = 0; tt < NT; ++tt) X[tt] = zero;
+    for (int x = 0; x < NX; ++x)
+#pragma unroll
+      for (int tt = 0; tt < NT; ++tt) X[x][tt] = zero;
     // behind each matrix instruction of a step stand one read and a share of the operand build of the next step, behind the step's first one a piece of the next
     // superblock's DMA: the wave's own vector and memory instructions run under its matrix instructions (scheduling barriers keep the order)
 #pragma unroll
@@ -607,47 +450,64 @@ __global__ void __launch_bounds__(256, NT == 1 ? 3 : 2) gemm_qi_wide_kernel(cons
       const h8 wk = mk_h8(w[k & 1][0], w[k & 1][1], w[k & 1][2], w[k & 1][3]);
 #pragma unroll
       for (int tt = 0; tt < NT; ++tt) {
-        X[tt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(fr[k & 1][tt], wk, X[tt], 0, 0, 0);
+        const int x = TYPE == T_Q5_K ? k >> 3 : 0;
+        X[x][tt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(fr[k & 1][tt], wk, X[x][tt], 0, 0, 0);
+        if constexpr (TYPE == T_Q6_K)
+          X[1][tt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(fr[k & 1][tt], mk_h8(w2[k & 1][0], w2[k & 1][1], w2[k & 1][2], w2[k & 1][3]), X[1][tt], 0, 0, 0);
         if (k + 1 < 16) {
           fr[(k + 1) & 1][tt] = frag(run_of(k + 1), tt);
-          if (tt == 0 && ((k + 1) & 3) == 0) scales((k + 1) >> 2, 0);  // the high nibbles' first step comes one later
-          if (tt == 0 && ((k + 1) & 3) == 1) scales((k + 1) >> 2, 1);
+          if (tt == 0) scales(k + 1);
 #pragma unroll
-          for (int p = tt * 4 / NT; p < (tt + 1) * 4 / NT; ++p) w[(k + 1) & 1][p] = pair_of(k + 1, p);
+          for (int p = tt * 4 / NT; p < (tt + 1) * 4 / NT; ++p) pair_of(k + 1, p, w[(k + 1) & 1][p], w2[(k + 1) & 1][p % NW2]);
         }
-        if (tt == 0 && more && (k + 1) % (4 / NT) == 0) stage_q(sb + 1, it + 1, (k + 1) / (4 / NT) - 1);
-        if (tt == NT - 1 && more && k == 0) stage_meta(sb + 1, it + 1);
-        if (tt == NT - 1 && (k & 3) == 2) wq[k >> 2] = load_q(rec_next, k >> 2);  // step k + 1, the piece's last, has been built
+        if (tt == 0 && (k + 1) % (16 / NSTAGE) == 0) stage_q(sb + 1, it + 1, (k + 1) / (16 / NSTAGE) - 1, more);
+        if (tt == NT - 1 && (TYPE == T_Q4_K ? (k & 3) == 2 : (k & 1) == 0)) wq[TYPE == T_Q4_K ? k >> 2 : k >> 1] = load_q(rec_next, TYPE == T_Q4_K ? k >> 2 : k >> 1);  // step k + 1, the piece's last, has been built
         __builtin_amdgcn_sched_barrier(0);
       }
     }
-    const float *yd_s = (const float *)(smem + (it & 1) * wide_buf<NT> + ACT_);
-    const char *bs_s = (const char *)yd_s + YD_;
-    // M = sum_run m_{run / 2} bsum_run, S = sum_run sc_{run / 2} bsum_run: operand slot (hf, jj) <-> run 8 hf + jj -> sub-block 4 hf + jj / 2
-    const unsigned mw = hf ? hs.w : hs.z, sw = hf ? hs.y : hs.x;
-    h8 wm, wsc;
-#pragma unroll
-    for (int k = 0; k < 4; ++k) {
-      const _Float16 mk = (_Float16)(float)byte_of(mw, k), sk = (_Float16)(float)byte_of(sw, k);
-      wm[2 * k] = mk; wm[2 * k + 1] = mk; wsc[2 * k] = sk; wsc[2 * k + 1] = sk;
-    }
-    // d yd and dmin yd of the tile's outputs, each product rounded once: one matrix instruction of two 32 x 32 outer products (lane halves = blocks)
-    const float dd = half_bits_to_float((uint16_t)(hf ? hd >> 16 : hd & 0xffff));
+    const float *yd_s = (const float *)meta_s;
     const float keep = (sb % Cs) == 0 ? 0.f : 1.f;  // the first term of a run of superblocks starts its sum (0 * run + t), the others add (1 * run + t: exact)
     const f32v zero32 = {0.f};
+    // d yd (and dmin yd) of the tile's outputs, each product rounded once: one matrix instruction of two 32 x 32 outer products (lane halves = blocks)
+    const float dd = half_bits_to_float((uint16_t)(hf ? hd >> 16 : hd & 0xffff));
+    auto products = [&](int tt) -> f32v { return __builtin_amdgcn_mfma_f32_32x32x1f32(yd_s[tt * 32 + nn], dd, zero32, 0, 0, 0); };
+    if constexpr (TYPE == T_Q6_K) {
 #pragma unroll
-    for (int tt = 0; tt < NT; ++tt) {
-      const h8 bsf = *(const h8 *)(bs_s + (tt * 32 + nn) * 32 + hf * 16);
-      const f32v dy = __builtin_amdgcn_mfma_f32_32x32x1f32(yd_s[tt * 32 + nn], dd, zero32, 0, 0, 0);
-      const f16v Sx = __builtin_amdgcn_mfma_f32_32x32x16_f16(bsf, wsc, zero, 0, 0, 0);
-      const f16v M = __builtin_amdgcn_mfma_f32_32x32x16_f16(bsf, wm, zero, 0, 0, 0);
+      for (int tt = 0; tt < NT; ++tt) {
+        const f32v dy = products(tt);
 #pragma unroll
-      for (int v = 0; v < 16; ++v) {
-        const float If = fmaf(8.0f, Sx[v], X[tt][v]);  // (float)isum: one rounding of the exact integer
-        const float t = fmaf(dy[v], If, -(dy[16 + v] * M[v]));
-        run[tt][v] = fmaf(run[tt][v], keep, t);
+        for (int v = 0; v < 16; ++v) {
+          const float If = fmaf(16.0f, X[1][tt][v], X[0][tt][v]);  // (float)isum: one rounding of the exact integer
+          run[tt][v] = fmaf(run[tt][v], keep, dy[v] * If);
+        }
+        __builtin_amdgcn_sched_barrier(0);
       }
-      __builtin_amdgcn_sched_barrier(0);  // one token tile at a time: the sums of all of them would not fit the registers
+    } else {
+      // M = sum_run m_{run / 2} bsum_run, S = sum_run sc_{run / 2} bsum_run: operand slot (hf, jj) <-> run 8 hf + jj -> sub-block 4 hf + jj / 2
+      const unsigned mw = hf ? hs.w : hs.z, sw = hf ? hs.y : hs.x;
+      h8 wm, wsc;
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        const _Float16 mk = (_Float16)(float)byte_of(mw, k), sk = (_Float16)(float)byte_of(sw, k);
+        wm[2 * k] = mk; wm[2 * k + 1] = mk; wsc[2 * k] = sk; wsc[2 * k + 1] = sk;
+      }
+#pragma unroll
+      for (int tt = 0; tt < NT; ++tt) {
+        const h8 bsf = *(const h8 *)(meta_s + YD_ + (tt * 32 + nn) * 32 + hf * 16);
+        const f32v dy = products(tt);
+        const f16v Sx = __builtin_amdgcn_mfma_f32_32x32x16_f16(bsf, wsc, zero, 0, 0, 0);
+        const f16v M = __builtin_amdgcn_mfma_f32_32x32x16_f16(bsf, wm, zero, 0, 0, 0);
+#pragma unroll
+        for (int v = 0; v < 16; ++v) {
+          float If;  // (float)isum: one rounding of the exact integer (Q5_K's reaches 64 M: formed in int32)
+          if constexpr (TYPE == T_Q4_K) If = fmaf(8.0f, Sx[v], X[0][tt][v]);
+          else If = (float)(((int)X[0][tt][v] + (int)X[NX - 1][tt][v]) + 16 * (int)Sx[v]);
+          const float t = fmaf(dy[v], If, -(dy[16 + v] * M[v]));
+          run[tt][v] = fmaf(run[tt][v], keep, t);
+        }
+        __builtin_amdgcn_sched_barrier(0);  // one token tile at a time: the sums of all of them would not fit the registers
+      }
+    }
     }
     if ((sb + 1) % Cs == 0 || sb + 1 == sb_end) {  // a run of superblocks ends: its sum joins the row's left-to-right combination
       const bool first = sb < Cs;
@@ -666,150 +526,6 @@ __global__ void __launch_bounds__(256, NT == 1 ? 3 : 2) gemm_qi_wide_kernel(cons
     }
 }
 
-// ------------------------------------------------------------------------------------------------ Q8_0 weights x Q8_0 activation rows (round 6)
-// The decode engine's Q8_0 term (dec_core2.cuh Tile<T_Q8_0>, oracle term_q8_0): per 32-value block the exact integer dot, p_b = ((float)isum_b dw_b) dx_b, the
-// superblock's T = p_0 + p_1 + ... + p_7 left to right; superblock terms and runs combine as for the K-quants.  One v_mfma_i32_32x32x32_i8 IS one block of 32 tokens x 32
-// weight rows (K = 32, int32 accumulate: exact); the fix-up (convert, two multiplies, one add per output and block) runs on the vector ALU beside the other wave's
-// MFMAs.  Same tile, staging and split scheme as gemm_qi_kernel; LDS per superblock: 128 tokens x 256 int8 (16-byte chunks XOR-swizzled by token & 15) + the block
-// scales [8][128] f32, double buffered by LDS-DMA.
-typedef int i4v __attribute__((ext_vector_type(4)));
-typedef int i16v __attribute__((ext_vector_type(16)));
-constexpr int L8_ACT = TT * 256, L8_YD = 8 * TT * 4, L8_BUF = L8_ACT + L8_YD, L8_TOTAL = 2 * L8_BUF;
-__global__ void __launch_bounds__(GT) gemm_q80_kernel(const GemmArgs a) {
-  extern __shared__ __attribute__((aligned(16))) char smem[];
-  const int tid = tid_opaque(), lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int nn = lane & 31, hf = lane >> 5;
-  const int n0 = blockIdx.x * TN;
-  int tbeg = 0, tend = a.T, yt = blockIdx.y, ex = 0;  // the workgroup's token rows [tbeg, tend) of the operand buffers (one expert's routes; all rows when dense)
-  if (a.bounds && !expert_tile(a.bounds, a.experts, TT, yt, ex, tbeg, tend)) return;
-  const uint8_t *wbase = a.w + (size_t)ex * a.w_bytes;
-  const int t0 = tbeg + yt * TT;
-  if (t0 >= tend) return;
-  const int wn = wave & 3, wt = wave >> 2;
-  const int S = a.K / 256, Cs = (S + 3) / 4;
-  const __amdgpu_buffer_rsrc_t rw = __builtin_amdgcn_make_buffer_rsrc((void *)wbase, (short)0, (int)a.w_bytes, 0x00020000);
-  constexpr int REC = REC_Q6K;
-  struct WRegs { v4u q[8]; v4u hs; };
-  const unsigned panel = (unsigned)((n0 + wn * 32) >> 5);
-  // the weight registers are a ring in place: piece b of superblock sb + 1 is requested as soon as piece b of sb has been multiplied (a second register set for
-  // the next superblock spilled 68 VGPRs)
-  auto rec_of = [&](int sb) { return (panel * (unsigned)S + (unsigned)sb) * (unsigned)REC; };
-  auto load_piece = [&](WRegs &wr, unsigned rec, int c) { wr.q[c] = __builtin_amdgcn_raw_buffer_load_b128(rw, rec + (unsigned)(c * 64 + lane) * 16u, 0, 0); };
-  auto load_hs = [&](WRegs &wr, unsigned rec) { wr.hs = __builtin_amdgcn_raw_buffer_load_b128(rw, rec + 8192u + (unsigned)nn * 16u, 0, 0); };
-  auto load_w = [&](WRegs &wr, int sb) {
-    const unsigned rec = rec_of(sb);
-#pragma unroll
-    for (int c = 0; c < 8; ++c) load_piece(wr, rec, c);
-    load_hs(wr, rec);
-  };
-  const int tlast = tend - 1 - t0;
-  const int8_t *q8 = (const int8_t *)a.qf;
-  const float *yd8 = (const float *)a.bsf;
-  auto stage = [&](int sb, int buf) {
-    char *base = smem + buf * L8_BUF;
-    const char *gq = (const char *)q8 + ((size_t)sb * a.T + t0) * 256;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {  // one DMA instruction = 1 KiB = 4 token rows; lane l -> row 4 quad + (l >> 4), chunk position l & 15
-      const int quad = wave * 4 + i;
-      const int tr = 4 * quad + (lane >> 4), trc = min(tr, tlast);
-      MRS_GLDS16(gq + (size_t)trc * 256 + (((lane & 15) ^ (tr & 15)) << 4), base + quad * 1024);
-    }
-#pragma unroll
-    for (int i = 0; i < 2; ++i) {  // block scales: wave w stages block w, 64 tokens per instruction
-      const int tr = i * 64 + lane;
-      MRS_GLDS4((const char *)yd8 + (((size_t)sb * 8 + wave) * a.T + t0 + min(tr, tlast)) * 4, base + L8_ACT + (wave * TT + i * 64) * 4);
-    }
-  };
-  float run[2][16], pend[2][16];
-#pragma unroll
-  for (int tt = 0; tt < 2; ++tt)
-#pragma unroll
-    for (int v = 0; v < 16; ++v) { run[tt][v] = 0.f; pend[tt][v] = 0.f; }
-  WRegs wr;
-  const int sb_begin = a.ksplit > 1 ? (int)blockIdx.z * Cs : 0, sb_end = a.ksplit > 1 ? min(S, sb_begin + Cs) : S;
-  if (sb_begin >= sb_end) {
-    if (a.ksplit > 1) {  // a run without superblocks contributes +0
-      const int n = n0 + wn * 32 + nn;
-#pragma unroll
-      for (int tt = 0; tt < 2; ++tt)
-#pragma unroll
-        for (int v = 0; v < 16; ++v) {
-          const int t = t0 + wt * 64 + tt * 32 + 8 * (v >> 2) + 4 * hf + (v & 3);
-          if (n < a.N && t < tend) a.part[((size_t)blockIdx.z * a.T + t) * a.N + n] = 0.f;
-        }
-    }
-    return;
-  }
-  load_w(wr, sb_begin); stage(sb_begin, sb_begin & 1);
-  const int trow = wt * 64 + nn;
-  const i16v zero = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
-  for (int sb = sb_begin; sb < sb_end; ++sb) {
-    const int buf = sb & 1;
-    MRS_WAIT_VMCNT0();
-    __syncthreads();
-    const bool more = sb + 1 < sb_end;
-    const unsigned rec_next = more ? rec_of(sb + 1) : 0xF0000000u;  // past the tensor: zeros, no traffic (the request stays unconditional: exact waits)
-    if (more) stage(sb + 1, buf ^ 1);
-    const char *act_s = smem + buf * L8_BUF;
-    const float *yd_s = (const float *)(act_s + L8_ACT);
-    float Tt[2][16];
-    auto act_frag8 = [&](int tt, int b) { return *(const i4v *)(act_s + (trow + 32 * tt) * 256 + (((2 * b + hf) ^ (nn & 15)) << 4)); };
-    i4v afn[2] = {act_frag8(0, 0), act_frag8(1, 0)};  // the fragments are read one block ahead of their MFMAs
-#pragma unroll
-    for (int b = 0; b < 8; ++b) {
-      const unsigned hw = b < 2 ? wr.hs.x : b < 4 ? wr.hs.y : b < 6 ? wr.hs.z : wr.hs.w;
-      const float dwb = half_bits_to_float((uint16_t)((b & 1) ? (hw >> 16) : (hw & 0xffffu)));
-      const i4v wq = __builtin_bit_cast(i4v, wr.q[b]);
-      const i4v afc[2] = {afn[0], afn[1]};
-      if (b + 1 < 8) { afn[0] = act_frag8(0, b + 1); afn[1] = act_frag8(1, b + 1); }
-#pragma unroll
-      for (int tt = 0; tt < 2; ++tt) {
-        const i4v af = afc[tt];
-        const i16v is = __builtin_amdgcn_mfma_i32_32x32x32_i8(af, wq, zero, 0, 0, 0);
-#pragma unroll
-        for (int q4 = 0; q4 < 4; ++q4) {
-          const float4 y4 = *(const float4 *)(yd_s + b * TT + wt * 64 + tt * 32 + 8 * q4 + 4 * hf);
-          const float yy[4] = {y4.x, y4.y, y4.z, y4.w};
-#pragma unroll
-          for (int k = 0; k < 4; ++k) {
-            const int v = 4 * q4 + k;
-            const float p = ((float)is[v] * dwb) * yy[k];
-            Tt[tt][v] = b == 0 ? p : Tt[tt][v] + p;
-          }
-        }
-      }
-      load_piece(wr, rec_next, b);
-      if (b == 7) load_hs(wr, rec_next);
-      __builtin_amdgcn_sched_barrier(0);  // one block at a time: hoisting the MFMAs of later blocks keeps 16 result registers each alive (37 spilled VGPRs)
-    }
-    const bool cfirst = (sb % Cs) == 0;
-#pragma unroll
-    for (int tt = 0; tt < 2; ++tt)
-#pragma unroll
-      for (int v = 0; v < 16; ++v) run[tt][v] = cfirst ? Tt[tt][v] : run[tt][v] + Tt[tt][v];
-    if ((sb + 1) % Cs == 0 || sb + 1 == sb_end) {
-      const bool first = sb < Cs;
-#pragma unroll
-      for (int tt = 0; tt < 2; ++tt)
-#pragma unroll
-        for (int v = 0; v < 16; ++v) pend[tt][v] = first ? run[tt][v] : pend[tt][v] + run[tt][v];
-    }
-  }
-  const int n = n0 + wn * 32 + nn;
-#pragma unroll
-  for (int tt = 0; tt < 2; ++tt)
-#pragma unroll
-    for (int v = 0; v < 16; ++v) {
-      const int t = t0 + wt * 64 + tt * 32 + 8 * (v >> 2) + 4 * hf + (v & 3);
-      if (n < a.N && t < tend) {
-        if (a.ksplit > 1) a.part[((size_t)blockIdx.z * a.T + t) * a.N + n] = run[tt][v];
-        else {
-          float *o = a.out + (size_t)t * a.ldo + n;
-          *o = a.accumulate ? *o + pend[tt][v] : pend[tt][v];
-        }
-      }
-    }
-}
 // out[t][n] (+)= ((c0 + c1) + c2) + c3 of the four run sums (the row combination of ORD-U)
 __global__ void __launch_bounds__(256) gemm_qi_reduce_kernel(const float *__restrict__ part, float *__restrict__ out, int T, int N, int ldo, int accumulate, int part_n) {
   const size_t i = ((size_t)blockIdx.x * 256 + threadIdx.x) * 4, tot = (size_t)T * part_n;  // `part`: the tensor's first column of the launch's [4][T][part_n] sums
@@ -896,11 +612,13 @@ extern "C" int mrs_gemm_qi_ws(const void *w_qi, int type, int N, int K, const vo
                               void *stream) {
   return mrs_gemm_qi_multi(type, 1, &w_qi, &N, K, act, T, &out, &ldo, accumulate, nullptr, 0, 0, workspace, workspace_bytes, stream);
 }
-template <int NT>
-static void wide_launch(const qi::WideArgs &a, dim3 grid, hipStream_t s) {
-  auto kern = qi::gemm_qi_wide_kernel<NT>;
-  lds_attr_once((const void *)kern, 158 * 1024);
-  hipLaunchKernelGGL(kern, grid, dim3(256), 2 * qi::wide_buf<NT>, s, a);
+template <int TYPE>
+static void wide_launch(int NT, const qi::WideArgs &a, dim3 grid, hipStream_t s) {
+  auto k1 = qi::gemm_qi_wide_kernel<TYPE, 1>;
+  auto k2 = qi::gemm_qi_wide_kernel<TYPE, 2>;
+  lds_attr_once((const void *)(NT == 2 ? k2 : k1), 158 * 1024);
+  if (NT == 2) hipLaunchKernelGGL(k2, grid, dim3(256), (2 * qi::wide_buf<TYPE, 2>), s, a);
+  else hipLaunchKernelGGL(k1, grid, dim3(256), (2 * qi::wide_buf<TYPE, 1>), s, a);
 }
 extern "C" int mrs_gemm_qi_multi(int type, int nt, const void *const *w_qi, const int *N, int K, const void *act, int T, float *const *out, const int *ldo, int accumulate,
                                  const int *bounds, int experts, int max_rows, void *workspace, size_t workspace_bytes, void *stream) {
@@ -920,36 +638,29 @@ extern "C" int mrs_gemm_qi_multi(int type, int nt, const void *const *w_qi, cons
   auto reduce = [&](const float *part, int i, int part_n) {
     hipLaunchKernelGGL(qi::gemm_qi_reduce_kernel, dim3((unsigned)(((size_t)T * N[i] / 4 + 255) / 256)), dim3(256), 0, s, part, out[i], T, N[i], ldo[i], accumulate, part_n);
   };
-  if (type == T_Q4_K) {
-    // token tiles per wave: 32 rows fill one; from 33 rows on two waste no more and build each operand once for both (measured, 28672 x 4096: 28 us against 38 us at 20
-    // rows, 37 / 37 at 37, 221 / 199 at 512)
-    const int NT = (bounds ? T / experts : T) <= 32 ? 1 : 2, tl = 32 * NT;
-    qi::WideArgs a{};
-    qi::QiSeg *sg[3] = {&a.s0, &a.s1, &a.s2};
-    int gx = 0, x[3] = {0, 0, 0};
-    for (int i = 0; i < nt; ++i) { *sg[i] = qi::QiSeg{(const uint8_t *)w_qi[i], (unsigned)qi::qi_tensor_bytes(type, N[i], K), N[i], out[i], ldo[i]}; gx += (N[i] + qi::WIDE_ROWS - 1) / qi::WIDE_ROWS; x[i] = gx; }
-    a.x1 = x[0]; a.x2 = nt > 1 ? x[1] : gx;
-    a.K = K; a.T = T; a.qf = qf; a.yd = yd; a.bsf = bsf; a.accumulate = accumulate; a.part = (float *)workspace; a.part_n = n_all; a.bounds = bounds; a.experts = experts; a.ksplit = 1;
-    dim3 grid(gx, bounds ? T / tl + experts : (T + tl - 1) / tl);
-    // two workgroups fit a CU: below 512 they are cut by runs of superblocks (4096 x 14336 at 512 tokens, 256 workgroups: 119 us whole, 102 us cut; at 1024 tokens 185 / 192)
-    if (split_ok && (int)(grid.x * grid.y) < 512) { a.ksplit = 4; grid.z = 4; }
-    if (NT == 2) wide_launch<2>(a, grid, s); else wide_launch<1>(a, grid, s);
-    for (int i = 0, c = 0; i < nt && a.ksplit > 1; c += N[i++]) reduce(a.part + c, i, n_all);
-    return 0;
+  // Token tiles per wave.  K-quants: 32 rows fill one; from 33 rows on two waste little and build each operand once for both (us, one / two tiles: Q4_K 28672 x 4096 28 / 38 at
+  // 20 rows, 37 / 37 at 37, 221 / 199 at 512;  Q6_K 4096 x 14336 32 / 38 at 20 rows, 33 / 38 at 37, 161 / 129 at 512, 570 / 457 at 1999).  Q8_0 has no operand to build and a
+  // smaller workgroup's registers let one more live on a CU (q / k / v 95 / 141 and gate / up 348 / 376 at 700 rows, gate / up 1012 / 1079 at 1999).
+  const int NT = type == T_Q8_0 || (bounds ? T / experts : T) <= 32 ? 1 : 2, tl = 32 * NT;
+  qi::WideArgs a{};
+  qi::QiSeg *sg[3] = {&a.s0, &a.s1, &a.s2};
+  int gx = 0, x[3] = {0, 0, 0};
+  for (int i = 0; i < nt; ++i) { *sg[i] = qi::QiSeg{(const uint8_t *)w_qi[i], (unsigned)qi::qi_tensor_bytes(type, N[i], K), N[i], out[i], ldo[i]}; gx += (N[i] + qi::WIDE_ROWS - 1) / qi::WIDE_ROWS; x[i] = gx; }
+  a.x1 = x[0]; a.x2 = nt > 1 ? x[1] : gx;
+  a.K = K; a.T = T; a.qf = qf; a.yd = yd; a.bsf = bsf; a.accumulate = accumulate; a.part = (float *)workspace; a.part_n = n_all; a.bounds = bounds; a.experts = experts; a.ksplit = 1;
+  dim3 grid(gx, bounds ? T / tl + experts : (T + tl - 1) / tl);
+  // Two (NT = 2) or three workgroups fit a CU.  Below 512 the launch is cut by runs of superblocks (4096 x 14336 Q4_K at 512 rows, 256 workgroups: 119 us whole, 102 us cut).
+  // Long rows also where a second, partly filled round of workgroups would take as long as the first (K = 14336, whole / cut: Q4_K 1600 rows 314 / 287 us, Q6_K 430 / 392,
+  // Q8_0 512 rows 175 / 129, 700 rows 194 / 168, 1000 rows 233 / 239; one full round, Q4_K 1024 rows: 178 / 191; K = 4096 at 1300 rows 90 / 97).
+  const int wgs = (int)(grid.x * grid.y), slots = NT == 1 ? 768 : 512;
+  if (split_ok && (wgs < 512 || (K >= 8192 && wgs < 896 && wgs % slots != 0))) { a.ksplit = 4; grid.z = 4; }
+  switch (type) {
+    case T_Q4_K: wide_launch<T_Q4_K>(NT, a, grid, s); break;
+    case T_Q5_K: wide_launch<T_Q5_K>(NT, a, grid, s); break;
+    case T_Q6_K: wide_launch<T_Q6_K>(NT, a, grid, s); break;
+    default: wide_launch<T_Q8_0>(NT, a, grid, s); break;
   }
-  for (int i = 0; i < nt; ++i) {
-    qi::GemmArgs a{};
-    a.w = (const uint8_t *)w_qi[i]; a.w_bytes = (unsigned)qi::qi_tensor_bytes(type, N[i], K); a.type = type; a.N = N[i]; a.K = K; a.T = T;
-    a.qf = qf; a.yd = yd; a.bsf = bsf; a.out = out[i]; a.ldo = ldo[i]; a.accumulate = accumulate; a.bounds = bounds; a.experts = experts;
-    dim3 grid((N[i] + qi::TN - 1) / qi::TN, bounds ? T / qi::TT + experts : (T + qi::TT - 1) / qi::TT);
-    // few workgroups (o_proj / down_proj of a 512-token prompt: 128): one workgroup per run of superblocks, then the reduce -- the same additions in the same order
-    a.ksplit = 1; a.part = nullptr;
-    if (split_ok && (int)(grid.x * grid.y) < 200) { a.ksplit = 4; a.part = (float *)workspace; grid.z = 4; }
-    if (type == T_Q8_0) { auto kern = qi::gemm_q80_kernel; lds_attr_once((const void *)kern, 158 * 1024); hipLaunchKernelGGL(kern, grid, dim3(qi::GT), qi::L8_TOTAL, s, a); }
-    else if (type == T_Q5_K) { auto kern = qi::gemm_qi_kernel<T_Q5_K>; lds_attr_once((const void *)kern, 158 * 1024); hipLaunchKernelGGL(kern, grid, dim3(qi::GT), qi::LDS_TOTAL, s, a); }
-    else { auto kern = qi::gemm_qi_kernel<T_Q6_K>; lds_attr_once((const void *)kern, 158 * 1024); hipLaunchKernelGGL(kern, grid, dim3(qi::GT), qi::LDS_TOTAL, s, a); }
-    if (a.ksplit > 1) reduce(a.part, i, N[i]);
-  }
+  for (int i = 0, c = 0; i < nt && a.ksplit > 1; c += N[i++]) reduce(a.part + c, i, n_all);
   return 0;
 }
 

@@ -387,8 +387,6 @@ namespace hiphost { inline unsigned long long fake_realtime() { static thread_lo
 #define __builtin_amdgcn_sched_barrier(MASK) ((void)0)                  /* instruction-order hint only */
 #define MRS_OPAQUE_TID(t) ((void)0)
 // LDS-DMA (global_load_lds): LDS destination = wave-uniform base + lane * size, source address per lane; synchronous here
-#define MRS_GLDS16(gptr, lbase) memcpy((char *)(lbase) + (hiphost::linear_tid() & 63) * 16, (const void *)(gptr), 16)
-#define MRS_GLDS4(gptr, lbase) memcpy((char *)(lbase) + (hiphost::linear_tid() & 63) * 4, (const void *)(gptr), 4)
 #define MRS_BLDS16(RSRC, LBASE, VOFF) hiphost_buffer_load_lds((RSRC), (char *)(LBASE) + (hiphost::linear_tid() & 63) * 16, 16, (VOFF))
 #define MRS_BLDS4(RSRC, LBASE, VOFF) hiphost_buffer_load_lds((RSRC), (char *)(LBASE) + (hiphost::linear_tid() & 63) * 4, 4, (VOFF))
 static inline void hiphost_buffer_load_lds(__amdgpu_buffer_rsrc_t r, char *dst, unsigned n, unsigned voff) {
@@ -396,7 +394,7 @@ static inline void hiphost_buffer_load_lds(__amdgpu_buffer_rsrc_t r, char *dst, 
   if (o + n <= r.bytes) memcpy(dst, r.base + o, n); else memset(dst, 0, n);
 }
 #define MRS_LDS_BASE(P) 0u
-#define MRS_LDS_H8(P, ADDR, OFF) (*(const h8 *)((P) + (ADDR) + (OFF)))
+#define MRS_LDS_FRAG(TYPE, P, ADDR, OFF) (*(const TYPE *)((P) + (ADDR) + (OFF)))
 #define MRS_WAIT_VMCNT0() ((void)0)                                     /* product code: s_waitcnt vmcnt(0) */
 #define __builtin_amdgcn_fence(ORDER, SCOPE) ((void)0)                  /* one workgroup runs at a time: nothing to order */
 #define __builtin_amdgcn_s_sleep(N) ((void)0)

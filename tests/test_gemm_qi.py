@@ -196,7 +196,10 @@ def run_multi(O, be, tname, ns, k, T, bounds=None, ws=False, acc=False, seed=0):
 MULTI = [("Q4_K", (40,), 512, 70, None, False, False), ("Q4_K", (130, 33, 64), 1280, 33, None, False, True), ("Q4_K", (128, 36), 1280, 65, None, True, True),
          ("Q4_K", (64, 32), 1024, 5, None, True, False), ("Q4_K", (32, 64), 512, 130, (0, 0, 64, 129, 130), False, False), ("Q4_K", (64,), 768, 40, (0, 33, 34, 34, 40), False, False),
          ("Q6_K", (40, 64), 512, 9, None, False, False), ("Q6_K", (64,), 512, 20, (0, 0, 1, 20), False, False), ("Q8_0", (40, 64), 512, 9, None, False, False),
-         ("Q8_0", (64,), 512, 20, (0, 0, 1, 20), False, False), ("Q5_K", (64,), 512, 20, (0, 7, 7, 20), False, False)]
+         ("Q8_0", (64,), 512, 20, (0, 0, 1, 20), False, False), ("Q5_K", (64,), 512, 20, (0, 7, 7, 20), False, False),
+         ("Q6_K", (130, 36), 1280, 65, None, True, True), ("Q5_K", (128, 36), 1280, 65, None, True, False), ("Q8_0", (132, 32), 1280, 65, None, True, True),
+         ("Q6_K", (130,), 768, 33, None, False, True), ("Q5_K", (33,), 768, 70, None, False, True), ("Q8_0", (33,), 768, 33, None, False, False),
+         ("Q6_K", (32, 64), 512, 130, (0, 0, 64, 129, 130), False, False), ("Q8_0", (64,), 512, 130, (0, 0, 64, 129, 130), False, False)]
 
 
 @pytest.mark.parametrize("case", MULTI)
@@ -208,3 +211,23 @@ def test_gemm_qi_multi_host_emulation(oracle, case):
 @pytest.mark.parametrize("case", MULTI + [("Q4_K", (1024, 256, 256), 4096, 200, None, True, True), ("Q4_K", (512,), 1024, 400, (0, 100, 100, 333, 400), False, False)])
 def test_gemm_qi_multi_gpu(oracle, dev, case):
     run_multi(oracle, GpuBackend(dev), *case, seed=4)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("tname,T", [("Q8_0", 2050), ("Q6_K", 4130), ("Q4_K", 4130)])
+def test_long_rows_cut_by_runs_equal_the_whole_launch(oracle, dev, tname, T):
+    """65 token tiles x 8 row tiles: one round of workgroups and part of a second; with a workspace the launch is cut by runs of superblocks, without it stays whole."""
+    be, t, n, k = GpuBackend(dev), getattr(oracle, tname), 1024, 8192
+    rng = np.random.default_rng(7)
+    p = oracle.quantize(t, (rng.standard_normal((n, k)) * 0.05).astype(np.float32))
+    src, wq = be.buf(np.ascontiguousarray(p).reshape(-1)), be.buf(np.zeros(be.sym("mrs_gemm_qi_repack_bytes", [CI, C.c_longlong, C.c_longlong], C.c_size_t)(t, n, k), np.uint8))
+    assert be.sym("mrs_gemm_qi_repack", [VP, CI, C.c_longlong, C.c_longlong, VP, VP], CI)(src.ptr, t, n, k, wq.ptr, be.stream) == 0
+    x, act = be.buf(rng.standard_normal((T, k)).astype(np.float32)), be.buf(np.zeros(be.sym("mrs_qi_act_bytes", [CI, CI], C.c_size_t)(T, k), np.uint8))
+    assert be.sym("mrs_qi_quantize_for", [CI, VP, VP, CI, VP, C.c_float, CI, CI, VP, VP, VP], CI)(t, x.ptr, None, k, None, 1e-5, T, k, act.ptr, None, be.stream) == 0
+    ws, got = be.buf(np.zeros(4 * T * n, np.float32)), []
+    for w in (ws, None):
+        o = be.buf(np.zeros((T, n), np.float32))
+        assert be.sym("mrs_gemm_qi_ws", [VP, CI, CI, CI, VP, CI, VP, CI, CI, VP, C.c_size_t, VP], CI)(
+            wq.ptr, t, n, k, act.ptr, T, o.ptr, n, 0, w.ptr if w else None, 4 * T * n * 4 if w else 0, be.stream) == 0
+        got.append(o.numpy())
+    assert got[0].any() and np.array_equal(got[0], got[1])
