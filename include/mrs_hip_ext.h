@@ -264,6 +264,12 @@ int mrs_gemm_qi_ws(const void *w_qi, int ggml_type, int N, int K, const void *ac
 int mrs_prefill_attention_exact(const float *q, const void *k_cache, const void *v_cache, const uint32_t *block_table, const uint32_t *context_lens, float *out, int T,
                                 int num_heads, int num_kv_heads, int head_size, int block_size, int q_stride, int kv_block_stride, int kv_head_stride, float scale,
                                 int max_context_len, int kv_dtype, int sliding_window, int max_prompt_ctx /* largest context_lens[t], or 0 */, void *stream);
+/* the same with a workspace for the probabilities (any size from one query tile's slots on; mrs_prefill_attention_workspace_bytes: one group, or 256 MiB): same bits, scores
+ * formed once.  Too small or NULL: mrs_prefill_attention_exact. */
+size_t mrs_prefill_attention_workspace_bytes(int T, int num_heads, int max_context_len);
+int mrs_prefill_attention_exact_ws(const float *q, const void *k_cache, const void *v_cache, const uint32_t *block_table, const uint32_t *context_lens, float *out, int T,
+                                   int num_heads, int num_kv_heads, int head_size, int block_size, int q_stride, int kv_block_stride, int kv_head_stride, float scale,
+                                   int max_context_len, int kv_dtype, int sliding_window, int max_prompt_ctx, void *workspace, size_t workspace_bytes, void *stream);
 /* round 6 -- the other vec_dot partners and callers of the reference path (gguf/mod.rs:465-478; moe/experts/backends.rs:969-1100; distributed/layers.rs:965-975):
  * mrs_qi_quantize_for: the operand rows in the format the weight type multiplies with (q8_0 weights: Q8_0 blocks per 32 values; K-quants: Q8_K; mrs_qi_quantize = the
  * K-quant form).  mrs_gemm_qi* take q8_0 weights too: one v_mfma_i32_32x32x32_i8 per block of 32, p_b = ((float)isum_b dw_b) dx_b, terms added in block order.

@@ -1053,14 +1053,269 @@ __global__ void __launch_bounds__(64 * PM_NW, 2) prefill_attn_mfma_kernel(const 
     *(float4 *)(og + 8 * aa + 4 * hf) = make_float4(acc[4 * aa] * inv, acc[4 * aa + 1] * inv, acc[4 * aa + 2] * inv, acc[4 * aa + 3] * inv);
 }
 
+// ------------------------------------------------------------------------------------------------ the same chains as two kernels over a workspace
+// The one-kernel form above computes every score twice (the merge weights need the maximum over all splits first), puts a barrier between its score and its value phase, and
+// has one workgroup per (head, 32 queries): 64 on 256 CUs for a prompt of 37 tokens.  With a workspace the probabilities are kept instead: prefill_scores_kernel forms them
+// once, one wave per split (or a few), any number of waves per query tile; prefill_values_kernel multiplies them by V, one wave per 32 dims, without LDS or barriers.
+// What bounds both: the f32 matrix instructions (64 cycles each, 64 + 64 of them per head, 32 queries and 32 tokens) take the SIMD's vector ALU with them -- measured, the times of
+// matrix and vector instructions add up (unlike the f16 ones'), so a vector instruction saved is time saved: halves of a dword by one permute, no masks where every query sees the
+// whole block, the exponential in 21 instructions, one-block splits without the running correction.  The probabilities cost 4 KiB per 128 matrix instructions, written and read once.
+// Attention of 32 heads, us per layer, one kernel / these two: 37 tokens at 300 48 / 22, 512 tokens 72 / 44, 1999 tokens 740 / 407 (floor of the matrix instructions alone 215).
+// A slot of the workspace, per (head, tile of 32 queries, 32-token block): the probabilities as the B operand of the P . V instructions, block sums, alphas, running maxima.
+#ifndef MRS_KEEP16
+#define MRS_KEEP16(x) asm volatile("" : "+v"(x[0]), "+v"(x[1]), "+v"(x[2]), "+v"(x[3]), "+v"(x[4]), "+v"(x[5]), "+v"(x[6]), "+v"(x[7]), "+v"(x[8]), "+v"(x[9]), "+v"(x[10]), "+v"(x[11]), "+v"(x[12]), "+v"(x[13]), "+v"(x[14]), "+v"(x[15]))
+#endif
+constexpr int PS_SLOT = 4096 + 3 * 128;
+struct PrefillWs { char *slots; int nb, head0, heads, tile0, ups; };  // nb: slots per (head, tile); heads: of this launch; ups: splits per wave of the scores kernel
+__device__ __forceinline__ char *pa_slots(const PrefillWs &w, int head_i, int tile_i) { return w.slots + (size_t)(tile_i * w.heads + head_i) * w.nb * PS_SLOT; }
+
+// the f32 value of a dword's low (hf = 0) or high half-word, the half chosen per lane
+template <class CT> __device__ __forceinline__ float cvt16_half(unsigned w, int hf);
+template <> __device__ __forceinline__ float cvt16_half<bf16_t>(unsigned w, int hf) { return __uint_as_float(__builtin_amdgcn_perm(w, 0u, hf ? 0x07060c0cu : 0x05040c0cu)); }
+template <> __device__ __forceinline__ float cvt16_half<f16_t>(unsigned w, int hf) { return half_bits_to_float((uint16_t)(w >> (hf ? 16 : 0))); }
+// fast_exp_ref(x) for x <= 0 (or NaN, which it clamps to -87 as well), 21 instructions instead of 25: the sign of the rounding constant is known, no upper clamp, and 2^z is added
+// to the exponent of 1 + p instead of multiplied (z >= -126 and 1 + p > 1.3 there: the result is a normal number, the product is exact)
+__device__ __forceinline__ float fast_exp_ref_neg(float x) {
+  const float LOG2E = 1.44269504088896340736f, C0 = 0.6933594f, C1 = -2.1219444e-4f;
+  x = fmaxf(x, -87.0f);
+  const float z = truncf(x * LOG2E - 0.49999997f);
+  const float r = x - z * C0 - z * C1;
+  const float r2 = r * r;
+  const float p = r + r2 * (0.5f + r * (0.16666546f + r * (0.041665795f + r * (0.00833345f + r * 0.0013920345f))));
+  return __uint_as_float(__float_as_uint(1.0f + p) + ((unsigned)(int)z << 23));
+}
+
+// ONE: one block per split (model contexts up to 2048)
+template <class CT, bool ONE>
+__global__ void __launch_bounds__(256, 3) prefill_scores_kernel(const dec::AttnArgs a, const PrefillWs w) {
+  __shared__ __attribute__((aligned(16))) float q_s[64 * 64];  // B operand of the score instructions, four steps to a lane: [step / 4][lane][step % 4]
+  const int tid = tid_opaque(), lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int j = lane & 31, hf = lane >> 5;
+  const int head = w.head0 + (int)blockIdx.x, tile = w.tile0 + (int)blockIdx.y, kvh = head / (a.num_heads / a.num_kv_heads);
+  const int T = a.num_seqs, bpw = ONE ? 1 : a.bpw;
+  const uint32_t *bt = a.block_tables;
+  const int t_q = min(tile * 32 + j, T - 1), b_beg = ((int)blockIdx.z * 4 + wave) * w.ups * bpw;
+  // contexts and queries are requested together, the keys before the barrier: a short prompt's wave scores one block and is mostly latency
+  const int ctx = (int)a.context_lens[t_q];
+  float4 qv8[8];
+  {
+    const float *qg = a.q + (size_t)t_q * a.q_stride + (size_t)head * 128;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) qv8[i] = *(const float4 *)(qg + 4 * (wave + 4 * i));  // dims 4 m .. 4 m + 3 = steps 2 m, 2 m + 1; a lane half takes the even / the odd ones
+  }
+  // consecutive positions: the tile's last token (lane 31) has the longest context
+  const int ctx_lo = __builtin_amdgcn_readlane(ctx, 0), ctx_hi = __builtin_amdgcn_readlane(ctx, 31);
+  const int nblk = min((ctx_hi + 31) / 32, w.nb);
+  if ((int)blockIdx.z * 4 * w.ups * bpw >= nblk) return;
+  const int b_end = min(nblk, b_beg + w.ups * bpw);
+  const unsigned k_lane = (unsigned)j * 16u, id0 = bt[min(b_beg, nblk - 1)];
+  unsigned id1 = bt[min(b_beg + 1, nblk - 1)];
+  auto k_ptr = [&](unsigned id) { return (const char *)(a.k_cache + (size_t)(unsigned)__builtin_amdgcn_readfirstlane((int)id) * a.kv_block_stride + (size_t)kvh * a.kv_head_stride); };
+  v4u kr[16];
+  if (b_beg < b_end) {
+    const char *kb = k_ptr(id0);
+#pragma unroll
+    for (int c = 0; c < 16; ++c) kr[c] = *(const v4u *)(kb + (k_lane + (unsigned)c * 512u));
+  }
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    const int m = wave + 4 * i;
+    *(float2 *)(q_s + ((m >> 1) * 64 + lane) * 4 + 2 * (m & 1)) = hf ? make_float2(qv8[i].y, qv8[i].w) : make_float2(qv8[i].x, qv8[i].z);
+  }
+  __syncthreads();
+  if (b_beg >= b_end) return;
+  const int lo = a.window > 0 && ctx > a.window ? ctx - a.window : 0, lo_hi = __builtin_amdgcn_readlane(lo, 31);
+  char *slot = pa_slots(w, (int)blockIdx.x, (int)blockIdx.y) + (size_t)b_beg * PS_SLOT;
+  float m_run = -FLT_MAX;
+  for (int b = b_beg, in_split = 0; b < b_end; ++b, slot += PS_SLOT) {
+    const bool first = ONE || in_split == 0;
+    in_split = in_split + 1 == bpw ? 0 : in_split + 1;
+    if (first) m_run = -FLT_MAX;
+    const char *kn = k_ptr(id1);  // the table is read two blocks ahead, the keys one (past the wave's last block: unused)
+    id1 = bt[min(b + 2, nblk - 1)];
+    f16v acc0, acc1;
+#pragma unroll
+    for (int v = 0; v < 16; ++v) { acc0[v] = 0.f; acc1[v] = 0.f; }
+    float4 qn[2] = {*(const float4 *)(q_s + lane * 4), *(const float4 *)(q_s + (8 * 64 + lane) * 4)};
+#pragma unroll
+    for (int c = 0; c < 8; ++c) {  // dims 8 c .. and 64 + 8 c .. : two independent chains
+      const unsigned w0[4] = {kr[c].x, kr[c].y, kr[c].z, kr[c].w}, w1[4] = {kr[8 + c].x, kr[8 + c].y, kr[8 + c].z, kr[8 + c].w};
+      const float q0[4] = {qn[0].x, qn[0].y, qn[0].z, qn[0].w}, q1[4] = {qn[1].x, qn[1].y, qn[1].z, qn[1].w};
+      float k0[4], k1[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) { k0[u] = cvt16_half<CT>(w0[u], hf); k1[u] = cvt16_half<CT>(w1[u], hf); }
+      kr[c] = *(const v4u *)(kn + (k_lane + (unsigned)c * 512u));
+      kr[8 + c] = *(const v4u *)(kn + (k_lane + (unsigned)(8 + c) * 512u));
+      if (c + 1 < 8) { qn[0] = *(const float4 *)(q_s + ((c + 1) * 64 + lane) * 4); qn[1] = *(const float4 *)(q_s + ((c + 9) * 64 + lane) * 4); }
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        acc0 = __builtin_amdgcn_mfma_f32_32x32x2f32(k0[u], q0[u], acc0, 0, 0, 0);
+        acc1 = __builtin_amdgcn_mfma_f32_32x32x2f32(k1[u], q1[u], acc1, 0, 0, 0);
+      }
+      __builtin_amdgcn_sched_barrier(0);  // the queries' reads stay one step ahead (all of them at once do not fit the registers)
+    }
+    // lane (query j, half hf) holds tokens 8 (v / 4) + 4 hf + v % 4 of the block
+    const bool full = b * 32 + 32 <= ctx_lo && b * 32 >= lo_hi;  // every query sees all 32 tokens
+    float val[16], pv[16], mx = -FLT_MAX;
+#pragma unroll
+    for (int v = 0; v < 16; ++v) { const float sv = acc0[v] + acc1[v]; val[v] = sv * a.scale; }
+    unsigned ok = 0xffffu;
+    if (!full) {
+      ok = 0u;
+#pragma unroll
+      for (int v = 0; v < 16; ++v) {
+        const int pos = b * 32 + 8 * (v >> 2) + 4 * hf + (v & 3);
+        const bool in = pos < ctx && pos >= lo;
+        ok |= (in ? 1u : 0u) << v;
+        val[v] = in ? val[v] : -FLT_MAX;
+      }
+    }
+#pragma unroll
+    for (int v = 0; v < 16; ++v) mx = fmaxf(mx, val[v]);
+    mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+    const float mn = fmaxf(m_run, mx);
+#pragma unroll
+    for (int v = 0; v < 16; ++v) pv[v] = fast_exp_ref_neg(val[v] - mn);
+    MRS_KEEP16(pv);  // all of them in every lane, side by side: a branch around each masked one puts sixteen serial chains behind one another
+    if (!full) {
+#pragma unroll
+      for (int v = 0; v < 16; ++v) pv[v] = (ok >> v) & 1u ? pv[v] : 0.f;
+    }
+    // the decode wave's sum over the block's 32 tokens: pairwise tree in token order
+    float o8[4];
+#pragma unroll
+    for (int aa = 0; aa < 4; ++aa) {
+      const float q4 = (pv[4 * aa] + pv[4 * aa + 1]) + (pv[4 * aa + 2] + pv[4 * aa + 3]);  // tokens 8 aa + 4 hf + 0 .. 3
+      o8[aa] = q4 + __shfl_xor(q4, 32, 64);
+    }
+    const float ps = (o8[0] + o8[1]) + (o8[2] + o8[3]);
+    // step s of P . V takes tokens 2 s (lanes 0 .. 31) and 2 s + 1: [s / 4][lane][s % 4]; this lane holds tokens 8 aa + 4 hf + 0 .. 3 = steps 4 aa + 2 hf + {0, 0, 1, 1}
+#pragma unroll
+    for (int aa = 0; aa < 4; ++aa)
+#pragma unroll
+      for (int h = 0; h < 2; ++h) *(float2 *)(slot + ((unsigned)(j * 16 + hf * 8) + (unsigned)(aa * 1024 + h * 512))) = make_float2(pv[4 * aa + h], pv[4 * aa + 2 + h]);
+    const float alpha = first ? 0.f : fast_exp_ref_neg(m_run - mn);
+    *(float *)(slot + ((unsigned)(j * 4 + hf * 256) + 4096u)) = hf ? mn : ps;
+    if (!ONE && hf == 0) *(float *)(slot + ((unsigned)(j * 4) + 4224u)) = alpha;
+    m_run = mn;
+  }
+}
+template <class CT, bool ONE>
+__global__ void __launch_bounds__(256, 4) prefill_values_kernel(const dec::AttnArgs a, const PrefillWs w) {
+  const int tid = tid_opaque(), lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int j = lane & 31, hf = lane >> 5;
+  // longest contexts first, every other 256 workgroups backwards: where all workgroups are resident at once (1024 fit) every CU gets long and short ones
+  const int id = (int)(blockIdx.y * gridDim.x + blockIdx.x), q256 = id >> 8;
+  const int rank = q256 & 1 ? (q256 << 8) + min(256, (int)(gridDim.x * gridDim.y) - (q256 << 8)) - 1 - (id & 255) : id;
+  const int tile_i = (int)gridDim.y - 1 - rank / (int)gridDim.x, head_i = rank % (int)gridDim.x;
+  const int head = w.head0 + head_i, tile = w.tile0 + tile_i, kvh = head / (a.num_heads / a.num_kv_heads);
+  const int T = a.num_seqs, bpw = ONE ? 1 : a.bpw;
+  const int ctx_max = (int)a.context_lens[min(tile * 32 + 31, T - 1)], nblk = min((ctx_max + 31) / 32, w.nb);
+  const uint32_t *bt = a.block_tables;
+  const char *slots = pa_slots(w, head_i, tile_i);
+  auto meta = [&](int b, unsigned i) { return *(const float *)(slots + (size_t)b * PS_SLOT + ((unsigned)j * 4u + 4096u + 128u * i)); };
+  // V of a block, dims 32 wave .. + 31, as the A operand: lane (dim row, half) supplies V[dim][token 2 s + half] = half of dword s of the dim's 32-token row
+  struct Blk { v4u v[4]; float4 p[4]; float ps, alpha, mn; };
+  auto id_of = [&](int b) { return bt[min(b, nblk - 1)]; };
+  auto load = [&](int b, unsigned bid, Blk &r) {
+    const char *vb = (const char *)(a.v_cache + (size_t)(unsigned)__builtin_amdgcn_readfirstlane((int)bid) * a.kv_block_stride + (size_t)kvh * a.kv_head_stride);
+    const char *pb = slots + (size_t)b * PS_SLOT;
+#pragma unroll
+    for (int c = 0; c < 4; ++c) { r.v[c] = *(const v4u *)(vb + ((unsigned)(32 * wave + j) * 64u + (unsigned)c * 16u)); r.p[c] = *(const float4 *)(pb + ((unsigned)lane * 16u + (unsigned)c * 1024u)); }
+    r.ps = meta(b, 0); r.mn = meta(b, 2);
+    if (!ONE) r.alpha = meta(b, 1);
+  };
+  Blk r0, r1;
+  unsigned id0 = id_of(0), id1 = id_of(1);  // the table is read two blocks ahead
+  load(0, id0, r0);
+  id0 = id_of(2);
+  float M = -FLT_MAX;  // over the splits: their last blocks' running maxima
+  for (int b = min((hf + 1) * bpw, nblk) - 1;; b = min(b + 2 * bpw, nblk - 1)) {
+    M = fmaxf(M, meta(b, 2));
+    if (b + 1 >= nblk) break;
+  }
+  M = fmaxf(M, __shfl_xor(M, 32, 64));
+  f16v acc, o;
+#pragma unroll
+  for (int v = 0; v < 16; ++v) { acc[v] = 0.f; o[v] = 0.f; }
+  float s_all = 0.f, l_run = 0.f;
+  int in_split = 0;
+  auto step = [&](int b, Blk &r) {
+    if (b + 1 == nblk) {  // slots past the tile's longest context may hold anything (their p are 0)
+#pragma unroll
+      for (int c = 0; c < 4; ++c) {
+        unsigned *vw = (unsigned *)&r.v[c];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) vw[u] = b * 32 + 2 * (4 * c + u) + hf < ctx_max ? vw[u] : 0u;
+      }
+    }
+    if (ONE || in_split == 0) {
+#pragma unroll
+      for (int v = 0; v < 16; ++v) o[v] = 0.f;
+      l_run = r.ps;
+    } else {
+#pragma unroll
+      for (int v = 0; v < 16; ++v) o[v] = o[v] * r.alpha;
+      l_run = l_run * r.alpha + r.ps;
+    }
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+      const unsigned w4[4] = {r.v[c].x, r.v[c].y, r.v[c].z, r.v[c].w};
+      const float pp[4] = {r.p[c].x, r.p[c].y, r.p[c].z, r.p[c].w};
+#pragma unroll
+      for (int u = 0; u < 4; ++u) o = __builtin_amdgcn_mfma_f32_32x32x2f32(cvt16_half<CT>(w4[u], hf), pp[u], o, 0, 0, 0);
+    }
+    if (ONE || ++in_split == bpw || b + 1 == nblk) {  // attn_merge_core: s += l_j w_j;  acc += o_j w_j  (multiply and add separate)
+      const float wj = fast_exp_ref_neg(r.mn - M), lw = l_run * wj;
+      s_all = s_all + lw;
+#pragma unroll
+      for (int v = 0; v < 16; ++v) { const float t0 = o[v] * wj; acc[v] = acc[v] + t0; }
+      in_split = 0;
+    }
+  };
+  for (int b = 0; b < nblk; b += 2) {
+    load(min(b + 1, nblk - 1), id1, r1);
+    id1 = id_of(b + 3);
+    step(b, r0);
+    if (b + 1 >= nblk) break;
+    load(min(b + 2, nblk - 1), id0, r0);
+    id0 = id_of(b + 4);
+    step(b + 1, r1);
+  }
+  if (tile * 32 + j >= T) return;
+  const float inv = 1.0f / s_all;
+  float *og = a.out + ((size_t)(tile * 32 + j) * a.num_heads + head) * 128 + 32 * wave;
+#pragma unroll
+  for (int aa = 0; aa < 4; ++aa)
+    *(float4 *)(og + 8 * aa + 4 * hf) = make_float4(acc[4 * aa] * inv, acc[4 * aa + 1] * inv, acc[4 * aa + 2] * inv, acc[4 * aa + 3] * inv);
+}
+
 }  // namespace qi
 }  // namespace mrs
 
+// workspace of mrs_prefill_attention_exact_ws: a slot per head, 32 queries and 32 tokens of context, at most 256 MiB (longer prompts go in groups of heads / of query tiles;
+// half of the slots of a causal prompt are never touched, so a group stays in the last-level cache)
+extern "C" size_t mrs_prefill_attention_workspace_bytes(int T, int num_heads, int max_context_len) {
+  if (T <= 0 || num_heads <= 0 || max_context_len <= 0) return 0;
+  const size_t pair = (size_t)((max_context_len + 31) / 32) * mrs::qi::PS_SLOT, all = pair * num_heads * (size_t)((T + 31) / 32);
+  return std::max(pair, std::min(all, (size_t)256 << 20));
+}
 // q f32 [T][q_stride] (RoPE applied), pages already hold the prompt's K / V; context_lens [T] = position + 1 of every prompt token (device), block_table = the
 // sequence's row; out f32 [T][num_heads * 128].  max_context_len = the model's (it fixes the split length exactly as in mrs_dec_attention).
+extern "C" int mrs_prefill_attention_exact_ws(const float *q, const void *k_cache, const void *v_cache, const uint32_t *block_table, const uint32_t *context_lens, float *out,
+                                              int T, int num_heads, int num_kv_heads, int head_size, int block_size, int q_stride, int kv_block_stride, int kv_head_stride,
+                                              float scale, int max_context_len, int kv_dtype, int sliding_window, int max_prompt_ctx, void *workspace, size_t workspace_bytes,
+                                              void *stream);
 extern "C" int mrs_prefill_attention_exact(const float *q, const void *k_cache, const void *v_cache, const uint32_t *block_table, const uint32_t *context_lens, float *out,
                                            int T, int num_heads, int num_kv_heads, int head_size, int block_size, int q_stride, int kv_block_stride, int kv_head_stride,
                                            float scale, int max_context_len, int kv_dtype, int sliding_window, int max_prompt_ctx, void *stream) {
+  return mrs_prefill_attention_exact_ws(q, k_cache, v_cache, block_table, context_lens, out, T, num_heads, num_kv_heads, head_size, block_size, q_stride, kv_block_stride,
+                                        kv_head_stride, scale, max_context_len, kv_dtype, sliding_window, max_prompt_ctx, nullptr, 0, stream);
+}
+extern "C" int mrs_prefill_attention_exact_ws(const float *q, const void *k_cache, const void *v_cache, const uint32_t *block_table, const uint32_t *context_lens, float *out,
+                                              int T, int num_heads, int num_kv_heads, int head_size, int block_size, int q_stride, int kv_block_stride, int kv_head_stride,
+                                              float scale, int max_context_len, int kv_dtype, int sliding_window, int max_prompt_ctx, void *workspace, size_t workspace_bytes,
+                                              void *stream) {
   if (!q || !out || head_size != 128 || block_size != 32 || T <= 0 || num_kv_heads <= 0 || num_heads % num_kv_heads || (kv_dtype != 0 && kv_dtype != 1)) return -1;
   const int G = num_heads / num_kv_heads;
   if (G != 1 && G != 2 && G != 4 && G != 8) return -1;
@@ -1073,10 +1328,33 @@ extern "C" int mrs_prefill_attention_exact(const float *q, const void *k_cache, 
   // (w_j, l_j) per split live in LDS: as many splits as the longest context of this prompt needs (<= 64 by the rule above)
   const int need_ctx = max_prompt_ctx > 0 && max_prompt_ctx < max_context_len ? max_prompt_ctx : max_context_len;
   a.max_splits = std::max(1, std::min(64, (((need_ctx + 31) / 32) + a.bpw - 1) / a.bpw));
-  // round 6: the matrix-core form (prefill_attn_mfma_kernel: the same chains on v_mfma_f32_32x32x2_f32); MRS_PREFILL_ATTN_MFMA=0 keeps the vector-ALU kernel
+  // with a workspace: the scores once, probabilities kept (prefill_scores_kernel, prefill_values_kernel); without: prefill_attn_mfma_kernel; MRS_PREFILL_ATTN_MFMA=0 keeps
+  // the vector-ALU kernel
   static const int use_mfma = [] { const char *e = getenv("MRS_PREFILL_ATTN_MFMA"); return e ? atoi(e) : 1; }();
   {
-    const int nb = (need_ctx + 31) / 32;
+    const int nb = (need_ctx + 31) / 32, tiles = (T + 31) / 32;
+    const size_t pair = (size_t)nb * mrs::qi::PS_SLOT, fit = workspace ? workspace_bytes / pair : 0;  // (head, tile) pairs per launch
+    if (use_mfma && fit > 0) {
+      const int ht = (int)std::min<size_t>(num_heads, fit / tiles), hgroups = ht ? (num_heads + ht - 1) / ht : num_heads;
+      const int hs = (num_heads + hgroups - 1) / hgroups, ts = ht ? tiles : (int)std::min<size_t>(tiles, fit);
+      for (int h0 = 0; h0 < num_heads; h0 += hs)
+        for (int t0 = 0; t0 < tiles; t0 += ts) {
+          mrs::qi::PrefillWs w{(char *)workspace, nb, h0, std::min(hs, num_heads - h0), t0, 1};
+          const int nt = std::min(ts, tiles - t0), splits = (nb + a.bpw - 1) / a.bpw;
+          // splits per wave: more where there are waves enough without (the queries are read once for all, a wave's next keys arrive under its instructions), few enough
+          // that the last round of workgroups stays short.  Scores, us, of 1 / 2 / 4 / 8 per wave: 512 tokens - 26.8 / 24.8, 1999 tokens (16 heads) - / 113.2 / 113.3 / 120.5
+          while (w.ups < 4 && (size_t)w.heads * nt * nb > (size_t)w.ups * w.ups * 4096) w.ups *= 2;
+          const dim3 gs(w.heads, nt, (splits + 4 * w.ups - 1) / (4 * w.ups)), gv(w.heads, nt);
+          auto go = [&](auto scores, auto values) {
+            hipLaunchKernelGGL(scores, gs, dim3(256), 0, (hipStream_t)stream, a, w);
+            hipLaunchKernelGGL(values, gv, dim3(256), 0, (hipStream_t)stream, a, w);
+          };
+          using namespace mrs::qi;
+          if (kv_dtype == 1) a.bpw == 1 ? go(prefill_scores_kernel<mrs::bf16_t, true>, prefill_values_kernel<mrs::bf16_t, true>) : go(prefill_scores_kernel<mrs::bf16_t, false>, prefill_values_kernel<mrs::bf16_t, false>);
+          else a.bpw == 1 ? go(prefill_scores_kernel<mrs::f16_t, true>, prefill_values_kernel<mrs::f16_t, true>) : go(prefill_scores_kernel<mrs::f16_t, false>, prefill_values_kernel<mrs::f16_t, false>);
+        }
+      return 0;
+    }
     const size_t lds_m = (size_t)mrs::qi::PM_Q + mrs::qi::PM_P + mrs::qi::PM_SC + (size_t)nb * 128;
     if (use_mfma && lds_m <= 158 * 1024) {
       const dim3 gm(num_heads, (T + 31) / 32);

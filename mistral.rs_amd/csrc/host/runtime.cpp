@@ -553,6 +553,11 @@ class Llama {
     const int nq = c.num_heads * c.head_dim, nkv = c.num_kv_heads * c.head_dim;
     return mrs_gemm_qi_workspace_bytes(T, std::max(std::max(c.hidden_size, nq + 2 * nkv), T <= 128 && c.num_experts == 0 ? 2 * c.intermediate_size : 0));
   }
+  // gate, up and act of T rows: not live during the attention, which keeps its probabilities there
+  static size_t ffn_bytes(const mrs_llama_config &c, int T) {
+    const int ctx = std::min(c.max_blocks_per_seq * c.block_size, (int)c.max_context_len);
+    return std::max(align((size_t)T * c.intermediate_size * 4) * 3, c.head_dim == 128 && c.block_size == 32 ? align(mrs_prefill_attention_workspace_bytes(T, c.num_heads, ctx)) : 0);
+  }
   static size_t prefill_workspace_bytes(const mrs_llama_config &c, int T) {
     const size_t t = (size_t)T, d = c.hidden_size, nq = (size_t)c.num_heads * c.head_dim, nkv = (size_t)c.num_kv_heads * c.head_dim;
     const size_t ff = c.intermediate_size;
@@ -560,7 +565,7 @@ class Llama {
     b += align(t * d * 4) * 2;        // h, xn
     b += align(t * nq * 4) * 2;       // q, attn
     b += align(t * nkv * 4) * 2;      // k, v
-    b += align(t * ff * 4) * 3;       // gate, up, act
+    b += ffn_bytes(c, T);             // gate, up, act;  before them: the attention's probabilities
     b += align((pad_to((int)d, MATRIX_ROW_PADDING) / 32) * 36);  // Q8_1 scratch of the last-token lm_head GEMV
     b += align(mrs_qi_act_bytes(T, (int)std::max(std::max(d, nq), ff))) + align(qi_split_bytes(c, T));  // exact prompt path: Q8_K operands of T rows (f16 quants, scales, run sums) + run sums of split launches
     if (T > prefill_big_min()) b += align(t * std::max(std::max(d, nq), ff) * 2) + align(mrs_gemm_q_bf16_workspace_bytes(T)) + align(t * ff * 2);  // bf16 activations + split-K partials + act(gate)*up slabs of the fused gate/up GEMM
@@ -676,7 +681,7 @@ class Llama {
     return all_reduce(h, (size_t)T * d, s) ? fail("prefill (exact): moe all-reduce failed: %s", g_last_error.c_str()) : 0;
   }
   int prefill_exact(const mrs_llama_prefill_args &pa, int T, float *h, float *xn, float *q, float *k, float *v, float *attn, float *g, float *u, float *act, void *qact,
-                    void *qws, size_t qws_bytes, const MoeExactBufs &mx, hipStream_t s) const {
+                    void *qws, size_t qws_bytes, void *attn_ws, const MoeExactBufs &mx, hipStream_t s) const {
     const int d = cfg.hidden_size, hd = cfg.head_dim, nq = cfg.num_heads * hd, nkv = cfg.num_kv_heads * hd, ff = cfg.intermediate_size;
     const int bs = cfg.block_size, kvh = cfg.num_kv_heads, kvd = cfg.kv_f16 ? 0 : 1;
     const int eff_max = std::min(cfg.max_blocks_per_seq * bs, cfg.max_context_len);
@@ -729,8 +734,8 @@ class Llama {
       rotary_embedding_positions(q, k, (void *)bufs.cos_table, (void *)bufs.sin_table, (void *)pa.positions, cfg.rope_interleaved ? 0 : 1, hd, T,
                                  cfg.rot_dim / 2, cfg.max_context_len, cfg.num_heads, cfg.num_kv_heads, nq, nkv, 2, st);
       reshape_and_cache(k, v, bl.key_cache, bl.value_cache, (int64_t *)pa.slot_mapping, T, cfg.num_kv_heads, hd, bs, 8, nkv, nkv, s, 2, kvd == 1 ? 1 : 0, nullptr, nullptr);
-      if (mrs_prefill_attention_exact(q, bl.key_cache, bl.value_cache, pa.block_tables, pa.context_lens, attn, T, cfg.num_heads, kvh, hd, bs, nq, kvh * hd * bs, hd * bs,
-                                      1.0f / sqrtf((float)hd), eff_max, kvd, cfg.sliding_window, pa.start_pos + T, s))
+      if (mrs_prefill_attention_exact_ws(q, bl.key_cache, bl.value_cache, pa.block_tables, pa.context_lens, attn, T, cfg.num_heads, kvh, hd, bs, nq, kvh * hd * bs, hd * bs,
+                                      1.0f / sqrtf((float)hd), eff_max, kvd, cfg.sliding_window, pa.start_pos + T, attn_ws, ffn_bytes(cfg, T), s))
         return fail("prefill (exact): attention refused the shape");
       if (row_parallel(*bl.o_proj, d, nq, attn, nullptr, nq, nullptr)) return -1;
       if (cfg.num_experts > 0) {
@@ -757,7 +762,8 @@ class Llama {
     float *h = (float *)take(t * d * 4), *xn = (float *)take(t * d * 4);
     float *q = (float *)take(t * nq * 4), *attn = (float *)take(t * nq * 4);
     float *k = (float *)take(t * nkv * 4), *v = (float *)take(t * nkv * 4);
-    float *g = (float *)take(t * ff * 4), *u = (float *)take(t * ff * 4), *act = (float *)take(t * ff * 4);
+    char *const ffn = take(ffn_bytes(cfg, T));
+    float *g = (float *)ffn, *u = (float *)(ffn + align(t * ff * 4)), *act = (float *)(ffn + align(t * ff * 4) * 2);
     if (prefill_exact_ok()) {
       void *qact = take(mrs_qi_act_bytes(T, std::max(std::max(d, nq), ff)));
       const size_t qws_bytes = qi_split_bytes(cfg, T);
@@ -771,7 +777,7 @@ class Llama {
         mx.y = (float *)take(r * d * 4);
         mx.qact_g = take(mrs_qi_act_bytes((int)r, d)); mx.qact_r = take(mrs_qi_act_bytes((int)r, ff));
       }
-      return prefill_exact(pa, T, h, xn, q, k, v, attn, g, u, act, qact, qws, qws_bytes, mx, s);
+      return prefill_exact(pa, T, h, xn, q, k, v, attn, g, u, act, qact, qws, qws_bytes, ffn, mx, s);
     }
     MoePrefillBufs moe{};
     if (cfg.num_experts > 0) {

@@ -386,6 +386,15 @@ namespace hiphost { inline unsigned long long fake_realtime() { static thread_lo
 #define __builtin_amdgcn_sched_group_barrier(MASK, SIZE, SYNC) ((void)0) /* instruction-order hint only */
 #define __builtin_amdgcn_sched_barrier(MASK) ((void)0)                  /* instruction-order hint only */
 #define MRS_OPAQUE_TID(t) ((void)0)
+#define MRS_KEEP16(x) ((void)0)
+static inline unsigned __builtin_amdgcn_perm(unsigned hi, unsigned lo, unsigned sel) {  // v_perm_b32: selector bytes 0 .. 3 = lo's, 4 .. 7 = hi's, 12 = zero
+  unsigned r = 0;
+  for (int i = 0; i < 4; ++i) {
+    const unsigned c = (sel >> (8 * i)) & 0xff;
+    r |= (c < 4 ? (lo >> (8 * c)) & 0xff : c < 8 ? (hi >> (8 * (c - 4))) & 0xff : 0u) << (8 * i);
+  }
+  return r;
+}
 // LDS-DMA (global_load_lds): LDS destination = wave-uniform base + lane * size, source address per lane; synchronous here
 #define MRS_BLDS16(RSRC, LBASE, VOFF) hiphost_buffer_load_lds((RSRC), (char *)(LBASE) + (hiphost::linear_tid() & 63) * 16, 16, (VOFF))
 #define MRS_BLDS4(RSRC, LBASE, VOFF) hiphost_buffer_load_lds((RSRC), (char *)(LBASE) + (hiphost::linear_tid() & 63) * 4, 4, (VOFF))

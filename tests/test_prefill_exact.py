@@ -58,6 +58,47 @@ def test_prompt_attention_equals_decode_attention_gpu(oracle, dev, heads, kvh, T
     check_attention(oracle, GpuBackend(dev), heads, kvh, T, max_ctx, kvd, window, start)
 
 
+# (heads, kv heads, T, model context, kv dtype, window, first position, (head, tile) pairs that fit the workspace): one block and several blocks per split, whole launches,
+# groups of heads, groups of query tiles
+WS = [(4, 1, 40, 64, 1, 0, 0, 99), (4, 2, 70, 128, 0, 0, 0, 7), (2, 2, 33, 96, 1, 0, 20, 1), (8, 2, 50, 4096, 1, 0, 200, 99), (4, 1, 90, 128, 1, 40, 0, 2), (3, 3, 1, 2304, 0, 0, 130, 99)]
+
+
+def check_attention_ws(O, be, heads, kvh, T, max_ctx, kv_dtype, window, start, pairs):
+    """mrs_prefill_attention_exact_ws == mrs_prefill_attention_exact bit for bit; slots past the context hold NaN."""
+    hd, bs, nq = 128, 32, heads * 128
+    rng = np.random.default_rng(heads + T)
+    mbs = (start + T + bs - 1) // bs
+    to16 = (lambda a: a.astype(np.float16).view(np.uint16)) if kv_dtype == 0 else O.to_bf16_bits
+    k_np, v_np = (rng.standard_normal((mbs, kvh, hd // 8, bs, 8)) * 0.7).astype(np.float32), rng.standard_normal((mbs, kvh, hd, bs)).astype(np.float32)
+    if (start + T) % bs:
+        k_np[-1, :, :, (start + T) % bs:], v_np[-1, :, :, (start + T) % bs:] = np.nan, np.nan
+    perm = rng.permutation(mbs)
+    kc, vc, bt = be.buf(to16(k_np)[np.argsort(perm)]), be.buf(to16(v_np)[np.argsort(perm)]), be.buf(perm.astype(np.uint32).reshape(1, mbs))
+    q, cl = be.buf((rng.standard_normal((T, nq)) * 0.5).astype(np.float32)), be.buf(np.arange(start + 1, start + T + 1, dtype=np.uint32))
+    need = be.sym("mrs_prefill_attention_workspace_bytes", [CI, CI, CI], C.c_size_t)
+    one = need(1, 1, start + T)
+    assert need(T, heads, start + T) == min(one * heads * ((T + 31) // 32), 256 << 20)
+    size = min(one * min(pairs, heads * ((T + 31) // 32)), 256 << 20)
+    ws, got = be.buf(np.full(size // 4, np.nan, np.float32)), []
+    for name, types, args in (("mrs_prefill_attention_exact", PA, ()), ("mrs_prefill_attention_exact_ws", PA[:-1] + [VP, C.c_size_t, VP], (ws.ptr, size))):
+        o = be.buf(np.full((T, nq), np.nan, np.float32))
+        assert be.sym(name, types, CI)(q.ptr, kc.ptr, vc.ptr, bt.ptr, cl.ptr, o.ptr, T, heads, kvh, hd, bs, nq, kvh * hd * bs, hd * bs, np.float32(hd ** -0.5), max_ctx, kv_dtype, window,
+                                       start + T, *args, be.stream) == 0
+        got.append(o.numpy())
+    assert np.isfinite(got[0]).all() and np.array_equal(got[0], got[1]), int((got[0] != got[1]).sum())
+
+
+@pytest.mark.parametrize("case", WS)
+def test_prompt_attention_with_a_workspace_host_emulation(oracle, case):
+    check_attention_ws(oracle, HostBackend(), *case)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("case", WS[:3] + WS[4:] + [(32, 8, 512, 1024, 1, 0, 0, 9999), (8, 2, 300, 4096, 1, 0, 1000, 40), (32, 8, 700, 832, 0, 256, 0, 50), (64, 8, 1100, 2304, 1, 0, 0, 9999)])
+def test_prompt_attention_with_a_workspace_gpu(oracle, dev, case):
+    check_attention_ws(oracle, GpuBackend(dev), *case)
+
+
 Q80 = lambda O: dict(embd=O.Q8_0, q=O.Q8_0, k=O.Q8_0, v=O.Q8_0, o=O.Q8_0, gate=O.Q8_0, up=O.Q8_0, down=O.Q8_0, output=O.Q8_0)  # BASELINE configs[2]: every linear Q8_0 (ISQ)
 MIXED = lambda O: dict(embd=O.Q4_K, q=O.Q8_0, k=O.Q8_0, v=O.Q8_0, o=O.Q4_K, gate=O.Q4_K, up=O.Q4_K, down=O.Q8_0, output=O.Q6_K)  # both activation formats in one model
 
