@@ -106,6 +106,15 @@ int mrs_dec_mm_supported(int type, int k, int b);
 unsigned long long mrs_dec_mm_launch_count(void); /* launches of the route since the library was loaded */
 void mrs_dec_mm_timeline(void *buf); /* experiments: [grid * 4][8] u64 s_memrealtime stamps of the following mrs_dec_mm_* launches, or NULL (off) */
 int mrs_dec_mm_proj(const void *qi, int type, int n, int k, const void *x_img, float *out, int ld_out, int mode, float resid_scale, int b, void *stream);
+/* experts of a sparse-MoE layer, b <= 8 tokens: every expert in use is read once.  ids: device int32 [b][top_k], distinct per token; stacks of `experts` tensors [n][k], n % 32 == 0;
+ * x_img: mrs_dec_act_image_rows of the b tokens (gate_up) / of the b * top_k routes (proj); outputs one row per route.  mrs_moe_fold_routes: h <- h * resid_scale + w_0 y_0, then
+ * + w_1 y_1 ... per token, in slot order (the roundings of mrs_dec_proj / mrs_dec_proj_top2 route by route). */
+int mrs_dec_mm_experts_supported(int type, int n, int k, int experts, int b, int top_k);
+int mrs_dec_mm_gate_up_experts(const void *qi_gate, const void *qi_up, int type, int n, int k, const int32_t *ids, int experts, int b, int top_k, const void *x_img, int activation,
+                               float *act_out, int ld_out, void *stream);
+int mrs_dec_mm_proj_experts(const void *qi, int type, int n, int k, const int32_t *ids, int experts, int b, int top_k, const void *x_img, float *out, int ld_out, void *stream);
+int mrs_dec_act_image_rows(const float *x, int ldx, const float *norm_w, float eps, int k, int weight_type, int rows, void *img_out, void *stream);
+int mrs_moe_fold_routes(float *h, float resid_scale, const float *y, const float *weights, int T, int d, int top_k, void *stream);
 int mrs_dec_mm_gate_up(const void *qi_gate, const void *qi_up, int type, int n, int k, const void *x_img, int activation, float *act_out, int ld_out, int b, void *stream);
 int mrs_dec_mm_qkv(const void *qi_q, int type_q, int nq, const void *qi_k, int type_k, int nk, const void *qi_v, int type_v, int nv, int k, const void *x_img, float *q_out,
                    void *k_cache, void *v_cache, const int64_t *slot_mapping, const int32_t *positions, const float *cos_t, const float *sin_t, int head_dim, int rot_pairs,

@@ -266,6 +266,7 @@ __global__ void __launch_bounds__(64 * ((G + 1) / 2)) dec_attn2_merge_kernel(con
 struct ActImgArgs {
   const float *x; int ldx; const float *norm_w; float eps; int K, mode;
   char *img;
+  int rows;           // != 0: any number of columns, an image of its own for each
   int gc0[8], gn[8];  // per column: first column and size of its group (the group's image starts at act_bytes(K, gc0))
 };
 __global__ void __launch_bounds__(NT) dec_act_image_kernel(const ActImgArgs a) {
@@ -276,7 +277,7 @@ __global__ void __launch_bounds__(NT) dec_act_image_kernel(const ActImgArgs a) {
   const ActRegs<1> pre = act_issue_all<1>(x, (unsigned)a.K * 4u, a.norm_w, a.K, wave);
   act_sumsq_all<1, 1>(red, pre, x, a.ldx, a.norm_w, a.K, wave);
   if (a.norm_w) __syncthreads();
-  const int c0 = a.gc0[c], n = a.gn[c];
+  const int c0 = a.rows ? c : a.gc0[c], n = a.rows ? 1 : a.gn[c];
   act_quantize_all<1, 1>(a.img + act_bytes(a.K, c0), red, pre, x, a.ldx, a.norm_w, a.eps, a.K, a.mode, wave, c - c0, n);
 }
 // the column groups of a batch of b columns of K values: halved until a group's image fits LDS (the same recursion as Launch::run)
@@ -506,6 +507,14 @@ extern "C" int mrs_dec_act_image(const float *x, int ldx, const float *norm_w, f
   a.x = x; a.ldx = ldx; a.norm_w = norm_w; a.eps = eps; a.K = k; a.mode = act_mode_for(weight_type); a.img = (char *)img_out;
   col_groups(k, 0, b, a.gc0, a.gn);
   hipLaunchKernelGGL(dec_act_image_kernel, dim3(b), dim3(NT), 0, (hipStream_t)stream, a);
+  return hipGetLastError() == hipSuccess ? 0 : -4;
+}
+// the same for any number of rows, row r's image alone at r * mrs_dec_act_image_bytes(k, 1): the operand rows of mrs_dec_mm_*_experts
+extern "C" int mrs_dec_act_image_rows(const float *x, int ldx, const float *norm_w, float eps, int k, int weight_type, int rows, void *img_out, void *stream) {
+  if (!x || !img_out || rows < 1 || k <= 0 || k % 256 || !dec_type(weight_type) || ((uintptr_t)img_out & 15)) return -1;
+  ActImgArgs a{};
+  a.x = x; a.ldx = ldx; a.norm_w = norm_w; a.eps = eps; a.K = k; a.mode = act_mode_for(weight_type); a.img = (char *)img_out; a.rows = rows;
+  hipLaunchKernelGGL(dec_act_image_kernel, dim3(rows), dim3(NT), 0, (hipStream_t)stream, a);
   return hipGetLastError() == hipSuccess ? 0 : -4;
 }
 // mrs_dec_qkv / mrs_dec_qkv_neox (neox != 0) on an image of RmsNorm(h) made by mrs_dec_act_image for these weights

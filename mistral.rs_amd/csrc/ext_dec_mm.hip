@@ -15,6 +15,9 @@
 //   * workgroup = 4 waves = the 4 ORD-U runs of superblocks of ONE 32-row panel at a time; the four run sums meet in LDS (double buffered: one barrier per panel),
 //     256 threads = 8 tokens x 32 rows finish ((c0 + c1) + c2) + c3 and run the phase's epilogue (store / residual / GLU / RoPE + paged-cache write).
 // The weight stream is what a launch costs: ~4.9 GB per step for the 8B Q4_K_M model whatever b is.
+// Sparse-MoE layers (MOE): a workgroup takes the panels of ONE expert that some token was routed to and multiplies them by that expert's tokens only (its columns: the routes
+// whose id is the expert's, at most one per token), so every expert's weights are read once per step instead of once per route; the workgroups are dealt to the experts in
+// use, which the kernel finds in the router's ids.
 #include "dec_gemv.cuh"
 #include <stdio.h>
 #include <stdlib.h>
@@ -46,6 +49,7 @@ struct MmArgs {
   float *out; int out_stride; float resid_scale; int activation;
   float *q_out; void *k_cache, *v_cache; const int64_t *slot_mapping; const int32_t *positions; const float *cos_t, *sin_t;
   int head_dim, rot_pairs, num_kv_heads, block_size, cache_x, kv_f16, hd_shift, bs_shift, x_shift;
+  const int32_t *ids; int nroutes, experts, route_div;  // MOE: the router's ids [nroutes <= 64] (npanels / nrows: of one expert); route r reads image row r / route_div, writes output row r
   unsigned long long *tl;  // experiments: 8 s_memrealtime stamps (100 MHz) per wave, or nullptr (mrs_dec_mm_timeline)
 };
 #ifdef MRS_MM_TIMELINE  // (a conditional store inside the streaming loop makes every wait of the ring stricter: off in the product build)
@@ -226,13 +230,13 @@ __device__ __forceinline__ void where_of(int epi, int np0, int np1, int u, int s
 // asks for the same number of loads (a cursor past its last record asks past the tensor: zeros, no traffic), so hipcc's waits come out exact (dec_core2.cuh stream()).
 template <int NPC, bool ONLY4>
 __device__ __forceinline__ void issue_rec(Rec<NPC> &slot, int &m, int &cu, int &cseg, int &ct, __amdgpu_buffer_rsrc_t rs0, __amdgpu_buffer_rsrc_t rs1, __amdgpu_buffer_rsrc_t rs2,
-                                          int ty0, int ty1, int ty2, int np0, int np1, int epi, int nseg, int units, int ntp, int p, int Cs, int S, int lane, int nn, int step) {
+                                          int ty0, int ty1, int ty2, int np0, int np1, int epi, int nseg, int units, int ntp, int p, int Cs, int S, int lane, int nn, int step, int pn0) {
   constexpr unsigned DEAD = 0xF0000000u;
   const bool live = cu < units && ntp > 0;
   int ti = 0, pn = 0;
   where_of(epi, np0, np1, live ? cu : 0, cseg, ti, pn);
   const int type = ti == 0 ? ty0 : (ti == 1 ? ty1 : ty2);
-  const unsigned rec = live ? ((unsigned)pn * (unsigned)S + (unsigned)(p * Cs + ct)) * (unsigned)rec_bytes(type) : DEAD;
+  const unsigned rec = live ? ((unsigned)(pn0 + pn) * (unsigned)S + (unsigned)(p * Cs + ct)) * (unsigned)rec_bytes(type) : DEAD;
   const __amdgpu_buffer_rsrc_t rs = ti == 0 ? rs0 : (ti == 1 ? rs1 : rs2);
   const bool small = ONLY4 || type == T_Q4_K;
   const unsigned tail = small ? 4096u : 8192u;
@@ -248,8 +252,9 @@ __device__ __forceinline__ void issue_rec(Rec<NPC> &slot, int &m, int &cu, int &
 
 // the epilogue of a finished (unit, segment): all 256 threads, thread = (token tid / 32, row tid % 32 of the panel); called behind the barrier that publishes ex[par].
 // (A plain function, not a lambda of the kernel: as a by-reference closure its stores kept every local of the kernel -- and a copy of the argument block -- in scratch memory.)
-__device__ __forceinline__ void finish_unit(const MmArgs &a, const float *ex, int par, int eu, int eseg, int tid, float &gsave) {
-  const int epi = a.epi, nc = a.nc, np0 = a.m[0].npanels, np1 = a.m[1].npanels, nr0 = a.m[0].nrows, nr1 = a.m[1].nrows, nr2 = a.m[2].nrows;
+template <bool MOE>
+__device__ __forceinline__ void finish_unit(const MmArgs &a, const float *ex, int par, int eu, int eseg, int tid, float &gsave, int nc, unsigned long long routes) {
+  const int epi = a.epi, np0 = a.m[0].npanels, np1 = a.m[1].npanels, nr0 = a.m[0].nrows, nr1 = a.m[1].nrows, nr2 = a.m[2].nrows;
 
   const int tok = tid >> 5, row = tid & 31;
   const float *e = ex + (size_t)par * 1024 + tok * 32 + row;
@@ -259,12 +264,13 @@ __device__ __forceinline__ void finish_unit(const MmArgs &a, const float *ex, in
   const int n = pn * 32 + row;
   const int nrows = ti == 0 ? nr0 : (ti == 1 ? nr1 : nr2);
   const bool ok = tok < nc && n < nrows;
-  if (epi == EPI_STORE) { if (ok) a.out[(size_t)tok * a.out_stride + n] = sum; }
+  const int orow = MOE ? (int)((routes >> (8 * tok)) & 255u) : tok;
+  if (epi == EPI_STORE) { if (ok) a.out[(size_t)orow * a.out_stride + n] = sum; }
   else if (epi == EPI_RESID) { if (ok) { float *o = a.out + (size_t)tok * a.out_stride + n; *o = *o * a.resid_scale + sum * 1.0f; } }
   else if (epi == EPI_GLU) {
     if (eseg == 0) gsave = sum;
-    else if (ok) a.out[(size_t)tok * a.out_stride + n] = (a.activation == 0 ? silu_engine(gsave) : glu_act(gsave, a.activation)) * sum;
-  } else {  // EPI_QKV, interleaved RoPE: rows 2 i, 2 i + 1 are a pair = lanes l, l ^ 1 of this wave (dec_gemv.cuh EPI_QKV, R >= 2)
+    else if (ok) a.out[(size_t)orow * a.out_stride + n] = (a.activation == 0 ? silu_engine(gsave) : glu_act(gsave, a.activation)) * sum;
+  } else if constexpr (!MOE) {  // EPI_QKV, interleaved RoPE: rows 2 i, 2 i + 1 are a pair = lanes l, l ^ 1 of this wave (dec_gemv.cuh EPI_QKV, R >= 2)
     const float other = __shfl_xor(sum, 1, 64);
     if (ok) {
       const int c = tok;
@@ -304,7 +310,7 @@ __device__ __forceinline__ void finish_unit(const MmArgs &a, const float *ex, in
   }
 }
 
-template <int TMASK>
+template <int TMASK, bool MOE>
 __device__ __forceinline__ void dec_mm_body(const MmArgs &a, char *smem) {
   constexpr bool ONLY4 = TMASK == TM_Q4K;
   constexpr int NPC = ONLY4 ? 4 : 8;
@@ -315,7 +321,30 @@ __device__ __forceinline__ void dec_mm_body(const MmArgs &a, char *smem) {
   constexpr int R = ONLY4 ? 3 : 2;
   const int tid = tid_opaque(), lane = tid & 63, p = __builtin_amdgcn_readfirstlane(tid >> 6);  // wave p = run p of the row's superblocks
   const int nn = lane & 31, hf = lane >> 5;
-  const int K = a.K, S = K / 256, Cs = (S + 3) / 4, Sp = 4 * Cs, CQ = act_cq(K), QCS = qcs_of(K), nc = a.nc;
+  const int K = a.K, S = K / 256, Cs = (S + 3) / 4, Sp = 4 * Cs, CQ = act_cq(K), QCS = qcs_of(K);
+  int nc = a.nc, unit0 = (int)blockIdx.x, ustep = (int)gridDim.x, pn0 = 0;
+  unsigned long long routes = 0, rows = 0;  // MOE: output and image row of the columns, a byte each
+  if constexpr (MOE) {  // (every wave finds the same: scalar values)
+    const int id = lane < a.nroutes ? (int)a.ids[lane] : -1;
+    int used = 0, e = -1;
+    unsigned long long mask = 0;
+    for (int i = 0; i < a.experts; ++i) used += __ballot(id == i) != 0 ? 1 : 0;
+    if (used == 0) return;
+    const int pick = (int)blockIdx.x % used;  // workgroup i works on the (i % used)-th expert in use
+    for (int i = 0, seen = 0; i < a.experts; ++i) {
+      const unsigned long long m = __ballot(id == i);
+      if (m != 0 && seen++ == pick) { mask = m; e = i; }
+    }
+    nc = min(__popcll(mask), a.nc);
+    for (int c = 0; c < nc; ++c) {
+      const int r = __ffsll((long long)mask) - 1;
+      mask &= mask - 1;
+      routes |= (unsigned long long)r << (8 * c); rows |= (unsigned long long)(r / a.route_div) << (8 * c);
+    }
+    pn0 = e * a.m[0].npanels;
+    unit0 = (int)blockIdx.x / used; ustep = ((int)gridDim.x - pick + used - 1) / used;
+    if (unit0 >= a.units) return;
+  }
   const int ntp = max(0, min(Cs, S - p * Cs));  // live superblocks of this wave's run
   char *qs = smem;
   char *ydl = smem + (size_t)nc * QCS;                                  // Q8K: [Sp][8] f32;  Q80: [Sp][8][8] f32
@@ -333,31 +362,33 @@ __device__ __forceinline__ void dec_mm_body(const MmArgs &a, char *smem) {
   const int ty0 = a.m[0].type, ty1 = a.m[1].type, ty2 = a.m[2].type;
   const int nr0 = a.m[0].nrows, nr1 = a.m[1].nrows, nr2 = a.m[2].nrows;
   const int epi = a.epi, nseg = a.nseg, units = a.units;
-  int cu = (int)blockIdx.x, cseg = 0, ct = 0;
+  int cu = unit0, cseg = 0, ct = 0;
   Rec<NPC> ring[R];
   int meta[R];  // type | ct << 8 | last << 24, or -1
   // (issue_rec / where_of are plain functions: as by-reference closures of the kernel their selects between captured variables -- which tensor's resource, type, panel
   // count -- became run-time offsets INTO the closure object, which then could not be dissolved: every local of the kernel lived in scratch memory)
   auto issue = [&](Rec<NPC> &slot, int &m) __attribute__((always_inline)) {
-    issue_rec<NPC, ONLY4>(slot, m, cu, cseg, ct, rs0, rs1, rs2, ty0, ty1, ty2, np0, np1, epi, nseg, units, ntp, p, Cs, S, lane, nn, (int)gridDim.x);
+    issue_rec<NPC, ONLY4>(slot, m, cu, cseg, ct, rs0, rs1, rs2, ty0, ty1, ty2, np0, np1, epi, nseg, units, ntp, p, Cs, S, lane, nn, ustep, pn0);
   };
   MRS_MM_TL(0);
   // ---- the activation image -> LDS (every workgroup).  The first batch of image requests leaves BEFORE the weight ring: loads return in order, the image comes out of
   // the L2 in ~1 us and is stored while the weights are still on their way from HBM (behind the ring it arrived 2.5 us later: timeline of the second GPU run)
-  auto gc0_of = [&](int c) __attribute__((always_inline)) { return (int)((a.gc0p >> (4 * c)) & 15u); };
-  auto gn_of = [&](int c) __attribute__((always_inline)) { return (int)((a.gnp >> (4 * c)) & 15u) + 1; };
+  // column c: its group's image, its place in it, the group's size (MOE: every row an image of its own)
+  auto in_grp = [&](int c) __attribute__((always_inline)) { return MOE ? 0 : c - (int)((a.gc0p >> (4 * c)) & 15u); };
+  auto gn_of = [&](int c) __attribute__((always_inline)) { return MOE ? 1 : (int)((a.gnp >> (4 * c)) & 15u) + 1; };
+  auto grp_at = [&](int c) __attribute__((always_inline)) { return (unsigned)act_bytes(K, MOE ? (int)((rows >> (8 * c)) & 255u) : (int)((a.gc0p >> (4 * c)) & 15u)); };
   // Every request of a stage leaves before the first of its values is stored (batches of up to 16 loads per lane): a load -> store loop is one memory round trip per
   // iteration (hipcc keeps them in order: both pointers are generic), 19 of them in a row at 8 columns of K = 4096 -- ~10 us in front of the first MFMA of every launch
   // (first GPU run of this file: o_proj 9.8 us at every batch size).  Requests go through ONE buffer resource over the image(s): a piece past its column asks past the
   // end (zeros, no branch).
   {
-    const unsigned img_bytes = (unsigned)act_bytes(K, nc);
+    const unsigned img_bytes = (unsigned)act_bytes(K, MOE ? (a.nroutes + a.route_div - 1) / a.route_div : nc);
     const __amdgpu_buffer_rsrc_t ri = __builtin_amdgcn_make_buffer_rsrc((void *)a.img, (short)0, (int)img_bytes, 0x00020000);
     constexpr unsigned PAST = 0xF0000000u;
     const int nv = 4 * CQ / 16;  // 16-byte pieces of a column
     // quants: wave p copies columns p and p + 4; 8 pieces of each per batch
     const int c0 = p, c1 = p + 4;
-    const unsigned s0 = (unsigned)(act_bytes(K, gc0_of(c0)) + (size_t)(c0 - gc0_of(c0)) * 4 * CQ), s1 = (unsigned)(act_bytes(K, gc0_of(c1 & 7)) + (size_t)((c1 & 7) - gc0_of(c1 & 7)) * 4 * CQ);
+    const unsigned s0 = grp_at(c0) + (unsigned)(in_grp(c0) * 4 * CQ), s1 = grp_at(c1 & 7) + (unsigned)(in_grp(c1 & 7) * 4 * CQ);
     const bool h0 = c0 < nc, h1 = c1 < nc;
     v4u r0[8], r1[8];
     auto ld_batch = [&](int j0) __attribute__((always_inline)) {
@@ -377,7 +408,7 @@ __device__ __forceinline__ void dec_mm_body(const MmArgs &a, char *smem) {
       }
     };
     // scales and run sums: item -> (superblock, column[, ...]); up to 8 items per thread and batch
-    auto col_base = [&](int c) __attribute__((always_inline)) { return (unsigned)(act_bytes(K, gc0_of(c)) + (size_t)gn_of(c) * 4 * CQ); };  // the group's d region
+    auto col_base = [&](int c) __attribute__((always_inline)) { return grp_at(c) + (unsigned)(gn_of(c) * 4 * CQ); };  // the group's d region
     const bool q80 = a.mode == ACT_Q80;
     const int nsc = q80 ? Sp * 64 : Sp * 32;  // Q80: block scales, image d [ncols][Sp][12] f32 (8 + pad) -> yd8 [sb][block][token];  Q8K: four run sums per item, the
                                               // superblock scale rides along (items with r4 == 0)
@@ -389,11 +420,11 @@ __device__ __forceinline__ void dec_mm_body(const MmArgs &a, char *smem) {
         if (q80) {
           const int sb = i >> 6, g = (i >> 3) & 7, c = i & 7;
           bq[j] = v4u{0u, 0u, 0u, 0u};
-          dv[j] = __builtin_amdgcn_raw_buffer_load_b32(ri, c < nc && i < nsc ? col_base(c) + (unsigned)(((c - gc0_of(c)) * Sp + sb) * 12 + g) * 4u : PAST, 0, 0);
+          dv[j] = __builtin_amdgcn_raw_buffer_load_b32(ri, c < nc && i < nsc ? col_base(c) + (unsigned)((in_grp(c) * Sp + sb) * 12 + g) * 4u : PAST, 0, 0);
         } else {
           const int sb = i >> 5, c = (i >> 2) & 7, r4 = i & 3;
           const bool ok = c < nc && i < nsc;
-          const unsigned db = col_base(c), cb = (unsigned)((c - gc0_of(c)) * Sp + sb);
+          const unsigned db = col_base(c), cb = (unsigned)(in_grp(c) * Sp + sb);
           bq[j] = __builtin_amdgcn_raw_buffer_load_b128(ri, ok ? db + (unsigned)gn_of(c) * (unsigned)Sp * 4u + (cb * ACT_BS + 4u * r4) * 4u : PAST, 0, 0);
           dv[j] = __builtin_amdgcn_raw_buffer_load_b32(ri, ok && r4 == 0 ? db + cb * 4u : PAST, 0, 0);
         }
@@ -437,10 +468,10 @@ __device__ __forceinline__ void dec_mm_body(const MmArgs &a, char *smem) {
   const char *qlane = qs + (size_t)tcol * QCS + (size_t)p * CQ;
   float acc[4] = {0.f, 0.f, 0.f, 0.f};
   float gsave = 0.f;
-  int eu = (int)blockIdx.x, eseg = 0, par = 0;  // the (unit, segment) whose run sums are being collected
+  int eu = unit0, eseg = 0, par = 0;  // the (unit, segment) whose run sums are being collected
   auto finish = [&]() __attribute__((always_inline)) {
-    finish_unit(a, ex, par, eu, eseg, tid, gsave);
-    if (++eseg == nseg) { eseg = 0; eu += (int)gridDim.x; }
+    finish_unit<MOE>(a, ex, par, eu, eseg, tid, gsave, nc, routes);
+    if (++eseg == nseg) { eseg = 0; eu += ustep; }
     par ^= 1;
   };
   auto publish = [&](const float (&v)[4]) __attribute__((always_inline)) {  // this wave's run sums of the finished (unit, segment) -> ex[par][p][token][row]
@@ -488,12 +519,22 @@ __device__ __forceinline__ void dec_mm_body(const MmArgs &a, char *smem) {
 // three and funnels every MFMA of a record through one accumulator tuple (exposed MFMA latency x 9 per record).
 __global__ void __launch_bounds__(MT) MRS_MM_WAVES_PER_EU(2, 2) dec_mm_kernel_q4k(const MmArgs a) {
   extern __shared__ __attribute__((aligned(16))) char smem[];
-  dec_mm_body<TM_Q4K>(a, smem);
+  dec_mm_body<TM_Q4K, false>(a, smem);
 }
 template <int TMASK>
 __global__ void __launch_bounds__(MT) MRS_MM_WAVES_PER_EU(1, 2) dec_mm_kernel(const MmArgs a) {
   extern __shared__ __attribute__((aligned(16))) char smem[];
-  dec_mm_body<TMASK>(a, smem);
+  dec_mm_body<TMASK, false>(a, smem);
+}
+// the experts of a sparse-MoE layer (one type per launch)
+__global__ void __launch_bounds__(MT) MRS_MM_WAVES_PER_EU(2, 2) dec_mm_experts_kernel_q4k(const MmArgs a) {
+  extern __shared__ __attribute__((aligned(16))) char smem[];
+  dec_mm_body<TM_Q4K, true>(a, smem);
+}
+template <int TMASK>
+__global__ void __launch_bounds__(MT) MRS_MM_WAVES_PER_EU(1, 2) dec_mm_experts_kernel(const MmArgs a) {
+  extern __shared__ __attribute__((aligned(16))) char smem[];
+  dec_mm_body<TMASK, true>(a, smem);
 }
 static unsigned long long *g_mm_tl = nullptr;
 static unsigned long long g_mm_launches = 0;  // launches of this route since the library was loaded (tests: did a batched step really take it?)
@@ -514,13 +555,19 @@ static int launch(const MmArgs &a0, hipStream_t s) {
   static const int wg_per_cu = [] { const char *e = getenv("MRS_DEC_MM_WG_PER_CU"); return e ? std::max(1, atoi(e)) : 2; }();
   const int fit = (tmask == TM_Q4K || tmask == TM_Q5K || tmask == TM_Q80) ? 2 : 1;  // workgroups per CU the kernel's registers admit (see the kernels above)
   const int cap = 256 * std::min<int>(std::min(wg_per_cu, fit), std::max<size_t>(1, ((size_t)160 * 1024) / lds));
-  const int grid = std::min(a.units, cap);
+  const int grid = std::min(a.units * (a.ids ? std::min(a.experts, a.nroutes) : 1), cap);
   auto go = [&](auto kern) {
     ++g_mm_launches;
     lds_attr_once((const void *)kern, 158 * 1024);
     hipLaunchKernelGGL(kern, dim3(grid), dim3(MT), lds, s, a);
     return hipGetLastError() == hipSuccess ? 0 : -4;
   };
+  if (a.ids) switch (tmask) {
+  case TM_Q4K: return go(dec_mm_experts_kernel_q4k);
+  case TM_Q5K: return go(dec_mm_experts_kernel<TM_Q5K>);
+  case TM_Q6K: return go(dec_mm_experts_kernel<TM_Q6K>);
+  default: return go(dec_mm_experts_kernel<TM_Q80>);
+  }
   switch (tmask) {
   case TM_Q4K: return go(dec_mm_kernel_q4k);
   case TM_Q6K: return go(dec_mm_kernel<TM_Q6K>);
@@ -596,4 +643,34 @@ extern "C" int mrs_dec_mm_qkv(const void *qi_q, int type_q, int nq, const void *
   a.hd_shift = lg2(head_dim); a.bs_shift = lg2(block_size); a.x_shift = lg2(a.cache_x);
   if (a.hd_shift < 0 || a.bs_shift < 0 || head_dim < a.cache_x || rot_pairs < 1) return -1;
   return launch(a, (hipStream_t)stream);
+}
+// ---- the experts of a sparse-MoE layer, b tokens with top_k distinct ids each (device int32 ids [b][top_k]); tensors are stacks of `experts` tensors [n][k] (n % 32 == 0)
+extern "C" int mrs_dec_mm_experts_supported(int type, int n, int k, int experts, int b, int top_k) {
+  return mrs_dec_mm_supported(type, k, b) && n > 0 && n % 32 == 0 && experts > 0 && top_k > 0 && b * top_k <= 64 &&
+         (size_t)experts * (n / 32) * (size_t)(k / 256) * rec_bytes(type) < 0xF0000000ull ? 1 : 0;
+}
+static int experts_launch(MmArgs &a, const void *const *qi, int type, int n, int k, const int32_t *ids, int experts, int b, int top_k, int route_div, const void *x_img, float *out,
+                          int ld_out, void *stream) {
+  if (!ids || !out || !mrs_dec_mm_experts_supported(type, n, k, experts, b, top_k) || !base(a, x_img, k, b, type)) return -1;
+  for (int i = 0; i < a.nseg; ++i) {
+    if (!set_tensor(a.m[i], qi[i], type, (long long)experts * n, k)) return -1;
+    a.m[i].npanels = n / 32; a.m[i].nrows = n;
+  }
+  a.units = n / 32; a.out = out; a.out_stride = ld_out; a.ids = ids; a.nroutes = b * top_k; a.experts = experts; a.route_div = route_div;
+  return launch(a, (hipStream_t)stream);
+}
+// act_out [b * top_k][ld_out] = act(W_g[e] . x) * (W_u[e] . x), e = ids[route], x = image row route / top_k of x_img (mrs_dec_act_image_rows of the b tokens)
+extern "C" int mrs_dec_mm_gate_up_experts(const void *qi_gate, const void *qi_up, int type, int n, int k, const int32_t *ids, int experts, int b, int top_k, const void *x_img,
+                                          int activation, float *act_out, int ld_out, void *stream) {
+  MmArgs a{};
+  const void *qi[2] = {qi_gate, qi_up};
+  a.epi = EPI_GLU; a.nseg = 2; a.activation = activation;
+  return experts_launch(a, qi, type, n, k, ids, experts, b, top_k, top_k, x_img, act_out, ld_out, stream);
+}
+// out [b * top_k][ld_out] = W[e] . x, e = ids[route], x = image row `route` of x_img (mrs_dec_act_image_rows of the b * top_k rows)
+extern "C" int mrs_dec_mm_proj_experts(const void *qi, int type, int n, int k, const int32_t *ids, int experts, int b, int top_k, const void *x_img, float *out, int ld_out,
+                                       void *stream) {
+  MmArgs a{};
+  a.epi = EPI_STORE; a.nseg = 1;
+  return experts_launch(a, &qi, type, n, k, ids, experts, b, top_k, 1, x_img, out, ld_out, stream);
 }

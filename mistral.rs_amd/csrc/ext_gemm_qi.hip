@@ -699,11 +699,12 @@ __global__ void __launch_bounds__(256) qi_gather_rows_kernel(const char *__restr
 __global__ void __launch_bounds__(256) moe_fold_exact_kernel(float *__restrict__ h, float rs, const float *__restrict__ y, const int *__restrict__ inv, const float *__restrict__ w,
                                                             int d, int tk) {
   const int t = blockIdx.x;
-  for (int n = threadIdx.x * 4; n < d; n += 1024) {
+  for (int n = (blockIdx.y * 256 + threadIdx.x) * 4; n < d; n += gridDim.y * 1024) {
     float4 v = *(const float4 *)(h + (size_t)t * d + n);
     for (int sl = 0; sl < tk; ++sl) {
       const float ws = w[(size_t)t * tk + sl], sc = sl == 0 ? rs : 1.0f;
-      const float4 yy = *(const float4 *)(y + (size_t)inv[(size_t)t * tk + sl] * d + n);
+      const size_t route = (size_t)t * tk + sl;
+      const float4 yy = *(const float4 *)(y + (inv ? (size_t)inv[route] : route) * d + n);
       v.x = v.x * sc + yy.x * ws; v.y = v.y * sc + yy.y * ws; v.z = v.z * sc + yy.z * ws; v.w = v.w * sc + yy.w * ws;
     }
     *(float4 *)(h + (size_t)t * d + n) = v;
@@ -733,6 +734,12 @@ extern "C" int mrs_qi_gather_rows(int w_type, const void *act_src, int T, void *
 extern "C" int mrs_moe_fold_exact(float *h, float resid_scale, const float *y_sorted, const int *inv, const float *weights, int T, int d, int top_k, void *stream) {
   if (!h || !y_sorted || !inv || !weights || T <= 0 || d <= 0 || d % 4 || top_k <= 0) return -1;
   hipLaunchKernelGGL(qi::moe_fold_exact_kernel, dim3(T), dim3(256), 0, (hipStream_t)stream, h, resid_scale, y_sorted, inv, weights, d, top_k);
+  return 0;
+}
+// the same on rows in route order (a decode step: few tokens, a row over several workgroups)
+extern "C" int mrs_moe_fold_routes(float *h, float resid_scale, const float *y, const float *weights, int T, int d, int top_k, void *stream) {
+  if (!h || !y || !weights || T <= 0 || d <= 0 || d % 4 || top_k <= 0) return -1;
+  hipLaunchKernelGGL(qi::moe_fold_exact_kernel, dim3(T, (d + 1023) / 1024), dim3(256), 0, (hipStream_t)stream, h, resid_scale, y, (const int *)nullptr, weights, d, top_k);
   return 0;
 }
 extern "C" int mrs_resid_scale_add_f32(float *h, float resid_scale, const float *y, size_t n, void *stream) {

@@ -158,3 +158,59 @@ def test_mm_store_gate_up_qkv_gpu(oracle, dev):
     check_mm_qkv(oracle, be, "Q4_K", "Q6_K", 32, 8, 4096, 8)
     check_mm_qkv(oracle, be, "Q4_K", "Q4_K", 32, 8, 4096, 4, kvd=0)
     check_mm_qkv(oracle, be, "Q8_0", "Q8_0", 8, 2, 2048, 2)
+
+
+def check_mm_experts(O, be, tname, tdown, ff, d, E, b, tk, ids):
+    """mrs_dec_mm_gate_up_experts == mrs_dec_mm_gate_up of each token on its expert's slice; mrs_dec_mm_proj_experts == the engine-order oracle; mrs_moe_fold_routes == slot by slot."""
+    VP, CI, CF = C.c_void_p, C.c_int, C.c_float
+    t, td, R = getattr(O, tname), getattr(O, tdown), b * tk
+    pg, pu, pd = _weights(O, t, E * ff, d, 71), _weights(O, t, E * ff, d, 72), _weights(O, td, E * d, ff, 73)
+    qg, qu, qd = qi_repack(be, t, pg, E * ff, d), qi_repack(be, t, pu, E * ff, d), qi_repack(be, td, pd, E * d, ff)
+    rng = np.random.default_rng(74)
+    x, nw = rng.standard_normal((b, d)).astype(np.float32), (1.0 + 0.1 * rng.standard_normal(d)).astype(np.float32)
+    xb, nb, idb = be.buf(x), be.buf(nw), be.buf(np.asarray(ids, np.int32).reshape(b, tk))
+    isz = be.sym("mrs_dec_act_image_bytes", [CI, CI], C.c_size_t)
+    rows_img = be.sym("mrs_dec_act_image_rows", [VP, CI, VP, CF, CI, CI, CI, VP, VP], CI)
+    ok = be.sym("mrs_dec_mm_experts_supported", [CI] * 6, CI)
+    assert ok(t, ff, d, E, b, tk) == 1 and ok(t, ff + 1, d, E, b, tk) == 0 and ok(t, ff, d, E, 9, tk) == 0
+    img, act = be.buf(np.zeros(isz(d, b), np.uint8)), be.buf(np.full((R, ff), np.nan, np.float32))
+    assert rows_img(xb.ptr, d, nb.ptr, 1e-5, d, t, b, img.ptr, be.stream) == 0
+    assert be.sym("mrs_dec_mm_gate_up_experts", [VP, VP, CI, CI, CI, VP, CI, CI, CI, VP, CI, VP, CI, VP], CI)(qg.ptr, qu.ptr, t, ff, d, idb.ptr, E, b, tk, img.ptr, 0, act.ptr, ff,
+                                                                                                             be.stream) == 0
+    a = act.numpy()
+    per = be.sym("mrs_gemm_qi_repack_bytes", [CI, C.c_longlong, C.c_longlong], C.c_size_t)(t, ff, d)
+    glu = be.sym("mrs_dec_mm_gate_up", MM_GLU, CI)
+    for r in range(R):
+        one, e = be.buf(np.zeros((1, ff), np.float32)), ids[r]
+        assert glu(qg.ptr + e * per, qu.ptr + e * per, t, ff, d, img.ptr + (r // tk) * isz(d, 1), 0, one.ptr, ff, 1, be.stream) == 0
+        assert np.array_equal(a[r], one.numpy()[0]) and np.count_nonzero(a[r]) > 0, r
+    img2, y = be.buf(np.zeros(isz(ff, R), np.uint8)), be.buf(np.full((R, d), np.nan, np.float32))
+    assert rows_img(act.ptr, ff, None, 0.0, ff, td, R, img2.ptr, be.stream) == 0
+    assert be.sym("mrs_dec_mm_proj_experts", [VP, CI, CI, CI, VP, CI, CI, CI, VP, VP, CI, VP], CI)(qd.ptr, td, d, ff, idb.ptr, E, b, tk, img2.ptr, y.ptr, d, be.stream) == 0
+    yn = y.numpy()
+    for r in range(R):
+        assert np.array_equal(yn[r], O.gemv_engine(td, pd.reshape(E, d, -1)[ids[r]], d, ff, a[r])[0]), r
+    h, w = rng.standard_normal((b, d)).astype(np.float32), rng.random((b, tk)).astype(np.float32)
+    hb, wb = be.buf(h.copy()), be.buf(w)
+    assert be.sym("mrs_moe_fold_routes", [VP, CF, VP, VP, CI, CI, CI, VP], CI)(hb.ptr, 0.5, y.ptr, wb.ptr, b, d, tk, be.stream) == 0
+    want = h
+    for s in range(tk):
+        want = want * np.float32(0.5 if s == 0 else 1.0) + yn.reshape(b, tk, d)[:, s] * w[:, s:s + 1]
+    assert np.array_equal(hb.numpy(), want)
+
+
+# all tokens on one pair of experts (8 columns), every route on an expert of its own, experts without tokens, one token
+EXPERTS = [("Q4_K", "Q6_K", 256, 256, 4, 8, 2, [1, 3] * 8), ("Q4_K", "Q4_K", 256, 512, 8, 4, 2, [0, 1, 2, 3, 4, 5, 7, 6]), ("Q5_K", "Q8_0", 256, 256, 3, 1, 1, [2]),
+           ("Q8_0", "Q5_K", 256, 256, 5, 3, 3, [4, 0, 1, 0, 4, 3, 1, 4, 0]), ("Q6_K", "Q4_K", 512, 256, 6, 5, 2, [0, 1, 0, 2, 5, 0, 2, 1, 0, 5])]
+
+
+@pytest.mark.parametrize("case", EXPERTS)
+def test_mm_experts_host_emulation(oracle, case):
+    check_mm_experts(oracle, HostBackend(), *case)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("case", [("Q4_K", "Q6_K", 14336, 1024, 8, 5, 2, [0, 1, 0, 2, 5, 0, 2, 1, 0, 5]), ("Q4_K", "Q4_K", 2048, 4096, 8, 8, 2, [7, 6] * 4 + [1, 2, 1, 0, 3, 7, 5, 4]),
+                                  ("Q8_0", "Q5_K", 512, 768, 5, 3, 3, [4, 0, 1, 0, 4, 3, 1, 4, 0])])
+def test_mm_experts_gpu(oracle, dev, case):
+    check_mm_experts(oracle, GpuBackend(dev), *case)
