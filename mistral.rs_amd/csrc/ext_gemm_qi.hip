@@ -143,25 +143,41 @@ struct QuantArgs {
   int mode;     // ACT_Q8K (K-quant weights) / ACT_Q80 (Q8_0 weights: quantize_row_q8_0 per 32 values; outputs q8 [S][T][256] int8 in element order at `qf`, the block
                 // scales f32(f16(d)) block-major [S][8][T] at `bsf`)
 };
-template <bool GLU>
+// GLU: 0: the row as it is; 1: silu_engine(g) * u formed in the registers the quantizer reads (rows of up to 2048 NPX values, no norm); 2: the same through xtmp.  Form 2 wrote
+// and re-read the row: 512 / 1999 tokens of 14336 values 26 / 85 us.
+template <int GLU>
 __global__ void __launch_bounds__(NT) qi_quantize_kernel(const QuantArgs a) {
   extern __shared__ __attribute__((aligned(16))) char smem[];
   __shared__ float red[8];
   const int tid = tid_opaque(), t = blockIdx.x, K = a.K, S = K / 256;
-  const float *xr = a.x + (size_t)t * a.ldx;
-  if constexpr (GLU) {
-    float *dst = a.xtmp + (size_t)t * K;
-    const float *ur = a.x2 + (size_t)t * a.ldx;
-    for (int e = tid * 4; e < K; e += NT * 4) {
-      const float4 g = *(const float4 *)(xr + e), u = *(const float4 *)(ur + e);
-      *(float4 *)(dst + e) = make_float4(silu_engine(g.x) * u.x, silu_engine(g.y) * u.y, silu_engine(g.z) * u.z, silu_engine(g.w) * u.w);
-    }
-    __syncthreads();  // the same threads read back what they wrote (tid * 4 + j * 2048), the barrier orders the other waves' view of nothing: cheap insurance
-    xr = dst;
-  }
+  const float *xr = a.x + (size_t)t * a.ldx, *ur = GLU ? a.x2 + (size_t)t * a.ldx : nullptr;
+  auto glu4 = [](float4 g, float4 u) { return make_float4(silu_engine(g.x) * u.x, silu_engine(g.y) * u.y, silu_engine(g.z) * u.z, silu_engine(g.w) * u.w); };
   const int qw = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const ActRegs<1> pre = act_issue_all<1>(xr, (unsigned)K * 4u, a.norm_w, K, qw);
-  act_finish_all<1>(smem, red, pre, xr, K, a.norm_w, a.eps, K, a.mode, qw);
+  if constexpr (GLU == 1) {
+    ActRegs<1> pre{};
+    float4 g[NPX], u[NPX];
+    const __amdgpu_buffer_rsrc_t rg = __builtin_amdgcn_make_buffer_rsrc((void *)xr, (short)0, K * 4, 0x00020000), ru = __builtin_amdgcn_make_buffer_rsrc((void *)ur, (short)0, K * 4, 0x00020000);
+#pragma unroll
+    for (int j = 0; j < NPX; ++j) {  // past the row: zeros
+      g[j] = as_f4(__builtin_amdgcn_raw_buffer_load_b128(rg, (unsigned)tid * 16u + (unsigned)j * 8192u, 0, 0));
+      u[j] = as_f4(__builtin_amdgcn_raw_buffer_load_b128(ru, (unsigned)tid * 16u + (unsigned)j * 8192u, 0, 0));
+    }
+#pragma unroll
+    for (int j = 0; j < NPX; ++j) {
+      const float4 v = glu4(g[j], u[j]);
+      pre.xv[0][j] = v4u{__float_as_uint(v.x), __float_as_uint(v.y), __float_as_uint(v.z), __float_as_uint(v.w)};
+    }
+    act_finish_all<1>(smem, red, pre, xr, K, nullptr, a.eps, K, a.mode, qw);
+  } else {
+    if constexpr (GLU == 2) {
+      float *dst = a.xtmp + (size_t)t * K;
+      for (int e = tid * 4; e < K; e += NT * 4) *(float4 *)(dst + e) = glu4(*(const float4 *)(xr + e), *(const float4 *)(ur + e));
+      __syncthreads();  // the same threads read back what they wrote (tid * 4 + j * 2048), the barrier orders the other waves' view of nothing: cheap insurance
+      xr = dst;
+    }
+    const ActRegs<1> pre = act_issue_all<1>(xr, (unsigned)K * 4u, a.norm_w, K, qw);
+    act_finish_all<1>(smem, red, pre, xr, K, a.norm_w, a.eps, K, a.mode, qw);
+  }
   __syncthreads();
   const Act act = act_view(smem, K, 1, a.mode);
   if (a.mode == ACT_Q80) {
@@ -526,16 +542,19 @@ __global__ void __launch_bounds__(256, NT == 1 && TYPE != T_Q5_K ? 3 : 2) gemm_q
     }
 }
 
-// out[t][n] (+)= ((c0 + c1) + c2) + c3 of the four run sums (the row combination of ORD-U)
-__global__ void __launch_bounds__(256) gemm_qi_reduce_kernel(const float *__restrict__ part, float *__restrict__ out, int T, int N, int ldo, int accumulate, int part_n) {
-  const size_t i = ((size_t)blockIdx.x * 256 + threadIdx.x) * 4, tot = (size_t)T * part_n;  // `part`: the tensor's first column of the launch's [4][T][part_n] sums
-  if (i >= (size_t)T * N) return;
-  const float *pp = part + (i / N) * part_n + i % N;
+// out[t][n] (+)= ((c0 + c1) + c2) + c3 of the four run sums (the row combination of ORD-U), all tensors of the launch: workgroup (row t, 1024 of its columns).  One launch per
+// tensor cost 3 - 5 us each at short prompts (7 of a layer's 16 launches at 37 tokens).
+__global__ void __launch_bounds__(256) gemm_qi_reduce_kernel(const WideArgs a) {
+  const int t = blockIdx.x, c = (blockIdx.y * 256 + threadIdx.x) * 4;
+  if (c >= a.part_n) return;
+  const size_t tot = (size_t)a.T * a.part_n;
+  const float *pp = a.part + (size_t)t * a.part_n + c;
   const float4 c0 = *(const float4 *)pp, c1 = *(const float4 *)(pp + tot), c2 = *(const float4 *)(pp + 2 * tot), c3 = *(const float4 *)(pp + 3 * tot);
   float4 r = make_float4(((c0.x + c1.x) + c2.x) + c3.x, ((c0.y + c1.y) + c2.y) + c3.y, ((c0.z + c1.z) + c2.z) + c3.z, ((c0.w + c1.w) + c2.w) + c3.w);
-  const size_t t = i / N, n = i % N;  // N % 4 == 0: the four values share a row
-  float4 *o = (float4 *)(out + t * ldo + n);
-  if (accumulate) { const float4 old = *o; r.x = old.x + r.x; r.y = old.y + r.y; r.z = old.z + r.z; r.w = old.w + r.w; }
+  const int n1 = a.s0.N, n2 = n1 + a.s1.N;  // every N is a multiple of 4: the four values share a row of one tensor
+  float *out = c < n1 ? a.s0.out + (size_t)t * a.s0.ldo + c : c < n2 ? a.s1.out + (size_t)t * a.s1.ldo + (c - n1) : a.s2.out + (size_t)t * a.s2.ldo + (c - n2);
+  float4 *o = (float4 *)out;
+  if (a.accumulate) { const float4 old = *o; r.x = old.x + r.x; r.y = old.y + r.y; r.z = old.z + r.z; r.w = old.w + r.w; }
   *o = r;
 }
 
@@ -588,8 +607,10 @@ extern "C" int mrs_qi_quantize_for(int w_type, const float *x, const float *x2, 
   qi_split(act, T, K, &a.qf, &a.yd, &a.bsf);
   const size_t lds = (dec2::act_bytes(K, 1) + 15) & ~(size_t)15;
   if (lds > 158 * 1024) return -2;
-  if (x2) { auto kern = qi::qi_quantize_kernel<true>; lds_attr_once((const void *)kern, 158 * 1024); hipLaunchKernelGGL(kern, dim3(T), dim3(dec2::NT), lds, (hipStream_t)stream, a); }
-  else { auto kern = qi::qi_quantize_kernel<false>; lds_attr_once((const void *)kern, 158 * 1024); hipLaunchKernelGGL(kern, dim3(T), dim3(dec2::NT), lds, (hipStream_t)stream, a); }
+  auto go = [&](auto kern) { lds_attr_once((const void *)kern, 158 * 1024); hipLaunchKernelGGL(kern, dim3(T), dim3(dec2::NT), lds, (hipStream_t)stream, a); };
+  if (!x2) go(qi::qi_quantize_kernel<0>);
+  else if (K <= 2048 * dec2::NPX && !norm_w) go(qi::qi_quantize_kernel<1>);
+  else go(qi::qi_quantize_kernel<2>);
   return 0;
 }
 // out[t * ldo + n] (+)= W[n] . act[t] for t < T, n < N in the decode engine's arithmetic and f32 order.  w_qi: mrs_gemm_qi_repack output; act: mrs_qi_quantize output.
@@ -635,9 +656,6 @@ extern "C" int mrs_gemm_qi_multi(int type, int nt, const void *const *w_qi, cons
   _Float16 *qf, *bsf; float *yd;
   qi_split((void *)act, T, K, &qf, &yd, &bsf);
   const bool split_ok = !bounds && K / 256 >= 4 && mult4 && workspace && workspace_bytes >= (size_t)4 * T * n_all * 4;
-  auto reduce = [&](const float *part, int i, int part_n) {
-    hipLaunchKernelGGL(qi::gemm_qi_reduce_kernel, dim3((unsigned)(((size_t)T * N[i] / 4 + 255) / 256)), dim3(256), 0, s, part, out[i], T, N[i], ldo[i], accumulate, part_n);
-  };
   // Token tiles per wave.  K-quants: 32 rows fill one; from 33 rows on two waste little and build each operand once for both (us, one / two tiles: Q4_K 28672 x 4096 28 / 38 at
   // 20 rows, 37 / 37 at 37, 221 / 199 at 512;  Q6_K 4096 x 14336 32 / 38 at 20 rows, 33 / 38 at 37, 161 / 129 at 512, 570 / 457 at 1999).  Q8_0 has no operand to build and a
   // smaller workgroup's registers let one more live on a CU (q / k / v 95 / 141 and gate / up 348 / 376 at 700 rows, gate / up 1012 / 1079 at 1999).
@@ -660,7 +678,7 @@ extern "C" int mrs_gemm_qi_multi(int type, int nt, const void *const *w_qi, cons
     case T_Q6_K: wide_launch<T_Q6_K>(NT, a, grid, s); break;
     default: wide_launch<T_Q8_0>(NT, a, grid, s); break;
   }
-  for (int i = 0, c = 0; i < nt && a.ksplit > 1; c += N[i++]) reduce(a.part + c, i, n_all);
+  if (a.ksplit > 1) hipLaunchKernelGGL(qi::gemm_qi_reduce_kernel, dim3(T, (n_all + 1023) / 1024), dim3(256), 0, s, a);
   return 0;
 }
 

@@ -156,6 +156,21 @@ def test_mfma_f16_accumulates_small_integers_exactly(dev):
     assert np.array_equal(got, ref) and ref[0, 0] == -16515072
 
 
+# silu(g) * u rows: the largest row formed in registers and one past it, for both image formats
+GLU_K = [("Q4_K", 14336), ("Q8_0", 14336), ("Q6_K", 14592)]
+
+
+@pytest.mark.parametrize("tname,k", GLU_K)
+def test_gemm_qi_glu_long_rows_host_emulation(oracle, tname, k):
+    run_gemm(oracle, HostBackend(), tname, 32, k, 3, 0, glu=True, seed=5)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("tname,k", GLU_K)
+def test_gemm_qi_glu_long_rows_gpu(oracle, dev, tname, k):
+    run_gemm(oracle, GpuBackend(dev), tname, 64, k, 5, 0, glu=True, seed=5)
+
+
 def run_multi(O, be, tname, ns, k, T, bounds=None, ws=False, acc=False, seed=0):
     """mrs_gemm_qi_multi: several tensors on the same operand rows; with `bounds` every tensor is a stack whose expert e takes the rows bounds[e] .. bounds[e + 1] - 1."""
     t = getattr(O, tname)
