@@ -11,6 +11,7 @@ reference CPU path (oracle/llama_ref.py + oracle/cpu_path_oracle.c).  Round 3: t
     implementation that does not reproduce one specific build's summation order; the tests hold the engine to the spread that two CPU orders show
     on the same model and tokens (factor 1.25 on the means), and to the size of one moved quant (3e-2) on the tiny model.
 KV pages: f16 (the reference CPU path's default KV dtype) and bf16 (the dtype of the GPU pipelines), each against the oracle with the same KV rounding."""
+import ctypes as C
 import os
 import numpy as np
 import pytest
@@ -508,6 +509,27 @@ def test_engine_mixtral_moe_vs_cpu_path_oracle(oracle, dev, request):
     from oracle import llama_ref
     cfg, w, m, cos, sin = _mk(oracle, dev, types, "bf16", experts=4)
     _vs_exact(m, cfg, w, cos, sin, "bf16", steps, "moe", check=steps >= 10, factor=1.1)  # 24 positions of a 4-expert toy: 1.046 x on the restatement
+
+
+@pytest.mark.parametrize("b", [2, 3, 4])
+def test_engine_mixtral_batched_steps_equal_single_ones(oracle, dev, b):
+    """A batched step multiplies every expert by all of its tokens at once; each sequence's logits are those of its own batch-1 steps, bit for bit."""
+    types = dict(embd=oracle.Q4_K, q=oracle.Q4_K, k=oracle.Q4_K, v=oracle.Q6_K, o=oracle.Q4_K, gate=oracle.Q4_K, up=oracle.Q4_K, down=oracle.Q6_K, output=oracle.Q6_K)
+    _, _, m, _, _ = _mk(oracle, dev, types, "bf16", experts=4, max_batch=4)
+    _, _, one, _, _ = _mk(oracle, dev, types, "bf16", experts=4, max_batch=1)
+    ids = np.random.default_rng(b).integers(0, 512, (2, b)).tolist()
+    count = m._L.mrs_dec_mm_launch_count
+    count.restype = C.c_ulonglong
+    for pos in range(2):
+        m.set_state(ids[pos], [pos] * b)
+        before = count()
+        got = m.forward_logits(b).clone()
+        assert count() > before  # the grouped launches did run
+    for i in range(b):
+        for pos in range(2):
+            one.set_state([ids[pos][i]], [pos])
+            want = one.forward_logits(1)[0].clone()
+        assert (got[i] == want).all(), i
 
 
 @pytest.mark.gpu
