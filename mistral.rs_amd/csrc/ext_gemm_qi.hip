@@ -315,11 +315,13 @@ __global__ void __launch_bounds__(256, NT == 1 && TYPE != T_Q5_K ? 3 : 2) gemm_q
     }
   };
   const int n = (int)panel * 32 + nn;
+  // sums start at -0: adding to it changes no value, so a run's first term and a row's first run need no case of their own (a factor of 0 on the run before would carry its
+  // infinity over as NaN)
   float run[NT][16], pend[NT][16];
 #pragma unroll
   for (int tt = 0; tt < NT; ++tt)
 #pragma unroll
-    for (int v = 0; v < 16; ++v) { run[tt][v] = 0.f; pend[tt][v] = 0.f; }
+    for (int v = 0; v < 16; ++v) { run[tt][v] = -0.f; pend[tt][v] = -0.f; }
   const int sb_begin = a.ksplit > 1 ? (int)blockIdx.z * Cs : 0, sb_end = a.ksplit > 1 ? min(S, sb_begin + Cs) : S;
   // outputs through bounded buffers that begin at the tile's first row: a lane holds column n, rows 32 tt + 8 (v / 4) + 4 hf + v % 4; a buffer ends behind the window's
   // last row, columns past N are pushed out of it
@@ -404,7 +406,7 @@ __global__ void __launch_bounds__(256, NT == 1 && TYPE != T_Q5_K ? 3 : 2) gemm_q
 #pragma unroll
       for (int tt = 0; tt < NT; ++tt)
 #pragma unroll
-        for (int v = 0; v < 16; ++v) run[tt][v] = (sb % Cs) == 0 ? Tt[tt][v] : run[tt][v] + Tt[tt][v];
+        for (int v = 0; v < 16; ++v) run[tt][v] = run[tt][v] + Tt[tt][v];
     } else {
     // ---- the weight operand of a run (16 values of 32 rows x 16 / 8 of the K order per lane) as exact small integers in f16, from packed integer and f16 instructions:
     //   Q4_K  sc (q - 8) = (64 + q) sc - 72 sc      (q at bits 7:4 of a half-word: 0x5400 = 64, one unit per 16 mantissa steps; 9 sc < 2^11)
@@ -482,7 +484,6 @@ __global__ void __launch_bounds__(256, NT == 1 && TYPE != T_Q5_K ? 3 : 2) gemm_q
       }
     }
     const float *yd_s = (const float *)meta_s;
-    const float keep = (sb % Cs) == 0 ? 0.f : 1.f;  // the first term of a run of superblocks starts its sum (0 * run + t), the others add (1 * run + t: exact)
     const f32v zero32 = {0.f};
     // d yd (and dmin yd) of the tile's outputs, each product rounded once: one matrix instruction of two 32 x 32 outer products (lane halves = blocks)
     const float dd = half_bits_to_float((uint16_t)(hf ? hd >> 16 : hd & 0xffff));
@@ -494,7 +495,7 @@ __global__ void __launch_bounds__(256, NT == 1 && TYPE != T_Q5_K ? 3 : 2) gemm_q
 #pragma unroll
         for (int v = 0; v < 16; ++v) {
           const float If = fmaf(16.0f, X[1][tt][v], X[0][tt][v]);  // (float)isum: one rounding of the exact integer
-          run[tt][v] = fmaf(run[tt][v], keep, dy[v] * If);
+          run[tt][v] = run[tt][v] + dy[v] * If;
         }
         __builtin_amdgcn_sched_barrier(0);
       }
@@ -519,25 +520,24 @@ __global__ void __launch_bounds__(256, NT == 1 && TYPE != T_Q5_K ? 3 : 2) gemm_q
           if constexpr (TYPE == T_Q4_K) If = fmaf(8.0f, Sx[v], X[0][tt][v]);
           else If = (float)(((int)X[0][tt][v] + (int)X[NX - 1][tt][v]) + 16 * (int)Sx[v]);
           const float t = fmaf(dy[v], If, -(dy[16 + v] * M[v]));
-          run[tt][v] = fmaf(run[tt][v], keep, t);
+          run[tt][v] = run[tt][v] + t;
         }
         __builtin_amdgcn_sched_barrier(0);  // one token tile at a time: the sums of all of them would not fit the registers
       }
     }
     }
     if ((sb + 1) % Cs == 0 || sb + 1 == sb_end) {  // a run of superblocks ends: its sum joins the row's left-to-right combination
-      const bool first = sb < Cs;
 #pragma unroll
       for (int tt = 0; tt < NT; ++tt)
 #pragma unroll
-        for (int v = 0; v < 16; ++v) pend[tt][v] = first ? run[tt][v] : pend[tt][v] + run[tt][v];
+        for (int v = 0; v < 16; ++v) { pend[tt][v] = pend[tt][v] + run[tt][v]; run[tt][v] = -0.f; }
     }
   }
 #pragma unroll
   for (int tt = 0; tt < NT; ++tt)
 #pragma unroll
     for (int v = 0; v < 16; ++v) {
-      if (split) st32(run[tt][v], ro, at(tt, v));  // one run per workgroup: combined by gemm_qi_reduce_kernel
+      if (split) st32(pend[tt][v], ro, at(tt, v));  // one run per workgroup: combined by gemm_qi_reduce_kernel
       else st32(a.accumulate ? ld32(ro, at(tt, v)) + pend[tt][v] : pend[tt][v], ro, at(tt, v));
     }
 }

@@ -246,3 +246,53 @@ def test_long_rows_cut_by_runs_equal_the_whole_launch(oracle, dev, tname, T):
             wq.ptr, t, n, k, act.ptr, T, o.ptr, n, 0, w.ptr if w else None, 4 * T * n * 4 if w else 0, be.stream) == 0
         got.append(o.numpy())
     assert got[0].any() and np.array_equal(got[0], got[1])
+
+
+def run_overflow(O, be, tname, T):
+    """A run of superblocks whose sum is +-inf: the runs behind it start from nothing (0 * inf would be NaN), whole and cut by runs, as in the decode engine's GEMV.
+    Four runs of one superblock; the first overflows f32 in every other row (K-quants: activations of 1e37; Q8_0, whose scales are f16: an infinite weight scale in every row)."""
+    t, n, k = getattr(O, tname), 36, 1024
+    rng = np.random.default_rng(11)
+    p = O.quantize(t, (rng.standard_normal((n, k)) * 40.0).astype(np.float32)).reshape(n, 4, -1)
+    x = rng.standard_normal((T, k)).astype(np.float32)
+    if tname == "Q8_0":
+        p[:, 0, 0:2] = np.frombuffer(np.float16(np.inf).tobytes(), np.uint8)
+    else:
+        x[::2, :256] *= np.float32(1e37)
+    if tname in ("Q4_K", "Q5_K"):
+        p[:, 0, 2:4] = 0  # dmin: the difference of two infinities is NaN in any order
+    p = p.reshape(n, -1)
+    want = np.concatenate([O.gemv_engine(t, p, n, k, r) for r in x], axis=0)
+    assert not np.isnan(want).any() and np.isinf(want[::2]).mean() > 0.9 and (tname == "Q8_0" or np.isfinite(want[1::2]).all())
+    for cut in (False, True):
+        got = gemm_rows(O, be, t, p, n, k, x, cut)
+        assert np.array_equal(got, want), (tname, cut, int(np.isnan(got).sum()))
+
+
+def gemm_rows(O, be, t, p, n, k, x, cut, ws_off=0, ldo=None):
+    """mrs_gemm_qi_ws on the rows x, with a workspace for the run sums (cut) or without; the first n columns of the output"""
+    T, ldo = len(x), ldo or n
+    src, wq = be.buf(np.ascontiguousarray(p).reshape(-1)), be.buf(np.zeros(be.sym("mrs_gemm_qi_repack_bytes", [CI, C.c_longlong, C.c_longlong], C.c_size_t)(t, n, k), np.uint8))
+    assert be.sym("mrs_gemm_qi_repack", [VP, CI, C.c_longlong, C.c_longlong, VP, VP], CI)(src.ptr, t, n, k, wq.ptr, be.stream) == 0
+    xb, act = be.buf(np.ascontiguousarray(x)), be.buf(np.zeros(be.sym("mrs_qi_act_bytes", [CI, CI], C.c_size_t)(T, k), np.uint8))
+    assert be.sym("mrs_qi_quantize_for", [CI, VP, VP, CI, VP, C.c_float, CI, CI, VP, VP, VP], CI)(t, xb.ptr, None, k, None, 1e-5, T, k, act.ptr, None, be.stream) == 0
+    ws, o = be.buf(np.zeros(4 * T * n + 8, np.float32)), be.buf(np.full((T, ldo), 7.0, np.float32))
+    assert be.sym("mrs_gemm_qi_ws", [VP, CI, CI, CI, VP, CI, VP, CI, CI, VP, C.c_size_t, VP], CI)(wq.ptr, t, n, k, act.ptr, T, o.ptr, ldo, 0, ws.ptr + ws_off if cut else None,
+                                                                                                 4 * T * n * 4 if cut else 0, be.stream) == 0
+    got = o.numpy()
+    assert (got[:, n:] == 7.0).all()
+    return got[:, :n]
+
+
+OVERFLOW = [("Q4_K", 5), ("Q4_K", 33), ("Q5_K", 34), ("Q6_K", 33), ("Q8_0", 5)]
+
+
+@pytest.mark.parametrize("tname,T", OVERFLOW)
+def test_gemm_qi_infinite_run_host_emulation(oracle, tname, T):
+    run_overflow(oracle, HostBackend(), tname, T)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("tname,T", OVERFLOW)
+def test_gemm_qi_infinite_run_gpu(oracle, dev, tname, T):
+    run_overflow(oracle, GpuBackend(dev), tname, T)
