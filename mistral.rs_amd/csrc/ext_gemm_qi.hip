@@ -622,7 +622,8 @@ extern "C" int mrs_gemm_qi(const void *w_qi, int type, int N, int K, const void 
   return mrs_gemm_qi_ws(w_qi, type, N, K, act, T, out, ldo, accumulate, nullptr, 0, stream);
 }
 // mrs_gemm_qi_multi: up to three tensors of one type that multiply the same operand rows, in one launch where the kernel takes segments.  bounds != NULL (device
-// [experts + 1]): every tensor is a stack of `experts` tensors and expert e multiplies (and writes) the rows [bounds[e], bounds[e + 1]); max_rows (host) bounds one expert's rows.
+// [experts + 1]): every tensor is a stack of `experts` tensors [N][K] (N a multiple of 32 where there are several) and expert e multiplies (and writes) the rows [bounds[e], bounds[e + 1]);
+// max_rows (host) bounds one expert's rows.
 extern "C" int mrs_gemm_qi_multi(int type, int nt, const void *const *w_qi, const int *N, int K, const void *act, int T, float *const *out, const int *ldo, int accumulate,
                                  const int *bounds, int experts, int max_rows, void *workspace, size_t workspace_bytes, void *stream);
 extern "C" int mrs_gemm_qi_win(const void *w_qi, int type, int N, int K, const void *act, int T_total, const int *win, int max_rows, float *out, int ldo, int accumulate, void *stream) {
@@ -647,7 +648,7 @@ extern "C" int mrs_gemm_qi_multi(int type, int nt, const void *const *w_qi, cons
   int n_all = 0;
   bool mult4 = true;
   for (int i = 0; i < nt; ++i) {
-    if (!w_qi[i] || !out[i] || N[i] <= 0) return -1;
+    if (!w_qi[i] || !out[i] || N[i] <= 0 || (bounds && experts > 1 && N[i] % 32)) return -1;  // an expert of a stack begins at a panel of 32 rows
     if (qi::qi_tensor_bytes(type, N[i], K) >= 0xffffff00ull) return -2;
     n_all += N[i]; mult4 = mult4 && N[i] % 4 == 0;
   }

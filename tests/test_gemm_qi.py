@@ -296,3 +296,23 @@ def test_gemm_qi_infinite_run_host_emulation(oracle, tname, T):
 @pytest.mark.parametrize("tname,T", OVERFLOW)
 def test_gemm_qi_infinite_run_gpu(oracle, dev, tname, T):
     run_overflow(oracle, GpuBackend(dev), tname, T)
+
+
+def multi_call(O, be, ns, k, T, bounds, experts, max_rows):
+    """mrs_gemm_qi_multi on buffers of zeros that are large enough for the call: its return code"""
+    t = O.Q4_K
+    w = [be.buf(np.zeros(be.sym("mrs_gemm_qi_repack_bytes", [CI, C.c_longlong, C.c_longlong], C.c_size_t)(t, experts * (n + 31) // 32 * 32, k), np.uint8)) for n in ns]
+    o = [be.buf(np.zeros((T, n), np.float32)) for n in ns]
+    act, bb = be.buf(np.zeros(be.sym("mrs_qi_act_bytes", [CI, CI], C.c_size_t)(T, k), np.uint8)), be.buf(np.asarray(bounds, np.int32))
+    ptrs = lambda bufs: (VP * len(ns))(*[b.ptr for b in bufs])  # noqa: E731
+    return be.sym("mrs_gemm_qi_multi", [CI, CI, VP, VP, CI, VP, CI, VP, VP, CI, VP, CI, CI, VP, C.c_size_t, VP], CI)(
+        t, len(ns), ptrs(w), (CI * len(ns))(*ns), k, act.ptr, T, ptrs(o), (CI * len(ns))(*ns), 0, bb.ptr, experts, max_rows, None, 0, be.stream)
+
+
+def test_stacks_whose_experts_share_a_panel_are_refused_host_emulation(oracle):
+    """The repack cuts a stack into panels of 32 rows: where an expert's rows are no multiple of 32, the next one begins inside a panel."""
+    be = HostBackend()
+    assert multi_call(oracle, be, (40,), 512, 20, (0, 7, 20), 2, 20) == -1
+    assert multi_call(oracle, be, (64, 40), 512, 20, (0, 7, 20), 2, 20) == -1
+    assert multi_call(oracle, be, (64, 32), 512, 20, (0, 7, 20), 2, 20) == 0
+    assert multi_call(oracle, be, (40,), 512, 20, (0, 20), 1, 20) == 0  # one expert: nothing behind it
