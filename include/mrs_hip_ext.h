@@ -290,7 +290,7 @@ int mrs_prefill_attention_exact_ws(const float *q, const void *k_cache, const vo
 int mrs_qi_quantize_for(int w_ggml_type, const float *x, const float *x2, int ldx, const float *norm_w, float eps, int T, int K, void *act, float *xtmp, void *stream);
 /* mrs_gemm_qi_multi: up to three tensors of one type that multiply the same operand rows (q / k / v, gate / up), in one launch where the kernel takes segments.  bounds != NULL
  * (device ints [experts + 1]): every tensor is a stack of `experts` tensors [N][K] (N % 32 == 0 where experts > 1: the copy's panels have 32 rows; else -1), expert e multiplies
- * and writes the rows [bounds[e], bounds[e + 1]); max_rows bounds one expert's rows */
+ * and writes the rows [bounds[e], bounds[e + 1]); max_rows bounds one expert's rows and sizes the grid */
 int mrs_gemm_qi_multi(int ggml_type, int n_tensors, const void *const *w_qi, const int *N, int K, const void *act, int T, float *const *out, const int *ldo, int accumulate,
                       const int *bounds, int experts, int max_rows, void *workspace, size_t workspace_bytes, void *stream);
 int mrs_gemm_qi_win(const void *w_qi, int ggml_type, int N, int K, const void *act, int T_total, const int *win, int max_rows, float *out, int ldo, int accumulate, void *stream);

@@ -623,7 +623,7 @@ extern "C" int mrs_gemm_qi(const void *w_qi, int type, int N, int K, const void 
 }
 // mrs_gemm_qi_multi: up to three tensors of one type that multiply the same operand rows, in one launch where the kernel takes segments.  bounds != NULL (device
 // [experts + 1]): every tensor is a stack of `experts` tensors [N][K] (N a multiple of 32 where there are several) and expert e multiplies (and writes) the rows [bounds[e], bounds[e + 1]);
-// max_rows (host) bounds one expert's rows.
+// max_rows (host) bounds one expert's rows, and with them the grid and the token tiles of a wave.
 extern "C" int mrs_gemm_qi_multi(int type, int nt, const void *const *w_qi, const int *N, int K, const void *act, int T, float *const *out, const int *ldo, int accumulate,
                                  const int *bounds, int experts, int max_rows, void *workspace, size_t workspace_bytes, void *stream);
 extern "C" int mrs_gemm_qi_win(const void *w_qi, int type, int N, int K, const void *act, int T_total, const int *win, int max_rows, float *out, int ldo, int accumulate, void *stream) {
@@ -660,14 +660,16 @@ extern "C" int mrs_gemm_qi_multi(int type, int nt, const void *const *w_qi, cons
   // Token tiles per wave.  K-quants: 32 rows fill one; from 33 rows on two waste little and build each operand once for both (us, one / two tiles: Q4_K 28672 x 4096 28 / 38 at
   // 20 rows, 37 / 37 at 37, 221 / 199 at 512;  Q6_K 4096 x 14336 32 / 38 at 20 rows, 33 / 38 at 37, 161 / 129 at 512, 570 / 457 at 1999).  Q8_0 has no operand to build and a
   // smaller workgroup's registers let one more live on a CU (q / k / v 95 / 141 and gate / up 348 / 376 at 700 rows, gate / up 1012 / 1079 at 1999).
-  const int NT = type == T_Q8_0 || (bounds ? T / experts : T) <= 32 ? 1 : 2, tl = 32 * NT;
+  max_rows = bounds ? std::min(max_rows, T) : T;
+  const int NT = type == T_Q8_0 || (bounds ? std::min(T / experts, max_rows) : T) <= 32 ? 1 : 2, tl = 32 * NT;
   qi::WideArgs a{};
   qi::QiSeg *sg[3] = {&a.s0, &a.s1, &a.s2};
   int gx = 0, x[3] = {0, 0, 0};
   for (int i = 0; i < nt; ++i) { *sg[i] = qi::QiSeg{(const uint8_t *)w_qi[i], (unsigned)qi::qi_tensor_bytes(type, N[i], K), N[i], out[i], ldo[i]}; gx += (N[i] + qi::WIDE_ROWS - 1) / qi::WIDE_ROWS; x[i] = gx; }
   a.x1 = x[0]; a.x2 = nt > 1 ? x[1] : gx;
   a.K = K; a.T = T; a.qf = qf; a.yd = yd; a.bsf = bsf; a.accumulate = accumulate; a.part = (float *)workspace; a.part_n = n_all; a.bounds = bounds; a.experts = experts; a.ksplit = 1;
-  dim3 grid(gx, bounds ? T / tl + experts : (T + tl - 1) / tl);
+  // windows: every expert's last tile may be partly filled, and none has more tiles than max_rows fill
+  dim3 grid(gx, bounds ? std::min(T / tl + experts, experts * ((max_rows + tl - 1) / tl)) : (T + tl - 1) / tl);
   // Two (NT = 2) or three workgroups fit a CU.  Below 512 the launch is cut by runs of superblocks (4096 x 14336 Q4_K at 512 rows, 256 workgroups: 119 us whole, 102 us cut).
   // Long rows also where a second, partly filled round of workgroups would take as long as the first (K = 14336, whole / cut: Q4_K 1600 rows 314 / 287 us, Q6_K 430 / 392,
   // Q8_0 512 rows 175 / 129, 700 rows 194 / 168, 1000 rows 233 / 239; one full round, Q4_K 1024 rows: 178 / 191; K = 4096 at 1300 rows 90 / 97).
@@ -687,7 +689,7 @@ extern "C" int mrs_gemm_qi_multi(int type, int nt, const void *const *w_qi, cons
 // The decode step of a sparse-MoE layer (host/runtime.cpp forward_engine; SparseMoeBlock::forward, models/mixtral.rs:280-304) multiplies ONE token's quantized row by its
 // top-k experts' gate / up rows, quantizes silu(g) * u per expert slot, multiplies by that expert's down rows and folds the slots into the residual stream in slot order:
 // h <- (h * rs + w_0 s_0) * 1 + w_1 s_1 ...  A prompt does the same per token through the grouped form of the exact GEMM: the tokens' operand rows are gathered into
-// expert-sorted order (launch_moe_dispatch's table), every expert multiplies its window of rows (mrs_gemm_qi_win), and the fold below restores slot order per token.
+// expert-sorted order (launch_moe_dispatch's table), every expert multiplies its window of rows (mrs_gemm_qi_multi), and the fold below restores slot order per token.
 namespace mrs {
 namespace qi {
 // operand rows of `src` (T rows) -> `dst` (R rows): dst row r = src row sorted[r] / tk (sorted == nullptr: r / tk ... unused); inv[sorted[r]] = r.  One workgroup per row r.

@@ -316,3 +316,50 @@ def test_stacks_whose_experts_share_a_panel_are_refused_host_emulation(oracle):
     assert multi_call(oracle, be, (64, 40), 512, 20, (0, 7, 20), 2, 20) == -1
     assert multi_call(oracle, be, (64, 32), 512, 20, (0, 7, 20), 2, 20) == 0
     assert multi_call(oracle, be, (40,), 512, 20, (0, 20), 1, 20) == 0  # one expert: nothing behind it
+
+
+def run_win(O, be, tname, n, k, T, win, max_rows, seed=0):
+    """mrs_gemm_qi_win: the window's rows are the decode engine's GEMV of those rows, the others stay as they are"""
+    t = getattr(O, tname)
+    rng = np.random.default_rng(seed)
+    p = O.quantize(t, (rng.standard_normal((n, k)) * 0.05).astype(np.float32)).reshape(n, -1)
+    x, base = rng.standard_normal((T, k)).astype(np.float32), rng.standard_normal((T, n)).astype(np.float32)
+    src, wq = be.buf(np.ascontiguousarray(p).reshape(-1)), be.buf(np.zeros(be.sym("mrs_gemm_qi_repack_bytes", [CI, C.c_longlong, C.c_longlong], C.c_size_t)(t, n, k), np.uint8))
+    assert be.sym("mrs_gemm_qi_repack", [VP, CI, C.c_longlong, C.c_longlong, VP, VP], CI)(src.ptr, t, n, k, wq.ptr, be.stream) == 0
+    xb, act = be.buf(x), be.buf(np.zeros(be.sym("mrs_qi_act_bytes", [CI, CI], C.c_size_t)(T, k), np.uint8))
+    assert be.sym("mrs_qi_quantize_for", [CI, VP, VP, CI, VP, C.c_float, CI, CI, VP, VP, VP], CI)(t, xb.ptr, None, k, None, 1e-5, T, k, act.ptr, None, be.stream) == 0
+    wb, o = be.buf(np.asarray(win, np.int32)), be.buf(base.copy())
+    fn = be.sym("mrs_gemm_qi_win", [VP, CI, CI, CI, VP, CI, VP, CI, VP, CI, CI, VP], CI)
+    assert fn(wq.ptr, t, n, k, act.ptr, T, wb.ptr, max_rows, o.ptr, n, 0, be.stream) == 0
+    want = base.copy()
+    for r in range(*win):
+        want[r] = O.gemv_engine(t, p, n, k, x[r])[0]
+    assert np.array_equal(o.numpy(), want)
+    assert fn(wq.ptr, t, n, k, act.ptr, T, wb.ptr, 0, o.ptr, n, 0, be.stream) == -1 and fn(wq.ptr, t, n, k, act.ptr, T, wb.ptr, T + 1, o.ptr, n, 0, be.stream) == -1
+
+
+# windows of a wave's one tile and of more, an empty one, one that ends with the operand rows
+WIN = [("Q4_K", 40, 512, 100, (33, 53), 20), ("Q4_K", 64, 512, 100, (10, 100), 90), ("Q6_K", 64, 512, 70, (69, 70), 1), ("Q5_K", 33, 512, 70, (5, 5), 7), ("Q8_0", 40, 512, 70, (1, 66), 65)]
+
+
+@pytest.mark.parametrize("case", WIN)
+def test_gemm_qi_window_host_emulation(oracle, case):
+    run_win(oracle, HostBackend(), *case, seed=6)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("case", WIN)
+def test_gemm_qi_window_gpu(oracle, dev, case):
+    run_win(oracle, GpuBackend(dev), *case, seed=6)
+
+
+def test_grid_of_a_window_follows_its_bound_host_emulation(oracle):
+    """max_rows sizes the grid: tiles past it have no workgroup.  The window names 64 rows more than max_rows allows; with a grid over all operand rows they would be written."""
+    be = HostBackend()
+    t, n, k, T = oracle.Q4_K, 32, 256, 96
+    wq, act, o = be.buf(np.zeros(be.sym("mrs_gemm_qi_repack_bytes", [CI, C.c_longlong, C.c_longlong], C.c_size_t)(t, n, k), np.uint8)), \
+        be.buf(np.zeros(be.sym("mrs_qi_act_bytes", [CI, CI], C.c_size_t)(T, k), np.uint8)), be.buf(np.full((T, n), 7.0, np.float32))
+    wb = be.buf(np.asarray((0, T), np.int32))
+    assert be.sym("mrs_gemm_qi_win", [VP, CI, CI, CI, VP, CI, VP, CI, VP, CI, CI, VP], CI)(wq.ptr, t, n, k, act.ptr, T, wb.ptr, 32, o.ptr, n, 0, be.stream) == 0
+    got = o.numpy()
+    assert (got[:32] == 0).all() and (got[32:] == 7.0).all()
