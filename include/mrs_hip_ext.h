@@ -274,7 +274,7 @@ int mrs_prefill_attention_exact(const float *q, const void *k_cache, const void 
                                 int num_heads, int num_kv_heads, int head_size, int block_size, int q_stride, int kv_block_stride, int kv_head_stride, float scale,
                                 int max_context_len, int kv_dtype, int sliding_window, int max_prompt_ctx /* largest context_lens[t], or 0 */, void *stream);
 /* the same with a workspace for the probabilities (any size from one query tile's slots on; mrs_prefill_attention_workspace_bytes: one group, or 256 MiB): same bits, scores
- * formed once.  Too small or NULL: mrs_prefill_attention_exact. */
+ * formed once.  Used from its first 16-byte boundary on; too small or NULL: mrs_prefill_attention_exact.  Both return -1 for max_context_len <= 0. */
 size_t mrs_prefill_attention_workspace_bytes(int T, int num_heads, int max_context_len);
 int mrs_prefill_attention_exact_ws(const float *q, const void *k_cache, const void *v_cache, const uint32_t *block_table, const uint32_t *context_lens, float *out, int T,
                                    int num_heads, int num_kv_heads, int head_size, int block_size, int q_stride, int kv_block_stride, int kv_head_stride, float scale,

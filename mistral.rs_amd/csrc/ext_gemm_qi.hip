@@ -1345,6 +1345,7 @@ extern "C" int mrs_prefill_attention_exact_ws(const float *q, const void *k_cach
                                               float scale, int max_context_len, int kv_dtype, int sliding_window, int max_prompt_ctx, void *workspace, size_t workspace_bytes,
                                               void *stream) {
   if (!q || !out || head_size != 128 || block_size != 32 || T <= 0 || num_kv_heads <= 0 || num_heads % num_kv_heads || (kv_dtype != 0 && kv_dtype != 1)) return -1;
+  if (max_context_len <= 0) return -1;  // no slots, no splits
   const int G = num_heads / num_kv_heads;
   if (G != 1 && G != 2 && G != 4 && G != 8) return -1;
   mrs::dec::AttnArgs a{};
@@ -1361,13 +1362,15 @@ extern "C" int mrs_prefill_attention_exact_ws(const float *q, const void *k_cach
   static const int use_mfma = [] { const char *e = getenv("MRS_PREFILL_ATTN_MFMA"); return e ? atoi(e) : 1; }();
   {
     const int nb = (need_ctx + 31) / 32, tiles = (T + 31) / 32;
-    const size_t pair = (size_t)nb * mrs::qi::PS_SLOT, fit = workspace ? workspace_bytes / pair : 0;  // (head, tile) pairs per launch
+    char *const slots = (char *)(((uintptr_t)workspace + 15) & ~(uintptr_t)15);  // a slot's rows are stored 8 and read 16 bytes at a time
+    const size_t off = (size_t)(slots - (char *)workspace), have = workspace && workspace_bytes > off ? workspace_bytes - off : 0;
+    const size_t pair = (size_t)nb * mrs::qi::PS_SLOT, fit = have / pair;  // (head, tile) pairs per launch
     if (use_mfma && fit > 0) {
       const int ht = (int)std::min<size_t>(num_heads, fit / tiles), hgroups = ht ? (num_heads + ht - 1) / ht : num_heads;
       const int hs = (num_heads + hgroups - 1) / hgroups, ts = ht ? tiles : (int)std::min<size_t>(tiles, fit);
       for (int h0 = 0; h0 < num_heads; h0 += hs)
         for (int t0 = 0; t0 < tiles; t0 += ts) {
-          mrs::qi::PrefillWs w{(char *)workspace, nb, h0, std::min(hs, num_heads - h0), t0, 1};
+          mrs::qi::PrefillWs w{slots, nb, h0, std::min(hs, num_heads - h0), t0, 1};
           const int nt = std::min(ts, tiles - t0), splits = (nb + a.bpw - 1) / a.bpw;
           // splits per wave: more where there are waves enough without (the queries are read once for all, a wave's next keys arrive under its instructions), few enough
           // that the last round of workgroups stays short.  Scores, us, of 1 / 2 / 4 / 8 per wave: 512 tokens - 26.8 / 24.8, 1999 tokens (16 heads) - / 113.2 / 113.3 / 120.5

@@ -99,6 +99,37 @@ def test_prompt_attention_with_a_workspace_gpu(oracle, dev, case):
     check_attention_ws(oracle, GpuBackend(dev), *case)
 
 
+def test_prompt_attention_workspace_edges_host_emulation(oracle):
+    """A model context below 1 is refused (a query tile's slots have no bytes: a division by zero).  A workspace off a 16-byte boundary is used from the next one on."""
+    be, heads, T, hd, bs, max_ctx = HostBackend(), 2, 33, 128, 32, 64
+    nq = heads * hd
+    rng = np.random.default_rng(1)
+    kc, vc = (be.buf(oracle.to_bf16_bits(rng.standard_normal((2, heads, hd * bs)).astype(np.float32))) for _ in range(2))
+    q, bt, cl = be.buf(rng.standard_normal((T, nq)).astype(np.float32)), be.buf(np.arange(2, dtype=np.uint32)), be.buf(np.arange(1, T + 1, dtype=np.uint32))
+    pair = be.sym("mrs_prefill_attention_workspace_bytes", [CI, CI, CI], C.c_size_t)(1, 1, T)
+    call = be.sym("mrs_prefill_attention_exact_ws", PA[:-1] + [VP, C.c_size_t, VP], CI)
+
+    def run(ctx_bound, ws, size):
+        o = be.buf(np.full((T, nq), np.nan, np.float32))
+        rc = call(q.ptr, kc.ptr, vc.ptr, bt.ptr, cl.ptr, o.ptr, T, heads, heads, hd, bs, nq, heads * hd * bs, hd * bs, np.float32(hd ** -0.5), ctx_bound, 1, 0, T, ws, size, be.stream)
+        return rc, o.numpy()
+
+    rc, want = run(max_ctx, None, 0)
+    assert rc == 0 and np.isfinite(want).all()
+    buf = be.buf(np.full(pair // 4 + 8, 7.0, np.float32))  # one (head, tile) pair and 32 bytes
+    for off in (0, 4, 8, 12):
+        buf.fill(7.0)
+        rc, got = run(max_ctx, buf.ptr + off, pair + 16)
+        base = (-(buf.ptr + off)) % 16 + off
+        assert rc == 0 and np.array_equal(got, want) and (buf.numpy()[:base // 4] == 7.0).all() and buf.numpy()[base // 4] != 7.0
+    rc, got = run(max_ctx, buf.ptr + 4, pair)  # one pair, less what the boundary takes: no slots
+    assert rc == 0 and np.array_equal(got, want)
+    o = be.buf(np.zeros((T, nq), np.float32))
+    for bound in (0, -40):
+        for ws, size in ((buf.ptr, pair), (None, 0)):
+            assert call(q.ptr, kc.ptr, vc.ptr, bt.ptr, cl.ptr, o.ptr, T, heads, heads, hd, bs, nq, heads * hd * bs, hd * bs, np.float32(1), bound, 1, 0, 0, ws, size, be.stream) == -1
+
+
 Q80 = lambda O: dict(embd=O.Q8_0, q=O.Q8_0, k=O.Q8_0, v=O.Q8_0, o=O.Q8_0, gate=O.Q8_0, up=O.Q8_0, down=O.Q8_0, output=O.Q8_0)  # BASELINE configs[2]: every linear Q8_0 (ISQ)
 MIXED = lambda O: dict(embd=O.Q4_K, q=O.Q8_0, k=O.Q8_0, v=O.Q8_0, o=O.Q4_K, gate=O.Q4_K, up=O.Q4_K, down=O.Q8_0, output=O.Q6_K)  # both activation formats in one model
 
