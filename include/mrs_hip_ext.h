@@ -126,12 +126,13 @@ int mrs_hqq_gemv(int bits, int dtype, const void *wq, const void *scale, const v
                  int N, int K, int b, void *stream);
 /* quantized (or f32/f16/bf16) embedding rows -> f32; role of QuantMethod::embedding_forward (lib.rs:1561, gguf/mod.rs:436) */
 int mrs_embedding(const void *table, int type, const int32_t *ids, float *out, int K, int tokens, void *stream);
+/* the decode state of b sequences (token ids, positions = HOST arrays, passed in the launch) -> input_ids, positions, context_lens = position + 1, slot_mapping by the block table;
+ * -1: arguments (b above 64, a negative position), -4: the launch failed */
+int mrs_set_state(const int32_t *ids, const int32_t *pos, int b, int32_t *input_ids, int32_t *positions, uint32_t *context_lens, int64_t *slot_mapping,
+                  const uint32_t *block_tables, int max_blocks, int block_size, void *stream);
 /* round 6, greedy batch-1 step: the arg-max of lm_head folded into its epilogue (mrs_dec_proj_argmax: one u64 packed (value, index) maximum, zero before the launch) and
  * ONE launch that turns it into the next id, advances the device-resident decode state (mrs_sample_greedy_advance's updates) and gathers the next id's embedding row into
  * h_next (mrs_embedding's values) -- the role of sample_cuda_top1_row (mistralrs-core/src/ops.rs:2206) + the next step's embedding lookup. */
-/* the decode state of b sequences (token ids, positions = HOST arrays, passed in the launch) -> input_ids, positions, context_lens = position + 1, slot_mapping by the block table */
-int mrs_set_state(const int32_t *ids, const int32_t *pos, int b, int32_t *input_ids, int32_t *positions, uint32_t *context_lens, int64_t *slot_mapping,
-                  const uint32_t *block_tables, int max_blocks, int block_size, void *stream);
 int mrs_sample_advance_embed(int32_t *next_ids, int32_t *tokens_out, int tokens_out_stride, int32_t *step_counter, int32_t *positions, uint32_t *context_lens,
                              int64_t *slot_mapping, const uint32_t *block_tables, int max_blocks, int block_size, void *scratch, const void *table, int type, float *h_next,
                              int K, void *stream);

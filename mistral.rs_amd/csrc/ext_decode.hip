@@ -826,7 +826,6 @@ extern "C" int mrs_quantize_rows_q8_1(const float *x, void *y, int K, int stride
   return 0;
 }
 
-// batch 1, the maximum already in scratch[0] (mrs_dec_proj_argmax): next id, state advance and h_next = embedding row of the next id (mrs_embedding's values)
 // ids / pos: HOST arrays [b]; the rest device buffers of at least b entries (block_tables [b][max_blocks])
 extern "C" int mrs_set_state(const int32_t *ids, const int32_t *pos, int b, int32_t *input_ids, int32_t *positions, uint32_t *context_lens, int64_t *slot_mapping,
                              const uint32_t *block_tables, int max_blocks, int block_size, void *stream) {
@@ -838,8 +837,9 @@ extern "C" int mrs_set_state(const int32_t *ids, const int32_t *pos, int b, int3
   a.input_ids = input_ids; a.positions = positions; a.context_lens = context_lens; a.slot_mapping = slot_mapping; a.block_tables = block_tables;
   a.b = b; a.max_blocks = max_blocks; a.block_size = block_size;
   hipLaunchKernelGGL(set_state_kernel, dim3(1), dim3(64), 0, (hipStream_t)stream, a);
-  return 0;
+  return hipGetLastError() == hipSuccess ? 0 : -4;
 }
+// batch 1, the maximum already in scratch[0] (mrs_dec_proj_argmax): next id, state advance and h_next = embedding row of the next id (mrs_embedding's values)
 extern "C" int mrs_sample_advance_embed(int32_t *next_ids, int32_t *tokens_out, int tokens_out_stride, int32_t *step_counter, int32_t *positions, uint32_t *context_lens,
                                         int64_t *slot_mapping, const uint32_t *block_tables, int max_blocks, int block_size, void *scratch, const void *table, int type,
                                         float *h_next, int K, void *stream) {

@@ -397,8 +397,11 @@ class Llama:
             raise ValueError(f"{b} sequences, the model was made for {cfg.max_batch}")
         ids = np.ascontiguousarray(token_ids, dtype=np.int32)
         pos = np.ascontiguousarray(np.broadcast_to(pos, (b,)), dtype=np.int32)
-        self._chk(self._L.mrs_set_state(ids.ctypes.data, pos.ctypes.data, b, self.input_ids.data_ptr(), self.positions.data_ptr(), self.context_lens.data_ptr(),
-                                        self.slot_mapping.data_ptr(), self.block_tables.data_ptr(), self.block_tables.shape[1], cfg.block_size, self._stream()))
+        self._state_pos = None
+        rc = self._L.mrs_set_state(ids.ctypes.data, pos.ctypes.data, b, self.input_ids.data_ptr(), self.positions.data_ptr(), self.context_lens.data_ptr(),
+                                   self.slot_mapping.data_ptr(), self.block_tables.data_ptr(), self.block_tables.shape[1], cfg.block_size, self._stream())
+        if rc:
+            raise RuntimeError(f"the decode state could not be set ({rc})")
         # what replay() would read back, unless `positions` is written to in between (an inference tensor does not count its writes: read it back)
         self._state_pos = None if self.positions.is_inference() else pos
         self._state_version = None if self._state_pos is None else self.positions._version

@@ -47,7 +47,8 @@ typedef void *hipStream_t;
 typedef int hipError_t;
 enum { hipSuccess = 0 };
 enum hipFuncAttribute { hipFuncAttributeMaxDynamicSharedMemorySize = 8 };
-static inline hipError_t hipGetLastError() { return hipSuccess; }
+extern "C" { inline int hiphost_next_error = 0; }  // a test of an error path sets it: what the next hipGetLastError() returns (and clears)
+static inline hipError_t hipGetLastError() { const int e = hiphost_next_error; hiphost_next_error = 0; return (hipError_t)e; }
 static inline hipError_t hipMemset(void *p, int v, size_t n) { memset(p, v, n); return hipSuccess; }  // "device" memory is host memory
 enum { hipDeviceMallocUncached = 3, hipDeviceMallocFinegrained = 1 };
 static inline hipError_t hipExtMallocWithFlags(void **p, size_t n, unsigned) { *p = malloc(n); return *p ? hipSuccess : (hipError_t)2; }
