@@ -395,8 +395,13 @@ class Llama:
             raise ValueError("negative position")
         if b > cfg.max_batch:
             raise ValueError(f"{b} sequences, the model was made for {cfg.max_batch}")
-        ids = np.ascontiguousarray(token_ids, dtype=np.int32)
-        pos = np.ascontiguousarray(np.broadcast_to(pos, (b,)), dtype=np.int32)
+
+        def row(a):  # what assigning `a` to b entries of a tensor takes: leading axes of length 1, one value for all
+            while a.ndim > 1 and a.shape[0] == 1:
+                a = a[0]
+            return np.ascontiguousarray(a if a.shape == (b,) else np.broadcast_to(a, (b,)), dtype=np.int32)
+
+        ids, pos = row(np.asarray(token_ids, dtype=np.int32)), row(pos)
         self._state_pos = None
         rc = self._L.mrs_set_state(ids.ctypes.data, pos.ctypes.data, b, self.input_ids.data_ptr(), self.positions.data_ptr(), self.context_lens.data_ptr(),
                                    self.slot_mapping.data_ptr(), self.block_tables.data_ptr(), self.block_tables.shape[1], cfg.block_size, self._stream())

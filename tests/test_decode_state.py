@@ -37,3 +37,33 @@ def test_set_state_raises_when_its_launch_fails_host_emulation(oracle):
     finally:
         error.value = 0
     assert m._state_pos is None
+
+
+def test_set_state_takes_the_shapes_a_row_of_the_state_takes_host_emulation(oracle):
+    """Token ids and positions broadcast to the b sequences like values assigned to a tensor's row: leading axes of length 1 and a single value for all are taken, a second axis
+    is refused (its first b values are not the sequences')."""
+    m = host_state()
+    table = m.block_tables.numpy()
+
+    def state(ids, pos):
+        m.set_state(ids, pos)
+        b = len(pos)
+        assert m.positions[:b].tolist() == pos and m.context_lens[:b].tolist() == [p + 1 for p in pos]
+        assert m.slot_mapping[:b].tolist() == [int(table[s, p // 32]) * 32 + p % 32 for s, p in enumerate(pos)]
+        return m.input_ids[:b].tolist()
+
+    assert state([1, 2, 3], [0, 31, 319]) == [1, 2, 3]
+    assert state(np.array([4, 5], dtype=np.int64), [64, 65]) == [4, 5] and state(torch.tensor([6, 7]), [66, 67]) == [6, 7]
+    for pos in (np.array([[8, 9]]), torch.tensor([[8, 9]]), [[8, 9]]):
+        m.set_state([1, 2], pos)
+        assert m.positions[:2].tolist() == [8, 9] and m._state_pos.tolist() == [8, 9]
+    for pos in (5, [5], np.int64(5), [[5]]):
+        m.set_state([1, 2], pos)
+        assert m.positions[:2].tolist() == [5, 5]
+    m.set_state([[9]], [3])
+    assert int(m.input_ids[0]) == 9
+    before = [t.clone() for t in (m.input_ids, m.positions)]
+    for ids, pos in (([[1, 2], [3, 4]], [0, 1]), ([[1], [2]], [0, 1]), ([1, 2], [[0], [1]]), ([1, 2], [0, 1, 2]), ([1, 2, 3], [0, 1]), ([1] * 5, [0] * 5), ([1], [320]), ([1], [-1]), ([], [])):
+        with pytest.raises(ValueError):
+            m.set_state(ids, pos)
+    assert all(torch.equal(a, b) for a, b in zip(before, (m.input_ids, m.positions)))
