@@ -292,6 +292,10 @@ int mrs_qi_quantize_for(int w_ggml_type, const float *x, const float *x2, int ld
 /* mrs_gemm_qi_multi: up to three tensors of one type that multiply the same operand rows (q / k / v, gate / up), in one launch where the kernel takes segments.  bounds != NULL
  * (device ints [experts + 1]): every tensor is a stack of `experts` tensors [N][K] (N % 32 == 0 where experts > 1: the copy's panels have 32 rows; else -1), expert e multiplies
  * and writes the rows [bounds[e], bounds[e + 1]); max_rows bounds one expert's rows and sizes the grid */
+/* mrs_gemm_qi_is_cut: 1 if mrs_gemm_qi_multi, given a workspace of 4 T sum(N) floats, cuts the launch by runs of superblocks; mrs_gemm_qi_cut_bytes: a workspace for every launch over
+ * at most n rows of weights and T tokens that is cut (never falls as T or n grow).  A smaller one, or NULL: the launch stays whole, same bits. */
+size_t mrs_gemm_qi_cut_bytes(int T, int n, int K);
+int mrs_gemm_qi_is_cut(int ggml_type, int n_tensors, const int *N, int K, int T);
 int mrs_gemm_qi_multi(int ggml_type, int n_tensors, const void *const *w_qi, const int *N, int K, const void *act, int T, float *const *out, const int *ldo, int accumulate,
                       const int *bounds, int experts, int max_rows, void *workspace, size_t workspace_bytes, void *stream);
 int mrs_gemm_qi_win(const void *w_qi, int ggml_type, int N, int K, const void *act, int T_total, const int *win, int max_rows, float *out, int ldo, int accumulate, void *stream);
@@ -353,10 +357,13 @@ typedef struct {
   const uint32_t *context_lens; /* [T] */
   float *logits;                /* [vocab] logits of the last prompt token */
   int32_t start_pos;            /* position of the first prompt token (= positions[0]) */
-  void *workspace;              /* >= mrs_llama_prefill_workspace_bytes(cfg, T) */
+  void *workspace;              /* mrs_llama_prefill_workspace_bytes(cfg, T), of this T or a larger one */
   size_t workspace_bytes;
 } mrs_llama_prefill_args;
+/* never falls as T grows: a buffer for the longest prompt serves the shorter ones.  A prompt in the decode engine's arithmetic also takes less, down to what
+ * mrs_llama_prefill_min_workspace_bytes says for the model's present path (it goes without cut launches, or without kept probabilities: slower, same bits) */
 size_t mrs_llama_prefill_workspace_bytes(const mrs_llama_config *cfg, int T);
+size_t mrs_llama_prefill_min_workspace_bytes(void *model, int T);
 int mrs_llama_prefill(void *model, const mrs_llama_prefill_args *args, int T, void *stream);
 /* floating-point operations of one prefill of T tokens starting at an empty context (MFMA roofline numerator) */
 double mrs_llama_prefill_flops(void *model, int T);

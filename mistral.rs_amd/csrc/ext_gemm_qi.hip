@@ -642,26 +642,48 @@ static void wide_launch(int NT, const qi::WideArgs &a, dim3 grid, hipStream_t s)
   if (NT == 2) hipLaunchKernelGGL(k2, grid, dim3(256), (2 * qi::wide_buf<TYPE, 2>), s, a);
   else hipLaunchKernelGGL(k1, grid, dim3(256), (2 * qi::wide_buf<TYPE, 1>), s, a);
 }
+// Token tiles per wave, by the rows of a launch (of an expert, where there are several).  K-quants: 32 rows fill one; from 33 rows on two waste little and build each operand once for both
+// (us, one / two tiles: Q4_K 28672 x 4096 28 / 38 at 20 rows, 37 / 37 at 37, 221 / 199 at 512;  Q6_K 4096 x 14336 32 / 38 at 20 rows, 161 / 129 at 512, 570 / 457 at 1999; the
+// line costs Q6_K something where it begins, 33 / 38 at 37).  Q8_0 has no operand to build and a smaller workgroup's registers let one more live on a CU (q / k / v 95 / 141 and
+// gate / up 348 / 376 at 700 rows, gate / up 1012 / 1079 at 1999).
+static int wide_tiles(int type, int rows) { return type == T_Q8_0 || rows <= 32 ? 1 : 2; }
+// Two (NT = 2) or three workgroups fit a CU.  Below 512 the launch is cut by runs of superblocks (4096 x 14336 Q4_K at 512 rows, 256 workgroups: 119 us whole, 102 us cut).
+// Long rows also where a second, partly filled round of workgroups would take as long as the first (K = 14336, whole / cut: Q4_K 1600 rows 314 / 287 us, Q6_K 430 / 392,
+// Q8_0 512 rows 175 / 129, 700 rows 194 / 168, 1000 rows 233 / 239; one full round, Q4_K 1024 rows: 178 / 191; K = 4096 at 1300 rows 90 / 97).
+static int cut_below(int K) { return K >= 8192 ? 896 : 512; }
+static bool wide_cut(int wgs, int K, int NT) { return K / 256 >= 4 && (wgs < 512 || (wgs < cut_below(K) && wgs % (NT == 1 ? 768 : 512) != 0)); }
+// workspace that holds the run sums of every launch over at most n rows of weights [K] and T tokens that is cut: four planes of its outputs, of which a workgroup writes at most
+// 64 x 128.  Never falls as T or n grow
+extern "C" size_t mrs_gemm_qi_cut_bytes(int T, int n, int K) {
+  if (T <= 0 || n <= 0 || K <= 0) return 0;
+  return (size_t)16 * std::min((size_t)T * n, (size_t)(cut_below(K) - 1) * 64 * qi::WIDE_ROWS);
+}
+// 1: mrs_gemm_qi_multi over T rows, given a workspace, is cut
+extern "C" int mrs_gemm_qi_is_cut(int type, int nt, const int *N, int K, int T) {
+  if (!N || nt < 1 || nt > 3 || !qi::qi_type(type) || T <= 0 || K <= 0 || K % 256) return 0;
+  const int NT = wide_tiles(type, T);
+  int gx = 0;
+  for (int i = 0; i < nt; ++i) {
+    if (N[i] <= 0 || N[i] % 4) return 0;
+    gx += (N[i] + qi::WIDE_ROWS - 1) / qi::WIDE_ROWS;
+  }
+  return wide_cut(gx * ((T + 32 * NT - 1) / (32 * NT)), K, NT);
+}
 extern "C" int mrs_gemm_qi_multi(int type, int nt, const void *const *w_qi, const int *N, int K, const void *act, int T, float *const *out, const int *ldo, int accumulate,
                                  const int *bounds, int experts, int max_rows, void *workspace, size_t workspace_bytes, void *stream) {
   if (!w_qi || !N || !act || !out || !ldo || nt < 1 || nt > 3 || !qi::qi_type(type) || T <= 0 || K <= 0 || K % 256 || (bounds && (experts <= 0 || max_rows <= 0))) return -1;
   int n_all = 0;
-  bool mult4 = true;
   for (int i = 0; i < nt; ++i) {
     if (!w_qi[i] || !out[i] || N[i] <= 0 || (bounds && experts > 1 && N[i] % 32)) return -1;  // an expert of a stack begins at a panel of 32 rows
     if (qi::qi_tensor_bytes(type, N[i], K) >= 0xffffff00ull) return -2;
-    n_all += N[i]; mult4 = mult4 && N[i] % 4 == 0;
+    n_all += N[i];
   }
   if ((size_t)(K / 256) * T * 512 >= 0x7fffffffull) return -2;
   hipStream_t s = (hipStream_t)stream;
   _Float16 *qf, *bsf; float *yd;
   qi_split((void *)act, T, K, &qf, &yd, &bsf);
-  const bool split_ok = !bounds && K / 256 >= 4 && mult4 && workspace && workspace_bytes >= (size_t)4 * T * n_all * 4;
-  // Token tiles per wave.  K-quants: 32 rows fill one; from 33 rows on two waste little and build each operand once for both (us, one / two tiles: Q4_K 28672 x 4096 28 / 38 at
-  // 20 rows, 37 / 37 at 37, 221 / 199 at 512;  Q6_K 4096 x 14336 32 / 38 at 20 rows, 33 / 38 at 37, 161 / 129 at 512, 570 / 457 at 1999).  Q8_0 has no operand to build and a
-  // smaller workgroup's registers let one more live on a CU (q / k / v 95 / 141 and gate / up 348 / 376 at 700 rows, gate / up 1012 / 1079 at 1999).
   max_rows = bounds ? std::min(max_rows, T) : T;
-  const int NT = type == T_Q8_0 || (bounds ? std::min(T / experts, max_rows) : T) <= 32 ? 1 : 2, tl = 32 * NT;
+  const int NT = wide_tiles(type, bounds ? std::min(T / experts, max_rows) : T), tl = 32 * NT;
   qi::WideArgs a{};
   qi::QiSeg *sg[3] = {&a.s0, &a.s1, &a.s2};
   int gx = 0, x[3] = {0, 0, 0};
@@ -670,11 +692,7 @@ extern "C" int mrs_gemm_qi_multi(int type, int nt, const void *const *w_qi, cons
   a.K = K; a.T = T; a.qf = qf; a.yd = yd; a.bsf = bsf; a.accumulate = accumulate; a.part = (float *)workspace; a.part_n = n_all; a.bounds = bounds; a.experts = experts; a.ksplit = 1;
   // windows: every expert's last tile may be partly filled, and none has more tiles than max_rows fill
   dim3 grid(gx, bounds ? std::min(T / tl + experts, experts * ((max_rows + tl - 1) / tl)) : (T + tl - 1) / tl);
-  // Two (NT = 2) or three workgroups fit a CU.  Below 512 the launch is cut by runs of superblocks (4096 x 14336 Q4_K at 512 rows, 256 workgroups: 119 us whole, 102 us cut).
-  // Long rows also where a second, partly filled round of workgroups would take as long as the first (K = 14336, whole / cut: Q4_K 1600 rows 314 / 287 us, Q6_K 430 / 392,
-  // Q8_0 512 rows 175 / 129, 700 rows 194 / 168, 1000 rows 233 / 239; one full round, Q4_K 1024 rows: 178 / 191; K = 4096 at 1300 rows 90 / 97).
-  const int wgs = (int)(grid.x * grid.y), slots = NT == 1 ? 768 : 512;
-  if (split_ok && (wgs < 512 || (K >= 8192 && wgs < 896 && wgs % slots != 0))) { a.ksplit = 4; grid.z = 4; }
+  if (!bounds && workspace && workspace_bytes >= (size_t)4 * T * n_all * 4 && mrs_gemm_qi_is_cut(type, nt, N, K, T)) { a.ksplit = 4; grid.z = 4; }
   switch (type) {
     case T_Q4_K: wide_launch<T_Q4_K>(NT, a, grid, s); break;
     case T_Q5_K: wide_launch<T_Q5_K>(NT, a, grid, s); break;

@@ -568,27 +568,41 @@ class Llama {
   // prompts longer than this use the 256-row-tile GEMM over bf16 slabs (its L1-bypassing A loads beat the 128-row f32 kernel even when
   // half of the tile rows are empty: TTFT 16.3 -> 10.1 ms at T = 128, 19.5 -> 8.3 ms at T = 64, 18.5 -> 7.7 ms at T = 32)
   static int prefill_big_min() { static int v = -1; if (v < 0) { const char *e = getenv("MRS_PREFILL_BIG_MIN"); v = e ? atoi(e) : 16; } return v; }
-  // run sums of the exact prompt GEMMs' split launches: q / k / v and o_proj / down_proj at any length, gate / up of short prompts (above 128 tokens they fill the chip)
-  static size_t qi_split_bytes(const mrs_llama_config &c, int T) {
-    const int nq = c.num_heads * c.head_dim, nkv = c.num_kv_heads * c.head_dim;
-    return mrs_gemm_qi_workspace_bytes(T, std::max(std::max(c.hidden_size, nq + 2 * nkv), T <= 128 && c.num_experts == 0 ? 2 * c.intermediate_size : 0));
-  }
-  // gate, up and act of T rows: not live during the attention, which keeps its probabilities there
-  static size_t ffn_bytes(const mrs_llama_config &c, int T) {
-    const int ctx = std::min(c.max_blocks_per_seq * c.block_size, (int)c.max_context_len);
-    return std::max(align((size_t)T * c.intermediate_size * 4) * 3, c.head_dim == 128 && c.block_size == 32 ? align(mrs_prefill_attention_workspace_bytes(T, c.num_heads, ctx)) : 0);
-  }
-  static size_t prefill_workspace_bytes(const mrs_llama_config &c, int T) {
+  // Workspace of a prompt.  Both paths: h, xn, q, attn, k, v and the last token's lm_head scratch.
+  static size_t prefill_rows_bytes(const mrs_llama_config &c, int T) {
     const size_t t = (size_t)T, d = c.hidden_size, nq = (size_t)c.num_heads * c.head_dim, nkv = (size_t)c.num_kv_heads * c.head_dim;
-    const size_t ff = c.intermediate_size;
-    size_t b = 0;
-    b += align(t * d * 4) * 2;        // h, xn
-    b += align(t * nq * 4) * 2;       // q, attn
-    b += align(t * nkv * 4) * 2;      // k, v
-    b += ffn_bytes(c, T);             // gate, up, act;  before them: the attention's probabilities
-    b += align((pad_to((int)d, MATRIX_ROW_PADDING) / 32) * 36);  // Q8_1 scratch of the last-token lm_head GEMV
-    b += align(mrs_qi_act_bytes(T, (int)std::max(std::max(d, nq), ff))) + align(qi_split_bytes(c, T));  // exact prompt path: Q8_K operands of T rows (f16 quants, scales, run sums) + run sums of split launches
-    if (T > prefill_big_min()) b += align(t * std::max(std::max(d, nq), ff) * 2) + align(mrs_gemm_q_bf16_workspace_bytes(T)) + align(t * ff * 2);  // bf16 activations + split-K partials + act(gate)*up slabs of the fused gate/up GEMM
+    return align(t * d * 4) * 2 + align(t * nq * 4) * 2 + align(t * nkv * 4) * 2 + align((pad_to((int)d, MATRIX_ROW_PADDING) / 32) * 36) + 4096;  // (4096: the base is aligned)
+  }
+  // gate, up and act: one row per token, in sparse-MoE layers per route
+  static size_t prefill_ffn_bytes(const mrs_llama_config &c, int T) {
+    return align((size_t)T * (c.num_experts > 0 ? std::max(1, (int)c.num_experts_per_tok) : 1) * c.intermediate_size * 4) * 3;
+  }
+  // The exact path's operand rows and tables, then gate / up / act at the END: what a call can do without stands behind them (run sums of cut launches) and over both of them
+  // (the attention's probabilities: neither gate / up / act nor run sums are live while it runs).
+  static size_t prefill_exact_bytes(const mrs_llama_config &c, int T) {
+    const size_t t = (size_t)T, d = c.hidden_size, nq = (size_t)c.num_heads * c.head_dim, ff = c.intermediate_size;
+    size_t b = prefill_rows_bytes(c, T) + align(mrs_qi_act_bytes(T, (int)std::max(std::max(d, nq), ff)));  // Q8_K operands of T rows (f16 quants, scales, run sums)
+    if (c.num_experts > 0) {  // routes = T * top_k rows in expert-sorted order
+      const size_t r = t * std::max(1, (int)c.num_experts_per_tok), E = (size_t)c.num_experts;
+      b += align(r * 4) * 4 + align((E + 1) * 4) + align(E * 4) * 2;  // ids, weights, sorted routes, inverse; bounds, counts, cursors
+      b += align(r * d * 4) + align(mrs_qi_act_bytes((int)r, (int)d)) + align(mrs_qi_act_bytes((int)r, (int)ff));  // per-route down outputs, gathered / per-route operand rows
+    }
+    return b + prefill_ffn_bytes(c, T);
+  }
+  static size_t prefill_cut_bytes(const mrs_llama_config &c, int T) {
+    const int nq = c.num_heads * c.head_dim, nkv = c.num_kv_heads * c.head_dim, d = c.hidden_size, ff = c.intermediate_size;
+    const size_t in = mrs_gemm_qi_cut_bytes(T, std::max(nq + 2 * nkv, c.num_experts > 0 ? 0 : 2 * ff), d);  // q / k / v, gate / up (experts' launches are never cut)
+    return align(std::max(std::max(in, mrs_gemm_qi_cut_bytes(T, d, nq)), c.num_experts > 0 ? 0 : mrs_gemm_qi_cut_bytes(T, d, ff)));
+  }
+  // probabilities of T tokens at the end of the model's window (a call knows its context, this size only T)
+  static size_t prefill_probs_bytes(const mrs_llama_config &c, int T) {
+    const int ctx = std::min(c.max_blocks_per_seq * c.block_size, (int)c.max_context_len);
+    return c.head_dim == 128 && c.block_size == 32 ? align(mrs_prefill_attention_workspace_bytes(T, c.num_heads, ctx)) : 0;
+  }
+  static size_t prefill_bf16_bytes(const mrs_llama_config &c, int T, size_t part) {
+    const size_t t = (size_t)T, d = c.hidden_size, nq = (size_t)c.num_heads * c.head_dim, ff = c.intermediate_size;
+    size_t b = prefill_rows_bytes(c, T) + align(t * ff * 4) * 3;
+    if (T > prefill_big_min()) b += align(t * std::max(std::max(d, nq), ff) * 2) + align(part) + align(t * ff * 2);  // bf16 activations + split-K partials + act(gate)*up slabs of the fused gate/up GEMM
     if (c.num_experts > 0) {  // MoE FFN of the prompt: routes = T * top_k rows in expert-sorted order
       const size_t tk = (size_t)std::max(1, (int)c.num_experts_per_tok), r = t * tk, E = (size_t)c.num_experts;
       b += align(r * ff * 4) * 3;                                                    // gate, up, act per route (replace the dense t * ff buffers)
@@ -597,9 +611,14 @@ class Llama {
       b += align(r * (pad_to((int)ff, MATRIX_ROW_PADDING) / 32) * 36);               // Q8_1 rows of the routes' activations
       b += align(t * d * 4);                                                         // sum of the weighted expert outputs
       if (T > prefill_big_min()) b += align(t * d * 2) + align(r * ff * 2);         // bf16 slabs of the normed tokens and of the routes' activations
-      b += align(r * 4) + align(r * d * 4) + align(mrs_qi_act_bytes((int)r, (int)d)) + align(mrs_qi_act_bytes((int)r, (int)ff));  // exact path: inverse route table, per-route down outputs, gathered / per-route operand rows
     }
-    return b + 4096;
+    return b;
+  }
+  // Either path, with everything it can use.  Never falls as T grows (a host keeps one buffer for all its prompts): the split-K partials shrink past a multiple of 256 rows, so
+  // their largest value up to T counts.
+  static size_t prefill_workspace_bytes(const mrs_llama_config &c, int T) {
+    const size_t ffn = prefill_ffn_bytes(c, T), exact = prefill_exact_bytes(c, T) - ffn + std::max(ffn + prefill_cut_bytes(c, T), prefill_probs_bytes(c, T));
+    return std::max(exact, prefill_bf16_bytes(c, T, mrs_gemm_q_bf16_workspace_bytes(std::min(T, 256))));
   }
   // MoE FFN of a prompt (SparseMoeBlock::forward on [T, hidden], models/mixtral.rs:280-304; the reference's prompt route is
   // FastExpertsWeights::forward_* -> moe_dispatch_build + grouped GEMM, moe/experts/backends.rs:969-1100, gguf/cuda.rs:590-640,1340-1420):
@@ -701,7 +720,7 @@ class Llama {
     return all_reduce(h, (size_t)T * d, s) ? fail("prefill (exact): moe all-reduce failed: %s", g_last_error.c_str()) : 0;
   }
   int prefill_exact(const mrs_llama_prefill_args &pa, int T, float *h, float *xn, float *q, float *k, float *v, float *attn, float *g, float *u, float *act, void *qact,
-                    void *qws, size_t qws_bytes, void *attn_ws, const MoeExactBufs &mx, hipStream_t s) const {
+                    void *qws, size_t qws_bytes, void *attn_ws, size_t attn_ws_bytes, const MoeExactBufs &mx, hipStream_t s) const {
     const int d = cfg.hidden_size, hd = cfg.head_dim, nq = cfg.num_heads * hd, nkv = cfg.num_kv_heads * hd, ff = cfg.intermediate_size;
     const int bs = cfg.block_size, kvh = cfg.num_kv_heads, kvd = cfg.kv_f16 ? 0 : 1;
     const int eff_max = std::min(cfg.max_blocks_per_seq * bs, cfg.max_context_len);
@@ -755,7 +774,7 @@ class Llama {
                                  cfg.rot_dim / 2, cfg.max_context_len, cfg.num_heads, cfg.num_kv_heads, nq, nkv, 2, st);
       reshape_and_cache(k, v, bl.key_cache, bl.value_cache, (int64_t *)pa.slot_mapping, T, cfg.num_kv_heads, hd, bs, 8, nkv, nkv, s, 2, kvd == 1 ? 1 : 0, nullptr, nullptr);
       if (mrs_prefill_attention_exact_ws(q, bl.key_cache, bl.value_cache, pa.block_tables, pa.context_lens, attn, T, cfg.num_heads, kvh, hd, bs, nq, kvh * hd * bs, hd * bs,
-                                      1.0f / sqrtf((float)hd), eff_max, kvd, cfg.sliding_window, pa.start_pos + T, attn_ws, ffn_bytes(cfg, T), s))
+                                      1.0f / sqrtf((float)hd), eff_max, kvd, cfg.sliding_window, pa.start_pos + T, attn_ws, attn_ws_bytes, s))
         return fail("prefill (exact): attention refused the shape");
       if (row_parallel(*bl.o_proj, d, nq, attn, nullptr, nq, nullptr)) return -1;
       if (cfg.num_experts > 0) {
@@ -770,11 +789,14 @@ class Llama {
       return fail("prefill (exact): lm_head refused");
     return 0;
   }
+  // of the path this model takes: without what the exact one can do without
+  size_t prefill_min_workspace_bytes(int T) const { return prefill_exact_ok() ? prefill_exact_bytes(cfg, T) : prefill_bf16_bytes(cfg, T, mrs_gemm_q_bf16_workspace_bytes(T)); }
   int prefill(const mrs_llama_prefill_args &pa, int T, hipStream_t s) const {
     if (T <= 0) return fail("prefill: T must be positive");
     const int start_pos = pa.start_pos;
     if (!wte || !lm_head || !ln_f) return fail("model is missing token_embd / output / output_norm");
-    if (pa.workspace_bytes < prefill_workspace_bytes(cfg, T)) return fail("prefill workspace too small");
+    const bool exact = prefill_exact_ok();
+    if (pa.workspace_bytes < prefill_min_workspace_bytes(T)) return fail("prefill workspace too small");
     const int d = cfg.hidden_size, hd = cfg.head_dim, nq = cfg.num_heads * hd, nkv = cfg.num_kv_heads * hd, ff = cfg.intermediate_size;
     const size_t t = (size_t)T;
     char *p = (char *)(((uintptr_t)pa.workspace + 255) & ~(uintptr_t)255);
@@ -782,23 +804,26 @@ class Llama {
     float *h = (float *)take(t * d * 4), *xn = (float *)take(t * d * 4);
     float *q = (float *)take(t * nq * 4), *attn = (float *)take(t * nq * 4);
     float *k = (float *)take(t * nkv * 4), *v = (float *)take(t * nkv * 4);
-    char *const ffn = take(ffn_bytes(cfg, T));
-    float *g = (float *)ffn, *u = (float *)(ffn + align(t * ff * 4)), *act = (float *)(ffn + align(t * ff * 4) * 2);
-    if (prefill_exact_ok()) {
+    float *g, *u, *act;
+    if (exact) {
       void *qact = take(mrs_qi_act_bytes(T, std::max(std::max(d, nq), ff)));
-      const size_t qws_bytes = qi_split_bytes(cfg, T);
-      void *qws = take(qws_bytes);
       MoeExactBufs mx{};
+      size_t rows = t;
       if (cfg.num_experts > 0) {  // routes = T * top_k rows in expert-sorted order; g / u / act become [routes][ff]
-        const size_t tk = (size_t)cfg.num_experts_per_tok, r = t * tk, E = (size_t)cfg.num_experts;
-        g = (float *)take(r * ff * 4); u = (float *)take(r * ff * 4); act = (float *)take(r * ff * 4);
+        const size_t r = t * (size_t)cfg.num_experts_per_tok, E = (size_t)cfg.num_experts;
         mx.ids = (int32_t *)take(r * 4); mx.w = (float *)take(r * 4); mx.sorted = (int32_t *)take(r * 4); mx.inv = (int32_t *)take(r * 4);
         mx.bounds = (int32_t *)take((E + 1) * 4); mx.counts = (int32_t *)take(E * 4); mx.cursors = (int32_t *)take(E * 4);
         mx.y = (float *)take(r * d * 4);
         mx.qact_g = take(mrs_qi_act_bytes((int)r, d)); mx.qact_r = take(mrs_qi_act_bytes((int)r, ff));
+        rows = r;
       }
-      return prefill_exact(pa, T, h, xn, q, k, v, attn, g, u, act, qact, qws, qws_bytes, ffn, mx, s);
+      char *const ffn = p, *const end = (char *)pa.workspace + pa.workspace_bytes;
+      g = (float *)take(rows * ff * 4); u = (float *)take(rows * ff * 4); act = (float *)take(rows * ff * 4);
+      // (at most what the size function asks for: the attention goes in groups whose probabilities stay in the last-level cache)
+      const size_t attn_bytes = std::min((size_t)(end - ffn), std::max(align(t * ff * 4) * 3, prefill_probs_bytes(cfg, T)));
+      return prefill_exact(pa, T, h, xn, q, k, v, attn, g, u, act, qact, p, (size_t)(end - p), ffn, attn_bytes, mx, s);
     }
+    g = (float *)take(t * ff * 4); u = (float *)take(t * ff * 4); act = (float *)take(t * ff * 4);
     MoePrefillBufs moe{};
     if (cfg.num_experts > 0) {
       const size_t tk = (size_t)cfg.num_experts_per_tok, r = t * tk, E = (size_t)cfg.num_experts;
@@ -1240,6 +1265,7 @@ extern "C" int mrs_llama_chained_ok(void *m, int b) { return ((Llama *)m)->chain
 extern "C" int mrs_llama_forward_logits(void *m, int b, void *stream) { return ((Llama *)m)->forward_logits(b, (hipStream_t)stream); }
 extern "C" double mrs_llama_decode_bytes(void *m, int b, int ctx) { return ((Llama *)m)->decode_bytes(b, ctx); }
 extern "C" size_t mrs_llama_prefill_workspace_bytes(const mrs_llama_config *cfg, int T) { return Llama::prefill_workspace_bytes(*cfg, T); }
+extern "C" size_t mrs_llama_prefill_min_workspace_bytes(void *model, int T) { return T > 0 ? ((const Llama *)model)->prefill_min_workspace_bytes(T) : 0; }
 extern "C" int mrs_llama_prefill(void *m, const mrs_llama_prefill_args *a, int T, void *stream) {
   Llama &l = *(Llama *)m;
   if (!l.have_bufs) return mrs_host::fail("mrs_llama_set_buffers was not called");

@@ -1,0 +1,96 @@
+"""Workspace of Llama::prefill (csrc/host/runtime.cpp): its size never falls as prompts grow, covers what the launches may use, and a smaller one is taken where only the parts
+are missing that a call can do without (probabilities of the two-kernel attention, run sums of launches cut by runs) -- with the same bits."""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+from mistralrs_amd.llama import LlamaConfig, _Cfg
+from tests.abi_backends import HostBackend
+from tests.test_dec_model import Q4KM, _mk
+
+CI = C.c_int
+CONFIGS = {"8b, 576": LlamaConfig.llama3_8b(max_context_len=576), "8b, 2048": LlamaConfig.llama3_8b(max_context_len=2048), "8b, 8192": LlamaConfig.llama3_8b(max_context_len=8192),
+           "70b, 2304": LlamaConfig.llama3_70b(max_context_len=2304), "moe, 1024": LlamaConfig.mixtral_8x7b(max_context_len=1024),
+           "small ffn": LlamaConfig(hidden_size=2048, intermediate_size=5632, num_layers=22, num_heads=32, num_kv_heads=4, vocab_size=32000, max_context_len=2048)}
+
+
+def c_config(cfg):
+    return _Cfg(cfg.hidden_size, cfg.intermediate_size, cfg.num_layers, cfg.num_heads, cfg.num_kv_heads, cfg.head_dim, cfg.vocab_size, cfg.head_dim, 1, cfg.rms_eps, cfg.block_size,
+                cfg.max_blocks_per_seq, cfg.max_batch, cfg.max_context_len, 1, 1, 0, cfg.num_experts, cfg.num_experts_per_tok if cfg.num_experts else 0, 0, 0)
+
+
+def sizes(cfg, lengths):
+    f = HostBackend().sym("mrs_llama_prefill_workspace_bytes", [C.POINTER(_Cfg), CI], C.c_size_t)
+    c = c_config(cfg)
+    return [f(C.byref(c), t) for t in lengths]
+
+
+@pytest.mark.parametrize("name", CONFIGS)
+def test_workspace_of_a_longer_prompt_holds_a_shorter_one(name):
+    cfg = CONFIGS[name]
+    s = sizes(cfg, range(1, min(cfg.max_context_len, 2100) + 1))
+    assert all(a <= b for a, b in zip(s, s[1:])), [t for t, (a, b) in enumerate(zip(s, s[1:]), 1) if a > b][:5]
+
+
+def test_cut_launches_fit_the_bytes_reserved_for_them():
+    """mrs_gemm_qi_cut_bytes(T, n, K) holds the run sums (4 T n_all floats) of every launch over n_all <= n rows of weights and up to T tokens that mrs_gemm_qi_multi would cut."""
+    be = HostBackend()
+    cut, room = be.sym("mrs_gemm_qi_is_cut", [CI, CI, C.c_void_p, CI, CI], CI), be.sym("mrs_gemm_qi_cut_bytes", [CI, CI, CI], C.c_size_t)
+    seen = 0
+    for k in (768, 1024, 4096, 8192, 14336):
+        for ns in ((1024,), (4096,), (4096, 1024, 1024), (4096, 1024), (5632, 5632), (14336, 14336), (28672, 28672), (36,)):
+            arr = (CI * len(ns))(*ns)
+            for T in list(range(1, 140)) + [500, 512, 513, 600, 960, 961, 1024, 1728, 1999, 4032, 4096]:
+                got = [cut(t, len(ns), arr, k, T) for t in (12, 13, 14, 8)]
+                seen += sum(got)
+                assert not any(got) or 16 * T * sum(ns) <= room(T, sum(ns), k), (k, ns, T, got)
+                assert not any(got) or k >= 1024
+    assert seen > 1000
+    assert cut(12, 1, (CI * 1)(4096), 4096, 512) == 1 and cut(12, 2, (CI * 2)(14336, 14336), 4096, 128) == 1 and cut(12, 2, (CI * 2)(14336, 14336), 4096, 129) == 0
+    assert cut(12, 2, (CI * 2)(5632, 5632), 2048, 300) == 1  # a smaller FFN is cut at longer prompts
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("experts", [0, 4])
+def test_prefill_takes_a_workspace_without_the_optional_parts(oracle, dev, request, experts):
+    """The smallest workspace that prefill() takes, the one that mrs_llama_prefill_workspace_bytes names and one between: same logits, same pages, nothing written past any."""
+    import torch
+    types = Q4KM(oracle)
+    T = 9 if request.config.getoption("--host-emulation") else 70
+    _, _, m, _, _ = _mk(oracle, dev, types, "bf16", experts=experts)
+    assert m.prefill_is_exact
+    prompt = [(1000 + 37 * i) % m.cfg.vocab_size for i in range(T)]
+    want = m.prefill(prompt, 0).clone()
+    pages = [t.clone() for t in m.key_caches + m.value_caches]
+    full = m._L.mrs_llama_prefill_workspace_bytes(C.byref(m._c), T)
+    real = m._L
+
+    class Sized:  # the library with another answer to how large the workspace has to be
+        def __getattr__(self, name):
+            return (lambda c, t: self.size) if name == "mrs_llama_prefill_workspace_bytes" else getattr(real, name)
+
+    shim = Sized()
+    guard = 1 << 16
+
+    def run(size):
+        for t in m.key_caches + m.value_caches:
+            t.zero_()
+        shim.size = size
+        whole = torch.full((size + guard,), 0xA5, dtype=torch.uint8, device=m.device)
+        m._prefill_ws, m._L = whole[:size], shim
+        try:
+            got = m.prefill(prompt, 0)
+        finally:
+            m._L = real
+        assert (whole[size:] == 0xA5).all(), size
+        assert torch.equal(got, want) and all(torch.equal(a.view(torch.int16), b.view(torch.int16)) for a, b in zip(pages, m.key_caches + m.value_caches)), size
+
+    f = real.mrs_llama_prefill_min_workspace_bytes
+    f.restype, f.argtypes = C.c_size_t, [C.c_void_p, CI]
+    least = f(m._h, T)
+    assert 0 < least < full
+    with pytest.raises(ValueError, match="too small"):
+        run(least - 1)
+    for size in (least, (least + full) // 2, full):
+        run(size)
