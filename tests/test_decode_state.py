@@ -67,3 +67,11 @@ def test_set_state_takes_the_shapes_a_row_of_the_state_takes_host_emulation(orac
         with pytest.raises(ValueError):
             m.set_state(ids, pos)
     assert all(torch.equal(a, b) for a, b in zip(before, (m.input_ids, m.positions)))
+
+
+def test_set_state_slot_of_a_block_without_a_number_host_emulation(oracle):
+    """Block tables are int32: an entry of -1 (no block) gives a negative slot, which the K / V writes drop, and no slot past the caches."""
+    m = host_state()
+    m.block_tables[1, 2] = -1
+    m.set_state([1, 2, 3], [70, 70, 70])
+    assert m.slot_mapping[:3].tolist() == [int(m.block_tables[0, 2]) * 32 + 6, -32 + 6, int(m.block_tables[2, 2]) * 32 + 6]
