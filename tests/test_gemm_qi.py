@@ -363,3 +363,34 @@ def test_grid_of_a_window_follows_its_bound_host_emulation(oracle):
     assert be.sym("mrs_gemm_qi_win", [VP, CI, CI, CI, VP, CI, VP, CI, VP, CI, CI, VP], CI)(wq.ptr, t, n, k, act.ptr, T, wb.ptr, 32, o.ptr, n, 0, be.stream) == 0
     got = o.numpy()
     assert (got[:32] == 0).all() and (got[32:] == 7.0).all()
+
+
+def run_bad_rows(O, be, tname, T):
+    """Activation rows with NaN and infinities share their tile's matrix instructions -- block scales included -- with rows that must not see them, whole and cut by runs."""
+    t, n, k = getattr(O, tname), 68, 1024
+    rng = np.random.default_rng(12)
+    p = O.quantize(t, (rng.standard_normal((n, k)) * 0.05).astype(np.float32)).reshape(n, -1)
+    x = rng.standard_normal((T, k)).astype(np.float32)
+    bad = [0, 3, T - 2]
+    x[0], x[3, 300], x[T - 2, 256:512] = np.nan, np.inf, -np.inf
+    good = [r for r in range(T) if r not in bad]
+    want = np.concatenate([O.gemv_engine(t, p, n, k, x[r]) for r in good], axis=0)
+    for cut in (False, True):
+        got = gemm_rows(O, be, t, p, n, k, x, cut)
+        assert np.array_equal(got[good], want), (tname, cut)
+        assert np.isnan(got[0]).all()  # the bad rows' own outputs stay bad
+        assert not np.isfinite(got[[3, T - 2]]).any()
+
+
+BAD_ROWS = [("Q4_K", 6), ("Q4_K", 40), ("Q5_K", 40), ("Q6_K", 6), ("Q6_K", 66), ("Q8_0", 40)]
+
+
+@pytest.mark.parametrize("tname,T", BAD_ROWS)
+def test_gemm_qi_rows_beside_nan_and_inf_host_emulation(oracle, tname, T):
+    run_bad_rows(oracle, HostBackend(), tname, T)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("tname,T", BAD_ROWS)
+def test_gemm_qi_rows_beside_nan_and_inf_gpu(oracle, dev, tname, T):
+    run_bad_rows(oracle, GpuBackend(dev), tname, T)
