@@ -239,6 +239,7 @@ def test_long_rows_cut_by_runs_equal_the_whole_launch(oracle, dev, tname, T):
     assert be.sym("mrs_gemm_qi_repack", [VP, CI, C.c_longlong, C.c_longlong, VP, VP], CI)(src.ptr, t, n, k, wq.ptr, be.stream) == 0
     x, act = be.buf(rng.standard_normal((T, k)).astype(np.float32)), be.buf(np.zeros(be.sym("mrs_qi_act_bytes", [CI, CI], C.c_size_t)(T, k), np.uint8))
     assert be.sym("mrs_qi_quantize_for", [CI, VP, VP, CI, VP, C.c_float, CI, CI, VP, VP, VP], CI)(t, x.ptr, None, k, None, 1e-5, T, k, act.ptr, None, be.stream) == 0
+    assert be.sym("mrs_gemm_qi_is_cut", [CI, CI, VP, CI, CI], CI)(t, 1, (CI * 1)(n), k, T) == 1
     ws, got = be.buf(np.zeros(4 * T * n, np.float32)), []
     for w in (ws, None):
         o = be.buf(np.zeros((T, n), np.float32))
