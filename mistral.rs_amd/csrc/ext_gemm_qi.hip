@@ -247,7 +247,7 @@ __device__ __forceinline__ h2 pkfma(h2 x, h2 s, h2 c) { return __builtin_element
 // 28672 x 4096 x 512 tokens.
 struct QiSeg { const uint8_t *w; unsigned w_bytes; int N; float *out; int ldo; };
 struct WideArgs {
-  QiSeg s0, s1, s2; int x1, x2;  // segment of a workgroup: blockIdx.x < x1: s0, < x2: s1, else s2 (x1 = x2 = gridDim.x for a single one)
+  QiSeg s0, s1, s2; int x1, x2;  // segment of a workgroup column: < x1: s0, < x2: s1, else s2 (x1 = x2 = gridDim.x for a single one)
   int K, T;
   const _Float16 *qf; const float *yd; const _Float16 *bsf;
   int accumulate, ksplit; float *part; int part_n;  // ksplit = 4: workgroup z multiplies run z only, plane z of part [4][T][part_n] takes its sums
@@ -259,6 +259,12 @@ struct WideArgs {
 template <int TYPE> constexpr int wide_row = TYPE == T_Q8_0 ? 256 : 512;
 template <int TYPE, int NT> constexpr int wide_buf = NT * 32 * wide_row<TYPE> + (TYPE == T_Q8_0 ? 0 : 512) + NT * 32 * 32;
 constexpr int WIDE_ROWS = 128;                                                      // weight rows of a workgroup: four waves
+// Order of the workgroups: all token tiles of 32 neighbouring workgroup columns (4096 weight rows), then of the next 32.  Workgroups go to the XCDs in turn, so those that live on
+// an XCD share four columns and read the same weights out of its L2; with all columns before the next token tile 28 (57344 rows: 56) columns were live there, and a wide tensor
+// was read again for every few token tiles.  us, all columns first / this order: Q8_0 28672 x 4096 1000 rows 510 / 441, 2000 rows 1037 / 822, 57344 x 8192 512 rows 1244 / 883,
+// 2000 rows 5482 / 3268 (a kernel of 128 x 128 tiles: 473, 923, 983, 3893); 57344 x 8192 2000 rows Q4_K 2687 / 2507, Q5_K 3969 / 3033, Q6_K 4326 / 3452; Q4_K 28672 x 4096 512
+// rows 168 / 165.  Up to 32 columns both orders are the same.
+constexpr int WIDE_COLS = 32;
 #ifndef MRS_BLDS16
 // buffer load to LDS, 16 / 4 bytes per lane: LDS destination = wave-uniform base + lane * size
 #define MRS_BLDS16(rsrc, lbase, voff) __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, (__attribute__((address_space(3))) void *)(lbase), 16, voff, 0, 0, 0)
@@ -273,10 +279,12 @@ __global__ void __launch_bounds__(256, NT == 1 && TYPE != T_Q5_K ? 3 : 2) gemm_q
   constexpr int NPC = TYPE == T_Q4_K ? 4 : 8;  // 1-KiB pieces of a record
   const int tid = tid_opaque(), lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int nn = lane & 31, hf = lane >> 5;
-  const int bx = blockIdx.x, seg = bx >= a.x2 ? 2 : bx >= a.x1 ? 1 : 0;
+  const int order = (int)(blockIdx.y * gridDim.x + blockIdx.x), cols0 = order / (WIDE_COLS * (int)gridDim.y) * WIDE_COLS, cols = min(WIDE_COLS, (int)gridDim.x - cols0);
+  const int in_cols = order - cols0 * (int)gridDim.y, by = in_cols / cols, bx = cols0 + in_cols % cols;
+  const int seg = bx >= a.x2 ? 2 : bx >= a.x1 ? 1 : 0;
   const QiSeg sg = seg == 2 ? a.s2 : seg == 1 ? a.s1 : a.s0;
   const int coff = seg == 2 ? a.s0.N + a.s1.N : seg == 1 ? a.s0.N : 0;
-  int tbeg = 0, tend = a.T, yt = blockIdx.y, ex = 0;
+  int tbeg = 0, tend = a.T, yt = by, ex = 0;
   if (a.bounds && !expert_tile(a.bounds, a.experts, TT_, yt, ex, tbeg, tend)) return;
   const uint8_t *wbase = sg.w + (size_t)ex * sg.w_bytes;
   const int t0 = tbeg + yt * TT_;

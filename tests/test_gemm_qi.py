@@ -228,6 +228,22 @@ def test_gemm_qi_multi_gpu(oracle, dev, case):
     run_multi(oracle, GpuBackend(dev), *case, seed=4)
 
 
+# more than 32 workgroup columns of 128 rows: whole groups of columns and a remainder, a segment that begins inside a group, windows, a launch cut by runs
+WIDE = [("Q8_0", (4224,), 256, 66, None, False, False), ("Q4_K", (4000, 200), 256, 130, None, True, False), ("Q6_K", (2176, 2176), 256, 40, (0, 33, 40), False, False),
+        ("Q8_0", (4100,), 1024, 40, None, True, True)]
+
+
+@pytest.mark.parametrize("case", WIDE)
+def test_gemm_qi_more_columns_than_a_group_host_emulation(oracle, case):
+    run_multi(oracle, HostBackend(), *case, seed=8)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("case", WIDE + [("Q8_0", (14336, 14336), 512, 200, None, False, False), ("Q5_K", (8200,), 512, 300, None, False, False)])
+def test_gemm_qi_more_columns_than_a_group_gpu(oracle, dev, case):
+    run_multi(oracle, GpuBackend(dev), *case, seed=8)
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("tname,T", [("Q8_0", 2050), ("Q6_K", 4130), ("Q4_K", 4130)])
 def test_long_rows_cut_by_runs_equal_the_whole_launch(oracle, dev, tname, T):
