@@ -655,16 +655,25 @@ static void wide_launch(int NT, const qi::WideArgs &a, dim3 grid, hipStream_t s)
 // line costs Q6_K something where it begins, 33 / 38 at 37).  Q8_0 has no operand to build and a smaller workgroup's registers let one more live on a CU (q / k / v 95 / 141 and
 // gate / up 348 / 376 at 700 rows, gate / up 1012 / 1079 at 1999).
 static int wide_tiles(int type, int rows) { return type == T_Q8_0 || rows <= 32 ? 1 : 2; }
-// Two (NT = 2) or three workgroups fit a CU.  Below 512 the launch is cut by runs of superblocks (4096 x 14336 Q4_K at 512 rows, 256 workgroups: 119 us whole, 102 us cut).
-// Long rows also where a second, partly filled round of workgroups would take as long as the first (K = 14336, whole / cut: Q4_K 1600 rows 314 / 287 us, Q6_K 430 / 392,
-// Q8_0 512 rows 175 / 129, 700 rows 194 / 168, 1000 rows 233 / 239; one full round, Q4_K 1024 rows: 178 / 191; K = 4096 at 1300 rows 90 / 97).
-static int cut_below(int K) { return K >= 8192 ? 896 : 512; }
-static bool wide_cut(int wgs, int K, int NT) { return K / 256 >= 4 && (wgs < 512 || (wgs < cut_below(K) && wgs % (NT == 1 ? 768 : 512) != 0)); }
+// A launch of few workgroups is cut by runs of superblocks: four times the workgroups, a quarter of the chain, for four planes of sums written and read again.  The planes cost the same
+// at any K and the chain saved grows with it, so the line lies at a number of workgroups in proportion to K.  Whole / cut, us: Q4_K, two tiles (workgroups in brackets), 2048 x 2048
+// 200 rows (64) 16.3 / 13.2, 400 rows (112) 16.4 / 19.2, 8192 x 2048 400 rows (448) 25.7 / 39.4; 4096 x 4096 256 rows (128) 28.8 / 23.0, 300 rows (160) 29.9 / 29.1, 512 rows (256)
+// 32.6 / 37.6; 28672 x 4096 128 rows (448) 48.5 / 60.5; 8192 x 8192 300 rows (320) 80.4 / 70.5, 400 rows (448) 87.9 / 95.3; 4096 x 14336 700 rows (352) 138.6 / 129.3, 1000 rows
+// (512) 159 / 172; 8192 x 28672 400 rows (448) 307 / 284.  One tile, 32 rows: 11264 x 2048 (88) 13.2 / 12.8, 28672 x 4096 (224) 26.9 / 25.9, 57344 x 8192 (448) 76.2 / 79.0, 65536 x 8192
+// (512) 76.7 / 84.3.  Q8_0: 2048 x 2048 300 rows (160) 20.0 / 18.1, 512 rows (256) 20.6 / 23.3; 4096 x 4096 512 rows (512) 45.7 / 44.5; 8192 x 8192 300 rows (640) 93.8 / 87.7.
+// Long rows are cut beyond it too where a second, partly filled round of workgroups (two or, Q8_0, three fit a CU) would take as long as the first: K = 14336, Q4_K 1600 rows 314 / 287,
+// Q6_K 430 / 392.
+static int cut_max(int type, int NT, int K) { return type == T_Q8_0 ? std::min(K / 8, 895) : NT == 1 ? std::min(K / 18, 400) : K >= 8192 ? 895 : K / 20; }
+static bool wide_cut(int type, int wgs, int K, int NT) {
+  if (K / 256 < 4 || wgs > cut_max(type, NT, K)) return false;
+  return type == T_Q8_0 ? wgs != 768 : NT == 1 || wgs <= std::min(K / 20, 511) || wgs > 512;
+}
 // workspace that holds the run sums of every launch over at most n rows of weights [K] and T tokens that is cut: four planes of its outputs, of which a workgroup writes at most
-// 64 x 128.  Never falls as T or n grow
+// 32 NT x 128.  Never falls as T or n grow
 extern "C" size_t mrs_gemm_qi_cut_bytes(int T, int n, int K) {
   if (T <= 0 || n <= 0 || K <= 0) return 0;
-  return (size_t)16 * std::min((size_t)T * n, (size_t)(cut_below(K) - 1) * 64 * qi::WIDE_ROWS);
+  const int tiles = std::max(std::max(cut_max(T_Q8_0, 1, K), cut_max(T_Q4_K, 1, K)), 2 * cut_max(T_Q4_K, 2, K));
+  return (size_t)16 * std::min((size_t)T * n, (size_t)tiles * 32 * qi::WIDE_ROWS);
 }
 // 1: mrs_gemm_qi_multi over T rows, given a workspace, is cut
 extern "C" int mrs_gemm_qi_is_cut(int type, int nt, const int *N, int K, int T) {
@@ -675,7 +684,7 @@ extern "C" int mrs_gemm_qi_is_cut(int type, int nt, const int *N, int K, int T) 
     if (N[i] <= 0 || N[i] % 4) return 0;
     gx += (N[i] + qi::WIDE_ROWS - 1) / qi::WIDE_ROWS;
   }
-  return wide_cut(gx * ((T + 32 * NT - 1) / (32 * NT)), K, NT);
+  return wide_cut(type, gx * ((T + 32 * NT - 1) / (32 * NT)), K, NT);
 }
 extern "C" int mrs_gemm_qi_multi(int type, int nt, const void *const *w_qi, const int *N, int K, const void *act, int T, float *const *out, const int *ldo, int accumulate,
                                  const int *bounds, int experts, int max_rows, void *workspace, size_t workspace_bytes, void *stream) {

@@ -47,8 +47,20 @@ def test_cut_launches_fit_the_bytes_reserved_for_them():
                 assert not any(got) or 16 * T * sum(ns) <= room(T, sum(ns), k), (k, ns, T, got)
                 assert not any(got) or k >= 1024
     assert seen > 1000
-    assert cut(12, 1, (CI * 1)(4096), 4096, 512) == 1 and cut(12, 2, (CI * 2)(14336, 14336), 4096, 128) == 1 and cut(12, 2, (CI * 2)(14336, 14336), 4096, 129) == 0
-    assert cut(12, 2, (CI * 2)(5632, 5632), 2048, 300) == 1  # a smaller FFN is cut at longer prompts
+    assert cut(12, 1, (CI * 1)(4096), 4096, 300) == 1 and cut(12, 2, (CI * 2)(14336, 14336), 4096, 32) == 1 and cut(12, 2, (CI * 2)(14336, 14336), 4096, 33) == 0
+    assert cut(12, 1, (CI * 1)(2048), 5632, 700) == 1  # fewer rows are cut at longer prompts
+
+
+def test_products_that_a_cut_slows_down_stay_whole():
+    """Sizes (type, rows, K, tokens) on both sides of the line: whole where the four planes of run sums cost more than the shorter chain gives back, cut where they cost less."""
+    cut = HostBackend().sym("mrs_gemm_qi_is_cut", [CI, CI, C.c_void_p, CI, CI], CI)
+    whole = [(12, 8192, 2048, 400), (13, 2048, 2048, 2000), (14, 3072, 1024, 1000), (12, 28672, 4096, 128), (13, 28672, 4096, 100), (14, 14336, 4096, 256), (12, 28672, 8192, 128),
+             (12, 8960, 1536, 300), (8, 8960, 1536, 160), (8, 3072, 1024, 512), (13, 65536, 8192, 20), (14, 65536, 8192, 32), (12, 4096, 14336, 1000)]
+    parts = [(12, 2048, 2048, 200), (13, 4096, 4096, 256), (12, 28672, 4096, 32), (14, 8192, 8192, 300), (12, 4096, 14336, 700), (14, 4096, 14336, 1600), (8, 4096, 4096, 512),
+             (8, 2048, 2048, 300), (8, 8192, 8192, 300), (12, 8192, 28672, 400)]
+    for case, want in [(c, 0) for c in whole] + [(c, 1) for c in parts]:
+        t, n, k, T = case
+        assert cut(t, 1, (CI * 1)(n), k, T) == want, case
 
 
 @pytest.mark.gpu
