@@ -650,11 +650,13 @@ static void wide_launch(int NT, const qi::WideArgs &a, dim3 grid, hipStream_t s)
   if (NT == 2) hipLaunchKernelGGL(k2, grid, dim3(256), (2 * qi::wide_buf<TYPE, 2>), s, a);
   else hipLaunchKernelGGL(k1, grid, dim3(256), (2 * qi::wide_buf<TYPE, 1>), s, a);
 }
-// Token tiles per wave, by the rows of a launch (of an expert, where there are several).  K-quants: 32 rows fill one; from 33 rows on two waste little and build each operand once for both
-// (us, one / two tiles: Q4_K 28672 x 4096 28 / 38 at 20 rows, 37 / 37 at 37, 221 / 199 at 512;  Q6_K 4096 x 14336 32 / 38 at 20 rows, 161 / 129 at 512, 570 / 457 at 1999; the
-// line costs Q6_K something where it begins, 33 / 38 at 37).  Q8_0 has no operand to build and a smaller workgroup's registers let one more live on a CU (q / k / v 95 / 141 and
-// gate / up 348 / 376 at 700 rows, gate / up 1012 / 1079 at 1999).
-static int wide_tiles(int type, int rows) { return type == T_Q8_0 || rows <= 32 ? 1 : 2; }
+// Token tiles per wave, by the rows of a launch (of an expert, where there are several) and its workgroup columns (of all experts).  K-quants: 32 rows fill one; two build each operand
+// once for both, but make the chain of a superblock longer, which is what a launch that leaves most of the chip idle waits for.  So two from 33 rows on where they make more than 32
+// workgroups (Q5_K, whose kernel of two tiles is the slowest: 96).  us, one / two tiles, each cut or whole as below (workgroups of two tiles in brackets): Q4_K 4096 x 4096 37 rows
+// (32) 11.3 / 13.7, 128 rows (64) 17.4 / 17.0, 6144 x 4096 37 rows (48) 14.7 / 14.2, 28672 x 4096 512 rows 221 / 199;  Q6_K 4096 x 14336 37 rows (32) 31.3 / 37.7, 128 rows (64)
+// 44.5 / 41.6, 1999 rows 570 / 457;  Q5_K 3072 x 1024 64 rows (24) 9.9 / 12.6, 4096 x 4096 160 rows (96) 22.0 / 25.5, 8192 x 8192 128 rows (128) 43.8 / 41.0.  Q8_0 has no operand to
+// build and a smaller workgroup's registers let one more live on a CU (q / k / v 95 / 141 and gate / up 348 / 376 at 700 rows).
+static int wide_tiles(int type, int rows, int cols) { return type == T_Q8_0 || rows <= 32 || cols * ((rows + 63) / 64) <= (type == T_Q5_K ? 96 : 32) ? 1 : 2; }
 // A launch of few workgroups is cut by runs of superblocks: four times the workgroups, a quarter of the chain, for four planes of sums written and read again.  The planes cost the same
 // at any K and the chain saved grows with it, so the line lies at a number of workgroups in proportion to K.  Whole / cut, us: Q4_K, two tiles (workgroups in brackets), 2048 x 2048
 // 200 rows (64) 16.3 / 13.2, 400 rows (112) 16.4 / 19.2, 8192 x 2048 400 rows (448) 25.7 / 39.4; 4096 x 4096 256 rows (128) 28.8 / 23.0, 300 rows (160) 29.9 / 29.1, 512 rows (256)
@@ -678,12 +680,12 @@ extern "C" size_t mrs_gemm_qi_cut_bytes(int T, int n, int K) {
 // 1: mrs_gemm_qi_multi over T rows, given a workspace, is cut
 extern "C" int mrs_gemm_qi_is_cut(int type, int nt, const int *N, int K, int T) {
   if (!N || nt < 1 || nt > 3 || !qi::qi_type(type) || T <= 0 || K <= 0 || K % 256) return 0;
-  const int NT = wide_tiles(type, T);
   int gx = 0;
   for (int i = 0; i < nt; ++i) {
     if (N[i] <= 0 || N[i] % 4) return 0;
     gx += (N[i] + qi::WIDE_ROWS - 1) / qi::WIDE_ROWS;
   }
+  const int NT = wide_tiles(type, T, gx);
   return wide_cut(type, gx * ((T + 32 * NT - 1) / (32 * NT)), K, NT);
 }
 extern "C" int mrs_gemm_qi_multi(int type, int nt, const void *const *w_qi, const int *N, int K, const void *act, int T, float *const *out, const int *ldo, int accumulate,
@@ -700,11 +702,11 @@ extern "C" int mrs_gemm_qi_multi(int type, int nt, const void *const *w_qi, cons
   _Float16 *qf, *bsf; float *yd;
   qi_split((void *)act, T, K, &qf, &yd, &bsf);
   max_rows = bounds ? std::min(max_rows, T) : T;
-  const int NT = wide_tiles(type, bounds ? std::min(T / experts, max_rows) : T), tl = 32 * NT;
   qi::WideArgs a{};
   qi::QiSeg *sg[3] = {&a.s0, &a.s1, &a.s2};
   int gx = 0, x[3] = {0, 0, 0};
   for (int i = 0; i < nt; ++i) { *sg[i] = qi::QiSeg{(const uint8_t *)w_qi[i], (unsigned)qi::qi_tensor_bytes(type, N[i], K), N[i], out[i], ldo[i]}; gx += (N[i] + qi::WIDE_ROWS - 1) / qi::WIDE_ROWS; x[i] = gx; }
+  const int NT = bounds ? wide_tiles(type, std::min(T / experts, max_rows), gx * experts) : wide_tiles(type, T, gx), tl = 32 * NT;
   a.x1 = x[0]; a.x2 = nt > 1 ? x[1] : gx;
   a.K = K; a.T = T; a.qf = qf; a.yd = yd; a.bsf = bsf; a.accumulate = accumulate; a.part = (float *)workspace; a.part_n = n_all; a.bounds = bounds; a.experts = experts; a.ksplit = 1;
   // windows: every expert's last tile may be partly filled, and none has more tiles than max_rows fill

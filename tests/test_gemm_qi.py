@@ -230,7 +230,11 @@ def test_gemm_qi_multi_gpu(oracle, dev, case):
 
 # more than 32 workgroup columns of 128 rows: whole groups of columns and a remainder, a segment that begins inside a group, windows, a launch cut by runs
 WIDE = [("Q8_0", (4224,), 256, 66, None, False, False), ("Q4_K", (4000, 200), 256, 130, None, True, False), ("Q6_K", (2176, 2176), 256, 40, (0, 33, 40), False, False),
-        ("Q8_0", (4100,), 1024, 40, None, True, True)]
+        ("Q8_0", (4100,), 1024, 40, None, True, True),
+        # the same sizes take two token tiles per wave (K-quants; Q5_K from 97 workgroups on): remainders of a tile, empty runs, launches cut by runs, windows
+        ("Q4_K", (4100, 160), 1280, 33, None, False, True), ("Q4_K", (4132,), 768, 65, None, True, False), ("Q4_K", (4224,), 512, 70, (0, 0, 64, 70), False, False),
+        ("Q6_K", (4130,), 768, 33, None, False, False), ("Q6_K", (4100, 36), 1280, 40, None, True, True), ("Q5_K", (6400,), 256, 65, None, False, False),
+        ("Q5_K", (6400,), 768, 98, None, True, False), ("Q5_K", (6400,), 256, 120, (0, 64, 120), False, False)]
 
 
 @pytest.mark.parametrize("case", WIDE)
@@ -239,7 +243,7 @@ def test_gemm_qi_more_columns_than_a_group_host_emulation(oracle, case):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("case", WIDE + [("Q8_0", (14336, 14336), 512, 200, None, False, False), ("Q5_K", (8200,), 512, 300, None, False, False)])
+@pytest.mark.parametrize("case", WIDE + [("Q8_0", (14336, 14336), 512, 200, None, False, False), ("Q5_K", (8200,), 512, 300, None, False, False), ("Q5_K", (3200,), 2304, 200, None, True, True)])
 def test_gemm_qi_more_columns_than_a_group_gpu(oracle, dev, case):
     run_multi(oracle, GpuBackend(dev), *case, seed=8)
 
@@ -265,10 +269,10 @@ def test_long_rows_cut_by_runs_equal_the_whole_launch(oracle, dev, tname, T):
     assert got[0].any() and np.array_equal(got[0], got[1])
 
 
-def run_overflow(O, be, tname, T):
+def run_overflow(O, be, tname, T, n=36):
     """A run of superblocks whose sum is +-inf: the runs behind it start from nothing (0 * inf would be NaN), whole and cut by runs, as in the decode engine's GEMV.
     Four runs of one superblock; the first overflows f32 in every other row (K-quants: activations of 1e37; Q8_0, whose scales are f16: an infinite weight scale in every row)."""
-    t, n, k = getattr(O, tname), 36, 1024
+    t, k = getattr(O, tname), 1024
     rng = np.random.default_rng(11)
     p = O.quantize(t, (rng.standard_normal((n, k)) * 40.0).astype(np.float32)).reshape(n, 4, -1)
     x = rng.standard_normal((T, k)).astype(np.float32)
@@ -301,18 +305,18 @@ def gemm_rows(O, be, t, p, n, k, x, cut, ws_off=0, ldo=None):
     return got[:, :n]
 
 
-OVERFLOW = [("Q4_K", 5), ("Q4_K", 33), ("Q5_K", 34), ("Q6_K", 33), ("Q8_0", 5)]
+OVERFLOW = [("Q4_K", 5, 36), ("Q4_K", 33, 4132), ("Q5_K", 34, 36), ("Q6_K", 33, 36), ("Q6_K", 33, 4100), ("Q8_0", 5, 36)]  # 33 columns of 128 rows: two token tiles per wave
 
 
-@pytest.mark.parametrize("tname,T", OVERFLOW)
-def test_gemm_qi_infinite_run_host_emulation(oracle, tname, T):
-    run_overflow(oracle, HostBackend(), tname, T)
+@pytest.mark.parametrize("tname,T,n", OVERFLOW)
+def test_gemm_qi_infinite_run_host_emulation(oracle, tname, T, n):
+    run_overflow(oracle, HostBackend(), tname, T, n)
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("tname,T", OVERFLOW)
-def test_gemm_qi_infinite_run_gpu(oracle, dev, tname, T):
-    run_overflow(oracle, GpuBackend(dev), tname, T)
+@pytest.mark.parametrize("tname,T,n", OVERFLOW + [("Q5_K", 200, 3200)])
+def test_gemm_qi_infinite_run_gpu(oracle, dev, tname, T, n):
+    run_overflow(oracle, GpuBackend(dev), tname, T, n)
 
 
 def multi_call(O, be, ns, k, T, bounds, experts, max_rows):
@@ -382,9 +386,9 @@ def test_grid_of_a_window_follows_its_bound_host_emulation(oracle):
     assert (got[:32] == 0).all() and (got[32:] == 7.0).all()
 
 
-def run_bad_rows(O, be, tname, T):
+def run_bad_rows(O, be, tname, T, n=68):
     """Activation rows with NaN and infinities share their tile's matrix instructions -- block scales included -- with rows that must not see them, whole and cut by runs."""
-    t, n, k = getattr(O, tname), 68, 1024
+    t, k = getattr(O, tname), 1024
     rng = np.random.default_rng(12)
     p = O.quantize(t, (rng.standard_normal((n, k)) * 0.05).astype(np.float32)).reshape(n, -1)
     x = rng.standard_normal((T, k)).astype(np.float32)
@@ -399,15 +403,15 @@ def run_bad_rows(O, be, tname, T):
         assert not np.isfinite(got[[3, T - 2]]).any()
 
 
-BAD_ROWS = [("Q4_K", 6), ("Q4_K", 40), ("Q5_K", 40), ("Q6_K", 6), ("Q6_K", 66), ("Q8_0", 40)]
+BAD_ROWS = [("Q4_K", 6, 68), ("Q4_K", 40, 68), ("Q4_K", 40, 4132), ("Q5_K", 40, 68), ("Q6_K", 6, 68), ("Q6_K", 66, 68), ("Q6_K", 40, 4100), ("Q8_0", 40, 68)]
 
 
-@pytest.mark.parametrize("tname,T", BAD_ROWS)
-def test_gemm_qi_rows_beside_nan_and_inf_host_emulation(oracle, tname, T):
-    run_bad_rows(oracle, HostBackend(), tname, T)
+@pytest.mark.parametrize("tname,T,n", BAD_ROWS)
+def test_gemm_qi_rows_beside_nan_and_inf_host_emulation(oracle, tname, T, n):
+    run_bad_rows(oracle, HostBackend(), tname, T, n)
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("tname,T", BAD_ROWS)
-def test_gemm_qi_rows_beside_nan_and_inf_gpu(oracle, dev, tname, T):
-    run_bad_rows(oracle, GpuBackend(dev), tname, T)
+@pytest.mark.parametrize("tname,T,n", BAD_ROWS)
+def test_gemm_qi_rows_beside_nan_and_inf_gpu(oracle, dev, tname, T, n):
+    run_bad_rows(oracle, GpuBackend(dev), tname, T, n)

@@ -58,6 +58,7 @@ def test_products_that_a_cut_slows_down_stay_whole():
              (12, 8960, 1536, 300), (8, 8960, 1536, 160), (8, 3072, 1024, 512), (13, 65536, 8192, 20), (14, 65536, 8192, 32), (12, 4096, 14336, 1000)]
     parts = [(12, 2048, 2048, 200), (13, 4096, 4096, 256), (12, 28672, 4096, 32), (14, 8192, 8192, 300), (12, 4096, 14336, 700), (14, 4096, 14336, 1600), (8, 4096, 4096, 512),
              (8, 2048, 2048, 300), (8, 8192, 8192, 300), (12, 8192, 28672, 400)]
+    whole.append((13, 3072, 1024, 100))  # 96 workgroups of one token tile, not 48 of two
     for case, want in [(c, 0) for c in whole] + [(c, 1) for c in parts]:
         t, n, k, T = case
         assert cut(t, 1, (CI * 1)(n), k, T) == want, case
