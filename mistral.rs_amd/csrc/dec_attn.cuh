@@ -26,28 +26,37 @@ struct AttnArgs {
 
 // One 32-token KV block of one kv head in registers: lane (t = lane & 31, half = lane >> 5) holds K dims [(half * 8 + c) * 8, +8) of token t in kr[c];
 // lane d holds V dims d (vr[0..3]) and d + 64 (vr[4..7]) of the 32 tokens.
+// bytes = 0: nothing is read (zeros), without a branch
+constexpr int KV_BLOCK_BYTES = 32 * 128 * 2;
+__device__ __forceinline__ int4 attn_load16(__amdgpu_buffer_rsrc_t r, unsigned off) { return __builtin_bit_cast(int4, __builtin_amdgcn_raw_buffer_load_b128(r, off, 0, 0)); }
+__device__ __forceinline__ void attn_load_k(const AttnArgs &a, size_t base, int4 (&kr)[8], int bytes = KV_BLOCK_BYTES) {
+  const int lane = lane_opaque(), t = lane & 31, half = lane >> 5;
+  const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc((void *)(a.k_cache + base), (short)0, bytes, 0x00020000);
+#pragma unroll
+  for (int c = 0; c < 8; ++c) kr[c] = attn_load16(r, (unsigned)(half * 4096 + t * 16 + c * 512));
+}
+__device__ __forceinline__ void attn_load_v(const AttnArgs &a, size_t base, int4 (&vr)[8], int bytes = KV_BLOCK_BYTES) {
+  const int lane = lane_opaque();
+  const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc((void *)(a.v_cache + base), (short)0, bytes, 0x00020000);
+#pragma unroll
+  for (int h = 0; h < 2; ++h)
+#pragma unroll
+    for (int c = 0; c < 4; ++c) vr[h * 4 + c] = attn_load16(r, (unsigned)((lane + 64 * h) * 64 + c * 16));
+}
 template <bool WITH_V>
 __device__ __forceinline__ void attn_load_block(const AttnArgs &a, size_t base, int4 (&kr)[8], int4 (&vr)[8]) {
-  constexpr int BS = 32;
-  const int lane = lane_opaque(), t = lane & 31, half = lane >> 5;
-  const uint16_t *kb = a.k_cache + base + (size_t)(half * 8) * BS * 8 + t * 8;
-  const uint16_t *vb = a.v_cache + base;
-#pragma unroll
-  for (int c = 0; c < 8; ++c) kr[c] = *(const int4 *)(kb + (size_t)c * BS * 8);
-  if (WITH_V) {
-#pragma unroll
-    for (int r = 0; r < 2; ++r)
-#pragma unroll
-      for (int c = 0; c < 4; ++c) vr[r * 4 + c] = *(const int4 *)(vb + (size_t)(lane + 64 * r) * BS + c * 8);
-  }
+  attn_load_k(a, base, kr);
+  if (WITH_V) attn_load_v(a, base, vr);
 }
 // The online-softmax update of one block for the G query heads in q_s (G * 128 floats of wave-private LDS; p_s: G * 32): scores by fma chains over the lane's 64
 // dims + the other half, block max / sum trees, fast_exp, (WITH_V) o = o * alpha + P.V by fma chains.  `first` = first block of the split (l = o = 0: no correction).
 // EVERY engine attention path (decode split kernel, prompt kernel) goes through this function: same bits.
-// TAIL = false: only the sequence's last block is cleared past the context (a wave-uniform branch; 64 selects per other block less)
-template <int G, class CT, bool WITH_V, bool TAIL = true>
-__device__ __forceinline__ void attn_block_update(const AttnArgs &a, const int4 (&kr)[8], const int4 (&vr)[8], const float *q_s, float *p_s, int b, bool first, int ctx,
-                                                  int lo, float (&m)[G], float (&l)[G], float (&o0)[G], float (&o1)[G]) {
+// TAIL = false: only the sequence's last block is cleared past the context, in vr (a wave-uniform branch; 64 selects per other block less)
+// keys_read() runs when the last key has been multiplied: kr may take the next block's
+struct AttnNothing { __device__ __forceinline__ void operator()() const {} };
+template <int G, class CT, bool WITH_V, bool TAIL = true, class F = AttnNothing>
+__device__ __forceinline__ void attn_block_update(const AttnArgs &a, const int4 (&kr)[8], int4 (&vr)[8], const float *q_s, float *p_s, int b, bool first, int ctx,
+                                                  int lo, float (&m)[G], float (&l)[G], float (&o0)[G], float (&o1)[G], F keys_read = F()) {
   constexpr int HD = 128, BS = 32;
   const int lane = lane_opaque(), t = lane & 31, half = lane >> 5;
   float s[G];
@@ -65,6 +74,7 @@ __device__ __forceinline__ void attn_block_update(const AttnArgs &a, const int4 
       s[g] = fmaf(qb.x, kf[4], s[g]); s[g] = fmaf(qb.y, kf[5], s[g]); s[g] = fmaf(qb.z, kf[6], s[g]); s[g] = fmaf(qb.w, kf[7], s[g]);
     }
   }
+  keys_read();
   const bool valid = b * BS + t < ctx && b * BS + t >= lo;
 #pragma unroll
   for (int g = 0; g < G; ++g) {
@@ -90,14 +100,24 @@ __device__ __forceinline__ void attn_block_update(const AttnArgs &a, const int4 
   }
   if (!WITH_V) return;
   MRS_WAVE_SYNC();
-  const bool cut = TAIL || (b + 1) * BS > ctx;
+  if (!TAIL && (b + 1) * BS > ctx) {
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      int *d = (int *)&vr[i];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const int left = ctx - (b * BS + (i & 3) * 8 + 2 * u);  // a dword holds two tokens
+        d[u] = left > 1 ? d[u] : left == 1 ? d[u] & 0xffff : 0;
+      }
+    }
+  }
 #pragma unroll
   for (int r = 0; r < 2; ++r) {
 #pragma unroll
     for (int c = 0; c < 4; ++c) {
       float vf[8];
       unpack16<CT>(vr[r * 4 + c], vf);
-      if (cut) {
+      if (TAIL) {
 #pragma unroll
         for (int j = 0; j < 8; ++j) vf[j] = (b * BS + c * 8 + j < ctx) ? vf[j] : 0.f;  // stale slots may hold NaNs
       }
@@ -110,7 +130,7 @@ __device__ __forceinline__ void attn_block_update(const AttnArgs &a, const int4 
         acc = fmaf(pb.x, vf[4], acc); acc = fmaf(pb.y, vf[5], acc); acc = fmaf(pb.z, vf[6], acc); acc = fmaf(pb.w, vf[7], acc);
         if (r == 0) o0[g] = acc; else o1[g] = acc;
       }
-    }
+      }
   }
   MRS_WAVE_SYNC();
 }
@@ -145,21 +165,24 @@ __device__ __forceinline__ void attn_split_core(const AttnArgs &a, int kvh, int 
     for (int g = 0; g < G; ++g) sink(g, o0[g], o1[g], m[g], l[g]);
     return;
   }
-  // The next block's K / V are in flight while a block is worked on (its page index was read one block earlier): a split of several blocks -- contexts above 2048 tokens --
-  // used to pay a memory latency per block (four at 7000 tokens: a Llama-3-8B step of 2644 us, 2591 us with the merge's partials requested ahead as well)
-  int4 kn[8], vn[8];
-  unsigned page = b0 + 1 < b1 ? bt[b0 + 1] : 0;
-  auto request = [&](int b, int4 (&k)[8], int4 (&v)[8]) {
-    const size_t base = (size_t)page * a.kv_block_stride + (size_t)kvh * a.kv_head_stride;
-    if (b + 1 < b1) page = bt[b + 1];
-    attn_load_block<true>(a, base, k, v);
-  };
-  for (int b = b0; b < b1; b += 2) {
-    if (b + 1 < b1) request(b + 1, kn, vn);
-    attn_block_update<G, CT, true, false>(a, kr, vr, q_s, p_s, b, b == b0, ctx, lo, m, l, o0, o1);
-    if (b + 1 >= b1) break;
-    if (b + 2 < b1) request(b + 2, kr, vr);
-    attn_block_update<G, CT, true, false>(a, kn, vn, q_s, p_s, b + 1, false, ctx, lo, m, l, o0, o1);
+  // Splits of several blocks (model contexts above 2048 tokens): the next block's keys are requested into this one's registers as soon as these are multiplied, its values when this
+  // block's are (its page index two blocks ahead): most of a memory latency passes under arithmetic, and four waves fit a SIMD (127 registers).  A second set of registers for
+  // the next block hid all of it, but two waves fitted (241): faster where the launch's waves all did (one sequence), slower for batches.  Decode steps at a context of 6000, us,
+  // no request ahead / second set / this: 4 layers of 4096, 32 heads of 4 key heads, 1 sequence 241 / 234 / 236, 5 sequences 411 / 452 / 410, 8 sequences 494 / 568 / 494;  2 layers
+  // of 8192, 64 heads of 8, 1 sequence 308 / 320 / 307, 8 sequences 762 / 840 / 766.
+  unsigned page = bt[min(b0 + 1, b1 - 1)];
+  for (int b = b0; b < b1; ++b) {
+    const int next_bytes = b + 1 < b1 ? KV_BLOCK_BYTES : 0;
+    const size_t next = (size_t)page * a.kv_block_stride + (size_t)kvh * a.kv_head_stride;
+    page = bt[min(b + 2, b1 - 1)];
+    attn_block_update<G, CT, true, false>(a, kr, vr, q_s, p_s, b, false, ctx, lo, m, l, o0, o1, [&] {
+      __builtin_amdgcn_sched_barrier(0);
+      attn_load_k(a, next, kr, next_bytes);
+      __builtin_amdgcn_sched_barrier(0);
+    });
+    __builtin_amdgcn_sched_barrier(0);
+    attn_load_v(a, next, vr, next_bytes);
+    __builtin_amdgcn_sched_barrier(0);
   }
 #pragma unroll
   for (int g = 0; g < G; ++g) sink(g, o0[g], o1[g], m[g], l[g]);

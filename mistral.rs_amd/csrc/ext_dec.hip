@@ -191,7 +191,7 @@ __device__ __forceinline__ void attn2_merge(const Attn2Args &a, int kvh, int seq
 // Round 5 geometry: grid (kv heads, sequences, splits), G waves per workgroup: wave g = query head head0 + g of ONE split (round 4: 4 splits per workgroup, every wave
 // all G heads: 56 workgroups of 329 VGPRs at a 512-token context).  The per-head arithmetic is the same function (attn_split_core<1>): same bits; the G waves read the
 // same 16 KB of K / V (L1 / L2 hits), every wave's serial chain is 1 / G as long, and a 512-token context fills 8 x 24 = 192 CUs.
-// ONE: splits of one block (contexts up to 2048 tokens); registers for four waves per SIMD, where a batch's many small splits are what fills the chip
+// ONE: splits of one block (model contexts up to 2048 tokens).  A batch's many small splits are what fills the chip: five waves of it fit a SIMD, four of the other form
 template <int G, class CT, bool TICKET, bool ONE>
 __global__ void __launch_bounds__(64 * G) dec_attn2_kernel(const Attn2Args a) {
   constexpr int HD = 128;
@@ -246,7 +246,7 @@ __global__ void __launch_bounds__(64 * G) dec_attn2_kernel(const Attn2Args a) {
     __syncthreads();
     if (!last_s) return;
     if (tid == 0) __hip_atomic_store(tk, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);  // every other workgroup of this (seq, kv head) has already drawn
-    attn2_merge<G, true, ONE ? 8 : 16>(a, kvh, seq, ns, wave, lane, gridDim.y);
+    attn2_merge<G, true, ONE ? 8 : 12>(a, kvh, seq, ns, wave, lane, gridDim.y);
   }
 }
 // the merge as its own launch: grid (kv heads, sequences), (G + 1) / 2 waves

@@ -375,7 +375,7 @@ def _gather_kv(kc, vc, bt_row, ctx, from16):
     return k, v
 
 
-def check_attention(O, be, heads, kvh, ctxs, max_ctx, kv_dtype=1, n_out=24, window=0):
+def check_attention(O, be, heads, kvh, ctxs, max_ctx, kv_dtype=1, n_out=24, window=0, nan_past=False):
     """mrs_dec_attention (split waves + last-arriver merge + Q8_K image, ONE launch): the f32 result equals the engine-order restatement
     (orc_attention_engine) BIT FOR BIT, agrees with the restated in-tree CPU attention (single_q.rs order) to f32 rounding, and o_proj on the
     image equals o_proj on the f32 vector bit for bit.  """
@@ -389,6 +389,11 @@ def check_attention(O, be, heads, kvh, ctxs, max_ctx, kv_dtype=1, n_out=24, wind
     kc_np = to16((rng.standard_normal((nblocks, kvh, hd // 8, bs, 8)) * 0.7).astype(np.float32))
     vc_np = to16(rng.standard_normal((nblocks, kvh, hd, bs)).astype(np.float32))
     bt_np = rng.permutation(nblocks - 1)[: b * mbs].reshape(b, mbs).astype(np.uint32) + 1
+    if nan_past:  # slots past a context hold whatever an earlier sequence left
+        for i, ctx in enumerate(ctxs):
+            for p in range(ctx, mbs * bs):
+                kc_np[bt_np[i, p // bs], :, :, p % bs, :] = 0x7fff
+                vc_np[bt_np[i, p // bs], :, :, p % bs] = 0x7fff
     kc, vc, bt = be.buf(kc_np), be.buf(vc_np), be.buf(bt_np)
     cl = be.buf(np.asarray(ctxs, dtype=np.uint32))
     q_np = (rng.standard_normal((b, nq)) * 0.5).astype(np.float32)
@@ -441,6 +446,21 @@ def test_fused_attention_host_emulation(oracle, heads, kvh, ctxs, max_ctx, kvd):
 @pytest.mark.parametrize("heads,kvh,ctxs,max_ctx,kvd", [(2, 2, [45], 64, 1), (8, 1, [100, 31], 128, 0), (4, 2, [2300], 4096, 1)])
 def test_attention_more_shapes_host_emulation(oracle, heads, kvh, ctxs, max_ctx, kvd):
     check_attention(oracle, HostBackend(), heads, kvh, ctxs, max_ctx, kvd)
+
+
+# splits of two to four blocks: one block, a part of one, odd and even tokens of a dword at the end, full splits, all splits; slots past the context are NaN
+BLOCKS = [(4, 1, [1, 33, 64, 95], 2080, 1, 0), (2, 2, [32, 97, 159], 4128, 0, 0), (4, 2, [130, 1001], 6300, 1, 100), (8, 1, [257], 8192, 0, 0)]
+
+
+@pytest.mark.parametrize("heads,kvh,ctxs,max_ctx,kvd,window", BLOCKS)
+def test_attention_splits_of_several_blocks_host_emulation(oracle, heads, kvh, ctxs, max_ctx, kvd, window):
+    check_attention(oracle, HostBackend(), heads, kvh, ctxs, max_ctx, kvd, window=window, nan_past=True)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("heads,kvh,ctxs,max_ctx,kvd,window", BLOCKS + [(32, 8, [2079, 2080, 1], 2080, 1, 0), (64, 8, [5999, 6000], 6400, 1, 0), (16, 16, [7001], 7040, 0, 4096)])
+def test_attention_splits_of_several_blocks_gpu(oracle, dev, heads, kvh, ctxs, max_ctx, kvd, window):
+    check_attention(oracle, GpuBackend(dev), heads, kvh, ctxs, max_ctx, kvd, n_out=256, window=window, nan_past=True)
 
 
 @pytest.mark.gpu
