@@ -460,8 +460,8 @@ class Llama {
     const bool mmb = imgb && b >= mm_min_b;
     // Two columns of a hidden-sized row: the GEMVs' own prologue hides most of its work behind the weight requests, an image launch in front of them cannot (8B Q4_K_M, image +
     // GEMV / GEMV alone: q / k / v 4.5 + 10.9 / 15.3 us, gate / up 4.5 + 17.4 / 21.1, lm_head 4.5 + 69.2 / 73.0, and a launch less each); rows of the FFN width keep the image
-    // (o_proj and down_proj of the two columns together 9.8 us, 14.3 without).
-    const bool imgn = imgb && (b >= 3 || mmb);
+    // (o_proj and down_proj of the two columns together 9.8 us, 14.3 without), and longer hidden rows too (two layers of 8192, whole step at 1500 tokens, image / prologue: 335 / 341).
+    const bool imgn = imgb && (b >= 3 || mmb || d > 4096);
     auto qi_of = [](const std::unique_ptr<GgufMatMul> &l) -> const void * { return l && l->get_qtensor() ? l->get_qtensor()->qi : nullptr; };
     auto mm_ok = [&](const void *qi, int type, int k) { return mmb && qi && mrs_dec_mm_supported(type, k, b); };
     for (const Block &bl : blocks) {
