@@ -2,7 +2,7 @@
 //
 // What the reference does on a CPU device for a T-token prompt: every linear goes through the same QMatMul f32 fallback as decode
 // (mistralrs-quant/src/gguf/mod.rs:465-478): each activation ROW is quantized to Q8_K (K-quants), every output is a sum over the row's superblocks of
-// (d_w d_x) <integer dot> - (dmin_w d_x) <integer min term>.  Rounds 1-3 ran prompts in a different arithmetic (weights and activations rounded to bf16);
+// (d_w d_x) <integer dot> - (dmin_w d_x) <integer min term>.  Prompts also have another arithmetic (ext_gemm.hip: weights and activations rounded to bf16);
 // this kernel computes the reference's integers EXACTLY on v_mfma_f32_32x32x16_f16 and combines them in the f32 order of the decode engine ("ORD-U",
 // dec_core2.cuh / oracle orc_gemv_engine), so a token's logits and KV pages do not depend on whether it was part of a prompt or decoded:
 //   * the 6-bit sub-block scale is folded INTO the weight operand as an exact small integer in f16: Q4_K  sc (q - 8);  Q6_K  two operands
@@ -39,7 +39,7 @@ typedef int i16v __attribute__((ext_vector_type(16)));
 
 constexpr int REC_Q4K = 4096 + 512 + 128, REC_Q6K = 8192 + 512 + 128, REC_Q5K = REC_Q6K;  // Q5_K: the 5-bit values as bytes, like Q6_K's 6-bit ones
 __host__ __device__ constexpr int rec_bytes_qi(int type) { return type == T_Q4_K ? REC_Q4K : REC_Q6K; }
-// Q8_0 (round 6): a "superblock" = 8 consecutive blocks of 32; the record holds the int8 quants as they are (8 pieces) + the 8 f16 block scales per row
+// Q8_0: a "superblock" = 8 consecutive blocks of 32; the record holds the int8 quants as they are (8 pieces) + the 8 f16 block scales per row
 __host__ __device__ inline bool qi_type(int t) { return t == T_Q4_K || t == T_Q5_K || t == T_Q6_K || t == T_Q8_0; }
 __host__ __device__ inline size_t qi_tensor_bytes(int type, long long n, long long k) { return (size_t)((n + 31) / 32) * (size_t)(k / 256) * rec_bytes_qi(type); }
 
@@ -239,8 +239,8 @@ __device__ __forceinline__ h2 pkfma(h2 x, h2 s, h2 c) { return __builtin_element
 //   * reads, operand build and the next superblock's LDS-DMA stand one by one behind the matrix instructions of the step before; small workgroups (4 waves, 32 weight rows
 //     each, NT token tiles) leave two (NT = 2) or three (NT = 1) workgroups per CU, so that one's barriers and latencies run under another's arithmetic;
 //   * the projections that share their input are segments of ONE launch, the experts of a sparse-MoE prompt (windows of the expert-sorted rows) token tiles of one launch.
-//   * Q6_K takes two matrix instructions per run (sl, sh), so its vector work hides better under them; Q8_0's bound is the four f32 instructions per output and block that the
-//     engine's order of terms asks for.
+//   * Q6_K takes two matrix instructions per run (sl, sh), so its vector work hides better under them; Q8_0's bound is the four instructions per output and block: a
+//     conversion, the two multiplies and the add of the engine's term (the conversion is not part of its order: an accumulator that starts at 1.5 x 2^23 could do without).
 // Against 512-thread workgroups of 128 x 128 tiles (one per CU, their phases in lockstep), 4096 x 14336 (down) and 2 x 14336 x 4096 (gate / up) weights:
 //   Q6_K  down  512 tokens 170 -> 129 us, 1999 tokens 628 -> 457;   Q8_0  gate / up  700 tokens 402 -> 348, q / k / v 700 tokens three launches -> one of 95 us.
 // NT = 4 (128 tokens per wave, the operand built once per four matrix instructions) needs 255 registers and the earlier runs' sums in memory: 343 us against 199 us for
@@ -722,7 +722,7 @@ extern "C" int mrs_gemm_qi_multi(int type, int nt, const void *const *w_qi, cons
   return 0;
 }
 
-// ------------------------------------------------------------------------------------------------ MoE prompts in the decode engine's arithmetic (round 6)
+// ------------------------------------------------------------------------------------------------ MoE prompts in the decode engine's arithmetic
 // The decode step of a sparse-MoE layer (host/runtime.cpp forward_engine; SparseMoeBlock::forward, models/mixtral.rs:280-304) multiplies ONE token's quantized row by its
 // top-k experts' gate / up rows, quantizes silu(g) * u per expert slot, multiplies by that expert's down rows and folds the slots into the residual stream in slot order:
 // h <- (h * rs + w_0 s_0) * 1 + w_1 s_1 ...  A prompt does the same per token through the grouped form of the exact GEMM: the tokens' operand rows are gathered into
@@ -906,7 +906,7 @@ __global__ void __launch_bounds__(256) prefill_attn_exact_kernel(const dec::Attn
       o[lane] = ao[lane] * inv; o[lane + 64] = ao[lane + 64] * inv;
     }
 }
-// ------------------------------------------------------------------------------------------------ the same attention on the matrix cores (round 6)
+// ------------------------------------------------------------------------------------------------ the same attention on the matrix cores
 // prefill_attn_exact_kernel spends a prompt's attention on the vector ALU (224 us per layer at 512 tokens: 30 % of the default TTFT; quadratic: most of a 2048-token
 // prompt).  v_mfma_f32_32x32x2_f32 takes f32 operands and IS the f32 FMA chain over k, bit for bit (d = fma(a1, b1, fma(a0, b0, c)): profiles/experiments/
 // mfma_f32_probe.hip on the MI355X; MI355X_MICROARCH.md, matrix cores), so the decode kernel's chains run on it unchanged:
