@@ -239,10 +239,10 @@ __device__ __forceinline__ h2 pkfma(h2 x, h2 s, h2 c) { return __builtin_element
 //   * reads, operand build and the next superblock's LDS-DMA stand one by one behind the matrix instructions of the step before; small workgroups (4 waves, 32 weight rows
 //     each, NT token tiles) leave two (NT = 2) or three (NT = 1) workgroups per CU, so that one's barriers and latencies run under another's arithmetic;
 //   * the projections that share their input are segments of ONE launch, the experts of a sparse-MoE prompt (windows of the expert-sorted rows) token tiles of one launch.
-//   * Q6_K takes two matrix instructions per run (sl, sh), so its vector work hides better under them; Q8_0's bound is the four instructions per output and block: a
-//     conversion, the two multiplies and the add of the engine's term (the conversion is not part of its order: an accumulator that starts at 1.5 x 2^23 could do without).
+//   * Q6_K takes two matrix instructions per run (sl, sh), so its vector work hides better under them; Q8_0's bound is the three instructions per output and block: the
+//     two multiplications and the addition of the engine's term.
 // Against 512-thread workgroups of 128 x 128 tiles (one per CU, their phases in lockstep), 4096 x 14336 (down) and 2 x 14336 x 4096 (gate / up) weights:
-//   Q6_K  down  512 tokens 170 -> 129 us, 1999 tokens 628 -> 457;   Q8_0  gate / up  700 tokens 402 -> 348, q / k / v 700 tokens three launches -> one of 95 us.
+//   Q6_K  down  512 tokens 170 -> 129 us, 1999 tokens 628 -> 457;   Q8_0  gate / up  700 tokens 402 -> 263, q / k / v 700 tokens three launches -> one of 95 us.
 // NT = 4 (128 tokens per wave, the operand built once per four matrix instructions) needs 255 registers and the earlier runs' sums in memory: 343 us against 199 us for
 // 28672 x 4096 x 512 tokens.
 struct QiSeg { const uint8_t *w; unsigned w_bytes; int N; float *out; int ldo; };
@@ -272,8 +272,22 @@ constexpr int WIDE_COLS = 32;
 #define MRS_LDS_BASE(p) ((unsigned)(size_t)(__attribute__((address_space(3))) char *)(p))
 #define MRS_LDS_FRAG(type, p, addr, off) (*(const __attribute__((address_space(3))) type *)(size_t)((addr) + (off)))
 #endif
+// Q8_0: the terms of one block (see gemm_qi_wide_kernel): T (+)= (isum dw) dx for the lane's weight row and 16 tokens, whose scales sit in the 16 lanes of its row of the wave: a
+// multiplication takes lane V's through DPP (row_newbcast).  Read from LDS as four float4 per lane they were what the kernel waited for, whatever it did on the vector ALU.
+template <int V> __device__ __forceinline__ float row_bcast(float y) { return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, y), 0x150 + V, 0xf, 0xf, true)); }
+template <int... V> __device__ __forceinline__ void scale_block(float (&p)[16], float y, std::integer_sequence<int, V...>) { ((p[V] = row_bcast<V>(y) * p[V]), ...); }
+template <class F> __device__ __forceinline__ void add_block(F is_dw, float y, float (&T)[16], bool first) {
+  float p[16];
+#pragma unroll
+  for (int v = 0; v < 16; ++v) p[v] = is_dw(v);
+  __builtin_amdgcn_sched_barrier(0);  // in three rows: a DPP instruction that follows close upon its register's last write waits
+  scale_block(p, y, std::make_integer_sequence<int, 16>());
+  __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+  for (int v = 0; v < 16; ++v) T[v] = first ? p[v] : T[v] + p[v];
+}
 template <int TYPE, int NT>
-__global__ void __launch_bounds__(256, NT == 1 && TYPE != T_Q5_K ? 3 : 2) gemm_qi_wide_kernel(const WideArgs a) {
+__global__ void __launch_bounds__(256, NT == 2 || TYPE == T_Q5_K ? 2 : TYPE == T_Q8_0 ? 4 : 3) gemm_qi_wide_kernel(const WideArgs a) {
   extern __shared__ __attribute__((aligned(16))) char smem[];
   constexpr int TT_ = NT * 32, ROWB = wide_row<TYPE>, ACT_ = TT_ * ROWB, BUF_ = wide_buf<TYPE, NT>, YD_ = 512;
   constexpr int NPC = TYPE == T_Q4_K ? 4 : 8;  // 1-KiB pieces of a record
@@ -296,6 +310,7 @@ __global__ void __launch_bounds__(256, NT == 1 && TYPE != T_Q5_K ? 3 : 2) gemm_q
   auto rec_of = [&](int sb) { return (panel * (unsigned)S + (unsigned)sb) * (unsigned)rec_bytes_qi(TYPE); };
   auto load_q = [&](unsigned rec, int c) { return __builtin_amdgcn_raw_buffer_load_b128(rw, rec + (unsigned)(c * 64 + lane) * 16u, 0, 0); };
   auto load_hs = [&](unsigned rec) { return __builtin_amdgcn_raw_buffer_load_b128(rw, rec + (unsigned)(NPC * 1024) + (unsigned)nn * 16u, 0, 0); };
+  auto load_hw = [&](unsigned rec, int i) { return __builtin_amdgcn_raw_buffer_load_b32(rw, rec + (unsigned)(NPC * 1024 + 4 * i) + (unsigned)nn * 16u, 0, 0); };  // dword i of the scales
   auto load_hd = [&](unsigned rec) { return __builtin_amdgcn_raw_buffer_load_b32(rw, rec + (unsigned)(NPC * 1024 + 512) + (unsigned)nn * 4u, 0, 0); };
   // LDS-DMA of superblock sb's rows (8 NT per wave): 16-byte chunk ch of row tr at position ch ^ (tr % chunks of a row), so that the fragments' reads hit every bank.  An
   // instruction fills 1 KiB = RPI rows.  Rows past the window hold whatever follows it in the operand buffer (their outputs are not stored), rows past the buffer zeros.
@@ -351,30 +366,43 @@ __global__ void __launch_bounds__(256, NT == 1 && TYPE != T_Q5_K ? 3 : 2) gemm_q
 #pragma unroll
   for (int i = 0; i < NSTAGE; ++i) stage_q(sb_begin, 0, i);
   stage_meta(sb_begin, 0);
-  v4u wq[NPC], hs_next;
+  // Q8_0: four pieces and the scales' dwords in place, each requested again when its last block has been multiplied -- half a superblock ahead; all eight would leave three
+  // workgroups on a CU instead of four
+  constexpr int NWQ = TYPE == T_Q8_0 ? 4 : NPC;
+  v4u wq[NWQ], hs_next;
   unsigned hd_next;
 #pragma unroll
-  for (int c = 0; c < NPC; ++c) wq[c] = load_q(rec_of(sb_begin), c);
-  hs_next = load_hs(rec_of(sb_begin)); hd_next = load_hd(rec_of(sb_begin));
+  for (int c = 0; c < NWQ; ++c) wq[c] = load_q(rec_of(sb_begin), c);
+  hs_next = load_hs(rec_of(sb_begin));
+  unsigned hw8[4] = {hs_next.x, hs_next.y, hs_next.z, hs_next.w};  // Q8_0
+  if (TYPE != T_Q8_0) hd_next = load_hd(rec_of(sb_begin));
   const f16v zero = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
   unsigned mg = TYPE == T_Q6_K ? 0x64006400u : 0x54005400u;
   MRS_OPAQUE_TID(mg);  // keeps the constant in a VGPR: v_and_or_b32 takes one literal
   for (int sb = sb_begin; sb < sb_end; ++sb) {
     const int it = sb - sb_begin;
     const bool more = sb + 1 < sb_end;
-    const v4u hs = hs_next;
-    const unsigned hd = hd_next, rec_next = more ? rec_of(sb + 1) : DEAD;
+    const v4u hs = hs_next;  // (Q8_0: not used)
+    const unsigned hd = hd_next, rec = rec_of(sb), rec_next = more ? rec_of(sb + 1) : DEAD;
     const char *meta_s = smem + (it & 1) * BUF_ + ACT_;
     unsigned abase = MRS_LDS_BASE(smem) + (unsigned)((it & 1) * BUF_ + nn * ROWB + (((nn % CPR) ^ hf) << 4));
     MRS_OPAQUE_TID(abase);  // one register: a fragment's offset is one exclusive or on it
     if constexpr (TYPE == T_Q8_0) {
-      // one v_mfma_i32_32x32x32_i8 IS one block of 32 tokens x 32 rows (int32: exact); p_b = ((float)isum_b dw_b) dx_b, T = p_0 + .. + p_7 left to right: four vector
-      // instructions per output and block, which is what bounds this format
+      // one v_mfma_i32_32x32x32_i8 IS one block of 32 tokens x 32 rows (int32: exact); p_b = ((float)isum_b dw_b) dx_b, T = p_0 + .. + p_7 left to right.  What bounds this
+      // format is the vector instructions per output and block, three of them: the accumulator starts at the bits of 1.5 x 2^23, so that its bits ARE the f32 value
+      // 1.5 x 2^23 + isum (|isum| <= 2^19), and one fma takes the offset off under the multiplication by dw -- 1.5 x 2^23 dw is exact (13 bits), so the fma rounds isum dw
+      // once, as the product alone would.  A scale that is not finite would make it inf - inf, a negative one would lose the sign of a zero: such a superblock is done over with
+      // a conversion.  Gate / up of 28672 x 4096, one token tile, us, a conversion and scales from LDS / this: 700 tokens 290 / 272, 2000 tokens 780 / 739 (the fma alone, scales from LDS:
+      // 311, 831); two token tiles 263, 720.
       MRS_WAIT_VMCNT0();
       __syncthreads();
       stage_meta(sb + 1, it + 1, more);
       auto frag8 = [&](int b, int tt) -> i4v { return MRS_LDS_FRAG(i4v, smem, abase ^ (unsigned)(32 * b), tt * (32 * ROWB)); };
-      const i16v izero = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
+      constexpr int MAGIC = 0x4B400000;  // 1.5 x 2^23
+      const i16v imagic = {MAGIC, MAGIC, MAGIC, MAGIC, MAGIC, MAGIC, MAGIC, MAGIC, MAGIC, MAGIC, MAGIC, MAGIC, MAGIC, MAGIC, MAGIC, MAGIC};
+      const unsigned y_lane = (unsigned)(8 * ((lane >> 2) & 3) + 4 * hf + (lane & 3)) * 4u;  // the scale of output v = lane % 16
+      unsigned odd = 0u;
+      auto odd16 = [](unsigned w) { return (((w & 0x7c007c00u) + 0x04000400u) | w) & 0x80008000u; };  // not finite, or negative
       i4v af[2][NT];
       float Tt[NT][16];
 #pragma unroll
@@ -388,29 +416,44 @@ __global__ void __launch_bounds__(256, NT == 1 && TYPE != T_Q5_K ? 3 : 2) gemm_q
           for (int tt = 0; tt < NT; ++tt) af[(b + 1) & 1][tt] = frag8(b + 1, tt);
         }
 #pragma unroll
-        for (int tt = 0; tt < NT; ++tt) is[tt] = __builtin_amdgcn_mfma_i32_32x32x32_i8(af[b & 1][tt], __builtin_bit_cast(i4v, wq[b]), izero, 0, 0, 0);
-        wq[b] = load_q(rec_next, b);
+        for (int tt = 0; tt < NT; ++tt) is[tt] = __builtin_amdgcn_mfma_i32_32x32x32_i8(af[b & 1][tt], __builtin_bit_cast(i4v, wq[b & 3]), imagic, 0, 0, 0);
+        wq[b & 3] = b < 4 ? load_q(rec, b + 4) : load_q(rec_next, b - 4);
         if (b < NSTAGE) stage_q(sb + 1, it + 1, b, more);
-        const unsigned hw = b < 2 ? hs.x : b < 4 ? hs.y : b < 6 ? hs.z : hs.w;
-        const float dwb = half_bits_to_float((uint16_t)((b & 1) ? (hw >> 16) : (hw & 0xffffu)));
+        const unsigned hw = hw8[b / 2];
+        if (b % 2 == 0) odd |= odd16(hw);
+        float dwb = half_bits_to_float((uint16_t)((b & 1) ? (hw >> 16) : (hw & 0xffffu)));
+        MRS_OPAQUE_TID(dwb);  // in f32: not converted anew in every fma
+        if (b % 2 == 1) hw8[b / 2] = load_hw(rec_next, b / 2);
+        const float ofs = -12582912.0f * dwb;
 #pragma unroll
         for (int tt = 0; tt < NT; ++tt) {
           __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-          for (int q4 = 0; q4 < 4; ++q4) {
-            const float4 y4 = *(const float4 *)(meta_s + (b * TT_ + tt * 32 + 8 * q4 + 4 * hf) * 4);
-            const float yy[4] = {y4.x, y4.y, y4.z, y4.w};
-#pragma unroll
-            for (int k = 0; k < 4; ++k) {
-              const int v = 4 * q4 + k;
-              const float p = ((float)is[tt][v] * dwb) * yy[k];
-              Tt[tt][v] = b == 0 ? p : Tt[tt][v] + p;
-            }
-          }
+          const float y = *(const float *)(meta_s + y_lane + (b * TT_ + tt * 32) * 4);
+          auto is_dw = [&](int v) { return fmaf(__uint_as_float((unsigned)is[tt][v]), dwb, ofs); };
+          add_block(is_dw, y, Tt[tt], b == 0);
         }
         __builtin_amdgcn_sched_barrier(0);  // one block at a time: more results in flight do not fit the registers
       }
-      hs_next = load_hs(rec_next);
+      if (__ballot(odd != 0u) != 0ull) {  // wave-uniform, never in a sound model
+        i16v izero;
+#pragma unroll
+        for (int v = 0; v < 16; ++v) izero[v] = 0;
+#pragma unroll 1
+        for (int b = 0; b < 8; ++b) {
+          const unsigned hw = load_hw(rec, b / 2);
+          const float dwb = half_bits_to_float((uint16_t)((b & 1) ? (hw >> 16) : (hw & 0xffffu)));
+          const i4v wb = __builtin_bit_cast(i4v, load_q(rec, b));
+#pragma unroll
+          for (int tt = 0; tt < NT; ++tt) {
+            const i16v is = __builtin_amdgcn_mfma_i32_32x32x32_i8(frag8(b, tt), wb, izero, 0, 0, 0);
+            if (b == 0) {
+#pragma unroll
+              for (int v = 0; v < 16; ++v) Tt[tt][v] = -0.f;
+            }
+            add_block([&](int v) { return (float)is[v] * dwb; }, *(const float *)(meta_s + y_lane + (b * TT_ + tt * 32) * 4), Tt[tt], false);
+          }
+        }
+      }
 #pragma unroll
       for (int tt = 0; tt < NT; ++tt)
 #pragma unroll
@@ -665,27 +708,29 @@ static void wide_launch(int NT, const qi::WideArgs &a, dim3 grid, hipStream_t s)
 // once for both, but make the chain of a superblock longer, which is what a launch that leaves most of the chip idle waits for.  So two from 33 rows on where they make more than 32
 // workgroups (Q5_K, whose kernel of two tiles is the slowest: 96).  us, one / two tiles, each cut or whole as below (workgroups of two tiles in brackets): Q4_K 4096 x 4096 37 rows
 // (32) 11.3 / 13.7, 128 rows (64) 17.4 / 17.0, 6144 x 4096 37 rows (48) 14.7 / 14.2, 28672 x 4096 512 rows 221 / 199;  Q6_K 4096 x 14336 37 rows (32) 31.3 / 37.7, 128 rows (64)
-// 44.5 / 41.6, 1999 rows 570 / 457;  Q5_K 3072 x 1024 64 rows (24) 9.9 / 12.6, 4096 x 4096 160 rows (96) 22.0 / 25.5, 8192 x 8192 128 rows (128) 43.8 / 41.0.  Q8_0 has no operand to
-// build and a smaller workgroup's registers let one more live on a CU (q / k / v 95 / 141 and gate / up 348 / 376 at 700 rows).
-static int wide_tiles(int type, int rows, int cols) { return type == T_Q8_0 || rows <= 32 || cols * ((rows + 63) / 64) <= (type == T_Q5_K ? 96 : 32) ? 1 : 2; }
+// 44.5 / 41.6, 1999 rows 570 / 457;  Q5_K 3072 x 1024 64 rows (24) 9.9 / 12.6, 4096 x 4096 160 rows (96) 22.0 / 25.5, 8192 x 8192 128 rows (128) 43.8 / 41.0;  Q8_0 4096 x 14336 64 rows
+// (32) 39.4 / 40.5, 6144 x 4096 64 rows (48) 20.1 / 18.0, 28672 x 4096 64 rows 51.9 / 43.2, 700 rows 285 / 263, 2000 rows 779 / 720.
+static int wide_tiles(int type, int rows, int cols) { return rows <= 32 || cols * ((rows + 63) / 64) <= (type == T_Q5_K ? 96 : 32) ? 1 : 2; }
 // A launch of few workgroups is cut by runs of superblocks: four times the workgroups, a quarter of the chain, for four planes of sums written and read again.  The planes cost the same
 // at any K and the chain saved grows with it, so the line lies at a number of workgroups in proportion to K.  Whole / cut, us: Q4_K, two tiles (workgroups in brackets), 2048 x 2048
 // 200 rows (64) 16.3 / 13.2, 400 rows (112) 16.4 / 19.2, 8192 x 2048 400 rows (448) 25.7 / 39.4; 4096 x 4096 256 rows (128) 28.8 / 23.0, 300 rows (160) 29.9 / 29.1, 512 rows (256)
 // 32.6 / 37.6; 28672 x 4096 128 rows (448) 48.5 / 60.5; 8192 x 8192 300 rows (320) 80.4 / 70.5, 400 rows (448) 87.9 / 95.3; 4096 x 14336 700 rows (352) 138.6 / 129.3, 1000 rows
 // (512) 159 / 172; 8192 x 28672 400 rows (448) 307 / 284.  One tile, 32 rows: 11264 x 2048 (88) 13.2 / 12.8, 28672 x 4096 (224) 26.9 / 25.9, 57344 x 8192 (448) 76.2 / 79.0, 65536 x 8192
-// (512) 76.7 / 84.3.  Q8_0: 2048 x 2048 300 rows (160) 20.0 / 18.1, 512 rows (256) 20.6 / 23.3; 4096 x 4096 512 rows (512) 45.7 / 44.5; 8192 x 8192 300 rows (640) 93.8 / 87.7.
-// Long rows are cut beyond it too where a second, partly filled round of workgroups (two or, Q8_0, three fit a CU) would take as long as the first: K = 14336, Q4_K 1600 rows 314 / 287,
-// Q6_K 430 / 392.
-static int cut_max(int type, int NT, int K) { return type == T_Q8_0 ? std::min(K / 8, 895) : NT == 1 ? std::min(K / 18, 400) : K >= 8192 ? 895 : K / 20; }
+// (512) 76.7 / 84.3.  Q8_0, one tile: 4096 x 4096 32 rows (32) 33.5 / 14.1, 28672 x 4096 32 rows (224) 42.5 / 36.1; two: 2048 x 2048 300 rows (80) 20.5 / 17.5, 512 rows (128) 20.8 /
+// 21.5; 4096 x 4096 400 rows (224) 39.5 / 38.5, 620 rows (320) 55.2 / 50.0, 800 rows (416) 55.9 / 63.1; 8192 x 8192 300 rows (320) 106 / 83, 512 rows (512) 108 / 124.
+// Long rows are cut beyond it too where a second, partly filled round of workgroups (two fit a CU) would take as long as the first: K = 14336, Q4_K 1600 rows 314 / 287,
+// Q6_K 430 / 392, Q8_0 349 / 310.
+static int cut_line(int type, int K) { return type == T_Q8_0 ? K / 12 : K / 20; }  // two tiles
+static int cut_max(int type, int NT, int K) { return NT == 2 ? (K >= 8192 ? 895 : cut_line(type, K)) : type == T_Q8_0 ? std::min(K / 8, 895) : std::min(K / 18, 400); }
 static bool wide_cut(int type, int wgs, int K, int NT) {
   if (K / 256 < 4 || wgs > cut_max(type, NT, K)) return false;
-  return type == T_Q8_0 ? wgs != 768 : NT == 1 || wgs <= std::min(K / 20, 511) || wgs > 512;
+  return NT == 1 || wgs <= std::min(cut_line(type, K), 511) || wgs > 512;
 }
 // workspace that holds the run sums of every launch over at most n rows of weights [K] and T tokens that is cut: four planes of its outputs, of which a workgroup writes at most
 // 32 NT x 128.  Never falls as T or n grow
 extern "C" size_t mrs_gemm_qi_cut_bytes(int T, int n, int K) {
   if (T <= 0 || n <= 0 || K <= 0) return 0;
-  const int tiles = std::max(std::max(cut_max(T_Q8_0, 1, K), cut_max(T_Q4_K, 1, K)), 2 * cut_max(T_Q4_K, 2, K));
+  const int tiles = std::max(std::max(cut_max(T_Q8_0, 1, K), cut_max(T_Q4_K, 1, K)), 2 * std::max(cut_max(T_Q8_0, 2, K), cut_max(T_Q4_K, 2, K)));
   return (size_t)16 * std::min((size_t)T * n, (size_t)tiles * 32 * qi::WIDE_ROWS);
 }
 // 1: mrs_gemm_qi_multi over T rows, given a workspace, is cut

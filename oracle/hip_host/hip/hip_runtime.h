@@ -132,13 +132,14 @@ static unsigned long long ballot(bool pred) {
   wave_barrier(w, lanes);
   return m;
 }
-// v_mov_b32_dpp source lane for the controls this repo uses (all of them permutations inside a row of 16 lanes, row_mask = bank_mask = 0xf)
+// v_mov_b32_dpp source lane for the controls this repo uses (all of them inside a row of 16 lanes, row_mask = bank_mask = 0xf)
 static inline int dpp_src_lane(int lane, int ctrl) {
   const int row = lane & ~15, i = lane & 15;
   if (ctrl >= 0x000 && ctrl <= 0x0FF) return (lane & ~3) | ((ctrl >> (2 * (lane & 3))) & 3);  // quad_perm
   if (ctrl >= 0x121 && ctrl <= 0x12F) return row | ((i - (ctrl - 0x120)) & 15);                // row_ror:n  (lane i reads lane i - n)
   if (ctrl == 0x140) return row | (15 - i);                                                     // row_mirror
   if (ctrl == 0x141) return row | (i & 8) | (7 - (i & 7));                                      // row_half_mirror
+  if (ctrl >= 0x150 && ctrl <= 0x15F) return row | (ctrl - 0x150);                              // row_newbcast:n
   abort();  // a control this shim does not model
 }
 static inline int dpp(int v, int ctrl) { return exchange(v, dpp_src_lane(linear_tid() & (WAVE - 1), ctrl)); }

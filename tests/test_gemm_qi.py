@@ -415,3 +415,35 @@ def test_gemm_qi_rows_beside_nan_and_inf_host_emulation(oracle, tname, T, n):
 @pytest.mark.parametrize("tname,T,n", BAD_ROWS)
 def test_gemm_qi_rows_beside_nan_and_inf_gpu(oracle, dev, tname, T, n):
     run_bad_rows(oracle, GpuBackend(dev), tname, T, n)
+
+
+def run_odd_scales(O, be, T, n):
+    """Q8_0 weights whose block scales are negative, zero, subnormal, the largest f16, infinite or NaN, one kind per row: every output as the decode engine gives it, neighbours included."""
+    t, k = O.Q8_0, 1280
+    rng = np.random.default_rng(21)
+    p = O.quantize(t, (rng.standard_normal((n, k)) * 0.05).astype(np.float32)).reshape(n, -1).copy()
+    kinds = [-0.01, 0.0, -0.0, 5.96e-8, 65504.0, np.inf, -np.inf, np.nan]
+    for r in range(1, n, 2):  # the rows between keep their scales
+        kind = np.asarray(kinds[(r // 2) % len(kinds)], np.float16).tobytes()
+        for b in {0, r % (k // 32), k // 32 - 1}:
+            p[r, 34 * b: 34 * b + 2] = np.frombuffer(kind, np.uint8)
+    x = rng.standard_normal((T, k)).astype(np.float32)
+    want = np.concatenate([O.gemv_engine(t, p, n, k, r) for r in x], axis=0)
+    for cut in (False, True):
+        got = gemm_rows(O, be, t, p, n, k, x, cut)
+        assert np.array_equal(got, want, equal_nan=True), cut
+        assert np.isfinite(got[:, 0::2]).all() and np.isinf(want).any() and np.isnan(want).any()
+
+
+ODD_SCALES = [(3, 36), (40, 36), (40, 4132)]  # 33 columns of 128 rows: two token tiles per wave
+
+
+@pytest.mark.parametrize("T,n", ODD_SCALES[:2])
+def test_gemm_qi_q8_0_odd_scales_host_emulation(oracle, T, n):
+    run_odd_scales(oracle, HostBackend(), T, n)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("T,n", ODD_SCALES)
+def test_gemm_qi_q8_0_odd_scales_gpu(oracle, dev, T, n):
+    run_odd_scales(oracle, GpuBackend(dev), T, n)
