@@ -298,6 +298,16 @@ size_t mrs_gemm_qi_cut_bytes(int T, int n, int K);
 int mrs_gemm_qi_is_cut(int ggml_type, int n_tensors, const int *N, int K, int T);
 int mrs_gemm_qi_multi(int ggml_type, int n_tensors, const void *const *w_qi, const int *N, int K, const void *act, int T, float *const *out, const int *ldo, int accumulate,
                       const int *bounds, int experts, int max_rows, void *workspace, size_t workspace_bytes, void *stream);
+/* What stands between a prompt's products, in fewer launches.  mrs_gemm_qi_multi_planes: mrs_gemm_qi_multi over T rows that leaves the run sums of a cut launch as they are: 1 = the
+ * workspace begins with the planes [4][T][sum N] and `out` is untouched, 0 = `out` is complete.  mrs_qi_quantize_added: h <- h + ((c0 + c1) + c2) + c3 of planes `part` [4][T][K], then
+ * mrs_qi_quantize_for of h with the norm (K up to 14336).  mrs_prefill_rope_cache: q / k / v rows [T][ld] (or, plane != 0, the first of four planes `plane` floats apart, added the same
+ * way) -> RoPE (`pairs` rotated pairs of 128 dims, interleaved or, neox, halves) -> q_out [T][heads * 128] and the pages of 32 tokens (kv_dtype 0 f16, 1 bf16; slot -1: none). */
+int mrs_gemm_qi_multi_planes(int ggml_type, int n_tensors, const void *const *w_qi, const int *N, int K, const void *act, int T, float *const *out, const int *ldo, int accumulate,
+                             void *workspace, size_t workspace_bytes, void *stream);
+int mrs_qi_quantize_added(int w_ggml_type, float *h, const float *part, const float *norm_w, float eps, int T, int K, void *act, void *stream);
+int mrs_prefill_rope_cache(const float *q, size_t q_plane, int q_ld, const float *k, size_t k_plane, int k_ld, const float *v, size_t v_plane, int v_ld, float *q_out, void *k_cache,
+                           void *v_cache, const int64_t *slots, const uint32_t *positions, const float *cos_t, const float *sin_t, int T, int heads, int kv_heads, int pairs, int neox,
+                           int kv_dtype, void *stream);
 int mrs_gemm_qi_win(const void *w_qi, int ggml_type, int N, int K, const void *act, int T_total, const int *win, int max_rows, float *out, int ldo, int accumulate, void *stream);
 int mrs_qi_gather_rows(int w_ggml_type, const void *act_src, int T, void *act_dst, int R, int K, const int *sorted_routes, int top_k, int *inv, void *stream);
 int mrs_moe_fold_exact(float *h, float resid_scale, const float *y_sorted, const int *inv, const float *weights, int T, int d, int top_k, void *stream);

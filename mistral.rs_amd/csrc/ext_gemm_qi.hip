@@ -132,81 +132,113 @@ __global__ void __launch_bounds__(256) qi_repack_kernel(const uint8_t *__restric
 }
 
 // ------------------------------------------------------------------------------------------------ activations: f32 rows -> operand buffers
-// One workgroup (512 threads) per token row: the decode engine's prologue (act_issue_all / act_finish_all: engine-order RmsNorm, candle's Q8_K quantizer)
-// builds the row's image in LDS; the image is then written out as the GEMM's operands:
+// Rows with an RmsNorm: one workgroup (512 threads) per token row, the decode engine's prologue (act_issue_all / act_finish_all: engine-order RmsNorm, candle's Q8_K quantizer)
+// builds the row's image in LDS.  Rows without: superblocks know nothing of each other, two per wave.  Either way the image is written out as the GEMM's operands:
 //   qf [S][T][256] f16: the int8 quants, inside every group of 8 in the operand's slot order;  yd [S][T] f32;  bsf [S][T][16] f16: the 16 run sums.
-// GLU = true: the row is silu_engine(g) * u (the decode engine's gate / up epilogue expression), g = x, u = x2.
+// GLU: the row is silu_engine(g) * u (the decode engine's gate / up epilogue expression), g = x, u = x2.
 struct QuantArgs {
   const float *x, *x2; int ldx; const float *norm_w; float eps; int K, T;
   _Float16 *qf; float *yd; _Float16 *bsf;
-  float *xtmp;  // GLU: f32 scratch [T][K] for the activated row (the prologue reads its input from memory)
+  float *xtmp;  // GLU and norm: f32 scratch [T][K] for the activated row (the prologue reads its input from memory)
   int mode;     // ACT_Q8K (K-quant weights) / ACT_Q80 (Q8_0 weights: quantize_row_q8_0 per 32 values; outputs q8 [S][T][256] int8 in element order at `qf`, the block
                 // scales f32(f16(d)) block-major [S][8][T] at `bsf`)
+  const float *part; float *h;  // PART: the four run sums [4][T][K] of the product that is added to the rows `h` first (x = h, ldx = K)
 };
-// GLU: 0: the row as it is; 1: silu_engine(g) * u formed in the registers the quantizer reads (rows of up to 2048 NPX values, no norm); 2: the same through xtmp.  Form 2 wrote
-// and re-read the row: 512 / 1999 tokens of 14336 values 26 / 85 us.
-template <int GLU>
+__device__ __forceinline__ float4 glu4(float4 g, float4 u) { return make_float4(silu_engine(g.x) * u.x, silu_engine(g.y) * u.y, silu_engine(g.z) * u.z, silu_engine(g.w) * u.w); }
+// superblock sb of token t out of an image: `q` its 256 int8, `d` its scale(s), `bs` its run sums; worker `i` of `n`
+__device__ __forceinline__ void store_operands(const QuantArgs &a, int sb, int t, const char *q, const float *d, const int *bs, int i, int n) {
+  const size_t row = (size_t)sb * a.T + t;
+  if (a.mode == ACT_Q80) {
+    for (int ch = i; ch < 16; ch += n) *(v4u *)((int8_t *)a.qf + row * 256 + ch * 16) = *(const v4u *)(q + ch * 16);
+    for (int b = i; b < 8; b += n) ((float *)a.bsf)[((size_t)sb * 8 + b) * a.T + t] = d[b];
+    return;
+  }
+  for (int g8 = i; g8 < 32; g8 += n) {
+    const int8_t *qg = (const int8_t *)(q + g8 * 8);
+    h8 o;
+#pragma unroll
+    for (int jj = 0; jj < 8; ++jj) o[jj] = (_Float16)(float)qg[perm8(jj)];
+    *(h8 *)(a.qf + row * 256 + g8 * 8) = o;
+  }
+  for (int r = i; r < 16; r += n) a.bsf[row * 16 + r] = (_Float16)(float)bs[r];
+  if (i == 0) a.yd[row] = d[0];
+}
+// rows with a norm.  GLU: the activated row goes through xtmp.  PART: the row is h + ((c0 + c1) + c2) + c3, the sum gemm_qi_reduce_kernel would have left in h (written there as
+// well), formed in the registers the norm reads: a launch less between a cut product and the next one's operands (rows of up to 2048 NPX values; 37 rows of 4096 4.1 + 4.9 us, here
+// 5.6, 512 rows 5.0 + 7.0, here 12.0 with the planes from memory).
+template <bool GLU, bool PART>
 __global__ void __launch_bounds__(NT) qi_quantize_kernel(const QuantArgs a) {
   extern __shared__ __attribute__((aligned(16))) char smem[];
   __shared__ float red[8];
   const int tid = tid_opaque(), t = blockIdx.x, K = a.K, S = K / 256;
   const float *xr = a.x + (size_t)t * a.ldx, *ur = GLU ? a.x2 + (size_t)t * a.ldx : nullptr;
-  auto glu4 = [](float4 g, float4 u) { return make_float4(silu_engine(g.x) * u.x, silu_engine(g.y) * u.y, silu_engine(g.z) * u.z, silu_engine(g.w) * u.w); };
   const int qw = __builtin_amdgcn_readfirstlane(tid >> 6);
-  if constexpr (GLU == 1) {
-    ActRegs<1> pre{};
-    float4 g[NPX], u[NPX];
-    const __amdgpu_buffer_rsrc_t rg = __builtin_amdgcn_make_buffer_rsrc((void *)xr, (short)0, K * 4, 0x00020000), ru = __builtin_amdgcn_make_buffer_rsrc((void *)ur, (short)0, K * 4, 0x00020000);
+  if constexpr (GLU) {
+    float *dst = a.xtmp + (size_t)t * K;
+    for (int e = tid * 4; e < K; e += NT * 4) *(float4 *)(dst + e) = glu4(*(const float4 *)(xr + e), *(const float4 *)(ur + e));
+    __syncthreads();  // the same threads read back what they wrote (tid * 4 + j * 2048), the barrier orders the other waves' view of nothing: cheap insurance
+    xr = dst;
+  }
+  ActRegs<1> pre = act_issue_all<1>(xr, (unsigned)K * 4u, a.norm_w, K, qw);
+  if constexpr (PART) {
+    const size_t tot = (size_t)a.T * K;
+    float4 c[4][2];  // two pieces in flight at a time
+    auto request = [&](int j) {
+      const int e = tid * 4 + j * 2048;
 #pragma unroll
-    for (int j = 0; j < NPX; ++j) {  // past the row: zeros
-      g[j] = as_f4(__builtin_amdgcn_raw_buffer_load_b128(rg, (unsigned)tid * 16u + (unsigned)j * 8192u, 0, 0));
-      u[j] = as_f4(__builtin_amdgcn_raw_buffer_load_b128(ru, (unsigned)tid * 16u + (unsigned)j * 8192u, 0, 0));
-    }
+      for (int p = 0; p < 4; ++p) c[p][j & 1] = e < K ? *(const float4 *)(a.part + p * tot + (size_t)t * K + e) : make_float4(0.f, 0.f, 0.f, 0.f);
+    };
+    request(0);
 #pragma unroll
     for (int j = 0; j < NPX; ++j) {
-      const float4 v = glu4(g[j], u[j]);
-      pre.xv[0][j] = v4u{__float_as_uint(v.x), __float_as_uint(v.y), __float_as_uint(v.z), __float_as_uint(v.w)};
+      if (j * 2048 >= K) break;
+      if (j + 1 < NPX) request(j + 1);
+      const int e = tid * 4 + j * 2048, o = j & 1;
+      const float4 old = as_f4(pre.xv[0][j]);
+      const float4 r = make_float4(old.x + (((c[0][o].x + c[1][o].x) + c[2][o].x) + c[3][o].x), old.y + (((c[0][o].y + c[1][o].y) + c[2][o].y) + c[3][o].y),
+                                   old.z + (((c[0][o].z + c[1][o].z) + c[2][o].z) + c[3][o].z), old.w + (((c[0][o].w + c[1][o].w) + c[2][o].w) + c[3][o].w));
+      if (e < K) *(float4 *)(a.h + (size_t)t * K + e) = r;
+      pre.xv[0][j] = v4u{__float_as_uint(r.x), __float_as_uint(r.y), __float_as_uint(r.z), __float_as_uint(r.w)};
     }
-    act_finish_all<1>(smem, red, pre, xr, K, nullptr, a.eps, K, a.mode, qw);
-  } else {
-    if constexpr (GLU == 2) {
-      float *dst = a.xtmp + (size_t)t * K;
-      for (int e = tid * 4; e < K; e += NT * 4) *(float4 *)(dst + e) = glu4(*(const float4 *)(xr + e), *(const float4 *)(ur + e));
-      __syncthreads();  // the same threads read back what they wrote (tid * 4 + j * 2048), the barrier orders the other waves' view of nothing: cheap insurance
-      xr = dst;
-    }
-    const ActRegs<1> pre = act_issue_all<1>(xr, (unsigned)K * 4u, a.norm_w, K, qw);
-    act_finish_all<1>(smem, red, pre, xr, K, a.norm_w, a.eps, K, a.mode, qw);
   }
+  act_finish_all<1>(smem, red, pre, xr, K, a.norm_w, a.eps, K, a.mode, qw);
   __syncthreads();
   const Act act = act_view(smem, K, 1, a.mode);
-  if (a.mode == ACT_Q80) {
-    int8_t *q8 = (int8_t *)a.qf;
-    float *yd8 = (float *)a.bsf;
-    for (int gi = tid; gi < S * 16; gi += NT) {  // 16-byte chunks of the superblock's 256 quants
-      const int sb = gi >> 4, ch = gi & 15;
-      *(v4u *)(q8 + ((size_t)sb * a.T + t) * 256 + ch * 16) = *(const v4u *)(act.q + act.qoff(sb) + ch * 16);
-    }
-    for (int i = tid; i < S * 8; i += NT) {
-      const int sb = i >> 3, b = i & 7;
-      yd8[((size_t)sb * 8 + b) * a.T + t] = act.d[(size_t)sb * act.dw + b];
-    }
-    return;
+  for (int gi = tid; gi < S * 32; gi += NT) {  // 32 workers per superblock
+    const int sb = gi >> 5;
+    store_operands(a, sb, t, act.q + act.qoff(sb), act.d + (size_t)sb * act.dw, act.bs + (size_t)sb * ACT_BS, gi & 31, 32);
   }
-  // thread -> (superblock, group of 8 elements): 32 groups per superblock
-  for (int gi = tid; gi < S * 32; gi += NT) {
-    const int sb = gi >> 5, g8 = gi & 31;
-    const int8_t *q = (const int8_t *)(act.q + act.qoff(sb) + g8 * 8);
-    h8 o;
+}
+// rows without a norm: wave w of the launch's row quantizes superblocks 2 w, 2 w + 1 (two interleaved chains) through an image of their own.  One workgroup per row left a short
+// prompt to T workgroups of a serial chain: 37 / 512 rows silu(g) u of 14336 values 10.0 / 22.0 us, here 5.0 / 17.5, of 4096 plain values 4.9 / 7.0, here 4.3 / 5.6.
+constexpr int QS_WAVES = 4, QS_SB = 2 * QS_WAVES;  // superblocks of a workgroup
+constexpr int QS_IMG = (4 * (256 + 16) + 4 * (48 + ACT_BS * 4) + 15) & ~15;  // act_bytes(512, 1)
+template <bool GLU>
+__global__ void __launch_bounds__(64 * QS_WAVES) qi_quantize_split_kernel(const QuantArgs a) {
+  __shared__ __attribute__((aligned(16))) char img_s[QS_WAVES][QS_IMG];
+  const int tid = tid_opaque(), lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), t = blockIdx.x, S = a.K / 256;
+  const int sb0 = ((int)blockIdx.y * QS_WAVES + wave) * 2;
+  if (sb0 >= S) return;  // no workgroup barrier below
+  const __amdgpu_buffer_rsrc_t rx = __builtin_amdgcn_make_buffer_rsrc((void *)(a.x + (size_t)t * a.ldx), (short)0, a.K * 4, 0x00020000);
+  const __amdgpu_buffer_rsrc_t ru = __builtin_amdgcn_make_buffer_rsrc((void *)((GLU ? a.x2 : a.x) + (size_t)t * a.ldx), (short)0, a.K * 4, 0x00020000);
+  float4 v[2], u[2];
 #pragma unroll
-    for (int jj = 0; jj < 8; ++jj) o[jj] = (_Float16)(float)q[perm8(jj)];
-    *(h8 *)(a.qf + ((size_t)sb * a.T + t) * 256 + g8 * 8) = o;
+  for (int n = 0; n < 2; ++n) {  // past the row: zeros
+    v[n] = as_f4(__builtin_amdgcn_raw_buffer_load_b128(rx, (unsigned)(sb0 + n) * 1024u + (unsigned)lane * 16u, 0, 0));
+    if (GLU) u[n] = as_f4(__builtin_amdgcn_raw_buffer_load_b128(ru, (unsigned)(sb0 + n) * 1024u + (unsigned)lane * 16u, 0, 0));
   }
-  for (int i = tid; i < S * 16; i += NT) {
-    const int sb = i >> 4, r = i & 15;
-    a.bsf[((size_t)sb * a.T + t) * 16 + r] = (_Float16)(float)act.bs[(size_t)sb * ACT_BS + r];
+  if (GLU) {
+#pragma unroll
+    for (int n = 0; n < 2; ++n) v[n] = glu4(v[n], u[n]);
   }
-  for (int sb = tid; sb < S; sb += NT) a.yd[(size_t)sb * a.T + t] = act.d[sb];
+  const int sbs[2] = {0, 1};
+  const bool live[2] = {true, true};
+  quantize_multi<2>(v, sbs, live, 0, a.mode, img_s[wave], 512, 1);
+  MRS_WAVE_SYNC();
+  const int n = lane >> 5;
+  if (sb0 + n >= S) return;
+  const Act act = act_view(img_s[wave], 512, 1, a.mode);
+  store_operands(a, sb0 + n, t, act.q + act.qoff(n), act.d + n * act.dw, act.bs + n * ACT_BS, lane & 31, 32);
 }
 
 // ------------------------------------------------------------------------------------------------ the GEMM
@@ -604,6 +636,88 @@ __global__ void __launch_bounds__(256, NT == 2 || TYPE == T_Q5_K ? 2 : TYPE == T
     for (int v = 0; v < 16; ++v) st32(pend[tt][v], ro, at(tt, v));
 }
 
+// The projections of a prompt's tokens on their way to the attention: RoPE on q and k (rope_pair in f32, as rotary_embedding_positions), k and v into their pages (rounded as
+// reshape_and_cache does), and where a projection's launch was cut its four run sums are added here.  One launch instead of two (up to four with the reductions), 4 - 5 us each at
+// short prompts (37 tokens 17 us, here 4.5); a page's values leave four tokens at a time instead of 2 bytes each, 64 bytes apart.
+// Workgroup = (8 tokens, one head of q, k or v).  head size 128, pages of 32 tokens.
+struct RopeSrc { const float *p; size_t plane; int ld; };  // rows [T][ld]; plane != 0: the first of four planes of run sums
+struct RopeCacheArgs {
+  RopeSrc q, k, v;
+  float *q_out;  // [T][heads * 128]
+  uint16_t *k_cache, *v_cache;
+  const int64_t *slots; const uint32_t *positions; const float *cos_t, *sin_t;
+  int T, heads, kv_heads, pairs, f16;
+};
+template <bool NEOX>
+__global__ void __launch_bounds__(256) prefill_rope_cache_kernel(const RopeCacheArgs a) {
+  const int tid = threadIdx.x, y = blockIdx.y, t0 = blockIdx.x * 8;
+  auto bits = [&](float f) { return a.f16 ? float_to_half_bits(f) : float_to_bf16_bits(f); };
+  if (y >= a.heads + a.kv_heads) {  // v: thread = (dim, four tokens)
+    const int head = y - a.heads - a.kv_heads, dim = tid & 127, tb = t0 + (tid >> 7) * 4;
+    float f[4], c[3][4]; uint16_t w[4]; int64_t slot[4];
+    auto row = [&](int i) { return a.v.p + (size_t)min(tb + i, a.T - 1) * a.v.ld + head * 128 + dim; };
+#pragma unroll
+    for (int i = 0; i < 4; ++i) { f[i] = *row(i); slot[i] = tb + i < a.T ? a.slots[tb + i] : -1; }
+    if (a.v.plane) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int p = 0; p < 3; ++p) c[p][i] = row(i)[(p + 1) * a.v.plane];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) f[i] = ((f[i] + c[0][i]) + c[1][i]) + c[2][i];
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) w[i] = bits(f[i]);
+    auto at = [&](int64_t s) { return a.v_cache + ((size_t)(s >> 5) * a.kv_heads + head) * 4096 + (size_t)dim * 32 + (s & 31); };
+    if (slot[0] >= 0 && (slot[0] & 3) == 0 && slot[1] == slot[0] + 1 && slot[2] == slot[0] + 2 && slot[3] == slot[0] + 3)
+      *(uint2 *)at(slot[0]) = make_uint2((unsigned)w[0] | ((unsigned)w[1] << 16), (unsigned)w[2] | ((unsigned)w[3] << 16));
+    else {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) if (slot[i] >= 0) *at(slot[i]) = w[i];  // a slot of -1: no page (a padding token)
+    }
+    return;
+  }
+  const bool is_q = y < a.heads;
+  const int head = is_q ? y : y - a.heads, t = t0 + (tid >> 5), quad = tid & 31;
+  if (t >= a.T) return;
+  const RopeSrc &src = is_q ? a.q : a.k;
+  const float *row = src.p + (size_t)t * src.ld + head * 128;
+  auto load = [&](int d) {
+    const float4 c0 = *(const float4 *)(row + d);
+    if (!src.plane) return c0;
+    const float4 c1 = *(const float4 *)(row + src.plane + d), c2 = *(const float4 *)(row + 2 * src.plane + d), c3 = *(const float4 *)(row + 3 * src.plane + d);
+    return make_float4(((c0.x + c1.x) + c2.x) + c3.x, ((c0.y + c1.y) + c2.y) + c3.y, ((c0.z + c1.z) + c2.z) + c3.z, ((c0.w + c1.w) + c2.w) + c3.w);
+  };
+  const int64_t slot = is_q ? 0 : a.slots[t];
+  auto put = [&](int d, float4 v) {  // dims d .. d + 3
+    if (is_q) *(float4 *)(a.q_out + ((size_t)t * a.heads + head) * 128 + d) = v;
+    else if (slot >= 0)
+      *(uint2 *)(a.k_cache + ((size_t)(slot >> 5) * a.kv_heads + head) * 4096 + (size_t)(d >> 3) * 256 + (size_t)(slot & 31) * 8 + (d & 7)) =
+          make_uint2((unsigned)bits(v.x) | ((unsigned)bits(v.y) << 16), (unsigned)bits(v.z) | ((unsigned)bits(v.w) << 16));
+  };
+  const size_t trow = (size_t)a.positions[t] * a.pairs;
+  if (NEOX) {  // pairs (i, i + 64): full rotation only
+    if (quad >= 16) return;
+    const float4 x = load(quad * 4), w = load(64 + quad * 4);
+    const float xs[4] = {x.x, x.y, x.z, x.w}, ys[4] = {w.x, w.y, w.z, w.w};
+    float xo[4], yo[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) rope_pair<float>(xs[i], ys[i], a.cos_t[trow + quad * 4 + i], a.sin_t[trow + quad * 4 + i], xo[i], yo[i]);
+    put(quad * 4, make_float4(xo[0], xo[1], xo[2], xo[3]));
+    put(64 + quad * 4, make_float4(yo[0], yo[1], yo[2], yo[3]));
+  } else {
+    float c0 = 1.f, s0 = 0.f, c1 = 1.f, s1 = 0.f;
+    if (a.pairs > 0) {  // requested before the row; pairs past the rotated ones take the last one's and are not used
+      const size_t p0 = trow + min(2 * quad, a.pairs - 1), p1 = trow + min(2 * quad + 1, a.pairs - 1);
+      c0 = a.cos_t[p0]; s0 = a.sin_t[p0]; c1 = a.cos_t[p1]; s1 = a.sin_t[p1];
+    }
+    float4 v = load(quad * 4);
+    if (2 * quad < a.pairs) rope_pair<float>(v.x, v.y, c0, s0, v.x, v.y);
+    if (2 * quad + 1 < a.pairs) rope_pair<float>(v.z, v.w, c1, s1, v.z, v.w);
+    put(quad * 4, v);
+  }
+}
+
 // out[t][n] (+)= ((c0 + c1) + c2) + c3 of the four run sums (the row combination of ORD-U), all tensors of the launch: workgroup (row t, 1024 of its columns).  One launch per
 // tensor cost 3 - 5 us each at short prompts (7 of a layer's 16 launches at 37 tokens).
 __global__ void __launch_bounds__(256) gemm_qi_reduce_kernel(const WideArgs a) {
@@ -662,18 +776,34 @@ extern "C" int mrs_qi_quantize_for(int w_type, const float *x, const float *x2, 
 extern "C" int mrs_qi_quantize(const float *x, const float *x2, int ldx, const float *norm_w, float eps, int T, int K, void *act, float *xtmp, void *stream) {
   return mrs_qi_quantize_for(T_Q4_K, x, x2, ldx, norm_w, eps, T, K, act, xtmp, stream);
 }
+template <bool GLU, bool PART> static int qi_quantize_rows(const qi::QuantArgs &a, void *stream) {  // rows with a norm
+  const size_t lds = (dec2::act_bytes(a.K, 1) + 15) & ~(size_t)15;
+  if (lds > 158 * 1024) return -2;
+  auto kern = qi::qi_quantize_kernel<GLU, PART>;
+  lds_attr_once((const void *)kern, 158 * 1024);
+  hipLaunchKernelGGL(kern, dim3(a.T), dim3(dec2::NT), lds, (hipStream_t)stream, a);
+  return 0;
+}
 extern "C" int mrs_qi_quantize_for(int w_type, const float *x, const float *x2, int ldx, const float *norm_w, float eps, int T, int K, void *act, float *xtmp, void *stream) {
   if (!x || !act || T <= 0 || K <= 0 || K % 256 || (x2 && !xtmp) || !qi::qi_type(w_type)) return -1;
   qi::QuantArgs a{};
   a.x = x; a.x2 = x2; a.ldx = ldx; a.norm_w = norm_w; a.eps = eps; a.K = K; a.T = T; a.xtmp = xtmp; a.mode = dec2::act_mode_for(w_type);
   qi_split(act, T, K, &a.qf, &a.yd, &a.bsf);
-  const size_t lds = (dec2::act_bytes(K, 1) + 15) & ~(size_t)15;
-  if (lds > 158 * 1024) return -2;
-  auto go = [&](auto kern) { lds_attr_once((const void *)kern, 158 * 1024); hipLaunchKernelGGL(kern, dim3(T), dim3(dec2::NT), lds, (hipStream_t)stream, a); };
-  if (!x2) go(qi::qi_quantize_kernel<0>);
-  else if (K <= 2048 * dec2::NPX && !norm_w) go(qi::qi_quantize_kernel<1>);
-  else go(qi::qi_quantize_kernel<2>);
-  return 0;
+  if (!norm_w) {
+    const dim3 grid(T, (K / 256 + qi::QS_SB - 1) / qi::QS_SB);
+    if (x2) hipLaunchKernelGGL(qi::qi_quantize_split_kernel<true>, grid, dim3(64 * qi::QS_WAVES), 0, (hipStream_t)stream, a);
+    else hipLaunchKernelGGL(qi::qi_quantize_split_kernel<false>, grid, dim3(64 * qi::QS_WAVES), 0, (hipStream_t)stream, a);
+    return 0;
+  }
+  return x2 ? qi_quantize_rows<true, false>(a, stream) : qi_quantize_rows<false, false>(a, stream);
+}
+// mrs_qi_quantize_for of the rows h + ((c0 + c1) + c2) + c3, c_p = plane p of part [4][T][K] (mrs_gemm_qi_multi_planes), which are also left in h: gemm_qi_reduce_kernel's sum
+extern "C" int mrs_qi_quantize_added(int w_type, float *h, const float *part, const float *norm_w, float eps, int T, int K, void *act, void *stream) {
+  if (!h || !part || !norm_w || !act || T <= 0 || K <= 0 || K % 256 || K > 2048 * dec2::NPX || !qi::qi_type(w_type) || (((uintptr_t)h | (uintptr_t)part) & 15)) return -1;
+  qi::QuantArgs a{};
+  a.x = h; a.ldx = K; a.norm_w = norm_w; a.eps = eps; a.K = K; a.T = T; a.mode = dec2::act_mode_for(w_type); a.part = part; a.h = h;
+  qi_split(act, T, K, &a.qf, &a.yd, &a.bsf);
+  return qi_quantize_rows<false, true>(a, stream);
 }
 // out[t * ldo + n] (+)= W[n] . act[t] for t < T, n < N in the decode engine's arithmetic and f32 order.  w_qi: mrs_gemm_qi_repack output; act: mrs_qi_quantize output.
 // workspace for the split launch of GEMMs with few workgroups (N * T small): 4 x T x N floats
@@ -744,8 +874,8 @@ extern "C" int mrs_gemm_qi_is_cut(int type, int nt, const int *N, int K, int T) 
   const int NT = wide_tiles(type, T, gx);
   return wide_cut(type, gx * ((T + 32 * NT - 1) / (32 * NT)), K, NT);
 }
-extern "C" int mrs_gemm_qi_multi(int type, int nt, const void *const *w_qi, const int *N, int K, const void *act, int T, float *const *out, const int *ldo, int accumulate,
-                                 const int *bounds, int experts, int max_rows, void *workspace, size_t workspace_bytes, void *stream) {
+static int gemm_qi_launch(int type, int nt, const void *const *w_qi, const int *N, int K, const void *act, int T, float *const *out, const int *ldo, int accumulate,
+                          const int *bounds, int experts, int max_rows, void *workspace, size_t workspace_bytes, bool keep_planes, void *stream) {
   if (!w_qi || !N || !act || !out || !ldo || nt < 1 || nt > 3 || !qi::qi_type(type) || T <= 0 || K <= 0 || K % 256 || (bounds && (experts <= 0 || max_rows <= 0))) return -1;
   int n_all = 0;
   for (int i = 0; i < nt; ++i) {
@@ -774,7 +904,31 @@ extern "C" int mrs_gemm_qi_multi(int type, int nt, const void *const *w_qi, cons
     case T_Q6_K: wide_launch<T_Q6_K>(NT, a, grid, s); break;
     default: wide_launch<T_Q8_0>(NT, a, grid, s); break;
   }
+  if (a.ksplit > 1 && keep_planes) return 1;
   if (a.ksplit > 1) hipLaunchKernelGGL(qi::gemm_qi_reduce_kernel, dim3(T, (n_all + 1023) / 1024), dim3(256), 0, s, a);
+  return 0;
+}
+extern "C" int mrs_gemm_qi_multi(int type, int nt, const void *const *w_qi, const int *N, int K, const void *act, int T, float *const *out, const int *ldo, int accumulate,
+                                 const int *bounds, int experts, int max_rows, void *workspace, size_t workspace_bytes, void *stream) {
+  return gemm_qi_launch(type, nt, w_qi, N, K, act, T, out, ldo, accumulate, bounds, experts, max_rows, workspace, workspace_bytes, false, stream);
+}
+// the same over T rows, but the run sums of a launch that is cut stay as they are: 1 = workspace holds the planes [4][T][sum N] (the tensors side by side) and `out` is as it was; 0 = out
+extern "C" int mrs_gemm_qi_multi_planes(int type, int nt, const void *const *w_qi, const int *N, int K, const void *act, int T, float *const *out, const int *ldo, int accumulate,
+                                        void *workspace, size_t workspace_bytes, void *stream) {
+  return gemm_qi_launch(type, nt, w_qi, N, K, act, T, out, ldo, accumulate, nullptr, 0, 0, workspace, workspace_bytes, true, stream);
+}
+// q / k / v rows of T prompt tokens (f32 [T][ld], or the four planes of run sums at `plane` floats from one another) -> RoPE -> q_out [T][heads * 128], pages (32 tokens, head size 128)
+extern "C" int mrs_prefill_rope_cache(const float *q, size_t q_plane, int q_ld, const float *k, size_t k_plane, int k_ld, const float *v, size_t v_plane, int v_ld, float *q_out, void *k_cache,
+                                      void *v_cache, const int64_t *slots, const uint32_t *positions, const float *cos_t, const float *sin_t, int T, int heads, int kv_heads, int pairs, int neox,
+                                      int kv_dtype, void *stream) {
+  if (!q || !k || !v || !q_out || !k_cache || !v_cache || !slots || !positions || !cos_t || !sin_t || T <= 0 || heads <= 0 || kv_heads <= 0 || pairs < 0 || pairs > 64 || (neox && pairs != 64) ||
+      (kv_dtype != 0 && kv_dtype != 1) || q_ld % 4 || k_ld % 4 || q_plane % 4 || k_plane % 4 || (((uintptr_t)q | (uintptr_t)k | (uintptr_t)q_out) & 15) ||
+      (((uintptr_t)k_cache | (uintptr_t)v_cache) & 7)) return -1;
+  const qi::RopeCacheArgs a{{q, q_plane, q_ld}, {k, k_plane, k_ld}, {v, v_plane, v_ld}, q_out, (uint16_t *)k_cache, (uint16_t *)v_cache, slots, positions, cos_t, sin_t, T, heads, kv_heads, pairs,
+                            kv_dtype == 0 ? 1 : 0};
+  const dim3 grid((T + 7) / 8, heads + 2 * kv_heads);
+  if (neox) hipLaunchKernelGGL(qi::prefill_rope_cache_kernel<true>, grid, dim3(256), 0, (hipStream_t)stream, a);
+  else hipLaunchKernelGGL(qi::prefill_rope_cache_kernel<false>, grid, dim3(256), 0, (hipStream_t)stream, a);
   return 0;
 }
 

@@ -724,44 +724,79 @@ class Llama {
     const int d = cfg.hidden_size, hd = cfg.head_dim, nq = cfg.num_heads * hd, nkv = cfg.num_kv_heads * hd, ff = cfg.intermediate_size;
     const int bs = cfg.block_size, kvh = cfg.num_kv_heads, kvd = cfg.kv_f16 ? 0 : 1;
     const int eff_max = std::min(cfg.max_blocks_per_seq * bs, cfg.max_context_len);
-    const int64_t st = (int64_t)(intptr_t)s;
     auto lins = [&](int nt, const GgufMatMul *const *m, const int *N, int K, float *const *out, int acc) -> int {  // tensors of one type
       const void *w[3];
       for (int i = 0; i < nt; ++i) w[i] = m[i]->get_qtensor()->qi;
       const int ty = m[0]->get_qtensor()->dtype;
       return mrs_gemm_qi_multi(ty, nt, w, N, K, qact, T, out, N, acc, nullptr, 0, 0, qws, qws_bytes, s) ? fail("prefill (exact): mrs_gemm_qi_multi refused ggml dtype %d (N=%d K=%d)", ty, N[0], K) : 0;
     };
+    // the same, but the four run sums of a launch that is cut stay in the workspace from `at` bytes on for the kernel that reads them next; 1 = they do
+    auto lins_planes = [&](int nt, const GgufMatMul *const *m, const int *N, int K, float *const *out, int acc, size_t at) -> int {
+      const void *w[3];
+      for (int i = 0; i < nt; ++i) w[i] = m[i]->get_qtensor()->qi;
+      const int ty = m[0]->get_qtensor()->dtype;
+      const int rc = mrs_gemm_qi_multi_planes(ty, nt, w, N, K, qact, T, out, N, acc, (char *)qws + at, qws_bytes - at, s);
+      return rc < 0 ? fail("prefill (exact): mrs_gemm_qi_multi refused ggml dtype %d (N=%d K=%d)", ty, N[0], K) : rc;
+    };
     auto lin = [&](const GgufMatMul &m, int N, int K, float *out, int acc) -> int { const GgufMatMul *p = &m; return lins(1, &p, &N, K, &out, acc); };
     // o_proj / down_proj: h <- h + W . x;  tensor parallel: h <- h * (1 / world) + W_shard . x on every rank (the decode step's RESID epilogue, two roundings), then ONE
     // sum all-reduce of h (distributed/layers.rs:965-975) -- the same sums as the decode step whenever the all-reduce adds the ranks in the same order (world 2: always;
     // the peer-mailbox route: rank order for every message it takes)
+    // `later`: the next kernel that reads h is normed()
     const float rs = 1.0f / (float)std::max(1, (int)cfg.world_size);
-    auto row_parallel = [&](const GgufMatMul &m, int N, int K, const float *x, const float *x2, int ldx, float *xtmp) -> int {
+    const float *pending = nullptr;  // four planes of run sums that h still lacks
+    auto row_parallel = [&](const GgufMatMul &m, int N, int K, const float *x, const float *x2, int ldx, float *xtmp, bool later) -> int {
       const int ty = m.get_qtensor()->dtype;
       if (mrs_qi_quantize_for(ty, x, x2, ldx, nullptr, 0.f, T, K, qact, xtmp, s)) return fail("prefill (exact): activation quantizer refused K=%d (ggml dtype %d)", K, ty);
-      if (cfg.world_size <= 1) return lin(m, N, K, h, 1);
+      if (cfg.world_size <= 1) {
+        if (!later || N > 14336) return lin(m, N, K, h, 1);
+        const GgufMatMul *p = &m;
+        const int rc = lins_planes(1, &p, &N, K, &h, 1, 0);
+        if (rc == 1) pending = (const float *)qws;
+        return rc < 0 ? -1 : 0;
+      }
       if (lin(m, N, K, xn, 0) || mrs_resid_scale_add_f32(h, rs, xn, (size_t)T * N, s)) return -1;
       return all_reduce(h, (size_t)T * N, s) ? fail("prefill (exact): all-reduce failed: %s", g_last_error.c_str()) : 0;
     };
+    auto normed = [&](int ty, const float *nw) -> int {
+      const int rc = pending ? mrs_qi_quantize_added(ty, h, pending, nw, cfg.rms_eps, T, d, qact, s) : mrs_qi_quantize_for(ty, h, nullptr, d, nw, cfg.rms_eps, T, d, qact, nullptr, s);
+      pending = nullptr;
+      return rc ? fail("prefill (exact): activation quantizer refused K=%d (ggml dtype %d)", d, ty) : 0;
+    };
     // one activation image per vec_dot partner (gguf/mod.rs:465-478: Q8_K rows for the K-quants, Q8_0 rows for Q8_0 weights): projections that share their input share
-    // the image when their weight formats ask for the same one (every model of BASELINE.json's configs: one image per group)
-    auto group = [&](std::initializer_list<const GgufMatMul *> ms, std::initializer_list<int> Ns, std::initializer_list<float *> outs, int K, const float *x, const float *x2, int ldx,
-                     const float *nw, float *xtmp, int acc) -> int {
+    // the image when their weight formats ask for the same one
+    // src != nullptr: where a tensor's result stands afterwards (its buffer, or its columns of the run sums)
+    struct Src { const float *p; size_t plane; int ld; };
+    auto group = [&](std::initializer_list<const GgufMatMul *> ms, std::initializer_list<int> Ns, std::initializer_list<float *> outs, const float *nw, Src *src) -> int {
       std::vector<const GgufMatMul *> m(ms);
       std::vector<int> n(Ns);
       std::vector<float *> o(outs);
       std::vector<bool> done(m.size(), false);
+      size_t at = 0;
       for (size_t i = 0; i < m.size(); ++i) {
         if (done[i]) continue;
         const int ty = m[i]->get_qtensor()->dtype, mode = ty == Q8_0 ? 1 : 0;
-        if (mrs_qi_quantize_for(ty, x, x2, ldx, nw, cfg.rms_eps, T, K, qact, xtmp, s)) return fail("prefill (exact): activation quantizer refused K=%d (ggml dtype %d)", K, ty);
+        if (normed(ty, nw)) return -1;
         for (size_t j = i; j < m.size(); ++j) {
           const int tj = m[j]->get_qtensor()->dtype;
           if (done[j] || (tj == Q8_0 ? 1 : 0) != mode) continue;
-          const GgufMatMul *mm[3]; int nn[3]; float *oo[3]; int c = 0;
-          for (size_t l = j; l < m.size(); ++l)
-            if (!done[l] && m[l]->get_qtensor()->dtype == tj) { mm[c] = m[l]; nn[c] = n[l]; oo[c] = o[l]; ++c; done[l] = true; }
-          if (lins(c, mm, nn, K, oo, acc)) return -1;
+          const GgufMatMul *mm[3]; int nn[3]; float *oo[3]; size_t ix[3]; int c = 0;
+          size_t cols = 0, left = 0;  // of this launch, of those still to come
+          for (size_t l = 0; l < m.size(); ++l) {
+            if (done[l]) continue;
+            if (l >= j && m[l]->get_qtensor()->dtype == tj) { mm[c] = m[l]; nn[c] = n[l]; oo[c] = o[l]; ix[c] = l; ++c; done[l] = true; cols += (size_t)n[l]; }
+            else left += (size_t)n[l];
+          }
+          const size_t plane = (size_t)T * cols;
+          const bool keep = src && at + 16 * ((size_t)T * (cols + left)) <= qws_bytes;  // (else the next launch would find no workspace)
+          const int rc = keep ? lins_planes(c, mm, nn, d, oo, 0, at) : lins(c, mm, nn, d, oo, 0);
+          if (rc < 0) return -1;
+          size_t col = 0;
+          for (int l = 0; src && l < c; ++l) {
+            src[ix[l]] = rc == 1 ? Src{(const float *)((const char *)qws + at) + col, plane, (int)cols} : Src{oo[l], 0, nn[l]};
+            col += (size_t)nn[l];
+          }
+          if (rc == 1) at += 16 * plane;
         }
       }
       return 0;
@@ -769,20 +804,21 @@ class Llama {
     if (wte->embedding_forward_raw(pa.token_ids, T, h, s)) return -1;
     for (size_t li = 0; li < blocks.size(); ++li) {
       const Block &bl = blocks[li];
-      if (group({bl.q_proj.get(), bl.k_proj.get(), bl.v_proj.get()}, {nq, nkv, nkv}, {q, k, v}, d, h, nullptr, d, bl.input_layernorm, nullptr, 0)) return -1;
-      rotary_embedding_positions(q, k, (void *)bufs.cos_table, (void *)bufs.sin_table, (void *)pa.positions, cfg.rope_interleaved ? 0 : 1, hd, T,
-                                 cfg.rot_dim / 2, cfg.max_context_len, cfg.num_heads, cfg.num_kv_heads, nq, nkv, 2, st);
-      reshape_and_cache(k, v, bl.key_cache, bl.value_cache, (int64_t *)pa.slot_mapping, T, cfg.num_kv_heads, hd, bs, 8, nkv, nkv, s, 2, kvd == 1 ? 1 : 0, nullptr, nullptr);
+      Src src[3];
+      if (group({bl.q_proj.get(), bl.k_proj.get(), bl.v_proj.get()}, {nq, nkv, nkv}, {q, k, v}, bl.input_layernorm, src)) return -1;
+      if (mrs_prefill_rope_cache(src[0].p, src[0].plane, src[0].ld, src[1].p, src[1].plane, src[1].ld, src[2].p, src[2].plane, src[2].ld, q, bl.key_cache, bl.value_cache, pa.slot_mapping,
+                                 (const uint32_t *)pa.positions, bufs.cos_table, bufs.sin_table, T, cfg.num_heads, kvh, cfg.rot_dim / 2, cfg.rope_interleaved ? 0 : 1, kvd, s))
+        return fail("prefill (exact): RoPE / cache write refused the shape");
       if (mrs_prefill_attention_exact_ws(q, bl.key_cache, bl.value_cache, pa.block_tables, pa.context_lens, attn, T, cfg.num_heads, kvh, hd, bs, nq, kvh * hd * bs, hd * bs,
                                       1.0f / sqrtf((float)hd), eff_max, kvd, cfg.sliding_window, pa.start_pos + T, attn_ws, attn_ws_bytes, s))
         return fail("prefill (exact): attention refused the shape");
-      if (row_parallel(*bl.o_proj, d, nq, attn, nullptr, nq, nullptr)) return -1;
+      if (row_parallel(*bl.o_proj, d, nq, attn, nullptr, nq, nullptr, cfg.num_experts <= 0)) return -1;
       if (cfg.num_experts > 0) {
         if (moe_ffn_exact(bl, T, h, g, u, act, qact, mx, s)) return -1;
         continue;
       }
-      if (group({bl.gate_proj.get(), bl.up_proj.get()}, {ff, ff}, {g, u}, d, h, nullptr, d, bl.post_attention_layernorm, nullptr, 0)) return -1;
-      if (row_parallel(*bl.down_proj, d, ff, g, u, ff, act)) return -1;
+      if (group({bl.gate_proj.get(), bl.up_proj.get()}, {ff, ff}, {g, u}, bl.post_attention_layernorm, nullptr)) return -1;
+      if (row_parallel(*bl.down_proj, d, ff, g, u, ff, act, li + 1 < blocks.size())) return -1;
     }
     // ctx.logits: only the last prompt token reaches lm_head (llama.rs:514-517): the decode engine's final norm + lm_head launch
     if (mrs_dec_proj(&dlm_head, cfg.vocab_size, nullptr, h + (size_t)(T - 1) * d, d, ln_f, cfg.rms_eps, pa.logits, cfg.vocab_size, 0, 1.0f, nullptr, 1, s))

@@ -447,3 +447,101 @@ def test_gemm_qi_q8_0_odd_scales_host_emulation(oracle, T, n):
 @pytest.mark.parametrize("T,n", ODD_SCALES)
 def test_gemm_qi_q8_0_odd_scales_gpu(oracle, dev, T, n):
     run_odd_scales(oracle, GpuBackend(dev), T, n)
+
+
+def run_added_rows(O, be, tname, T, d, k):
+    """h + a cut product by its run sums and the quantizer that adds them (mrs_gemm_qi_multi_planes, mrs_qi_quantize_added) == the accumulating product and the quantizer of h."""
+    t = getattr(O, tname)
+    rng = np.random.default_rng(31)
+    p = O.quantize(t, (rng.standard_normal((d, k)) * 0.05).astype(np.float32)).reshape(d, -1)
+    nb = be.sym("mrs_gemm_qi_repack_bytes", [CI, C.c_longlong, C.c_longlong], C.c_size_t)(t, d, k)
+    src, wq = be.buf(np.ascontiguousarray(p).reshape(-1)), be.buf(np.zeros(nb, np.uint8))
+    assert be.sym("mrs_gemm_qi_repack", [VP, CI, C.c_longlong, C.c_longlong, VP, VP], CI)(src.ptr, t, d, k, wq.ptr, be.stream) == 0
+    x, h0, nw = (rng.standard_normal((T, k)).astype(np.float32), rng.standard_normal((T, d)).astype(np.float32), (1 + 0.1 * rng.standard_normal(d)).astype(np.float32))
+    h0[T - 1, : min(256, d)] = 0.0
+    quantize = be.sym("mrs_qi_quantize_for", [CI, VP, VP, CI, VP, C.c_float, CI, CI, VP, VP, VP], CI)
+    nbytes = be.sym("mrs_qi_act_bytes", [CI, CI], C.c_size_t)
+    xb, nwb, act, ws = be.buf(x), be.buf(nw), be.buf(np.zeros(nbytes(T, k), np.uint8)), be.buf(np.full(4 * T * d, np.nan, np.float32))
+    assert quantize(t, xb.ptr, None, k, None, 0.0, T, k, act.ptr, None, be.stream) == 0
+    a1, a2, h1, h2 = be.buf(np.zeros(nbytes(T, d), np.uint8)), be.buf(np.zeros(nbytes(T, d), np.uint8)), be.buf(h0.copy()), be.buf(h0.copy())
+    assert be.sym("mrs_gemm_qi", [VP, CI, CI, CI, VP, CI, VP, CI, CI, VP], CI)(wq.ptr, t, d, k, act.ptr, T, h1.ptr, d, 1, be.stream) == 0
+    assert quantize(t, h1.ptr, None, d, nwb.ptr, 1e-5, T, d, a1.ptr, None, be.stream) == 0
+    w, n, o, ld = (VP * 1)(wq.ptr), (CI * 1)(d), (VP * 1)(h2.ptr), (CI * 1)(d)
+    assert be.sym("mrs_gemm_qi_multi_planes", [CI, CI, VP, VP, CI, VP, CI, VP, VP, CI, VP, C.c_size_t, VP], CI)(t, 1, w, n, k, act.ptr, T, o, ld, 1, ws.ptr, 16 * T * d, be.stream) == 1
+    assert np.array_equal(h2.numpy(), h0)
+    assert be.sym("mrs_qi_quantize_added", [CI, VP, VP, VP, C.c_float, CI, CI, VP, VP], CI)(t, h2.ptr, ws.ptr, nwb.ptr, 1e-5, T, d, a2.ptr, be.stream) == 0
+    assert np.array_equal(h1.numpy(), h2.numpy()) and np.array_equal(a1.numpy(), a2.numpy())
+
+
+ADDED = [("Q4_K", 1, 256, 1024), ("Q8_0", 5, 2304, 1280), ("Q6_K", 37, 768, 1024)]  # rows of one superblock, of more than the 2048 values of a thread's first piece
+
+
+@pytest.mark.parametrize("tname,T,d,k", ADDED)
+def test_added_rows_host_emulation(oracle, tname, T, d, k):
+    run_added_rows(oracle, HostBackend(), tname, T, d, k)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("tname,T,d,k", ADDED + [("Q4_K", 37, 4096, 4096), ("Q4_K", 9, 14336, 4096)])
+def test_added_rows_gpu(oracle, dev, tname, T, d, k):
+    run_added_rows(oracle, GpuBackend(dev), tname, T, d, k)
+
+
+def run_rope_cache(be, T, heads, kvh, pairs, neox, kv_dtype, planes):
+    """mrs_prefill_rope_cache against the two products and their sum / difference in f32 (nothing contracted), K / V rounded to the page's type; rows whole and as four planes of run sums."""
+    rng = np.random.default_rng(41)
+    pages = 3 + (T + 5) // 32
+    tables = [rng.standard_normal((T + 9, max(pairs, 1))).astype(np.float32) for _ in range(2)]
+    pos = rng.permutation(T + 9)[:T].astype(np.uint32)
+    order = rng.permutation(pages)
+    slots = np.array([order[(i + 5) // 32] * 32 + (i + 5) % 32 for i in range(T)], np.int64)
+    slots[T // 2] = -1  # a padding token
+    raw = [rng.standard_normal((4 if planes else 1, T, n * 128)).astype(np.float32) for n in (heads, kvh, kvh)]
+    q, k, v = (((r[0] + r[1]) + r[2]) + r[3] if planes else r[0] for r in raw)
+
+    def rope(x):
+        x = x.reshape(T, -1, 128).copy()
+        a, b = (slice(0, 64), slice(64, 128)) if neox else (slice(0, 2 * pairs, 2), slice(1, 2 * pairs, 2))
+        c, s = (t[pos][:, None, :pairs] for t in tables)
+        xs, ys = x[..., a].copy(), x[..., b].copy()
+        x[..., a], x[..., b] = xs * c - ys * s, ys * c + xs * s
+        return x
+
+    def bits(x):
+        if kv_dtype == 0:
+            return x.astype(np.float16).view(np.uint16)
+        u = x.astype(np.float32).view(np.uint32).astype(np.uint64)
+        return ((u + 0x7FFF + ((u >> 16) & 1)) >> 16).astype(np.uint16)
+
+    kc, vc = np.full((pages, kvh, 16, 32, 8), 7, np.uint16), np.full((pages, kvh, 128, 32), 7, np.uint16)
+    kb, vb, qb = be.buf(kc), be.buf(vc), be.buf(np.full((T, heads * 128), np.nan, np.float32) if planes else q.copy())
+    ins = [be.buf(r) for r in raw]
+    if not planes:
+        ins[0] = qb  # in place
+    cb, sb, pb, slb = (be.buf(z) for z in (tables[0], tables[1], pos, slots))
+    fn = be.sym("mrs_prefill_rope_cache", [VP, C.c_size_t, CI] * 3 + [VP] * 7 + [CI] * 6 + [VP], CI)
+    args = [z for b, n in zip(ins, (heads, kvh, kvh)) for z in (b.ptr, T * n * 128 if planes else 0, n * 128)]
+    assert fn(*args, qb.ptr, kb.ptr, vb.ptr, slb.ptr, pb.ptr, cb.ptr, sb.ptr, T, heads, kvh, pairs, neox, kv_dtype, be.stream) == 0
+    assert np.array_equal(qb.numpy().reshape(T, heads, 128), rope(q))
+    want_k, want_v = kc.copy(), vc.copy()
+    kr, vr = bits(rope(k)), bits(v.reshape(T, kvh, 128))
+    for t, s in enumerate(slots):
+        if s >= 0:
+            want_k[s // 32, :, :, s % 32] = kr[t].reshape(kvh, 16, 8)
+            want_v[s // 32, :, :, s % 32] = vr[t]
+    assert np.array_equal(kb.numpy().reshape(kc.shape), want_k) and np.array_equal(vb.numpy().reshape(vc.shape), want_v)
+    assert fn(*args, qb.ptr, kb.ptr, vb.ptr, slb.ptr, pb.ptr, cb.ptr, sb.ptr, T, heads, kvh, 65, 0, kv_dtype, be.stream) == -1
+
+
+ROPE = [(1, 1, 1, 64, 0, 1, False), (8, 4, 2, 64, 1, 0, True), (37, 2, 1, 31, 0, 1, True), (45, 2, 2, 64, 1, 1, False), (9, 1, 1, 0, 0, 0, False)]
+
+
+@pytest.mark.parametrize("case", ROPE)
+def test_prefill_rope_cache_host_emulation(case):
+    run_rope_cache(HostBackend(), *case)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("case", ROPE + [(1999, 32, 8, 64, 0, 1, False)])
+def test_prefill_rope_cache_gpu(dev, case):
+    run_rope_cache(GpuBackend(dev), *case)
