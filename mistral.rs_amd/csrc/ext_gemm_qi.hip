@@ -318,12 +318,20 @@ template <class F> __device__ __forceinline__ void add_block(F is_dw, float y, f
 #pragma unroll
   for (int v = 0; v < 16; ++v) T[v] = first ? p[v] : T[v] + p[v];
 }
-template <int TYPE, int NT>
-__global__ void __launch_bounds__(256, NT == 2 || TYPE == T_Q5_K ? 2 : TYPE == T_Q8_0 ? 4 : 3) gemm_qi_wide_kernel(const WideArgs a) {
-  extern __shared__ __attribute__((aligned(16))) char smem[];
+// Launches that leave a CU one workgroup or none wait for the chain of a wave's superblocks (1.2 us each of one token tile, 2.0 of two, whatever the memory does), one wave to a
+// SIMD.  Workgroups of several GROUPS of four waves put more of them on a SIMD without more planes of sums:
+//   W_RUNS2 / W_RUNS4: a group takes two / one of the row's four runs; the run sums meet in LDS at the end, a share of the outputs per group;
+//   W_PAIR (a launch that is cut: one run): the first group takes its even superblocks and the sums, the second the odd ones, whose terms the first adds from LDS one step later.
+enum { W_ONE, W_PAIR, W_RUNS2, W_RUNS4 };
+constexpr int wide_groups(int mode) { return mode == W_ONE ? 1 : mode == W_RUNS4 ? 4 : 2; }
+template <int TYPE, int NT, int MODE>
+__global__ void __launch_bounds__(256 * wide_groups(MODE), MODE == W_ONE ? (NT == 2 || TYPE == T_Q5_K ? 2 : TYPE == T_Q8_0 ? 4 : 3) : MODE == W_RUNS4 ? 4 : 2) gemm_qi_wide_kernel(const WideArgs a) {
+  extern __shared__ __attribute__((aligned(16))) char smem_all[];
   constexpr int TT_ = NT * 32, ROWB = wide_row<TYPE>, ACT_ = TT_ * ROWB, BUF_ = wide_buf<TYPE, NT>, YD_ = 512;
   constexpr int NPC = TYPE == T_Q4_K ? 4 : 8;  // 1-KiB pieces of a record
-  const int tid = tid_opaque(), lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  constexpr int GROUPS = wide_groups(MODE), STEP = MODE == W_PAIR ? 2 : 1;
+  const int tid = tid_opaque(), lane = tid & 63, wave_all = __builtin_amdgcn_readfirstlane(tid >> 6), wave = wave_all & 3, grp = GROUPS > 1 ? wave_all >> 2 : 0;
+  char *const smem = smem_all + grp * 2 * BUF_;
   const int nn = lane & 31, hf = lane >> 5;
   const int order = (int)(blockIdx.y * gridDim.x + blockIdx.x), cols0 = order / (WIDE_COLS * (int)gridDim.y) * WIDE_COLS, cols = min(WIDE_COLS, (int)gridDim.x - cols0);
   const int in_cols = order - cols0 * (int)gridDim.y, by = in_cols / cols, bx = cols0 + in_cols % cols;
@@ -377,7 +385,13 @@ __global__ void __launch_bounds__(256, NT == 2 || TYPE == T_Q5_K ? 2 : TYPE == T
   for (int tt = 0; tt < NT; ++tt)
 #pragma unroll
     for (int v = 0; v < 16; ++v) { run[tt][v] = -0.f; pend[tt][v] = -0.f; }
-  const int sb_begin = a.ksplit > 1 ? (int)blockIdx.z * Cs : 0, sb_end = a.ksplit > 1 ? min(S, sb_begin + Cs) : S;
+  // the group's superblocks: sb_begin, sb_begin + STEP, .. < sb_end; `steps` of them at most in any group
+  constexpr int RUNS = 4 / GROUPS;  // W_RUNS2 / 4: of a group
+  const int z_begin = a.ksplit > 1 ? (int)blockIdx.z * Cs : 0, z_end = a.ksplit > 1 ? min(S, z_begin + Cs) : S;
+  const int sb_begin = MODE == W_ONE ? z_begin : MODE == W_PAIR ? z_begin + grp : min(S, grp * RUNS * Cs);
+  const int sb_end = MODE == W_ONE || MODE == W_PAIR ? z_end : min(S, (grp + 1) * RUNS * Cs);
+  const int steps = MODE == W_ONE ? sb_end - sb_begin : MODE == W_PAIR ? (z_end - z_begin + 1) / 2 : RUNS * Cs;
+  float *const pair_s = (float *)(smem_all + GROUPS * 2 * BUF_) + (size_t)wave * NT * 1024 + lane * 4;  // W_PAIR: [2][4 waves][4 NT][64 lanes][4] terms on their way
   // outputs through bounded buffers that begin at the tile's first row: a lane holds column n, rows 32 tt + 8 (v / 4) + 4 hf + v % 4; a buffer ends behind the window's
   // last row, columns past N are pushed out of it
   const bool split = a.ksplit > 1;
@@ -388,34 +402,48 @@ __global__ void __launch_bounds__(256, NT == 2 || TYPE == T_Q5_K ? 2 : TYPE == T
   auto at = [&](int tt, int v) -> unsigned { return vo + (unsigned)((tt * 32 + 8 * (v >> 2) + (v & 3)) * ldo); };
   auto ld32 = [&](__amdgpu_buffer_rsrc_t r, unsigned off) { return __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(r, off, 0, 0)); };
   auto st32 = [&](float v, __amdgpu_buffer_rsrc_t r, unsigned off) { __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(v), r, off, 0, 0); };
-  if (sb_begin >= sb_end) {  // a run without superblocks contributes +0 (only with ksplit: S >= 1)
+  if (z_begin >= z_end) {  // a run without superblocks contributes +0 (only with ksplit: S >= 1)
+    if (grp == 0) {
 #pragma unroll
-    for (int tt = 0; tt < NT; ++tt)
+      for (int tt = 0; tt < NT; ++tt)
 #pragma unroll
-      for (int v = 0; v < 16; ++v) st32(0.f, ro, at(tt, v));
+        for (int v = 0; v < 16; ++v) st32(0.f, ro, at(tt, v));
+    }
     return;
   }
+  const bool any = GROUPS == 1 || sb_begin < sb_end;
 #pragma unroll
-  for (int i = 0; i < NSTAGE; ++i) stage_q(sb_begin, 0, i);
-  stage_meta(sb_begin, 0);
+  for (int i = 0; i < NSTAGE; ++i) stage_q(sb_begin, 0, i, any);
+  stage_meta(sb_begin, 0, any);
+  const unsigned rec_first = any ? rec_of(sb_begin) : DEAD;
   // Q8_0: four pieces and the scales' dwords in place, each requested again when its last block has been multiplied -- half a superblock ahead; all eight would leave three
   // workgroups on a CU instead of four
   constexpr int NWQ = TYPE == T_Q8_0 ? 4 : NPC;
   v4u wq[NWQ], hs_next;
   unsigned hd_next;
 #pragma unroll
-  for (int c = 0; c < NWQ; ++c) wq[c] = load_q(rec_of(sb_begin), c);
-  hs_next = load_hs(rec_of(sb_begin));
+  for (int c = 0; c < NWQ; ++c) wq[c] = load_q(rec_first, c);
+  hs_next = load_hs(rec_first);
   unsigned hw8[4] = {hs_next.x, hs_next.y, hs_next.z, hs_next.w};  // Q8_0
-  if (TYPE != T_Q8_0) hd_next = load_hd(rec_of(sb_begin));
+  if (TYPE != T_Q8_0) hd_next = load_hd(rec_first);
   const f16v zero = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
   unsigned mg = TYPE == T_Q6_K ? 0x64006400u : 0x54005400u;
   MRS_OPAQUE_TID(mg);  // keeps the constant in a VGPR: v_and_or_b32 takes one literal
-  for (int sb = sb_begin; sb < sb_end; ++sb) {
-    const int it = sb - sb_begin;
-    const bool more = sb + 1 < sb_end;
+  auto add_pair = [&](int i) {  // W_PAIR: the second group's terms of its step i
+#pragma unroll
+    for (int tt = 0; tt < NT; ++tt)
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const float4 t = *(const float4 *)(pair_s + (i & 1) * 4 * NT * 1024 + (tt * 4 + q) * 256);
+        run[tt][4 * q] = run[tt][4 * q] + t.x; run[tt][4 * q + 1] = run[tt][4 * q + 1] + t.y; run[tt][4 * q + 2] = run[tt][4 * q + 2] + t.z; run[tt][4 * q + 3] = run[tt][4 * q + 3] + t.w;
+      }
+  };
+  for (int it = 0; it < steps; ++it) {
+    const int sb = sb_begin + it * STEP;
+    if (GROUPS > 1 && sb >= sb_end) { __syncthreads(); continue; }  // the other groups' barrier
+    const bool more = sb + STEP < sb_end;
     const v4u hs = hs_next;  // (Q8_0: not used)
-    const unsigned hd = hd_next, rec = rec_of(sb), rec_next = more ? rec_of(sb + 1) : DEAD;
+    const unsigned hd = hd_next, rec = rec_of(sb), rec_next = more ? rec_of(sb + STEP) : DEAD;
     const char *meta_s = smem + (it & 1) * BUF_ + ACT_;
     unsigned abase = MRS_LDS_BASE(smem) + (unsigned)((it & 1) * BUF_ + nn * ROWB + (((nn % CPR) ^ hf) << 4));
     MRS_OPAQUE_TID(abase);  // one register: a fragment's offset is one exclusive or on it
@@ -428,7 +456,8 @@ __global__ void __launch_bounds__(256, NT == 2 || TYPE == T_Q5_K ? 2 : TYPE == T
       // 311, 831); two token tiles 263, 720.
       MRS_WAIT_VMCNT0();
       __syncthreads();
-      stage_meta(sb + 1, it + 1, more);
+      if (MODE == W_PAIR && grp == 0 && it > 0) add_pair(it - 1);
+      stage_meta(sb + STEP, it + 1, more);
       auto frag8 = [&](int b, int tt) -> i4v { return MRS_LDS_FRAG(i4v, smem, abase ^ (unsigned)(32 * b), tt * (32 * ROWB)); };
       constexpr int MAGIC = 0x4B400000;  // 1.5 x 2^23
       const i16v imagic = {MAGIC, MAGIC, MAGIC, MAGIC, MAGIC, MAGIC, MAGIC, MAGIC, MAGIC, MAGIC, MAGIC, MAGIC, MAGIC, MAGIC, MAGIC, MAGIC};
@@ -450,7 +479,7 @@ __global__ void __launch_bounds__(256, NT == 2 || TYPE == T_Q5_K ? 2 : TYPE == T
 #pragma unroll
         for (int tt = 0; tt < NT; ++tt) is[tt] = __builtin_amdgcn_mfma_i32_32x32x32_i8(af[b & 1][tt], __builtin_bit_cast(i4v, wq[b & 3]), imagic, 0, 0, 0);
         wq[b & 3] = b < 4 ? load_q(rec, b + 4) : load_q(rec_next, b - 4);
-        if (b < NSTAGE) stage_q(sb + 1, it + 1, b, more);
+        if (b < NSTAGE) stage_q(sb + STEP, it + 1, b, more);
         const unsigned hw = hw8[b / 2];
         if (b % 2 == 0) odd |= odd16(hw);
         float dwb = half_bits_to_float((uint16_t)((b & 1) ? (hw >> 16) : (hw & 0xffffu)));
@@ -532,7 +561,8 @@ __global__ void __launch_bounds__(256, NT == 2 || TYPE == T_Q5_K ? 2 : TYPE == T
     __builtin_amdgcn_sched_barrier(0);
     MRS_WAIT_VMCNT0();  // this wave's DMA pieces of superblock sb have landed
     __syncthreads();    // everyone's have, and every wave has finished reading the other buffer
-    stage_meta(sb + 1, it + 1, more);
+    if (MODE == W_PAIR && grp == 0 && it > 0) add_pair(it - 1);
+    stage_meta(sb + STEP, it + 1, more);
     hs_next = load_hs(rec_next); hd_next = load_hd(rec_next);
     auto frag = [&](int r, int tt) -> h8 { return MRS_LDS_FRAG(h8, smem, abase ^ (unsigned)(32 * r), tt * (32 * ROWB)); };
     constexpr int NX = TYPE == T_Q4_K ? 1 : 2;  // accumulators: Q5_K: runs 0 .. 7 | 8 .. 15 (|.| <= 16.5 M each);  Q6_K: the sl | sh operands
@@ -561,7 +591,7 @@ __global__ void __launch_bounds__(256, NT == 2 || TYPE == T_Q5_K ? 2 : TYPE == T
 #pragma unroll
           for (int p = tt * 4 / NT; p < (tt + 1) * 4 / NT; ++p) pair_of(k + 1, p, w[(k + 1) & 1][p], w2[(k + 1) & 1][p % NW2]);
         }
-        if (tt == 0 && (k + 1) % (16 / NSTAGE) == 0) stage_q(sb + 1, it + 1, (k + 1) / (16 / NSTAGE) - 1, more);
+        if (tt == 0 && (k + 1) % (16 / NSTAGE) == 0) stage_q(sb + STEP, it + 1, (k + 1) / (16 / NSTAGE) - 1, more);
         if (tt == NT - 1 && (TYPE == T_Q4_K ? (k & 3) == 2 : (k & 1) == 0)) wq[TYPE == T_Q4_K ? k >> 2 : k >> 1] = load_q(rec_next, TYPE == T_Q4_K ? k >> 2 : k >> 1);  // step k + 1, the piece's last, has been built
         __builtin_amdgcn_sched_barrier(0);
       }
@@ -609,16 +639,75 @@ __global__ void __launch_bounds__(256, NT == 2 || TYPE == T_Q5_K ? 2 : TYPE == T
       }
     }
     }
-    if ((sb + 1) % Cs == 0 || sb + 1 == sb_end) {  // a run of superblocks ends: its sum joins the row's left-to-right combination
+    if constexpr (MODE == W_PAIR) {
+      if (grp == 1) {  // run is this superblock's term
+#pragma unroll
+        for (int tt = 0; tt < NT; ++tt)
+#pragma unroll
+          for (int q = 0; q < 4; ++q) {
+            *(float4 *)(pair_s + (it & 1) * 4 * NT * 1024 + (tt * 4 + q) * 256) = make_float4(run[tt][4 * q], run[tt][4 * q + 1], run[tt][4 * q + 2], run[tt][4 * q + 3]);
+            run[tt][4 * q] = run[tt][4 * q + 1] = run[tt][4 * q + 2] = run[tt][4 * q + 3] = -0.f;
+          }
+      }
+    } else if (MODE != W_RUNS4 && ((sb + 1) % Cs == 0 || sb + 1 == sb_end)) {  // a run of superblocks ends: its sum joins the row's left-to-right combination
+      if (MODE == W_ONE || grp == 0 || it < Cs) {  // (W_RUNS2's second group keeps c2 in pend and c3 in run)
+#pragma unroll
+        for (int tt = 0; tt < NT; ++tt)
+#pragma unroll
+          for (int v = 0; v < 16; ++v) { pend[tt][v] = pend[tt][v] + run[tt][v]; run[tt][v] = -0.f; }
+      }
+    }
+  }
+  if constexpr (MODE == W_PAIR) {
+    __syncthreads();
+    if (grp == 1) return;
+    if (z_begin + 2 * steps <= z_end) add_pair(steps - 1);
+  }
+  if constexpr (MODE == W_RUNS2 || MODE == W_RUNS4) {
+    constexpr int PL = MODE == W_RUNS4 ? 4 : 3, VG = 16 / GROUPS;  // planes: c0 .. c3 | c0 + c1, c2, c3;  outputs of a group, of every token tile
+    MRS_WAIT_VMCNT0();  // the last requests to LDS (out of range: zeros) have landed
+    __syncthreads();
+    float *const sums = (float *)smem_all + (size_t)wave * PL * NT * 1024 + lane * 4;  // [4 waves][planes][4 NT][64 lanes][4]
+    auto put = [&](int plane, const float (&c)[NT][16]) {
 #pragma unroll
       for (int tt = 0; tt < NT; ++tt)
 #pragma unroll
-        for (int v = 0; v < 16; ++v) { pend[tt][v] = pend[tt][v] + run[tt][v]; run[tt][v] = -0.f; }
+        for (int q = 0; q < 4; ++q) *(float4 *)(sums + ((plane * NT + tt) * 4 + q) * 256) = make_float4(c[tt][4 * q], c[tt][4 * q + 1], c[tt][4 * q + 2], c[tt][4 * q + 3]);
+    };
+    if (MODE == W_RUNS4) put(grp, run);
+    else if (grp == 0) put(0, pend);
+    else { put(1, pend); put(2, run); }
+    __syncthreads();
+    float old[NT][VG];
+    if (a.accumulate) {
+#pragma unroll
+      for (int tt = 0; tt < NT; ++tt)
+#pragma unroll
+        for (int i = 0; i < VG; ++i) old[tt][i] = ld32(ro, vo + (unsigned)((tt * 32 + 8 * ((grp * VG + i) >> 2) + (i & 3)) * ldo));
     }
+#pragma unroll
+    for (int tt = 0; tt < NT; ++tt)
+#pragma unroll
+      for (int q = 0; q < VG / 4; ++q) {
+        auto get = [&](int plane) { return *(const float4 *)(sums + ((plane * NT + tt) * 4 + grp * (VG / 4) + q) * 256); };
+        const float4 c0 = get(0), c1 = get(1), c2 = get(2), c3 = MODE == W_RUNS4 ? get(PL - 1) : make_float4(0.f, 0.f, 0.f, 0.f);
+        float r[4] = {(c0.x + c1.x) + c2.x, (c0.y + c1.y) + c2.y, (c0.z + c1.z) + c2.z, (c0.w + c1.w) + c2.w};
+        if (MODE == W_RUNS4) { r[0] = r[0] + c3.x; r[1] = r[1] + c3.y; r[2] = r[2] + c3.z; r[3] = r[3] + c3.w; }
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          st32(a.accumulate ? old[tt][4 * q + i] + r[i] : r[i], ro, vo + (unsigned)((tt * 32 + 8 * (grp * (VG / 4) + q) + i) * ldo));
+      }
+    return;
   }
   // (split: one run per workgroup, combined by gemm_qi_reduce_kernel)
   // all the old values are requested before the first is needed: a request and its wait per value were 32 memory latencies one after another (us, Q4_K 4096 x 4096 accumulating,
   // one by one / together: 512 tokens 41.7 / 33.3, 2000 tokens 106.7 / 91.9)
+  if constexpr (MODE == W_PAIR) {
+#pragma unroll
+    for (int tt = 0; tt < NT; ++tt)
+#pragma unroll
+      for (int v = 0; v < 16; ++v) pend[tt][v] = run[tt][v];
+  }
   if (a.accumulate && !split) {
     float old[NT][16];
 #pragma unroll
@@ -826,13 +915,21 @@ extern "C" int mrs_gemm_qi_ws(const void *w_qi, int type, int N, int K, const vo
                               void *stream) {
   return mrs_gemm_qi_multi(type, 1, &w_qi, &N, K, act, T, &out, &ldo, accumulate, nullptr, 0, 0, workspace, workspace_bytes, stream);
 }
-template <int TYPE>
-static void wide_launch(int NT, const qi::WideArgs &a, dim3 grid, hipStream_t s) {
-  auto k1 = qi::gemm_qi_wide_kernel<TYPE, 1>;
-  auto k2 = qi::gemm_qi_wide_kernel<TYPE, 2>;
-  lds_attr_once((const void *)(NT == 2 ? k2 : k1), 158 * 1024);
-  if (NT == 2) hipLaunchKernelGGL(k2, grid, dim3(256), (2 * qi::wide_buf<TYPE, 2>), s, a);
-  else hipLaunchKernelGGL(k1, grid, dim3(256), (2 * qi::wide_buf<TYPE, 1>), s, a);
+template <int TYPE, int NT, int MODE> static void wide_go(const qi::WideArgs &a, dim3 grid, hipStream_t s) {
+  constexpr int bufs = qi::wide_groups(MODE) * 2 * qi::wide_buf<TYPE, NT>, sums = MODE == qi::W_RUNS2 ? 3 * 4 * NT * 4096 : MODE == qi::W_RUNS4 ? 4 * 4 * NT * 4096 : 0;
+  constexpr int lds = std::max(bufs, sums) + (MODE == qi::W_PAIR ? 2 * 4 * NT * 4096 : 0);
+  static_assert(lds <= 158 * 1024, "LDS of a workgroup");
+  auto kern = qi::gemm_qi_wide_kernel<TYPE, NT, MODE>;
+  lds_attr_once((const void *)kern, 158 * 1024);
+  hipLaunchKernelGGL(kern, grid, dim3(256 * qi::wide_groups(MODE)), lds, s, a);
+}
+template <int TYPE> static void wide_launch(int NT, int mode, const qi::WideArgs &a, dim3 grid, hipStream_t s) {
+  if (mode == qi::W_PAIR) return wide_go<TYPE, 1, qi::W_PAIR>(a, grid, s);
+  if constexpr (TYPE != T_Q5_K) {
+    if (mode == qi::W_RUNS2) return wide_go<TYPE, 2, qi::W_RUNS2>(a, grid, s);
+    if (mode == qi::W_RUNS4) return wide_go<TYPE, 1, qi::W_RUNS4>(a, grid, s);
+  }
+  NT == 2 ? wide_go<TYPE, 2, qi::W_ONE>(a, grid, s) : wide_go<TYPE, 1, qi::W_ONE>(a, grid, s);
 }
 // Token tiles per wave, by the rows of a launch (of an expert, where there are several) and its workgroup columns (of all experts).  K-quants: 32 rows fill one; two build each operand
 // once for both, but make the chain of a superblock longer, which is what a launch that leaves most of the chip idle waits for.  So two from 33 rows on where they make more than 32
@@ -852,6 +949,18 @@ static int wide_tiles(int type, int rows, int cols) { return rows <= 32 || cols 
 // Q6_K 430 / 392, Q8_0 349 / 310.
 static int cut_line(int type, int K) { return type == T_Q8_0 ? K / 12 : K / 20; }  // two tiles
 static int cut_max(int type, int NT, int K) { return NT == 2 ? (K >= 8192 ? 895 : cut_line(type, K)) : type == T_Q8_0 ? std::min(K / 8, 895) : std::min(K / 18, 400); }
+// Whole launches of up to a workgroup per CU, but not so few that cutting them is better: workgroups of several groups of waves, each with its own runs (W_RUNS4 of one token tile,
+// W_RUNS2 of two).  us, cut / one group / so: Q4_K one tile 6144 x 4096 37 rows (96) 14.1 / 19.9 / 16.1, 4096 x 4096 128 rows (128) 16.9 / 20.1 / 16.3, 28672 x 4096 32 rows (224) 27.0 /
+// 25.0 / 20.7, two tiles 64 rows (224) 37.4 / 29.8 / 28.2;  Q6_K one tile 4096 x 4096 128 rows 19.1 / 25.7 / 21.6, 28672 x 4096 32 rows 36.4 / 32.2 / 31.6;  Q8_0 4096 x 4096 128 rows
+// 18.5 / 30.6 / 17.8, 28672 x 4096 32 rows 34.2 / 35.7 / 26.5, two tiles 64 rows 43.3 / 41.5 / 33.9.  Long rows have chains that only more workgroups shorten (Q4_K 4096 x 14336 128 rows
+// (128) 34.9 / 71.5 / 49.0).  Q5_K's kernel spills at 16 waves and is slower in both forms (30.2 -> 37.5, 36.2 -> 39.1).
+static bool wide_runs(int type, int wgs, int K, int NT) {
+  return type != T_Q5_K && K / 256 >= 4 && wgs <= 256 && wgs >= K / (NT == 2 ? 24 : type == T_Q4_K ? 36 : type == T_Q8_0 ? 32 : 22);
+}
+// Cut launches of one token tile: two groups take a run's superblocks in turn where the grid leaves a CU room for both (workgroups of all runs; Q8_0's fit twice).  us, one group /
+// two: K = 14336, 4096 rows of weights, 37 tokens (256) Q4_K 25.0 / 22.8, Q6_K 30.8 / 28.8, Q5_K 28.0 / 26.5, Q8_0 34.2 / 25.5, 128 tokens (512) Q4_K 34.9 / 40.1, Q8_0 41.8 / 36.4;
+// 4096 x 4096 37 tokens Q4_K 11.0 / 10.9, Q8_0 13.8 / 11.7; 6144 x 4096 128 tokens (768) Q8_0 22.4 / 23.1.
+static bool wide_pair(int type, int wgs, int NT) { return NT == 1 && wgs <= (type == T_Q8_0 ? 512 : 256); }
 static bool wide_cut(int type, int wgs, int K, int NT) {
   if (K / 256 < 4 || wgs > cut_max(type, NT, K)) return false;
   return NT == 1 || wgs <= std::min(cut_line(type, K), 511) || wgs > 512;
@@ -863,7 +972,7 @@ extern "C" size_t mrs_gemm_qi_cut_bytes(int T, int n, int K) {
   const int tiles = std::max(std::max(cut_max(T_Q8_0, 1, K), cut_max(T_Q4_K, 1, K)), 2 * std::max(cut_max(T_Q8_0, 2, K), cut_max(T_Q4_K, 2, K)));
   return (size_t)16 * std::min((size_t)T * n, (size_t)tiles * 32 * qi::WIDE_ROWS);
 }
-// 1: mrs_gemm_qi_multi over T rows, given a workspace, is cut
+// 1: mrs_gemm_qi_multi over T rows, given a workspace, is cut (unless its workgroups split the runs among their own waves: wide_runs)
 extern "C" int mrs_gemm_qi_is_cut(int type, int nt, const int *N, int K, int T) {
   if (!N || nt < 1 || nt > 3 || !qi::qi_type(type) || T <= 0 || K <= 0 || K % 256) return 0;
   int gx = 0;
@@ -897,12 +1006,14 @@ static int gemm_qi_launch(int type, int nt, const void *const *w_qi, const int *
   a.K = K; a.T = T; a.qf = qf; a.yd = yd; a.bsf = bsf; a.accumulate = accumulate; a.part = (float *)workspace; a.part_n = n_all; a.bounds = bounds; a.experts = experts; a.ksplit = 1;
   // windows: every expert's last tile may be partly filled, and none has more tiles than max_rows fill
   dim3 grid(gx, bounds ? std::min(T / tl + experts, experts * ((max_rows + tl - 1) / tl)) : (T + tl - 1) / tl);
-  if (!bounds && workspace && workspace_bytes >= (size_t)4 * T * n_all * 4 && mrs_gemm_qi_is_cut(type, nt, N, K, T)) { a.ksplit = 4; grid.z = 4; }
+  if (!bounds && workspace && workspace_bytes >= (size_t)4 * T * n_all * 4 && mrs_gemm_qi_is_cut(type, nt, N, K, T) && !wide_runs(type, (int)(grid.x * grid.y), K, NT)) { a.ksplit = 4; grid.z = 4; }
+  const int wgs = (int)std::min<size_t>((size_t)grid.x * grid.y * grid.z, 1 << 20);
+  const int mode = a.ksplit > 1 ? (wide_pair(type, wgs, NT) ? qi::W_PAIR : qi::W_ONE) : !bounds && wide_runs(type, wgs, K, NT) ? (NT == 2 ? qi::W_RUNS2 : qi::W_RUNS4) : qi::W_ONE;
   switch (type) {
-    case T_Q4_K: wide_launch<T_Q4_K>(NT, a, grid, s); break;
-    case T_Q5_K: wide_launch<T_Q5_K>(NT, a, grid, s); break;
-    case T_Q6_K: wide_launch<T_Q6_K>(NT, a, grid, s); break;
-    default: wide_launch<T_Q8_0>(NT, a, grid, s); break;
+    case T_Q4_K: wide_launch<T_Q4_K>(NT, mode, a, grid, s); break;
+    case T_Q5_K: wide_launch<T_Q5_K>(NT, mode, a, grid, s); break;
+    case T_Q6_K: wide_launch<T_Q6_K>(NT, mode, a, grid, s); break;
+    default: wide_launch<T_Q8_0>(NT, mode, a, grid, s); break;
   }
   if (a.ksplit > 1 && keep_planes) return 1;
   if (a.ksplit > 1) hipLaunchKernelGGL(qi::gemm_qi_reduce_kernel, dim3(T, (n_all + 1023) / 1024), dim3(256), 0, s, a);

@@ -248,6 +248,23 @@ def test_gemm_qi_more_columns_than_a_group_gpu(oracle, dev, case):
     run_multi(oracle, GpuBackend(dev), *case, seed=8)
 
 
+# whole launches whose workgroups split the row's runs over groups of waves (from K / 36, K / 32, K / 22, two token tiles K / 24 workgroups on): runs of one superblock, unequal and
+# empty ones (5 superblocks: 2, 2, 1, 0), two segments, a partly filled last column, one row and full tiles
+RUNS = [("Q4_K", (3500, 100), 1024, 9, None, False, True), ("Q8_0", (5180,), 1280, 3, None, True, False), ("Q6_K", (5900,), 1024, 1, None, True, True), ("Q4_K", (5400,), 1024, 34, None, True, True)]
+
+
+@pytest.mark.parametrize("case", RUNS)
+def test_gemm_qi_runs_in_a_workgroup_host_emulation(oracle, case):
+    run_multi(oracle, HostBackend(), *case, seed=9)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("case", RUNS + [("Q8_0", (6850,), 1280, 33, None, False, True), ("Q8_0", (14336, 14336), 4096, 64, None, True, False), ("Q6_K", (5400,), 1024, 64, None, True, False),
+                                         ("Q6_K", (8200,), 1280, 64, None, False, True), ("Q4_K", (28672,), 4096, 32, None, True, False), ("Q4_K", (11000,), 2304, 64, None, False, True)])
+def test_gemm_qi_runs_in_a_workgroup_gpu(oracle, dev, case):
+    run_multi(oracle, GpuBackend(dev), *case, seed=9)
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("tname,T", [("Q8_0", 2050), ("Q6_K", 4130), ("Q4_K", 4130)])
 def test_long_rows_cut_by_runs_equal_the_whole_launch(oracle, dev, tname, T):
