@@ -249,6 +249,309 @@ __global__ void __launch_bounds__(64 * G) dec_attn2_kernel(const Attn2Args a) {
     attn2_merge<G, true, ONE ? 8 : 12>(a, kvh, seq, ns, wave, lane, gridDim.y);
   }
 }
+// ------------------------------------------------------------------------------------------------ groups of four and eight heads: the same chains on the matrix cores
+// dec_attn2_kernel gives every query head a wave: four of them convert the same keys and values and run four serial chains.  v_mfma_f32_4x4x1_16b_f32 is sixteen outer products
+// of 4 x 4, one f32 fma per output, so ONE wave runs the chains of four heads, term by term in the order of attn_block_update (dec_attn.cuh):
+//   scores  block i < 8: tokens 4 i .. 4 i + 3, dims 0 .. 63 one after another, block 8 + i: the same tokens, dims 64 .. 127;  A = the key lane l holds (token l % 32, half l / 32),
+//           B = the query of head l % 4;  lane l receives tokens 4 (l / 4 % 8) + v of head l % 4; the two halves are added across lanes l, l ^ 32
+//   P . V   block i: dims 4 i .. 4 i + 3 (and 64 more), tokens one after another;  A = the value of dim l, B = the probability of head l % 4
+//   and the maximum, the exponentials (two tokens per lane half) and the sum tree run for four heads at once.
+// What bounds both kernels is latency: page index, keys and values (2.5 us from HBM behind the step's weights), the hand-off, the merge.  So everything is requested at once -- values
+// by LDS-DMA, 1 KiB of consecutive bytes per instruction (a lane's own 64-byte row of them would be 64 lines per instruction) -- and the last arriver requests all its partials.
+// us per launch in a captured step, caches evicted, 32 heads of 8 key heads, a wave per head / this: one sequence of 513 9.96 / 9.0, of 7002 21.8 / 20.0, two of 1501 and 751
+// 18.4 / 12.1, five of 151 .. 301 10.65 / 8.9, eight of 501 .. 1001 20.4 / 14.3.  The last is 25 MB of keys and values, 10 of its 14 us.
+typedef float f4v __attribute__((ext_vector_type(4)));
+constexpr int A4_P = 36, A4_Q = 68, A4_V = 8192;  // LDS: rows of a head's 32 probabilities and of 64 of its query values (a wave's heads begin in different banks); a block's values
+#ifndef MRS_BLDS16
+#define MRS_BLDS16(rsrc, lbase, voff) __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, (__attribute__((address_space(3))) void *)(lbase), 16, voff, 0, 0, 0)
+#endif
+// V of a block -> LDS: the 16-byte chunk c (tokens 8 c ..) of dim d at position 4 d + (c ^ (d / 4 % 4)): the reads of 16 neighbouring dims hit every bank
+__device__ __forceinline__ void attn4_stage_v(const AttnArgs &t, size_t base, char *lds, int lane) {
+  const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc((void *)(t.v_cache + base), (short)0, KV_BLOCK_BYTES, 0x00020000);
+#pragma unroll
+  for (int i = 0; i < 8; ++i) MRS_BLDS16(r, lds + i * 1024, (unsigned)(i * 1024 + (lane & ~3) * 16 + (((lane & 3) ^ ((lane >> 4) & 3)) << 4)));
+}
+__device__ __forceinline__ int4 attn4_read_v(const char *lds, int dim, int c) { return *(const int4 *)(lds + dim * 64 + ((c ^ ((dim >> 2) & 3)) << 4)); }
+// queries of four heads -> LDS: rows (head, half)
+__device__ __forceinline__ void attn4_stage_q(const AttnArgs &t, int seq, int head0, float *q_s, int lane) {
+  const float *qg = t.q + (size_t)seq * t.q_stride + (size_t)head0 * 128;
+  float4 v[2];
+#pragma unroll
+  for (int i = 0; i < 2; ++i) v[i] = *(const float4 *)(qg + i * 256 + lane * 4);
+#pragma unroll
+  for (int i = 0; i < 2; ++i) *(float4 *)(q_s + (i * 4 + (lane >> 4)) * A4_Q + (lane & 15) * 4) = v[i];
+}
+// scores of a block for four heads: the lane's two tokens 4 (lane / 4 % 8) + 2 (lane / 32) + {0, 1} of head lane % 4, scaled, -FLT_MAX where masked; returns the head's block maximum
+template <class CT>
+__device__ __forceinline__ float attn4_scores(const AttnArgs &t, const int4 (&kr)[8], const float *q_s, int b, int ctx, int lo, int lane, float (&val)[2], bool (&ok)[2]) {
+  const int half = lane >> 5, hd = lane & 3;
+  const float *qw = q_s + (hd * 2 + half) * A4_Q;
+  f4v s = {0.f, 0.f, 0.f, 0.f};
+  float4 qv[2][2];  // of eight dims, the next eight's
+  auto read_q = [&](int c) {
+#pragma unroll
+    for (int j = 0; j < 2; ++j) qv[c & 1][j] = *(const float4 *)(qw + 8 * c + 4 * j);
+  };
+  read_q(0);
+#pragma unroll
+  for (int c = 0; c < 8; ++c) {
+    float kf[8];
+    unpack16<CT>(kr[c], kf);
+    if (c + 1 < 8) read_q(c + 1);
+    const float4 q0 = qv[c & 1][0], q1 = qv[c & 1][1];
+    const float qs[8] = {q0.x, q0.y, q0.z, q0.w, q1.x, q1.y, q1.z, q1.w};
+#pragma unroll
+    for (int j = 0; j < 8; ++j) s = __builtin_amdgcn_mfma_f32_4x4x1f32(kf[j], qs[j], s, 0, 0, 0);
+  }
+  const int pos0 = b * 32 + 4 * ((lane >> 2) & 7) + 2 * half;
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const float keep = half ? s[2 + i] : s[i], give = half ? s[i] : s[2 + i];
+    const float sv = keep + __shfl_xor(give, 32, 64);
+    ok[i] = pos0 + i < ctx && pos0 + i >= lo;
+    val[i] = ok[i] ? sv * t.scale : -FLT_MAX;
+  }
+  float mx = fmaxf(val[0], val[1]);
+  mx = fmaxf(mx, dpp_f<0x124>(mx)); mx = fmaxf(mx, dpp_f<0x128>(mx));  // the head's lanes in the row of 16
+  mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
+  return fmaxf(mx, __shfl_xor(mx, 32, 64));
+}
+// probabilities against the running maximum mn -> LDS row of the head; returns their sum (the pairwise tree in token order)
+__device__ __forceinline__ float attn4_probs(const float (&val)[2], const bool (&ok)[2], float mn, float *p_s, int lane) {
+  float p[2];
+#pragma unroll
+  for (int i = 0; i < 2; ++i) { const float e = fast_exp_ref(val[i] - mn); p[i] = ok[i] ? e : 0.f; }
+  *(float2 *)(p_s + (lane & 3) * A4_P + 4 * ((lane >> 2) & 7) + 2 * (lane >> 5)) = make_float2(p[0], p[1]);
+  float ps = p[0] + p[1];
+  ps = ps + __shfl_xor(ps, 32, 64);
+  ps = ps + dpp_f<0x141>(dpp_f<0x1B>(ps));  // lane ^ 4
+  ps = ps + dpp_f<0x128>(ps);               // lane ^ 8
+  return ps + __shfl_xor(ps, 16, 64);
+}
+// o += P V over the block's tokens, dims dim0 + 4 (lane / 4) + v of head lane % 4
+template <class CT, int ND>
+__device__ __forceinline__ void attn4_values(const char *v_s, const float *p_s, int b, int ctx, int dim0, int lane, f4v (&o)[ND]) {
+  const bool tail = (b + 1) * 32 > ctx;  // slots past the context may hold NaNs
+#pragma unroll
+  for (int c = 0; c < 4; ++c) {
+    const float4 p0 = *(const float4 *)(p_s + (lane & 3) * A4_P + 8 * c), p1 = *(const float4 *)(p_s + (lane & 3) * A4_P + 8 * c + 4);
+    float vf[ND][8];
+#pragma unroll
+    for (int n = 0; n < ND; ++n) {
+      int4 raw = attn4_read_v(v_s, dim0 + 64 * n + lane, c);
+      if (tail) {
+        int *d = (int *)&raw;
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+          const int left = ctx - (b * 32 + c * 8 + 2 * u);  // a dword holds two tokens
+          d[u] = left > 1 ? d[u] : left == 1 ? d[u] & 0xffff : 0;
+        }
+      }
+      unpack16<CT>(raw, vf[n]);
+    }
+    const float pb[8] = {p0.x, p0.y, p0.z, p0.w, p1.x, p1.y, p1.z, p1.w};
+#pragma unroll
+    for (int j = 0; j < 8; ++j)
+#pragma unroll
+      for (int n = 0; n < ND; ++n) o[n] = __builtin_amdgcn_mfma_f32_4x4x1f32(vf[n][j], pb[j], o[n], 0, 0, 0);
+  }
+}
+// dims dim0 + 4 (lane / 4) + v of head head0 + lane % 4 of a split's partial
+template <bool AGENT>
+__device__ __forceinline__ void attn4_publish_o(const AttnArgs &t, int seq, int head0, int split, int dim0, int lane, f4v o) {
+  const __amdgpu_buffer_rsrc_t r =
+      __builtin_amdgcn_make_buffer_rsrc((void *)(t.part_o + ((size_t)seq * t.num_heads + head0) * t.max_splits * 128), (short)0, 4 * t.max_splits * 512, 0x00020000);
+  const v4u w = {__float_as_uint(o[0]), __float_as_uint(o[1]), __float_as_uint(o[2]), __float_as_uint(o[3])};
+  constexpr int AUX = AGENT ? 16 : 0;  // write-through at agent scope
+  __builtin_amdgcn_raw_buffer_store_b128(w, r, (unsigned)((lane & 3) * t.max_splits + split) * 512u + (unsigned)(dim0 * 4 + (lane >> 2) * 16), 0, AUX);
+}
+template <bool AGENT>
+__device__ __forceinline__ void attn4_publish_ml(const AttnArgs &t, int seq, int head, int split, float m, float l) {
+  const size_t pi = ((size_t)seq * t.num_heads + head) * t.max_splits + split;
+  if constexpr (AGENT) {
+    __hip_atomic_store(t.part_m + pi, m, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __hip_atomic_store(t.part_l + pi, l, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  } else { t.part_m[pi] = m; t.part_l[pi] = l; }
+}
+// the last arriver: ns (<= 64) partials of heads head0 + wave (+ 4), all requested before the first is added; lane = dims 2 lane, 2 lane + 1; attn_merge_core's order
+template <int G>
+__device__ __forceinline__ void attn4_merge(const Attn2Args &a, int kvh, int seq, int ns, int wave, int lane, int ncols, float (*o_s)[128]) {
+  constexpr int HD = 128, MB = 16;
+  const AttnArgs &t = a.t;
+#pragma unroll
+  for (int i = 0; i < G / 4; ++i) {
+    const size_t p0 = ((size_t)seq * t.num_heads + kvh * G + wave + 4 * i) * t.max_splits;
+    auto ldw = [&](const float *p) { return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); };
+    const float m = lane < ns ? ldw(t.part_m + p0 + lane) : -FLT_MAX, l = lane < ns ? ldw(t.part_l + p0 + lane) : 0.f;
+    const __amdgpu_buffer_rsrc_t ro = __builtin_amdgcn_make_buffer_rsrc((void *)(t.part_o + p0 * HD), (short)0, ns * HD * 4, 0x00020000);
+    v2u r[4][MB];
+#pragma unroll
+    for (int g = 0; g < 4; ++g)
+      if (g * MB < ns) {  // wave-uniform; past the last split: zeros
+#pragma unroll
+        for (int k = 0; k < MB; ++k) r[g][k] = __builtin_amdgcn_raw_buffer_load_b64(ro, (unsigned)lane * 8u + (unsigned)(g * MB + k) * 512u, 0, 16);
+      }
+    const float w = fast_exp_ref(m - dec2::wave_max_all(m)), lw = l * w;  // split j's in lane j
+    float s_all = 0.f, a0 = 0.f, a1 = 0.f;
+#pragma unroll
+    for (int g = 0; g < 4; ++g)
+      if (g * MB < ns) {
+#pragma unroll
+        for (int k = 0; k < MB; ++k)
+          if (g * MB + k < ns) {
+            const float wj = dec2::rlf(w, g * MB + k), lwj = dec2::rlf(lw, g * MB + k);
+            const float t0 = __uint_as_float(r[g][k].x) * wj, t1 = __uint_as_float(r[g][k].y) * wj;
+            s_all = s_all + lwj;
+            a0 = a0 + t0; a1 = a1 + t1;
+          }
+      }
+    const float inv = 1.0f / s_all;
+    *(float2 *)&o_s[wave + 4 * i][2 * lane] = make_float2(a0 * inv, a1 * inv);
+  }
+  __syncthreads();
+  if (wave >= G / 2) return;  // wave w: heads 2 w, 2 w + 1 = superblock (kvh G / 2 + w) of the attention vector
+  const float4 v = *(const float4 *)&o_s[2 * wave + (lane >> 5)][(lane & 31) * 4];
+  const int head0 = kvh * G + 2 * wave;
+  if (t.out) *(float4 *)(t.out + ((size_t)seq * t.num_heads + head0) * HD + lane * 4) = v;
+  if (a.img) quantize_sb(v, head0 >> 1, seq, ACT_Q8K, (char *)a.img, t.num_heads * HD, ncols);
+}
+// the hand-off of dec_attn2_kernel: true in the workgroup that arrives last of `wgs`
+__device__ __forceinline__ bool attn4_last(const Attn2Args &a, int kvh, int seq, int wgs, int tid, int *last_s) {
+  MRS_WAIT_VMCNT0();  // this wave's partials have left the CU
+  __syncthreads();
+  unsigned *tk = a.ticket + (size_t)seq * a.t.num_kv_heads + kvh;
+  if (tid == 0) *last_s = __hip_atomic_fetch_add(tk, 1u, MRS_DEC_ATTN_TICKET_ORDER, __HIP_MEMORY_SCOPE_AGENT) == (unsigned)(wgs - 1);
+  __syncthreads();
+  if (!*last_s) return false;
+  if (tid == 0) __hip_atomic_store(tk, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);  // every other workgroup of this (seq, kv head) has already drawn
+  return true;
+}
+// Splits of one block (model contexts up to 2048): workgroup = four waves = splits 4 z .. 4 z + 3 of a (sequence, kv head); G = 8: two splits, two groups of heads each
+template <int G, class CT, bool TICKET>
+__global__ void __launch_bounds__(256, 3) dec_attn4_kernel(const Attn2Args a) {
+  constexpr int HG = G / 4, SPW = 4 / HG;  // groups of four heads; splits of a workgroup
+  __shared__ __attribute__((aligned(16))) char v_s[4][A4_V];
+  __shared__ __attribute__((aligned(16))) float p_s[4][4 * A4_P], q_s[4][8 * A4_Q], o_s[G][128];
+  __shared__ int last_s;
+  const AttnArgs &t = a.t;
+  const int tid = tid_opaque(), lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int kvh = blockIdx.x, seq = blockIdx.y, split0 = blockIdx.z * SPW, split = split0 + wave / HG, head0 = kvh * G + wave % HG * 4;
+  // the page index does not depend on the context length: both scalar loads leave together
+  const unsigned page = t.block_tables[(size_t)seq * t.max_blocks_per_seq + min(split, t.max_blocks_per_seq - 1)];
+  const int ctx = (int)t.context_lens[seq], ns = (ctx + 31) / 32;
+  if (split0 >= ns) return;  // workgroup-uniform: no split of this sequence lands here
+  if (split < ns) {
+    const int lo = t.window > 0 && ctx > t.window ? ctx - t.window : 0;
+    float m = -FLT_MAX, l = 0.f;
+    f4v o[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+    if ((split + 1) * 32 > lo) {  // else the block lies before the sliding window: the partial a fully masked pass would give, without reading K / V
+      const size_t base = (size_t)page * t.kv_block_stride + (size_t)kvh * t.kv_head_stride;
+      int4 kr[8];
+      attn_load_k(t, base, kr);
+      attn4_stage_q(t, seq, head0, q_s[wave], lane);
+      attn4_stage_v(t, base, v_s[wave], lane);
+      MRS_WAVE_SYNC();
+      float val[2]; bool ok[2];
+      m = attn4_scores<CT>(t, kr, q_s[wave], split, ctx, lo, lane, val, ok);
+      l = attn4_probs(val, ok, m, p_s[wave], lane);
+      MRS_WAIT_VMCNT0();  // the values have landed
+      MRS_WAVE_SYNC();
+      attn4_values<CT, 2>(v_s[wave], p_s[wave], split, ctx, 0, lane, o);
+    }
+    attn4_publish_o<TICKET>(t, seq, head0, split, 0, lane, o[0]);
+    attn4_publish_o<TICKET>(t, seq, head0, split, 64, lane, o[1]);
+    if (lane < 4) attn4_publish_ml<TICKET>(t, seq, head0 + lane, split, m, l);
+  }
+  if constexpr (TICKET) {
+    if (attn4_last(a, kvh, seq, (ns + SPW - 1) / SPW, tid, &last_s)) attn4_merge<G>(a, kvh, seq, ns, wave, lane, gridDim.y, o_s);
+  }
+}
+// Splits of several blocks: a workgroup per split, its blocks in groups of four.  Wave w scores block w of the group (all heads); the running maximum over the blocks is known from
+// their maxima, so the probabilities are formed side by side too, and only P . V walks the blocks: wave w owns 64 dims of four heads (G = 4: waves 0 and 1).  All four blocks
+// are requested at once -- one after another they were four memory latencies of 2.5 - 3 us -- the next group's while this one's are multiplied.
+template <int G, class CT, bool TICKET>
+__global__ void __launch_bounds__(256, 2) dec_attn4_long_kernel(const Attn2Args a) {
+  constexpr int HG = G / 4;
+  extern __shared__ __attribute__((aligned(16))) char v_dyn[];  // [bpw > 4 ? 2 : 1][4][A4_V]
+  __shared__ __attribute__((aligned(16))) float p_s[4][HG][4 * A4_P], q_s[HG][8 * A4_Q], o_s[G][128], mx_s[2][4][G], ps_s[4][G];  // mx_s: the waves without P . V write the next group's maxima while the others still read these
+  __shared__ int last_s;
+  const AttnArgs &t = a.t;
+  const int tid = tid_opaque(), lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), hd = lane & 3;
+  const int kvh = blockIdx.x, seq = blockIdx.y, split = blockIdx.z;
+  const uint32_t *bt = t.block_tables + (size_t)seq * t.max_blocks_per_seq;
+  unsigned page = bt[min(split * t.bpw + wave, t.max_blocks_per_seq - 1)];
+  const int ctx = (int)t.context_lens[seq], nblk = (ctx + 31) / 32, ns = (nblk + t.bpw - 1) / t.bpw;
+  if (split >= ns) return;  // workgroup-uniform
+  const int b0 = split * t.bpw, b1 = min(b0 + t.bpw, nblk), lo = t.window > 0 && ctx > t.window ? ctx - t.window : 0;
+  const int pv_hg = G == 8 ? wave >> 1 : 0, pv_dim = (wave & 1) * 64;  // P . V: the wave's group of heads and dims
+  const bool pv = G == 8 || wave < 2;
+  float m_run[HG], l = 0.f, m_pv = -FLT_MAX;
+  f4v o[1] = {{0.f, 0.f, 0.f, 0.f}};
+#pragma unroll
+  for (int h = 0; h < HG; ++h) m_run[h] = -FLT_MAX;
+  if (b1 * 32 > lo) {  // else every block lies before the sliding window
+    auto base_of = [&](unsigned pg) { return (size_t)pg * t.kv_block_stride + (size_t)kvh * t.kv_head_stride; };
+    int4 kr[8];
+    attn_load_k(t, base_of(page), kr, b0 + wave < b1 ? KV_BLOCK_BYTES : 0);
+    if (wave < HG) attn4_stage_q(t, seq, kvh * G + wave * 4, q_s[wave], lane);
+    if (b0 + wave < b1) attn4_stage_v(t, base_of(page), v_dyn + wave * A4_V, lane);
+    page = bt[min(b0 + 4 + wave, b1 - 1)];
+    __syncthreads();
+    for (int g0 = b0, it = 0; g0 < b1; g0 += 4, ++it) {
+      const int b = g0 + wave, nb = min(4, b1 - g0);
+      const size_t next = base_of(page);
+      float val[HG][2]; bool ok[HG][2];
+      if (b < b1) {
+#pragma unroll
+        for (int h = 0; h < HG; ++h) {
+          const float mx = attn4_scores<CT>(t, kr, q_s[h], b, ctx, lo, lane, val[h], ok[h]);
+          if (lane < 4) mx_s[it & 1][wave][h * 4 + lane] = mx;
+        }
+      }
+      MRS_WAIT_VMCNT0();  // (the values of this group: requested a group ago)
+      __syncthreads();    // A: the maxima; everyone has finished with the last group's probabilities and values
+      if (g0 + 4 < b1) {
+        attn_load_k(t, next, kr, b + 4 < b1 ? KV_BLOCK_BYTES : 0);
+        if (b + 4 < b1) attn4_stage_v(t, next, v_dyn + ((it + 1) & 1) * 4 * A4_V + wave * A4_V, lane);
+        page = bt[min(b + 8, b1 - 1)];
+      }
+      if (b < b1) {
+#pragma unroll
+        for (int h = 0; h < HG; ++h) {
+          float mn = m_run[h];
+          for (int w = 0; w <= wave; ++w) mn = fmaxf(mn, mx_s[it & 1][w][h * 4 + hd]);
+          const float ps = attn4_probs(val[h], ok[h], mn, p_s[wave][h], lane);
+          if (lane < 4) ps_s[wave][h * 4 + lane] = ps;
+        }
+      }
+#pragma unroll
+      for (int h = 0; h < HG; ++h)
+        for (int w = 0; w < nb; ++w) m_run[h] = fmaxf(m_run[h], mx_s[it & 1][w][h * 4 + hd]);
+      __syncthreads();  // B: the probabilities
+      if (pv) {
+        for (int w = 0; w < nb; ++w) {
+          const float mn = fmaxf(m_pv, mx_s[it & 1][w][pv_hg * 4 + hd]), ps = ps_s[w][pv_hg * 4 + hd];
+          if (g0 + w == b0) {
+            l = ps;
+          } else {
+            const float alpha = fast_exp_ref(m_pv - mn);
+            l = l * alpha + ps;
+            o[0] = o[0] * alpha;
+          }
+          m_pv = mn;
+          attn4_values<CT, 1>(v_dyn + (it & 1) * 4 * A4_V + w * A4_V, p_s[w][pv_hg], g0 + w, ctx, pv_dim, lane, o);
+        }
+      }
+    }
+  }
+  if (pv) {
+    attn4_publish_o<TICKET>(t, seq, kvh * G + pv_hg * 4, split, pv_dim, lane, o[0]);
+    if (pv_dim == 0 && lane < 4) attn4_publish_ml<TICKET>(t, seq, kvh * G + pv_hg * 4 + lane, split, m_pv, l);
+  }
+  if constexpr (TICKET) {
+    if (attn4_last(a, kvh, seq, ns, tid, &last_s)) attn4_merge<G>(a, kvh, seq, ns, wave, lane, gridDim.y, o_s);
+  }
+}
 // the merge as its own launch: grid (kv heads, sequences), (G + 1) / 2 waves
 template <int G>
 __global__ void __launch_bounds__(64 * ((G + 1) / 2)) dec_attn2_merge_kernel(const Attn2Args a) {
@@ -578,9 +881,24 @@ extern "C" int mrs_dec_attention(float *out_f32, void *img_out, unsigned *ticket
       hipLaunchKernelGGL((dec_attn2_merge_kernel<GG>), mgrid, dim3(64 * ((GG + 1) / 2)), 0, s, a);                       \
     }                                                                                                                    \
   } while (0)
-#define MRS_A2G(CT) switch (G) { case 1: MRS_A2(1, CT); break; case 2: MRS_A2(2, CT); break; case 4: MRS_A2(4, CT); break; default: MRS_A2(8, CT); break; }
+  // groups of four and eight heads
+#define MRS_A4(GG, CT)                                                                                                   \
+  do {                                                                                                                   \
+    const dim3 grid4(num_kv_heads, num_seqs, (nsplit + 16 / GG - 1) / (16 / GG));                                        \
+    const size_t lds = (t.bpw > 4 ? 2 : 1) * 4 * A4_V;                                                                   \
+    if (t.bpw == 1 && one_launch) hipLaunchKernelGGL((dec_attn4_kernel<GG, CT, true>), grid4, dim3(256), 0, s, a);           \
+    else if (t.bpw == 1) hipLaunchKernelGGL((dec_attn4_kernel<GG, CT, false>), grid4, dim3(256), 0, s, a);                   \
+    else {                                                                                                               \
+      auto kern = one_launch ? dec_attn4_long_kernel<GG, CT, true> : dec_attn4_long_kernel<GG, CT, false>;                 \
+      lds_attr_once((const void *)kern, 2 * 4 * A4_V);                                                                   \
+      hipLaunchKernelGGL(kern, grid, dim3(256), lds, s, a);                                                              \
+    }                                                                                                                    \
+    if (!one_launch) hipLaunchKernelGGL((dec_attn2_merge_kernel<GG>), mgrid, dim3(64 * ((GG + 1) / 2)), 0, s, a);            \
+  } while (0)
+#define MRS_A2G(CT) switch (G) { case 1: MRS_A2(1, CT); break; case 2: MRS_A2(2, CT); break; case 4: MRS_A4(4, CT); break; default: MRS_A4(8, CT); break; }
   if (kv_dtype == 1) { MRS_A2G(bf16_t) } else { MRS_A2G(f16_t) }
 #undef MRS_A2G
+#undef MRS_A4
 #undef MRS_A2
   return with_img ? 1 : 0;
 }

@@ -285,6 +285,21 @@ static hiphost_f32x32 mfma_32x32x1_f32(float a, float b, hiphost_f32x32 c) {
 }
 }  // namespace hiphost
 #define __builtin_amdgcn_mfma_f32_32x32x1f32(A, B, C, CBSZ, ABID, BLGP) hiphost::mfma_32x32x1_f32((A), (B), (C))
+// v_mfma_f32_4x4x1_16b_f32: sixteen blocks of 4 x 4 outer products, D_b = C_b + a_b b_b: lane l holds a_b[l % 4] and b_b[l % 4] of block b = l / 4 and receives column l % 4, row v in
+// register v
+typedef float hiphost_f32x4 __attribute__((ext_vector_type(4)));
+namespace hiphost {
+static hiphost_f32x4 mfma_4x4x1_f32(float a, float b, hiphost_f32x4 c) {
+  const int tid = linear_tid(), w = tid / WAVE, lane = tid & (WAVE - 1), base = w * WAVE;
+  mfma_af[tid] = a; mfma_bf[tid] = b;
+  wave_barrier(w, 0);
+  hiphost_f32x4 d = c;
+  for (int i = 0; i < 4; ++i) d[i] = fmaf(mfma_af[base + (lane & ~3) + i], mfma_bf[base + lane], c[i]);
+  wave_barrier(w, 0);
+  return d;
+}
+}  // namespace hiphost
+#define __builtin_amdgcn_mfma_f32_4x4x1f32(A, B, C, CBSZ, ABID, BLGP) hiphost::mfma_4x4x1_f32((A), (B), (C))
 // v_mfma_i32_32x32x32_i8: D = A (32 x 32 int8) * B (32 x 32 int8) + C, exact in int32.  Lane l holds A[l % 32][16 * (l / 32) + j] and
 // B[16 * (l / 32) + j][l % 32] (j = 0..15, 16 consecutive bytes); C / D as every 32 x 32 MFMA (the layout of the accumulators is dtype-independent).
 // Which 16 k a lane half holds does not change the result as long as A and B agree -- they do by symmetry.
@@ -357,6 +372,10 @@ static inline short hiphost_raw_buffer_load_b16(__amdgpu_buffer_rsrc_t r, unsign
 static inline void hiphost_raw_buffer_store_b32(unsigned v, __amdgpu_buffer_rsrc_t r, unsigned voff) {
   if ((unsigned long long)voff + 4 <= r.bytes) memcpy((char *)r.base + voff, &v, 4);
 }
+static inline void hiphost_raw_buffer_store_b128(hiphost_v4u v, __amdgpu_buffer_rsrc_t r, unsigned voff) {
+  if ((unsigned long long)voff + 16 <= r.bytes) memcpy((char *)r.base + voff, &v, 16);
+}
+#define __builtin_amdgcn_raw_buffer_store_b128(V, R, VOFF, SOFF, AUX) hiphost_raw_buffer_store_b128((V), (R), (VOFF))
 #define __builtin_amdgcn_raw_buffer_store_b32(V, R, VOFF, SOFF, AUX) hiphost_raw_buffer_store_b32((V), (R), (VOFF))
 typedef _Float16 hiphost_h2 __attribute__((ext_vector_type(2)));
 #define __builtin_amdgcn_cvt_pkrtz(A, B) (hiphost_h2{(_Float16)(A), (_Float16)(B)}) /* used on values that f16 holds exactly */

@@ -463,6 +463,21 @@ def test_attention_splits_of_several_blocks_gpu(oracle, dev, heads, kvh, ctxs, m
     check_attention(oracle, GpuBackend(dev), heads, kvh, ctxs, max_ctx, kvd, n_out=256, window=window, nan_past=True)
 
 
+# splits of 5, 8 and 9 blocks: a workgroup's groups of four with remainders, a last split of one block, a window that begins inside a group; groups of four and eight heads
+GROUPS = [(4, 1, [517, 33], 8224, 1, 0), (8, 1, [513, 1], 16384, 1, 0), (8, 2, [900], 18400, 0, 300)]
+
+
+@pytest.mark.parametrize("heads,kvh,ctxs,max_ctx,kvd,window", GROUPS)
+def test_attention_splits_of_more_than_four_blocks_host_emulation(oracle, heads, kvh, ctxs, max_ctx, kvd, window):
+    check_attention(oracle, HostBackend(), heads, kvh, ctxs, max_ctx, kvd, window=window, nan_past=True)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("heads,kvh,ctxs,max_ctx,kvd,window", GROUPS + [(32, 8, [9001, 2000], 9024, 1, 0), (64, 8, [9001, 160], 9024, 1, 4000)])
+def test_attention_splits_of_more_than_four_blocks_gpu(oracle, dev, heads, kvh, ctxs, max_ctx, kvd, window):
+    check_attention(oracle, GpuBackend(dev), heads, kvh, ctxs, max_ctx, kvd, n_out=256, window=window, nan_past=True)
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("heads,kvh,ctxs,max_ctx,kvd", [(32, 8, [700], 832, 1), (32, 8, [1024, 3, 515], 1024, 1), (8, 4, [129], 160, 0), (64, 8, [333, 1000], 1024, 1)])
 def test_fused_attention_gpu(oracle, dev, heads, kvh, ctxs, max_ctx, kvd):
