@@ -583,6 +583,26 @@ __global__ void __launch_bounds__(NT) dec_act_image_kernel(const ActImgArgs a) {
   const int c0 = a.rows ? c : a.gc0[c], n = a.rows ? 1 : a.gn[c];
   act_quantize_all<1, 1>(a.img + act_bytes(a.K, c0), red, pre, x, a.ldx, a.norm_w, a.eps, a.K, a.mode, wave, c - c0, n);
 }
+// Rows without a norm (down_proj's): a superblock knows nothing of the others, so four waves take two each and a row spreads over K / 2048 workgroups; one workgroup per row was a
+// serial chain of seven superblocks per wave.  A decode step of 32 layers with 14336 values per row, us: 2 rows 2487 / 2363, 8 rows 2875 / 2726 (the launch alone: 4.7 and 4.4, of
+// which about 3 are an empty launch's in the trace).
+__global__ void __launch_bounds__(256) dec_act_image_split_kernel(const ActImgArgs a) {
+  const int tid = tid_opaque(), lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int c = (int)blockIdx.x, sb0 = ((int)blockIdx.y * 4 + wave) * 2, S = a.K / 256;
+  if (sb0 >= S) return;
+  const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc((void *)(a.x + (size_t)c * a.ldx), (short)0, a.K * 4, 0x00020000);
+  float4 v[2];
+#pragma unroll
+  for (int n = 0; n < 2; ++n) v[n] = as_f4(__builtin_amdgcn_raw_buffer_load_b128(r, (unsigned)(sb0 + n) * 1024u + (unsigned)lane * 16u, 0, 0));  // past the row: zeros
+  const int sb[2] = {sb0, sb0 + 1};
+  const bool live[2] = {true, sb0 + 1 < S};
+  const int c0 = a.rows ? c : a.gc0[c], n = a.rows ? 1 : a.gn[c];
+  quantize_multi<2>(v, sb, live, c - c0, a.mode, a.img + act_bytes(a.K, c0), a.K, n);
+}
+static void act_image_launch(const ActImgArgs &a, int rows, hipStream_t s) {
+  if (a.norm_w) hipLaunchKernelGGL(dec_act_image_kernel, dim3(rows), dim3(NT), 0, s, a);
+  else hipLaunchKernelGGL(dec_act_image_split_kernel, dim3(rows, (a.K / 256 + 7) / 8), dim3(256), 0, s, a);
+}
 // the column groups of a batch of b columns of K values: halved until a group's image fits LDS (the same recursion as Launch::run)
 constexpr size_t LDS_IMG_MAX = (size_t)158 * 1024;
 static void col_groups(int K, int c0, int b, int *gc0, int *gn) {
@@ -809,7 +829,7 @@ extern "C" int mrs_dec_act_image(const float *x, int ldx, const float *norm_w, f
   ActImgArgs a{};
   a.x = x; a.ldx = ldx; a.norm_w = norm_w; a.eps = eps; a.K = k; a.mode = act_mode_for(weight_type); a.img = (char *)img_out;
   col_groups(k, 0, b, a.gc0, a.gn);
-  hipLaunchKernelGGL(dec_act_image_kernel, dim3(b), dim3(NT), 0, (hipStream_t)stream, a);
+  act_image_launch(a, b, (hipStream_t)stream);
   return hipGetLastError() == hipSuccess ? 0 : -4;
 }
 // the same for any number of rows, row r's image alone at r * mrs_dec_act_image_bytes(k, 1): the operand rows of mrs_dec_mm_*_experts
@@ -817,7 +837,7 @@ extern "C" int mrs_dec_act_image_rows(const float *x, int ldx, const float *norm
   if (!x || !img_out || rows < 1 || k <= 0 || k % 256 || !dec_type(weight_type) || ((uintptr_t)img_out & 15)) return -1;
   ActImgArgs a{};
   a.x = x; a.ldx = ldx; a.norm_w = norm_w; a.eps = eps; a.K = k; a.mode = act_mode_for(weight_type); a.img = (char *)img_out; a.rows = rows;
-  hipLaunchKernelGGL(dec_act_image_kernel, dim3(rows), dim3(NT), 0, (hipStream_t)stream, a);
+  act_image_launch(a, rows, (hipStream_t)stream);
   return hipGetLastError() == hipSuccess ? 0 : -4;
 }
 // mrs_dec_qkv / mrs_dec_qkv_neox (neox != 0) on an image of RmsNorm(h) made by mrs_dec_act_image for these weights
