@@ -3,18 +3,20 @@
 // Reference role: the MMVQ launchers take 1 .. 8 activation columns from ONE pass over the weights (mistralrs-quant/kernels/mmvq_gguf/mmvq_gguf.cu:724-792,
 // gguf/fast_mmvq.rs:52 MMVQ_MAX_BATCH; GgufMatMul::try_fast_forward, gguf/mod.rs:298-323).  The engine's batched GEMV (dec_core2.cuh, NCOLS = 2 .. 8) does that on the
 // vector ALU: 535 VALU + 48 ds_read per tile of 16 superblocks x 8 columns -- at batch 8 the launches are bound by that arithmetic, not by the weight stream
-// (profiles/round5_decode.md: 0.13 of the step roofline).  Here the integer dots run on v_mfma_i32_32x32x32_i8 / 32x32x16_i8:
+// (profiles/round5_decode.md: 0.13 of the step roofline).  Here the integer dots run on v_mfma_i32_16x16x64_i8 / 16x16x32_i8:
 //   * weights: the MFMA-order copy the exact prompt GEMM already keeps in HBM (ext_gemm_qi.hip qi_repack_kernel: 32-row panels, one record per panel and superblock,
-//     every lane's 16 bytes of a piece contiguous): a record is 4.6 KB (Q4_K) / 8.6 KB (Q5_K, Q6_K, Q8_0) of consecutive bytes, `nt` loads, 2-3 records in flight per wave;
+//     every lane's 16 bytes of a piece contiguous): a record is 4.6 KB (Q4_K) / 8.6 KB (Q5_K, Q6_K, Q8_0) of consecutive bytes, of which a unit of 16 rows takes 256 consecutive bytes
+//     of every half piece; `nt` loads, two pairs of records in flight per wave;
 //   * activations: the image mrs_dec_act_image builds once per phase (int8 quants, block scales, run sums: dec_core2.cuh), copied into LDS by every workgroup; the MFMA's
-//     A operand = 8 or 16 int8 of a token read straight from it (tokens are the M rows: lane l supplies token l % 32, only rows < b are real), B = the weight bytes;
-//     the accumulator registers 0 .. 3 of a lane are tokens 4 (l / 32) + i of weight row l % 32: four live outputs per lane for b <= 8;
+//     A operand = 8 or 16 int8 of a token read straight from it, B = the weight bytes: two superblocks of 16 rows x 8 tokens per wave and step (term());
 //   * per sub-block the exact int32 dot times the 6 / 8-bit scale (v_mad per live output), mins / offsets as ONE f16 MFMA over the 16 run sums, then the engine's
 //     f32 term per superblock -- ORD-U, the order of dec_core2.cuh / ext_gemm_qi.hip / oracle orc_gemv_engine: a token's result is bit for bit what the batch-1 GEMV,
 //     the batched VALU GEMV and the prompt GEMM give (tests/test_dec_mm.py);
-//   * workgroup = 4 waves = the 4 ORD-U runs of superblocks of ONE 32-row panel at a time; the four run sums meet in LDS (double buffered: one barrier per panel),
-//     256 threads = 8 tokens x 32 rows finish ((c0 + c1) + c2) + c3 and run the phase's epilogue (store / residual / GLU / RoPE + paged-cache write).
-// The weight stream is what a launch costs: ~4.9 GB per step for the 8B Q4_K_M model whatever b is.
+//   * workgroup = 4 waves = the 4 ORD-U runs of superblocks of ONE unit of 16 rows at a time; the four run sums meet in LDS (double buffered: one barrier per unit),
+//     128 threads = 8 tokens x 16 rows finish ((c0 + c1) + c2) + c3 and run the phase's epilogue (store / residual / GLU / RoPE + paged-cache write).
+// Units of 16 rows, not of the panel's 32: o_proj and down_proj of 4096 rows are 128 panels, half the chip, and their launches are bound by the chain of a wave's records.
+// us per launch, weights from HBM, 8 columns, units of 32 rows on the 32-row MFMAs / this: 4096 x 4096 Q4_K 9.15 / 7.8, 4096 x 14336 Q4_K 17.2 / 13.5, Q6_K 22.4 / 18.1; gate + up of
+// 14336 x 4096 17.3 / 17.3 (66 MB: 11 us of stream, 3 of prologue).
 // Sparse-MoE layers (MOE): a workgroup takes the panels of ONE expert that some token was routed to and multiplies them by that expert's tokens only (its columns: the routes
 // whose id is the expert's, at most one per token), so every expert's weights are read once per step instead of once per route; the workgroups are dealt to the experts in
 // use, which the kernel finds in the router's ids.
@@ -29,9 +31,22 @@ using namespace mrs::dec2;
 using mrs::dec::EPI_STORE; using mrs::dec::EPI_RESID; using mrs::dec::EPI_GLU; using mrs::dec::EPI_QKV;
 using mrs::dec::TM_Q4K; using mrs::dec::TM_Q5K; using mrs::dec::TM_Q6K; using mrs::dec::TM_Q80; using mrs::dec::tmask_of;
 
+#ifndef MRS_BLDS16  // (the host build of the kernels has its own)
+#define MRS_BLDS16(rsrc, lbase, voff) __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, (__attribute__((address_space(3))) void *)(lbase), 16, voff, 0, 0, 0)
+#define MRS_BLDS4(rsrc, lbase, voff) __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, (__attribute__((address_space(3))) void *)(lbase), 4, voff, 0, 0, 0)
+#endif
+#ifndef MRS_KEEP_BRANCH  // (a uniform branch instead of a select per value)
+#define MRS_KEEP_BRANCH() asm volatile("")
+#endif
+#ifndef MRS_OPAQUE
+#define MRS_OPAQUE(v) asm("" : "+v"(v))
+#endif
+#ifndef MRS_WAIT_VMCNT  // (the builtin: hipcc's own waits count it, an asm's they do not)
+#define MRS_WAIT_VMCNT(n) do { __builtin_amdgcn_s_waitcnt(0x0F70 | ((n) & 15) | (((n) >> 4) << 14)); asm volatile("" ::: "memory"); } while (0)
+#endif
+
 typedef int i4v __attribute__((ext_vector_type(4)));
-typedef int i16v __attribute__((ext_vector_type(16)));
-typedef float f16v __attribute__((ext_vector_type(16)));
+typedef float f4v __attribute__((ext_vector_type(4)));
 typedef _Float16 h8 __attribute__((ext_vector_type(8)));
 
 constexpr int MT = 256;                                  // 4 waves
@@ -39,17 +54,17 @@ constexpr int REC_Q4K = 4096 + 512 + 128, REC_BIG = 8192 + 512 + 128;  // == ext
 __host__ __device__ constexpr int rec_bytes(int type) { return type == T_Q4_K ? REC_Q4K : REC_BIG; }
 __host__ __device__ inline bool mm_type(int t) { return t == T_Q4_K || t == T_Q5_K || t == T_Q6_K || t == T_Q8_0; }
 
-struct MmTensor { const uint8_t *w; unsigned bytes; int type, npanels, nrows; };
+struct MmTensor { const uint8_t *w; unsigned bytes; int type, nhalves, nrows; };  // nhalves: 16-row halves of its panels
 struct MmArgs {
   MmTensor m[3];
-  int epi, nseg, units;        // GLU: a unit = panel u of m[0] (gate) then panel u of m[1] (up); QKV: units enumerate the panels of m[0], m[1], m[2]; else panels of m[0]
+  int epi, nseg, units;        // a unit = 16 rows.  GLU: half panel u of m[0] (gate), then of m[1] (up); QKV: units enumerate the half panels of m[0], m[1], m[2]; else of m[0]
   int K, nc, mode;             // activation columns (<= 8), ACT_Q8K / ACT_Q80
   const char *img; unsigned gc0p, gnp;  // the image(s) mrs_dec_act_image wrote: column c lives in the group image at act_bytes(K, gc0), gn columns wide (gc0 / gn - 1: 4 bits per column; an
                                        // array indexed by a run-time column would make hipcc copy the whole argument block to scratch memory)
   float *out; int out_stride; float resid_scale; int activation;
   float *q_out; void *k_cache, *v_cache; const int64_t *slot_mapping; const int32_t *positions; const float *cos_t, *sin_t;
   int head_dim, rot_pairs, num_kv_heads, block_size, cache_x, kv_f16, hd_shift, bs_shift, x_shift;
-  const int32_t *ids; int nroutes, experts, route_div;  // MOE: the router's ids [nroutes <= 64] (npanels / nrows: of one expert); route r reads image row r / route_div, writes output row r
+  const int32_t *ids; int nroutes, experts, route_div;  // MOE: the router's ids [nroutes <= 64] (nhalves / nrows: of one expert); route r reads image row r / route_div, writes output row r
   unsigned long long *tl;  // experiments: 8 s_memrealtime stamps (100 MHz) per wave, or nullptr (mrs_dec_mm_timeline)
 };
 #ifdef MRS_MM_TIMELINE  // (a conditional store inside the streaming loop makes every wait of the ring stricter: off in the product build)
@@ -58,12 +73,13 @@ struct MmArgs {
 #define MRS_MM_TL(i) do { } while (0)
 #endif
 
+constexpr int LDS_ZEROS = 256, LDS_MAX = 158 * 1024 - 3840;  // (rows and columns are accepted as when the sums took 8 KB)
 // LDS: quants [nc][QCS] (a column = the image's 4 runs of CQ bytes, + 32 bytes of skew: the 8 tokens of a ds_read_b64 lane group land in 8 different bank pairs);
-// Q8K mode: yd [Sp][8] f32, bsf [Sp][8][16] f16;  Q80 mode: yd8 [Sp][8 blocks][8] f32;  ex [2][4][8][32] f32
+// Q8K mode: yd [Sp][8] f32, bsf [Sp][8][16] f16;  Q80 mode: yd8 [Sp][8 blocks][8] f32;  ex [2][4][8][16] f32;  256 bytes of zeros
 __host__ __device__ inline int qcs_of(int K) { return 4 * act_cq(K) + 32; }
 __host__ __device__ inline size_t lds_bytes(int K, int nc, int mode) {
   const size_t sp = (size_t)act_sp(K);
-  return (size_t)nc * qcs_of(K) + (mode == ACT_Q80 ? sp * 256 : sp * (32 + 256)) + 2 * 4 * 8 * 32 * 4;
+  return (size_t)nc * qcs_of(K) + (mode == ACT_Q80 ? sp * 256 : sp * (32 + 256)) + 2 * 4 * 8 * 16 * 4 + LDS_ZEROS;
 }
 
 template <int NPC> struct Rec { v4u q[NPC]; v4u hs; unsigned hd; };
@@ -71,197 +87,161 @@ template <int NPC> struct Rec { v4u q[NPC]; v4u hs; unsigned hd; };
 __device__ __forceinline__ i4v mk_i4(v2u a, v2u b) { return i4v{(int)a.x, (int)a.y, (int)b.x, (int)b.y}; }
 __device__ __forceinline__ long mk_l(unsigned lo, unsigned hi) { return (long)(((unsigned long long)hi << 32) | lo); }
 
-// the engine's f32 term T of superblock sb for the lane's four live tokens 4 hf + i (weight row nn of the panel), from the record's registers
-template <int TYPE, int NPC>
-__device__ __forceinline__ void term(const Rec<NPC> &w, int sb, const char *qcol /* the lane's token column + the superblock's offset */, const char *ydp, const char *bsp,
-                                     int hf, float (&T)[4]) {
-  const i16v zero = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
+// The operands of two superblocks that come from LDS, read one record ahead: the 16 reads of a record, of four waves in step, take longer than half of its arithmetic.  A: K-quants the
+// 8 elements 16 k + 8 hf .. of the token's superblock, Q8_0 8 bytes each of elements 32 g + 16 hf ..; the token's run sums; the four tokens' scales (Q8_0: per block, term()).
+struct Ops { v2u A[16]; h8 bsf; float4 y4; };
+template <bool Q80>
+__device__ __forceinline__ void read_ops(Ops &o, const char *qa, const char *bsp, const char *ydp, int hf) {
+#pragma unroll
+  for (int k = 0; k < 16; ++k) o.A[k] = *(const v2u *)(qa + (Q80 ? 32 * (k >> 1) + 8 * (k & 1) : 16 * k));
+  if constexpr (!Q80) { o.bsf = *(const h8 *)bsp; o.y4 = *(const float4 *)(ydp + 4 * hf * 4); }
+}
+
+// acc += s d, one v_mad_i32_i24 each: opaque scale and sums keep hipcc from multiplying with a byte select and adding threes (1.5 instructions instead of 1.25 with the extraction)
+__device__ __forceinline__ void mad4(int (&acc)[4], int s, const i4v &d) {
+  MRS_OPAQUE(s);
+#pragma unroll
+  for (int i = 0; i < 4; ++i) { acc[i] += __mul24(s, d[i]); MRS_OPAQUE(acc[i]); }
+}
+
+// The engine's f32 term T of TWO superblocks of a run at once -- a lane's own is t + l / 32 --, for the lane's row l % 16 of 16 and its tokens 4 (l / 16 % 2) + i.  The 16-row shapes,
+// every result register live: tokens are only 8 rows of A, so rows 0 .. 7 are the tokens against superblock t and rows 8 .. 15 the same tokens against t + 1, each in its own half of k
+// (lanes 0 .. 31 supply the k of t, 32 .. 63 of t + 1; the A lanes of the other rows read the zeros at the end of LDS), and B's lanes hold their own superblock's weights as loaded.
+// What bounds a launch is this chain, not the stream: one wave per SIMD (LDS admits one workgroup per CU at 14336 values) that waits for nothing in memory.  On the 32-row shapes 12 of
+// 16 result registers are dead, hipcc lays the next result over them and the products wait for one another: a record took a wave 0.71 us (Q4_K) and 1.05 us (Q6_K) for 32 rows of one
+// superblock, now 0.55 and 0.8 us for 16 rows of two, on twice the CUs.
+// `next` asks for the operands of the following record as soon as the products have taken these: the scale arithmetic covers their way.
+template <int TYPE, int NPC, class Next>
+__device__ __forceinline__ void term(const Rec<NPC> &w, Ops &o, Next next, const char *ydp, int hf, float (&T)[4]) {
+  const i4v zero = {0, 0, 0, 0};
   if constexpr (TYPE == T_Q8_0) {
-    // block g: 32 int8 of the weight row x 32 int8 of the token: one MFMA; p_g = ((float)isum dw_g) dx_g, T = p_0 + p_1 + ... left to right (Tile<T_Q8_0>)
+    // block g: 32 int8 of the weight row x 32 int8 of the token; p_g = ((float)isum dw_g) dx_g, T = p_0 + p_1 + ... left to right (Tile<T_Q8_0>)
+    i4v d[8];
 #pragma unroll
-    for (int g2 = 0; g2 < 2; ++g2) {
-      i16v d[4];
-      i4v wa[4];
+    for (int g = 0; g < 8; ++g) d[g] = __builtin_amdgcn_mfma_i32_16x16x64_i8(mk_i4(o.A[2 * g], o.A[2 * g + 1]), __builtin_bit_cast(i4v, w.q[g % NPC]), zero, 0, 0, 0);
+    __builtin_amdgcn_sched_barrier(0);
+    next();
+    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-      for (int h = 0; h < 4; ++h) wa[h] = *(const i4v *)(qcol + 32 * (4 * g2 + h) + 16 * hf);
-      __builtin_amdgcn_sched_barrier(0);
+    for (int g = 0; g < 8; ++g) {
+      const unsigned hw = w.hs[g >> 1];
+      const float dwg = half_bits_to_float((uint16_t)((g & 1) ? (hw >> 16) : (hw & 0xffffu)));
+      const float4 y4 = *(const float4 *)(ydp + (g * 8 + 4 * hf) * 4);
+      const float yy[4] = {y4.x, y4.y, y4.z, y4.w};
 #pragma unroll
-      for (int h = 0; h < 4; ++h) d[h] = __builtin_amdgcn_mfma_i32_32x32x32_i8(wa[h], __builtin_bit_cast(i4v, w.q[4 * g2 + h]), zero, 0, 0, 0);
-      __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-      for (int h = 0; h < 4; ++h) {
-        const int g = 4 * g2 + h;
-        const unsigned hw = g < 2 ? w.hs.x : g < 4 ? w.hs.y : g < 6 ? w.hs.z : w.hs.w;
-        const float dwg = half_bits_to_float((uint16_t)((g & 1) ? (hw >> 16) : (hw & 0xffffu)));
-        const float4 y4 = *(const float4 *)(ydp + (g * 8 + 4 * hf) * 4);
-        const float yy[4] = {y4.x, y4.y, y4.z, y4.w};
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const float p = ((float)d[h][i] * dwg) * yy[i];
-          T[i] = g == 0 ? p : T[i] + p;
-        }
+      for (int i = 0; i < 4; ++i) {
+        const float p = ((float)d[g][i] * dwg) * yy[i];
+        T[i] = g == 0 ? p : T[i] + p;
       }
-      __builtin_amdgcn_sched_barrier(0);
     }
   } else {
-    int isum[4] = {0, 0, 0, 0};
-    i16v dq[TYPE == T_Q4_K ? 4 : 1];  // Q4_K: the results of the second group of MFMAs wait here for the mins' MFMA to be issued
-    if constexpr (TYPE == T_Q4_K) {
-      // piece c: bytes 0 .. 7 = qs[32 c + 8 hf ..], 8 .. 15 = qs[32 c + 16 + 8 hf ..]: low nibbles = elements 64 c + {8 hf .., 16 + 8 hf ..} (sub-block 2 c), high = + 32 (2 c + 1)
-      // FOUR independent MFMAs per group, then their scale products (first GPU run: hipcc funnelled every MFMA of a record through one accumulator tuple -- read the
-      // four live results back, overwrite -- and a record cost a wave 0.66 us: nine exposed MFMA latencies; the scheduling barriers keep a group's MFMAs together)
-      // Schedule of a record (scheduling barriers pin it; one wave per SIMD has nobody to hide a latency behind): operands of the first four sub-blocks | their MFMAs |
-      // LDS reads + unpack of the other four and the mins' operand WHILE those run | scale products of the first four | MFMAs of the other four + the mins' MFMA (issued
-      // by the caller's code right behind) | scale products.
-      auto operands = [&](int g2, i4v (&wa)[4], i4v (&wb)[4]) __attribute__((always_inline)) {
-#pragma unroll
-        for (int h = 0; h < 2; ++h) {
-          const int c = 2 * g2 + h;
-          const v4u lo = w.q[c] & 0x0F0F0F0Fu, hi = (w.q[c] >> 4) & 0x0F0F0F0Fu;
-          const char *qa = qcol + 64 * c + 8 * hf;
-          wa[2 * h] = mk_i4(*(const v2u *)(qa), *(const v2u *)(qa + 16)); wa[2 * h + 1] = mk_i4(*(const v2u *)(qa + 32), *(const v2u *)(qa + 48));
-          wb[2 * h] = __builtin_bit_cast(i4v, lo); wb[2 * h + 1] = __builtin_bit_cast(i4v, hi);
-        }
-      };
-      auto products = [&](unsigned scw, const i16v (&d)[4]) __attribute__((always_inline)) {
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-          isum[i] += (__mul24(byte_of(scw, 0), d[0][i]) + __mul24(byte_of(scw, 1), d[1][i])) + (__mul24(byte_of(scw, 2), d[2][i]) + __mul24(byte_of(scw, 3), d[3][i]));
-      };
-      i4v wa0[4], wb0[4], wa1[4], wb1[4];
-      operands(0, wa0, wb0);
-      __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-      for (int h = 0; h < 4; ++h) dq[h] = __builtin_amdgcn_mfma_i32_32x32x32_i8(wa0[h], wb0[h], zero, 0, 0, 0);
-      __builtin_amdgcn_sched_barrier(0);
-      operands(1, wa1, wb1);  // in the shadow of the four MFMAs above
-      __builtin_amdgcn_sched_barrier(0);
-      products(w.hs.x, dq);
-      __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-      for (int h = 0; h < 4; ++h) dq[h] = __builtin_amdgcn_mfma_i32_32x32x32_i8(wa1[h], wb1[h], zero, 0, 0, 0);
-      // (their scale products follow the mins' MFMA below: its operand build runs in the shadow of these four)
-    } else if constexpr (TYPE == T_Q5_K) {
-      // piece g = sub-block g, the 5-bit values as bytes: bytes 0 .. 7 = elements 32 g + 8 hf .., 8 .. 15 = 32 g + 16 + 8 hf ..
-#pragma unroll
-      for (int g2 = 0; g2 < 2; ++g2) {
-        i16v d[4];
-        i4v wa[4];
-#pragma unroll
-        for (int h = 0; h < 4; ++h) {
-          const char *qa = qcol + 32 * (4 * g2 + h) + 8 * hf;
-          wa[h] = mk_i4(*(const v2u *)(qa), *(const v2u *)(qa + 16));
-        }
-        __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-        for (int h = 0; h < 4; ++h) d[h] = __builtin_amdgcn_mfma_i32_32x32x32_i8(wa[h], __builtin_bit_cast(i4v, w.q[4 * g2 + h]), zero, 0, 0, 0);
-        __builtin_amdgcn_sched_barrier(0);
-        const unsigned scw = g2 == 0 ? w.hs.x : w.hs.y;
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-          isum[i] += (__mul24(byte_of(scw, 0), d[0][i]) + __mul24(byte_of(scw, 1), d[1][i])) + (__mul24(byte_of(scw, 2), d[2][i]) + __mul24(byte_of(scw, 3), d[3][i]));
-        __builtin_amdgcn_sched_barrier(0);
-      }
-    } else {  // Q6_K: piece g = runs 2 g, 2 g + 1, the 6-bit values as bytes 0 .. 63 (the - 32 goes through the run sums below): one 32x32x16 MFMA per run of 16
-#pragma unroll
-      for (int g4 = 0; g4 < 4; ++g4) {  // runs 4 g4 .. 4 g4 + 3 = pieces 2 g4, 2 g4 + 1
-        i16v d[4];
-        long wa[4], wb[4];
-#pragma unroll
-        for (int h = 0; h < 4; ++h) {
-          const int r = 4 * g4 + h, g = r >> 1;
-          const v2u a8 = *(const v2u *)(qcol + 16 * r + 8 * hf);
-          wa[h] = mk_l(a8.x, a8.y);
-          wb[h] = (h & 1) == 0 ? mk_l(w.q[g].x, w.q[g].y) : mk_l(w.q[g].z, w.q[g].w);
-        }
-        __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-        for (int h = 0; h < 4; ++h) d[h] = __builtin_amdgcn_mfma_i32_32x32x16_i8(wa[h], wb[h], zero, 0, 0, 0);
-        __builtin_amdgcn_sched_barrier(0);
-        const unsigned scw = g4 == 0 ? w.hs.x : g4 == 1 ? w.hs.y : g4 == 2 ? w.hs.z : w.hs.w;
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-          isum[i] += (__mul24(sbyte_of(scw, 0), d[0][i]) + __mul24(sbyte_of(scw, 1), d[1][i])) + (__mul24(sbyte_of(scw, 2), d[2][i]) + __mul24(sbyte_of(scw, 3), d[3][i]));
-        __builtin_amdgcn_sched_barrier(0);
-      }
-    }
     // the terms over the 16 run sums of the token's superblock: K-quants with mins: M = sum_j m_j bsum_j;  Q6_K: S = sum_r sc_r bsum_r (isum -= 32 S).  One f16 MFMA:
     // A = the run sums (|.| <= 2032: exact in f16), B = the row's 6-bit mins, each twice (two runs per sub-block) / the int8 run scales; products and sums < 2^24: exact
-    const h8 bsf = *(const h8 *)(bsp + hf * 16);
     h8 wm;
     if constexpr (TYPE == T_Q6_K) {
-      const unsigned s0 = hf ? w.hs.z : w.hs.x, s1 = hf ? w.hs.w : w.hs.y;  // runs 8 hf .. 8 hf + 7
+      const unsigned m0 = hf ? w.hs.z : w.hs.x, m1 = hf ? w.hs.w : w.hs.y;  // runs 8 hf .. 8 hf + 7
 #pragma unroll
-      for (int k = 0; k < 4; ++k) { wm[k] = (_Float16)(float)sbyte_of(s0, k); wm[4 + k] = (_Float16)(float)sbyte_of(s1, k); }
+      for (int k = 0; k < 4; ++k) { wm[k] = (_Float16)(float)sbyte_of(m0, k); wm[4 + k] = (_Float16)(float)sbyte_of(m1, k); }
     } else {
       const unsigned mw = hf ? w.hs.w : w.hs.z;  // operand slot (hf, jj) <-> run 8 hf + jj -> sub-block 4 hf + jj / 2
 #pragma unroll
       for (int k = 0; k < 4; ++k) { const _Float16 mk = (_Float16)(float)byte_of(mw, k); wm[2 * k] = mk; wm[2 * k + 1] = mk; }
     }
-    const f16v zf = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-    if constexpr (TYPE == T_Q4_K) __builtin_amdgcn_sched_barrier(0);
-    const f16v M = __builtin_amdgcn_mfma_f32_32x32x16_f16(bsf, wm, zf, 0, 0, 0);
-    if constexpr (TYPE == T_Q4_K) {
-      __builtin_amdgcn_sched_barrier(0);
+    const f4v zf = {0.f, 0.f, 0.f, 0.f};
+    // products d[2 c], d[2 c + 1]; two 8-byte halves of k each.  Q6_K: piece g = runs 2 g, 2 g + 1 of 16, the 6-bit values as bytes 0 .. 63 (the - 32 goes through the run sums):
+    // bytes 0 .. 7 / 8 .. 15 = elements 8 hf .. of either.  Q4_K piece c: bytes 0 .. 7 = qs[32 c + 8 hf ..], 8 .. 15 = qs[32 c + 16 + 8 hf ..]: low nibbles = elements 64 c + {8 hf ..,
+    // 16 + 8 hf ..} (sub-block 2 c), high = sub-block 2 c + 1.  Q5_K: piece g = sub-block g, the 5-bit values as bytes in the same order.
+    constexpr int ND = TYPE == T_Q6_K ? 16 : 8;
+    i4v d[ND];
 #pragma unroll
-      for (int i = 0; i < 4; ++i)
-        isum[i] += (__mul24(byte_of(w.hs.y, 0), dq[0][i]) + __mul24(byte_of(w.hs.y, 1), dq[1][i])) + (__mul24(byte_of(w.hs.y, 2), dq[2][i]) + __mul24(byte_of(w.hs.y, 3), dq[3][i]));
+    for (int c = 0; c < ND / 2; ++c) {
+      if constexpr (TYPE == T_Q6_K) {
+        d[2 * c] = __builtin_amdgcn_mfma_i32_16x16x32_i8(mk_l(o.A[2 * c].x, o.A[2 * c].y), mk_l(w.q[c % NPC].x, w.q[c % NPC].y), zero, 0, 0, 0);
+        d[2 * c + 1] = __builtin_amdgcn_mfma_i32_16x16x32_i8(mk_l(o.A[2 * c + 1].x, o.A[2 * c + 1].y), mk_l(w.q[c % NPC].z, w.q[c % NPC].w), zero, 0, 0, 0);
+      } else {
+        const v4u lo = TYPE == T_Q4_K ? w.q[c] & 0x0F0F0F0Fu : w.q[(2 * c) % NPC], hi = TYPE == T_Q4_K ? (w.q[c] >> 4) & 0x0F0F0F0Fu : w.q[(2 * c + 1) % NPC];
+        d[2 * c] = __builtin_amdgcn_mfma_i32_16x16x64_i8(mk_i4(o.A[4 * c], o.A[4 * c + 1]), __builtin_bit_cast(i4v, lo), zero, 0, 0, 0);
+        d[2 * c + 1] = __builtin_amdgcn_mfma_i32_16x16x64_i8(mk_i4(o.A[4 * c + 2], o.A[4 * c + 3]), __builtin_bit_cast(i4v, hi), zero, 0, 0, 0);
+      }
     }
-    const float4 y4 = *(const float4 *)(ydp + 4 * hf * 4);
-    const float yy[4] = {y4.x, y4.y, y4.z, y4.w};
-    const float d = half_bits_to_float((uint16_t)(w.hd & 0xffff));
-    if constexpr (TYPE == T_Q6_K) {
+    const f4v M = __builtin_amdgcn_mfma_f32_16x16x32_f16(o.bsf, wm, zf, 0, 0, 0);
+    const float yy[4] = {o.y4.x, o.y4.y, o.y4.z, o.y4.w};
+    __builtin_amdgcn_sched_barrier(0);
+    next();
+    __builtin_amdgcn_sched_barrier(0);
+    int isum[4] = {0, 0, 0, 0};
 #pragma unroll
-      for (int i = 0; i < 4; ++i) T[i] = (d * yy[i]) * (float)(isum[i] - ((int)M[i] << 5));
-    } else {
-      const float dmin = half_bits_to_float((uint16_t)(w.hd >> 16));
+    for (int g = 0; g < ND; ++g) {
+      if constexpr (TYPE == T_Q6_K) mad4(isum, sbyte_of(w.hs[g >> 2], g & 3), d[g]);
+      else mad4(isum, byte_of(g < 4 ? w.hs.x : w.hs.y, g & 3), d[g]);
+    }
+    const float dd = half_bits_to_float((uint16_t)(w.hd & 0xffff)), dmin = half_bits_to_float((uint16_t)(w.hd >> 16));
 #pragma unroll
-      for (int i = 0; i < 4; ++i) T[i] = fmaf(d * yy[i], (float)isum[i], -((dmin * yy[i]) * M[i]));
+    for (int i = 0; i < 4; ++i) {
+      if constexpr (TYPE == T_Q6_K) T[i] = (dd * yy[i]) * (float)(isum[i] - ((int)M[i] << 5));
+      else T[i] = fmaf(dd * yy[i], (float)isum[i], -((dmin * yy[i]) * M[i]));
     }
   }
 }
 
-// tensor index and panel of (unit, segment)
-__device__ __forceinline__ void where_of(int epi, int np0, int np1, int u, int seg, int &ti, int &pn) {
-  if (epi == EPI_QKV) { ti = u >= np0 + np1 ? 2 : (u >= np0 ? 1 : 0); pn = u - (ti == 2 ? np0 + np1 : (ti == 1 ? np0 : 0)); }
-  else { ti = seg; pn = u; }
+// tensor index and group of 16 rows of (unit, segment)
+__device__ __forceinline__ void where_of(int epi, int nh0, int nh1, int u, int seg, int &ti, int &hn) {
+  if (epi == EPI_QKV) { ti = u >= nh0 + nh1 ? 2 : (u >= nh0 ? 1 : 0); hn = u - (ti == 2 ? nh0 + nh1 : (ti == 1 ? nh0 : 0)); }
+  else { ti = seg; hn = u; }
 }
-// request the next record of the wave's stream (unit cu, segment cseg, superblock ct of run p) into a ring slot and advance the cursor.  Every request is unconditional and
-// asks for the same number of loads (a cursor past its last record asks past the tensor: zeros, no traffic), so hipcc's waits come out exact (dec_core2.cuh stream()).
-template <int NPC, bool ONLY4>
-__device__ __forceinline__ void issue_rec(Rec<NPC> &slot, int &m, int &cu, int &cseg, int &ct, __amdgpu_buffer_rsrc_t rs0, __amdgpu_buffer_rsrc_t rs1, __amdgpu_buffer_rsrc_t rs2,
-                                          int ty0, int ty1, int ty2, int np0, int np1, int epi, int nseg, int units, int ntp, int p, int Cs, int S, int lane, int nn, int step, int pn0) {
-  constexpr unsigned DEAD = 0xF0000000u;
-  const bool live = cu < units && ntp > 0;
-  int ti = 0, pn = 0;
-  where_of(epi, np0, np1, live ? cu : 0, cseg, ti, pn);
-  const int type = ti == 0 ? ty0 : (ti == 1 ? ty1 : ty2);
-  const unsigned rec = live ? ((unsigned)(pn0 + pn) * (unsigned)S + (unsigned)(p * Cs + ct)) * (unsigned)rec_bytes(type) : DEAD;
-  const __amdgpu_buffer_rsrc_t rs = ti == 0 ? rs0 : (ti == 1 ? rs1 : rs2);
-  const bool small = ONLY4 || type == T_Q4_K;
-  const unsigned tail = small ? 4096u : 8192u;
+// The request cursor of a wave's stream: unit cu, segment cseg, superblock ct of run p, and what a request needs of them, kept between requests (scalars; where_of() and the products
+// per request were 60 scalar instructions in front of every record): the tensor, its type, the byte offset of record ct and of the unit's half of its rows.
+struct Cursor { int cu, cseg, ct, ti, type; unsigned rec, half; };
+__device__ __forceinline__ void open_segment(Cursor &k, int ty0, int ty1, int ty2, int nh0, int nh1, int epi, int units, int p, int Cs, int S, int pn0) {
+  int hn = 0;
+  where_of(epi, nh0, nh1, k.cu < units ? k.cu : 0, k.cseg, k.ti, hn);
+  k.type = k.ti == 0 ? ty0 : (k.ti == 1 ? ty1 : ty2);
+  k.rec = ((unsigned)(pn0 + (hn >> 1)) * (unsigned)S + (unsigned)(p * Cs)) * (unsigned)rec_bytes(k.type);
+  k.half = (unsigned)(hn & 1);
+  k.ct = 0;
+}
+// request the next two records and advance.  Lane l: row l % 16 of the unit's 16, k half l / 16 % 2, superblock ct + l / 32.  Every request is unconditional and asks for the same
+// number of loads (a cursor past its last record, and the second half of a run's odd last one, ask past the tensor: zeros, no traffic), so hipcc's waits come out exact
+// (dec_core2.cuh stream()).
+template <int NPC, int TMASK>
+__device__ __forceinline__ void issue_rec(Rec<NPC> &slot, int &m, Cursor &k, __amdgpu_buffer_rsrc_t rs0, __amdgpu_buffer_rsrc_t rs1, __amdgpu_buffer_rsrc_t rs2, int ty0, int ty1, int ty2,
+                                          int nh0, int nh1, int epi, int nseg, int units, int ntp, int p, int Cs, int S, int lane, int step, int pn0) {
+  constexpr unsigned DEAD = 0xF0000000u;  // beyond every tensor, whatever the scalar offset; + a piece's offset: no wrap
+  constexpr bool ONLY4 = TMASK == TM_Q4K, HAS4 = (TMASK & TM_Q4K) != 0;
+  const bool live = k.cu < units && ntp > 0, two = k.ct + 1 < ntp, small = ONLY4 || (HAS4 && k.type == T_Q4_K), hi = lane >= 32;
+  const unsigned rb = small ? REC_Q4K : REC_BIG, tail = small ? 4096u : 8192u;
+  const __amdgpu_buffer_rsrc_t rs = k.ti == 0 ? rs0 : (k.ti == 1 ? rs1 : rs2);
+  const bool mine = live && (two || !hi);
+  const unsigned par = hi ? rb : 0u;
+  const unsigned vq = mine ? par + (unsigned)(lane & 15) * 16u + (unsigned)((lane >> 4) & 1) * 512u : DEAD, vh = mine ? par + (unsigned)(lane & 15) * 16u : DEAD,
+                 vd = mine ? par + (unsigned)(lane & 15) * 4u : DEAD;
+  const unsigned so = live ? k.rec + k.half * 256u : 0u;
 #pragma unroll
-  for (int c = 0; c < NPC; ++c) slot.q[c] = ldb128(rs, (c < 4 || !small) ? rec + (unsigned)(c * 64 + lane) * 16u : DEAD);  // a Q4_K record in a mixed launch: pieces 4 .. 7 ask past the tensor
-  slot.hs = ldb128(rs, rec + tail + (unsigned)nn * 16u);
-  slot.hd = ldb32(rs, rec + tail + 512u + (unsigned)nn * 4u);
-  m = live ? (type | (ct << 8) | ((ct == ntp - 1 ? 1 : 0) << 24)) : -1;
+  for (int c = 0; c < NPC; ++c)  // (a Q4_K record in a mixed launch: pieces 4 .. 7 ask past the tensor)
+    slot.q[c] = __builtin_amdgcn_raw_buffer_load_b128(rs, (c < 4 || !small) ? vq + (unsigned)(c & 3) * 1024u : DEAD, so + (c < 4 ? 0u : 4096u), MRS_DEC2_LD_AUX);
+  slot.hs = __builtin_amdgcn_raw_buffer_load_b128(rs, vh, so + tail, MRS_DEC2_LD_AUX);
+  slot.hd = __builtin_amdgcn_raw_buffer_load_b32(rs, vd, so + tail + 512u - k.half * 192u, MRS_DEC2_LD_AUX);
+  m = live ? (k.type | (k.ct << 8) | ((two ? 1 : 0) << 23) | ((k.ct + 2 >= ntp ? 1 : 0) << 24)) : -1;
   if (live) {  // scalar bookkeeping only
-    if (++ct == ntp) { ct = 0; if (++cseg == nseg) { cseg = 0; cu += step; } }
+    k.ct += 2; k.rec += 2u * rb;
+    if (k.ct >= ntp) {
+      if (++k.cseg == nseg) { k.cseg = 0; k.cu += step; }
+      open_segment(k, ty0, ty1, ty2, nh0, nh1, epi, units, p, Cs, S, pn0);
+    }
   }
 }
 
-// the epilogue of a finished (unit, segment): all 256 threads, thread = (token tid / 32, row tid % 32 of the panel); called behind the barrier that publishes ex[par].
+// the epilogue of a finished (unit, segment): the first two waves, thread = (token tid / 16, row tid % 16); called behind the barrier that publishes ex[par].
 // (A plain function, not a lambda of the kernel: as a by-reference closure its stores kept every local of the kernel -- and a copy of the argument block -- in scratch memory.)
 template <bool MOE>
 __device__ __forceinline__ void finish_unit(const MmArgs &a, const float *ex, int par, int eu, int eseg, int tid, float &gsave, int nc, unsigned long long routes) {
-  const int epi = a.epi, np0 = a.m[0].npanels, np1 = a.m[1].npanels, nr0 = a.m[0].nrows, nr1 = a.m[1].nrows, nr2 = a.m[2].nrows;
-
-  const int tok = tid >> 5, row = tid & 31;
-  const float *e = ex + (size_t)par * 1024 + tok * 32 + row;
-  const float sum = ((e[0] + e[256]) + e[512]) + e[768];
-  int ti = 0, pn = 0;
-  if (epi == EPI_QKV) { ti = eu >= np0 + np1 ? 2 : (eu >= np0 ? 1 : 0); pn = eu - (ti == 2 ? np0 + np1 : (ti == 1 ? np0 : 0)); } else { ti = eseg; pn = eu; }
-  const int n = pn * 32 + row;
+  const int epi = a.epi, nh0 = a.m[0].nhalves, nh1 = a.m[1].nhalves, nr0 = a.m[0].nrows, nr1 = a.m[1].nrows, nr2 = a.m[2].nrows;
+  const int tok = tid >> 4, row = tid & 15;
+  const float *e = ex + (size_t)par * 512 + (tid & 127);
+  const float sum = ((e[0] + e[128]) + e[256]) + e[384];
+  int ti = 0, hn = 0;
+  where_of(epi, nh0, nh1, eu, eseg, ti, hn);
+  const int n = hn * 16 + row;
   const int nrows = ti == 0 ? nr0 : (ti == 1 ? nr1 : nr2);
   const bool ok = tok < nc && n < nrows;
   const int orow = MOE ? (int)((routes >> (8 * tok)) & 255u) : tok;
@@ -314,13 +294,11 @@ template <int TMASK, bool MOE>
 __device__ __forceinline__ void dec_mm_body(const MmArgs &a, char *smem) {
   constexpr bool ONLY4 = TMASK == TM_Q4K;
   constexpr int NPC = ONLY4 ? 4 : 8;
-  // Records in flight per wave.  Measured and NOT adopted on the launches of <= 256 panels (o_proj, down_proj, q / k / v: one workgroup per CU at best): rings of 8 / 4 records
-  // at one wave per SIMD (o_proj 8.1 -> 10.3 us, down_proj 16.2 -> 20.3) and eight waves per workgroup, two per run of superblocks, their terms exchanged through LDS at a
-  // barrier per step (o_proj 7.95 -> 8.63, down_proj 15.7 -> 16.2): neither more bytes in flight nor more waves per CU moves these launches -- a CU draws ~25 GB/s through
-  // this path and 128 panels occupy 128 CUs (profiles/round6_decode.md section 5).
-  constexpr int R = ONLY4 ? 3 : 2;
+  // Pairs of records in flight per wave: 2 / 3 / 4 pairs of Q4_K took 4096 x 4096 7.8 / 8.3 / 8.8 us and gate + up 17.3 / 18.6 / 19.9 -- a wave that asks for more is blocked in its
+  // requests while it should be storing the image, and the waits inside the loop are short already.
+  constexpr int R = 2;
   const int tid = tid_opaque(), lane = tid & 63, p = __builtin_amdgcn_readfirstlane(tid >> 6);  // wave p = run p of the row's superblocks
-  const int nn = lane & 31, hf = lane >> 5;
+  const int hf = (lane >> 4) & 1;  // the lane's half of k, and of the tokens of a result
   const int K = a.K, S = K / 256, Cs = (S + 3) / 4, Sp = 4 * Cs, CQ = act_cq(K), QCS = qcs_of(K);
   int nc = a.nc, unit0 = (int)blockIdx.x, ustep = (int)gridDim.x, pn0 = 0;
   unsigned long long routes = 0, rows = 0;  // MOE: output and image row of the columns, a byte each
@@ -341,7 +319,7 @@ __device__ __forceinline__ void dec_mm_body(const MmArgs &a, char *smem) {
       mask &= mask - 1;
       routes |= (unsigned long long)r << (8 * c); rows |= (unsigned long long)(r / a.route_div) << (8 * c);
     }
-    pn0 = e * a.m[0].npanels;
+    pn0 = e * (a.m[0].nhalves >> 1);
     unit0 = (int)blockIdx.x / used; ustep = ((int)gridDim.x - pick + used - 1) / used;
     if (unit0 >= a.units) return;
   }
@@ -350,6 +328,7 @@ __device__ __forceinline__ void dec_mm_body(const MmArgs &a, char *smem) {
   char *ydl = smem + (size_t)nc * QCS;                                  // Q8K: [Sp][8] f32;  Q80: [Sp][8][8] f32
   char *bsl = ydl + (a.mode == ACT_Q80 ? 0 : (size_t)Sp * 32);         // Q8K: [Sp][8][16] f16
   float *ex = (float *)(ydl + (a.mode == ACT_Q80 ? (size_t)Sp * 256 : (size_t)Sp * (32 + 256)));
+  char *zeros = (char *)(ex + 2 * 4 * 8 * 16);
   // ---- the record stream of this wave: unit cu, segment cseg, superblock ct of the run
   // (every field is read into a local first: a select between kernel-argument ADDRESSES makes hipcc copy the whole argument block to scratch memory; the launcher
   // points the unused tensors of a launch at m[0] with 0 bytes)
@@ -358,115 +337,96 @@ __device__ __forceinline__ void dec_mm_body(const MmArgs &a, char *smem) {
   const __amdgpu_buffer_rsrc_t rs0 = __builtin_amdgcn_make_buffer_rsrc((void *)wp0, (short)0, (int)wb0, 0x00020000);
   const __amdgpu_buffer_rsrc_t rs1 = __builtin_amdgcn_make_buffer_rsrc((void *)wp1, (short)0, (int)wb1, 0x00020000);
   const __amdgpu_buffer_rsrc_t rs2 = __builtin_amdgcn_make_buffer_rsrc((void *)wp2, (short)0, (int)wb2, 0x00020000);
-  const int np0 = a.m[0].npanels, np1 = a.m[1].npanels;
+  const int nh0 = a.m[0].nhalves, nh1 = a.m[1].nhalves;
   const int ty0 = a.m[0].type, ty1 = a.m[1].type, ty2 = a.m[2].type;
-  const int nr0 = a.m[0].nrows, nr1 = a.m[1].nrows, nr2 = a.m[2].nrows;
   const int epi = a.epi, nseg = a.nseg, units = a.units;
-  int cu = unit0, cseg = 0, ct = 0;
+  Cursor cur{unit0, 0, 0, 0, 0, 0u, 0u};
+  open_segment(cur, ty0, ty1, ty2, nh0, nh1, epi, units, p, Cs, S, pn0);
   Rec<NPC> ring[R];
-  int meta[R];  // type | ct << 8 | last << 24, or -1
+  int meta[R];  // type | ct << 8 | the second record exists << 23 | last << 24, or -1
   // (issue_rec / where_of are plain functions: as by-reference closures of the kernel their selects between captured variables -- which tensor's resource, type, panel
   // count -- became run-time offsets INTO the closure object, which then could not be dissolved: every local of the kernel lived in scratch memory)
   auto issue = [&](Rec<NPC> &slot, int &m) __attribute__((always_inline)) {
-    issue_rec<NPC, ONLY4>(slot, m, cu, cseg, ct, rs0, rs1, rs2, ty0, ty1, ty2, np0, np1, epi, nseg, units, ntp, p, Cs, S, lane, nn, ustep, pn0);
+    issue_rec<NPC, TMASK>(slot, m, cur, rs0, rs1, rs2, ty0, ty1, ty2, nh0, nh1, epi, nseg, units, ntp, p, Cs, S, lane, ustep, pn0);
   };
   MRS_MM_TL(0);
-  // ---- the activation image -> LDS (every workgroup).  The first batch of image requests leaves BEFORE the weight ring: loads return in order, the image comes out of
-  // the L2 in ~1 us and is stored while the weights are still on their way from HBM (behind the ring it arrived 2.5 us later: timeline of the second GPU run)
+  // ---- the activation image -> LDS (every workgroup), requested BEFORE the weight ring: it comes out of the L2 while the weights are on their way
   // column c: its group's image, its place in it, the group's size (MOE: every row an image of its own)
   auto in_grp = [&](int c) __attribute__((always_inline)) { return MOE ? 0 : c - (int)((a.gc0p >> (4 * c)) & 15u); };
   auto gn_of = [&](int c) __attribute__((always_inline)) { return MOE ? 1 : (int)((a.gnp >> (4 * c)) & 15u) + 1; };
   auto grp_at = [&](int c) __attribute__((always_inline)) { return (unsigned)act_bytes(K, MOE ? (int)((rows >> (8 * c)) & 255u) : (int)((a.gc0p >> (4 * c)) & 15u)); };
-  // Every request of a stage leaves before the first of its values is stored (batches of up to 16 loads per lane): a load -> store loop is one memory round trip per
-  // iteration (hipcc keeps them in order: both pointers are generic), 19 of them in a row at 8 columns of K = 4096 -- ~10 us in front of the first MFMA of every launch
-  // (first GPU run of this file: o_proj 9.8 us at every batch size).  Requests go through ONE buffer resource over the image(s): a piece past its column asks past the
-  // end (zeros, no branch).
+  // Quants, superblock scales and Q8_0's block scales are copied by LDS-DMA, as many requests as there are pieces of 1 KiB and no registers in between; only the run sums, which
+  // the mins' MFMA reads as f16, pass through registers, a batch of up to 8 per thread.  Everything is requested at once, the weight ring last (with image requests behind it
+  // the waits of its first records come out as full drains), and the wait before the barrier leaves exactly the ring in flight.  Requests go through ONE buffer resource over
+  // the image(s): a column that does not exist asks past the end (zeros).
+  // (Batches of 8 + 8 + 16 register loads whatever the row's length, each stored before the next was requested, had 18 of 48 requests dead at 4096 values and four round trips at
+  // 14336: start of a launch to its first record, us, 8 columns: 3.5 / 5.8 of K = 4096 / 14336.)
   {
     const unsigned img_bytes = (unsigned)act_bytes(K, MOE ? (a.nroutes + a.route_div - 1) / a.route_div : nc);
     const __amdgpu_buffer_rsrc_t ri = __builtin_amdgcn_make_buffer_rsrc((void *)a.img, (short)0, (int)img_bytes, 0x00020000);
     constexpr unsigned PAST = 0xF0000000u;
-    const int nv = 4 * CQ / 16;  // 16-byte pieces of a column
-    // quants: wave p copies columns p and p + 4; 8 pieces of each per batch
-    const int c0 = p, c1 = p + 4;
-    const unsigned s0 = grp_at(c0) + (unsigned)(in_grp(c0) * 4 * CQ), s1 = grp_at(c1 & 7) + (unsigned)(in_grp(c1 & 7) * 4 * CQ);
-    const bool h0 = c0 < nc, h1 = c1 < nc;
-    v4u r0[8], r1[8];
-    auto ld_batch = [&](int j0) __attribute__((always_inline)) {
-#pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        const int i = j0 + j * 64 + lane;
-        r0[j] = __builtin_amdgcn_raw_buffer_load_b128(ri, h0 && i < nv ? s0 + (unsigned)i * 16u : PAST, 0, 0);
-        r1[j] = __builtin_amdgcn_raw_buffer_load_b128(ri, h1 && i < nv ? s1 + (unsigned)i * 16u : PAST, 0, 0);
-      }
-    };
-    auto st_batch = [&](int j0) __attribute__((always_inline)) {
-#pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        const int i = j0 + j * 64 + lane;
-        if (h0 && i < nv) *(v4u *)(qs + (size_t)c0 * QCS + i * 16) = r0[j];
-        if (h1 && i < nv) *(v4u *)(qs + (size_t)c1 * QCS + i * 16) = r1[j];
-      }
-    };
-    // scales and run sums: item -> (superblock, column[, ...]); up to 8 items per thread and batch
-    auto col_base = [&](int c) __attribute__((always_inline)) { return grp_at(c) + (unsigned)(gn_of(c) * 4 * CQ); };  // the group's d region
     const bool q80 = a.mode == ACT_Q80;
-    const int nsc = q80 ? Sp * 64 : Sp * 32;  // Q80: block scales, image d [ncols][Sp][12] f32 (8 + pad) -> yd8 [sb][block][token];  Q8K: four run sums per item, the
-                                              // superblock scale rides along (items with r4 == 0)
-    v4u bq[8]; unsigned dv[8];
-    auto ld_sc = [&](int i0) __attribute__((always_inline)) {
-#pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        const int i = i0 + j * MT + tid;
-        if (q80) {
-          const int sb = i >> 6, g = (i >> 3) & 7, c = i & 7;
-          bq[j] = v4u{0u, 0u, 0u, 0u};
-          dv[j] = __builtin_amdgcn_raw_buffer_load_b32(ri, c < nc && i < nsc ? col_base(c) + (unsigned)((in_grp(c) * Sp + sb) * 12 + g) * 4u : PAST, 0, 0);
-        } else {
-          const int sb = i >> 5, c = (i >> 2) & 7, r4 = i & 3;
-          const bool ok = c < nc && i < nsc;
-          const unsigned db = col_base(c), cb = (unsigned)(in_grp(c) * Sp + sb);
-          bq[j] = __builtin_amdgcn_raw_buffer_load_b128(ri, ok ? db + (unsigned)gn_of(c) * (unsigned)Sp * 4u + (cb * ACT_BS + 4u * r4) * 4u : PAST, 0, 0);
-          dv[j] = __builtin_amdgcn_raw_buffer_load_b32(ri, ok && r4 == 0 ? db + cb * 4u : PAST, 0, 0);
-        }
-      }
+    const int nv = 4 * CQ / 16, npc = (nv + 63) / 64;  // 16-byte pieces of a column's quants, requests of 64 of them
+    for (int c = 0, j = p;; j += 4) {  // wave p: requests p, p + 4, ... of all columns
+      while (j >= npc) { j -= npc; ++c; }
+      if (c >= nc) break;
+      const unsigned src = grp_at(c) + (unsigned)(in_grp(c) * 4 * CQ + j * 1024);
+      if (j * 64 + lane < nv) MRS_BLDS16(ri, qs + (size_t)c * QCS + j * 1024, src + (unsigned)lane * 16u);
+    }
+    auto col_base = [&](int c) __attribute__((always_inline)) { return grp_at(c) + (unsigned)(gn_of(c) * 4 * CQ); };  // the group's d region
+    // scales, token fastest: Q8K d [ncols][Sp] -> yd [sb][8];  Q80 d [ncols][Sp][12] (8 blocks + pad) -> yd8 [sb][block][8]
+    const int nd = q80 ? Sp * 64 : Sp * 8;
+    const int tc = lane & 7;
+    const unsigned db = tc < nc ? col_base(tc) : PAST, dcol = tc < nc ? db + (unsigned)(in_grp(tc) * Sp) * (q80 ? 48u : 4u) : PAST;
+    for (int i0 = p * 64; i0 < nd; i0 += MT) {
+      const int r = (i0 + lane) >> 3;  // superblock, or superblock and block
+      if (i0 + lane < nd) MRS_BLDS4(ri, ydl + (size_t)i0 * 4, tc < nc ? dcol + (unsigned)(q80 ? (r >> 3) * 12 + (r & 7) : r) * 4u : PAST);
+    }
+    // run sums: item = (superblock, column, four of the 16)
+    const int nsc = q80 ? 0 : Sp * 32, bc = (tid >> 2) & 7, r4 = tid & 3;
+    const unsigned bcol = bc < nc ? col_base(bc) + (unsigned)gn_of(bc) * (unsigned)Sp * 4u + (unsigned)(in_grp(bc) * Sp * ACT_BS + 4 * r4) * 4u : PAST;
+    v4u bq[8];
+    auto ld_sum = [&](int i) __attribute__((always_inline)) {
+      return __builtin_amdgcn_raw_buffer_load_b128(ri, bc < nc && i < nsc ? bcol + (unsigned)(i >> 5) * (ACT_BS * 4u) : PAST, 0, 0);
     };
-    auto st_sc = [&](int i0) __attribute__((always_inline)) {
+    auto st_sums = [&](int i0) __attribute__((always_inline)) {
 #pragma unroll
       for (int j = 0; j < 8; ++j) {
         const int i = i0 + j * MT + tid;
         if (i < nsc) {
-          if (q80) ((unsigned *)ydl)[i] = dv[j];
-          else {
-            const int sb = i >> 5, c = (i >> 2) & 7, r4 = i & 3;
-            _Float16 *o = (_Float16 *)(bsl + ((size_t)sb * 8 + c) * 32 + r4 * 8);
-            o[0] = (_Float16)(float)(int)bq[j].x; o[1] = (_Float16)(float)(int)bq[j].y; o[2] = (_Float16)(float)(int)bq[j].z; o[3] = (_Float16)(float)(int)bq[j].w;
-            if (r4 == 0) ((unsigned *)ydl)[sb * 8 + c] = dv[j];
-          }
+          typedef _Float16 h4 __attribute__((ext_vector_type(4)));
+          *(h4 *)(bsl + ((size_t)(i >> 5) * 8 + bc) * 32 + r4 * 8) =
+              h4{(_Float16)(float)(int)bq[j].x, (_Float16)(float)(int)bq[j].y, (_Float16)(float)(int)bq[j].z, (_Float16)(float)(int)bq[j].w};
         }
       }
     };
-    // Order: every image batch but the last of each kind is requested and stored; the LAST quant batch and the LAST scale batch are requested, then the weight ring, then
-    // they are stored (their values come out of the L2 while the weights are on their way).  The ring must be the last thing requested in front of the streaming loop:
-    // with image requests behind it hipcc's waits inside the loop came out as vmcnt(0) / (6) / (12) for the three ring slots instead of (12) each (the third GPU run:
-    // 0.65 us per record and wave, one record in flight).
-    const int qlast = ((nv - 1) / (64 * 8)) * (64 * 8), slast = ((nsc - 1) / (MT * 8)) * (MT * 8);
-    for (int j0 = 0; j0 < qlast; j0 += 64 * 8) { ld_batch(j0); st_batch(j0); }
-    for (int i0 = 0; i0 < slast; i0 += MT * 8) { ld_sc(i0); st_sc(i0); }
-    ld_batch(qlast);
-    ld_sc(slast);
+    const int slast = nsc > 0 ? ((nsc - 1) / (MT * 8)) * (MT * 8) : 0;  // (unconditional requests, those past the row dead: a branch around one would make the waits behind it full drains)
+    for (int i0 = 0; i0 < slast; i0 += MT * 8) {
+#pragma unroll
+      for (int j = 0; j < 8; ++j) bq[j] = ld_sum(i0 + j * MT + tid);
+      MRS_WAIT_VMCNT(0);
+      st_sums(i0);
+    }
+#pragma unroll
+    for (int j = 0; j < 8; ++j) bq[j] = ld_sum(slast + j * MT + tid);
+    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int i = 0; i < R; ++i) issue(ring[i], meta[i]);  // the weight ring
+    __builtin_amdgcn_sched_barrier(0);
     MRS_MM_TL(1);
-    st_batch(qlast);
-    st_sc(slast);
+    MRS_WAIT_VMCNT(R * (NPC + 2));  // the image has landed
+    st_sums(slast);
+    if (tid < 64) ((unsigned *)zeros)[tid] = 0u;
   }
   MRS_MM_TL(2);
   __syncthreads();
   MRS_MM_TL(3);
-  // ---- per-lane constants: the token column this lane supplies as the MFMA's A row (rows >= nc repeat column 0: their results are never read)
-  const int tcol = nn < nc ? nn : 0;
-  const char *qlane = qs + (size_t)tcol * QCS + (size_t)p * CQ;
-  float acc[4] = {0.f, 0.f, 0.f, 0.f};
+  // ---- per-lane constants: what the lane supplies of the MFMAs' A (term()): token l % 8 of superblock t + l / 32 if that is its row's superblock, zeros otherwise
+  const int tcol = lane & 7, second = lane >> 5;
+  const bool alive = ((lane >> 3) & 1) == second && tcol < nc;
+  const char *qlane = alive ? qs + (size_t)tcol * QCS + (size_t)p * CQ + second * 256 + hf * (TMASK == TM_Q80 ? 16 : 8) : zeros, *blane = alive ? bsl + tcol * 32 + hf * 16 + second * 256 : zeros;
+  const int qstep = alive ? 256 : 0;
+  float acc[4] = {-0.f, -0.f, -0.f, -0.f};  // (- 0 + x is x for every x: a run begins without a special case)
   float gsave = 0.f;
   int eu = unit0, eseg = 0, par = 0;  // the (unit, segment) whose run sums are being collected
   auto finish = [&]() __attribute__((always_inline)) {
@@ -476,34 +436,48 @@ __device__ __forceinline__ void dec_mm_body(const MmArgs &a, char *smem) {
   };
   auto publish = [&](const float (&v)[4]) __attribute__((always_inline)) {  // this wave's run sums of the finished (unit, segment) -> ex[par][p][token][row]
 #pragma unroll
-    for (int i = 0; i < 4; ++i) ex[(size_t)par * 1024 + p * 256 + (4 * hf + i) * 32 + nn] = v[i];
+    for (int i = 0; i < 4; ++i) if (lane < 32) ex[(size_t)par * 512 + p * 128 + (4 * hf + i) * 16 + (lane & 15)] = v[i];
   };
   if (ntp == 0) {  // a run without superblocks contributes + 0 (rows of fewer than four superblocks): no records, the barriers and its share of the epilogues
     const float z[4] = {0.f, 0.f, 0.f, 0.f};
     while (eu < units) { publish(z); __syncthreads(); finish(); }
     return;
   }
-  auto compute = [&](const Rec<NPC> &w, int m) __attribute__((always_inline)) -> bool {
+  constexpr bool Q80 = TMASK == TM_Q80;
+  constexpr unsigned ystep = Q80 ? 256 : 32;
+  auto ops_of = [&](Ops &o, int m) __attribute__((always_inline)) {  // the operands of the record pair of meta m (one that does not exist: some pair's)
+    const int t = m < 0 ? 0 : (m >> 8) & 0x7fff;
+    read_ops<Q80>(o, qlane + t * qstep, blane + (p * Cs + t) * qstep, ydl + (size_t)(p * Cs + t + second) * ystep, hf);
+  };
+  auto compute = [&](const Rec<NPC> &w, Ops &o, int m, int m_next) __attribute__((always_inline)) -> bool {
     if (m < 0) return false;  // wave-uniform
-    const int type = m & 0xff, t = (m >> 8) & 0xffff, sb = p * Cs + t;
+    const int type = m & 0xff, t = (m >> 8) & 0x7fff;
     float T[4];
-    const char *qcol = qlane + t * 256;
-    const char *ydp = ydl + (size_t)sb * (a.mode == ACT_Q80 ? 256 : 32);
-    const char *bsp = bsl + ((size_t)sb * 8 + (tcol & 7)) * 32;
+    const char *ydp = ydl + (size_t)(p * Cs + t + second) * ystep;
+    auto next = [&]() __attribute__((always_inline)) { ops_of(o, m_next); };
     switch (type) {
-    case T_Q4_K: if constexpr ((TMASK & TM_Q4K) != 0) term<T_Q4_K, NPC>(w, sb, qcol, ydp, bsp, hf, T); break;
-    case T_Q5_K: if constexpr ((TMASK & TM_Q5K) != 0) term<T_Q5_K, NPC>(w, sb, qcol, ydp, bsp, hf, T); break;
-    case T_Q6_K: if constexpr ((TMASK & TM_Q6K) != 0) term<T_Q6_K, NPC>(w, sb, qcol, ydp, bsp, hf, T); break;
-    default: if constexpr ((TMASK & TM_Q80) != 0) term<T_Q8_0, NPC>(w, sb, qcol, ydp, bsp, hf, T); break;
+    case T_Q4_K: if constexpr ((TMASK & TM_Q4K) != 0) term<T_Q4_K, NPC>(w, o, next, ydp, hf, T); break;
+    case T_Q5_K: if constexpr ((TMASK & TM_Q5K) != 0) term<T_Q5_K, NPC>(w, o, next, ydp, hf, T); break;
+    case T_Q6_K: if constexpr ((TMASK & TM_Q6K) != 0) term<T_Q6_K, NPC>(w, o, next, ydp, hf, T); break;
+    default: if constexpr ((TMASK & TM_Q80) != 0) term<T_Q8_0, NPC>(w, o, next, ydp, hf, T); break;
     }
 #pragma unroll
-    for (int i = 0; i < 4; ++i) acc[i] = t == 0 ? T[i] : acc[i] + T[i];
+    for (int i = 0; i < 4; ++i) acc[i] += T[i];  // lanes 0 .. 31: T of t
+    if ((m >> 23) & 1) {  // ... then of t + 1, from lanes 32 .. 63: the run's order
+      MRS_KEEP_BRANCH();
+#pragma unroll
+      for (int i = 0; i < 4; ++i) acc[i] += __uint_as_float(__builtin_amdgcn_permlane32_swap(__float_as_uint(T[i]), __float_as_uint(T[i]), false, false)[1]);
+    }
     return (m >> 24) != 0;  // the run of this (unit, segment) is complete
   };
+  Ops ops;
+  ops_of(ops, meta[0]);
   while (eu < units) {
 #pragma unroll
     for (int i = 0; i < R; ++i) {
-      if (compute(ring[i], meta[i])) { MRS_MM_TL(4); publish(acc); __syncthreads(); MRS_MM_TL(5); finish(); MRS_MM_TL(6); }
+      if (compute(ring[i], ops, meta[i], meta[(i + 1) % R])) {
+        MRS_MM_TL(4); publish(acc); acc[0] = acc[1] = acc[2] = acc[3] = -0.f; __syncthreads(); MRS_MM_TL(5); finish(); MRS_MM_TL(6);
+      }
       issue(ring[i], meta[i]);
     }
   }
@@ -514,15 +488,14 @@ __device__ __forceinline__ void dec_mm_body(const MmArgs &a, char *smem) {
 #else
 #define MRS_MM_WAVES_PER_EU(lo, hi)  // (the kernel sources also compile for the host: test infrastructure)
 #endif
-// The kernels: Q4_K alone (4.6 KB records, three in flight) fits two workgroups per CU in 256 registers; the 8.6 KB records of the other formats (two in flight + four
-// accumulator tuples) take one workgroup's worth -- asking for two spilled 26 registers into the streaming loop.  Without a cap on waves per SIMD hipcc schedules for
-// three and funnels every MFMA of a record through one accumulator tuple (exposed MFMA latency x 9 per record).
+// The kernels: two workgroups per CU where LDS admits them (256 registers).  Three gained nothing (gate + up 17.3 -> 18.2: more images to copy).  The two mixes with Q5_K, three format
+// bodies in one loop, spill at 256 and take one.
 __global__ void __launch_bounds__(MT) MRS_MM_WAVES_PER_EU(2, 2) dec_mm_kernel_q4k(const MmArgs a) {
   extern __shared__ __attribute__((aligned(16))) char smem[];
   dec_mm_body<TM_Q4K, false>(a, smem);
 }
 template <int TMASK>
-__global__ void __launch_bounds__(MT) MRS_MM_WAVES_PER_EU(1, 2) dec_mm_kernel(const MmArgs a) {
+__global__ void __launch_bounds__(MT) MRS_MM_WAVES_PER_EU((TMASK & TM_Q5K) != 0 && TMASK != TM_Q5K ? 1 : 2, 2) dec_mm_kernel(const MmArgs a) {
   extern __shared__ __attribute__((aligned(16))) char smem[];
   dec_mm_body<TMASK, false>(a, smem);
 }
@@ -532,7 +505,7 @@ __global__ void __launch_bounds__(MT) MRS_MM_WAVES_PER_EU(2, 2) dec_mm_experts_k
   dec_mm_body<TM_Q4K, true>(a, smem);
 }
 template <int TMASK>
-__global__ void __launch_bounds__(MT) MRS_MM_WAVES_PER_EU(1, 2) dec_mm_experts_kernel(const MmArgs a) {
+__global__ void __launch_bounds__(MT) MRS_MM_WAVES_PER_EU(2, 2) dec_mm_experts_kernel(const MmArgs a) {
   extern __shared__ __attribute__((aligned(16))) char smem[];
   dec_mm_body<TMASK, true>(a, smem);
 }
@@ -548,13 +521,12 @@ static int launch(const MmArgs &a0, hipStream_t s) {
     if (act_mode_for(a.m[i].type) != a.mode) return -1;
     tmask |= tmask_of(a.m[i].type);
   }
-  for (int i = nt; i < 3; ++i) { a.m[i] = a.m[0]; a.m[i].bytes = 0; a.m[i].npanels = 0; }
+  for (int i = nt; i < 3; ++i) { a.m[i] = a.m[0]; a.m[i].bytes = 0; a.m[i].nhalves = 0; }
   if (a.K <= 0 || a.K % 256 || a.nc < 1 || a.nc > 8 || !a.img || a.units < 1) return -1;
   const size_t lds = (lds_bytes(a.K, a.nc, a.mode) + 15) & ~(size_t)15;
-  if (lds > (size_t)158 * 1024) return -2;
+  if (lds > (size_t)LDS_MAX) return -2;
   static const int wg_per_cu = [] { const char *e = getenv("MRS_DEC_MM_WG_PER_CU"); return e ? std::max(1, atoi(e)) : 2; }();
-  const int fit = (tmask == TM_Q4K || tmask == TM_Q5K || tmask == TM_Q80) ? 2 : 1;  // workgroups per CU the kernel's registers admit (see the kernels above)
-  const int cap = 256 * std::min<int>(std::min(wg_per_cu, fit), std::max<size_t>(1, ((size_t)160 * 1024) / lds));
+  const int cap = 256 * std::min<int>(wg_per_cu, std::max<size_t>(1, ((size_t)160 * 1024) / lds));
   const int grid = std::min(a.units * (a.ids ? std::min(a.experts, a.nroutes) : 1), cap);
   auto go = [&](auto kern) {
     ++g_mm_launches;
@@ -588,7 +560,7 @@ static bool set_tensor(MmTensor &t, const void *qi, int type, long long n, long 
   if (!qi || !mm_type(type) || n <= 0 || k <= 0 || k % 256) return false;
   const size_t bytes = (size_t)((n + 31) / 32) * (size_t)(k / 256) * rec_bytes(type);
   if (bytes >= 0xF0000000ull) return false;
-  t.w = (const uint8_t *)qi; t.bytes = (unsigned)bytes; t.type = type; t.npanels = (int)((n + 31) / 32); t.nrows = (int)n;
+  t.w = (const uint8_t *)qi; t.bytes = (unsigned)bytes; t.type = type; t.nhalves = 2 * (int)((n + 31) / 32); t.nrows = (int)n;
   return true;
 }
 static bool base(MmArgs &a, const void *x_img, int k, int b, int type0) {
@@ -611,13 +583,13 @@ extern "C" void mrs_dec_mm_timeline(void *buf) { g_mm_tl = (unsigned long long *
 // Can the batched matrix-core route take a launch of this weight type / reduction length / column count?  (K-quants and Q8_0; the LDS budget bounds k x b)
 extern "C" int mrs_dec_mm_supported(int type, int k, int b) {
   if (!mm_type(type) || k <= 0 || k % 256 || b < 1 || b > 8) return 0;
-  return lds_bytes(k, b, dec2::act_mode_for(type)) + 15 <= (size_t)158 * 1024 ? 1 : 0;
+  return lds_bytes(k, b, dec2::act_mode_for(type)) + 15 <= (size_t)LDS_MAX ? 1 : 0;
 }
 // out [b][ld_out] = W . x (mode 0) or out * resid_scale + W . x (mode 1); qi = the MFMA-order copy of W (mrs_gemm_qi_repack), x_img = mrs_dec_act_image(.., type, b, ..)
 extern "C" int mrs_dec_mm_proj(const void *qi, int type, int n, int k, const void *x_img, float *out, int ld_out, int mode, float resid_scale, int b, void *stream) {
   MmArgs a{};
   if (!out || !set_tensor(a.m[0], qi, type, n, k) || !base(a, x_img, k, b, type)) return -1;
-  a.epi = mode ? EPI_RESID : EPI_STORE; a.nseg = 1; a.units = a.m[0].npanels; a.out = out; a.out_stride = ld_out; a.resid_scale = resid_scale;
+  a.epi = mode ? EPI_RESID : EPI_STORE; a.nseg = 1; a.units = a.m[0].nhalves; a.out = out; a.out_stride = ld_out; a.resid_scale = resid_scale;
   return launch(a, (hipStream_t)stream);
 }
 // act_out [b][ld_out] = act(W_g . x) * (W_u . x)
@@ -625,7 +597,7 @@ extern "C" int mrs_dec_mm_gate_up(const void *qi_gate, const void *qi_up, int ty
                                   void *stream) {
   MmArgs a{};
   if (!act_out || !set_tensor(a.m[0], qi_gate, type, n, k) || !set_tensor(a.m[1], qi_up, type, n, k) || !base(a, x_img, k, b, type)) return -1;
-  a.epi = EPI_GLU; a.nseg = 2; a.units = a.m[0].npanels; a.out = act_out; a.out_stride = ld_out; a.activation = activation;
+  a.epi = EPI_GLU; a.nseg = 2; a.units = a.m[0].nhalves; a.out = act_out; a.out_stride = ld_out; a.activation = activation;
   return launch(a, (hipStream_t)stream);
 }
 // q / k / v projections + interleaved RoPE + paged-cache write (mrs_dec_qkv_img's contract, neox = 0 only: a rotate-half pair spans two panels)
@@ -637,7 +609,7 @@ extern "C" int mrs_dec_mm_qkv(const void *qi_q, int type_q, int nq, const void *
   if (!set_tensor(a.m[0], qi_q, type_q, nq, k) || !set_tensor(a.m[1], qi_k, type_k, nk, k) || !set_tensor(a.m[2], qi_v, type_v, nv, k) || !base(a, x_img, k, b, type_q)) return -1;
   if (((nq | nk | nv | head_dim) & 1) || (kv_dtype != 0 && kv_dtype != 1)) return -1;
   auto lg2 = [](int v) { int s = 0; while ((1 << s) < v) ++s; return (1 << s) == v ? s : -1; };
-  a.epi = EPI_QKV; a.nseg = 1; a.units = a.m[0].npanels + a.m[1].npanels + a.m[2].npanels;
+  a.epi = EPI_QKV; a.nseg = 1; a.units = a.m[0].nhalves + a.m[1].nhalves + a.m[2].nhalves;
   a.q_out = q_out; a.k_cache = k_cache; a.v_cache = v_cache; a.slot_mapping = slot_mapping; a.positions = positions; a.cos_t = cos_t; a.sin_t = sin_t;
   a.head_dim = head_dim; a.rot_pairs = rot_pairs; a.num_kv_heads = num_kv_heads; a.block_size = block_size; a.cache_x = 8; a.kv_f16 = kv_dtype == 0;
   a.hd_shift = lg2(head_dim); a.bs_shift = lg2(block_size); a.x_shift = lg2(a.cache_x);
@@ -654,9 +626,9 @@ static int experts_launch(MmArgs &a, const void *const *qi, int type, int n, int
   if (!ids || !out || !mrs_dec_mm_experts_supported(type, n, k, experts, b, top_k) || !base(a, x_img, k, b, type)) return -1;
   for (int i = 0; i < a.nseg; ++i) {
     if (!set_tensor(a.m[i], qi[i], type, (long long)experts * n, k)) return -1;
-    a.m[i].npanels = n / 32; a.m[i].nrows = n;
+    a.m[i].nhalves = n / 16; a.m[i].nrows = n;
   }
-  a.units = n / 32; a.out = out; a.out_stride = ld_out; a.ids = ids; a.nroutes = b * top_k; a.experts = experts; a.route_div = route_div;
+  a.units = n / 16; a.out = out; a.out_stride = ld_out; a.ids = ids; a.nroutes = b * top_k; a.experts = experts; a.route_div = route_div;
   return launch(a, (hipStream_t)stream);
 }
 // act_out [b * top_k][ld_out] = act(W_g[e] . x) * (W_u[e] . x), e = ids[route], x = image row route / top_k of x_img (mrs_dec_act_image_rows of the b tokens)

@@ -345,6 +345,52 @@ static hiphost_i32x16 mfma_32x32x16_i8(long a, long b, hiphost_i32x16 c) {
 }
 }  // namespace hiphost
 #define __builtin_amdgcn_mfma_i32_32x32x16_i8(A, B, C, CBSZ, ABID, BLGP) hiphost::mfma_32x32x16_i8((A), (B), (C))
+// The 16-row shapes: lane l holds A[l % 16][K / 4 (l / 16) + j] and B[K / 4 (l / 16) + j][l % 16] and receives rows 4 (l / 16) + i of column l % 16.  v_mfma_i32_16x16x64_i8 (16 bytes
+// per lane), v_mfma_i32_16x16x32_i8 (8 bytes), v_mfma_f32_16x16x32_f16 (8 values; as the 32-row form: exact for the small integers it is fed)
+namespace hiphost {
+template <int KL> static hiphost_i32x4 mfma_16x16_i8(const void *a, const void *b, hiphost_i32x4 c) {
+  const int tid = linear_tid(), w = tid / WAVE, lane = tid & (WAVE - 1), base = w * WAVE;
+  memcpy(mfma_a8[tid], a, KL);
+  memcpy(mfma_b8[tid], b, KL);
+  wave_barrier(w, 0);
+  const int col = lane & 15, g = lane >> 4;
+  hiphost_i32x4 d = c;
+  for (int i = 0; i < 4; ++i) {
+    int acc = 0;
+    for (int k = 0; k < 4 * KL; ++k) acc += (int)mfma_a8[base + 4 * g + i + 16 * (k / KL)][k % KL] * (int)mfma_b8[base + col + 16 * (k / KL)][k % KL];
+    d[i] = c[i] + acc;
+  }
+  wave_barrier(w, 0);
+  return d;
+}
+static hiphost_i32x4 mfma_16x16x64_i8(hiphost_i32x4 a, hiphost_i32x4 b, hiphost_i32x4 c) { return mfma_16x16_i8<16>(&a, &b, c); }
+static hiphost_i32x4 mfma_16x16x32_i8(long a, long b, hiphost_i32x4 c) { return mfma_16x16_i8<8>(&a, &b, c); }
+static hiphost_f32x4 mfma_16x16x32_f16(hiphost_f16x8 a, hiphost_f16x8 b, hiphost_f32x4 c) {
+  const int tid = linear_tid(), w = tid / WAVE, lane = tid & (WAVE - 1), base = w * WAVE;
+  for (int j = 0; j < 8; ++j) { mfma_ah[tid][j] = a[j]; mfma_bh[tid][j] = b[j]; }
+  wave_barrier(w, 0);
+  const int col = lane & 15, g = lane >> 4;
+  hiphost_f32x4 d = c;
+  for (int i = 0; i < 4; ++i) {
+    float acc = c[i];
+    for (int k = 0; k < 32; ++k) acc += (float)mfma_ah[base + 4 * g + i + 16 * (k / 8)][k % 8] * (float)mfma_bh[base + col + 16 * (k / 8)][k % 8];
+    d[i] = acc;
+  }
+  wave_barrier(w, 0);
+  return d;
+}
+// v_permlane32_swap_b32: the upper half of the first operand against the lower half of the second
+typedef unsigned hiphost_u32x2 __attribute__((ext_vector_type(2)));
+static hiphost_u32x2 permlane32_swap(unsigned a, unsigned b) {
+  const int lane = linear_tid() & (WAVE - 1);
+  const unsigned ao = exchange(a, lane ^ 32), bo = exchange(b, lane ^ 32);
+  return lane >= 32 ? hiphost_u32x2{bo, b} : hiphost_u32x2{a, ao};
+}
+}  // namespace hiphost
+#define __builtin_amdgcn_mfma_i32_16x16x64_i8(A, B, C, CBSZ, ABID, BLGP) hiphost::mfma_16x16x64_i8((A), (B), (C))
+#define __builtin_amdgcn_mfma_i32_16x16x32_i8(A, B, C, CBSZ, ABID, BLGP) hiphost::mfma_16x16x32_i8((A), (B), (C))
+#define __builtin_amdgcn_mfma_f32_16x16x32_f16(A, B, C, CBSZ, ABID, BLGP) hiphost::mfma_16x16x32_f16((A), (B), (C))
+#define __builtin_amdgcn_permlane32_swap(A, B, FI, BC) hiphost::permlane32_swap((A), (B))
 // buffer resource: base + byte range; raw_buffer_load returns zeros out of range (as the hardware's bounds check does)
 struct __amdgpu_buffer_rsrc_t { const char *base; unsigned bytes; };
 static inline __amdgpu_buffer_rsrc_t hiphost_make_rsrc(void *p, int bytes) { return __amdgpu_buffer_rsrc_t{(const char *)p, (unsigned)bytes}; }
@@ -426,6 +472,9 @@ static inline void hiphost_buffer_load_lds(__amdgpu_buffer_rsrc_t r, char *dst, 
 #define MRS_LDS_BASE(P) 0u
 #define MRS_LDS_FRAG(TYPE, P, ADDR, OFF) (*(const TYPE *)((P) + (ADDR) + (OFF)))
 #define MRS_WAIT_VMCNT0() ((void)0)                                     /* product code: s_waitcnt vmcnt(0) */
+#define MRS_WAIT_VMCNT(N) ((void)0)                                     /* product code: s_waitcnt vmcnt(N) */
+#define MRS_OPAQUE(V) ((void)0)                                         /* product code: an empty asm that hides the value from the optimizer */
+#define MRS_KEEP_BRANCH() ((void)0)
 #define __builtin_amdgcn_fence(ORDER, SCOPE) ((void)0)                  /* one workgroup runs at a time: nothing to order */
 #define __builtin_amdgcn_s_sleep(N) ((void)0)
 #define __HIP_MEMORY_SCOPE_AGENT 4

@@ -110,6 +110,20 @@ def test_mm_proj_host_emulation(oracle, tname, n, k, b, norm):
     check_mm_proj(oracle, HostBackend(), tname, n, k, b, norm)  # (n = 33 / 40 / 16: a ragged last panel; k = 768: runs of one superblock, the fourth empty; k = 256: three empty runs)
 
 
+# runs of superblocks taken two at a time (an odd run's last step has one: 1; 3; 4, 4, 4, 1), units of 16 rows (n = 48 ends inside a panel), columns that do not exist (b < 8)
+@pytest.mark.parametrize("tname", ["Q4_K", "Q5_K", "Q6_K", "Q8_0"])
+@pytest.mark.parametrize("n,k,b", [(48, 768, 1), (16, 2816, 6), (80, 3328, 8)])
+def test_mm_odd_runs_and_half_panels_host_emulation(oracle, tname, n, k, b):
+    check_mm_proj(oracle, HostBackend(), tname, n, k, b, True)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("tname", ["Q4_K", "Q5_K", "Q6_K", "Q8_0"])
+@pytest.mark.parametrize("n,k,b", [(48, 768, 1), (16, 2816, 6), (80, 3328, 8), (4112, 1280, 2)])
+def test_mm_odd_runs_and_half_panels_gpu(oracle, dev, tname, n, k, b):
+    check_mm_proj(oracle, GpuBackend(dev), tname, n, k, b, True)
+
+
 def test_mm_store_gate_up_qkv_host_emulation(oracle):
     be = HostBackend()
     check_mm_proj(oracle, be, "Q6_K", 96, 512, 2, True, mode=0)
