@@ -1446,7 +1446,7 @@ __global__ void __launch_bounds__(64 * PM_NW, 2) prefill_attn_mfma_kernel(const 
 // What bounds both: the f32 matrix instructions (64 cycles each, 64 + 64 of them per head, 32 queries and 32 tokens) take the SIMD's vector ALU with them -- measured, the times of
 // matrix and vector instructions add up (unlike the f16 ones'), so a vector instruction saved is time saved: halves of a dword by one permute, no masks where every query sees the
 // whole block, the exponential in 21 instructions, one-block splits without the running correction.  The probabilities cost 4 KiB per 128 matrix instructions, written and read once.
-// Attention of 32 heads, us per layer, one kernel / these two: 37 tokens at 300 48 / 22, 512 tokens 72 / 44, 1999 tokens 740 / 407 (floor of the matrix instructions alone 215).
+// Attention of 32 heads, us per layer, one kernel / these two: 37 tokens at 300 48 / 13.8, 512 tokens 72 / 41, 1999 tokens 740 / 440 (floor of the matrix instructions alone 215).
 // A slot of the workspace, per (head, tile of 32 queries, 32-token block): the probabilities as the B operand of the P . V instructions, block sums, alphas, running maxima.
 #ifndef MRS_KEEP16
 #define MRS_KEEP16(x) asm volatile("" : "+v"(x[0]), "+v"(x[1]), "+v"(x[2]), "+v"(x[3]), "+v"(x[4]), "+v"(x[5]), "+v"(x[6]), "+v"(x[7]), "+v"(x[8]), "+v"(x[9]), "+v"(x[10]), "+v"(x[11]), "+v"(x[12]), "+v"(x[13]), "+v"(x[14]), "+v"(x[15]))
@@ -1586,9 +1586,15 @@ __global__ void __launch_bounds__(256, 3) prefill_scores_kernel(const dec::AttnA
     m_run = mn;
   }
 }
-template <class CT, bool ONE>
+// G groups of waves: group g takes splits g, g + G, ..; the first group adds the others' products (LDS, two buffers, one barrier per G splits) to its own in the splits' order.
+// A workgroup is four waves whatever G is -- 32 x 4 / G dims, grid z = G of them --, so that G times as many SIMDs share a (head, tile) pair: few pairs leave the chip to one long
+// chain each (37 tokens at 300: 64 workgroups, 11 blocks one after another).  Groups inside one workgroup of 4 G waves, on the same four SIMDs, gained nothing (19.7 us against 19.4).
+constexpr int pv_lds(int G) { return G > 1 ? 2 * (G - 1) * (4 / G) * 64 * 17 * 4 : 0; }  // [buffer][group - 1][wave of the group]: products [4][64 lanes][4], l w [64]
+template <class CT, bool ONE, int G>
 __global__ void __launch_bounds__(256, 4) prefill_values_kernel(const dec::AttnArgs a, const PrefillWs w) {
-  const int tid = tid_opaque(), lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  extern __shared__ __attribute__((aligned(16))) char pv_s[];
+  constexpr int WG_ = 4 / G;  // waves of a group
+  const int tid = tid_opaque(), lane = tid & 63, wave_all = __builtin_amdgcn_readfirstlane(tid >> 6), wave = (int)blockIdx.z * WG_ + wave_all % WG_, grp = wave_all / WG_;
   const int j = lane & 31, hf = lane >> 5;
   // longest contexts first, every other 256 workgroups backwards: where all workgroups are resident at once (1024 fit) every CU gets long and short ones
   const int id = (int)(blockIdx.y * gridDim.x + blockIdx.x), q256 = id >> 8;
@@ -1611,63 +1617,106 @@ __global__ void __launch_bounds__(256, 4) prefill_values_kernel(const dec::AttnA
     r.ps = meta(b, 0); r.mn = meta(b, 2);
     if (!ONE) r.alpha = meta(b, 1);
   };
+  const int nsp = ONE ? nblk : (nblk + bpw - 1) / bpw, rounds = (nsp + G - 1) / G;
+  // the wave's blocks: those of splits grp, grp + G, .. one after another; past the last one: the last
+  int b = ONE ? grp : grp * bpw, in_split = 0, b1 = b, in1 = 0;
+  auto advance = [&](int &bb, int &in) { if (ONE || ++in == bpw) { in = 0; bb += ONE ? G : 1 + (G - 1) * bpw; } else ++bb; };
+  advance(b1, in1);
+  int b2 = b1, in2 = in1;
+  advance(b2, in2);
   Blk r0, r1;
-  unsigned id0 = id_of(0), id1 = id_of(1);  // the table is read two blocks ahead
-  load(0, id0, r0);
-  id0 = id_of(2);
-  float M = -FLT_MAX;  // over the splits: their last blocks' running maxima
-  for (int b = min((hf + 1) * bpw, nblk) - 1;; b = min(b + 2 * bpw, nblk - 1)) {
-    M = fmaxf(M, meta(b, 2));
-    if (b + 1 >= nblk) break;
+  unsigned id0 = id_of(b), id1 = id_of(b1);  // the table is read two blocks ahead
+  load(min(b, nblk - 1), id0, r0);
+  id0 = id_of(b2);
+  float M = -FLT_MAX;  // over the splits: their last blocks' running maxima, eight requests at a time (one by one they are a memory latency each)
+  for (int s0 = hf; s0 < nsp; s0 += 16) {
+    float m8[8];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) m8[u] = meta(ONE ? min(s0 + 2 * u, nblk - 1) : min((s0 + 2 * u + 1) * bpw, nblk) - 1, 2);
+#pragma unroll
+    for (int u = 0; u < 8; ++u) M = fmaxf(M, m8[u]);
   }
   M = fmaxf(M, __shfl_xor(M, 32, 64));
   f16v acc, o;
 #pragma unroll
   for (int v = 0; v < 16; ++v) { acc[v] = 0.f; o[v] = 0.f; }
   float s_all = 0.f, l_run = 0.f;
-  int in_split = 0;
-  auto step = [&](int b, Blk &r) {
-    if (b + 1 == nblk) {  // slots past the tile's longest context may hold anything (their p are 0)
+  float *const lds = (float *)pv_s + ((grp > 0 ? grp - 1 : 0) * WG_ + wave_all % WG_) * 64 * 17;  // this wave's products (the first group: those of group 1)
+  constexpr int LBUF = (G - 1) * WG_ * 64 * 17;
+  auto step = [&](Blk &r, int rd) {
+    const bool have = b < nblk;  // (uniform)
+    if (have) {
+      if (b + 1 == nblk) {  // slots past the tile's longest context may hold anything (their p are 0)
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+          unsigned *vw = (unsigned *)&r.v[c];
+#pragma unroll
+          for (int u = 0; u < 4; ++u) vw[u] = b * 32 + 2 * (4 * c + u) + hf < ctx_max ? vw[u] : 0u;
+        }
+      }
+      if (ONE || in_split == 0) {
+#pragma unroll
+        for (int v = 0; v < 16; ++v) o[v] = 0.f;
+        l_run = r.ps;
+      } else {
+#pragma unroll
+        for (int v = 0; v < 16; ++v) o[v] = o[v] * r.alpha;
+        l_run = l_run * r.alpha + r.ps;
+      }
 #pragma unroll
       for (int c = 0; c < 4; ++c) {
-        unsigned *vw = (unsigned *)&r.v[c];
+        const unsigned w4[4] = {r.v[c].x, r.v[c].y, r.v[c].z, r.v[c].w};
+        const float pp[4] = {r.p[c].x, r.p[c].y, r.p[c].z, r.p[c].w};
 #pragma unroll
-        for (int u = 0; u < 4; ++u) vw[u] = b * 32 + 2 * (4 * c + u) + hf < ctx_max ? vw[u] : 0u;
+        for (int u = 0; u < 4; ++u) o = __builtin_amdgcn_mfma_f32_32x32x2f32(cvt16_half<CT>(w4[u], hf), pp[u], o, 0, 0, 0);
+      }
+      if (ONE || in_split + 1 == bpw || b + 1 == nblk) {  // attn_merge_core: s += l_j w_j;  acc += o_j w_j  (multiply and add separate)
+        const float wj = fast_exp_ref_neg(r.mn - M), lw = l_run * wj;
+        if (G == 1 || grp == 0) {
+          s_all = s_all + lw;
+#pragma unroll
+          for (int v = 0; v < 16; ++v) { const float t0 = o[v] * wj; acc[v] = acc[v] + t0; }
+        } else {
+          float *const t = lds + (rd & 1) * LBUF;
+#pragma unroll
+          for (int q = 0; q < 4; ++q) *(float4 *)(t + (q * 64 + lane) * 4) = make_float4(o[4 * q] * wj, o[4 * q + 1] * wj, o[4 * q + 2] * wj, o[4 * q + 3] * wj);
+          t[1024 + lane] = lw;
+        }
       }
     }
-    if (ONE || in_split == 0) {
+    if (G > 1 && (ONE || in_split + 1 == bpw)) {  // the round's splits are there (a buffer is written again behind the next round's barrier, in front of which its reader has passed)
+      __syncthreads();
+      if (grp == 0) {
+        const int n = min(G, nsp - rd * G);
+#pragma unroll 1
+        for (int g = 1; g < n; ++g) {
+          const float *t = lds + (rd & 1) * LBUF + (g - 1) * WG_ * 64 * 17;
+          s_all = s_all + t[1024 + lane];
 #pragma unroll
-      for (int v = 0; v < 16; ++v) o[v] = 0.f;
-      l_run = r.ps;
-    } else {
-#pragma unroll
-      for (int v = 0; v < 16; ++v) o[v] = o[v] * r.alpha;
-      l_run = l_run * r.alpha + r.ps;
+          for (int q = 0; q < 4; ++q) {
+            const float4 t4 = *(const float4 *)(t + (q * 64 + lane) * 4);
+            acc[4 * q] = acc[4 * q] + t4.x; acc[4 * q + 1] = acc[4 * q + 1] + t4.y; acc[4 * q + 2] = acc[4 * q + 2] + t4.z; acc[4 * q + 3] = acc[4 * q + 3] + t4.w;
+          }
+        }
+      }
     }
-#pragma unroll
-    for (int c = 0; c < 4; ++c) {
-      const unsigned w4[4] = {r.v[c].x, r.v[c].y, r.v[c].z, r.v[c].w};
-      const float pp[4] = {r.p[c].x, r.p[c].y, r.p[c].z, r.p[c].w};
-#pragma unroll
-      for (int u = 0; u < 4; ++u) o = __builtin_amdgcn_mfma_f32_32x32x2f32(cvt16_half<CT>(w4[u], hf), pp[u], o, 0, 0, 0);
-    }
-    if (ONE || ++in_split == bpw || b + 1 == nblk) {  // attn_merge_core: s += l_j w_j;  acc += o_j w_j  (multiply and add separate)
-      const float wj = fast_exp_ref_neg(r.mn - M), lw = l_run * wj;
-      s_all = s_all + lw;
-#pragma unroll
-      for (int v = 0; v < 16; ++v) { const float t0 = o[v] * wj; acc[v] = acc[v] + t0; }
-      in_split = 0;
-    }
+    b = b1; in_split = in1; b1 = b2; in1 = in2;
+    advance(b2, in2);
   };
-  for (int b = 0; b < nblk; b += 2) {
-    load(min(b + 1, nblk - 1), id1, r1);
-    id1 = id_of(b + 3);
-    step(b, r0);
-    if (b + 1 >= nblk) break;
-    load(min(b + 2, nblk - 1), id0, r0);
-    id0 = id_of(b + 4);
-    step(b + 1, r1);
+  auto third = [&]() { int b3 = b2, in3 = in2; advance(b3, in3); return b3; };
+  const int steps = ONE ? rounds : rounds * bpw;  // of every wave: the barriers are met by all
+  for (int k = 0, rd = 0, in = 0; k < steps; k += 2) {
+    load(min(b1, nblk - 1), id1, r1);
+    id1 = id_of(third());
+    step(r0, rd);
+    if (ONE || ++in == bpw) { in = 0; ++rd; }
+    if (k + 1 >= steps) break;
+    load(min(b1, nblk - 1), id0, r0);
+    id0 = id_of(third());
+    step(r1, rd);
+    if (ONE || ++in == bpw) { in = 0; ++rd; }
   }
+  if (grp > 0) return;
   if (tile * 32 + j >= T) return;
   const float inv = 1.0f / s_all;
   float *og = a.out + ((size_t)(tile * 32 + j) * a.num_heads + head) * 128 + 32 * wave;
@@ -1733,14 +1782,25 @@ extern "C" int mrs_prefill_attention_exact_ws(const float *q, const void *k_cach
           // splits per wave: more where there are waves enough without (the queries are read once for all, a wave's next keys arrive under its instructions), few enough
           // that the last round of workgroups stays short.  Scores, us, of 1 / 2 / 4 / 8 per wave: 512 tokens - 26.8 / 24.8, 1999 tokens (16 heads) - / 113.2 / 113.3 / 120.5
           while (w.ups < 4 && (size_t)w.heads * nt * nb > (size_t)w.ups * w.ups * 4096) w.ups *= 2;
-          const dim3 gs(w.heads, nt, (splits + 4 * w.ups - 1) / (4 * w.ups)), gv(w.heads, nt);
-          auto go = [&](auto scores, auto values) {
-            hipLaunchKernelGGL(scores, gs, dim3(256), 0, (hipStream_t)stream, a, w);
-            hipLaunchKernelGGL(values, gv, dim3(256), 0, (hipStream_t)stream, a, w);
-          };
+          const dim3 gs(w.heads, nt, (splits + 4 * w.ups - 1) / (4 * w.ups));
           using namespace mrs::qi;
-          if (kv_dtype == 1) a.bpw == 1 ? go(prefill_scores_kernel<mrs::bf16_t, true>, prefill_values_kernel<mrs::bf16_t, true>) : go(prefill_scores_kernel<mrs::bf16_t, false>, prefill_values_kernel<mrs::bf16_t, false>);
-          else a.bpw == 1 ? go(prefill_scores_kernel<mrs::f16_t, true>, prefill_values_kernel<mrs::f16_t, true>) : go(prefill_scores_kernel<mrs::f16_t, false>, prefill_values_kernel<mrs::f16_t, false>);
+          // groups of splits: as many as leave a CU per workgroup.  Scores and values of 32 heads, us, 1 / 2 / 4 groups: 64 pairs, 37 tokens at 300 19.0 / 16.4 / 13.8, 33 at 1900
+          // 69 / 53 / 41, 37 at 3000 107 / 77 / 56; 128 pairs, 100 tokens 13.1 / 12.1 / 12.2, 64 of 64 heads at 100 15.1 / 13.3 / 14.0; 224 pairs, 200 tokens at 100
+          // 26.0 / 26.4 / 26.5; 512 pairs, 512 tokens 41.1 / 42.9 / 45.5
+          const int pairs = w.heads * nt, groups = pairs <= 64 ? 4 : pairs <= 128 ? 2 : 1;
+          auto go = [&](auto scores, auto values, int g) {
+            hipLaunchKernelGGL(scores, gs, dim3(256), 0, (hipStream_t)stream, a, w);
+            hipLaunchKernelGGL(values, dim3(w.heads, nt, g), dim3(256), pv_lds(g), (hipStream_t)stream, a, w);
+          };
+          auto of = [&](auto ct, auto one) {
+            using CT = decltype(ct);
+            constexpr bool ONE = decltype(one)::value;
+            if (groups == 4) go(prefill_scores_kernel<CT, ONE>, prefill_values_kernel<CT, ONE, 4>, 4);
+            else if (groups == 2) go(prefill_scores_kernel<CT, ONE>, prefill_values_kernel<CT, ONE, 2>, 2);
+            else go(prefill_scores_kernel<CT, ONE>, prefill_values_kernel<CT, ONE, 1>, 1);
+          };
+          if (kv_dtype == 1) a.bpw == 1 ? of(mrs::bf16_t{}, std::true_type{}) : of(mrs::bf16_t{}, std::false_type{});
+          else a.bpw == 1 ? of(mrs::f16_t{}, std::true_type{}) : of(mrs::f16_t{}, std::false_type{});
         }
       return 0;
     }

@@ -59,8 +59,9 @@ def test_prompt_attention_equals_decode_attention_gpu(oracle, dev, heads, kvh, T
 
 
 # (heads, kv heads, T, model context, kv dtype, window, first position, (head, tile) pairs that fit the workspace): one block and several blocks per split, whole launches,
-# groups of heads, groups of query tiles
-WS = [(4, 1, 40, 64, 1, 0, 0, 99), (4, 2, 70, 128, 0, 0, 0, 7), (2, 2, 33, 96, 1, 0, 20, 1), (8, 2, 50, 4096, 1, 0, 200, 99), (4, 1, 90, 128, 1, 40, 0, 2), (3, 3, 1, 2304, 0, 0, 130, 99)]
+# groups of heads, groups of query tiles; up to 64 / 128 / more pairs per launch (the split groups of the values kernel: 4, 2, 1), the last round of groups short
+WS = [(4, 1, 40, 64, 1, 0, 0, 99), (4, 2, 70, 128, 0, 0, 0, 7), (2, 2, 33, 96, 1, 0, 20, 1), (8, 2, 50, 4096, 1, 0, 200, 99), (4, 1, 90, 128, 1, 40, 0, 2), (3, 3, 1, 2304, 0, 0, 130, 99),
+      (2, 2, 3, 512, 1, 0, 190, 99), (48, 48, 40, 128, 1, 0, 40, 99), (72, 9, 40, 128, 0, 0, 0, 999), (40, 5, 33, 4096, 1, 0, 80, 99)]
 
 
 def check_attention_ws(O, be, heads, kvh, T, max_ctx, kv_dtype, window, start, pairs):
