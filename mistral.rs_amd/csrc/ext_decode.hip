@@ -688,74 +688,86 @@ __global__ void __launch_bounds__(1024) moe_router_kernel(const float *__restric
 #ifndef MRS_WAIT_VMCNT0
 #define MRS_WAIT_VMCNT0() asm volatile("s_waitcnt vmcnt(0)" ::: "memory")
 #endif
+// What bounds it is the chain of latencies, so the row, the norm's weights and the expert's row are requested at once (ROUTER_R float4 per thread / lane in registers; longer rows load the
+// rest where they need it), and the last arriver's wave reads the logits from lanes instead of LDS and takes all exponentials at once, in the serial code's order of comparisons and
+// additions.  us per launch, one token, 8 experts of 4096 values,
+// weights from HBM, loads where they are used and one lane's softmax / this: 8.5 / 6.6.
+constexpr int ROUTER_R = 16;
 __global__ void __launch_bounds__(256) moe_router_split_kernel(const float *__restrict__ x, const float *__restrict__ gate_w, int E, int K, int top_k, int renormalize,
                                                                int32_t *__restrict__ ids, float *__restrict__ weights, const float *__restrict__ norm_w, float eps,
                                                                float *__restrict__ scratch) {
-  __shared__ float lg[64];
   __shared__ float red[4];
-  __shared__ int last_s;
   extern __shared__ __attribute__((aligned(16))) char xn_s[];
   const int e = blockIdx.x, tok = blockIdx.y, tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-  const float *xr = x + (size_t)tok * K;
+  const float *xr = x + (size_t)tok * K, *wr = gate_w + (size_t)e * K;
   float *xn = (float *)xn_s;
   const int nvec = K / 4;
-  float sum = 0.f;
-  for (int v = tid; v < nvec; v += 256) {
-    const float4 t = *(const float4 *)(xr + 4 * v);
-    sum = fmaf(t.x, t.x, sum); sum = fmaf(t.y, t.y, sum); sum = fmaf(t.z, t.z, sum); sum = fmaf(t.w, t.w, sum);
+  float4 xv[ROUTER_R / 4], nv[ROUTER_R / 4], gv[ROUTER_R];
+  if (nvec > 0) {
+#pragma unroll
+    for (int u = 0; u < ROUTER_R / 4; ++u) xv[u] = *(const float4 *)(xr + 4 * min(tid + 256 * u, nvec - 1));
+#pragma unroll
+    for (int u = 0; u < ROUTER_R / 4; ++u) nv[u] = *(const float4 *)(norm_w + 4 * min(tid + 256 * u, nvec - 1));
+    if (wave == 0) {
+#pragma unroll
+      for (int u = 0; u < ROUTER_R; ++u) gv[u] = *(const float4 *)(wr + 4 * min(lane + 64 * u, nvec - 1));
+    }
   }
+  float sum = 0.f;
+  auto square = [&](const float4 &t) { sum = fmaf(t.x, t.x, sum); sum = fmaf(t.y, t.y, sum); sum = fmaf(t.z, t.z, sum); sum = fmaf(t.w, t.w, sum); };
+#pragma unroll
+  for (int u = 0; u < ROUTER_R / 4; ++u) if (tid + 256 * u < nvec) square(xv[u]);
+  for (int v = tid + 64 * ROUTER_R; v < nvec; v += 256) square(*(const float4 *)(xr + 4 * v));
   sum = wave_sum(sum);
   if (lane == 0) red[wave] = sum;
   __syncthreads();
   const float inv = rsqrtf((red[0] + red[1] + red[2] + red[3]) / (float)K + eps);
-  for (int v = tid; v < nvec; v += 256) {
-    const float4 t = *(const float4 *)(xr + 4 * v), w = *(const float4 *)(norm_w + 4 * v);
-    *(float4 *)(xn + 4 * v) = make_float4(t.x * inv * w.x, t.y * inv * w.y, t.z * inv * w.z, t.w * inv * w.w);
-  }
+  auto normed = [&](const float4 &t, const float4 &w) { return make_float4(t.x * inv * w.x, t.y * inv * w.y, t.z * inv * w.z, t.w * inv * w.w); };
+#pragma unroll
+  for (int u = 0; u < ROUTER_R / 4; ++u) if (tid + 256 * u < nvec) *(float4 *)(xn + 4 * (tid + 256 * u)) = normed(xv[u], nv[u]);
+  for (int v = tid + 64 * ROUTER_R; v < nvec; v += 256) *(float4 *)(xn + 4 * v) = normed(*(const float4 *)(xr + 4 * v), *(const float4 *)(norm_w + 4 * v));
   __syncthreads();
+  if (wave != 0) return;
   float *slog = scratch + (size_t)tok * (E + 1);
   unsigned *ticket = (unsigned *)(slog + E);
-  if (wave == 0) {
-    float s = 0.f;
-    const float *wr = gate_w + (size_t)e * K;
-#pragma unroll 8
-    for (int i = lane * 4; i < K; i += 256) {
-      const float4 a4 = *(const float4 *)(xn + i), w4 = *(const float4 *)(wr + i);
-      s = fmaf(a4.x, w4.x, s); s = fmaf(a4.y, w4.y, s); s = fmaf(a4.z, w4.z, s); s = fmaf(a4.w, w4.w, s);
-    }
-    s = wave_sum(s);
-    if (lane == 0) {
-      __hip_atomic_store(slog + e, s, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);  // write-through
-      MRS_WAIT_VMCNT0();
-      last_s = __hip_atomic_fetch_add(ticket, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == (unsigned)(E - 1);
-      if (last_s) __hip_atomic_store(ticket, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    }
+  float s = 0.f;
+  auto dot = [&](const float4 &a4, const float4 &w4) { s = fmaf(a4.x, w4.x, s); s = fmaf(a4.y, w4.y, s); s = fmaf(a4.z, w4.z, s); s = fmaf(a4.w, w4.w, s); };
+#pragma unroll
+  for (int u = 0; u < ROUTER_R; ++u) if (lane + 64 * u < nvec) dot(*(const float4 *)(xn + 4 * (lane + 64 * u)), gv[u]);
+  for (int v = lane + 64 * ROUTER_R; v < nvec; v += 64) dot(*(const float4 *)(xn + 4 * v), *(const float4 *)(wr + 4 * v));
+  s = wave_sum(s);
+  int last = 0;
+  if (lane == 0) {
+    __hip_atomic_store(slog + e, s, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);  // write-through
+    MRS_WAIT_VMCNT0();
+    last = __hip_atomic_fetch_add(ticket, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == (unsigned)(E - 1);
+    if (last) __hip_atomic_store(ticket, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   }
-  __syncthreads();
-  if (!last_s) return;
-  if (tid < E) lg[tid] = __hip_atomic_load(slog + tid, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);  // sc1: past L1
-  __syncthreads();
-  if (tid == 0) {  // moe_router_kernel's serial softmax / top-k, unchanged
-    float mx = -INFINITY;
-    for (int j = 0; j < E; ++j) mx = fmaxf(mx, lg[j]);
-    float den = 0.f;
-    for (int j = 0; j < E; ++j) den += expf(lg[j] - mx);
-    float sel = 0.f;
-    unsigned long long used = 0;
-    for (int k = 0; k < top_k; ++k) {
-      int best = -1; float bv = -INFINITY;
-      for (int j = 0; j < E; ++j) if (!((used >> j) & 1ull) && lg[j] > bv) { bv = lg[j]; best = j; }
-      if (best < 0) {
-        for (int j = 0; j < E && best < 0; ++j) if (!((used >> j) & 1ull)) best = j;
-        bv = lg[best];
-      }
-      used |= 1ull << best;
-      const float p = expf(bv - mx) / den;
-      ids[(size_t)tok * top_k + k] = best;
-      weights[(size_t)tok * top_k + k] = p;
-      sel += p;
-    }
-    if (renormalize) for (int k = 0; k < top_k; ++k) weights[(size_t)tok * top_k + k] /= sel;
+  if (!__builtin_amdgcn_readfirstlane(last)) return;
+  // moe_router_kernel's serial softmax / top-k: lane j holds logit j (E <= 64)
+  const float lgv = __hip_atomic_load(slog + min(lane, E - 1), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);  // sc1: past L1
+  auto of_lane = [](float v, int j) { return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), j)); };
+  float mx = -INFINITY;
+  for (int j = 0; j < E; ++j) mx = fmaxf(mx, of_lane(lgv, j));
+  const float ex = expf(lgv - mx);
+  float den = 0.f;
+  for (int j = 0; j < E; ++j) den += of_lane(ex, j);
+  float sel = 0.f, mine = 0.f;  // lane k keeps the k-th weight and id
+  int my_id = 0;
+  unsigned long long used = 0;
+  for (int k = 0; k < top_k; ++k) {
+    int best = -1; float bv = -INFINITY;
+    for (int j = 0; j < E; ++j) { const float v = of_lane(lgv, j); if (!((used >> j) & 1ull) && v > bv) { bv = v; best = j; } }
+    if (best < 0) best = __ffsll((long long)~used) - 1;  // every remaining logit is NaN or -inf: the lowest unused expert
+    best = __builtin_amdgcn_readfirstlane(best);
+    used |= 1ull << best;
+    const float p = of_lane(ex, best) / den;
+    if (lane == k) { mine = p; my_id = best; }
+    sel += p;
+  }
+  if (lane < top_k) {
+    ids[(size_t)tok * top_k + lane] = my_id;
+    weights[(size_t)tok * top_k + lane] = renormalize ? mine / sel : mine;
   }
 }
 }  // namespace mrs

@@ -637,12 +637,15 @@ def test_proj_top2_gpu(oracle, dev, tname, n, k, experts, sels):
     check_proj_top2(oracle, GpuBackend(dev), tname, n, k, experts, sels)
 
 
-def _check_router_norm(be, tokens, E, K, topk):
+def _check_router_norm(be, tokens, E, K, topk, bad=()):
     """mrs_moe_router_topk_norm (RmsNorm inside the router's workgroup) == mrs_rms_norm_f32 followed by mrs_moe_router_topk: same ids, same weights bit for bit."""
     rng = np.random.default_rng(E + K + tokens)
     h = (rng.standard_normal((tokens, K)) * 1.7).astype(np.float32)
     nw = (1.0 + 0.05 * rng.standard_normal(K)).astype(np.float32)
     gw = (rng.standard_normal((E, K)) * 0.05).astype(np.float32)
+    for e, v in bad:
+        gw[e] = 0.0
+        gw[e, 0] = v
     hb, nb, gb = be.buf(h), be.buf(nw), be.buf(gw)
     xn = be.buf(np.zeros((tokens, K), np.float32))
     ids_a, w_a = be.buf(np.full((tokens, topk), -1, np.int32)), be.buf(np.zeros((tokens, topk), np.float32))
@@ -669,6 +672,13 @@ def _check_router_norm(be, tokens, E, K, topk):
 @pytest.mark.parametrize("tokens,E,K,topk", [(1, 8, 4096, 2), (3, 4, 512, 2), (2, 16, 1024, 3), (1, 3, 256, 1)])
 def test_router_with_fused_norm_host_emulation(tokens, E, K, topk):
     _check_router_norm(HostBackend(), tokens, E, K, topk)
+
+
+# rows longer than the split router's registers, the shortest, every lane an expert; equal logits, logits of NaN, of infinities and nothing else
+@pytest.mark.parametrize("tokens,E,K,topk,bad", [(1, 5, 4356, 2, ()), (2, 2, 4, 1, ()), (1, 64, 256, 8, ()), (1, 4, 64, 3, [(1, 0.0), (2, 0.0)]), (1, 4, 64, 2, [(0, np.nan), (3, -np.inf)]),
+                                                 (1, 3, 64, 3, [(0, np.nan), (1, np.nan), (2, np.nan)]), (1, 4, 64, 4, [(1, np.inf), (2, -np.inf), (3, np.nan)])])
+def test_router_rows_and_logits_at_their_limits_host_emulation(tokens, E, K, topk, bad):
+    _check_router_norm(HostBackend(), tokens, E, K, topk, bad)
 
 
 @pytest.mark.gpu
