@@ -1,5 +1,5 @@
 // dec_attn.cuh -- decode attention of the decode engine as wave-level device functions: the split kernel with the last-arriver merge
-// (ext_dec.hip dec_attn2_kernel, the default), the persistent step kernel and the one-launch short-context kernel all call these, so every
+// (ext_dec.hip dec_attn2_kernel: groups of one and two heads; dec_attn4_kernel restates the same chains for four and eight), the persistent step kernel and the one-launch short-context kernel all call these, so every
 // engine path produces the same bits.  One wave per range of 32-token KV blocks of one (sequence, kv head): online softmax in f32 for the G query
 // heads of the GQA group, probabilities kept in f32, partial (m, l, o) per split; then the splits are merged per head.
 // Arithmetic = the reference CPU attention (mistralrs-core/src/attention/backends/cpu/single_q.rs): tile max, correction and probabilities

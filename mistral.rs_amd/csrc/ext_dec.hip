@@ -858,7 +858,7 @@ extern "C" int mrs_dec_gate_up_img(const mrs_dec_mat_c *wg, const mrs_dec_mat_c 
   return Launch<EPI_GLU>::run(a, b, (hipStream_t)stream);
 }
 
-// Decode attention of the engine, one launch (dec_attn2_kernel).  out_f32 [b][num_heads * 128] (may be NULL when an image is written);
+// Decode attention of the engine, one launch (dec_attn4_kernel: four and eight heads per key head; dec_attn2_kernel: one and two).  out_f32 [b][num_heads * 128] (may be NULL when an image is written);
 // img_out: Q8_K activation image for mrs_dec_proj_img (written when the GQA group is even; may be NULL); ticket: [b * num_kv_heads] u32, zero
 // before the first call (the kernel leaves it zero); part_*: the partials workspace of mrs_decode_attention_f32_*.  Returns 1 when the image
 // was written, 0 when only out_f32 was, < 0 on a shape outside the kernel (head size 128, 32-token pages, GQA group 1 / 2 / 4 / 8).
