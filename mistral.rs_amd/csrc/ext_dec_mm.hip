@@ -82,7 +82,8 @@ __host__ __device__ inline size_t lds_bytes(int K, int nc, int mode) {
   return (size_t)nc * qcs_of(K) + (mode == ACT_Q80 ? sp * 256 : sp * (32 + 256)) + 2 * 4 * 8 * 16 * 4 + LDS_ZEROS;
 }
 
-template <int NPC> struct Rec { v4u q[NPC]; v4u hs; unsigned hd; };
+template <int NPC> struct Rec { v4u q[NPC]; v4u hs; unsigned hd; };  // hd: the superblock scales (not Q8_0's, whose block scales are hs)
+template <int NPC, int TMASK> constexpr int rec_requests = NPC + 1 + (TMASK == TM_Q80 ? 0 : 1);  // issue_rec()'s requests: what a wait counts
 
 __device__ __forceinline__ i4v mk_i4(v2u a, v2u b) { return i4v{(int)a.x, (int)a.y, (int)b.x, (int)b.y}; }
 __device__ __forceinline__ long mk_l(unsigned lo, unsigned hi) { return (long)(((unsigned long long)hi << 32) | lo); }
@@ -220,7 +221,7 @@ __device__ __forceinline__ void issue_rec(Rec<NPC> &slot, int &m, Cursor &k, __a
   for (int c = 0; c < NPC; ++c)  // (a Q4_K record in a mixed launch: pieces 4 .. 7 ask past the tensor)
     slot.q[c] = __builtin_amdgcn_raw_buffer_load_b128(rs, (c < 4 || !small) ? vq + (unsigned)(c & 3) * 1024u : DEAD, so + (c < 4 ? 0u : 4096u), MRS_DEC2_LD_AUX);
   slot.hs = __builtin_amdgcn_raw_buffer_load_b128(rs, vh, so + tail, MRS_DEC2_LD_AUX);
-  slot.hd = __builtin_amdgcn_raw_buffer_load_b32(rs, vd, so + tail + 512u - k.half * 192u, MRS_DEC2_LD_AUX);
+  if constexpr (TMASK != TM_Q80) slot.hd = __builtin_amdgcn_raw_buffer_load_b32(rs, vd, so + tail + 512u - k.half * 192u, MRS_DEC2_LD_AUX);
   m = live ? (k.type | (k.ct << 8) | ((two ? 1 : 0) << 23) | ((k.ct + 2 >= ntp ? 1 : 0) << 24)) : -1;
   if (live) {  // scalar bookkeeping only
     k.ct += 2; k.rec += 2u * rb;
@@ -357,7 +358,8 @@ __device__ __forceinline__ void dec_mm_body(const MmArgs &a, char *smem) {
   auto grp_at = [&](int c) __attribute__((always_inline)) { return (unsigned)act_bytes(K, MOE ? (int)((rows >> (8 * c)) & 255u) : (int)((a.gc0p >> (4 * c)) & 15u)); };
   // Quants, superblock scales and Q8_0's block scales are copied by LDS-DMA, as many requests as there are pieces of 1 KiB and no registers in between; only the run sums, which
   // the mins' MFMA reads as f16, pass through registers, a batch of up to 8 per thread.  Everything is requested at once, the weight ring last (with image requests behind it
-  // the waits of its first records come out as full drains), and the wait before the barrier leaves exactly the ring in flight.  Requests go through ONE buffer resource over
+  // the waits of its first records come out as full drains), and the wait before the barrier leaves exactly the ring in flight: it counts the requests that issue_rec() makes,
+  // so every one of them has to be used (hipcc drops the others, and the wait would let as many of the image's pass).  Requests go through ONE buffer resource over
   // the image(s): a column that does not exist asks past the end (zeros).
   // (Batches of 8 + 8 + 16 register loads whatever the row's length, each stored before the next was requested, had 18 of 48 requests dead at 4096 values and four round trips at
   // 14336: start of a launch to its first record, us, 8 columns: 3.5 / 5.8 of K = 4096 / 14336.)
@@ -414,7 +416,7 @@ __device__ __forceinline__ void dec_mm_body(const MmArgs &a, char *smem) {
     for (int i = 0; i < R; ++i) issue(ring[i], meta[i]);  // the weight ring
     __builtin_amdgcn_sched_barrier(0);
     MRS_MM_TL(1);
-    MRS_WAIT_VMCNT(R * (NPC + 2));  // the image has landed
+    MRS_WAIT_VMCNT((R * rec_requests<NPC, TMASK>));  // the image has landed
     st_sums(slast);
     if (tid < 64) ((unsigned *)zeros)[tid] = 0u;
   }

@@ -4,6 +4,9 @@ SAME BITS for every column count 1..8 -- a token's result must not depend on whi
 engine-order restatement of the oracle (oracle/cpu_path_oracle.c orc_gemv_engine).  Reference role: MMVQ's batch 1..8 from one pass over the weights
 (mistralrs-quant/kernels/mmvq_gguf/mmvq_gguf.cu:724-792, gguf/fast_mmvq.rs:52).  Same bodies on the wave64 host emulation (CPU suite) and on the MI355X."""
 import ctypes as C
+import os
+import re
+import subprocess
 
 import numpy as np
 import pytest
@@ -228,3 +231,23 @@ def test_mm_experts_host_emulation(oracle, case):
                                   ("Q8_0", "Q5_K", 512, 768, 5, 3, 3, [4, 0, 1, 0, 4, 3, 1, 4, 0])])
 def test_mm_experts_gpu(oracle, dev, case):
     check_mm_experts(oracle, GpuBackend(dev), *case)
+
+
+def test_the_wait_for_the_image_leaves_exactly_the_weight_ring_in_flight(tmp_path):
+    """The kernels wait for the image in front of the first barrier by a count of the requests behind it: the weight ring's, which alone are non-temporal.  A count above theirs (a
+    request that the compiler drops) would let as many of the image's requests pass."""
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    csrc, hipcc, out = os.path.join(root, "mistral.rs_amd", "csrc"), os.environ.get("HIPCC", "/opt/rocm/bin/hipcc"), str(tmp_path / "mm.s")
+    subprocess.run([hipcc, "--offload-arch=gfx950", "-O3", "-std=c++17", "-ffp-contract=off", "-w", "-I" + csrc, "-I" + os.path.join(root, "include"), "-Xclang", "-target-feature", "-Xclang",
+                    "-packed-fp32-ops", "--cuda-device-only", "-S", os.path.join(csrc, "ext_dec_mm.hip"), "-o", out], check=True)
+    kernels = re.findall(r"^(_Z\w*dec_mm\w*):(.*?)s_barrier", open(out).read(), re.M | re.S)
+    assert len(kernels) >= 11
+    for name, code in kernels:
+        image, ring = code.rfind(" lds\n"), 0
+        assert image > 0, name
+        for line in code[image:].splitlines():
+            ring += bool(re.match(r"\s+buffer_load.* nt\b", line))
+            wait = re.match(r"\s+s_waitcnt vmcnt\((\d+)\)", line)
+            if ring and wait:
+                break
+        assert wait and int(wait.group(1)) == ring, (name, line, ring)
