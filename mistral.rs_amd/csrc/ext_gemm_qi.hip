@@ -31,6 +31,7 @@ namespace qi {
 using namespace mrs::dec2;
 
 typedef _Float16 h2 __attribute__((ext_vector_type(2)));
+typedef unsigned short us2 __attribute__((ext_vector_type(2)));
 typedef _Float16 h8 __attribute__((ext_vector_type(8)));
 typedef float f16v __attribute__((ext_vector_type(16)));
 typedef float f32v __attribute__((ext_vector_type(32)));
@@ -451,8 +452,8 @@ __global__ void __launch_bounds__(256 * wide_groups(MODE), MODE == W_ONE ? (NT =
       // one v_mfma_i32_32x32x32_i8 IS one block of 32 tokens x 32 rows (int32: exact); p_b = ((float)isum_b dw_b) dx_b, T = p_0 + .. + p_7 left to right.  What bounds this
       // format is the vector instructions per output and block, three of them: the accumulator starts at the bits of 1.5 x 2^23, so that its bits ARE the f32 value
       // 1.5 x 2^23 + isum (|isum| <= 2^19), and one fma takes the offset off under the multiplication by dw -- 1.5 x 2^23 dw is exact (13 bits), so the fma rounds isum dw
-      // once, as the product alone would.  A scale that is not finite would make it inf - inf, a negative one would lose the sign of a zero: such a superblock is done over with
-      // a conversion.  Gate / up of 28672 x 4096, one token tile, us, a conversion and scales from LDS / this: 700 tokens 290 / 272, 2000 tokens 780 / 739 (the fma alone, scales from LDS:
+      // once, as the product alone would.  A scale that is not finite would make it inf - inf, a negative one or a zero (with quants that are not all zeros) would lose the sign of
+      // a zero: such a superblock is done over with a conversion.  Gate / up of 28672 x 4096, one token tile, us, a conversion and scales from LDS / this: 700 tokens 290 / 272, 2000 tokens 780 / 739 (the fma alone, scales from LDS:
       // 311, 831); two token tiles 263, 720.
       MRS_WAIT_VMCNT0();
       __syncthreads();
@@ -462,8 +463,7 @@ __global__ void __launch_bounds__(256 * wide_groups(MODE), MODE == W_ONE ? (NT =
       constexpr int MAGIC = 0x4B400000;  // 1.5 x 2^23
       const i16v imagic = {MAGIC, MAGIC, MAGIC, MAGIC, MAGIC, MAGIC, MAGIC, MAGIC, MAGIC, MAGIC, MAGIC, MAGIC, MAGIC, MAGIC, MAGIC, MAGIC};
       const unsigned y_lane = (unsigned)(8 * ((lane >> 2) & 3) + 4 * hf + (lane & 3)) * 4u;  // the scale of output v = lane % 16
-      unsigned odd = 0u;
-      auto odd16 = [](unsigned w) { return (((w & 0x7c007c00u) + 0x04000400u) | w) & 0x80008000u; };  // not finite, or negative
+      us2 odd = {0, 0};  // of the scales' bits - 1: positive finite ones are 0 .. 0x7bfe
       i4v af[2][NT];
       float Tt[NT][16];
 #pragma unroll
@@ -481,7 +481,7 @@ __global__ void __launch_bounds__(256 * wide_groups(MODE), MODE == W_ONE ? (NT =
         wq[b & 3] = b < 4 ? load_q(rec, b + 4) : load_q(rec_next, b - 4);
         if (b < NSTAGE) stage_q(sb + STEP, it + 1, b, more);
         const unsigned hw = hw8[b / 2];
-        if (b % 2 == 0) odd |= odd16(hw);
+        if (b % 2 == 0) odd = __builtin_elementwise_max(odd, (us2)(__builtin_bit_cast(us2, hw) - us2{1, 1}));
         float dwb = half_bits_to_float((uint16_t)((b & 1) ? (hw >> 16) : (hw & 0xffffu)));
         MRS_OPAQUE_TID(dwb);  // in f32: not converted anew in every fma
         if (b % 2 == 1) hw8[b / 2] = load_hw(rec_next, b / 2);
@@ -495,7 +495,18 @@ __global__ void __launch_bounds__(256 * wide_groups(MODE), MODE == W_ONE ? (NT =
         }
         __builtin_amdgcn_sched_barrier(0);  // one block at a time: more results in flight do not fit the registers
       }
-      if (__ballot(odd != 0u) != 0ull) {  // wave-uniform, never in a sound model
+      bool over = __ballot(odd.x > 0x7bfe || odd.y > 0x7bfe) != 0ull;  // wave-uniform
+      if (over) {  // blocks of zeros have a scale of zero and may stay
+        unsigned redo = 0u;
+#pragma unroll
+        for (int b = 0; b < 8; ++b) {
+          const unsigned hw = load_hw(rec, b / 2), h16 = (b & 1) ? hw >> 16 : hw & 0xffffu;
+          const v4u w = load_q(rec, b);
+          redo |= h16 == 0u ? w.x | w.y | w.z | w.w : (unsigned)(h16 > 0x7bffu);
+        }
+        over = __ballot(redo != 0u) != 0ull;
+      }
+      if (over) {  // never in a sound model
         i16v izero;
 #pragma unroll
         for (int v = 0; v < 16; ++v) izero[v] = 0;
