@@ -674,6 +674,7 @@ __global__ void __launch_bounds__(256 * wide_groups(MODE), MODE == W_ONE ? (NT =
     if (grp == 1) return;
     if (z_begin + 2 * steps <= z_end) add_pair(steps - 1);
   }
+  const bool gap = S <= 3 * Cs;  // a row's last run(s) are empty: + 0, the neutral - 0 of `run` in its place would leave the sign to a sum of negative zeros
   if constexpr (MODE == W_RUNS2 || MODE == W_RUNS4) {
     constexpr int PL = MODE == W_RUNS4 ? 4 : 3, VG = 16 / GROUPS;  // planes: c0 .. c3 | c0 + c1, c2, c3;  outputs of a group, of every token tile
     MRS_WAIT_VMCNT0();  // the last requests to LDS (out of range: zeros) have landed
@@ -704,6 +705,7 @@ __global__ void __launch_bounds__(256 * wide_groups(MODE), MODE == W_ONE ? (NT =
         const float4 c0 = get(0), c1 = get(1), c2 = get(2), c3 = MODE == W_RUNS4 ? get(PL - 1) : make_float4(0.f, 0.f, 0.f, 0.f);
         float r[4] = {(c0.x + c1.x) + c2.x, (c0.y + c1.y) + c2.y, (c0.z + c1.z) + c2.z, (c0.w + c1.w) + c2.w};
         if (MODE == W_RUNS4) { r[0] = r[0] + c3.x; r[1] = r[1] + c3.y; r[2] = r[2] + c3.z; r[3] = r[3] + c3.w; }
+        if (gap) { r[0] = r[0] + 0.f; r[1] = r[1] + 0.f; r[2] = r[2] + 0.f; r[3] = r[3] + 0.f; }
 #pragma unroll
         for (int i = 0; i < 4; ++i)
           st32(a.accumulate ? old[tt][4 * q + i] + r[i] : r[i], ro, vo + (unsigned)((tt * 32 + 8 * (grp * (VG / 4) + q) + i) * ldo));
@@ -718,6 +720,12 @@ __global__ void __launch_bounds__(256 * wide_groups(MODE), MODE == W_ONE ? (NT =
     for (int tt = 0; tt < NT; ++tt)
 #pragma unroll
       for (int v = 0; v < 16; ++v) pend[tt][v] = run[tt][v];
+  }
+  if (gap && !split) {
+#pragma unroll
+    for (int tt = 0; tt < NT; ++tt)
+#pragma unroll
+      for (int v = 0; v < 16; ++v) pend[tt][v] = pend[tt][v] + 0.f;
   }
   if (a.accumulate && !split) {
     float old[NT][16];
