@@ -292,7 +292,7 @@ int mrs_qi_quantize_for(int w_ggml_type, const float *x, const float *x2, int ld
 /* mrs_gemm_qi_multi: up to three tensors of one type that multiply the same operand rows (q / k / v, gate / up), in one launch where the kernel takes segments.  bounds != NULL
  * (device ints [experts + 1]): every tensor is a stack of `experts` tensors [N][K] (N % 32 == 0 where experts > 1: the copy's panels have 32 rows; else -1), expert e multiplies
  * and writes the rows [bounds[e], bounds[e + 1]); max_rows bounds one expert's rows and sizes the grid */
-/* mrs_gemm_qi_is_cut: 1 if mrs_gemm_qi_multi, given a workspace of 4 T sum(N) floats, may cut the launch by runs of superblocks; mrs_gemm_qi_cut_bytes: a workspace for every launch over
+/* mrs_gemm_qi_is_cut: 1 if mrs_gemm_qi_multi, given a workspace of 4 T sum(N) floats, cuts the launch by runs of superblocks; mrs_gemm_qi_cut_bytes: a workspace for every launch over
  * at most n rows of weights and T tokens that is cut (never falls as T or n grow).  A smaller one, or NULL: the launch stays whole, same bits. */
 size_t mrs_gemm_qi_cut_bytes(int T, int n, int K);
 int mrs_gemm_qi_is_cut(int ggml_type, int n_tensors, const int *N, int K, int T);

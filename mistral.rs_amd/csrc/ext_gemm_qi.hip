@@ -991,7 +991,7 @@ extern "C" size_t mrs_gemm_qi_cut_bytes(int T, int n, int K) {
   const int tiles = std::max(std::max(cut_max(T_Q8_0, 1, K), cut_max(T_Q4_K, 1, K)), 2 * std::max(cut_max(T_Q8_0, 2, K), cut_max(T_Q4_K, 2, K)));
   return (size_t)16 * std::min((size_t)T * n, (size_t)tiles * 32 * qi::WIDE_ROWS);
 }
-// 1: mrs_gemm_qi_multi over T rows, given a workspace, is cut (unless its workgroups split the runs among their own waves: wide_runs)
+// 1: mrs_gemm_qi_multi over T rows, given a workspace, is cut (the launch itself asks here)
 extern "C" int mrs_gemm_qi_is_cut(int type, int nt, const int *N, int K, int T) {
   if (!N || nt < 1 || nt > 3 || !qi::qi_type(type) || T <= 0 || K <= 0 || K % 256) return 0;
   int gx = 0;
@@ -999,8 +999,8 @@ extern "C" int mrs_gemm_qi_is_cut(int type, int nt, const int *N, int K, int T) 
     if (N[i] <= 0 || N[i] % 4) return 0;
     gx += (N[i] + qi::WIDE_ROWS - 1) / qi::WIDE_ROWS;
   }
-  const int NT = wide_tiles(type, T, gx);
-  return wide_cut(type, gx * ((T + 32 * NT - 1) / (32 * NT)), K, NT);
+  const int NT = wide_tiles(type, T, gx), wgs = gx * ((T + 32 * NT - 1) / (32 * NT));
+  return wide_cut(type, wgs, K, NT) && !wide_runs(type, wgs, K, NT);
 }
 static int gemm_qi_launch(int type, int nt, const void *const *w_qi, const int *N, int K, const void *act, int T, float *const *out, const int *ldo, int accumulate,
                           const int *bounds, int experts, int max_rows, void *workspace, size_t workspace_bytes, bool keep_planes, void *stream) {
@@ -1025,7 +1025,7 @@ static int gemm_qi_launch(int type, int nt, const void *const *w_qi, const int *
   a.K = K; a.T = T; a.qf = qf; a.yd = yd; a.bsf = bsf; a.accumulate = accumulate; a.part = (float *)workspace; a.part_n = n_all; a.bounds = bounds; a.experts = experts; a.ksplit = 1;
   // windows: every expert's last tile may be partly filled, and none has more tiles than max_rows fill
   dim3 grid(gx, bounds ? std::min(T / tl + experts, experts * ((max_rows + tl - 1) / tl)) : (T + tl - 1) / tl);
-  if (!bounds && workspace && workspace_bytes >= (size_t)4 * T * n_all * 4 && mrs_gemm_qi_is_cut(type, nt, N, K, T) && !wide_runs(type, (int)(grid.x * grid.y), K, NT)) { a.ksplit = 4; grid.z = 4; }
+  if (!bounds && workspace && workspace_bytes >= (size_t)4 * T * n_all * 4 && mrs_gemm_qi_is_cut(type, nt, N, K, T)) { a.ksplit = 4; grid.z = 4; }
   const int wgs = (int)std::min<size_t>((size_t)grid.x * grid.y * grid.z, 1 << 20);
   const int mode = a.ksplit > 1 ? (wide_pair(type, wgs, NT) ? qi::W_PAIR : qi::W_ONE) : !bounds && wide_runs(type, wgs, K, NT) ? (NT == 2 ? qi::W_RUNS2 : qi::W_RUNS4) : qi::W_ONE;
   switch (type) {

@@ -503,6 +503,43 @@ def run_added_rows(O, be, tname, T, d, k):
     assert np.array_equal(h1.numpy(), h2.numpy()) and np.array_equal(a1.numpy(), a2.numpy())
 
 
+def run_planes_or_rows(O, be, tname, n, k, T, cut):
+    """The return code of mrs_gemm_qi_multi_planes is what mrs_gemm_qi_is_cut says: 1 and four planes, `out` as it was, or 0 and the rows, the workspace as it was."""
+    t = getattr(O, tname)
+    rng = np.random.default_rng(37)
+    p = O.quantize(t, (rng.standard_normal((n, k)) * 0.05).astype(np.float32)).reshape(n, -1)
+    x = rng.standard_normal((T, k)).astype(np.float32)
+    src, wq = be.buf(np.ascontiguousarray(p).reshape(-1)), be.buf(np.zeros(be.sym("mrs_gemm_qi_repack_bytes", [CI, C.c_longlong, C.c_longlong], C.c_size_t)(t, n, k), np.uint8))
+    assert be.sym("mrs_gemm_qi_repack", [VP, CI, C.c_longlong, C.c_longlong, VP, VP], CI)(src.ptr, t, n, k, wq.ptr, be.stream) == 0
+    xb, act = be.buf(x), be.buf(np.zeros(be.sym("mrs_qi_act_bytes", [CI, CI], C.c_size_t)(T, k), np.uint8))
+    assert be.sym("mrs_qi_quantize_for", [CI, VP, VP, CI, VP, C.c_float, CI, CI, VP, VP, VP], CI)(t, xb.ptr, None, k, None, 0.0, T, k, act.ptr, None, be.stream) == 0
+    ws, o, ns = be.buf(np.full((4, T, n), 3.0, np.float32)), be.buf(np.full((T, n), 7.0, np.float32)), (CI * 1)(n)
+    got = be.sym("mrs_gemm_qi_multi_planes", [CI, CI, VP, VP, CI, VP, CI, VP, VP, CI, VP, C.c_size_t, VP], CI)(t, 1, (VP * 1)(wq.ptr), ns, k, act.ptr, T, (VP * 1)(o.ptr), ns, 0, ws.ptr,
+                                                                                                             16 * T * n, be.stream)
+    assert got == cut == be.sym("mrs_gemm_qi_is_cut", [CI, CI, VP, CI, CI], CI)(t, 1, ns, k, T)
+    planes, rows = ws.numpy().reshape(4, T, n), o.numpy().reshape(T, n)
+    assert (rows == 7.0).all() if cut else (planes == 3.0).all()
+    out = ((planes[0] + planes[1]) + planes[2]) + planes[3] if cut else rows
+    assert np.array_equal(out, np.concatenate([O.gemv_engine(t, p, n, k, r) for r in x], axis=0))
+
+
+# either side of the lines from which a workgroup's groups of waves share the runs, one and two token tiles
+PLANES = [("Q4_K", 3456, 1024, 1, 1), ("Q4_K", 3584, 1024, 1, 0), ("Q4_K", 5248, 1024, 33, 1), ("Q4_K", 5376, 1024, 33, 0), ("Q8_0", 3968, 1024, 3, 1), ("Q8_0", 4096, 1024, 3, 0),
+          ("Q8_0", 5248, 1024, 40, 1), ("Q8_0", 5376, 1024, 40, 0), ("Q6_K", 5760, 1024, 3, 1), ("Q6_K", 5888, 1024, 3, 0), ("Q6_K", 5248, 1024, 33, 1), ("Q6_K", 5376, 1024, 33, 0),
+          ("Q5_K", 3584, 1024, 3, 1), ("Q4_K", 36, 768, 3, 0)]
+
+
+@pytest.mark.parametrize("case", PLANES[:2] + PLANES[-1:])
+def test_planes_or_rows_host_emulation(oracle, case):
+    run_planes_or_rows(oracle, HostBackend(), *case)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("case", PLANES)
+def test_planes_or_rows_gpu(oracle, dev, case):
+    run_planes_or_rows(oracle, GpuBackend(dev), *case)
+
+
 ADDED = [("Q4_K", 1, 256, 1024), ("Q8_0", 5, 2304, 1280), ("Q6_K", 37, 768, 1024)]  # rows of one superblock, of more than the 2048 values of a thread's first piece
 
 
