@@ -495,7 +495,7 @@ __global__ void __launch_bounds__(256 * wide_groups(MODE), MODE == W_ONE ? (NT =
         }
         __builtin_amdgcn_sched_barrier(0);  // one block at a time: more results in flight do not fit the registers
       }
-      bool over = __ballot(odd.x > 0x7bfe || odd.y > 0x7bfe) != 0ull;  // wave-uniform
+      bool over = __ballot((odd.x > 0x7bfe || odd.y > 0x7bfe) && vo < 0x80000000u) != 0ull;  // wave-uniform; rows past N are zeros
       if (over) {  // blocks of zeros have a scale of zero and may stay
         unsigned redo = 0u;
 #pragma unroll
