@@ -296,6 +296,7 @@ int mrs_qi_quantize_for(int w_ggml_type, const float *x, const float *x2, int ld
  * at most n rows of weights and T tokens that is cut (never falls as T or n grow).  A smaller one, or NULL: the launch stays whole, same bits. */
 size_t mrs_gemm_qi_cut_bytes(int T, int n, int K);
 int mrs_gemm_qi_is_cut(int ggml_type, int n_tensors, const int *N, int K, int T);
+int mrs_gemm_qi_form(int ggml_type, int n_tensors, const int *N, int K, int T, int room);  /* token tiles of a wave | groups of waves << 4 | cut << 8 (room: there is a workspace) */
 int mrs_gemm_qi_multi(int ggml_type, int n_tensors, const void *const *w_qi, const int *N, int K, const void *act, int T, float *const *out, const int *ldo, int accumulate,
                       const int *bounds, int experts, int max_rows, void *workspace, size_t workspace_bytes, void *stream);
 /* What stands between a prompt's products, in fewer launches.  mrs_gemm_qi_multi_planes: mrs_gemm_qi_multi over T rows that leaves the run sums of a cut launch as they are: 1 = the

@@ -950,39 +950,48 @@ template <int TYPE> static void wide_launch(int NT, int mode, const qi::WideArgs
   }
   NT == 2 ? wide_go<TYPE, 2, qi::W_ONE>(a, grid, s) : wide_go<TYPE, 1, qi::W_ONE>(a, grid, s);
 }
-// Token tiles per wave, by the rows of a launch (of an expert, where there are several) and its workgroup columns (of all experts).  K-quants: 32 rows fill one; two build each operand
-// once for both, but make the chain of a superblock longer, which is what a launch that leaves most of the chip idle waits for.  So two from 33 rows on where they make more than 32
-// workgroups (Q5_K, whose kernel of two tiles is the slowest: 96).  us, one / two tiles, each cut or whole as below (workgroups of two tiles in brackets): Q4_K 4096 x 4096 37 rows
-// (32) 11.3 / 13.7, 128 rows (64) 17.4 / 17.0, 6144 x 4096 37 rows (48) 14.7 / 14.2, 28672 x 4096 512 rows 221 / 199;  Q6_K 4096 x 14336 37 rows (32) 31.3 / 37.7, 128 rows (64)
-// 44.5 / 41.6, 1999 rows 570 / 457;  Q5_K 3072 x 1024 64 rows (24) 9.9 / 12.6, 4096 x 4096 160 rows (96) 22.0 / 25.5, 8192 x 8192 128 rows (128) 43.8 / 41.0;  Q8_0 4096 x 14336 64 rows
-// (32) 39.4 / 40.5, 6144 x 4096 64 rows (48) 20.1 / 18.0, 28672 x 4096 64 rows 51.9 / 43.2, 700 rows 285 / 263, 2000 rows 779 / 720.
-static int wide_tiles(int type, int rows, int cols) { return rows <= 32 || cols * ((rows + 63) / 64) <= (type == T_Q5_K ? 96 : 32) ? 1 : 2; }
-// A launch of few workgroups is cut by runs of superblocks: four times the workgroups, a quarter of the chain, for four planes of sums written and read again.  The planes cost the same
-// at any K and the chain saved grows with it, so the line lies at a number of workgroups in proportion to K.  Whole / cut, us: Q4_K, two tiles (workgroups in brackets), 2048 x 2048
-// 200 rows (64) 16.3 / 13.2, 400 rows (112) 16.4 / 19.2, 8192 x 2048 400 rows (448) 25.7 / 39.4; 4096 x 4096 256 rows (128) 28.8 / 23.0, 300 rows (160) 29.9 / 29.1, 512 rows (256)
-// 32.6 / 37.6; 28672 x 4096 128 rows (448) 48.5 / 60.5; 8192 x 8192 300 rows (320) 80.4 / 70.5, 400 rows (448) 87.9 / 95.3; 4096 x 14336 700 rows (352) 138.6 / 129.3, 1000 rows
-// (512) 159 / 172; 8192 x 28672 400 rows (448) 307 / 284.  One tile, 32 rows: 11264 x 2048 (88) 13.2 / 12.8, 28672 x 4096 (224) 26.9 / 25.9, 57344 x 8192 (448) 76.2 / 79.0, 65536 x 8192
-// (512) 76.7 / 84.3.  Q8_0, one tile: 4096 x 4096 32 rows (32) 33.5 / 14.1, 28672 x 4096 32 rows (224) 42.5 / 36.1; two: 2048 x 2048 300 rows (80) 20.5 / 17.5, 512 rows (128) 20.8 /
-// 21.5; 4096 x 4096 400 rows (224) 39.5 / 38.5, 620 rows (320) 55.2 / 50.0, 800 rows (416) 55.9 / 63.1; 8192 x 8192 300 rows (320) 106 / 83, 512 rows (512) 108 / 124.
-// Long rows are cut beyond it too where a second, partly filled round of workgroups (two fit a CU) would take as long as the first: K = 14336, Q4_K 1600 rows 314 / 287,
-// Q6_K 430 / 392, Q8_0 349 / 310.
-static int cut_line(int type, int K) { return type == T_Q8_0 ? K / 12 : K / 20; }  // two tiles
-static int cut_max(int type, int NT, int K) { return NT == 2 ? (K >= 8192 ? 895 : cut_line(type, K)) : type == T_Q8_0 ? std::min(K / 8, 895) : std::min(K / 18, 400); }
-// Whole launches of up to a workgroup per CU, but not so few that cutting them is better: workgroups of several groups of waves, each with its own runs (W_RUNS4 of one token tile,
-// W_RUNS2 of two).  us, cut / one group / so: Q4_K one tile 6144 x 4096 37 rows (96) 14.1 / 19.9 / 16.1, 4096 x 4096 128 rows (128) 16.9 / 20.1 / 16.3, 28672 x 4096 32 rows (224) 27.0 /
-// 25.0 / 20.7, two tiles 64 rows (224) 37.4 / 29.8 / 28.2;  Q6_K one tile 4096 x 4096 128 rows 19.1 / 25.7 / 21.6, 28672 x 4096 32 rows 36.4 / 32.2 / 31.6;  Q8_0 4096 x 4096 128 rows
-// 18.5 / 30.6 / 17.8, 28672 x 4096 32 rows 34.2 / 35.7 / 26.5, two tiles 64 rows 43.3 / 41.5 / 33.9.  Long rows have chains that only more workgroups shorten (Q4_K 4096 x 14336 128 rows
-// (128) 34.9 / 71.5 / 49.0).  Q5_K's kernel spills at 16 waves and is slower in both forms (30.2 -> 37.5, 36.2 -> 39.1).
-static bool wide_runs(int type, int wgs, int K, int NT) {
-  return type != T_Q5_K && K / 256 >= 4 && wgs <= 256 && wgs >= K / (NT == 2 ? 24 : type == T_Q4_K ? 36 : type == T_Q8_0 ? 32 : 22);
-}
-// Cut launches of one token tile: two groups take a run's superblocks in turn where the grid leaves a CU room for both (workgroups of all runs; Q8_0's fit twice).  us, one group /
-// two: K = 14336, 4096 rows of weights, 37 tokens (256) Q4_K 25.0 / 22.8, Q6_K 30.8 / 28.8, Q5_K 28.0 / 26.5, Q8_0 34.2 / 25.5, 128 tokens (512) Q4_K 34.9 / 40.1, Q8_0 41.8 / 36.4;
-// 4096 x 4096 37 tokens Q4_K 11.0 / 10.9, Q8_0 13.8 / 11.7; 6144 x 4096 128 tokens (768) Q8_0 22.4 / 23.1.
-static bool wide_pair(int type, int wgs, int NT) { return NT == 1 && wgs <= (type == T_Q8_0 ? 512 : 256); }
-static bool wide_cut(int type, int wgs, int K, int NT) {
-  if (K / 256 < 4 || wgs > cut_max(type, NT, K)) return false;
-  return NT == 1 || wgs <= std::min(cut_line(type, K), 511) || wgs > 512;
+// The experts' windows: token tiles per wave by the rows of an expert and the workgroup columns of all of them; always whole.  One tile fills with 32 rows; two build each operand once
+// for both, but make the chain of a superblock longer, which is what a launch that leaves most of the chip idle waits for.
+static int window_tiles(int type, int rows, int cols) { return rows <= 32 || cols * ((rows + 63) / 64) <= (type == T_Q5_K ? 96 : 32) ? 1 : 2; }
+// Every other launch: token tiles per wave (NT), groups of waves per workgroup (mode), cut by runs of superblocks (cut) or whole.  The lines are drawn through the times of all seven forms
+// at 9900 sizes (512 .. 32768 rows of weights, K = 1024 .. 28672, 1 .. 2000 tokens, weights from HBM): against the fastest form of each size the one taken costs 0.1 - 0.3 % on average
+// for 1 .. 32 tokens, 0.2 - 0.4 % to 128, 0.4 - 1.0 % beyond; lines drawn through some 40 sizes whose weights lay in the last-level cache cost 1 - 8 % and were up to 1.25 times slower
+// than no groups at all.  w1, w2: workgroups of one and of two token tiles.  Times in us, Q4_K unless named:
+//   * at most a workgroup per CU, and `line` of them or more: whole, one tile, the four runs in four groups.  A cut launch has more of the chip but writes and reads four planes of the
+//     outputs, so the line falls as the tiles fill.  Cut / so: 2048 x 2048, 128 tokens (w1 64) 10.3 / 11.7, 3072 x 2048 (96) 12.8 / 12.3; 16384 x 4096, 5 tokens (128) 15.9 / 19.0,
+//     28672 x 4096 (224) 24.8 / 21.6; cut with two tiles / so: 5120 x 4096, 128 tokens (160) 21.8 / 18.4.  With one tile or an odd number of them nothing above 208 is cut: four times
+//     that is a little more than three rounds (28672 x 8192, 5 tokens (224) 39.9 / 36.1).  One group instead of four: Q5_K, whose kernel spills at 16 waves; Q4_K and Q6_K where a run is
+//     one superblock (Q6_K 16384 x 1024, 32 tokens 11.3 / 12.8); Q6_K with 32 tokens or less below K = 4096 (28672 x 2048, 5 tokens 18.7 / 21.3).
+//   * two tiles, at most a workgroup per CU: two groups.  Cut / so: 28672 x 8192, 64 tokens (w2 224) 59.4 / 52.5, 8192 x 8192, 256 tokens (256) 58.5 / 51.1, whole / so 54.0 / 51.1.
+//   * else one tile or two by time(), the superblocks in a row on the busiest CU, of which two tiles take 1.5 - 1.8 times as long.  One / two: 12288 x 4096, 160 tokens (w1 480, w2 288)
+//     33.0 / 42.2, 28672 x 4096, 512 tokens 198 / 164; Q8_0 5120 x 4096, 800 tokens (1000, 520) 63.2 / 88.7; cut: 4096 x 4096, 64 tokens (64, 32) 13.5 / 14.9, 96 tokens (96, 64)
+//     16.9 / 16.4.  Whole / cut with two tiles: 8192 x 8192, 320 tokens (w2 320) 81.0 / 73.3, 448 tokens (448) 88.8 / 98.5; long rows also where a second, partly filled round of
+//     workgroups (two fit a CU) would take as long as the first.
+//   * cut, one tile: two groups take a run's superblocks in turn where a CU has room for both and a run is long enough to halve (K-quants: K / 128 workgroups from K = 4096 on; Q8_0,
+//     whose groups fit a CU twice: always).  One group / two: 4096 x 14336, 33 tokens 25.7 / 23.7, Q8_0 35.3 / 25.9; Q6_K 8192 x 2048, 5 tokens 11.3 / 12.0.
+static int cut_line(int type, int K) { return type == T_Q8_0 ? K / 12 : K / 20; }
+static int cut_max(int type, int NT, int K) { return NT == 2 ? (K >= 8192 ? 895 : cut_line(type, K)) : type == T_Q8_0 ? std::min(K / 8, 895) : std::max(std::min(K / 18, 400), std::min(K / 12, 256)); }
+struct WideForm { int NT, mode; bool cut; };
+// room: there is a workspace for the planes
+static WideForm wide_form(int type, int cols, int T, int K, bool room) {
+  const int S = K / 256, Cs = (S + 3) / 4, t1 = (T + 31) / 32, fill = T / t1;  // rows in a tile
+  const long long w1 = (long long)cols * t1, w2 = (long long)cols * ((T + 63) / 64);
+  const bool q8 = type == T_Q8_0, q4 = type == T_Q4_K, q5 = type == T_Q5_K, one_only = T <= 32;
+  if (S >= 4 && w1 <= 256) {
+    int line = q8 || q4 ? K / (12 + fill / 2) : K / (14 + fill / 10);
+    if (K <= 14336 && (one_only || ((t1 & 1) && (q8 || q4)))) line = std::min(line, 208);
+    if (!room || w1 >= line) return {1, !q5 && (q8 || (K > 1024 && (q4 || !one_only || K >= 4096))) ? qi::W_RUNS4 : qi::W_ONE, false};
+  }
+  if (S >= 4 && !one_only && w1 > 256 && w2 <= 256 && !q5 && K >= (q8 ? 1024 : q4 ? 2048 : 3072) && (!room || w2 >= std::min(K / 44, 208))) return {2, qi::W_RUNS2, false};
+  const bool can = room && S >= 4;
+  const bool cut1 = can && w1 <= (w1 <= 256 ? 256 : q8 ? std::min(K / 8, 895) : std::min(K / 18, 400));
+  bool cut2 = can && w2 <= cut_max(type, 2, K) && (w2 <= std::min(cut_line(type, K), 511) || w2 > 512);  // (513 .. 895: a second, partly filled round of two workgroups per CU)
+  if (q5 && w1 > 256 && w2 <= 256 && w2 >= std::min(K / 22, 208) && K <= 14336) cut2 = false;
+  const bool pair = cut1 && (q8 ? 4 * w1 <= 512 : K >= 4096 && w1 <= std::min(K / 128, 64));
+  auto time = [&](long long w, bool cut) { return cut ? Cs * ((w * ((S + Cs - 1) / Cs) + 255) / 256) : S * ((w + 255) / 256); };
+  const int ratio = cut1 ? (type == T_Q6_K ? 15 : 17) : q8 ? 18 : q5 ? 17 : 15;  // two tiles' time per superblock, in tenths of one's
+  if (one_only || (q8 && pair) || time(w1, cut1) * 10 < time(w2, cut2) * ratio) return {1, pair ? qi::W_PAIR : qi::W_ONE, cut1};
+  return {2, qi::W_ONE, cut2};
 }
 // workspace that holds the run sums of every launch over at most n rows of weights [K] and T tokens that is cut: four planes of its outputs, of which a workgroup writes at most
 // 32 NT x 128.  Never falls as T or n grow
@@ -991,17 +1000,20 @@ extern "C" size_t mrs_gemm_qi_cut_bytes(int T, int n, int K) {
   const int tiles = std::max(std::max(cut_max(T_Q8_0, 1, K), cut_max(T_Q4_K, 1, K)), 2 * std::max(cut_max(T_Q8_0, 2, K), cut_max(T_Q4_K, 2, K)));
   return (size_t)16 * std::min((size_t)T * n, (size_t)tiles * 32 * qi::WIDE_ROWS);
 }
-// 1: mrs_gemm_qi_multi over T rows, given a workspace, is cut (the launch itself asks here)
-extern "C" int mrs_gemm_qi_is_cut(int type, int nt, const int *N, int K, int T) {
+// the form of mrs_gemm_qi_multi over T rows with or without (room 0) the workspace: token tiles per wave | groups of waves << 4 | cut << 8;  is_cut: with it
+extern "C" int mrs_gemm_qi_form(int type, int nt, const int *N, int K, int T, int room) {
   if (!N || nt < 1 || nt > 3 || !qi::qi_type(type) || T <= 0 || K <= 0 || K % 256) return 0;
   int gx = 0;
+  bool r = room != 0;
   for (int i = 0; i < nt; ++i) {
-    if (N[i] <= 0 || N[i] % 4) return 0;
+    if (N[i] <= 0) return 0;
     gx += (N[i] + qi::WIDE_ROWS - 1) / qi::WIDE_ROWS;
+    r = r && N[i] % 4 == 0;  // (the planes are added four columns at a time)
   }
-  const int NT = wide_tiles(type, T, gx), wgs = gx * ((T + 32 * NT - 1) / (32 * NT));
-  return wide_cut(type, wgs, K, NT) && !wide_runs(type, wgs, K, NT);
+  const WideForm f = wide_form(type, gx, T, K, r);
+  return f.NT | qi::wide_groups(f.mode) << 4 | (f.cut ? 1 << 8 : 0);
 }
+extern "C" int mrs_gemm_qi_is_cut(int type, int nt, const int *N, int K, int T) { return mrs_gemm_qi_form(type, nt, N, K, T, 1) >> 8; }
 static int gemm_qi_launch(int type, int nt, const void *const *w_qi, const int *N, int K, const void *act, int T, float *const *out, const int *ldo, int accumulate,
                           const int *bounds, int experts, int max_rows, void *workspace, size_t workspace_bytes, bool keep_planes, void *stream) {
   if (!w_qi || !N || !act || !out || !ldo || nt < 1 || nt > 3 || !qi::qi_type(type) || T <= 0 || K <= 0 || K % 256 || (bounds && (experts <= 0 || max_rows <= 0))) return -1;
@@ -1020,14 +1032,15 @@ static int gemm_qi_launch(int type, int nt, const void *const *w_qi, const int *
   qi::QiSeg *sg[3] = {&a.s0, &a.s1, &a.s2};
   int gx = 0, x[3] = {0, 0, 0};
   for (int i = 0; i < nt; ++i) { *sg[i] = qi::QiSeg{(const uint8_t *)w_qi[i], (unsigned)qi::qi_tensor_bytes(type, N[i], K), N[i], out[i], ldo[i]}; gx += (N[i] + qi::WIDE_ROWS - 1) / qi::WIDE_ROWS; x[i] = gx; }
-  const int NT = bounds ? wide_tiles(type, std::min(T / experts, max_rows), gx * experts) : wide_tiles(type, T, gx), tl = 32 * NT;
+  bool room = workspace && workspace_bytes >= (size_t)4 * T * n_all * 4;
+  for (int i = 0; i < nt; ++i) room = room && N[i] % 4 == 0;
+  const WideForm form = bounds ? WideForm{window_tiles(type, std::min(T / experts, max_rows), gx * experts), qi::W_ONE, false} : wide_form(type, gx, T, K, room);
+  const int NT = form.NT, mode = form.mode, tl = 32 * NT;
   a.x1 = x[0]; a.x2 = nt > 1 ? x[1] : gx;
   a.K = K; a.T = T; a.qf = qf; a.yd = yd; a.bsf = bsf; a.accumulate = accumulate; a.part = (float *)workspace; a.part_n = n_all; a.bounds = bounds; a.experts = experts; a.ksplit = 1;
   // windows: every expert's last tile may be partly filled, and none has more tiles than max_rows fill
   dim3 grid(gx, bounds ? std::min(T / tl + experts, experts * ((max_rows + tl - 1) / tl)) : (T + tl - 1) / tl);
-  if (!bounds && workspace && workspace_bytes >= (size_t)4 * T * n_all * 4 && mrs_gemm_qi_is_cut(type, nt, N, K, T)) { a.ksplit = 4; grid.z = 4; }
-  const int wgs = (int)std::min<size_t>((size_t)grid.x * grid.y * grid.z, 1 << 20);
-  const int mode = a.ksplit > 1 ? (wide_pair(type, wgs, NT) ? qi::W_PAIR : qi::W_ONE) : !bounds && wide_runs(type, wgs, K, NT) ? (NT == 2 ? qi::W_RUNS2 : qi::W_RUNS4) : qi::W_ONE;
+  if (form.cut) { a.ksplit = 4; grid.z = 4; }
   switch (type) {
     case T_Q4_K: wide_launch<T_Q4_K>(NT, mode, a, grid, s); break;
     case T_Q5_K: wide_launch<T_Q5_K>(NT, mode, a, grid, s); break;

@@ -47,8 +47,8 @@ def test_cut_launches_fit_the_bytes_reserved_for_them():
                 assert not any(got) or 16 * T * sum(ns) <= room(T, sum(ns), k), (k, ns, T, got)
                 assert not any(got) or k >= 1024
     assert seen > 1000
-    assert cut(12, 1, (CI * 1)(4096), 4096, 300) == 1 and cut(13, 2, (CI * 2)(14336, 14336), 4096, 32) == 1 and cut(13, 2, (CI * 2)(14336, 14336), 4096, 33) == 0
-    assert cut(12, 1, (CI * 1)(2048), 5632, 700) == 1  # fewer rows are cut at longer prompts
+    assert cut(12, 1, (CI * 1)(4096), 4096, 100) == 1 and cut(13, 2, (CI * 2)(12288, 12288), 4096, 32) == 1 and cut(13, 2, (CI * 2)(14336, 14336), 4096, 33) == 0
+    assert cut(12, 1, (CI * 1)(1024), 8192, 700) == 1  # fewer rows are cut at longer prompts
 
 
 def test_products_that_a_cut_slows_down_stay_whole():
@@ -56,12 +56,11 @@ def test_products_that_a_cut_slows_down_stay_whole():
     cut = HostBackend().sym("mrs_gemm_qi_is_cut", [CI, CI, C.c_void_p, CI, CI], CI)
     whole = [(12, 8192, 2048, 400), (13, 2048, 2048, 2000), (14, 3072, 1024, 1000), (12, 28672, 4096, 128), (13, 28672, 4096, 100), (14, 14336, 4096, 256), (12, 28672, 8192, 128),
              (12, 8960, 1536, 300), (8, 8960, 1536, 160), (8, 3072, 1024, 512), (13, 65536, 8192, 20), (14, 65536, 8192, 32), (12, 4096, 14336, 1000)]
-    parts = [(12, 2048, 2048, 200), (13, 4096, 4096, 256), (13, 28672, 4096, 32), (14, 8192, 8192, 300), (12, 4096, 14336, 700), (14, 4096, 14336, 1600), (8, 2048, 2048, 300),
+    parts = [(12, 2048, 2048, 100), (13, 4096, 4096, 200), (13, 24576, 4096, 32), (14, 8192, 8192, 300), (12, 4096, 14336, 700), (14, 4096, 14336, 1600), (8, 2048, 2048, 128),
              (8, 8192, 8192, 300), (12, 8192, 28672, 400)]
-    # whole because a workgroup's groups of waves share the runs, and just below that line: one token tile from K / 36 (Q4_K), K / 32 (Q8_0), K / 22 (Q6_K) workgroups on, two from K / 24
-    whole += [(12, 28672, 4096, 32), (12, 14592, 4096, 32), (8, 16384, 4096, 1), (14, 23808, 4096, 20), (12, 21760, 4096, 64), (8, 4096, 4096, 512), (14, 21760, 4096, 33)]
-    parts += [(12, 14336, 4096, 32), (8, 16256, 4096, 1), (14, 23680, 4096, 20), (12, 21632, 4096, 64), (8, 21632, 4096, 33), (14, 21632, 4096, 33)]
-    whole.append((13, 3072, 1024, 100))  # 96 workgroups of one token tile, not 48 of two
+    # whole because a workgroup's groups of waves share the runs, and just below that line
+    whole += [(12, 28672, 4096, 32), (12, 18816, 4096, 32), (8, 4096, 4096, 512), (14, 26624, 4096, 20), (12, 21632, 4096, 64), (12, 2048, 2048, 200), (8, 2048, 2048, 300)]
+    parts += [(12, 18560, 4096, 32), (8, 26496, 4096, 1), (14, 26496, 4096, 20), (12, 8192, 4096, 64), (8, 8192, 4096, 33), (14, 8192, 4096, 33)]
     for case, want in [(c, 0) for c in whole] + [(c, 1) for c in parts]:
         t, n, k, T = case
         assert cut(t, 1, (CI * 1)(n), k, T) == want, case
