@@ -951,8 +951,12 @@ template <int TYPE> static void wide_launch(int NT, int mode, const qi::WideArgs
   NT == 2 ? wide_go<TYPE, 2, qi::W_ONE>(a, grid, s) : wide_go<TYPE, 1, qi::W_ONE>(a, grid, s);
 }
 // The experts' windows: token tiles per wave by the rows of an expert and the workgroup columns of all of them; always whole.  One tile fills with 32 rows; two build each operand once
-// for both, but make the chain of a superblock longer, which is what a launch that leaves most of the chip idle waits for.
-static int window_tiles(int type, int rows, int cols) { return rows <= 32 || cols * ((rows + 63) / 64) <= (type == T_Q5_K ? 96 : 32) ? 1 : 2; }
+// for both, but make the chain of a superblock longer, which is what a launch that leaves most of the chip idle waits for.  Q8_0 has no operand to build: two tiles only where one
+// expert's rows fill them, or are so many that a last tile that is half empty costs little.  One / two, gate and up of 8 experts of 14336 x 4096 Q8_0, us: 400 rows in all 268 / 247,
+// 600 328 / 398, 1024 485 / 529, 1600 658 / 750, 2400 949 / 938;  Q4_K 400 rows 217 / 181, 600 310 / 322, 1024 467 / 429, 2400 943 / 800.
+static int window_tiles(int type, int rows, int cols) {
+  return rows <= 32 || (type == T_Q8_0 && rows > 64 && rows < 256) || cols * ((rows + 63) / 64) <= (type == T_Q5_K ? 96 : 32) ? 1 : 2;
+}
 // Every other launch: token tiles per wave (NT), groups of waves per workgroup (mode), cut by runs of superblocks (cut) or whole.  The lines are drawn through the times of all seven forms
 // at 9900 sizes (512 .. 32768 rows of weights, K = 1024 .. 28672, 1 .. 2000 tokens, weights from HBM): against the fastest form of each size the one taken costs 0.1 - 0.3 % on average
 // for 1 .. 32 tokens, 0.2 - 0.4 % to 128, 0.4 - 1.0 % beyond; lines drawn through some 40 sizes whose weights lay in the last-level cache cost 1 - 8 % and were up to 1.25 times slower

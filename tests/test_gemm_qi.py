@@ -228,13 +228,14 @@ def test_gemm_qi_multi_gpu(oracle, dev, case):
     run_multi(oracle, GpuBackend(dev), *case, seed=4)
 
 
-# more than 32 workgroup columns of 128 rows: whole groups of columns and a remainder, a segment that begins inside a group, windows, a launch cut by runs
+# more than 32 workgroup columns of 128 rows: whole groups of columns and a remainder, a segment that begins inside a group, windows
 WIDE = [("Q8_0", (4224,), 256, 66, None, False, False), ("Q4_K", (4000, 200), 256, 130, None, True, False), ("Q6_K", (2176, 2176), 256, 40, (0, 33, 40), False, False),
         ("Q8_0", (4100,), 1024, 40, None, True, True),
-        # the same sizes take two token tiles per wave (K-quants; Q5_K from 97 workgroups on): remainders of a tile, empty runs, launches cut by runs, windows
+        # remainders of a tile, empty runs; windows of two token tiles per wave
         ("Q4_K", (4100, 160), 1280, 33, None, False, True), ("Q4_K", (4132,), 768, 65, None, True, False), ("Q4_K", (4224,), 512, 70, (0, 0, 64, 70), False, False),
         ("Q6_K", (4130,), 768, 33, None, False, False), ("Q6_K", (4100, 36), 1280, 40, None, True, True), ("Q5_K", (6400,), 256, 65, None, False, False),
-        ("Q5_K", (6400,), 768, 98, None, True, False), ("Q5_K", (6400,), 256, 120, (0, 64, 120), False, False)]
+        ("Q5_K", (6400,), 768, 98, None, True, False), ("Q5_K", (6400,), 256, 120, (0, 64, 120), False, False),
+        ("Q8_0", (4224,), 256, 120, (0, 64, 120), False, False), ("Q8_0", (4224,), 256, 140, (0, 71, 140), False, False)]  # two tiles, one
 
 
 @pytest.mark.parametrize("case", WIDE)
