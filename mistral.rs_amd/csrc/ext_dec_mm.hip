@@ -527,9 +527,14 @@ static int launch(const MmArgs &a0, hipStream_t s) {
   if (a.K <= 0 || a.K % 256 || a.nc < 1 || a.nc > 8 || !a.img || a.units < 1) return -1;
   const size_t lds = (lds_bytes(a.K, a.nc, a.mode) + 15) & ~(size_t)15;
   if (lds > (size_t)LDS_MAX) return -2;
+  // Workgroups.  Two fit a CU, but for the mixes with Q5_K (268 registers): those are alone on their CU, and each takes as many units as any other (one that has to wait for a second
+  // round copies an image of its own).  q / k / v of Q5_K, Q5_K, Q6_K, 8 columns, us, workgroups of 512 / of 256: 4096 15.7 / 12.3, 8192 26.1 / 22.9.
   static const int wg_per_cu = [] { const char *e = getenv("MRS_DEC_MM_WG_PER_CU"); return e ? std::max(1, atoi(e)) : 2; }();
-  const int cap = 256 * std::min<int>(wg_per_cu, std::max<size_t>(1, ((size_t)160 * 1024) / lds));
-  const int grid = std::min(a.units * (a.ids ? std::min(a.experts, a.nroutes) : 1), cap);
+  const bool q5_mix = (tmask & TM_Q5K) != 0 && tmask != TM_Q5K;
+  const int fit = std::min<int>(std::min(wg_per_cu, q5_mix ? 1 : 2), std::max<size_t>(1, ((size_t)160 * 1024) / lds));
+  const int jobs = a.units * (a.ids ? std::min(a.experts, a.nroutes) : 1);
+  const bool alone = q5_mix;
+  const int cap = alone ? 256 : 256 * fit, rounds = (jobs + cap - 1) / cap, grid = alone ? (jobs + rounds - 1) / rounds : std::min(jobs, cap);
   auto go = [&](auto kern) {
     ++g_mm_launches;
     lds_attr_once((const void *)kern, 158 * 1024);

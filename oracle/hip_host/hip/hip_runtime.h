@@ -171,7 +171,9 @@ static void run_block(const dim3 &block, const std::function<void()> &k) {
         swapcontext(&main_ctx, &fibers[t].ctx);
       }
 }
+extern "C" __attribute__((weak)) unsigned hiphost_last_launch[4] = {0, 0, 0, 0};  // grid and workgroup of the last launch, for tests
 static void launch(const dim3 &grid, const dim3 &block, size_t lds, const std::function<void()> &k) {
+  hiphost_last_launch[0] = grid.x; hiphost_last_launch[1] = grid.y; hiphost_last_launch[2] = grid.z; hiphost_last_launch[3] = block.x;
   if (lds > sizeof(dyn_lds)) abort();  // more dynamic LDS than a gfx950 workgroup can have
   dyn_lds_bytes = lds;
   gridDim = grid;

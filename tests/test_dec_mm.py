@@ -251,3 +251,21 @@ def test_the_wait_for_the_image_leaves_exactly_the_weight_ring_in_flight(tmp_pat
             if ring and wait:
                 break
         assert wait and int(wait.group(1)) == ring, (name, line, ring)
+
+
+def last_grid():
+    """workgroups of the last launch of the host build"""
+    return int((C.c_uint * 4).in_dll(HostBackend.lib(), "hiphost_last_launch")[0])
+
+
+def test_mixes_with_q5_k_have_one_workgroup_per_cu_host_emulation(oracle):
+    """Their kernels' registers admit no second one; 384 units (40 + 4 + 4 heads of 128 rows) are two for each of 192 workgroups, not a second round of 128."""
+    be = HostBackend()
+    check_mm_qkv(oracle, be, "Q5_K", "Q6_K", 40, 4, 256, 2)
+    assert last_grid() == 192
+
+
+@pytest.mark.gpu
+def test_mixes_with_q5_k_gpu(oracle, dev):
+    check_mm_qkv(oracle, GpuBackend(dev), "Q5_K", "Q6_K", 40, 4, 256, 8)
+    check_mm_qkv(oracle, GpuBackend(dev), "Q4_K", "Q5_K", 32, 8, 4096, 3)
