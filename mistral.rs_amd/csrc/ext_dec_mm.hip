@@ -57,7 +57,7 @@ __host__ __device__ inline bool mm_type(int t) { return t == T_Q4_K || t == T_Q5
 struct MmTensor { const uint8_t *w; unsigned bytes; int type, nhalves, nrows; };  // nhalves: 16-row halves of its panels
 struct MmArgs {
   MmTensor m[3];
-  int epi, nseg, units;        // a unit = 16 rows.  GLU: half panel u of m[0] (gate), then of m[1] (up); QKV: units enumerate the half panels of m[0], m[1], m[2]; else of m[0]
+  int epi, nseg, units, panels;  // panels != 0: a workgroup takes both units of a 32-row panel one after the other.  A unit = 16 rows.  GLU: half panel u of m[0] (gate), then of m[1] (up); QKV: units enumerate the half panels of m[0], m[1], m[2]; else of m[0]
   int K, nc, mode;             // activation columns (<= 8), ACT_Q8K / ACT_Q80
   const char *img; unsigned gc0p, gnp;  // the image(s) mrs_dec_act_image wrote: column c lives in the group image at act_bytes(K, gc0), gn columns wide (gc0 / gn - 1: 4 bits per column; an
                                        // array indexed by a run-time column would make hipcc copy the whole argument block to scratch memory)
@@ -190,6 +190,7 @@ __device__ __forceinline__ void where_of(int epi, int nh0, int nh1, int u, int s
   if (epi == EPI_QKV) { ti = u >= nh0 + nh1 ? 2 : (u >= nh0 ? 1 : 0); hn = u - (ti == 2 ? nh0 + nh1 : (ti == 1 ? nh0 : 0)); }
   else { ti = seg; hn = u; }
 }
+__device__ __forceinline__ int next_unit(int u, int step, int panels) { return panels && !(u & 1) ? u + 1 : u + step; }
 // The request cursor of a wave's stream: unit cu, segment cseg, superblock ct of run p, and what a request needs of them, kept between requests (scalars; where_of() and the products
 // per request were 60 scalar instructions in front of every record): the tensor, its type, the byte offset of record ct and of the unit's half of its rows.
 struct Cursor { int cu, cseg, ct, ti, type; unsigned rec, half; };
@@ -206,7 +207,7 @@ __device__ __forceinline__ void open_segment(Cursor &k, int ty0, int ty1, int ty
 // (dec_core2.cuh stream()).
 template <int NPC, int TMASK>
 __device__ __forceinline__ void issue_rec(Rec<NPC> &slot, int &m, Cursor &k, __amdgpu_buffer_rsrc_t rs0, __amdgpu_buffer_rsrc_t rs1, __amdgpu_buffer_rsrc_t rs2, int ty0, int ty1, int ty2,
-                                          int nh0, int nh1, int epi, int nseg, int units, int ntp, int p, int Cs, int S, int lane, int step, int pn0) {
+                                          int nh0, int nh1, int epi, int nseg, int units, int ntp, int p, int Cs, int S, int lane, int step, int panels, int pn0) {
   constexpr unsigned DEAD = 0xF0000000u;  // beyond every tensor, whatever the scalar offset; + a piece's offset: no wrap
   constexpr bool ONLY4 = TMASK == TM_Q4K, HAS4 = (TMASK & TM_Q4K) != 0;
   const bool live = k.cu < units && ntp > 0, two = k.ct + 1 < ntp, small = ONLY4 || (HAS4 && k.type == T_Q4_K), hi = lane >= 32;
@@ -226,7 +227,7 @@ __device__ __forceinline__ void issue_rec(Rec<NPC> &slot, int &m, Cursor &k, __a
   if (live) {  // scalar bookkeeping only
     k.ct += 2; k.rec += 2u * rb;
     if (k.ct >= ntp) {
-      if (++k.cseg == nseg) { k.cseg = 0; k.cu += step; }
+      if (++k.cseg == nseg) { k.cseg = 0; k.cu = next_unit(k.cu, step, panels); }
       open_segment(k, ty0, ty1, ty2, nh0, nh1, epi, units, p, Cs, S, pn0);
     }
   }
@@ -302,6 +303,8 @@ __device__ __forceinline__ void dec_mm_body(const MmArgs &a, char *smem) {
   const int hf = (lane >> 4) & 1;  // the lane's half of k, and of the tokens of a result
   const int K = a.K, S = K / 256, Cs = (S + 3) / 4, Sp = 4 * Cs, CQ = act_cq(K), QCS = qcs_of(K);
   int nc = a.nc, unit0 = (int)blockIdx.x, ustep = (int)gridDim.x, pn0 = 0;
+  const int panels = MOE ? 0 : a.panels;
+  if (panels) { unit0 *= 2; ustep = 2 * ustep - 1; }
   unsigned long long routes = 0, rows = 0;  // MOE: output and image row of the columns, a byte each
   if constexpr (MOE) {  // (every wave finds the same: scalar values)
     const int id = lane < a.nroutes ? (int)a.ids[lane] : -1;
@@ -348,7 +351,7 @@ __device__ __forceinline__ void dec_mm_body(const MmArgs &a, char *smem) {
   // (issue_rec / where_of are plain functions: as by-reference closures of the kernel their selects between captured variables -- which tensor's resource, type, panel
   // count -- became run-time offsets INTO the closure object, which then could not be dissolved: every local of the kernel lived in scratch memory)
   auto issue = [&](Rec<NPC> &slot, int &m) __attribute__((always_inline)) {
-    issue_rec<NPC, TMASK>(slot, m, cur, rs0, rs1, rs2, ty0, ty1, ty2, nh0, nh1, epi, nseg, units, ntp, p, Cs, S, lane, ustep, pn0);
+    issue_rec<NPC, TMASK>(slot, m, cur, rs0, rs1, rs2, ty0, ty1, ty2, nh0, nh1, epi, nseg, units, ntp, p, Cs, S, lane, ustep, panels, pn0);
   };
   MRS_MM_TL(0);
   // ---- the activation image -> LDS (every workgroup), requested BEFORE the weight ring: it comes out of the L2 while the weights are on their way
@@ -433,7 +436,7 @@ __device__ __forceinline__ void dec_mm_body(const MmArgs &a, char *smem) {
   int eu = unit0, eseg = 0, par = 0;  // the (unit, segment) whose run sums are being collected
   auto finish = [&]() __attribute__((always_inline)) {
     finish_unit<MOE>(a, ex, par, eu, eseg, tid, gsave, nc, routes);
-    if (++eseg == nseg) { eseg = 0; eu += ustep; }
+    if (++eseg == nseg) { eseg = 0; eu = next_unit(eu, ustep, panels); }
     par ^= 1;
   };
   auto publish = [&](const float (&v)[4]) __attribute__((always_inline)) {  // this wave's run sums of the finished (unit, segment) -> ex[par][p][token][row]
@@ -527,14 +530,18 @@ static int launch(const MmArgs &a0, hipStream_t s) {
   if (a.K <= 0 || a.K % 256 || a.nc < 1 || a.nc > 8 || !a.img || a.units < 1) return -1;
   const size_t lds = (lds_bytes(a.K, a.nc, a.mode) + 15) & ~(size_t)15;
   if (lds > (size_t)LDS_MAX) return -2;
-  // Workgroups.  Two fit a CU, but for the mixes with Q5_K (268 registers): those are alone on their CU, and each takes as many units as any other (one that has to wait for a second
-  // round copies an image of its own).  q / k / v of Q5_K, Q5_K, Q6_K, 8 columns, us, workgroups of 512 / of 256: 4096 15.7 / 12.3, 8192 26.1 / 22.9.
+  // Workgroups.  Two fit a CU, but for the mixes with Q5_K (268 registers).  Of those that copy the image and stream alone on their CU, each takes as many units as any other:
+  //   * the mixes with Q5_K (a workgroup that has to wait for a second round copies an image of its own): q / k / v of Q5_K, Q5_K, Q6_K, 8 columns, us, workgroups of 512 / of 256:
+  //     4096 15.7 / 12.3, 8192 26.1 / 22.9.
+  //   * from 2000 units (lm_head) on, both units of a panel one after the other: pieces of 512 consecutive bytes again.  Units as they come / so, 128256 x 4096 Q6_K 94.1 / 90.1, Q8_0
+  //     95.0 / 88.3, Q5_K 94.7 / 89.9, Q4_K (two workgroups per CU) 57.4 / 54.9, 32000 x 4096 Q6_K 27.8 / 27.8;  units of 32 rows 93.0, 90.9, 93.1, 54.7, 27.5.
   static const int wg_per_cu = [] { const char *e = getenv("MRS_DEC_MM_WG_PER_CU"); return e ? std::max(1, atoi(e)) : 2; }();
-  const bool q5_mix = (tmask & TM_Q5K) != 0 && tmask != TM_Q5K;
+  const bool q5_mix = (tmask & TM_Q5K) != 0 && tmask != TM_Q5K, large = (tmask & TM_Q4K) == 0;
   const int fit = std::min<int>(std::min(wg_per_cu, q5_mix ? 1 : 2), std::max<size_t>(1, ((size_t)160 * 1024) / lds));
-  const int jobs = a.units * (a.ids ? std::min(a.experts, a.nroutes) : 1);
-  const bool alone = q5_mix;
-  const int cap = alone ? 256 : 256 * fit, rounds = (jobs + cap - 1) / cap, grid = alone ? (jobs + rounds - 1) / rounds : std::min(jobs, cap);
+  a.panels = !a.ids && a.units >= 2000 && a.units % 2 == 0;
+  const int jobs = a.panels ? a.units / 2 : a.units * (a.ids ? std::min(a.experts, a.nroutes) : 1);
+  const bool alone = q5_mix || (a.panels && large);
+  const int cap = alone ? 256 : 256 * fit, rounds = (jobs + cap - 1) / cap, grid = alone || a.panels ? (jobs + rounds - 1) / rounds : std::min(jobs, cap);
   auto go = [&](auto kern) {
     ++g_mm_launches;
     lds_attr_once((const void *)kern, 158 * 1024);

@@ -269,3 +269,21 @@ def test_mixes_with_q5_k_have_one_workgroup_per_cu_host_emulation(oracle):
 def test_mixes_with_q5_k_gpu(oracle, dev):
     check_mm_qkv(oracle, GpuBackend(dev), "Q5_K", "Q6_K", 40, 4, 256, 8)
     check_mm_qkv(oracle, GpuBackend(dev), "Q4_K", "Q5_K", 32, 8, 4096, 3)
+
+
+# 1001 panels, the last one of 20 rows: both units of one belong to a workgroup; 1000 and one on the last
+@pytest.mark.parametrize("tname,grid", [("Q6_K", 251), ("Q4_K", 501)])
+def test_mm_panels_stay_together_in_long_launches_host_emulation(oracle, tname, grid):
+    check_mm_proj(oracle, HostBackend(), tname, 32020, 256, 2, False, mode=0)
+    assert last_grid() == grid
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("tname,n,k,b", [("Q4_K", 32020, 256, 8), ("Q5_K", 32020, 512, 3), ("Q6_K", 32052, 1024, 8), ("Q8_0", 65536, 1280, 5), ("Q6_K", 128256, 2048, 3)])
+def test_mm_panels_stay_together_in_long_launches_gpu(oracle, dev, tname, n, k, b):
+    check_mm_proj(oracle, GpuBackend(dev), tname, n, k, b, False, mode=0)
+
+
+@pytest.mark.gpu
+def test_mm_gate_up_of_long_launches_gpu(oracle, dev):
+    check_mm_gate_up(oracle, GpuBackend(dev), "Q4_K", 32020, 512, 4)
