@@ -118,6 +118,9 @@ __device__ __forceinline__ void term(const Rec<NPC> &w, Ops &o, Next next, const
   if constexpr (TYPE == T_Q8_0) {
     // block g: 32 int8 of the weight row x 32 int8 of the token; p_g = ((float)isum dw_g) dx_g, T = p_0 + p_1 + ... left to right (Tile<T_Q8_0>)
     i4v d[8];
+    float4 y4[8];  // read in front of the next record's operands: LDS answers in order
+#pragma unroll
+    for (int g = 0; g < 8; ++g) y4[g] = *(const float4 *)(ydp + (g * 8 + 4 * hf) * 4);
 #pragma unroll
     for (int g = 0; g < 8; ++g) d[g] = __builtin_amdgcn_mfma_i32_16x16x64_i8(mk_i4(o.A[2 * g], o.A[2 * g + 1]), __builtin_bit_cast(i4v, w.q[g % NPC]), zero, 0, 0, 0);
     __builtin_amdgcn_sched_barrier(0);
@@ -127,8 +130,7 @@ __device__ __forceinline__ void term(const Rec<NPC> &w, Ops &o, Next next, const
     for (int g = 0; g < 8; ++g) {
       const unsigned hw = w.hs[g >> 1];
       const float dwg = half_bits_to_float((uint16_t)((g & 1) ? (hw >> 16) : (hw & 0xffffu)));
-      const float4 y4 = *(const float4 *)(ydp + (g * 8 + 4 * hf) * 4);
-      const float yy[4] = {y4.x, y4.y, y4.z, y4.w};
+      const float yy[4] = {y4[g].x, y4[g].y, y4[g].z, y4[g].w};
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         const float p = ((float)d[g][i] * dwg) * yy[i];
@@ -531,8 +533,9 @@ static int launch(const MmArgs &a0, hipStream_t s) {
   const size_t lds = (lds_bytes(a.K, a.nc, a.mode) + 15) & ~(size_t)15;
   if (lds > (size_t)LDS_MAX) return -2;
   // Workgroups.  Two fit a CU, but for the mixes with Q5_K (268 registers).  Of those that copy the image and stream alone on their CU, each takes as many units as any other:
-  //   * the mixes with Q5_K (a workgroup that has to wait for a second round copies an image of its own): q / k / v of Q5_K, Q5_K, Q6_K, 8 columns, us, workgroups of 512 / of 256:
-  //     4096 15.7 / 12.3, 8192 26.1 / 22.9.
+  //   * the mixes with Q5_K, and 321 .. 512 units of the large records (a workgroup per unit would put two images on half the CUs and one on the others; Q4_K's records beside them:
+  //     from 385), and projections beyond.  us, 8 columns, workgroups of 512 / of 256: q / k / v of Q5_K, Q5_K, Q6_K at 4096 15.7 / 12.3, Q6_K 12.5 / 12.1, Q8_0 12.9 / 12.6;
+  //     8192 x 4096 Q6_K 12.7 / 11.8, Q8_0 13.1 / 11.8.  Not 256 of 3072 (288 units, Q8_0) 11.5 / 11.9, gate and up of 18944 x 3584 Q8_0 28.1 / 31.0, Q4_K 10240 x 5120 12.4 / 13.0.
   //   * from 2000 units (lm_head) on, both units of a panel one after the other: pieces of 512 consecutive bytes again.  Units as they come / so, 128256 x 4096 Q6_K 94.1 / 90.1, Q8_0
   //     95.0 / 88.3, Q5_K 94.7 / 89.9, Q4_K (two workgroups per CU) 57.4 / 54.9, 32000 x 4096 Q6_K 27.8 / 27.8;  units of 32 rows 93.0, 90.9, 93.1, 54.7, 27.5.
   static const int wg_per_cu = [] { const char *e = getenv("MRS_DEC_MM_WG_PER_CU"); return e ? std::max(1, atoi(e)) : 2; }();
@@ -540,8 +543,8 @@ static int launch(const MmArgs &a0, hipStream_t s) {
   const int fit = std::min<int>(std::min(wg_per_cu, q5_mix ? 1 : 2), std::max<size_t>(1, ((size_t)160 * 1024) / lds));
   a.panels = !a.ids && a.units >= 2000 && a.units % 2 == 0;
   const int jobs = a.panels ? a.units / 2 : a.units * (a.ids ? std::min(a.experts, a.nroutes) : 1);
-  const bool alone = q5_mix || (a.panels && large);
-  const int cap = alone ? 256 : 256 * fit, rounds = (jobs + cap - 1) / cap, grid = alone || a.panels ? (jobs + rounds - 1) / rounds : std::min(jobs, cap);
+  const bool alone = fit == 1 || (!a.ids && (a.panels ? large : a.epi != EPI_GLU && (large ? a.units > 320 && (a.units <= 512 || a.epi != EPI_QKV) : tmask != TM_Q4K && a.units > 384 && a.units <= 512)));
+  const int cap = alone ? 256 : 256 * fit, rounds = (jobs + cap - 1) / cap, grid = (alone || a.panels) && !a.ids ? (jobs + rounds - 1) / rounds : std::min(jobs, cap);
   auto go = [&](auto kern) {
     ++g_mm_launches;
     lds_attr_once((const void *)kern, 158 * 1024);

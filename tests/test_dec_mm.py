@@ -279,7 +279,7 @@ def test_mm_panels_stay_together_in_long_launches_host_emulation(oracle, tname, 
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("tname,n,k,b", [("Q4_K", 32020, 256, 8), ("Q5_K", 32020, 512, 3), ("Q6_K", 32052, 1024, 8), ("Q8_0", 65536, 1280, 5), ("Q6_K", 128256, 2048, 3)])
+@pytest.mark.parametrize("tname,n,k,b", [("Q4_K", 32020, 256, 8), ("Q5_K", 32020, 512, 3), ("Q6_K", 32052, 1024, 8), ("Q8_0", 49168, 768, 5)])
 def test_mm_panels_stay_together_in_long_launches_gpu(oracle, dev, tname, n, k, b):
     check_mm_proj(oracle, GpuBackend(dev), tname, n, k, b, False, mode=0)
 
@@ -287,3 +287,19 @@ def test_mm_panels_stay_together_in_long_launches_gpu(oracle, dev, tname, n, k, 
 @pytest.mark.gpu
 def test_mm_gate_up_of_long_launches_gpu(oracle, dev):
     check_mm_gate_up(oracle, GpuBackend(dev), "Q4_K", 32020, 512, 4)
+
+
+def test_units_of_large_records_are_dealt_evenly_host_emulation(oracle):
+    """Between one and two units per CU: 384 units of Q8_0 are two for each of 192 workgroups; 288 of them, and Q4_K's smaller records, a workgroup each."""
+    be = HostBackend()
+    for tname, heads, grid in (("Q8_0", 40, 192), ("Q8_0", 28, 288), ("Q4_K", 40, 384)):
+        check_mm_qkv(oracle, be, tname, tname, heads, 4, 256, 2)
+        assert last_grid() == grid, (tname, heads)
+    check_mm_proj(oracle, be, "Q6_K", 10256, 256, 1, False)  # 642 units: three each
+    assert last_grid() == 214
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("tname,n,k,b", [("Q8_0", 8192, 4096, 8), ("Q6_K", 10256, 1280, 3), ("Q5_K", 16384, 1024, 5)])
+def test_units_of_large_records_are_dealt_evenly_gpu(oracle, dev, tname, n, k, b):
+    check_mm_proj(oracle, GpuBackend(dev), tname, n, k, b, False)
