@@ -858,7 +858,7 @@ extern "C" int mrs_dec_gate_up_img(const mrs_dec_mat_c *wg, const mrs_dec_mat_c 
   return Launch<EPI_GLU>::run(a, b, (hipStream_t)stream);
 }
 
-// Decode attention of the engine, one launch (dec_attn4_kernel: four and eight heads per key head; dec_attn2_kernel: one and two).  out_f32 [b][num_heads * 128] (may be NULL when an image is written);
+// Decode attention of the engine, one launch (dec_attn4_kernel: four and eight heads per key head; dec_attn2_kernel: one and two, and eight of up to four (sequence, key head) pairs).  out_f32 [b][num_heads * 128] (may be NULL when an image is written);
 // img_out: Q8_K activation image for mrs_dec_proj_img (written when the GQA group is even; may be NULL); ticket: [b * num_kv_heads] u32, zero
 // before the first call (the kernel leaves it zero); part_*: the partials workspace of mrs_decode_attention_f32_*.  Returns 1 when the image
 // was written, 0 when only out_f32 was, < 0 on a shape outside the kernel (head size 128, 32-token pages, GQA group 1 / 2 / 4 / 8).
@@ -915,7 +915,11 @@ extern "C" int mrs_dec_attention(float *out_f32, void *img_out, unsigned *ticket
     }                                                                                                                    \
     if (!one_launch) hipLaunchKernelGGL((dec_attn2_merge_kernel<GG>), mgrid, dim3(64 * ((GG + 1) / 2)), 0, s, a);            \
   } while (0)
-#define MRS_A2G(CT) switch (G) { case 1: MRS_A2(1, CT); break; case 2: MRS_A2(2, CT); break; case 4: MRS_A4(4, CT); break; default: MRS_A4(8, CT); break; }
+  // Eight heads of few (sequence, key head) pairs: a wave's two groups of four heads are two chains where eight waves have one each, and the chip is empty enough for these.  A wave per
+  // head / four heads per wave, us per launch in a captured step, caches evicted, contexts of 513, 2000, 7002: 1 pair 10.1, 14.1, 19.1 / 11.1, 15.4, 19.7, 4 pairs 10.4, 16.4, 21.4 /
+  // 11.1, 16.2, 23.3; 6 pairs 10.9, 18.0, 28.5 / 11.4, 17.2, 26.5, 8 pairs 11.4, 19.5, 28.9 / 11.5, 18.1, 27.6, 16 pairs 13.7, 26.8, 45.4 / 12.6, 22.9, 35.3.
+  const bool few = num_kv_heads * num_seqs <= 4;
+#define MRS_A2G(CT) switch (G) { case 1: MRS_A2(1, CT); break; case 2: MRS_A2(2, CT); break; case 4: MRS_A4(4, CT); break; default: if (few) MRS_A2(8, CT); else MRS_A4(8, CT); break; }
   if (kv_dtype == 1) { MRS_A2G(bf16_t) } else { MRS_A2G(f16_t) }
 #undef MRS_A2G
 #undef MRS_A4

@@ -413,6 +413,7 @@ def check_attention(O, be, heads, kvh, ctxs, max_ctx, kv_dtype=1, n_out=24, wind
                 hd * bs, kv_dtype, window, be.stream)
         assert rc == (1 if even else 0)
         assert not ticket.numpy().any()
+    threads = int((C.c_uint * 4).in_dll(HostBackend.lib(), "hiphost_last_launch")[3]) if isinstance(be, HostBackend) else None
     res = got.numpy()
     nblk_max = (max_ctx + 31) // 32
     bpw = 1 if nblk_max <= 64 else (nblk_max + 63) // 64
@@ -424,7 +425,7 @@ def check_attention(O, be, heads, kvh, ctxs, max_ctx, kv_dtype=1, n_out=24, wind
         cpu = O.attention_single_q_cpu(q_np[i].reshape(heads, hd), k[lo:], v[lo:], scale, 1)
         assert np.abs(res[i].reshape(heads, hd) - cpu).max() <= 2e-6 * max(1.0, np.abs(cpu).max()), ("single_q.rs order", i, ctx)
     if not even:
-        return
+        return threads
     # o_proj on the image == o_proj on the f32 vector (the same quantizer ran in a different kernel)
     t = O.Q4_K
     packed = _weights(O, t, n_out, nq, 7)
@@ -436,6 +437,7 @@ def check_attention(O, be, heads, kvh, ctxs, max_ctx, kv_dtype=1, n_out=24, wind
     np.testing.assert_array_equal(o_img.numpy(), o_ref.numpy())
     eng_o = base * np.float32(0.5) + np.concatenate([O.gemv_engine(t, packed, n_out, nq, r) for r in res], axis=0) * np.float32(1.0)
     np.testing.assert_array_equal(o_img.numpy(), eng_o)
+    return threads
 
 
 @pytest.mark.parametrize("heads,kvh,ctxs,max_ctx,kvd", [(4, 2, [70], 128, 1), (4, 1, [33, 200], 224, 1), (2, 1, [1], 64, 0), (8, 2, [500, 17, 96], 512, 1)])
@@ -475,6 +477,22 @@ def test_attention_splits_of_more_than_four_blocks_host_emulation(oracle, heads,
 @pytest.mark.gpu
 @pytest.mark.parametrize("heads,kvh,ctxs,max_ctx,kvd,window", GROUPS + [(32, 8, [9001, 2000], 9024, 1, 0), (64, 8, [9001, 160], 9024, 1, 4000)])
 def test_attention_splits_of_more_than_four_blocks_gpu(oracle, dev, heads, kvh, ctxs, max_ctx, kvd, window):
+    check_attention(oracle, GpuBackend(dev), heads, kvh, ctxs, max_ctx, kvd, n_out=256, window=window, nan_past=True)
+
+
+# eight heads per key head: a wave per head up to four (sequence, key head) pairs, four heads per wave beyond; splits of one, four, eight and nine blocks
+EIGHT = [(8, 1, [100, 31, 64, 33], 128, 0, 0, 512), (8, 1, [100, 31, 64, 33, 1], 128, 0, 0, 256), (16, 2, [257, 40], 8192, 1, 0, 512), (8, 1, [257, 31, 130, 33, 1], 8192, 1, 100, 256),
+         (8, 1, [513, 40, 1, 100, 260], 16384, 1, 0, 256), (40, 5, [330], 18400, 0, 300, 256)]
+
+
+@pytest.mark.parametrize("heads,kvh,ctxs,max_ctx,kvd,window,threads", EIGHT)
+def test_attention_of_eight_heads_host_emulation(oracle, heads, kvh, ctxs, max_ctx, kvd, window, threads):
+    assert check_attention(oracle, HostBackend(), heads, kvh, ctxs, max_ctx, kvd, window=window, nan_past=True) == threads
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("heads,kvh,ctxs,max_ctx,kvd,window,threads", EIGHT + [(16, 2, [2047, 700], 2048, 1, 0, 512), (32, 4, [9001], 9024, 1, 0, 512), (64, 8, [2047, 700], 2048, 1, 0, 256)])
+def test_attention_of_eight_heads_gpu(oracle, dev, heads, kvh, ctxs, max_ctx, kvd, window, threads):
     check_attention(oracle, GpuBackend(dev), heads, kvh, ctxs, max_ctx, kvd, n_out=256, window=window, nan_past=True)
 
 
