@@ -884,16 +884,18 @@ extern "C" int mrs_qi_quantize_for(int w_type, const float *x, const float *x2, 
 extern "C" int mrs_qi_quantize(const float *x, const float *x2, int ldx, const float *norm_w, float eps, int T, int K, void *act, float *xtmp, void *stream) {
   return mrs_qi_quantize_for(T_Q4_K, x, x2, ldx, norm_w, eps, T, K, act, xtmp, stream);
 }
+static size_t row_image_lds(int K) { return (dec2::act_bytes(K, 1) + 15) & ~(size_t)15; }
+constexpr size_t ROW_IMAGE_MAX = (size_t)158 * 1024;
 template <bool GLU, bool PART> static int qi_quantize_rows(const qi::QuantArgs &a, void *stream) {  // rows with a norm
-  const size_t lds = (dec2::act_bytes(a.K, 1) + 15) & ~(size_t)15;
-  if (lds > 158 * 1024) return -2;
+  const size_t lds = row_image_lds(a.K);
   auto kern = qi::qi_quantize_kernel<GLU, PART>;
-  lds_attr_once((const void *)kern, 158 * 1024);
+  lds_attr_once((const void *)kern, ROW_IMAGE_MAX);
   hipLaunchKernelGGL(kern, dim3(a.T), dim3(dec2::NT), lds, (hipStream_t)stream, a);
   return 0;
 }
 extern "C" int mrs_qi_quantize_for(int w_type, const float *x, const float *x2, int ldx, const float *norm_w, float eps, int T, int K, void *act, float *xtmp, void *stream) {
   if (!x || !act || T <= 0 || K <= 0 || K % 256 || (x2 && !xtmp) || !qi::qi_type(w_type)) return -1;
+  if (row_image_lds(K) > ROW_IMAGE_MAX) return -2;  // with a norm or without
   qi::QuantArgs a{};
   a.x = x; a.x2 = x2; a.ldx = ldx; a.norm_w = norm_w; a.eps = eps; a.K = K; a.T = T; a.xtmp = xtmp; a.mode = dec2::act_mode_for(w_type);
   qi_split(act, T, K, &a.qf, &a.yd, &a.bsf);

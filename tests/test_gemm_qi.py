@@ -501,6 +501,19 @@ def test_gemm_qi_q8_0_odd_scales_gpu(oracle, dev, T, n, k):
     run_odd_scales(oracle, GpuBackend(dev), T, n, k)
 
 
+def test_rows_beyond_an_image_are_refused_host_emulation(oracle):
+    """A row whose image does not fit LDS (from some 108000 values on) is refused with a norm and without, and nothing is written."""
+    be = HostBackend()
+    quantize = be.sym("mrs_qi_quantize_for", [CI, VP, VP, CI, VP, C.c_float, CI, CI, VP, VP, VP], CI)
+    k = 131072
+    x, act = be.buf(np.ones(k, np.float32)), be.buf(np.full(be.sym("mrs_qi_act_bytes", [CI, CI], C.c_size_t)(1, k), 0xA5, np.uint8))
+    for t in (oracle.Q4_K, oracle.Q8_0):
+        for norm in (None, x.ptr):
+            assert quantize(t, x.ptr, None, k, norm, 1e-5, 1, k, act.ptr, None, be.stream) == -2
+        assert quantize(t, x.ptr, x.ptr, k, None, 1e-5, 1, k, act.ptr, x.ptr, be.stream) == -2
+    assert (act.numpy() == 0xA5).all()
+
+
 def run_added_rows(O, be, tname, T, d, k):
     """h + a cut product by its run sums and the quantizer that adds them (mrs_gemm_qi_multi_planes, mrs_qi_quantize_added) == the accumulating product and the quantizer of h."""
     t = getattr(O, tname)
