@@ -1742,7 +1742,8 @@ __global__ void __launch_bounds__(256, 4) prefill_values_kernel(const dec::AttnA
     advance(b2, in2);
   };
   auto third = [&]() { int b3 = b2, in3 = in2; advance(b3, in3); return b3; };
-  const int steps = ONE ? rounds : rounds * bpw;  // of every wave: the barriers are met by all
+  // of every wave: the barriers are met by all.  A last round of one short split ends with its blocks: nothing is added behind it
+  const int steps = ONE ? rounds : (rounds - 1) * bpw + min(bpw, nblk - (rounds - 1) * G * bpw);
   for (int k = 0, rd = 0, in = 0; k < steps; k += 2) {
     load(min(b1, nblk - 1), id1, r1);
     id1 = id_of(third());
@@ -1824,8 +1825,10 @@ extern "C" int mrs_prefill_attention_exact_ws(const float *q, const void *k_cach
           using namespace mrs::qi;
           // groups of splits: as many as leave a CU per workgroup.  Scores and values of 32 heads, us, 1 / 2 / 4 groups: 64 pairs, 37 tokens at 300 19.0 / 16.4 / 13.8, 33 at 1900
           // 69 / 53 / 41, 37 at 3000 107 / 77 / 56; 128 pairs, 100 tokens 13.1 / 12.1 / 12.2, 64 of 64 heads at 100 15.1 / 13.3 / 14.0; 224 pairs, 200 tokens at 100
-          // 26.0 / 26.4 / 26.5; 512 pairs, 512 tokens 41.1 / 42.9 / 45.5
-          const int pairs = w.heads * nt, groups = pairs <= 64 ? 4 : pairs <= 128 ? 2 : 1;
+          // 26.0 / 26.4 / 26.5; 512 pairs, 512 tokens 41.1 / 42.9 / 45.5.  No group without a split
+          const int pairs = w.heads * nt;
+          int groups = pairs <= 64 ? 4 : pairs <= 128 ? 2 : 1;
+          while (groups / 2 >= splits) groups /= 2;
           auto go = [&](auto scores, auto values, int g) {
             hipLaunchKernelGGL(scores, gs, dim3(256), 0, (hipStream_t)stream, a, w);
             hipLaunchKernelGGL(values, dim3(w.heads, nt, g), dim3(256), pv_lds(g), (hipStream_t)stream, a, w);

@@ -62,6 +62,8 @@ def test_prompt_attention_equals_decode_attention_gpu(oracle, dev, heads, kvh, T
 # groups of heads, groups of query tiles; up to 64 / 128 / more pairs per launch (the split groups of the values kernel: 4, 2, 1), the last round of groups short
 WS = [(4, 1, 40, 64, 1, 0, 0, 99), (4, 2, 70, 128, 0, 0, 0, 7), (2, 2, 33, 96, 1, 0, 20, 1), (8, 2, 50, 4096, 1, 0, 200, 99), (4, 1, 90, 128, 1, 40, 0, 2), (3, 3, 1, 2304, 0, 0, 130, 99),
       (2, 2, 3, 512, 1, 0, 190, 99), (48, 48, 40, 128, 1, 0, 40, 99), (72, 9, 40, 128, 0, 0, 0, 999), (40, 5, 33, 4096, 1, 0, 80, 99)]
+# four blocks per split: contexts of one block, of one short split, of two, three and five splits (the last round: one short split) and the groups of the values kernel that these leave
+FEW = [((2, 1, 1, 8192, 1, 0, 0, 99), 1), ((2, 2, 33, 8192, 0, 0, 50, 99), 1), ((2, 2, 40, 8192, 1, 0, 110, 99), 2), ((3, 3, 20, 8192, 1, 0, 300, 99), 4), ((2, 1, 10, 8192, 0, 0, 520, 99), 4)]
 
 
 def check_attention_ws(O, be, heads, kvh, T, max_ctx, kv_dtype, window, start, pairs):
@@ -94,8 +96,15 @@ def test_prompt_attention_with_a_workspace_host_emulation(oracle, case):
     check_attention_ws(oracle, HostBackend(), *case)
 
 
+@pytest.mark.parametrize("case,groups", FEW)
+def test_prompt_attention_of_few_splits_host_emulation(oracle, case, groups):
+    be = HostBackend()
+    check_attention_ws(oracle, be, *case)
+    assert (C.c_uint * 4).in_dll(HostBackend.lib(), "hiphost_last_launch")[2] == groups  # no group without a split
+
+
 @pytest.mark.gpu
-@pytest.mark.parametrize("case", WS[:3] + WS[4:] + [(32, 8, 512, 1024, 1, 0, 0, 9999), (8, 2, 300, 4096, 1, 0, 1000, 40), (32, 8, 700, 832, 0, 256, 0, 50), (64, 8, 1100, 2304, 1, 0, 0, 9999)])
+@pytest.mark.parametrize("case", WS[:3] + WS[4:] + [c for c, _ in FEW] + [(32, 8, 512, 1024, 1, 0, 0, 9999), (8, 2, 300, 4096, 1, 0, 1000, 40), (32, 8, 700, 832, 0, 256, 0, 50), (64, 8, 1100, 2304, 1, 0, 0, 9999)])
 def test_prompt_attention_with_a_workspace_gpu(oracle, dev, case):
     check_attention_ws(oracle, GpuBackend(dev), *case)
 
