@@ -688,11 +688,12 @@ __global__ void __launch_bounds__(1024) moe_router_kernel(const float *__restric
 #ifndef MRS_WAIT_VMCNT0
 #define MRS_WAIT_VMCNT0() asm volatile("s_waitcnt vmcnt(0)" ::: "memory")
 #endif
-// What bounds it is the chain of latencies, so the row, the norm's weights and the expert's row are requested at once (ROUTER_R float4 per thread / lane in registers; longer rows load the
-// rest where they need it), and the last arriver's wave reads the logits from lanes instead of LDS and takes all exponentials at once, in the serial code's order of comparisons and
-// additions.  us per launch, one token, 8 experts of 4096 values,
-// weights from HBM, loads where they are used and one lane's softmax / this: 8.5 / 6.6.
+// What bounds it is the chain of latencies, so the row, the norm's weights and the expert's row are requested at once (R float4 per thread / lane in registers), and the last arriver's
+// wave reads the logits from lanes instead of LDS and takes all exponentials at once, in the serial code's order of comparisons and additions.  us per launch, one token, 8 experts of
+// 4096 values, weights from HBM, loads where they are used and one lane's softmax / this: 7.7 / 6.8.  Rows that do not fit the registers (more than 64 R float4: R = 0) are loaded where
+// they are used, the expert's row eight at a time; with the registers in front of such loops 12288 values took 11.2 - 12.7 us, without 9.7 (6144: 8.2 - 9.3 and 7.6).
 constexpr int ROUTER_R = 16;
+template <int R>
 __global__ void __launch_bounds__(256) moe_router_split_kernel(const float *__restrict__ x, const float *__restrict__ gate_w, int E, int K, int top_k, int renormalize,
                                                                int32_t *__restrict__ ids, float *__restrict__ weights, const float *__restrict__ norm_w, float eps,
                                                                float *__restrict__ scratch) {
@@ -702,39 +703,50 @@ __global__ void __launch_bounds__(256) moe_router_split_kernel(const float *__re
   const float *xr = x + (size_t)tok * K, *wr = gate_w + (size_t)e * K;
   float *xn = (float *)xn_s;
   const int nvec = K / 4;
-  float4 xv[ROUTER_R / 4], nv[ROUTER_R / 4], gv[ROUTER_R];
-  if (nvec > 0) {
+  constexpr int RA = R ? R : 4;
+  float4 xv[RA / 4], nv[RA / 4], gv[RA];
+  if (R && nvec > 0) {
 #pragma unroll
-    for (int u = 0; u < ROUTER_R / 4; ++u) xv[u] = *(const float4 *)(xr + 4 * min(tid + 256 * u, nvec - 1));
+    for (int u = 0; u < R / 4; ++u) xv[u] = *(const float4 *)(xr + 4 * min(tid + 256 * u, nvec - 1));
 #pragma unroll
-    for (int u = 0; u < ROUTER_R / 4; ++u) nv[u] = *(const float4 *)(norm_w + 4 * min(tid + 256 * u, nvec - 1));
+    for (int u = 0; u < R / 4; ++u) nv[u] = *(const float4 *)(norm_w + 4 * min(tid + 256 * u, nvec - 1));
     if (wave == 0) {
 #pragma unroll
-      for (int u = 0; u < ROUTER_R; ++u) gv[u] = *(const float4 *)(wr + 4 * min(lane + 64 * u, nvec - 1));
+      for (int u = 0; u < R; ++u) gv[u] = *(const float4 *)(wr + 4 * min(lane + 64 * u, nvec - 1));
     }
   }
   float sum = 0.f;
   auto square = [&](const float4 &t) { sum = fmaf(t.x, t.x, sum); sum = fmaf(t.y, t.y, sum); sum = fmaf(t.z, t.z, sum); sum = fmaf(t.w, t.w, sum); };
+  if constexpr (R > 0) {
 #pragma unroll
-  for (int u = 0; u < ROUTER_R / 4; ++u) if (tid + 256 * u < nvec) square(xv[u]);
-  for (int v = tid + 64 * ROUTER_R; v < nvec; v += 256) square(*(const float4 *)(xr + 4 * v));
+    for (int u = 0; u < R / 4; ++u) if (tid + 256 * u < nvec) square(xv[u]);
+  } else {
+    for (int v = tid; v < nvec; v += 256) square(*(const float4 *)(xr + 4 * v));
+  }
   sum = wave_sum(sum);
   if (lane == 0) red[wave] = sum;
   __syncthreads();
   const float inv = rsqrtf((red[0] + red[1] + red[2] + red[3]) / (float)K + eps);
   auto normed = [&](const float4 &t, const float4 &w) { return make_float4(t.x * inv * w.x, t.y * inv * w.y, t.z * inv * w.z, t.w * inv * w.w); };
+  if constexpr (R > 0) {
 #pragma unroll
-  for (int u = 0; u < ROUTER_R / 4; ++u) if (tid + 256 * u < nvec) *(float4 *)(xn + 4 * (tid + 256 * u)) = normed(xv[u], nv[u]);
-  for (int v = tid + 64 * ROUTER_R; v < nvec; v += 256) *(float4 *)(xn + 4 * v) = normed(*(const float4 *)(xr + 4 * v), *(const float4 *)(norm_w + 4 * v));
+    for (int u = 0; u < R / 4; ++u) if (tid + 256 * u < nvec) *(float4 *)(xn + 4 * (tid + 256 * u)) = normed(xv[u], nv[u]);
+  } else {
+    for (int v = tid; v < nvec; v += 256) *(float4 *)(xn + 4 * v) = normed(*(const float4 *)(xr + 4 * v), *(const float4 *)(norm_w + 4 * v));
+  }
   __syncthreads();
   if (wave != 0) return;
   float *slog = scratch + (size_t)tok * (E + 1);
   unsigned *ticket = (unsigned *)(slog + E);
   float s = 0.f;
   auto dot = [&](const float4 &a4, const float4 &w4) { s = fmaf(a4.x, w4.x, s); s = fmaf(a4.y, w4.y, s); s = fmaf(a4.z, w4.z, s); s = fmaf(a4.w, w4.w, s); };
+  if constexpr (R > 0) {
 #pragma unroll
-  for (int u = 0; u < ROUTER_R; ++u) if (lane + 64 * u < nvec) dot(*(const float4 *)(xn + 4 * (lane + 64 * u)), gv[u]);
-  for (int v = lane + 64 * ROUTER_R; v < nvec; v += 64) dot(*(const float4 *)(xn + 4 * v), *(const float4 *)(wr + 4 * v));
+    for (int u = 0; u < R; ++u) if (lane + 64 * u < nvec) dot(*(const float4 *)(xn + 4 * (lane + 64 * u)), gv[u]);
+  } else {
+#pragma unroll 8
+    for (int v = lane; v < nvec; v += 64) dot(*(const float4 *)(xn + 4 * v), *(const float4 *)(wr + 4 * v));
+  }
   s = wave_sum(s);
   int last = 0;
   if (lane == 0) {
@@ -799,7 +811,8 @@ extern "C" int mrs_moe_router_topk_norm_split(const float *h, const float *norm_
   if (tokens <= 0) return 0;
   if (n_experts < 1 || n_experts > 64 || top_k < 1 || top_k > n_experts || (K & 3) || !norm_w || !scratch) return -1;
   if ((size_t)K * 4 > 64 * 1024) return -3;
-  hipLaunchKernelGGL(mrs::moe_router_split_kernel, dim3(n_experts, tokens), dim3(256), (size_t)K * 4, (hipStream_t)stream, h, gate_w, n_experts, K, top_k, renormalize, ids, weights,
+  const auto kern = K <= 256 * mrs::ROUTER_R ? mrs::moe_router_split_kernel<mrs::ROUTER_R> : mrs::moe_router_split_kernel<0>;
+  hipLaunchKernelGGL(kern, dim3(n_experts, tokens), dim3(256), (size_t)K * 4, (hipStream_t)stream, h, gate_w, n_experts, K, top_k, renormalize, ids, weights,
                      norm_w, eps, (float *)scratch);
   return 0;
 }

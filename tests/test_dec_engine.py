@@ -693,8 +693,11 @@ def test_router_with_fused_norm_host_emulation(tokens, E, K, topk):
 
 
 # rows longer than the split router's registers, the shortest, every lane an expert; equal logits, logits of NaN, of infinities and nothing else
-@pytest.mark.parametrize("tokens,E,K,topk,bad", [(1, 5, 4356, 2, ()), (2, 2, 4, 1, ()), (1, 64, 256, 8, ()), (1, 4, 64, 3, [(1, 0.0), (2, 0.0)]), (1, 4, 64, 2, [(0, np.nan), (3, -np.inf)]),
-                                                 (1, 3, 64, 3, [(0, np.nan), (1, np.nan), (2, np.nan)]), (1, 4, 64, 4, [(1, np.inf), (2, -np.inf), (3, np.nan)])])
+ROUTER_LIMITS = [(1, 5, 4356, 2, ()), (1, 2, 4100, 1, ()), (2, 3, 12288, 2, ()), (2, 2, 4, 1, ()), (1, 64, 256, 8, ()), (1, 4, 64, 3, [(1, 0.0), (2, 0.0)]),
+                 (1, 4, 64, 2, [(0, np.nan), (3, -np.inf)]), (1, 3, 64, 3, [(0, np.nan), (1, np.nan), (2, np.nan)]), (1, 4, 64, 4, [(1, np.inf), (2, -np.inf), (3, np.nan)])]
+
+
+@pytest.mark.parametrize("tokens,E,K,topk,bad", ROUTER_LIMITS)
 def test_router_rows_and_logits_at_their_limits_host_emulation(tokens, E, K, topk, bad):
     _check_router_norm(HostBackend(), tokens, E, K, topk, bad)
 
@@ -703,3 +706,9 @@ def test_router_rows_and_logits_at_their_limits_host_emulation(tokens, E, K, top
 @pytest.mark.parametrize("tokens,E,K,topk", [(1, 8, 4096, 2), (8, 8, 4096, 2), (2, 64, 2048, 6)])
 def test_router_with_fused_norm_gpu(dev, tokens, E, K, topk):
     _check_router_norm(GpuBackend(dev), tokens, E, K, topk)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("tokens,E,K,topk,bad", ROUTER_LIMITS)
+def test_router_rows_and_logits_at_their_limits_gpu(dev, tokens, E, K, topk, bad):
+    _check_router_norm(GpuBackend(dev), tokens, E, K, topk, bad)
