@@ -1,6 +1,6 @@
-// dec_attn.cuh -- decode attention of the decode engine as wave-level device functions: the split kernel with the last-arriver merge
-// (ext_dec.hip dec_attn2_kernel: groups of one and two heads; dec_attn4_kernel restates the same chains for four and eight), the persistent step kernel and the one-launch short-context kernel all call these, so every
-// engine path produces the same bits.  One wave per range of 32-token KV blocks of one (sequence, kv head): online softmax in f32 for the G query
+// dec_attn.cuh -- decode attention of the decode engine as wave-level device functions, called by the split kernel with the last-arriver merge (ext_dec.hip dec_attn2_kernel: groups of
+// one and two heads, and of eight in launches of up to four (sequence, key head) pairs); dec_attn4_kernel and dec_attn4_long_kernel restate the same chains for four and eight on
+// the matrix cores, prompts for many queries (ext_gemm_qi.hip): every engine path produces the same bits.  One wave per range of 32-token KV blocks of one (sequence, kv head): online softmax in f32 for the G query
 // heads of the GQA group, probabilities kept in f32, partial (m, l, o) per split; then the splits are merged per head.
 // Arithmetic = the reference CPU attention (mistralrs-core/src/attention/backends/cpu/single_q.rs): tile max, correction and probabilities
 // through the reference's fast_exp (elem.rs:417-433, common.cuh fast_exp_ref), merge as run_barrier (:108-157: weights exp(m_c - m_all), sums and
@@ -167,8 +167,8 @@ __device__ __forceinline__ void attn_split_core(const AttnArgs &a, int kvh, int 
   }
   // Splits of several blocks (model contexts above 2048 tokens): the next block's keys are requested into this one's registers as soon as these are multiplied, its values when this
   // block's are (its page index two blocks ahead): most of a memory latency passes under arithmetic, and four waves fit a SIMD (127 registers).  A second set of registers for
-  // the next block hid all of it, but two waves fitted (241): faster where the launch's waves all did (one sequence), slower for batches.  Decode steps at a context of 6000, us,
-  // no request ahead / second set / this: 4 layers of 4096, 32 heads of 4 key heads, 1 sequence 241 / 234 / 236, 5 sequences 411 / 452 / 410, 8 sequences 494 / 568 / 494;  2 layers
+  // the next block hid all of it, but two waves fitted (241): faster where the launch's waves all did (one sequence), slower for batches.  Decode steps at a context of 6000, us, timed
+  // when groups of four and eight ran here too (dec_attn4_long_kernel has most of them now), no request ahead / second set / this: 4 layers of 4096, 32 heads of 4 key heads, 1 sequence 241 / 234 / 236, 5 sequences 411 / 452 / 410, 8 sequences 494 / 568 / 494;  2 layers
   // of 8192, 64 heads of 8, 1 sequence 308 / 320 / 307, 8 sequences 762 / 840 / 766.
   unsigned page = bt[min(b0 + 1, b1 - 1)];
   for (int b = b0; b < b1; ++b) {

@@ -563,7 +563,7 @@ __global__ void __launch_bounds__(64 * ((G + 1) / 2)) dec_attn2_merge_kernel(con
 
 // ------------------------------------------------------------------------------------------------ the activation image as its own launch (batched decode)
 // A GEMV workgroup builds the image of ALL activation columns before it streams: at 8 columns that is 16 (K = 4096) to 28 (K = 14336, 4 columns per launch)
-// superblocks per wave, 256 times over -- 17-25 us of a 40-60 us launch (rocprofv3, round 5).  dec_act_image_kernel builds it ONCE, one workgroup per column
+// superblocks per wave, 256 times over -- 17-25 us of a 40-60 us launch (rocprofv3, round 5).  dec_act_image_kernel (rows with a norm) builds it ONCE, one workgroup per column
 // with the GEMV prologue's own functions (same virtual waves, same bytes), in column groups that each fit LDS (Launch::run's halving); the GEMV then copies its
 // group's image (GemvArgs::x_img, like o_proj after mrs_dec_attention).
 struct ActImgArgs {
@@ -579,7 +579,7 @@ __global__ void __launch_bounds__(NT) dec_act_image_kernel(const ActImgArgs a) {
   const float *x = a.x + (size_t)c * a.ldx;
   const ActRegs<1> pre = act_issue_all<1>(x, (unsigned)a.K * 4u, a.norm_w, a.K, wave);
   act_sumsq_all<1, 1>(red, pre, x, a.ldx, a.norm_w, a.K, wave);
-  if (a.norm_w) __syncthreads();
+  __syncthreads();
   const int c0 = a.rows ? c : a.gc0[c], n = a.rows ? 1 : a.gn[c];
   act_quantize_all<1, 1>(a.img + act_bytes(a.K, c0), red, pre, x, a.ldx, a.norm_w, a.eps, a.K, a.mode, wave, c - c0, n);
 }

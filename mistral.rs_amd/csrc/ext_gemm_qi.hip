@@ -275,7 +275,7 @@ __device__ __forceinline__ h2 pkfma(h2 x, h2 s, h2 c) { return __builtin_element
 //   * Q6_K takes two matrix instructions per run (sl, sh), so its vector work hides better under them; Q8_0's bound is the three instructions per output and block: the
 //     two multiplications and the addition of the engine's term.
 // Against 512-thread workgroups of 128 x 128 tiles (one per CU, their phases in lockstep), 4096 x 14336 (down) and 2 x 14336 x 4096 (gate / up) weights:
-//   Q6_K  down  512 tokens 170 -> 129 us, 1999 tokens 628 -> 457;   Q8_0  gate / up  700 tokens 402 -> 263, q / k / v 700 tokens three launches -> one of 95 us.
+//   Q6_K  down  512 tokens 170 -> 129 us, 1999 tokens 628 -> 457;   Q8_0  gate / up  700 tokens 402 -> 263, q / k / v 700 tokens three launches -> one of 78 us.
 // NT = 4 (128 tokens per wave, the operand built once per four matrix instructions) needs 255 registers and the earlier runs' sums in memory: 343 us against 199 us for
 // 28672 x 4096 x 512 tokens.
 struct QiSeg { const uint8_t *w; unsigned w_bytes; int N; float *out; int ldo; };
@@ -609,7 +609,8 @@ __global__ void __launch_bounds__(256 * wide_groups(MODE), MODE == W_ONE ? (NT =
     }
     const float *yd_s = (const float *)meta_s;
     const f32v zero32 = {0.f};
-    // d yd (and dmin yd) of the tile's outputs, each product rounded once: one matrix instruction of two 32 x 32 outer products (lane halves = blocks)
+    // d yd (and dmin yd) of the tile's outputs, each product rounded once: one matrix instruction of two 32 x 32 outer products (lane halves = blocks).  It adds the products to + 0, so
+    // one that is - 0 (a negative d of a token block of zeros) comes out as + 0: an output all of whose terms are zeros may have the other sign than in the decode engine
     const float dd = half_bits_to_float((uint16_t)(hf ? hd >> 16 : hd & 0xffff));
     auto products = [&](int tt) -> f32v { return __builtin_amdgcn_mfma_f32_32x32x1f32(yd_s[tt * 32 + nn], dd, zero32, 0, 0, 0); };
     if constexpr (TYPE == T_Q6_K) {
@@ -1484,7 +1485,8 @@ __global__ void __launch_bounds__(64 * PM_NW, 2) prefill_attn_mfma_kernel(const 
 // What bounds both: the f32 matrix instructions (64 cycles each, 64 + 64 of them per head, 32 queries and 32 tokens) take the SIMD's vector ALU with them -- measured, the times of
 // matrix and vector instructions add up (unlike the f16 ones'), so a vector instruction saved is time saved: halves of a dword by one permute, no masks where every query sees the
 // whole block, the exponential in 21 instructions, one-block splits without the running correction.  The probabilities cost 4 KiB per 128 matrix instructions, written and read once.
-// Attention of 32 heads, us per layer, one kernel / these two: 37 tokens at 300 48 / 13.8, 512 tokens 72 / 41, 1999 tokens 740 / 440 (floor of the matrix instructions alone 215).
+// Attention of 32 heads, us per layer, one kernel / these two: 37 tokens at 300 48 / 13.8, 512 tokens 72 / 41, 1999 tokens 740 / 440 (floor of the matrix instructions alone 215;
+// 436 - 446 on several cards, alone and inside a prompt).
 // A slot of the workspace, per (head, tile of 32 queries, 32-token block): the probabilities as the B operand of the P . V instructions, block sums, alphas, running maxima.
 #ifndef MRS_KEEP16
 #define MRS_KEEP16(x) asm volatile("" : "+v"(x[0]), "+v"(x[1]), "+v"(x[2]), "+v"(x[3]), "+v"(x[4]), "+v"(x[5]), "+v"(x[6]), "+v"(x[7]), "+v"(x[8]), "+v"(x[9]), "+v"(x[10]), "+v"(x[11]), "+v"(x[12]), "+v"(x[13]), "+v"(x[14]), "+v"(x[15]))

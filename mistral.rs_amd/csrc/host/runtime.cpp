@@ -455,8 +455,8 @@ class Llama {
     const bool imgb = b >= img_min_b && b >= 2 && b <= 8;
     auto image = [&](const float *x, int ldx, const float *nw, int k, int wtype) { return mrs_dec_act_image(x, ldx, nw, cfg.rms_eps, k, wtype, b, ws.act_img, s); };
     // (round 6) batched steps on the matrix cores (ext_dec_mm.hip): the same launches on the MFMA-order copy of the weights the exact prompt path keeps (QTensor::qi) -- integer
-    // dots on v_mfma_i32_32x32x32_i8 instead of 535 VALU per 8-column tile, the same bits.  MRS_DEC_MM=0 keeps the vector-ALU kernels; MRS_DEC_MM_MIN_B: smallest batch that takes it.
-    static const int mm_min_b = [] { const char *e = getenv("MRS_DEC_MM"); if (e && atoi(e) == 0) return 1 << 30; const char *m = getenv("MRS_DEC_MM_MIN_B"); return m ? atoi(m) : 3; }();  // measured (MI355X, 8B Q4_K_M): batch 2 / 3 / 4 / 8 = 760 / 1128 / 1518 / 2722 tok/s here, 824 / 1103 / 1315 / 1685 on the vector ALU
+    // dots on v_mfma_i32_16x16x64_i8 / 16x16x32_i8 instead of 535 VALU per 8-column tile, the same bits.  MRS_DEC_MM=0 keeps the vector-ALU kernels; MRS_DEC_MM_MIN_B: smallest batch that takes it.
+    static const int mm_min_b = [] { const char *e = getenv("MRS_DEC_MM"); if (e && atoi(e) == 0) return 1 << 30; const char *m = getenv("MRS_DEC_MM_MIN_B"); return m ? atoi(m) : 3; }();  // 8B Q4_K_M at 1500 tokens, us per step of two sequences, here / vector ALU: 2297 / 2356; they stay there (the same bits, 2.5 %)
     const bool mmb = imgb && b >= mm_min_b;
     // Two columns of a hidden-sized row: the GEMVs' own prologue hides most of its work behind the weight requests, an image launch in front of them cannot (8B Q4_K_M, image +
     // GEMV / GEMV alone: q / k / v 4.5 + 10.9 / 15.3 us, gate / up 4.5 + 17.4 / 21.1, lm_head 4.5 + 69.2 / 73.0, and a launch less each); rows of the FFN width keep the image
@@ -573,12 +573,13 @@ class Llama {
     const size_t t = (size_t)T, d = c.hidden_size, nq = (size_t)c.num_heads * c.head_dim, nkv = (size_t)c.num_kv_heads * c.head_dim;
     return align(t * d * 4) * 2 + align(t * nq * 4) * 2 + align(t * nkv * 4) * 2 + align((pad_to((int)d, MATRIX_ROW_PADDING) / 32) * 36) + 4096;  // (4096: the base is aligned)
   }
-  // gate, up and act: one row per token, in sparse-MoE layers per route
+  // Three slabs of one row per token (in sparse-MoE layers per route): gate and up, and a third that the operand quantizer no longer needs for silu(gate) up.  It stays: the
+  // attention's probabilities lie over all three, and with two of them 1999 tokens would go in three groups of heads instead of two.
   static size_t prefill_ffn_bytes(const mrs_llama_config &c, int T) {
     return align((size_t)T * (c.num_experts > 0 ? std::max(1, (int)c.num_experts_per_tok) : 1) * c.intermediate_size * 4) * 3;
   }
-  // The exact path's operand rows and tables, then gate / up / act at the END: what a call can do without stands behind them (run sums of cut launches) and over both of them
-  // (the attention's probabilities: neither gate / up / act nor run sums are live while it runs).
+  // The exact path's operand rows and tables, then gate / up and the third slab at the END: what a call can do without stands behind them (run sums of cut launches) and over both of them
+  // (the attention's probabilities: neither gate / up nor run sums are live while it runs).
   static size_t prefill_exact_bytes(const mrs_llama_config &c, int T) {
     const size_t t = (size_t)T, d = c.hidden_size, nq = (size_t)c.num_heads * c.head_dim, ff = c.intermediate_size;
     size_t b = prefill_rows_bytes(c, T) + align(mrs_qi_act_bytes(T, (int)std::max(std::max(d, nq), ff)));  // Q8_K operands of T rows (f16 quants, scales, run sums)
