@@ -3,22 +3,19 @@
 // What the reference does on a CPU device for a T-token prompt: every linear goes through the same QMatMul f32 fallback as decode
 // (mistralrs-quant/src/gguf/mod.rs:465-478): each activation ROW is quantized to Q8_K (K-quants), every output is a sum over the row's superblocks of
 // (d_w d_x) <integer dot> - (dmin_w d_x) <integer min term>.  Prompts also have another arithmetic (ext_gemm.hip: weights and activations rounded to bf16);
-// this kernel computes the reference's integers EXACTLY on v_mfma_f32_32x32x16_f16 and combines them in the f32 order of the decode engine ("ORD-U",
+// this kernel computes the reference's integers EXACTLY on v_mfma_i32_32x32x32_i8 and combines them in the f32 order of the decode engine ("ORD-U",
 // dec_core2.cuh / oracle orc_gemv_engine), so a token's logits and KV pages do not depend on whether it was part of a prompt or decoded:
-//   * the 6-bit sub-block scale is folded INTO the weight operand as an exact small integer in f16: Q4_K  sc (q - 8);  Q6_K  two operands
-//     sl (q - 32) and sh (q - 32) with sc = 16 sh + sl, |.| <= 480 / 256.  The activation operand is the Q8_K quant as f16.  Every product and every partial
-//     sum of a superblock is an integer below 2^24, so the f32 accumulator of the matrix core holds the EXACT sum (tests/test_gemm_qi.py holds
-//     v_mfma_f32_32x32x16_f16 to that on adversarial operands); no per-sub-block scale multiply is left on the vector ALU;
-//   * Q4_K: the operand is sc (q - 8), the 8 sum_j sc_j bsum_j the offset leaves out and msum = sum_j m_j bsum_j are one more MFMA each per superblock
-//     (K = the 16 run sums of the Q8_K block, scales / mins duplicated per run); (float)isum = X + 8 S is one rounding of the exact integer -- what (float)int gives;
-//   * Q5_K: the operand is sc (q - 16) (|.| <= 1008), two accumulators (<= 16.5 M each), and the 16 sum_j sc_j bsum_j the offset leaves out is one more MFMA (S);
-//     isum = XA + XB + 16 S is formed in int32 (a superblock's sum reaches 64 M: two f32 additions would round twice) and converted once; the mins' M as for Q4_K;
+//   * the activation operand is the Q8_K quant as it is; the sub-block scale is folded INTO the weight operand, an exact integer of two int8 digits, each with a matrix instruction
+//     and an int32 accumulator of its own: Q4_K  sc q = 8 (sh q) + sl q with sc = 8 sh + sl, each <= 105;  Q5_K  sc q <= 1953 and  Q6_K  sc (q - 32), |.| <= 4096, = 256 hi + lo
+//     with lo in -128 .. 127, |hi| <= 16.  No accumulator exceeds 128 x 128 x 256; no per-sub-block scale multiply is left on the vector ALU, (float)isum is one rounding;
+//   * Q4_K / Q5_K: msum = sum_j m_j bsum_j is one v_mfma_f32_32x32x16_f16 per superblock (K = the 16 run sums of the Q8_K block, the mins duplicated per run; every product and
+//     partial sum is an integer below 2^24, which its f32 accumulator holds exactly: tests/test_gemm_qi.py holds it to that on adversarial operands);
 //   * Q8_0: blocks of 32 int8 are one v_mfma_i32_32x32x32_i8 each, the block term in the engine's f32 expression;
 //   * per superblock and output ONE f32 term T (the decode engine's expression), terms added left to right inside each of the row's four runs of
 //     superblocks, the four run sums left to right (dec_core2.cuh header).
 // Operands: weights in an MFMA-order copy made at load time (mrs_gemm_qi_repack: per 32-row panel and superblock, every lane's 16 bytes of a piece
 // contiguous: one buffer_load_dwordx4 per lane and piece, straight into registers); activations from mrs_qi_quantize (engine-order RmsNorm + the candle
-// Q8_K quantizer of dec_core2.cuh, then f16 in the operand's k order, slab-major [superblock][token][256]).
+// Q8_K quantizer of dec_core2.cuh, int8 in the operand's k order, slab-major [superblock][token][256]).
 // One kernel, gemm_qi_wide_kernel<type, token tiles of a wave>, multiplies all four types at all prompt lengths.
 #include "dec_core2.cuh"
 #include <stdio.h>
@@ -44,9 +41,7 @@ __host__ __device__ constexpr int rec_bytes_qi(int type) { return type == T_Q4_K
 __host__ __device__ inline bool qi_type(int t) { return t == T_Q4_K || t == T_Q5_K || t == T_Q6_K || t == T_Q8_0; }
 __host__ __device__ inline size_t qi_tensor_bytes(int type, long long n, long long k) { return (size_t)((n + 31) / 32) * (size_t)(k / 256) * rec_bytes_qi(type); }
 
-// the k order inside a group of 8 operand slots: slot jj holds element PERM[jj] (the half2 registers of the weight operand are (e0, e2), (e1, e3), (e4, e6), (e5, e7):
-// what two masks and a shift take out of a dword of nibbles / bytes)
-__host__ __device__ constexpr int perm8(int jj) { return jj == 1 ? 2 : jj == 2 ? 1 : jj == 5 ? 6 : jj == 6 ? 5 : jj; }
+// the k order of the K-quants' int8 operands inside a sub-block of 32: lane half h holds values 8 h .. 8 h + 7 and 16 + 8 h .. 16 + 8 h + 7 (a lane's 16 bytes of a piece)
 
 // ------------------------------------------------------------------------------------------------ weights: GGUF blocks -> MFMA-order copy
 // one thread per (panel, superblock, lane)
@@ -135,13 +130,13 @@ __global__ void __launch_bounds__(256) qi_repack_kernel(const uint8_t *__restric
 // ------------------------------------------------------------------------------------------------ activations: f32 rows -> operand buffers
 // Rows with an RmsNorm: one workgroup (512 threads) per token row, the decode engine's prologue (act_issue_all / act_finish_all: engine-order RmsNorm, candle's Q8_K quantizer)
 // builds the row's image in LDS.  Rows without: superblocks know nothing of each other, two per wave.  Either way the image is written out as the GEMM's operands:
-//   qf [S][T][256] f16: the int8 quants, inside every group of 8 in the operand's slot order;  yd [S][T] f32;  bsf [S][T][16] f16: the 16 run sums.
+//   qf [S][T][256] int8: the quants, inside every sub-block of 32 in the operand's k order;  yd [S][T] f32;  bsf [S][T][16] f16: the 16 run sums.
 // GLU: the row is silu_engine(g) * u (the decode engine's gate / up epilogue expression), g = x, u = x2.
 struct QuantArgs {
   const float *x, *x2; int ldx; const float *norm_w; float eps; int K, T;
-  _Float16 *qf; float *yd; _Float16 *bsf;
+  int8_t *qf; float *yd; _Float16 *bsf;
   float *xtmp;  // GLU and norm: f32 scratch [T][K] for the activated row (the prologue reads its input from memory)
-  int mode;     // ACT_Q8K (K-quant weights) / ACT_Q80 (Q8_0 weights: quantize_row_q8_0 per 32 values; outputs q8 [S][T][256] int8 in element order at `qf`, the block
+  int mode;     // ACT_Q8K (K-quant weights) / ACT_Q80 (Q8_0 weights: quantize_row_q8_0 per 32 values; `qf` in element order, the block
                 // scales f32(f16(d)) block-major [S][8][T] at `bsf`)
   const float *part; float *h;  // PART: the four run sums [4][T][K] of the product that is added to the rows `h` first (x = h, ldx = K)
 };
@@ -149,19 +144,18 @@ __device__ __forceinline__ float4 glu4(float4 g, float4 u) { return make_float4(
 // superblock sb of token t out of an image: `q` its 256 int8, `d` its scale(s), `bs` its run sums; worker `i` of `n`
 __device__ __forceinline__ void store_operands(const QuantArgs &a, int sb, int t, const char *q, const float *d, const int *bs, int i, int n) {
   const size_t row = (size_t)sb * a.T + t;
+  int8_t *dst = a.qf + row * 256;
   if (a.mode == ACT_Q80) {
-    for (int ch = i; ch < 16; ch += n) *(v4u *)((int8_t *)a.qf + row * 256 + ch * 16) = *(const v4u *)(q + ch * 16);
+    for (int ch = i; ch < 16; ch += n) *(v4u *)(dst + ch * 16) = *(const v4u *)(q + ch * 16);
     for (int b = i; b < 8; b += n) ((float *)a.bsf)[((size_t)sb * 8 + b) * a.T + t] = d[b];
     return;
   }
-  for (int g8 = i; g8 < 32; g8 += n) {
-    const int8_t *qg = (const int8_t *)(q + g8 * 8);
-    h8 o;
-#pragma unroll
-    for (int jj = 0; jj < 8; ++jj) o[jj] = (_Float16)(float)qg[perm8(jj)];
-    *(h8 *)(a.qf + row * 256 + g8 * 8) = o;
+  for (int ch = i; ch < 16; ch += n) {  // half ch % 2 of sub-block ch / 2: values 8 h .. 8 h + 7 and 16 + 8 h .. of its 32
+    const char *qg = q + (ch >> 1) * 32 + (ch & 1) * 8;
+    const uint2 lo = *(const uint2 *)qg, hi = *(const uint2 *)(qg + 16);
+    *(v4u *)(dst + ch * 16) = v4u{lo.x, lo.y, hi.x, hi.y};
   }
-  for (int r = i; r < 16; r += n) a.bsf[row * 16 + r] = (_Float16)(float)bs[r];
+  for (int r = (i + n / 2) % n; r < 16; r += n) a.bsf[row * 16 + r] = (_Float16)(float)bs[r];
   if (i == 0) a.yd[row] = d[0];
 }
 // rows with a norm.  GLU: the activated row goes through xtmp.  PART: the row is h + ((c0 + c1) + c2) + c3, the sum gemm_qi_reduce_kernel would have left in h (written there as
@@ -258,39 +252,39 @@ __device__ __forceinline__ bool expert_tile(const int *bounds, int experts, int 
 #endif
 
 __device__ __forceinline__ h2 as_h2(unsigned v) { return __builtin_bit_cast(h2, v); }
+__device__ __forceinline__ us2 as_us2(unsigned v) { return __builtin_bit_cast(us2, v); }
+__device__ __forceinline__ unsigned as_u32(us2 v) { return __builtin_bit_cast(unsigned, v); }
 __device__ __forceinline__ h8 mk_h8(h2 a, h2 b, h2 c, h2 d) { h8 r; r[0] = a[0]; r[1] = a[1]; r[2] = b[0]; r[3] = b[1]; r[4] = c[0]; r[5] = c[1]; r[6] = d[0]; r[7] = d[1]; return r; }
-__device__ __forceinline__ h2 pkfma(h2 x, h2 s, h2 c) { return __builtin_elementwise_fma(x, s, c); }
 
 // ------------------------------------------------------------------------------------------------ the kernel
-// What bounds this product is the vector ALU beside the matrix cores: building a run's f16 operand costs ~12 instructions per 32 weight rows, the f32 term 4 per output and
-// superblock, one matrix instruction covers 1024 outputs x 16 values and hides about five of them (measured: 4.3 cycles per vector, ~9 issue cycles per matrix instruction
-// of a SIMD, 32 cycles of matrix pipe; at full matrix rate the card also drops to ~1.5 GHz).  So:
-//   * Q4_K's operand is sc (q - 8), |.| <= 504: a superblock's sum stays below 504 x 128 x 256 = 16.5 M < 2^24, ONE exact accumulator; the 8 sum_j sc_j bsum_j that the
-//     offset leaves out are a matrix instruction over the run sums (S, like the mins' M), and isum = X + 8 S is one rounding of the exact integer: fma(8, S, X);
-//   * its nibbles go to bits 7:4 of a half-word: 64 + q is one v_and_or (0x5400 = 64, 1/16 per mantissa step), sc (q - 8) = (64 + q) sc - 72 sc exactly (9 sc < 2^11);
+// What bounds this product is the vector ALU beside the matrix cores: a superblock of 32 weight rows costs ~134 (Q4_K) .. 290 (Q6_K) vector instructions of operand build, the f32
+// term 5 (Q6_K: 4) per output and superblock, a 32 x 32 tile 16 matrix instructions of 32 cycles (and 3 for the products below).  The times of two waves of a SIMD hardly overlap:
+// 28672 x 4096 x 2000 tokens of Q4_K takes 2400 cycles per wave and superblock (two tiles) at 2.05 GHz, 1220 of them matrix, 1580 vector issue (rocprofv3); without the term's
+// vector instructions it is 8 % faster, without the build not at all.  Operands in f16 (one digit of up to 504, K = 16 per matrix instruction, S = sum_j sc_j bsum_j beside M) cost 92 vector
+// instructions more per superblock of two tiles and twice the LDS reads, Q6_K's two f16 digits twice the matrix time:  us, f16 / int8 digits: Q4_K 28672 x 4096, 512 tokens 167 / 144,
+// 1999 640 / 545, 4096 x 14336, 1999 313 / 265; Q6_K 4096 x 14336, 512 tokens 117 / 85, 1999 438 / 305; Q5_K 28672 x 4096, 512 tokens 201 / 167.  So:
+//   * Q4_K: one multiplication of packed half-words multiplies two nibbles by a digit of the scale; Q5_K / Q6_K form sc (q - 32) + 128 in packed half-words and take them apart into
+//     bytes (v_perm_b32): digits of the half-words cost three instructions per four weights more than products of bytes, which Q6_K's signed scales and Q5_K's 31 x 7 do not fit;
 //   * d yd and dmin yd of a tile are one v_mfma_f32_32x32x1_2b (two outer products, each rounded once) instead of 32 multiplies;
 //   * reads, operand build and the next superblock's LDS-DMA stand one by one behind the matrix instructions of the step before; small workgroups (4 waves, 32 weight rows
 //     each, NT token tiles) leave two (NT = 2) or three (NT = 1) workgroups per CU, so that one's barriers and latencies run under another's arithmetic;
 //   * the projections that share their input are segments of ONE launch, the experts of a sparse-MoE prompt (windows of the expert-sorted rows) token tiles of one launch.
-//   * Q6_K takes two matrix instructions per run (sl, sh), so its vector work hides better under them; Q8_0's bound is the three instructions per output and block: the
-//     two multiplications and the addition of the engine's term.
+//   * Q8_0's bound is the three instructions per output and block: the two multiplications and the addition of the engine's term.
 // Against 512-thread workgroups of 128 x 128 tiles (one per CU, their phases in lockstep), 4096 x 14336 (down) and 2 x 14336 x 4096 (gate / up) weights:
 //   Q6_K  down  512 tokens 170 -> 129 us, 1999 tokens 628 -> 457;   Q8_0  gate / up  700 tokens 402 -> 263, q / k / v 700 tokens three launches -> one of 78 us.
-// NT = 4 (128 tokens per wave, the operand built once per four matrix instructions) needs 255 registers and the earlier runs' sums in memory: 343 us against 199 us for
-// 28672 x 4096 x 512 tokens.
 struct QiSeg { const uint8_t *w; unsigned w_bytes; int N; float *out; int ldo; };
 struct WideArgs {
   QiSeg s0, s1, s2; int x1, x2;  // segment of a workgroup column: < x1: s0, < x2: s1, else s2 (x1 = x2 = gridDim.x for a single one)
   int K, T;
-  const _Float16 *qf; const float *yd; const _Float16 *bsf;
+  const int8_t *qf; const float *yd; const _Float16 *bsf;
   int accumulate, ksplit; float *part; int part_n;  // ksplit = 4: workgroup z multiplies run z only, plane z of part [4][T][part_n] takes its sums
   const int *bounds; int experts;       // expert e multiplies the operand rows [bounds[e], bounds[e + 1]) by the weights at w + e * w_bytes (a grouped MoE prompt GEMM: the
                                         // bounds come from launch_moe_dispatch on the device, the grid is sized for the worst case and tiles past it leave); nullptr = all T rows
 };
-// LDS of a superblock of a workgroup's tokens, two buffers: K-quants: f16 quants [32 NT][512], block scales [32 NT] f32 (512 bytes), run sums [32 NT][16] f16;  Q8_0: int8
+// LDS of a superblock of a workgroup's tokens, two buffers: K-quants: int8 quants [32 NT][256], block scales [32 NT] f32 (512 bytes), run sums [32 NT][16] f16;  Q8_0: int8
 // quants [32 NT][256], scales [8 blocks][32 NT] f32.  A buffer is a multiple of a token's row (the fragments' exclusive or)
-template <int TYPE> constexpr int wide_row = TYPE == T_Q8_0 ? 256 : 512;
-template <int TYPE, int NT> constexpr int wide_buf = NT * 32 * wide_row<TYPE> + (TYPE == T_Q8_0 ? 0 : 512) + NT * 32 * 32;
+constexpr int WIDE_ROW = 256;
+template <int TYPE, int NT> constexpr int wide_buf = NT * 32 * WIDE_ROW + (TYPE == T_Q8_0 ? 0 : 512) + NT * 32 * 32;
 constexpr int WIDE_ROWS = 128;                                                      // weight rows of a workgroup: four waves
 // Order of the workgroups: all token tiles of 32 neighbouring workgroup columns (4096 weight rows), then of the next 32.  Workgroups go to the XCDs in turn, so those that live on
 // an XCD share four columns and read the same weights out of its L2; with all columns before the next token tile 28 (57344 rows: 56) columns were live there, and a wide tensor
@@ -328,7 +322,7 @@ constexpr int wide_groups(int mode) { return mode == W_ONE ? 1 : mode == W_RUNS4
 template <int TYPE, int NT, int MODE>
 __global__ void __launch_bounds__(256 * wide_groups(MODE), MODE == W_ONE ? (NT == 2 || TYPE == T_Q5_K ? 2 : TYPE == T_Q8_0 ? 4 : 3) : MODE == W_RUNS4 ? 4 : 2) gemm_qi_wide_kernel(const WideArgs a) {
   extern __shared__ __attribute__((aligned(16))) char smem_all[];
-  constexpr int TT_ = NT * 32, ROWB = wide_row<TYPE>, ACT_ = TT_ * ROWB, BUF_ = wide_buf<TYPE, NT>, YD_ = 512;
+  constexpr int TT_ = NT * 32, ROWB = WIDE_ROW, ACT_ = TT_ * ROWB, BUF_ = wide_buf<TYPE, NT>, YD_ = 512;
   constexpr int NPC = TYPE == T_Q4_K ? 4 : 8;  // 1-KiB pieces of a record
   constexpr int GROUPS = wide_groups(MODE), STEP = MODE == W_PAIR ? 2 : 1;
   const int tid = tid_opaque(), lane = tid & 63, wave_all = __builtin_amdgcn_readfirstlane(tid >> 6), wave = wave_all & 3, grp = GROUPS > 1 ? wave_all >> 2 : 0;
@@ -428,8 +422,6 @@ __global__ void __launch_bounds__(256 * wide_groups(MODE), MODE == W_ONE ? (NT =
   unsigned hw8[4] = {hs_next.x, hs_next.y, hs_next.z, hs_next.w};  // Q8_0
   if (TYPE != T_Q8_0) hd_next = load_hd(rec_first);
   const f16v zero = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-  unsigned mg = TYPE == T_Q6_K ? 0x64006400u : 0x54005400u;
-  MRS_OPAQUE_TID(mg);  // keeps the constant in a VGPR: v_and_or_b32 takes one literal
   auto add_pair = [&](int i) {  // W_PAIR: the second group's terms of its step i
 #pragma unroll
     for (int tt = 0; tt < NT; ++tt)
@@ -531,79 +523,96 @@ __global__ void __launch_bounds__(256 * wide_groups(MODE), MODE == W_ONE ? (NT =
 #pragma unroll
         for (int v = 0; v < 16; ++v) run[tt][v] = run[tt][v] + Tt[tt][v];
     } else {
-    // ---- the weight operand of a run (16 values of 32 rows x 16 / 8 of the K order per lane) as exact small integers in f16, from packed integer and f16 instructions:
-    //   Q4_K  sc (q - 8) = (64 + q) sc - 72 sc      (q at bits 7:4 of a half-word: 0x5400 = 64, one unit per 16 mantissa steps; 9 sc < 2^11)
-    //   Q5_K  sc (q - 16) = (64 + q) sc - 80 sc     (q at bits 8:4)
-    //   Q6_K  sl (q - 32), sh (q - 32) with sc = 16 sh + sl: (1024 + u) s - 1056 s (0x6400 = 1024, one unit per mantissa step; 1056 s is an f16 value for |s| <= 15)
-    h2 sc2[2], of2[2];  // Q4_K: of the low / high nibbles' sub-block;  Q5_K: [0];  Q6_K: sl, sh
-    auto scales = [&](int k) {  // of step k and, where they share one, the steps behind it
-      auto put = [&](int i, float f, float c) {
-        sc2[i] = __builtin_bit_cast(h2, __builtin_amdgcn_cvt_pkrtz(f, f));  // a small integer: exact
-        of2[i] = sc2[i] * h2{(_Float16)c, (_Float16)c};
-      };
+    // ---- the weight operand of step k = sub-block k (32 values of 32 rows; lane: row, values 8 hf .. 8 hf + 7 and 16 + 8 hf ..): sc q as two int8 digits, from packed 16-bit instructions
+    //   Q4_K  sc = 8 sh + sl: sl q and sh q, each <= 7 * 15: one multiplication of half-words multiplies two bytes (no carry between them)
+    //   Q5_K / Q6_K  sc q / sc (q - 32) = 256 hi + lo, of the half-word w = value + 128: lo = (w & 255) - 128, hi = w >> 8 (|hi| <= 16)
+    unsigned sdig[4];  // Q4_K: the scales' low digits of sub-blocks 0 .. 3 | 4 .. 7, the high ones
+    if constexpr (TYPE == T_Q4_K) { sdig[0] = hs.x & 0x07070707u; sdig[1] = hs.y & 0x07070707u; sdig[2] = (hs.x >> 3) & 0x07070707u; sdig[3] = (hs.y >> 3) & 0x07070707u; }
+    unsigned m32 = 0xFFE0FFE0u;
+    MRS_OPAQUE_TID(m32);  // a factor, not a shift and a subtraction
+    us2 sA, sB, cA, cB;  // Q4_K: low, high digit;  Q5_K: the scale;  Q6_K: the scales of runs 2 k and 2 k + 1, and what is added to their products
+    auto scales = [&](int k) {
       if constexpr (TYPE == T_Q4_K) {
-        if ((k & 3) < 2) { const int c = k >> 2, hi = k & 1; put(hi, (float)byte_of(c < 2 ? hs.x : hs.y, 2 * (c & 1) + hi), -72.0f); }  // the high nibbles' first step comes one later
+        const unsigned sel = 0x0c000c00u | (unsigned)(k & 3) * 0x00010001u;
+        sA = as_us2(__builtin_amdgcn_perm(0u, sdig[k >> 2], sel)); sB = as_us2(__builtin_amdgcn_perm(0u, sdig[2 + (k >> 2)], sel));
       } else if constexpr (TYPE == T_Q5_K) {
-        if ((k & 1) == 0) { const int g = k >> 1; put(0, (float)byte_of(g < 4 ? hs.x : hs.y, g & 3), -80.0f); }
+        sA = sB = as_us2(__builtin_amdgcn_perm(0u, k < 4 ? hs.x : hs.y, 0x0c000c00u | (unsigned)(k & 3) * 0x00010001u));
+        cA = cB = us2{128, 128};
       } else {
-        const int sc = sbyte_of(k < 4 ? hs.x : k < 8 ? hs.y : k < 12 ? hs.z : hs.w, k & 3);
-        put(0, (float)(sc & 15), -1056.0f); put(1, (float)(sc >> 4), -1056.0f);
+        const unsigned w = k < 2 ? hs.x : k < 4 ? hs.y : k < 6 ? hs.z : hs.w, a0 = (unsigned)sbyte_of(w, 2 * (k & 1)), a1 = (unsigned)sbyte_of(w, 2 * (k & 1) + 1);
+        sA = as_us2(__builtin_amdgcn_perm(a0, a0, 0x01000100u)); sB = as_us2(__builtin_amdgcn_perm(a1, a1, 0x01000100u));
+        cA = sA * as_us2(m32) + us2{128, 128}; cB = sB * as_us2(m32) + us2{128, 128};  // 128 - 32 sc
       }
     };
-    // step k: Q4_K: run 4 c + h (low nibbles) or 4 c + 2 + h (high nibbles) of piece c, in the order (c, h, hi);  else run k = half k % 2 of piece k / 2
-    auto run_of = [](int k) { return TYPE == T_Q4_K ? 4 * (k >> 2) + 2 * (k & 1) + ((k >> 1) & 1) : k; };
-    auto pair_of = [&](int k, int p, h2 &w, h2 &w2) {  // operand slots 2 p, 2 p + 1
-      const int c = TYPE == T_Q4_K ? k >> 2 : k >> 1, h = TYPE == T_Q4_K ? (k >> 1) & 1 : k & 1, hi = k & 1;
-      const unsigned d = h == 0 ? (p < 2 ? wq[c].x : wq[c].y) : (p < 2 ? wq[c].z : wq[c].w);
-      if constexpr (TYPE == T_Q4_K) w = pkfma(as_h2(((hi ? ((p & 1) ? d >> 8 : d) : ((p & 1) ? d >> 4 : d << 4)) & 0x00F000F0u) | mg), sc2[hi], of2[hi]);
-      else if constexpr (TYPE == T_Q5_K) w = pkfma(as_h2((((p & 1) ? d >> 4 : d << 4) & 0x01F001F0u) | mg), sc2[0], of2[0]);
-      else {
-        const h2 u = as_h2((((p & 1) ? d >> 8 : d) & 0x00FF00FFu) | mg);
-        w = pkfma(u, sc2[0], of2[0]); w2 = pkfma(u, sc2[1], of2[1]);
+    auto digits = [&](int k, int p, unsigned &lo, unsigned &hi) {  // dword p of the operand
+      const v4u w = wq[TYPE == T_Q4_K ? k >> 1 : k];
+      const unsigned d = p == 0 ? w.x : p == 1 ? w.y : p == 2 ? w.z : w.w;
+      if constexpr (TYPE == T_Q4_K) {
+        const us2 q = as_us2(((k & 1) ? d >> 4 : d) & 0x0F0F0F0Fu);
+        lo = as_u32(q * sA); hi = as_u32(q * sB);
+      } else {
+        const us2 s = p < 2 ? sA : sB, c = p < 2 ? cA : cB;
+        const unsigned e = as_u32(as_us2(d & 0x00FF00FFu) * s + c), o = as_u32(as_us2(__builtin_amdgcn_perm(0u, d, 0x0c030c01u)) * s + c);
+        lo = __builtin_amdgcn_perm(o, e, 0x06020400u) ^ 0x80808080u;
+        hi = __builtin_amdgcn_perm(o, e, 0x07030501u);
       }
     };
-    constexpr int NW2 = TYPE == T_Q6_K ? 4 : 1;
-    h8 fr[2][NT];
-    h2 w[2][4], w2[2][NW2];
+    constexpr int DIGIT = TYPE == T_Q4_K ? 3 : 8;
+    constexpr bool EARLY = MODE != W_RUNS4;  // the next superblock's rows are requested in front of the matrix instructions, all of them (in 16 waves' 128 registers: one by one behind them)
+    i4v fr[2][NT];
+    unsigned wl[2][4], wh[2][4];
     scales(0);
-    if (TYPE == T_Q4_K) scales(1);
 #pragma unroll
-    for (int p = 0; p < 4; ++p) pair_of(0, p, w[0][p], w2[0][p % NW2]);
+    for (int p = 0; p < 4; ++p) digits(0, p, wl[0][p], wh[0][p]);
     __builtin_amdgcn_sched_barrier(0);
     MRS_WAIT_VMCNT0();  // this wave's DMA pieces of superblock sb have landed
     __syncthreads();    // everyone's have, and every wave has finished reading the other buffer
     if (MODE == W_PAIR && grp == 0 && it > 0) add_pair(it - 1);
     stage_meta(sb + STEP, it + 1, more);
+    if constexpr (EARLY) {
+#pragma unroll
+      for (int i = 0; i < NSTAGE; ++i) stage_q(sb + STEP, it + 1, i, more);
+      __builtin_amdgcn_sched_barrier(0);
+    }
     hs_next = load_hs(rec_next); hd_next = load_hd(rec_next);
-    auto frag = [&](int r, int tt) -> h8 { return MRS_LDS_FRAG(h8, smem, abase ^ (unsigned)(32 * r), tt * (32 * ROWB)); };
-    constexpr int NX = TYPE == T_Q4_K ? 1 : 2;  // accumulators: Q5_K: runs 0 .. 7 | 8 .. 15 (|.| <= 16.5 M each);  Q6_K: the sl | sh operands
-    f16v X[NX][NT];
+    if (TYPE != T_Q4_K) wq[0] = load_q(rec_next, 0);
+    auto frag = [&](int k, int tt) -> i4v { return MRS_LDS_FRAG(i4v, smem, abase ^ (unsigned)(32 * k), tt * (32 * ROWB)); };
+    i16v XL[NT], XH[NT];
 #pragma unroll
-    for (int x = 0; x < NX; ++x)
+    for (int tt = 0; tt < NT; ++tt)
 #pragma unroll
-      for (int tt = 0; tt < NT; ++tt) X[x][tt] = zero;
-    // behind each matrix instruction of a step stand one read and a share of the operand build of the next step, behind the step's first one a piece of the next
+      for (int v = 0; v < 16; ++v) { XL[tt][v] = 0; XH[tt][v] = 0; }
+    // behind each matrix instruction of a step stands a share of the next step's operand build, behind the first of a token tile also the tile's next read and a piece of the next
     // superblock's DMA: the wave's own vector and memory instructions run under its matrix instructions (scheduling barriers keep the order)
 #pragma unroll
-    for (int tt = 0; tt < NT; ++tt) fr[0][tt] = frag(run_of(0), tt);
+    for (int tt = 0; tt < NT; ++tt) fr[0][tt] = frag(0, tt);
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-    for (int k = 0; k < 16; ++k) {
-      const h8 wk = mk_h8(w[k & 1][0], w[k & 1][1], w[k & 1][2], w[k & 1][3]);
+    for (int k = 0; k < 8; ++k) {
+      const int c = k & 1, nx = c ^ 1;
+      const i4v lo = {(int)wl[c][0], (int)wl[c][1], (int)wl[c][2], (int)wl[c][3]}, hi = {(int)wh[c][0], (int)wh[c][1], (int)wh[c][2], (int)wh[c][3]};
 #pragma unroll
       for (int tt = 0; tt < NT; ++tt) {
-        const int x = TYPE == T_Q5_K ? k >> 3 : 0;
-        X[x][tt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(fr[k & 1][tt], wk, X[x][tt], 0, 0, 0);
-        if constexpr (TYPE == T_Q6_K)
-          X[1][tt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(fr[k & 1][tt], mk_h8(w2[k & 1][0], w2[k & 1][1], w2[k & 1][2], w2[k & 1][3]), X[1][tt], 0, 0, 0);
-        if (k + 1 < 16) {
-          fr[(k + 1) & 1][tt] = frag(run_of(k + 1), tt);
+        XL[tt] = __builtin_amdgcn_mfma_i32_32x32x32_i8(fr[c][tt], lo, XL[tt], 0, 0, 0);
+        if (k + 1 < 8) {
+          fr[nx][tt] = frag(k + 1, tt);
           if (tt == 0) scales(k + 1);
 #pragma unroll
-          for (int p = tt * 4 / NT; p < (tt + 1) * 4 / NT; ++p) pair_of(k + 1, p, w[(k + 1) & 1][p], w2[(k + 1) & 1][p % NW2]);
+          for (int p = tt * 4 / NT; p < tt * 4 / NT + 2 / NT; ++p) digits(k + 1, p, wl[nx][p], wh[nx][p]);
         }
-        if (tt == 0 && (k + 1) % (16 / NSTAGE) == 0) stage_q(sb + STEP, it + 1, (k + 1) / (16 / NSTAGE) - 1, more);
-        if (tt == NT - 1 && (TYPE == T_Q4_K ? (k & 3) == 2 : (k & 1) == 0)) wq[TYPE == T_Q4_K ? k >> 2 : k >> 1] = load_q(rec_next, TYPE == T_Q4_K ? k >> 2 : k >> 1);  // step k + 1, the piece's last, has been built
+        if constexpr (!EARLY) {
+#pragma unroll
+          for (int i = 0; i < NSTAGE; ++i) if (tt == 0 && k == i * (8 / NSTAGE)) stage_q(sb + STEP, it + 1, i, more);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        XH[tt] = __builtin_amdgcn_mfma_i32_32x32x32_i8(fr[c][tt], hi, XH[tt], 0, 0, 0);
+        if (k + 1 < 8) {
+#pragma unroll
+          for (int p = tt * 4 / NT + 2 / NT; p < (tt + 1) * 4 / NT; ++p) digits(k + 1, p, wl[nx][p], wh[nx][p]);
+        }
+        if (tt == NT - 1) {  // step k + 1 has been built
+          if (TYPE == T_Q4_K ? (k & 1) == 0 : k + 1 < 8) { const int i = TYPE == T_Q4_K ? k >> 1 : (k + 1) & 7; wq[i] = load_q(rec_next, i); }
+        }
         __builtin_amdgcn_sched_barrier(0);
       }
     }
@@ -613,40 +622,29 @@ __global__ void __launch_bounds__(256 * wide_groups(MODE), MODE == W_ONE ? (NT =
     // one that is - 0 (a negative d of a token block of zeros) comes out as + 0: an output all of whose terms are zeros may have the other sign than in the decode engine
     const float dd = half_bits_to_float((uint16_t)(hf ? hd >> 16 : hd & 0xffff));
     auto products = [&](int tt) -> f32v { return __builtin_amdgcn_mfma_f32_32x32x1f32(yd_s[tt * 32 + nn], dd, zero32, 0, 0, 0); };
+    auto isum = [&](int tt, int v) { return (float)(XL[tt][v] + (int)((unsigned)XH[tt][v] << DIGIT)); };
     if constexpr (TYPE == T_Q6_K) {
 #pragma unroll
       for (int tt = 0; tt < NT; ++tt) {
-        const f32v dy = products(tt);
+        const f16v dy = __builtin_amdgcn_mfma_f32_32x32x2f32(hf ? 0.f : yd_s[tt * 32 + nn], hf ? 0.f : dd, zero, 0, 0, 0);  // one block: half of the registers
 #pragma unroll
-        for (int v = 0; v < 16; ++v) {
-          const float If = fmaf(16.0f, X[1][tt][v], X[0][tt][v]);  // (float)isum: one rounding of the exact integer
-          run[tt][v] = run[tt][v] + dy[v] * If;
-        }
+        for (int v = 0; v < 16; ++v) run[tt][v] = run[tt][v] + dy[v] * isum(tt, v);
         __builtin_amdgcn_sched_barrier(0);
       }
     } else {
-      // M = sum_run m_{run / 2} bsum_run, S = sum_run sc_{run / 2} bsum_run: operand slot (hf, jj) <-> run 8 hf + jj -> sub-block 4 hf + jj / 2
-      const unsigned mw = hf ? hs.w : hs.z, sw = hf ? hs.y : hs.x;
-      h8 wm, wsc;
+      // M = sum_run m_{run / 2} bsum_run: operand slot (hf, jj) <-> run 8 hf + jj -> sub-block 4 hf + jj / 2
+      const unsigned mw = hf ? hs.w : hs.z;
+      h2 wm[4];  // a byte under 0x64 is 1024 + m
 #pragma unroll
-      for (int k = 0; k < 4; ++k) {
-        const _Float16 mk = (_Float16)(float)byte_of(mw, k), sk = (_Float16)(float)byte_of(sw, k);
-        wm[2 * k] = mk; wm[2 * k + 1] = mk; wsc[2 * k] = sk; wsc[2 * k + 1] = sk;
-      }
+      for (int k = 0; k < 4; ++k) wm[k] = as_h2(__builtin_amdgcn_perm(0x64646464u, mw, 0x04000400u | (unsigned)k * 0x00010001u)) - h2{(_Float16)1024.f, (_Float16)1024.f};
+      const h8 wm8 = mk_h8(wm[0], wm[1], wm[2], wm[3]);
 #pragma unroll
       for (int tt = 0; tt < NT; ++tt) {
         const h8 bsf = *(const h8 *)(meta_s + YD_ + (tt * 32 + nn) * 32 + hf * 16);
         const f32v dy = products(tt);
-        const f16v Sx = __builtin_amdgcn_mfma_f32_32x32x16_f16(bsf, wsc, zero, 0, 0, 0);
-        const f16v M = __builtin_amdgcn_mfma_f32_32x32x16_f16(bsf, wm, zero, 0, 0, 0);
+        const f16v M = __builtin_amdgcn_mfma_f32_32x32x16_f16(bsf, wm8, zero, 0, 0, 0);
 #pragma unroll
-        for (int v = 0; v < 16; ++v) {
-          float If;  // (float)isum: one rounding of the exact integer (Q5_K's reaches 64 M: formed in int32)
-          if constexpr (TYPE == T_Q4_K) If = fmaf(8.0f, Sx[v], X[0][tt][v]);
-          else If = (float)(((int)X[0][tt][v] + (int)X[NX - 1][tt][v]) + 16 * (int)Sx[v]);
-          const float t = fmaf(dy[v], If, -(dy[16 + v] * M[v]));
-          run[tt][v] = run[tt][v] + t;
-        }
+        for (int v = 0; v < 16; ++v) run[tt][v] = run[tt][v] + fmaf(dy[v], isum(tt, v), -(dy[16 + v] * M[v]));
         __builtin_amdgcn_sched_barrier(0);  // one token tile at a time: the sums of all of them would not fit the registers
       }
     }
@@ -863,17 +861,17 @@ extern "C" int mrs_gemm_qi_repack(const void *gguf_blocks, int type, long long n
   else hipLaunchKernelGGL(qi::qi_repack_kernel<T_Q6_K>, grid, dim3(256), 0, (hipStream_t)stream, (const uint8_t *)gguf_blocks, (uint8_t *)dst, n, (int)k, total);
   return 0;
 }
-// bytes of the three operand buffers of T rows of K values: qf (f16 quants), yd (f32 block scales), bsf (f16 run sums), each 256-byte aligned inside ONE buffer
+// bytes of the three operand buffers of T rows of K values: qf (int8 quants), yd (f32 block scales), bsf (f16 run sums), each 256-byte aligned inside ONE buffer
 extern "C" size_t mrs_qi_act_bytes(int T, int K) {
   const size_t S = (size_t)(K / 256), t = (size_t)T;
   auto al = [](size_t v) { return (v + 255) & ~(size_t)255; };
-  return al(S * t * 512) + al(S * t * 4) + al(S * t * 32);
+  return al(S * t * 256) + al(S * t * 4) + al(S * t * 32);
 }
-static void qi_split(void *buf, int T, int K, _Float16 **qf, float **yd, _Float16 **bsf) {
+static void qi_split(void *buf, int T, int K, int8_t **qf, float **yd, _Float16 **bsf) {
   const size_t S = (size_t)(K / 256), t = (size_t)T;
   auto al = [](size_t v) { return (v + 255) & ~(size_t)255; };
   char *p = (char *)buf;
-  *qf = (_Float16 *)p; p += al(S * t * 512);
+  *qf = (int8_t *)p; p += al(S * t * 256);
   *yd = (float *)p; p += al(S * t * 4);
   *bsf = (_Float16 *)p;
 }
@@ -1030,9 +1028,9 @@ static int gemm_qi_launch(int type, int nt, const void *const *w_qi, const int *
     if (qi::qi_tensor_bytes(type, N[i], K) >= 0xffffff00ull) return -2;
     n_all += N[i];
   }
-  if ((size_t)(K / 256) * T * 512 >= 0x7fffffffull) return -2;
+  if ((size_t)(K / 256) * T * 512 >= 0x7fffffffull) return -2;  // (twice the operands' bytes)
   hipStream_t s = (hipStream_t)stream;
-  _Float16 *qf, *bsf; float *yd;
+  int8_t *qf; _Float16 *bsf; float *yd;
   qi_split((void *)act, T, K, &qf, &yd, &bsf);
   max_rows = bounds ? std::min(max_rows, T) : T;
   qi::WideArgs a{};
@@ -1094,17 +1092,13 @@ __global__ void __launch_bounds__(256) qi_gather_rows_kernel(const char *__restr
                                                              int tk, int *__restrict__ inv, size_t off1s, size_t off2s, size_t off1d, size_t off2d) {
   const int r = blockIdx.x, route = sorted[r], t = route / tk;
   if (threadIdx.x == 0 && inv) inv[route] = r;
-  if (mode == ACT_Q80) {  // q8 [S][rows][256] at 0; block scales [S][8][rows] f32 at off2
-    for (int i = threadIdx.x; i < S * 16; i += 256) {
-      const int sb = i >> 4, ch = i & 15;
-      *(v4u *)(dst + ((size_t)sb * R + r) * 256 + ch * 16) = *(const v4u *)(src + ((size_t)sb * T + t) * 256 + ch * 16);
-    }
+  for (int i = threadIdx.x; i < S * 16; i += 256) {  // int8 quants [S][rows][256] at 0
+    const int sb = i >> 4, ch = i & 15;
+    *(v4u *)(dst + ((size_t)sb * R + r) * 256 + ch * 16) = *(const v4u *)(src + ((size_t)sb * T + t) * 256 + ch * 16);
+  }
+  if (mode == ACT_Q80) {  // block scales [S][8][rows] f32 at off2
     for (int i = threadIdx.x; i < S * 8; i += 256) ((float *)(dst + off2d))[(size_t)i * R + r] = ((const float *)(src + off2s))[(size_t)i * T + t];
-  } else {  // qf [S][rows][256] f16 at 0; yd [S][rows] f32 at off1; bsf [S][rows][16] f16 at off2
-    for (int i = threadIdx.x; i < S * 32; i += 256) {
-      const int sb = i >> 5, ch = i & 31;
-      *(v4u *)(dst + ((size_t)sb * R + r) * 512 + ch * 16) = *(const v4u *)(src + ((size_t)sb * T + t) * 512 + ch * 16);
-    }
+  } else {  // yd [S][rows] f32 at off1; bsf [S][rows][16] f16 at off2
     for (int i = threadIdx.x; i < S * 2; i += 256) {
       const int sb = i >> 1, ch = i & 1;
       *(v4u *)(dst + off2d + ((size_t)sb * R + r) * 32 + ch * 16) = *(const v4u *)(src + off2s + ((size_t)sb * T + t) * 32 + ch * 16);
@@ -1142,7 +1136,7 @@ __global__ void __launch_bounds__(256) resid_scale_add_kernel(float *__restrict_
 }  // namespace mrs
 extern "C" int mrs_qi_gather_rows(int w_type, const void *act_src, int T, void *act_dst, int R, int K, const int *sorted_routes, int top_k, int *inv, void *stream) {
   if (!act_src || !act_dst || !sorted_routes || T <= 0 || R <= 0 || K <= 0 || K % 256 || top_k <= 0 || !qi::qi_type(w_type)) return -1;
-  _Float16 *qs, *bs, *qd, *bd; float *ys, *yd;
+  int8_t *qs, *qd; _Float16 *bs, *bd; float *ys, *yd;
   qi_split((void *)act_src, T, K, &qs, &ys, &bs);
   qi_split(act_dst, R, K, &qd, &yd, &bd);
   hipLaunchKernelGGL(qi::qi_gather_rows_kernel, dim3(R), dim3(256), 0, (hipStream_t)stream, (const char *)act_src, (char *)act_dst, T, R, K / 256, dec2::act_mode_for(w_type),

@@ -582,7 +582,7 @@ class Llama {
   // (the attention's probabilities: neither gate / up nor run sums are live while it runs).
   static size_t prefill_exact_bytes(const mrs_llama_config &c, int T) {
     const size_t t = (size_t)T, d = c.hidden_size, nq = (size_t)c.num_heads * c.head_dim, ff = c.intermediate_size;
-    size_t b = prefill_rows_bytes(c, T) + align(mrs_qi_act_bytes(T, (int)std::max(std::max(d, nq), ff)));  // Q8_K operands of T rows (f16 quants, scales, run sums)
+    size_t b = prefill_rows_bytes(c, T) + align(mrs_qi_act_bytes(T, (int)std::max(std::max(d, nq), ff)));  // Q8_K operands of T rows (int8 quants, scales, run sums)
     if (c.num_experts > 0) {  // routes = T * top_k rows in expert-sorted order
       const size_t r = t * std::max(1, (int)c.num_experts_per_tok), E = (size_t)c.num_experts;
       b += align(r * 4) * 4 + align((E + 1) * 4) + align(E * 4) * 2;  // ids, weights, sorted routes, inverse; bounds, counts, cursors

@@ -98,6 +98,45 @@ def run_q5k_extremes(O, be):
     run_gemm(O, be, "Q5_K", n, k, T, 0, seed=5, packed=packed, x_override=x)
 
 
+def digit_extreme_blocks(tname, n, k):
+    """Blocks at the ends of the weight operand's digits.  Q4_K: every scale and min 63, values 15 (sc q = 945, both digits 105), 0, or a mix;  Q6_K: scales -128 / 127 and values
+    0 / 63 (sc (q - 32) = 4096, -3968, -4064, 3937: hi = 16 .. -16, lo = 0, -128, 32, 97)."""
+    S = k // 256
+    if tname == "Q4_K":
+        out = np.full((n, S, 144), 0xFF, np.uint8)
+        out[:, :, 0:4] = np.frombuffer(np.array([1.0, 0.5], np.float16).tobytes(), np.uint8)
+        out[1::3, :, 16:] = 0x00
+        out[2::3, :, 16:] = 0x0F  # low nibbles 15, high 0
+    else:
+        out = np.zeros((n, S, 210), np.uint8)
+        out[:, :, 208:210] = np.frombuffer(np.float16(0.5).tobytes(), np.uint8)
+        for i in range(4):
+            out[i::4, :, :192] = 0xFF if i & 1 else 0x00
+            out[i::4, :, 192:208] = 0x7F if i & 2 else 0x80
+        out[3::5, :, 192:208:2] = 0x80
+    return out.reshape(n, -1)
+
+
+def run_digit_extremes(O, be, tname):
+    n, k, T = 37, 1280, 4
+    x = np.ones((T, k), np.float32)  # every quant -128
+    x[1] = -3.0                      # every quant 127
+    x[2, ::2] = -1.0                 # -128 / 127 in turn
+    x[3, 256:512] = 0.0
+    run_gemm(O, be, tname, n, k, T, 0, seed=6, packed=digit_extreme_blocks(tname, n, k), x_override=x)
+
+
+@pytest.mark.parametrize("tname", ["Q4_K", "Q6_K"])
+def test_gemm_qi_digit_extremes_host_emulation(oracle, tname):
+    run_digit_extremes(oracle, HostBackend(), tname)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("tname", ["Q4_K", "Q6_K"])
+def test_gemm_qi_digit_extremes_gpu(oracle, dev, tname):
+    run_digit_extremes(oracle, GpuBackend(dev), tname)
+
+
 def test_gemm_qi_q5k_extreme_magnitudes_host_emulation(oracle):
     run_q5k_extremes(oracle, HostBackend())
 
