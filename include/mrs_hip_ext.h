@@ -299,6 +299,10 @@ int mrs_gemm_qi_is_cut(int ggml_type, int n_tensors, const int *N, int K, int T)
 int mrs_gemm_qi_form(int ggml_type, int n_tensors, const int *N, int K, int T, int room);  /* token tiles of a wave | groups of waves << 4 | cut << 8 (room: there is a workspace) */
 int mrs_gemm_qi_multi(int ggml_type, int n_tensors, const void *const *w_qi, const int *N, int K, const void *act, int T, float *const *out, const int *ldo, int accumulate,
                       const int *bounds, int experts, int max_rows, void *workspace, size_t workspace_bytes, void *stream);
+/* mrs_gemm_qi_mixed: tensors of two K-quants (types[]: Q6_K first, then Q4_K or Q5_K) on the same rows in one launch; keep: run sums stay in the workspace as in mrs_gemm_qi_multi_planes
+ * (returns 1), else rows.  -1: other types. */
+int mrs_gemm_qi_mixed(const int *types, int n_tensors, const void *const *w_qi, const int *N, int K, const void *act, int T, float *const *out, const int *ldo, void *workspace,
+                      size_t workspace_bytes, int keep, void *stream);
 /* What stands between a prompt's products, in fewer launches.  mrs_gemm_qi_multi_planes: mrs_gemm_qi_multi over T rows that leaves the run sums of a cut launch as they are: 1 = the
  * workspace begins with the planes [4][T][sum N] and `out` is untouched, 0 = `out` is complete.  mrs_qi_quantize_added: h <- h + ((c0 + c1) + c2) + c3 of planes `part` [4][T][K], then
  * mrs_qi_quantize_for of h with the norm (K up to 14336).  mrs_prefill_rope_cache: q / k / v rows [T][ld] (or, plane != 0, the first of four planes `plane` floats apart, added the same

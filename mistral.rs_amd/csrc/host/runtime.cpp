@@ -739,6 +739,13 @@ class Llama {
       const int rc = mrs_gemm_qi_multi_planes(ty, nt, w, N, K, qact, T, out, N, acc, (char *)qws + at, qws_bytes - at, s);
       return rc < 0 ? fail("prefill (exact): mrs_gemm_qi_multi refused ggml dtype %d (N=%d K=%d)", ty, N[0], K) : rc;
     };
+    // tensors of two types
+    auto lins_mixed = [&](const int *types, int nt, const GgufMatMul *const *m, const int *N, int K, float *const *out, bool keep, size_t at) -> int {
+      const void *w[3];
+      for (int i = 0; i < nt; ++i) w[i] = m[i]->get_qtensor()->qi;
+      const int rc = mrs_gemm_qi_mixed(types, nt, w, N, K, qact, T, out, N, (char *)qws + at, qws_bytes - at, keep ? 1 : 0, s);
+      return rc < 0 ? fail("prefill (exact): mrs_gemm_qi_mixed refused ggml dtypes %d / %d (N=%d K=%d)", types[0], types[nt - 1], N[0], K) : rc;
+    };
     auto lin = [&](const GgufMatMul &m, int N, int K, float *out, int acc) -> int { const GgufMatMul *p = &m; return lins(1, &p, &N, K, &out, acc); };
     // o_proj / down_proj: h <- h + W . x;  tensor parallel: h <- h * (1 / world) + W_shard . x on every rank (the decode step's RESID epilogue, two roundings), then ONE
     // sum all-reduce of h (distributed/layers.rs:965-975) -- the same sums as the decode step whenever the all-reduce adds the ranks in the same order (world 2: always;
@@ -783,14 +790,22 @@ class Llama {
           if (done[j] || (tj == Q8_0 ? 1 : 0) != mode) continue;
           const GgufMatMul *mm[3]; int nn[3]; float *oo[3]; size_t ix[3]; int c = 0;
           size_t cols = 0, left = 0;  // of this launch, of those still to come
+          // Q6_K beside Q4_K or Q5_K (the value projections of half of the layers): one launch, Q6_K first
+          int second = 0, types[3];  // the other type of the tensors to come; -1: several
           for (size_t l = 0; l < m.size(); ++l) {
-            if (done[l]) continue;
-            if (l >= j && m[l]->get_qtensor()->dtype == tj) { mm[c] = m[l]; nn[c] = n[l]; oo[c] = o[l]; ix[c] = l; ++c; done[l] = true; cols += (size_t)n[l]; }
-            else left += (size_t)n[l];
+            const int tl = m[l]->get_qtensor()->dtype;
+            if (!done[l] && tl != tj && tl != Q8_0) second = second == 0 || second == tl ? tl : -1;
           }
+          const bool mixed = (tj == Q6K && (second == Q4K || second == Q5K)) || (second == Q6K && (tj == Q4K || tj == Q5K));
+          for (int pass = 0; pass < (mixed ? 2 : 1); ++pass) {
+            const int tp = !mixed ? tj : pass == 0 ? (int)Q6K : tj == Q6K ? second : tj;
+            for (size_t l = 0; l < m.size(); ++l)
+              if (!done[l] && m[l]->get_qtensor()->dtype == tp) { mm[c] = m[l]; nn[c] = n[l]; oo[c] = o[l]; ix[c] = l; types[c] = tp; ++c; done[l] = true; cols += (size_t)n[l]; }
+          }
+          for (size_t l = 0; l < m.size(); ++l) if (!done[l]) left += (size_t)n[l];
           const size_t plane = (size_t)T * cols;
           const bool keep = src && at + 16 * ((size_t)T * (cols + left)) <= qws_bytes;  // (else the next launch would find no workspace)
-          const int rc = keep ? lins_planes(c, mm, nn, d, oo, 0, at) : lins(c, mm, nn, d, oo, 0);
+          const int rc = mixed ? lins_mixed(types, c, mm, nn, d, oo, keep, keep ? at : 0) : keep ? lins_planes(c, mm, nn, d, oo, 0, at) : lins(c, mm, nn, d, oo, 0);
           if (rc < 0) return -1;
           size_t col = 0;
           for (int l = 0; src && l < c; ++l) {

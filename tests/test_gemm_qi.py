@@ -686,3 +686,57 @@ def test_prefill_rope_cache_host_emulation(case):
 @pytest.mark.parametrize("case", ROPE + [(1999, 32, 8, 64, 0, 1, False)])
 def test_prefill_rope_cache_gpu(dev, case):
     run_rope_cache(GpuBackend(dev), *case)
+
+
+def run_mixed(O, be, tname, ns, k, T, ws, keep=False, seed=0):
+    """mrs_gemm_qi_mixed: tensors of Q6_K (all but the last `second` ones) and of another K-quant in one launch == every tensor's own launch, bit for bit."""
+    t6, t2 = O.Q6_K, getattr(O, tname)
+    types = [t6] + [t2] * (len(ns) - 1) if len(ns) < 3 or seed % 2 == 0 else [t6, t6, t2]
+    rng = np.random.default_rng(seed)
+    x = be.buf(rng.standard_normal((T, k)).astype(np.float32))
+    act = be.buf(np.zeros(be.sym("mrs_qi_act_bytes", [CI, CI], C.c_size_t)(T, k), np.uint8))
+    assert be.sym("mrs_qi_quantize_for", [CI, VP, VP, CI, VP, C.c_float, CI, CI, VP, VP, VP], CI)(t2, x.ptr, None, k, None, 1e-5, T, k, act.ptr, None, be.stream) == 0
+    wq, want = [], []
+    for i, (t, n) in enumerate(zip(types, ns)):
+        packed = O.quantize(t, (rng.standard_normal((n, k)) * 0.05).astype(np.float32)).reshape(n, -1)
+        src, w = be.buf(np.ascontiguousarray(packed).reshape(-1)), be.buf(np.zeros(be.sym("mrs_gemm_qi_repack_bytes", [CI, C.c_longlong, C.c_longlong], C.c_size_t)(t, n, k), np.uint8))
+        assert be.sym("mrs_gemm_qi_repack", [VP, CI, C.c_longlong, C.c_longlong, VP, VP], CI)(src.ptr, t, n, k, w.ptr, be.stream) == 0
+        o = be.buf(np.full((T, n), np.nan, np.float32))
+        assert be.sym("mrs_gemm_qi", [VP, CI, CI, CI, VP, CI, VP, CI, CI, VP], CI)(w.ptr, t, n, k, act.ptr, T, o.ptr, n, 0, be.stream) == 0
+        wq.append(w)
+        want.append(o.numpy())
+    outs = [be.buf(np.full((T, n + 3), 7.0, np.float32)) for n in ns]
+    nt, n_all = len(ns), sum(ns)
+    planes = be.buf(np.zeros(4 * T * n_all if ws else 1, np.float32))
+    f = be.sym("mrs_gemm_qi_mixed", [VP, CI, VP, VP, CI, VP, CI, VP, VP, VP, C.c_size_t, CI, VP], CI)
+    args = ((CI * nt)(*types), nt, (VP * nt)(*[w.ptr for w in wq]), (CI * nt)(*ns), k, act.ptr, T, (VP * nt)(*[o.ptr for o in outs]), (CI * nt)(*[n + 3 for n in ns]))
+    rc = f(*args, planes.ptr if ws else None, 16 * T * n_all if ws else 0, int(keep), be.stream)
+    assert rc == (be.sym("mrs_gemm_qi_is_cut", [CI, CI, VP, CI, CI], CI)(t2, nt, (CI * nt)(*ns), k, T) if keep and ws else 0)
+    if rc == 1:
+        p = planes.numpy().reshape(4, T, n_all)
+        got = np.split(((p[0] + p[1]) + p[2]) + p[3], np.cumsum(ns)[:-1], axis=1)
+    else:
+        got = [o.numpy()[:, :n] for o, n in zip(outs, ns)]
+        assert all((o.numpy()[:, n:] == 7.0).all() for o, n in zip(outs, ns))
+    for g, w in zip(got, want):
+        assert np.array_equal(g, w), (tname, ns, k, T, ws)
+    bad = (CI * nt)(*types[::-1])
+    assert f(bad, *args[1:], None, 0, 0, be.stream) == -1
+
+
+# one token tile and two, cut and whole, groups of runs, columns that do not fill a workgroup, both orders of three tensors
+MIXED = [("Q4_K", [40, 36], 512, 5, 0), ("Q4_K", [32, 132, 64], 1280, 34, 1), ("Q5_K", [64, 32, 160], 1024, 33, 1), ("Q4_K", [132, 8], 1024, 70, 0), ("Q5_K", [36, 128], 2816, 3, 1)]
+
+
+@pytest.mark.parametrize("tname,ns,k,T,ws", MIXED)
+def test_gemm_qi_mixed_host_emulation(oracle, tname, ns, k, T, ws):
+    run_mixed(oracle, HostBackend(), tname, ns, k, T, ws, seed=T)
+    run_mixed(oracle, HostBackend(), tname, ns, k, T, ws, keep=True, seed=T + 1)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("tname,ns,k,T,ws", MIXED + [("Q4_K", [1024, 4096, 1024], 4096, T, 1) for T in (4, 37, 64, 130, 300, 700)] + [("Q4_K", [1024, 12288], 4096, 33, 0),
+                                                    ("Q5_K", [1024, 4096], 4096, 200, 1), ("Q4_K", [1024, 27648], 4096, 5, 0)])
+def test_gemm_qi_mixed_gpu(oracle, dev, tname, ns, k, T, ws):
+    run_mixed(oracle, GpuBackend(dev), tname, ns, k, T, ws, seed=T)
+    run_mixed(oracle, GpuBackend(dev), tname, ns, k, T, ws, keep=True, seed=T + 1)
