@@ -326,15 +326,24 @@ __device__ __forceinline__ void wide_place(int &bx, int &by) {  // workgroup col
   const int in_cols = order - cols0 * (int)gridDim.y;
   by = in_cols / cols; bx = cols0 + in_cols % cols;
 }
+// the rows from token tile by's first (of `tile` rows each) to its window's last, and its expert; false: past the last tile
+__device__ __forceinline__ bool wide_rows(const WideArgs &a, int by, int tile, int &t0, int &tend, int &ex) {
+  int tbeg = 0, yt = by;
+  tend = a.T; ex = 0;
+  if (a.bounds && !expert_tile(a.bounds, a.experts, tile, yt, ex, tbeg, tend)) return false;
+  t0 = tbeg + yt * tile;
+  return t0 < tend;
+}
 template <int TYPE, int NT, int MODE>
-__device__ __forceinline__ void wide_body(const WideArgs &a, const int bx, const int by, char *const smem_all) {
+__device__ __forceinline__ void wide_body(const WideArgs &a, const int bx, const int t0, const int tend, const int ex, char *const smem_all) {
 #include "qi_wide_body.cuh"
 }
 template <int TYPE, int NT, int MODE>
 __global__ void __launch_bounds__(256 * wide_groups(MODE), (wide_waves<TYPE, NT, MODE>)) gemm_qi_wide_kernel(const WideArgs a) {
   extern __shared__ __attribute__((aligned(16))) char smem_all[];
-  int bx, by;
+  int bx, by, t0, tend, ex;
   wide_place(bx, by);
+  if (!wide_rows(a, by, 32 * NT, t0, tend, ex)) return;
 #include "qi_wide_body.cuh"
 }
 // Tensors of two K-quants on the same operand rows (value projections of Q6_K beside queries and keys of Q4_K) in one launch: the columns before a.xm hold TA, the others TB.  A launch of
@@ -345,10 +354,22 @@ __global__ void __launch_bounds__(256 * wide_groups(MODE), (wide_waves<TYPE, NT,
 template <int TA, int TB, int NT, int MODE>
 __global__ void __launch_bounds__(256 * wide_groups(MODE), (wide_waves<TA, NT, MODE> < wide_waves<TB, NT, MODE> ? wide_waves<TA, NT, MODE> : wide_waves<TB, NT, MODE>)) gemm_qi_mixed_kernel(const WideArgs a) {
   extern __shared__ __attribute__((aligned(16))) char smem_all[];
-  int bx, by;
+  int bx, by, t0, tend, ex;
   wide_place(bx, by);
-  if (bx < a.xm) wide_body<TA, NT, MODE>(a, bx, by, smem_all);
-  else wide_body<TB, NT, MODE>(a, bx, by, smem_all);
+  if (!wide_rows(a, by, 32 * NT, t0, tend, ex)) return;
+  if (bx < a.xm) wide_body<TA, NT, MODE>(a, bx, t0, tend, ex, smem_all);
+  else wide_body<TB, NT, MODE>(a, bx, t0, tend, ex, smem_all);
+}
+// Experts' windows in workgroups of two token tiles: where a window's last workgroup has 32 rows or less (every other one on average), one tile does (K-quants; the Q8_0 form would spill).
+// gate and up of 8 experts of 14336 x 4096, top-2, us, without / with: Q4_K 300 tokens 297 / 260, 512 375 / 351, 800 513 / 490, 1200 717 / 709; Q5_K 300 354 / 322, 600 512 / 479.
+template <int TYPE>
+__global__ void __launch_bounds__(256, 2) gemm_qi_tail_kernel(const WideArgs a) {
+  extern __shared__ __attribute__((aligned(16))) char smem_all[];
+  int bx, by, t0, tend, ex;
+  wide_place(bx, by);
+  if (!wide_rows(a, by, 64, t0, tend, ex)) return;
+  if (tend - t0 <= 32) wide_body<TYPE, 1, W_ONE>(a, bx, t0, tend, ex, smem_all);
+  else wide_body<TYPE, 2, W_ONE>(a, bx, t0, tend, ex, smem_all);
 }
 
 // The projections of a prompt's tokens on their way to the attention: RoPE on q and k (rope_pair in f32, as rotary_embedding_positions), k and v into their pages (rounded as
@@ -568,11 +589,23 @@ template <int TB> static void mixed_launch(int NT, int mode, const qi::WideArgs 
   }
   NT == 2 ? mixed_go<T_Q6_K, TB, 2, qi::W_ONE>(a, grid, s) : mixed_go<T_Q6_K, TB, 1, qi::W_ONE>(a, grid, s);
 }
+// gemm_qi_tail_kernel from this many workgroups on.  Fewer are a few rounds of the 512 that are resident, whose last is as long either way, and a launch of uneven workgroups meets it
+// later (down of 4096 x 14336, us, without / with: Q4_K 512 tokens 201 / 216, 600 228 / 244, 1200 (1440 workgroups) 358 / 360; Q6_K 200 122 / 130).  Rows without windows (one last tile of
+// many) gain and lose under 1 %: 28672 x 4096, 650 tokens 194 / 193, 1999 541 / 549.
+constexpr unsigned TAIL_MIN = 2048;
 template <int TYPE> static void wide_launch(int NT, int mode, const qi::WideArgs &a, dim3 grid, hipStream_t s) {
   if (mode == qi::W_PAIR) return wide_go<TYPE, 1, qi::W_PAIR>(a, grid, s);
   if constexpr (TYPE != T_Q5_K) {
     if (mode == qi::W_RUNS2) return wide_go<TYPE, 2, qi::W_RUNS2>(a, grid, s);
     if (mode == qi::W_RUNS4) return wide_go<TYPE, 1, qi::W_RUNS4>(a, grid, s);
+  }
+  if constexpr (TYPE != T_Q8_0) {
+    if (NT == 2 && a.bounds && grid.x * grid.y >= TAIL_MIN) {
+      auto kern = qi::gemm_qi_tail_kernel<TYPE>;
+      lds_attr_once((const void *)kern, 158 * 1024);
+      hipLaunchKernelGGL(kern, grid, dim3(256), (wide_lds<TYPE, 2, qi::W_ONE>), s, a);
+      return;
+    }
   }
   NT == 2 ? wide_go<TYPE, 2, qi::W_ONE>(a, grid, s) : wide_go<TYPE, 1, qi::W_ONE>(a, grid, s);
 }

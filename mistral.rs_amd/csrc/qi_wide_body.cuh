@@ -1,5 +1,5 @@
-// qi_wide_body.cuh -- the body of gemm_qi_wide_kernel<TYPE, NT, MODE> and of wide_body<TYPE, NT, MODE> (ext_gemm_qi.hip): `a` the arguments, `bx`, `by` the workgroup's column and token tile,
-// `smem_all` its LDS.  Text of both and not a function that the kernel calls: hipcc allocates the registers of an inlined function otherwise, and the Q8_0 forms, which fill theirs, spill
+// qi_wide_body.cuh -- the body of gemm_qi_wide_kernel<TYPE, NT, MODE> and of wide_body<TYPE, NT, MODE> (ext_gemm_qi.hip): `a` the arguments, `bx` the workgroup's column, `t0` .. `tend` the rows
+// from its tile's first to its window's last, `ex` its expert, `smem_all` its LDS.  Text of both and not a function that the kernel calls: hipcc allocates the registers of an inlined function otherwise, and the Q8_0 forms, which fill theirs, spill
 // (two token tiles 208 -> 256 registers and 400 bytes of scratch per lane).
   constexpr int TT_ = NT * 32, ROWB = WIDE_ROW, ACT_ = TT_ * ROWB, BUF_ = wide_buf<TYPE, NT>, YD_ = 512;
   constexpr int NPC = TYPE == T_Q4_K ? 4 : 8;  // 1-KiB pieces of a record
@@ -10,11 +10,7 @@
   const int seg = bx >= a.x2 ? 2 : bx >= a.x1 ? 1 : 0;
   const QiSeg sg = seg == 2 ? a.s2 : seg == 1 ? a.s1 : a.s0;
   const int coff = seg == 2 ? a.s0.N + a.s1.N : seg == 1 ? a.s0.N : 0;
-  int tbeg = 0, tend = a.T, yt = by, ex = 0;
-  if (a.bounds && !expert_tile(a.bounds, a.experts, TT_, yt, ex, tbeg, tend)) return;
   const uint8_t *wbase = sg.w + (size_t)ex * sg.w_bytes;
-  const int t0 = tbeg + yt * TT_;
-  if (t0 >= tend) return;
   const int S = a.K / 256, Cs = (S + 3) / 4;
   const __amdgpu_buffer_rsrc_t rw = __builtin_amdgcn_make_buffer_rsrc((void *)wbase, (short)0, (int)sg.w_bytes, 0x00020000);
   const unsigned panel = (unsigned)((bx - (seg == 2 ? a.x2 : seg == 1 ? a.x1 : 0)) * 4 + wave);

@@ -740,3 +740,17 @@ def test_gemm_qi_mixed_host_emulation(oracle, tname, ns, k, T, ws):
 def test_gemm_qi_mixed_gpu(oracle, dev, tname, ns, k, T, ws):
     run_mixed(oracle, GpuBackend(dev), tname, ns, k, T, ws, seed=T)
     run_mixed(oracle, GpuBackend(dev), tname, ns, k, T, ws, keep=True, seed=T + 1)
+
+
+# windows that end with 1, 32, 33 and 64 rows in their last workgroup of 64, an empty one, and enough workgroups (2048) for the kernel that takes a short end in one token tile
+TAIL = [0, 65, 65, 161, 258, 322]
+
+
+def test_gemm_qi_window_tails_host_emulation(oracle):
+    run_multi(oracle, HostBackend(), "Q4_K", [26624], 256, TAIL[-1], bounds=TAIL, seed=9)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("tname,ns,k", [("Q4_K", [14336, 14336], 512), ("Q6_K", [26624], 256), ("Q5_K", [14336, 14336], 256)])
+def test_gemm_qi_window_tails_gpu(oracle, dev, tname, ns, k):
+    run_multi(oracle, GpuBackend(dev), tname, ns, k, TAIL[-1], bounds=TAIL, seed=9)
