@@ -159,8 +159,7 @@ __device__ __forceinline__ void store_operands(const QuantArgs &a, int sb, int t
   if (i == 0) a.yd[row] = d[0];
 }
 // rows with a norm.  GLU: the activated row goes through xtmp.  PART: the row is h + ((c0 + c1) + c2) + c3, the sum gemm_qi_reduce_kernel would have left in h (written there as
-// well), formed in the registers the norm reads: a launch less between a cut product and the next one's operands (rows of up to 2048 NPX values; 37 rows of 4096 4.1 + 4.9 us, here
-// 5.6, 512 rows 5.0 + 7.0, here 12.0 with the planes from memory).
+// well), formed in the registers the norm reads: a launch less between a cut product and the next one's operands (rows of up to 2048 NPX values).
 template <bool GLU, bool PART>
 __global__ void __launch_bounds__(NT) qi_quantize_kernel(const QuantArgs a) {
   extern __shared__ __attribute__((aligned(16))) char smem[];
@@ -234,6 +233,65 @@ __global__ void __launch_bounds__(64 * QS_WAVES) qi_quantize_split_kernel(const 
   if (sb0 + n >= S) return;
   const Act act = act_view(img_s[wave], 512, 1, a.mode);
   store_operands(a, sb0 + n, t, act.q + act.qoff(n), act.d + n * act.dw, act.bs + n * ACT_BS, lane & 31, 32);
+}
+
+// rows with a norm of up to 4096 values (two superblocks per wave).  A launch of few rows is one chain of latencies, one of many rows as many chains as fit: here a wave's superblocks v
+// and v + 8 stay in its registers from the request to the quants and the wave writes its own operands through an image of its own, so that one barrier is left (the sums of
+// squares) and 30 registers (PART 53, where the kernel above takes 98: four workgroups per CU instead of two).  Rows of 4096, us, the kernel above / this: 4 rows 3.8 / 3.3, 37
+// 4.1 / 3.4, 512 5.5 / 4.7, 1999 13.3 / 11.0 (49 MB); PART 37 4.9 / 4.0, 512 11.3 / 9.4, 700 15.1 / 12.4 (80 MB); rows of 2048, 37 3.9 / 3.4, 1999 11.1 / 9.9.
+template <bool PART>
+__global__ void __launch_bounds__(NT, 8) qi_quantize_norm_kernel(const QuantArgs a) {
+  __shared__ __attribute__((aligned(16))) char img_s[8][QS_IMG];
+  __shared__ float red[8];
+  const int tid = tid_opaque(), lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), t = blockIdx.x, S = a.K / 256;
+  const __amdgpu_buffer_rsrc_t rx = __builtin_amdgcn_make_buffer_rsrc((void *)(a.x + (size_t)t * a.ldx), (short)0, a.K * 4, 0x00020000);
+  const __amdgpu_buffer_rsrc_t rw = __builtin_amdgcn_make_buffer_rsrc((void *)a.norm_w, (short)0, a.K * 4, 0x00020000);
+  const unsigned off = (unsigned)tid * 16u;  // of piece 0 = superblock `wave`; piece 1 = superblock wave + 8 (past the row: zeros)
+  float4 v[2], w[2];
+#pragma unroll
+  for (int n = 0; n < 2; ++n) v[n] = as_f4(__builtin_amdgcn_raw_buffer_load_b128(rx, off + (unsigned)n * 8192u, 0, 0));
+  if constexpr (PART) {
+    const size_t tot = (size_t)a.T * a.K;
+    float4 c[4][2];
+#pragma unroll
+    for (int p = 0; p < 4; ++p) {
+      const __amdgpu_buffer_rsrc_t rp = __builtin_amdgcn_make_buffer_rsrc((void *)(a.part + p * tot + (size_t)t * a.K), (short)0, a.K * 4, 0x00020000);
+#pragma unroll
+      for (int n = 0; n < 2; ++n) c[p][n] = as_f4(__builtin_amdgcn_raw_buffer_load_b128(rp, off + (unsigned)n * 8192u, 0, 0));
+    }
+#pragma unroll
+    for (int n = 0; n < 2; ++n) w[n] = as_f4(__builtin_amdgcn_raw_buffer_load_b128(rw, off + (unsigned)n * 8192u, 0, 0));
+    const __amdgpu_buffer_rsrc_t rh = __builtin_amdgcn_make_buffer_rsrc((void *)(a.h + (size_t)t * a.K), (short)0, a.K * 4, 0x00020000);
+#pragma unroll
+    for (int n = 0; n < 2; ++n) {
+      v[n] = make_float4(v[n].x + (((c[0][n].x + c[1][n].x) + c[2][n].x) + c[3][n].x), v[n].y + (((c[0][n].y + c[1][n].y) + c[2][n].y) + c[3][n].y),
+                         v[n].z + (((c[0][n].z + c[1][n].z) + c[2][n].z) + c[3][n].z), v[n].w + (((c[0][n].w + c[1][n].w) + c[2][n].w) + c[3][n].w));
+      const v4u h4 = {__float_as_uint(v[n].x), __float_as_uint(v[n].y), __float_as_uint(v[n].z), __float_as_uint(v[n].w)};
+      __builtin_amdgcn_raw_buffer_store_b128(h4, rh, off + (unsigned)n * 8192u, 0, 0);
+    }
+  } else {
+#pragma unroll
+    for (int n = 0; n < 2; ++n) w[n] = as_f4(__builtin_amdgcn_raw_buffer_load_b128(rw, off + (unsigned)n * 8192u, 0, 0));
+  }
+  float ss = 0.f;  // the engine's order: x y z w of piece 0, then of piece 1 (zeros past the row change nothing)
+#pragma unroll
+  for (int n = 0; n < 2; ++n) { ss = fmaf(v[n].x, v[n].x, ss); ss = fmaf(v[n].y, v[n].y, ss); ss = fmaf(v[n].z, v[n].z, ss); ss = fmaf(v[n].w, v[n].w, ss); }
+  ss = wave_sum_all(ss);
+  if (lane == 0) red[wave] = ss;
+  __syncthreads();
+  if (wave >= S) return;  // no workgroup barrier below
+  const float total = ((red[0] + red[1]) + (red[2] + red[3])) + ((red[4] + red[5]) + (red[6] + red[7]));
+  const float nm = sqrtf(total / (float)a.K + a.eps), inv = 1.0f / nm;
+#pragma unroll
+  for (int n = 0; n < 2; ++n) v[n] = norm4(v[n], w[n], nm, inv);
+  const int sbs[2] = {0, 1};
+  const bool live[2] = {true, true};
+  quantize_multi<2>(v, sbs, live, 0, a.mode, img_s[wave], 512, 1);
+  MRS_WAVE_SYNC();
+  const int n = lane >> 5, sb = wave + 8 * n;
+  if (sb >= S) return;
+  const Act act = act_view(img_s[wave], 512, 1, a.mode);
+  store_operands(a, sb, t, act.q + act.qoff(n), act.d + n * act.dw, act.bs + n * ACT_BS, lane & 31, 32);
 }
 
 // ------------------------------------------------------------------------------------------------ the GEMM
@@ -515,6 +573,12 @@ extern "C" int mrs_qi_quantize(const float *x, const float *x2, int ldx, const f
 static size_t row_image_lds(int K) { return (dec2::act_bytes(K, 1) + 15) & ~(size_t)15; }
 constexpr size_t ROW_IMAGE_MAX = (size_t)158 * 1024;
 template <bool GLU, bool PART> static int qi_quantize_rows(const qi::QuantArgs &a, void *stream) {  // rows with a norm
+  if constexpr (!GLU) {
+    if (a.K <= 4096) {  // 16 superblocks, two of each wave: longer rows keep the image of a whole row
+      hipLaunchKernelGGL(qi::qi_quantize_norm_kernel<PART>, dim3(a.T), dim3(dec2::NT), 0, (hipStream_t)stream, a);
+      return 0;
+    }
+  }
   const size_t lds = row_image_lds(a.K);
   auto kern = qi::qi_quantize_kernel<GLU, PART>;
   lds_attr_once((const void *)kern, ROW_IMAGE_MAX);

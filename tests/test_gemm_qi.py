@@ -754,3 +754,40 @@ def test_gemm_qi_window_tails_host_emulation(oracle):
 @pytest.mark.parametrize("tname,ns,k", [("Q4_K", [14336, 14336], 512), ("Q6_K", [26624], 256), ("Q5_K", [14336, 14336], 256)])
 def test_gemm_qi_window_tails_gpu(oracle, dev, tname, ns, k):
     run_multi(oracle, GpuBackend(dev), tname, ns, k, TAIL[-1], bounds=TAIL, seed=9)
+
+
+def run_norm_rows(O, be, tname, T, k):
+    """The quantizer of rows with a norm == the engine's norm and the quantizer of rows without, byte for byte."""
+    t = getattr(O, tname)
+    rng = np.random.default_rng(k + T)
+    x, nw = rng.standard_normal((T, k + 8)).astype(np.float32), (1 + 0.1 * rng.standard_normal(k)).astype(np.float32)
+    x[T - 1, k - min(k, 256):] = 0.0  # the last superblock
+    x[0, :k] *= np.float32(1e4)
+    nbytes = be.sym("mrs_qi_act_bytes", [CI, CI], C.c_size_t)(T, k)
+    xb, yb, nwb = be.buf(x), be.buf(O.rms_norm_engine(np.ascontiguousarray(x[:, :k]), nw, 1e-5)), be.buf(nw)
+    got, want = be.buf(np.full(nbytes, 0xA5, np.uint8)), be.buf(np.full(nbytes, 0xA5, np.uint8))
+    quantize = be.sym("mrs_qi_quantize_for", [CI, VP, VP, CI, VP, C.c_float, CI, CI, VP, VP, VP], CI)
+    assert quantize(t, xb.ptr, None, k + 8, nwb.ptr, 1e-5, T, k, got.ptr, None, be.stream) == 0
+    assert quantize(t, yb.ptr, None, k, None, 0.0, T, k, want.ptr, None, be.stream) == 0
+    assert np.array_equal(got.numpy(), want.numpy())
+
+
+# waves without a superblock, with one and with two, and the first row that is too long for two per wave; rows that are not next to each other
+NORM_ROWS = [(tname, T, k) for tname in ("Q4_K", "Q8_0") for T, k in ((3, 256), (2, 1792), (1, 2048), (2, 2304), (5, 4096), (2, 4352))]
+
+
+@pytest.mark.parametrize("tname,T,k", NORM_ROWS)
+def test_norm_rows_host_emulation(oracle, tname, T, k):
+    run_norm_rows(oracle, HostBackend(), tname, T, k)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("tname,T,k", NORM_ROWS + [("Q4_K", 1025, 4096), ("Q8_0", 700, 2560)])
+def test_norm_rows_gpu(oracle, dev, tname, T, k):
+    run_norm_rows(oracle, GpuBackend(dev), tname, T, k)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("tname,T,d", [("Q4_K", 2, 1792), ("Q8_0", 3, 2304), ("Q4_K", 2, 4352)])
+def test_added_rows_of_every_length_gpu(oracle, dev, tname, T, d):
+    run_added_rows(oracle, GpuBackend(dev), tname, T, d, 2048)
