@@ -232,7 +232,9 @@
     };
     constexpr int DIGIT = TYPE == T_Q4_K ? 3 : 8;
     constexpr bool EARLY = MODE != W_RUNS4;  // the next superblock's rows are requested in front of the matrix instructions, all of them (in 16 waves' 128 registers: one by one behind them)
-    i4v fr[2][NT];
+    // the activations' fragments are read from LDS two steps ahead where the registers hold them (not in 16 waves' 128; Q5_K spills)
+    constexpr int AHEAD = MODE == W_RUNS4 || TYPE == T_Q5_K ? 1 : 2;
+    i4v fr[AHEAD + 1][NT];
     unsigned wl[2][4], wh[2][4];
     scales(0);
 #pragma unroll
@@ -258,17 +260,24 @@
     // behind each matrix instruction of a step stands a share of the next step's operand build, behind the first of a token tile also the tile's next read and a piece of the next
     // superblock's DMA: the wave's own vector and memory instructions run under its matrix instructions (scheduling barriers keep the order)
 #pragma unroll
-    for (int tt = 0; tt < NT; ++tt) fr[0][tt] = frag(0, tt);
+    for (int i = 0; i < AHEAD; ++i)
+#pragma unroll
+      for (int tt = 0; tt < NT; ++tt) fr[i][tt] = frag(i, tt);
     __builtin_amdgcn_sched_barrier(0);
+    // the matrix instructions' part of a superblock goes in front of the other waves' terms and operand builds: with equal priorities two waves of a SIMD drift into step, both in the
+    // matrix instructions or both in the terms, and neither pipe is full.  us, equal / so: Q4_K 6144 x 4096, 512 tokens 36.8 / 34.7, 4096 x 14336, 1999 tokens 262 / 252; Q6_K
+    // 4096 x 14336, 512 tokens 85.1 / 81.2, 1999 306 / 301; Q4_K 28672 x 4096, 1999 tokens 527 / 521 (the clock falls).  The other way round (the terms in front) and the barrier's part
+    // with the matrix instructions': nothing
+    __builtin_amdgcn_s_setprio(1);
 #pragma unroll
     for (int k = 0; k < 8; ++k) {
       const int c = k & 1, nx = c ^ 1;
       const i4v lo = {(int)wl[c][0], (int)wl[c][1], (int)wl[c][2], (int)wl[c][3]}, hi = {(int)wh[c][0], (int)wh[c][1], (int)wh[c][2], (int)wh[c][3]};
 #pragma unroll
       for (int tt = 0; tt < NT; ++tt) {
-        XL[tt] = __builtin_amdgcn_mfma_i32_32x32x32_i8(fr[c][tt], lo, XL[tt], 0, 0, 0);
+        XL[tt] = __builtin_amdgcn_mfma_i32_32x32x32_i8(fr[k % (AHEAD + 1)][tt], lo, XL[tt], 0, 0, 0);
+        if (k + AHEAD < 8) fr[(k + AHEAD) % (AHEAD + 1)][tt] = frag(k + AHEAD, tt);
         if (k + 1 < 8) {
-          fr[nx][tt] = frag(k + 1, tt);
           if (tt == 0) scales(k + 1);
 #pragma unroll
           for (int p = tt * 4 / NT; p < tt * 4 / NT + 2 / NT; ++p) digits(k + 1, p, wl[nx][p], wh[nx][p]);
@@ -278,7 +287,7 @@
           for (int i = 0; i < NSTAGE; ++i) if (tt == 0 && k == i * (8 / NSTAGE)) stage_q(sb + STEP, it + 1, i, more);
         }
         __builtin_amdgcn_sched_barrier(0);
-        XH[tt] = __builtin_amdgcn_mfma_i32_32x32x32_i8(fr[c][tt], hi, XH[tt], 0, 0, 0);
+        XH[tt] = __builtin_amdgcn_mfma_i32_32x32x32_i8(fr[k % (AHEAD + 1)][tt], hi, XH[tt], 0, 0, 0);
         if (k + 1 < 8) {
 #pragma unroll
           for (int p = tt * 4 / NT + 2 / NT; p < (tt + 1) * 4 / NT; ++p) digits(k + 1, p, wl[nx][p], wh[nx][p]);
@@ -289,6 +298,7 @@
         __builtin_amdgcn_sched_barrier(0);
       }
     }
+    __builtin_amdgcn_s_setprio(0);
     const float *yd_s = (const float *)meta_s;
     const f32v zero32 = {0.f};
     // d yd (and dmin yd) of the tile's outputs, each product rounded once: one matrix instruction of two 32 x 32 outer products (lane halves = blocks).  It adds the products to + 0, so

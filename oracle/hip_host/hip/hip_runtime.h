@@ -479,6 +479,7 @@ static inline void hiphost_buffer_load_lds(__amdgpu_buffer_rsrc_t r, char *dst, 
 #define MRS_KEEP_BRANCH() ((void)0)
 #define __builtin_amdgcn_fence(ORDER, SCOPE) ((void)0)                  /* one workgroup runs at a time: nothing to order */
 #define __builtin_amdgcn_s_sleep(N) ((void)0)
+#define __builtin_amdgcn_s_setprio(N) ((void)0)                     /* issue-order hint only */
 #define __HIP_MEMORY_SCOPE_AGENT 4
 #define __hip_atomic_fetch_add(P, V, ORDER, SCOPE) atomicAdd((P), (V))
 static inline void __threadfence() {}
