@@ -583,6 +583,35 @@ __global__ void __launch_bounds__(NT) dec_act_image_kernel(const ActImgArgs a) {
   const int c0 = a.rows ? c : a.gc0[c], n = a.rows ? 1 : a.gn[c];
   act_quantize_all<1, 1>(a.img + act_bytes(a.K, c0), red, pre, x, a.ldx, a.norm_w, a.eps, a.K, a.mode, wave, c - c0, n);
 }
+// Rows with a norm of up to 4096 values: a wave has two superblocks and keeps them in 8 registers; without the paths of longer rows the launch, one chain of latencies, is shorter by
+// what it takes to fetch and pass them.  8 rows of 4096 for K-quants, us, the kernel above / this: 3.86 / 3.57; a decode step of 32 layers (65 such launches) 2481 / 2454.
+__global__ void __launch_bounds__(NT) dec_act_image_short_kernel(const ActImgArgs a) {
+  __shared__ float red[8];
+  const int tid = tid_opaque(), lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int c = (int)blockIdx.x, S = a.K / 256;
+  const __amdgpu_buffer_rsrc_t rx = __builtin_amdgcn_make_buffer_rsrc((void *)(a.x + (size_t)c * a.ldx), (short)0, a.K * 4, 0x00020000);
+  const __amdgpu_buffer_rsrc_t rw = __builtin_amdgcn_make_buffer_rsrc((void *)a.norm_w, (short)0, a.K * 4, 0x00020000);
+  float4 v[2], w[2];
+#pragma unroll
+  for (int n = 0; n < 2; ++n) v[n] = as_f4(__builtin_amdgcn_raw_buffer_load_b128(rx, (unsigned)tid * 16u + (unsigned)n * 8192u, 0, 0));  // superblocks wave, wave + 8; past the row: zeros
+#pragma unroll
+  for (int n = 0; n < 2; ++n) w[n] = as_f4(__builtin_amdgcn_raw_buffer_load_b128(rw, (unsigned)tid * 16u + (unsigned)n * 8192u, 0, 0));
+  float ss = 0.f;  // the order of act_sumsq_all
+#pragma unroll
+  for (int n = 0; n < 2; ++n) { ss = fmaf(v[n].x, v[n].x, ss); ss = fmaf(v[n].y, v[n].y, ss); ss = fmaf(v[n].z, v[n].z, ss); ss = fmaf(v[n].w, v[n].w, ss); }
+  ss = wave_sum_all(ss);
+  if (lane == 0) red[wave] = ss;
+  __syncthreads();
+  if (wave >= S) return;
+  const float tot = ((red[0] + red[1]) + (red[2] + red[3])) + ((red[4] + red[5]) + (red[6] + red[7]));
+  const float nm = sqrtf(tot / (float)a.K + a.eps), inv = 1.0f / nm;
+#pragma unroll
+  for (int n = 0; n < 2; ++n) v[n] = norm4(v[n], w[n], nm, inv);
+  const int sb[2] = {wave, wave + 8};
+  const bool live[2] = {true, wave + 8 < S};
+  const int c0 = a.rows ? c : a.gc0[c], n = a.rows ? 1 : a.gn[c];
+  quantize_multi<2>(v, sb, live, c - c0, a.mode, a.img + act_bytes(a.K, c0), a.K, n);
+}
 // Rows without a norm (down_proj's): a superblock knows nothing of the others, so four waves take two each and a row spreads over K / 2048 workgroups; one workgroup per row was a
 // serial chain of seven superblocks per wave.  A decode step of 32 layers with 14336 values per row, us: 2 rows 2487 / 2363, 8 rows 2875 / 2726 (the launch alone: 4.7 and 4.4, of
 // which about 3 are an empty launch's in the trace).
@@ -600,7 +629,8 @@ __global__ void __launch_bounds__(256) dec_act_image_split_kernel(const ActImgAr
   quantize_multi<2>(v, sb, live, c - c0, a.mode, a.img + act_bytes(a.K, c0), a.K, n);
 }
 static void act_image_launch(const ActImgArgs &a, int rows, hipStream_t s) {
-  if (a.norm_w) hipLaunchKernelGGL(dec_act_image_kernel, dim3(rows), dim3(NT), 0, s, a);
+  if (a.norm_w && a.K <= 4096) hipLaunchKernelGGL(dec_act_image_short_kernel, dim3(rows), dim3(NT), 0, s, a);
+  else if (a.norm_w) hipLaunchKernelGGL(dec_act_image_kernel, dim3(rows), dim3(NT), 0, s, a);
   else hipLaunchKernelGGL(dec_act_image_split_kernel, dim3(rows, (a.K / 256 + 7) / 8), dim3(256), 0, s, a);
 }
 // the column groups of a batch of b columns of K values: halved until a group's image fits LDS (the same recursion as Launch::run)

@@ -712,3 +712,28 @@ def test_router_with_fused_norm_gpu(dev, tokens, E, K, topk):
 @pytest.mark.parametrize("tokens,E,K,topk,bad", ROUTER_LIMITS)
 def test_router_rows_and_logits_at_their_limits_gpu(dev, tokens, E, K, topk, bad):
     _check_router_norm(GpuBackend(dev), tokens, E, K, topk, bad)
+
+
+def check_norm_image(O, be, tname, k, b):
+    """The image of rows with a norm == the image of the engine's normed rows, byte for byte."""
+    t = getattr(O, tname)
+    rng = np.random.default_rng(k + b)
+    x, nw = rng.standard_normal((b, k)).astype(np.float32), (1.0 + 0.1 * rng.standard_normal(k)).astype(np.float32)
+    x[b - 1, k - 256:] = 0.0
+    xb, yb, nb = be.buf(x), be.buf(O.rms_norm_engine(x, nw, 1e-5)), be.buf(nw)
+    assert np.array_equal(_act_image(be, t, xb, nb, k, b).numpy(), _act_image(be, t, yb, None, k, b).numpy())
+
+
+# waves without a superblock, with one and with two, and the first row that is too long for two per wave
+NORM_IMAGES = [(tname, k, b) for tname in ("Q4_K", "Q8_0") for k, b in ((256, 3), (1792, 2), (2048, 1), (2304, 8), (4096, 8), (4352, 2))]
+
+
+@pytest.mark.parametrize("tname,k,b", NORM_IMAGES)
+def test_norm_image_host_emulation(oracle, tname, k, b):
+    check_norm_image(oracle, HostBackend(), tname, k, b)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("tname,k,b", NORM_IMAGES)
+def test_norm_image_gpu(oracle, dev, tname, k, b):
+    check_norm_image(oracle, GpuBackend(dev), tname, k, b)
