@@ -681,22 +681,23 @@ static int window_tiles(int type, int rows, int cols) {
   return rows <= 32 || (type == T_Q8_0 && rows > 64 && rows < 256) || cols * ((rows + 63) / 64) <= (type == T_Q5_K ? 96 : 32) ? 1 : 2;
 }
 // Every other launch: token tiles per wave (NT), groups of waves per workgroup (mode), cut by runs of superblocks (cut) or whole.  The lines are drawn through the times of all seven forms
-// at 9900 sizes (512 .. 32768 rows of weights, K = 1024 .. 28672, 1 .. 2000 tokens, weights from HBM): against the fastest form of each size the one taken costs 0.1 - 0.3 % on average
-// for 1 .. 32 tokens, 0.2 - 0.4 % to 128, 0.4 - 1.0 % beyond; lines drawn through some 40 sizes whose weights lay in the last-level cache cost 1 - 8 % and were up to 1.25 times slower
+// at 9900 sizes (512 .. 32768 rows of weights, K = 1024 .. 28672, 1 .. 2000 tokens, weights from HBM), and those of the K-quants again at 9100 sizes (1000 .. 32000 rows, K = 1024 ..
+// 14336) since their products multiply in int8: against the fastest form of each size the one taken costs 1.3 % on average (Q4_K; K = 1024, cut where whole is 15 % faster, 3.8), 0.5 %
+// (Q5_K; 1.2 before), 0.8 % (Q6_K), Q8_0 0.1 - 1.0 %; lines drawn through some 40 sizes whose weights lay in the last-level cache cost 1 - 8 % and were up to 1.25 times slower
 // than no groups at all.  w1, w2: workgroups of one and of two token tiles.  Times in us, Q4_K unless named:
 //   * at most a workgroup per CU, and `line` of them or more: whole, one tile, the four runs in four groups.  A cut launch has more of the chip but writes and reads four planes of the
 //     outputs, so the line falls as the tiles fill.  Cut / so: 2048 x 2048, 128 tokens (w1 64) 10.3 / 11.7, 3072 x 2048 (96) 12.8 / 12.3; 16384 x 4096, 5 tokens (128) 15.9 / 19.0,
-//     28672 x 4096 (224) 24.8 / 21.6; cut with two tiles / so: 5120 x 4096, 128 tokens (160) 21.8 / 18.4.  With one tile or an odd number of them nothing above 208 is cut: four times
-//     that is a little more than three rounds (28672 x 8192, 5 tokens (224) 39.9 / 36.1).  One group instead of four: Q5_K, whose kernel spills at 16 waves; Q4_K and Q6_K where a run is
+//     28672 x 4096 (224) 24.8 / 21.6; cut with two tiles / so: 5120 x 4096, 128 tokens (160) 21.8 / 18.4.  With one tile or an odd number of them nothing above 208 is cut (Q4_K with one tile: 192): four
+//     times that is three rounds or a little more (28672 x 8192, 5 tokens (224) 39.9 / 36.1; 24832 x 4096 (194), 5 tokens 23.4 / 18.9).  One group instead of four: Q5_K, whose kernel spills at 16 waves; Q4_K and Q6_K where a run is
 //     one superblock (Q6_K 16384 x 1024, 32 tokens 11.3 / 12.8); Q6_K with 32 tokens or less below K = 4096 (28672 x 2048, 5 tokens 18.7 / 21.3).
 //   * two tiles, at most a workgroup per CU: two groups.  Cut / so: 28672 x 8192, 64 tokens (w2 224) 59.4 / 52.5, 8192 x 8192, 256 tokens (256) 58.5 / 51.1, whole / so 54.0 / 51.1.
-//   * else one tile or two by time(), the superblocks in a row on the busiest CU, of which two tiles take 1.5 - 1.8 times as long.  One / two: 12288 x 4096, 160 tokens (w1 480, w2 288)
-//     33.0 / 42.2, 28672 x 4096, 512 tokens 198 / 164; Q8_0 5120 x 4096, 800 tokens (1000, 520) 63.2 / 88.7; cut: 4096 x 4096, 64 tokens (64, 32) 13.5 / 14.9, 96 tokens (96, 64)
-//     16.9 / 16.4.  Whole / cut with two tiles: 8192 x 8192, 320 tokens (w2 320) 81.0 / 73.3, 448 tokens (448) 88.8 / 98.5; long rows also where a second, partly filled round of
+//   * else one tile or two by time(), the superblocks in a row on the busiest CU, of which two tiles take 1.4 (Q5_K) - 1.8 times as long.  One / two: 12288 x 4096, 160 tokens (w1 480, w2 288)
+//     33.0 / 42.2, 28672 x 4096, 512 tokens 198 / 164; Q5_K 7808 x 4096, 1047 tokens 140 / 124, cut 3200 x 4096, 188 tokens 23.1 / 19.5; Q8_0 5120 x 4096, 800 tokens (1000, 520) 63.2 / 88.7; cut: 4096 x 4096, 64 tokens (64, 32) 13.5 / 14.9, 96 tokens (96, 64)
+//     16.9 / 16.4.  Whole / cut with two tiles: 8192 x 8192, 320 tokens (w2 320; before the int8 products) 81.0 / 73.3, 448 tokens (448) 88.8 / 98.5; 5120 x 8192, 619 tokens (400) 71.9 / 87.0; long rows also where a second, partly filled round of
 //     workgroups (two fit a CU) would take as long as the first.
 //   * cut, one tile: two groups take a run's superblocks in turn where a CU has room for both and a run is long enough to halve (K-quants: K / 128 workgroups from K = 4096 on; Q8_0,
 //     whose groups fit a CU twice: always).  One group / two: 4096 x 14336, 33 tokens 25.7 / 23.7, Q8_0 35.3 / 25.9; Q6_K 8192 x 2048, 5 tokens 11.3 / 12.0.
-static int cut_line(int type, int K) { return type == T_Q8_0 ? K / 12 : K / 20; }
+static int cut_line(int type, int K) { return type == T_Q8_0 ? K / 12 : K / 25; }
 static int cut_max(int type, int NT, int K) { return NT == 2 ? (K >= 8192 ? 895 : cut_line(type, K)) : type == T_Q8_0 ? std::min(K / 8, 895) : std::max(std::min(K / 18, 400), std::min(K / 12, 256)); }
 struct WideForm { int NT, mode; bool cut; };
 // room: there is a workspace for the planes
@@ -706,7 +707,7 @@ static WideForm wide_form(int type, int cols, int T, int K, bool room) {
   const bool q8 = type == T_Q8_0, q4 = type == T_Q4_K, q5 = type == T_Q5_K, one_only = T <= 32;
   if (S >= 4 && w1 <= 256) {
     int line = q8 || q4 ? K / (12 + fill / 2) : K / (14 + fill / 10);
-    if (K <= 14336 && (one_only || ((t1 & 1) && (q8 || q4)))) line = std::min(line, 208);
+    if (K <= 14336 && (one_only || ((t1 & 1) && (q8 || q4)))) line = std::min(line, one_only && q4 ? 192 : 208);
     if (!room || w1 >= line) return {1, !q5 && (q8 || (K > 1024 && (q4 || !one_only || K >= 4096))) ? qi::W_RUNS4 : qi::W_ONE, false};
   }
   if (S >= 4 && !one_only && w1 > 256 && w2 <= 256 && !q5 && K >= (q8 ? 1024 : q4 ? 2048 : 3072) && (!room || w2 >= std::min(K / 44, 208))) return {2, qi::W_RUNS2, false};
@@ -716,7 +717,7 @@ static WideForm wide_form(int type, int cols, int T, int K, bool room) {
   if (q5 && w1 > 256 && w2 <= 256 && w2 >= std::min(K / 22, 208) && K <= 14336) cut2 = false;
   const bool pair = cut1 && (q8 ? 4 * w1 <= 512 : K >= 4096 && w1 <= std::min(K / 128, 64));
   auto time = [&](long long w, bool cut) { return cut ? Cs * ((w * ((S + Cs - 1) / Cs) + 255) / 256) : S * ((w + 255) / 256); };
-  const int ratio = cut1 ? (type == T_Q6_K ? 15 : 17) : q8 ? 18 : q5 ? 17 : 15;  // two tiles' time per superblock, in tenths of one's
+  const int ratio = q5 ? 14 : cut1 ? (type == T_Q6_K ? 15 : 17) : q8 ? 18 : 15;  // two tiles' time per superblock, in tenths of one's
   if (one_only || (q8 && pair) || time(w1, cut1) * 10 < time(w2, cut2) * ratio) return {1, pair ? qi::W_PAIR : qi::W_ONE, cut1};
   return {2, qi::W_ONE, cut2};
 }

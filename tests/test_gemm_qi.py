@@ -791,3 +791,14 @@ def test_norm_rows_gpu(oracle, dev, tname, T, k):
 @pytest.mark.parametrize("tname,T,d", [("Q4_K", 2, 1792), ("Q8_0", 3, 2304), ("Q4_K", 2, 4352)])
 def test_added_rows_of_every_length_gpu(oracle, dev, tname, T, d):
     run_added_rows(oracle, GpuBackend(dev), tname, T, d, 2048)
+
+
+# either side of the lines of the K-quants' int8 products: three rounds of workgroups with one tile, Q5_K in two tiles, cut and whole, two tiles whole above the cut's line
+LINES = [("Q4_K", (24448,), 4096, 5, False, True, (1, 1, 1)), ("Q4_K", (24576,), 4096, 5, False, True, (1, 4, 0)), ("Q5_K", (8320,), 3072, 40, True, True, (2, 1, 1)),
+         ("Q5_K", (16512,), 2048, 100, False, True, (2, 1, 0)), ("Q6_K", (13952,), 8192, 130, True, True, (2, 1, 1)), ("Q6_K", (14080,), 8192, 130, True, True, (2, 1, 0))]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("case", LINES)
+def test_gemm_qi_lines_gpu(oracle, dev, case):
+    run_form(oracle, GpuBackend(dev), *case)
