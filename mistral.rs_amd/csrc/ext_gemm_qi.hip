@@ -687,8 +687,10 @@ static int window_tiles(int type, int rows, int cols) {
 // than no groups at all.  w1, w2: workgroups of one and of two token tiles.  Times in us, Q4_K unless named:
 //   * at most a workgroup per CU, and `line` of them or more: whole, one tile, the four runs in four groups.  A cut launch has more of the chip but writes and reads four planes of the
 //     outputs, so the line falls as the tiles fill.  Cut / so: 2048 x 2048, 128 tokens (w1 64) 10.3 / 11.7, 3072 x 2048 (96) 12.8 / 12.3; 16384 x 4096, 5 tokens (128) 15.9 / 19.0,
-//     28672 x 4096 (224) 24.8 / 21.6; cut with two tiles / so: 5120 x 4096, 128 tokens (160) 21.8 / 18.4.  With one tile or an odd number of them nothing above 208 is cut (Q4_K with one tile: 192): four
-//     times that is three rounds or a little more (28672 x 8192, 5 tokens (224) 39.9 / 36.1; 24832 x 4096 (194), 5 tokens 23.4 / 18.9).  One group instead of four: Q5_K, whose kernel spills at 16 waves; Q4_K and Q6_K where a run is
+//     28672 x 4096 (224) 24.8 / 21.6; cut with two tiles / so: 5120 x 4096, 128 tokens (160) 21.8 / 18.4.  With one tile or an odd number of them nothing above 208 is cut (28672 x 8192, 5 tokens
+//     (224) 39.9 / 36.1).  Q4_K with one tile: nothing above 192, four times which is three full rounds (193 at K = 4096 .. 14336, 1 .. 32 tokens: whole 0.70 - 0.99 of cut); 192 itself is
+//     cut where a row is long or the tile nearly empty (whole / cut, 11 tokens: K = 14336 1.16, 11008 1.06, 8192 and 9216 1.0, 6144 0.96, 4096 0.90; 1 and 2 tokens 1.0 - 1.2 from
+//     K = 3072 on).  One group instead of four: Q5_K, whose kernel spills at 16 waves; Q4_K and Q6_K where a run is
 //     one superblock (Q6_K 16384 x 1024, 32 tokens 11.3 / 12.8); Q6_K with 32 tokens or less below K = 4096 (28672 x 2048, 5 tokens 18.7 / 21.3).
 //   * two tiles, at most a workgroup per CU: two groups.  Cut / so: 28672 x 8192, 64 tokens (w2 224) 59.4 / 52.5, 8192 x 8192, 256 tokens (256) 58.5 / 51.1, whole / so 54.0 / 51.1.
 //   * else one tile or two by time(), the superblocks in a row on the busiest CU, of which two tiles take 1.4 (Q5_K) - 1.8 times as long.  One / two: 12288 x 4096, 160 tokens (w1 480, w2 288)
@@ -707,7 +709,7 @@ static WideForm wide_form(int type, int cols, int T, int K, bool room) {
   const bool q8 = type == T_Q8_0, q4 = type == T_Q4_K, q5 = type == T_Q5_K, one_only = T <= 32;
   if (S >= 4 && w1 <= 256) {
     int line = q8 || q4 ? K / (12 + fill / 2) : K / (14 + fill / 10);
-    if (K <= 14336 && (one_only || ((t1 & 1) && (q8 || q4)))) line = std::min(line, one_only && q4 ? 192 : 208);
+    if (K <= 14336 && (one_only || ((t1 & 1) && (q8 || q4)))) line = std::min(line, !one_only || !q4 ? 208 : K >= 7168 || T <= 2 ? 193 : 192);
     if (!room || w1 >= line) return {1, !q5 && (q8 || (K > 1024 && (q4 || !one_only || K >= 4096))) ? qi::W_RUNS4 : qi::W_ONE, false};
   }
   if (S >= 4 && !one_only && w1 > 256 && w2 <= 256 && !q5 && K >= (q8 ? 1024 : q4 ? 2048 : 3072) && (!room || w2 >= std::min(K / 44, 208))) return {2, qi::W_RUNS2, false};

@@ -802,3 +802,15 @@ LINES = [("Q4_K", (24448,), 4096, 5, False, True, (1, 1, 1)), ("Q4_K", (24576,),
 @pytest.mark.parametrize("case", LINES)
 def test_gemm_qi_lines_gpu(oracle, dev, case):
     run_form(oracle, GpuBackend(dev), *case)
+
+
+# the form on either side of a line, at sizes that the host emulation would multiply for minutes.  192 workgroups of Q4_K are three full rounds cut: whole one workgroup above it, at 192 itself
+# where a row is shorter than 7168 values and the tile has more than two rows
+FORM_LINES = [("Q4_K", 24576, 14336, 11, (1, 1, 1)), ("Q4_K", 24704, 14336, 11, (1, 4, 0)), ("Q4_K", 24576, 7168, 32, (1, 1, 1)), ("Q4_K", 24576, 6912, 32, (1, 4, 0)),
+              ("Q4_K", 24576, 4096, 2, (1, 1, 1)), ("Q4_K", 24576, 4096, 3, (1, 4, 0)), ("Q4_K", 24704, 4096, 1, (1, 4, 0))]
+
+
+@pytest.mark.parametrize("tname,n,k,T,want", FORM_LINES)
+def test_gemm_qi_form_lines(oracle, tname, n, k, T, want):
+    f = HostBackend().sym("mrs_gemm_qi_form", [CI, CI, VP, CI, CI, CI], CI)(getattr(oracle, tname), 1, (CI * 1)(n), k, T, 1)
+    assert (f & 15, f >> 4 & 15, f >> 8) == want
