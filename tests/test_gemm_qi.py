@@ -807,7 +807,10 @@ def test_gemm_qi_lines_gpu(oracle, dev, case):
 # the form on either side of a line, at sizes that the host emulation would multiply for minutes.  192 workgroups of Q4_K are three full rounds cut: whole one workgroup above it, at 192 itself
 # where a row is shorter than 7168 values and the tile has more than two rows
 FORM_LINES = [("Q4_K", 24576, 14336, 11, (1, 1, 1)), ("Q4_K", 24704, 14336, 11, (1, 4, 0)), ("Q4_K", 24576, 7168, 32, (1, 1, 1)), ("Q4_K", 24576, 6912, 32, (1, 4, 0)),
-              ("Q4_K", 24576, 4096, 2, (1, 1, 1)), ("Q4_K", 24576, 4096, 3, (1, 4, 0)), ("Q4_K", 24704, 4096, 1, (1, 4, 0))]
+              ("Q4_K", 24576, 4096, 2, (1, 1, 1)), ("Q4_K", 24576, 4096, 3, (1, 4, 0)), ("Q4_K", 24704, 4096, 1, (1, 4, 0)),
+              # two token tiles of Q5_K and Q6_K: cut up to K / 20 workgroups where these are few, up to K / 25 else
+              ("Q6_K", 9600, 6144, 200, (2, 1, 1)), ("Q6_K", 9856, 6144, 200, (2, 1, 0)), ("Q5_K", 4608, 7168, 500, (2, 1, 1)), ("Q6_K", 12160, 9216, 220, (2, 1, 1)),
+              ("Q6_K", 12416, 9216, 220, (2, 1, 0)), ("Q6_K", 13952, 11008, 200, (2, 1, 1)), ("Q6_K", 14208, 11008, 200, (2, 1, 0)), ("Q4_K", 9600, 6144, 200, (2, 1, 0))]
 
 
 @pytest.mark.parametrize("tname,n,k,T,want", FORM_LINES)
