@@ -694,7 +694,8 @@ static int window_tiles(int type, int rows, int cols) {
 //     one superblock (Q6_K 16384 x 1024, 32 tokens 11.3 / 12.8); Q6_K with 32 tokens or less below K = 4096 (28672 x 2048, 5 tokens 18.7 / 21.3).
 //   * two tiles, at most a workgroup per CU: two groups.  Cut / so: 28672 x 8192, 64 tokens (w2 224) 59.4 / 52.5, 8192 x 8192, 256 tokens (256) 58.5 / 51.1, whole / so 54.0 / 51.1.
 //   * else one tile or two by time(), the superblocks in a row on the busiest CU, of which two tiles take 1.4 (Q5_K) - 1.8 times as long.  One / two: 12288 x 4096, 160 tokens (w1 480, w2 288)
-//     33.0 / 42.2, 28672 x 4096, 512 tokens 198 / 164; Q5_K 7808 x 4096, 1047 tokens 140 / 124, cut 3200 x 4096, 188 tokens 23.1 / 19.5, but 15360 x 13824, 73 tokens cut / whole 89.7 / 112, cut 20352 x 9216, 64
+//     33.0 / 42.2, 28672 x 4096, 512 tokens 198 / 164; where both would take as long, 65 .. 96 tokens one (0.94 of two on average of 126 sizes, 29696 x 11008, 79 tokens 0.93; 97 .. 128 tokens
+//     and from 193 on two are as fast or up to 8 % faster); Q5_K 7808 x 4096, 1047 tokens 140 / 124, cut 3200 x 4096, 188 tokens 23.1 / 19.5, but 15360 x 13824, 73 tokens cut / whole 89.7 / 112, cut 20352 x 9216, 64
 //     tokens (318, 159) two tiles 1.17 times one, 6016 x 2560, 90 tokens 1.15; Q8_0 5120 x 4096, 800 tokens (1000, 520) 63.2 / 88.7; cut: 4096 x 4096, 64 tokens (64, 32) 13.5 / 14.9, 96 tokens (96, 64)
 //     16.9 / 16.4.  Whole / cut with two tiles: 8192 x 8192, 320 tokens (w2 320; before the int8 products) 81.0 / 73.3, 448 tokens (448) 88.8 / 98.5; 5120 x 8192, 619 tokens (400) 71.9 / 87.0; long rows also where a second, partly filled round of
 //     workgroups (two fit a CU) would take as long as the first.  Q5_K and Q6_K, whose two tiles take longer, are cut up to K / 20 where that is at most some 330 - 380 workgroups (whole /
@@ -728,7 +729,8 @@ static WideForm wide_form(int type, int cols, int T, int K, bool room) {
   // workgroup anyway and two tiles are a little more than the 512 that are resident when cut
   const bool q5_one = (cut1 && !cut2) || (t1 == 3 && (cut1 || cut2)) || (t1 == 2 && cut1 && w2 > 128);
   const int ratio = q5 ? (q5_one ? 17 : 14) : cut1 ? (type == T_Q6_K ? 15 : 17) : q8 ? 18 : 15;
-  if (one_only || (q8 && pair) || time(w1, cut1) * 10 < time(w2, cut2) * ratio) return {1, pair ? qi::W_PAIR : qi::W_ONE, cut1};
+  const bool tie = q4 && t1 == 3 && K > 1024;  // 65 .. 96 tokens: the second of two tiles is half empty
+  if (one_only || (q8 && pair) || time(w1, cut1) * 10 < time(w2, cut2) * ratio + (tie ? 1 : 0)) return {1, pair ? qi::W_PAIR : qi::W_ONE, cut1};
   return {2, qi::W_ONE, cut2};
 }
 // workspace that holds the run sums of every launch over at most n rows of weights [K] and T tokens that is cut: four planes of its outputs, of which a workgroup writes at most
