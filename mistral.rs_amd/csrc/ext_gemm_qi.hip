@@ -725,9 +725,10 @@ static WideForm wide_form(int type, int cols, int T, int K, bool room) {
   if (q5 && w1 > 256 && w2 <= 256 && w2 >= std::min(K / 22, 208) && K <= 14336) cut2 = false;
   const bool pair = cut1 && (q8 ? 4 * w1 <= 512 : K >= 4096 && w1 <= std::min(K / 128, 64));
   auto time = [&](long long w, bool cut) { return cut ? Cs * ((w * ((S + Cs - 1) / Cs) + 255) / 256) : S * ((w + 255) / 256); };
-  // two tiles' time per superblock, in tenths of one's.  Q5_K 17: where one tile is cut and two are not, where the last of few tiles is half empty, and where each weight is read by one
-  // workgroup anyway and two tiles are a little more than the 512 that are resident when cut
-  const bool q5_one = (cut1 && !cut2) || (t1 == 3 && (cut1 || cut2)) || (t1 == 2 && cut1 && w2 > 128);
+  // two tiles' time per superblock, in tenths of one's.  Q5_K 17: where one tile is cut and two are not, where the last of few tiles is half empty (short rows or many workgroups: else
+  // both are as fast, and beside Q6_K in one launch two are 12 - 18 % faster), and where each weight is read by one workgroup anyway and two tiles are a little more than the 512 that are
+  // resident when cut
+  const bool q5_one = (cut1 && !cut2) || (t1 == 3 && (cut1 || cut2) && (K < 4096 || w2 > 128)) || (t1 == 2 && cut1 && w2 > 128);
   const int ratio = q5 ? (q5_one ? 17 : 14) : cut1 ? (type == T_Q6_K ? 15 : 17) : q8 ? 18 : 15;
   const bool tie = q4 && t1 == 3 && K > 1024;  // 65 .. 96 tokens: the second of two tiles is half empty
   if (one_only || (q8 && pair) || time(w1, cut1) * 10 < time(w2, cut2) * ratio + (tie ? 1 : 0)) return {1, pair ? qi::W_PAIR : qi::W_ONE, cut1};
