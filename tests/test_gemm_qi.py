@@ -734,12 +734,44 @@ def test_gemm_qi_mixed_host_emulation(oracle, tname, ns, k, T, ws):
     run_mixed(oracle, HostBackend(), tname, ns, k, T, ws, keep=True, seed=T + 1)
 
 
+MIXED_GPU = MIXED + [("Q4_K", [1024, 4096, 1024], 4096, T, 1) for T in (4, 37, 64, 130, 300, 700)] + [("Q4_K", [1024, 12288], 4096, 33, 0), ("Q5_K", [1024, 4096], 4096, 200, 1),
+                                                                                                         ("Q4_K", [1024, 27648], 4096, 5, 0)]
+
+
 @pytest.mark.gpu
-@pytest.mark.parametrize("tname,ns,k,T,ws", MIXED + [("Q4_K", [1024, 4096, 1024], 4096, T, 1) for T in (4, 37, 64, 130, 300, 700)] + [("Q4_K", [1024, 12288], 4096, 33, 0),
-                                                    ("Q5_K", [1024, 4096], 4096, 200, 1), ("Q4_K", [1024, 27648], 4096, 5, 0)])
+@pytest.mark.parametrize("tname,ns,k,T,ws", MIXED_GPU)
 def test_gemm_qi_mixed_gpu(oracle, dev, tname, ns, k, T, ws):
     run_mixed(oracle, GpuBackend(dev), tname, ns, k, T, ws, seed=T)
     run_mixed(oracle, GpuBackend(dev), tname, ns, k, T, ws, keep=True, seed=T + 1)
+
+
+# two groups of waves that take a run's superblocks in turn: 17 superblocks = runs of 5, 5, 5 and 2, whose last step has no second term; one tile with a remainder and two; both orders of three
+MIXED_PAIR = [("Q4_K", [36, 132], 4352, 3, 1), ("Q4_K", [64, 40, 132], 4352, 33, 1), ("Q5_K", [132, 64], 4352, 33, 1), ("Q5_K", [40, 64, 32], 4352, 3, 1)]
+MIXED_PAIR_GPU = MIXED_PAIR + [("Q4_K", [512, 2048, 512], 4096, 5, 1), ("Q5_K", [512, 2048, 512], 4096, 5, 1)]
+
+
+@pytest.mark.parametrize("tname,ns,k,T,ws", MIXED_PAIR)
+def test_gemm_qi_mixed_pair_host_emulation(oracle, tname, ns, k, T, ws):
+    run_mixed(oracle, HostBackend(), tname, ns, k, T, ws, seed=T)
+    run_mixed(oracle, HostBackend(), tname, ns, k, T, ws, keep=True, seed=T + 1)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("tname,ns,k,T,ws", MIXED_PAIR_GPU)
+def test_gemm_qi_mixed_pair_gpu(oracle, dev, tname, ns, k, T, ws):
+    run_mixed(oracle, GpuBackend(dev), tname, ns, k, T, ws, seed=T)
+    run_mixed(oracle, GpuBackend(dev), tname, ns, k, T, ws, keep=True, seed=T + 1)
+
+
+def test_gemm_qi_mixed_forms(oracle):
+    """Every form that a launch of two types can take is run above: a line that moves shows here where a case has lost its form."""
+    form = HostBackend().sym("mrs_gemm_qi_form", [CI, CI, VP, CI, CI, CI], CI)
+    want = [(1, 1, 0), (1, 1, 1), (1, 1, 1), (1, 1, 0), (1, 1, 1), (1, 1, 1), (2, 1, 1), (2, 1, 1), (1, 4, 0), (2, 2, 0), (2, 1, 0), (1, 4, 0), (2, 1, 1), (1, 4, 0)] + 6 * [(1, 2, 1)]
+    got = []
+    for tname, ns, k, T, ws in MIXED_GPU + MIXED_PAIR_GPU:
+        f = form(getattr(oracle, tname), len(ns), (CI * len(ns))(*ns), k, T, ws)
+        got.append((f & 15, f >> 4 & 15, f >> 8))
+    assert got == want
 
 
 # windows that end with 1, 32, 33 and 64 rows in their last workgroup of 64, an empty one, and enough workgroups (2048) for the kernel that takes a short end in one token tile
