@@ -151,3 +151,20 @@ def test_gpu_suite_slice_on_host_emulation(path, expr):
     tail = "\n".join(r.stdout.splitlines()[-15:])
     assert r.returncode == 0, tail
     assert " passed" in tail and "failed" not in tail, tail
+
+
+def test_partial_rebuild_copies_every_header_its_units_include():
+    """scripts/rebuild_hiphost_dec.sh compiles copies of the sources: a header that it does not refresh would be the one of the last full build."""
+    import glob
+    import re
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    csrc = os.path.join(root, "mistral.rs_amd", "csrc")
+    script = open(os.path.join(root, "scripts", "rebuild_hiphost_dec.sh")).read()
+    copied = {os.path.basename(p) for pat in re.findall(r'"\$CSRC"/(\S+?);?(?=\s)', script.split("for f in", 1)[1].split("do\n", 1)[0]) for p in glob.glob(os.path.join(csrc, pat))}
+    todo, seen = ["ext_dec.hip", "ext_dec_gemv.hip", "ext_gemm_qi.hip"], set()
+    while todo:
+        f = todo.pop()
+        if f not in seen and os.path.exists(os.path.join(csrc, f)):
+            seen.add(f)
+            todo += re.findall(r'#include "([\w.]+)"', open(os.path.join(csrc, f)).read())
+    assert "qi_wide_body.cuh" in seen and seen <= copied, seen - copied
