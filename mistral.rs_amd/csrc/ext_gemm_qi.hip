@@ -16,7 +16,8 @@
 // Operands: weights in an MFMA-order copy made at load time (mrs_gemm_qi_repack: per 32-row panel and superblock, every lane's 16 bytes of a piece
 // contiguous: one buffer_load_dwordx4 per lane and piece, straight into registers); activations from mrs_qi_quantize (engine-order RmsNorm + the candle
 // Q8_K quantizer of dec_core2.cuh, int8 in the operand's k order, slab-major [superblock][token][256]).
-// One kernel, gemm_qi_wide_kernel<type, token tiles of a wave>, multiplies all four types at all prompt lengths.
+// One body (qi_wide_body.cuh) multiplies all four types at all prompt lengths: gemm_qi_wide_kernel<type, token tiles of a wave, groups of waves>, gemm_qi_mixed_kernel (two K-quants on
+// the same rows in one launch) and gemm_qi_tail_kernel (experts' windows whose last workgroup is short).
 #include "dec_core2.cuh"
 #include <stdio.h>
 #include <stdlib.h>
@@ -317,8 +318,8 @@ __device__ __forceinline__ h8 mk_h8(h2 a, h2 b, h2 c, h2 d) { h8 r; r[0] = a[0];
 // ------------------------------------------------------------------------------------------------ the kernel
 // What bounds this product is the vector ALU beside the matrix cores: a superblock of 32 weight rows costs ~134 (Q4_K) .. 290 (Q6_K) vector instructions of operand build, the f32
 // term 5 (Q6_K: 4) per output and superblock, a 32 x 32 tile 16 matrix instructions of 32 cycles (and 3 for the products below).  The times of two waves of a SIMD hardly overlap:
-// 28672 x 4096 x 2000 tokens of Q4_K takes 2400 cycles per wave and superblock (two tiles) at 2.05 GHz, 1220 of them matrix, 1580 vector issue (rocprofv3); without the term's
-// vector instructions it is 8 % faster, without the build not at all.  Operands in f16 (one digit of up to 504, K = 16 per matrix instruction, S = sum_j sc_j bsum_j beside M) cost 92 vector
+// 28672 x 4096 x 1999 tokens of Q4_K issues vector instructions 70 % of its time and matrix instructions 54 %, 4096 x 14336 of Q6_K 74 and 45 (rocprofv3); without the term's
+// vector instructions the first is 8 % faster, without the build not at all.  Operands in f16 (one digit of up to 504, K = 16 per matrix instruction, S = sum_j sc_j bsum_j beside M) cost 92 vector
 // instructions more per superblock of two tiles and twice the LDS reads, Q6_K's two f16 digits twice the matrix time:  us, f16 / int8 digits: Q4_K 28672 x 4096, 512 tokens 167 / 144,
 // 1999 640 / 545, 4096 x 14336, 1999 313 / 265; Q6_K 4096 x 14336, 512 tokens 117 / 85, 1999 438 / 305; Q5_K 28672 x 4096, 512 tokens 201 / 167.  So:
 //   * Q4_K: one multiplication of packed half-words multiplies two nibbles by a digit of the scale; Q5_K / Q6_K form sc (q - 32) + 128 in packed half-words and take them apart into
@@ -408,7 +409,11 @@ __global__ void __launch_bounds__(256 * wide_groups(MODE), (wide_waves<TYPE, NT,
 // 1024 rows of its own is a few workgroups that fill no chip, 8.5 us at 37 tokens and 12.6 at 512.  The larger type comes first: its columns take longer.
 // q / k / v of 4096 + 1024 + 1024 x 4096, Q4_K, Q4_K, Q6_K, us, two launches / one: 4 tokens 15.9 / 9.5, 37
 // 17.8 / 10.4, 512 49.3 / 38.7, 1000 84.8 / 64.9, 1999 134.8 / 131.2; 8192 + 1024 + 1024 x 8192 29.3 / 17.8, 34.9 / 25.5, 118 / 112, 217 / 200, 394 / 395; Q5_K beside Q6_K 18.4 / 10.4,
-// 19.3 / 11.3, 60.4 / 55.6, 103 / 78, 151 / 141.
+// 19.3 / 11.3, 60.4 / 55.6, 103 / 78, 151 / 141.  With the rotation behind them, hidden sizes 1024 .. 8192, 1 .. 1999 tokens, the one launch takes 0.79 of two on average of 480 sizes (to 64
+// tokens 0.69; 0.81 and 0.86 with two of three tensors, or one of two, of Q6_K) and never more than two launches of the f16 products did; it is behind two of the present ones at 3 % of
+// the sizes, where its workgroups are just over a round of 512 (4096 + 1024 + 1024 x 4096, 768 tokens 77.2 / 69.4; 5120 + 1024 + 1024 x 5120, 640 tokens 92.6 / 79.4).  The form with four
+// groups (Q4_K, 97 .. 160 tokens of hidden size 4096) spills 6 registers: 97 tokens 24.0, two launches 28.0, two tiles cut in one launch 22.1; 160 tokens 25.4, 31.9, 29.6; at hidden
+// size 2048, 97 tokens 15.5, 17.9, 12.3.
 template <int TA, int TB, int NT, int MODE>
 __global__ void __launch_bounds__(256 * wide_groups(MODE), (wide_waves<TA, NT, MODE> < wide_waves<TB, NT, MODE> ? wide_waves<TA, NT, MODE> : wide_waves<TB, NT, MODE>)) gemm_qi_mixed_kernel(const WideArgs a) {
   extern __shared__ __attribute__((aligned(16))) char smem_all[];
@@ -654,7 +659,8 @@ template <int TB> static void mixed_launch(int NT, int mode, const qi::WideArgs 
   NT == 2 ? mixed_go<T_Q6_K, TB, 2, qi::W_ONE>(a, grid, s) : mixed_go<T_Q6_K, TB, 1, qi::W_ONE>(a, grid, s);
 }
 // gemm_qi_tail_kernel from this many workgroups on.  Fewer are a few rounds of the 512 that are resident, whose last is as long either way, and a launch of uneven workgroups meets it
-// later (down of 4096 x 14336, us, without / with: Q4_K 512 tokens 201 / 216, 600 228 / 244, 1200 (1440 workgroups) 358 / 360; Q6_K 200 122 / 130).  Rows without windows (one last tile of
+// later.  With / without over gate and up and down of eight expert shapes (8 .. 128 experts of 768 .. 16384 x 1024 .. 6144, top-2 .. 8, 100 .. 1999 tokens, all three types): to 1024
+// workgroups 1.03 on average, to 2048 1.01, above 0.997 (0.90 .. 1.05, by how full the last tiles are) (down of 4096 x 14336, us, without / with: Q4_K 512 tokens 201 / 216, 600 228 / 244, 1200 (1440 workgroups) 358 / 360; Q6_K 200 122 / 130).  Rows without windows (one last tile of
 // many) gain and lose under 1 %: 28672 x 4096, 650 tokens 194 / 193, 1999 541 / 549.
 constexpr unsigned TAIL_MIN = 2048;
 template <int TYPE> static void wide_launch(int NT, int mode, const qi::WideArgs &a, dim3 grid, hipStream_t s) {
@@ -683,7 +689,8 @@ static int window_tiles(int type, int rows, int cols) {
 // Every other launch: token tiles per wave (NT), groups of waves per workgroup (mode), cut by runs of superblocks (cut) or whole.  The lines are drawn through the times of all seven forms
 // at 9900 sizes (512 .. 32768 rows of weights, K = 1024 .. 28672, 1 .. 2000 tokens, weights from HBM), and those of the K-quants again at 9100 sizes (1000 .. 32000 rows, K = 1024 ..
 // 14336) since their products multiply in int8: against the fastest form of each size the one taken costs 1.3 % on average (Q4_K; K = 1024, cut where whole is 15 % faster, 3.8), 0.5 %
-// (Q5_K; 1.2 before), 0.8 % (Q6_K), Q8_0 0.1 - 1.0 %; lines drawn through some 40 sizes whose weights lay in the last-level cache cost 1 - 8 % and were up to 1.25 times slower
+// (Q5_K; 1.2 before), 0.8 % (Q6_K), Q8_0 0.1 - 1.0 %.  Where that had taken another form than before, the lines were then moved again by both forms' times at 3972 sizes (by more than 3 %
+// slower than the older form 360 -> 54); lines drawn through some 40 sizes whose weights lay in the last-level cache cost 1 - 8 % and were up to 1.25 times slower
 // than no groups at all.  w1, w2: workgroups of one and of two token tiles.  Times in us, Q4_K unless named:
 //   * at most a workgroup per CU, and `line` of them or more: whole, one tile, the four runs in four groups.  A cut launch has more of the chip but writes and reads four planes of the
 //     outputs, so the line falls as the tiles fill.  Cut / so: 2048 x 2048, 128 tokens (w1 64) 10.3 / 11.7, 3072 x 2048 (96) 12.8 / 12.3; 16384 x 4096, 5 tokens (128) 15.9 / 19.0,

@@ -1,7 +1,7 @@
 """Prompt GEMM in the reference CPU path's arithmetic on the matrix cores (csrc/ext_gemm_qi.hip): Q8_K activation rows (engine-order RmsNorm + candle's
-quantizer) x Q4_K / Q5_K / Q6_K weights through v_mfma_f32_32x32x16_f16 on exact small integers, combined in the decode engine's f32 order (ORD-U).
+quantizer) x Q4_K / Q5_K / Q6_K weights through v_mfma_i32_32x32x32_i8 on exact integers (scale x quant as two int8 digits), combined in the decode engine's f32 order (ORD-U).
 Every output row equals the decode engine's GEMV of that token (oracle/cpu_path_oracle.c orc_gemv_engine) BIT FOR BIT -- so does the GPU result against the
-batch-1 decode kernel itself.  Also: the matrix core's f32 accumulator is exact on the integer operands the kernel feeds it (adversarial magnitudes)."""
+batch-1 decode kernel itself.  Also: v_mfma_f32_32x32x16_f16, which sums the mins (run sums x mins), is exact on integers below 2^24 (adversarial magnitudes)."""
 import ctypes as C
 
 import numpy as np
@@ -162,7 +162,8 @@ def test_gemm_qi_glu_and_accumulate_gpu(oracle, dev):
 
 @pytest.mark.gpu
 def test_mfma_f16_accumulates_small_integers_exactly(dev):
-    """The premise of the kernel: every partial sum of a superblock is an integer below 2^24, and v_mfma_f32_32x32x16_f16 keeps it exact."""
+    """The premise of the min terms, sum of mins (<= 63) x run sums (<= 2048) in one instruction: v_mfma_f32_32x32x16_f16 keeps integers below 2^24 exact.  The other magnitudes go
+    further than any operand of the products (whose scale x quant are int8 digits), through chains of 16 instructions."""
     import torch
     from mistralrs_amd import _lib
     L = _lib.load("ext")
@@ -191,7 +192,7 @@ def test_mfma_f16_accumulates_small_integers_exactly(dev):
             A = rng.integers(-amax, amax + 1, (ks, 32, 16)); B = rng.integers(-128, 128, (ks, 32, 16)) if amax != 2048 else rng.integers(0, 64, (ks, 32, 16))
             got, ref = run(A, B)
             assert np.array_equal(got, ref)
-    got, ref = run(np.full((16, 32, 16), 504), np.full((16, 32, 16), -128))  # |sum| = 16.5 M, the largest a Q4_K superblock can reach
+    got, ref = run(np.full((16, 32, 16), 504), np.full((16, 32, 16), -128))  # |sum| = 16.5 M, just below 2^24
     assert np.array_equal(got, ref) and ref[0, 0] == -16515072
 
 
