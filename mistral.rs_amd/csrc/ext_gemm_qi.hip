@@ -705,14 +705,12 @@ static int window_tiles(int type, int rows, int cols) {
 //     and from 193 on two are as fast or up to 8 % faster); Q5_K 7808 x 4096, 1047 tokens 140 / 124, cut 3200 x 4096, 188 tokens 23.1 / 19.5, but 15360 x 13824, 73 tokens cut / whole 89.7 / 112, cut 20352 x 9216, 64
 //     tokens (318, 159) two tiles 1.17 times one, 6016 x 2560, 90 tokens 1.15; Q8_0 5120 x 4096, 800 tokens (1000, 520) 63.2 / 88.7; cut: 4096 x 4096, 64 tokens (64, 32) 13.5 / 14.9, 96 tokens (96, 64)
 //     16.9 / 16.4.  Whole / cut with two tiles: 8192 x 8192, 320 tokens (w2 320; before the int8 products) 81.0 / 73.3, 448 tokens (448) 88.8 / 98.5; 5120 x 8192, 619 tokens (400) 71.9 / 87.0; long rows also where a second, partly filled round of
-//     workgroups (two fit a CU) would take as long as the first.  Q5_K and Q6_K, whose two tiles take longer, are cut up to K / 20 where that is at most some 330 - 380 workgroups (whole /
-//     cut, on average, w2 260 .. 320: K = 6144 Q6_K 1.04, 7168 1.03 - 1.06, Q5_K 1.03 - 1.09; above 384: 0.87 - 0.95).
+//     workgroups (two fit a CU) would take as long as the first.  Q5_K and Q6_K, whose two tiles take longer, are cut up to K / 20 where that is at most some 330 - 380 workgroups, if two tiles
+//     are taken at all (whole / cut, on average, w2 260 .. 320: K = 6144 Q6_K 1.04, 7168 1.03 - 1.06, Q5_K 1.03 - 1.09; above 384: 0.87 - 0.95; one tile whole where that beats two tiles
+//     whole: Q6_K 19584 x 6144, 81 tokens 54.0, two cut 61.9).
 //   * cut, one tile: two groups take a run's superblocks in turn where a CU has room for both and a run is long enough to halve (K-quants: K / 128 workgroups from K = 4096 on; Q8_0,
 //     whose groups fit a CU twice: always).  One group / two: 4096 x 14336, 33 tokens 25.7 / 23.7, Q8_0 35.3 / 25.9; Q6_K 8192 x 2048, 5 tokens 11.3 / 12.0.
-static int cut_line(int type, int K) {
-  if (type == T_Q8_0) return K / 12;
-  return type == T_Q4_K || K < 3584 ? K / 25 : std::max(K / 25, std::min(K / 20, K > 8192 ? 384 : 328));
-}
+static int cut_line(int type, int K) { return type == T_Q8_0 ? K / 12 : K / 25; }
 static int cut_max(int type, int NT, int K) { return NT == 2 ? (K >= 8192 ? 895 : cut_line(type, K)) : type == T_Q8_0 ? std::min(K / 8, 895) : std::max(std::min(K / 18, 400), std::min(K / 12, 256)); }
 struct WideForm { int NT, mode; bool cut; };
 // room: there is a workspace for the planes
@@ -739,7 +737,8 @@ static WideForm wide_form(int type, int cols, int T, int K, bool room) {
   const int ratio = q5 ? (q5_one ? 17 : 14) : cut1 ? (type == T_Q6_K ? 15 : 17) : q8 ? 18 : 15;
   const bool tie = q4 && t1 == 3 && K > 1024;  // 65 .. 96 tokens: the second of two tiles is half empty
   if (one_only || (q8 && pair) || time(w1, cut1) * 10 < time(w2, cut2) * ratio + (tie ? 1 : 0)) return {1, pair ? qi::W_PAIR : qi::W_ONE, cut1};
-  return {2, qi::W_ONE, cut2};
+  const bool cut2_few = can && !q8 && !q4 && w2 > 256 && w2 <= std::min(K / 20, K > 8192 ? 384 : 328);
+  return {2, qi::W_ONE, cut2 || cut2_few};
 }
 // workspace that holds the run sums of every launch over at most n rows of weights [K] and T tokens that is cut: four planes of its outputs, of which a workgroup writes at most
 // 32 NT x 128.  Never falls as T or n grow

@@ -844,6 +844,8 @@ FORM_LINES = [("Q4_K", 24576, 14336, 11, (1, 1, 1)), ("Q4_K", 24704, 14336, 11, 
               # two token tiles of Q5_K and Q6_K: cut up to K / 20 workgroups where these are few, up to K / 25 else
               ("Q6_K", 9600, 6144, 200, (2, 1, 1)), ("Q6_K", 9856, 6144, 200, (2, 1, 0)), ("Q5_K", 4608, 7168, 500, (2, 1, 1)), ("Q6_K", 12160, 9216, 220, (2, 1, 1)),
               ("Q6_K", 12416, 9216, 220, (2, 1, 0)), ("Q6_K", 13952, 11008, 200, (2, 1, 1)), ("Q6_K", 14208, 11008, 200, (2, 1, 0)), ("Q4_K", 9600, 6144, 200, (2, 1, 0)),
+              # .. which does not bring two tiles where one is taken else, nor is it drawn for rows of up to 5120 values
+              ("Q6_K", 19584, 6144, 81, (1, 1, 0)), ("Q5_K", 6784, 5632, 257, (1, 1, 0)), ("Q5_K", 21120, 4096, 47, (2, 1, 0)),
               # Q5_K in one tile: cut beside two that are not, 65 .. 96 tokens, few more than 128 workgroups of two; in two tiles on the other side
               ("Q5_K", 15360, 13824, 73, (1, 1, 1)), ("Q5_K", 9344, 11008, 132, (1, 1, 1)), ("Q5_K", 6016, 2560, 96, (1, 1, 1)), ("Q5_K", 6016, 2560, 64, (2, 1, 1)),
               ("Q5_K", 6144, 4096, 80, (2, 1, 1)),
