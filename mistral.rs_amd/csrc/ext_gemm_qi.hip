@@ -702,8 +702,8 @@ static int window_tiles(int type, int rows, int cols) {
 //   * two tiles, at most a workgroup per CU: two groups.  Cut / so: 28672 x 8192, 64 tokens (w2 224) 59.4 / 52.5, 8192 x 8192, 256 tokens (256) 58.5 / 51.1, whole / so 54.0 / 51.1.
 //   * else one tile or two by time(), the superblocks in a row on the busiest CU, of which two tiles take 1.4 (Q5_K) - 1.8 times as long.  One / two: 12288 x 4096, 160 tokens (w1 480, w2 288)
 //     33.0 / 42.2, 28672 x 4096, 512 tokens 198 / 164; where both would take as long, 65 .. 96 tokens one (0.94 of two on average of 126 sizes, 29696 x 11008, 79 tokens 0.93; 97 .. 128 tokens
-//     and from 193 on two are as fast or up to 8 % faster); Q5_K 7808 x 4096, 1047 tokens 140 / 124, cut 3200 x 4096, 188 tokens 23.1 / 19.5, but 15360 x 13824, 73 tokens cut / whole 89.7 / 112, cut 20352 x 9216, 64
-//     tokens (318, 159) two tiles 1.17 times one, 6016 x 2560, 90 tokens 1.15; Q8_0 5120 x 4096, 800 tokens (1000, 520) 63.2 / 88.7; cut: 4096 x 4096, 64 tokens (64, 32) 13.5 / 14.9, 96 tokens (96, 64)
+//     and from 193 on two are as fast or up to 8 % faster); Q5_K 7808 x 4096, 1047 tokens 140 / 124, cut 3200 x 4096, 188 tokens 23.1 / 19.5, but 15360 x 13824, 73 tokens cut / whole 89.7 / 112, 6016 x 2560,
+//     90 tokens two tiles 1.15 times one; Q8_0 5120 x 4096, 800 tokens (1000, 520) 63.2 / 88.7; cut: 4096 x 4096, 64 tokens (64, 32) 13.5 / 14.9, 96 tokens (96, 64)
 //     16.9 / 16.4.  Whole / cut with two tiles: 8192 x 8192, 320 tokens (w2 320; before the int8 products) 81.0 / 73.3, 448 tokens (448) 88.8 / 98.5; 5120 x 8192, 619 tokens (400) 71.9 / 87.0; long rows also where a second, partly filled round of
 //     workgroups (two fit a CU) would take as long as the first.  Q5_K and Q6_K, whose two tiles take longer, are cut up to K / 20 where that is at most some 330 - 380 workgroups, if two tiles
 //     are taken at all (whole / cut, on average, w2 260 .. 320: K = 6144 Q6_K 1.04, 7168 1.03 - 1.06, Q5_K 1.03 - 1.09; above 384: 0.87 - 0.95; one tile whole where that beats two tiles
@@ -730,10 +730,10 @@ static WideForm wide_form(int type, int cols, int T, int K, bool room) {
   if (q5 && w1 > 256 && w2 <= 256 && w2 >= std::min(K / 22, 208) && K <= 14336) cut2 = false;
   const bool pair = cut1 && (q8 ? 4 * w1 <= 512 : K >= 4096 && w1 <= std::min(K / 128, 64));
   auto time = [&](long long w, bool cut) { return cut ? Cs * ((w * ((S + Cs - 1) / Cs) + 255) / 256) : S * ((w + 255) / 256); };
-  // two tiles' time per superblock, in tenths of one's.  Q5_K 17: where one tile is cut and two are not, where the last of few tiles is half empty (short rows or many workgroups: else
-  // both are as fast, and beside Q6_K in one launch two are 12 - 18 % faster), and where each weight is read by one workgroup anyway and two tiles are a little more than the 512 that are
-  // resident when cut
-  const bool q5_one = (cut1 && !cut2) || (t1 == 3 && (cut1 || cut2) && (K < 4096 || w2 > 128)) || (t1 == 2 && cut1 && w2 > 128);
+  // two tiles' time per superblock, in tenths of one's.  Q5_K 14, but 17 where two tiles are slower (times of one as a share of two's, 1600 sizes): where only one tile is cut (0.91); with
+  // 65 .. 96 tokens, whose last tile is half empty, both cut, where a row is short (0.90 - 1.01) or two make more than two rounds of the 512 resident (0.93), and one whole, two cut, up to
+  // 10240 values (0.92 - 0.96) or from 448 workgroups on (0.95); with 33 .. 64 tokens, both cut, of long rows where two make a little more than one round (0.97).  Elsewhere 1.0 - 1.2
+  const bool q5_one = (cut1 && !cut2) || (t1 == 3 && cut2 && (cut1 ? K < 4096 || w2 > 256 : K < 10240 || w2 > 448)) || (t1 == 2 && cut1 && w2 > 128 && K >= 12288);
   const int ratio = q5 ? (q5_one ? 17 : 14) : cut1 ? (type == T_Q6_K ? 15 : 17) : q8 ? 18 : 15;
   const bool tie = q4 && t1 == 3 && K > 1024;  // 65 .. 96 tokens: the second of two tiles is half empty
   if (one_only || (q8 && pair) || time(w1, cut1) * 10 < time(w2, cut2) * ratio + (tie ? 1 : 0)) return {1, pair ? qi::W_PAIR : qi::W_ONE, cut1};
