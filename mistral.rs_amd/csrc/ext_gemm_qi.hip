@@ -690,7 +690,7 @@ static int window_tiles(int type, int rows, int cols) {
 // at 9900 sizes (512 .. 32768 rows of weights, K = 1024 .. 28672, 1 .. 2000 tokens, weights from HBM), and those of the K-quants again at 9100 sizes (1000 .. 32000 rows, K = 1024 ..
 // 14336) since their products multiply in int8: against the fastest form of each size the one taken costs 1.3 % on average (Q4_K; K = 1024, cut where whole is 15 % faster, 3.8), 0.5 %
 // (Q5_K; 1.2 before), 0.8 % (Q6_K), Q8_0 0.1 - 1.0 %.  Where that had taken another form than before, the lines were then moved again by both forms' times at 3972 sizes (by more than 3 %
-// slower than the older form 360 -> 54); lines drawn through some 40 sizes whose weights lay in the last-level cache cost 1 - 8 % and were up to 1.25 times slower
+// slower than the older form 360 -> 99, of which 60 turn with the place of the weights in memory); lines drawn through some 40 sizes whose weights lay in the last-level cache cost 1 - 8 % and were up to 1.25 times slower
 // than no groups at all.  w1, w2: workgroups of one and of two token tiles.  Times in us, Q4_K unless named:
 //   * at most a workgroup per CU, and `line` of them or more: whole, one tile, the four runs in four groups.  A cut launch has more of the chip but writes and reads four planes of the
 //     outputs, so the line falls as the tiles fill.  Cut / so: 2048 x 2048, 128 tokens (w1 64) 10.3 / 11.7, 3072 x 2048 (96) 12.8 / 12.3; 16384 x 4096, 5 tokens (128) 15.9 / 19.0,
@@ -732,8 +732,8 @@ static WideForm wide_form(int type, int cols, int T, int K, bool room) {
   auto time = [&](long long w, bool cut) { return cut ? Cs * ((w * ((S + Cs - 1) / Cs) + 255) / 256) : S * ((w + 255) / 256); };
   // two tiles' time per superblock, in tenths of one's.  Q5_K 14, but 17 where two tiles are slower (times of one as a share of two's, 1600 sizes): where only one tile is cut (0.91); with
   // 65 .. 96 tokens, whose last tile is half empty, both cut, where a row is short (0.90 - 1.01) or two make more than two rounds of the 512 resident (0.93), and one whole, two cut, up to
-  // 10240 values (0.92 - 0.96) or from 448 workgroups on (0.95); with 33 .. 64 tokens, both cut, of long rows where two make a little more than one round (0.97).  Elsewhere 1.0 - 1.2
-  const bool q5_one = (cut1 && !cut2) || (t1 == 3 && cut2 && (cut1 ? K < 4096 || w2 > 256 : K < 10240 || w2 > 448)) || (t1 == 2 && cut1 && w2 > 128 && K >= 12288);
+  // 10240 values (0.92 - 0.96) or from 448 workgroups on (0.95).  Elsewhere 1.0 - 1.2, but for 33 .. 64 tokens just above 128 workgroups of two tiles 0.94 - 1.09 by where the weights lie
+  const bool q5_one = (cut1 && !cut2) || (t1 == 3 && cut2 && (cut1 ? K < 4096 || w2 > 256 : K < 10240 || w2 > 448));
   const int ratio = q5 ? (q5_one ? 17 : 14) : cut1 ? (type == T_Q6_K ? 15 : 17) : q8 ? 18 : 15;
   const bool tie = q4 && t1 == 3 && K > 1024;  // 65 .. 96 tokens: the second of two tiles is half empty
   if (one_only || (q8 && pair) || time(w1, cut1) * 10 < time(w2, cut2) * ratio + (tie ? 1 : 0)) return {1, pair ? qi::W_PAIR : qi::W_ONE, cut1};

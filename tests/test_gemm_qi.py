@@ -846,10 +846,10 @@ FORM_LINES = [("Q4_K", 24576, 14336, 11, (1, 1, 1)), ("Q4_K", 24704, 14336, 11, 
               ("Q6_K", 12416, 9216, 220, (2, 1, 0)), ("Q6_K", 13952, 11008, 200, (2, 1, 1)), ("Q6_K", 14208, 11008, 200, (2, 1, 0)), ("Q4_K", 9600, 6144, 200, (2, 1, 0)),
               # .. which does not bring two tiles where one is taken else, nor is it drawn for rows of up to 5120 values
               ("Q6_K", 19584, 6144, 81, (1, 1, 0)), ("Q5_K", 6784, 5632, 257, (1, 1, 0)), ("Q5_K", 21120, 4096, 47, (2, 1, 0)),
-              # Q5_K in one tile: cut beside two that are not; 65 .. 96 tokens, short rows, more than two rounds, one whole and two cut; 33 .. 64 tokens of long rows; and the other sides
+              # Q5_K in one tile: cut beside two that are not; 65 .. 96 tokens, short rows, more than two rounds, one whole and two cut; and the other sides
               ("Q5_K", 15360, 13824, 73, (1, 1, 1)), ("Q5_K", 9344, 11008, 132, (1, 1, 1)), ("Q5_K", 6016, 2560, 96, (1, 1, 1)), ("Q5_K", 6016, 2560, 64, (2, 1, 1)),
               ("Q5_K", 6144, 4096, 80, (2, 1, 1)), ("Q5_K", 16896, 9216, 90, (1, 1, 1)), ("Q5_K", 11776, 9216, 90, (2, 1, 1)), ("Q5_K", 18048, 7168, 96, (1, 1, 0)),
-              ("Q5_K", 18432, 12288, 70, (2, 1, 1)), ("Q5_K", 18432, 14336, 64, (1, 1, 1)), ("Q5_K", 18432, 9216, 64, (2, 1, 1)),
+              ("Q5_K", 18432, 12288, 70, (2, 1, 1)), ("Q5_K", 18432, 14336, 64, (2, 1, 1)), ("Q5_K", 18432, 9216, 64, (2, 1, 1)),
               # one and two tiles of Q4_K that would take as long
               ("Q4_K", 29696, 11008, 79, (1, 1, 0)), ("Q4_K", 29696, 11008, 97, (2, 1, 0)), ("Q4_K", 28672, 4096, 96, (1, 1, 0)), ("Q4_K", 31104, 1024, 72, (2, 1, 0))]
 
