@@ -690,7 +690,7 @@ static int window_tiles(int type, int rows, int cols) {
 // at 9900 sizes (512 .. 32768 rows of weights, K = 1024 .. 28672, 1 .. 2000 tokens, weights from HBM), and those of the K-quants again at 9100 sizes (1000 .. 32000 rows, K = 1024 ..
 // 14336) since their products multiply in int8: against the fastest form of each size the one taken costs 1.3 % on average (Q4_K; K = 1024, cut where whole is 15 % faster, 3.8), 0.5 %
 // (Q5_K; 1.2 before), 0.8 % (Q6_K), Q8_0 0.1 - 1.0 %.  Where that had taken another form than before, the lines were then moved again by both forms' times at 3972 sizes (by more than 3 %
-// slower than the older form 360 -> 99, of which 60 turn with the place of the weights in memory); lines drawn through some 40 sizes whose weights lay in the last-level cache cost 1 - 8 % and were up to 1.25 times slower
+// slower than the older form 360 -> 99, of which 31 turn with the place of the weights in memory); lines drawn through some 40 sizes whose weights lay in the last-level cache cost 1 - 8 % and were up to 1.25 times slower
 // than no groups at all.  w1, w2: workgroups of one and of two token tiles.  Times in us, Q4_K unless named:
 //   * at most a workgroup per CU, and `line` of them or more: whole, one tile, the four runs in four groups.  A cut launch has more of the chip but writes and reads four planes of the
 //     outputs, so the line falls as the tiles fill.  Cut / so: 2048 x 2048, 128 tokens (w1 64) 10.3 / 11.7, 3072 x 2048 (96) 12.8 / 12.3; 16384 x 4096, 5 tokens (128) 15.9 / 19.0,
