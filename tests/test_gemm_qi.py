@@ -310,7 +310,7 @@ FORMS_GPU = [("Q4_K", (5400,), 1280, 34, True, True, (1, 4, 0)), ("Q4_K", (28672
 def run_form(O, be, tname, ns, k, T, acc, ws, want):
     f = be.sym("mrs_gemm_qi_form", [CI, CI, VP, CI, CI, CI], CI)(getattr(O, tname), len(ns), (CI * len(ns))(*ns), k, T, int(ws))
     assert (f & 15, f >> 4 & 15, f >> 8) == want
-    run_multi(O, be, tname, ns, k, T, None, acc, ws, seed=9)
+    run_multi(O, be, tname, ns, k, T, None, ws=ws, acc=acc, seed=9)
 
 
 @pytest.mark.parametrize("case", FORMS)
