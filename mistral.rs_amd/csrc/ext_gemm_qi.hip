@@ -306,8 +306,8 @@ __device__ __forceinline__ bool expert_tile(const int *bounds, int experts, int 
   }
   return false;
 }
-#ifndef MRS_WAIT_VMCNT0
-#define MRS_WAIT_VMCNT0() asm volatile("s_waitcnt vmcnt(0)" ::: "memory")
+#ifndef MRS_WAIT_VMCNT  // (the builtin: hipcc's own waits count it, an asm's they do not)
+#define MRS_WAIT_VMCNT(n) do { __builtin_amdgcn_s_waitcnt(0x0F70 | ((n) & 15) | (((n) >> 4) << 14)); asm volatile("" ::: "memory"); } while (0)
 #endif
 
 __device__ __forceinline__ h2 as_h2(unsigned v) { return __builtin_bit_cast(h2, v); }

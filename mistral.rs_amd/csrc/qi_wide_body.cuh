@@ -87,13 +87,20 @@
   // Q8_0: four pieces and the scales' dwords in place, each requested again when its last block has been multiplied -- half a superblock ahead; all eight would leave three
   // workgroups on a CU instead of four
   constexpr int NWQ = TYPE == T_Q8_0 ? 4 : NPC;
+  // in the order of a superblock's requests (scales, then the pieces as they are used): hipcc counts a wait in the loop by the stricter of the way in and the way round
   v4u wq[NWQ], hs_next;
   unsigned hd_next;
-#pragma unroll
-  for (int c = 0; c < NWQ; ++c) wq[c] = load_q(rec_first, c);
+  __builtin_amdgcn_sched_barrier(0);
   hs_next = load_hs(rec_first);
-  unsigned hw8[4] = {hs_next.x, hs_next.y, hs_next.z, hs_next.w};  // Q8_0
   if (TYPE != T_Q8_0) hd_next = load_hd(rec_first);
+#pragma unroll
+  for (int c = 0; c < NWQ; ++c) { __builtin_amdgcn_sched_barrier(0); wq[c] = load_q(rec_first, c); }
+  unsigned hw8[4] = {hs_next.x, hs_next.y, hs_next.z, hs_next.w};  // Q8_0
+  // requests of a wave behind its last DMA piece of a superblock, at least: all that may be in flight when the superblock is read from LDS.  They are weights, which the registers' own
+  // waits see to, one piece at a time; a wait for all of them stood for the last one's round trip in front of every superblock.  us, that / this: Q4_K 28672 x 4096, 512 tokens
+  // 150 / 139, 1999 541 / 526, 4096 x 14336, 512 tokens 74.0 / 69.6, 4096 x 4096 24.5 / 23.4, 28672 x 4096, 37 tokens 26.3 / 24.7; Q6_K 4096 x 14336, 512 tokens 85.5 / 81.5, 1999
+  // 315 / 305; Q5_K 4096 x 14336, 512 tokens 99.9 / 89.8
+  constexpr int behind = TYPE == T_Q8_0 ? 5 : NT == 2 ? (TYPE == T_Q4_K ? 2 : 4) : (TYPE == T_Q4_K ? 3 : 6);
   const f16v zero = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
   auto add_pair = [&](int i) {  // W_PAIR: the second group's terms of its step i
 #pragma unroll
@@ -120,7 +127,7 @@
       // once, as the product alone would.  A scale that is not finite would make it inf - inf, a negative one or a zero (with quants that are not all zeros) would lose the sign of
       // a zero: such a superblock is done over with a conversion.  Gate / up of 28672 x 4096, one token tile, us, a conversion and scales from LDS / this: 700 tokens 290 / 272, 2000 tokens 780 / 739 (the fma alone, scales from LDS:
       // 311, 831); two token tiles 263, 720.
-      MRS_WAIT_VMCNT0();
+      MRS_WAIT_VMCNT(behind);
       __syncthreads();
       if (MODE == W_PAIR && grp == 0 && it > 0) add_pair(it - 1);
       stage_meta(sb + STEP, it + 1, more);
@@ -231,7 +238,6 @@
       }
     };
     constexpr int DIGIT = TYPE == T_Q4_K ? 3 : 8;
-    constexpr bool EARLY = MODE != W_RUNS4;  // the next superblock's rows are requested in front of the matrix instructions, all of them (in 16 waves' 128 registers: one by one behind them)
     // the activations' fragments are read from LDS two steps ahead where the registers hold them (not in 16 waves' 128; Q5_K spills)
     constexpr int AHEAD = MODE == W_RUNS4 || TYPE == T_Q5_K ? 1 : 2;
     i4v fr[AHEAD + 1][NT];
@@ -240,15 +246,10 @@
 #pragma unroll
     for (int p = 0; p < 4; ++p) digits(0, p, wl[0][p], wh[0][p]);
     __builtin_amdgcn_sched_barrier(0);
-    MRS_WAIT_VMCNT0();  // this wave's DMA pieces of superblock sb have landed
+    MRS_WAIT_VMCNT(behind);  // this wave's DMA pieces of superblock sb have landed
     __syncthreads();    // everyone's have, and every wave has finished reading the other buffer
     if (MODE == W_PAIR && grp == 0 && it > 0) add_pair(it - 1);
     stage_meta(sb + STEP, it + 1, more);
-    if constexpr (EARLY) {
-#pragma unroll
-      for (int i = 0; i < NSTAGE; ++i) stage_q(sb + STEP, it + 1, i, more);
-      __builtin_amdgcn_sched_barrier(0);
-    }
     hs_next = load_hs(rec_next); hd_next = load_hd(rec_next);
     if (TYPE != T_Q4_K) wq[0] = load_q(rec_next, 0);
     auto frag = [&](int k, int tt) -> i4v { return MRS_LDS_FRAG(i4v, smem, abase ^ (unsigned)(32 * k), tt * (32 * ROWB)); };
@@ -282,10 +283,7 @@
 #pragma unroll
           for (int p = tt * 4 / NT; p < tt * 4 / NT + 2 / NT; ++p) digits(k + 1, p, wl[nx][p], wh[nx][p]);
         }
-        if constexpr (!EARLY) {
-#pragma unroll
-          for (int i = 0; i < NSTAGE; ++i) if (tt == 0 && k == i * (8 / NSTAGE)) stage_q(sb + STEP, it + 1, i, more);
-        }
+        if (tt == 0 && k < NSTAGE) stage_q(sb + STEP, it + 1, k, more);
         __builtin_amdgcn_sched_barrier(0);
         XH[tt] = __builtin_amdgcn_mfma_i32_32x32x32_i8(fr[k % (AHEAD + 1)][tt], hi, XH[tt], 0, 0, 0);
         if (k + 1 < 8) {
@@ -359,7 +357,7 @@
   const bool gap = S <= 3 * Cs;  // a row's last run(s) are empty: + 0, the neutral - 0 of `run` in its place would leave the sign to a sum of negative zeros
   if constexpr (MODE == W_RUNS2 || MODE == W_RUNS4) {
     constexpr int PL = MODE == W_RUNS4 ? 4 : 3, VG = 16 / GROUPS;  // planes: c0 .. c3 | c0 + c1, c2, c3;  outputs of a group, of every token tile
-    MRS_WAIT_VMCNT0();  // the last requests to LDS (out of range: zeros) have landed
+    MRS_WAIT_VMCNT(0);  // the last requests to LDS (out of range: zeros) have landed
     __syncthreads();
     float *const sums = (float *)smem_all + (size_t)wave * PL * NT * 1024 + lane * 4;  // [4 waves][planes][4 NT][64 lanes][4]
     auto put = [&](int plane, const float (&c)[NT][16]) {

@@ -3,6 +3,9 @@ quantizer) x Q4_K / Q5_K / Q6_K weights through v_mfma_i32_32x32x32_i8 on exact 
 Every output row equals the decode engine's GEMV of that token (oracle/cpu_path_oracle.c orc_gemv_engine) BIT FOR BIT -- so does the GPU result against the
 batch-1 decode kernel itself.  Also: v_mfma_f32_32x32x16_f16, which sums the mins (run sums x mins), is exact on integers below 2^24 (adversarial magnitudes)."""
 import ctypes as C
+import os
+import re
+import subprocess
 
 import numpy as np
 import pytest
@@ -858,3 +861,64 @@ FORM_LINES = [("Q4_K", 24576, 14336, 11, (1, 1, 1)), ("Q4_K", 24704, 14336, 11, 
 def test_gemm_qi_form_lines(oracle, tname, n, k, T, want):
     f = HostBackend().sym("mrs_gemm_qi_form", [CI, CI, VP, CI, CI, CI], CI)(getattr(oracle, tname), 1, (CI * 1)(n), k, T, 1)
     assert (f & 15, f >> 4 & 15, f >> 8) == want
+
+
+def test_the_wait_of_a_superblock_covers_its_dma(tmp_path):
+    """A superblock's rows are read from LDS behind a wait that leaves the requests behind its last DMA piece in flight, by their count.  Every way through the generated code to such a wait
+    has to have made that many (one that the compiler drops, or moves in front of the DMA, would let a piece pass).  State: requests since the last DMA piece, at least; None: no piece in flight."""
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    csrc, hipcc, out = os.path.join(root, "mistral.rs_amd", "csrc"), os.environ.get("HIPCC", "/opt/rocm/bin/hipcc"), str(tmp_path / "qi.s")
+    subprocess.run([hipcc, "--offload-arch=gfx950", "-O3", "-std=c++17", "-ffp-contract=off", "-w", "-I" + csrc, "-I" + os.path.join(root, "include"), "-Xclang", "-target-feature", "-Xclang",
+                    "-packed-fp32-ops", "--cuda-device-only", "-S", os.path.join(csrc, "ext_gemm_qi.hip"), "-o", out], check=True)
+    kernels = re.findall(r"^(_Z\w*gemm_qi_(?:wide|mixed|tail)_kernel\w*):(.*?)\.end_amdhsa_kernel", open(out).read(), re.M | re.S)
+    assert len(kernels) >= 20
+    for name, code in kernels:
+        blocks, order = {"entry": []}, ["entry"]
+        for line in code.splitlines():
+            label = re.match(r"(\.LBB\w+):", line)
+            if label:
+                order.append(label.group(1))
+                blocks[order[-1]] = []
+            elif re.match(r"\s+[a-z]\w+", line):
+                blocks[order[-1]].append(line.split())
+                if line.split()[0].startswith("s_cbranch"):  # what follows is reached by falling through
+                    order.append("%s+%d" % (order[-1], len(order)))
+                    blocks[order[-1]] = []
+        states, work, waits = {"entry": None}, ["entry"], {}
+
+        def reach(block, state, states=states, work=work):
+            if block not in states:
+                states[block] = state
+            elif state is None or (states[block] is not None and states[block] <= state):
+                return
+            else:
+                states[block] = state
+            work.append(block)
+        while work:
+            block = work.pop()
+            d, waited, through = states[block], None, True
+            for i, op in enumerate(blocks[block]):
+                if op[0].startswith(("buffer_", "global_")):
+                    d = 0 if op[-1] == "lds" else None if d is None else d + 1
+                elif op[0] == "s_waitcnt" and any(o.startswith("vmcnt") for o in op):
+                    n = int(re.search(r"vmcnt\((\d+)\)", " ".join(op)).group(1))
+                    d = None if d is not None and n <= d else d
+                    waited = n
+                elif op[0] == "s_barrier":
+                    if waited is not None:
+                        waits[block, i] = (d, waited)
+                    waited = None
+                elif op[0].startswith(("s_cbranch", "s_branch")):
+                    reach(op[1], d)
+                    through = op[0] != "s_branch"
+                elif op[0] == "s_endpgm":
+                    through = False
+            if through and order.index(block) + 1 < len(order):
+                reach(order[order.index(block) + 1], d)
+        # the kernels' own waits, by type and token tiles (a group of waves past its last superblock keeps the others' barriers behind a looser one of the compiler's: it reads nothing)
+        form = [int(v) for v in re.findall(r"Li(\d+)E", name)]
+        types, tiles = (form[:2], form[2:3]) if "mixed" in name else (form[:1], form[1:2] if "wide" in name else [1, 2])
+        own = {5 if t == 8 else {(12, 2): 2, (12, 1): 3}.get((t, nt), 4 if nt == 2 else 6) for t in types for nt in tiles}
+        seen = [(n, d) for d, n in waits.values() if n in own]
+        assert {n for n, _ in seen} == own, (name, own, waits)
+        assert all(d is None for _, d in seen), (name, waits)
