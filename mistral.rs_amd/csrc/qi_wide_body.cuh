@@ -254,6 +254,13 @@
     if (TYPE != T_Q4_K) wq[0] = load_q(rec_next, 0);
     auto frag = [&](int k, int tt) -> i4v { return MRS_LDS_FRAG(i4v, smem, abase ^ (unsigned)(32 * k), tt * (32 * ROWB)); };
     i16v XL[NT], XH[NT];
+    // the terms' operands leave LDS behind step 6 (Q5_K's registers are full: in front of the terms, a round trip per token tile).  us, that / this: Q4_K 4096 x 14336, 1999 tokens
+    // 258 / 250, 6144 x 4096, 512 tokens 37.7 / 35.0, 28672 x 4096, 1999 tokens 528 / 523; Q6_K 4096 x 14336, 1999 tokens 301 / 298
+    constexpr bool EARLY = TYPE != T_Q5_K;
+    const float *yd_s = (const float *)meta_s;
+    auto run_sums = [&](int tt) { return *(const h8 *)(meta_s + YD_ + (tt * 32 + nn) * 32 + hf * 16); };
+    float yd[NT];
+    h8 bsf[NT];
 #pragma unroll
     for (int tt = 0; tt < NT; ++tt)
 #pragma unroll
@@ -290,6 +297,10 @@
 #pragma unroll
           for (int p = tt * 4 / NT + 2 / NT; p < (tt + 1) * 4 / NT; ++p) digits(k + 1, p, wl[nx][p], wh[nx][p]);
         }
+        if (EARLY && k == 6) {
+          yd[tt] = yd_s[tt * 32 + nn];
+          if (TYPE != T_Q6_K) bsf[tt] = run_sums(tt);
+        }
         if (tt == NT - 1) {  // step k + 1 has been built
           if (TYPE == T_Q4_K ? (k & 1) == 0 : k + 1 < 8) { const int i = TYPE == T_Q4_K ? k >> 1 : (k + 1) & 7; wq[i] = load_q(rec_next, i); }
         }
@@ -297,17 +308,16 @@
       }
     }
     __builtin_amdgcn_s_setprio(0);
-    const float *yd_s = (const float *)meta_s;
     const f32v zero32 = {0.f};
     // d yd (and dmin yd) of the tile's outputs, each product rounded once: one matrix instruction of two 32 x 32 outer products (lane halves = blocks).  It adds the products to + 0, so
     // one that is - 0 (a negative d of a token block of zeros) comes out as + 0: an output all of whose terms are zeros may have the other sign than in the decode engine
     const float dd = half_bits_to_float((uint16_t)(hf ? hd >> 16 : hd & 0xffff));
-    auto products = [&](int tt) -> f32v { return __builtin_amdgcn_mfma_f32_32x32x1f32(yd_s[tt * 32 + nn], dd, zero32, 0, 0, 0); };
+    auto products = [&](int tt) -> f32v { return __builtin_amdgcn_mfma_f32_32x32x1f32(yd[tt], dd, zero32, 0, 0, 0); };
     auto isum = [&](int tt, int v) { return (float)(XL[tt][v] + (int)((unsigned)XH[tt][v] << DIGIT)); };
     if constexpr (TYPE == T_Q6_K) {
 #pragma unroll
       for (int tt = 0; tt < NT; ++tt) {
-        const f16v dy = __builtin_amdgcn_mfma_f32_32x32x2f32(hf ? 0.f : yd_s[tt * 32 + nn], hf ? 0.f : dd, zero, 0, 0, 0);  // one block: half of the registers
+        const f16v dy = __builtin_amdgcn_mfma_f32_32x32x2f32(hf ? 0.f : yd[tt], hf ? 0.f : dd, zero, 0, 0, 0);  // one block: half of the registers
 #pragma unroll
         for (int v = 0; v < 16; ++v) run[tt][v] = run[tt][v] + dy[v] * isum(tt, v);
         __builtin_amdgcn_sched_barrier(0);
@@ -321,9 +331,9 @@
       const h8 wm8 = mk_h8(wm[0], wm[1], wm[2], wm[3]);
 #pragma unroll
       for (int tt = 0; tt < NT; ++tt) {
-        const h8 bsf = *(const h8 *)(meta_s + YD_ + (tt * 32 + nn) * 32 + hf * 16);
+        if constexpr (!EARLY) { yd[tt] = yd_s[tt * 32 + nn]; bsf[tt] = run_sums(tt); }
         const f32v dy = products(tt);
-        const f16v M = __builtin_amdgcn_mfma_f32_32x32x16_f16(bsf, wm8, zero, 0, 0, 0);
+        const f16v M = __builtin_amdgcn_mfma_f32_32x32x16_f16(bsf[tt], wm8, zero, 0, 0, 0);
 #pragma unroll
         for (int v = 0; v < 16; ++v) run[tt][v] = run[tt][v] + fmaf(dy[v], isum(tt, v), -(dy[16 + v] * M[v]));
         __builtin_amdgcn_sched_barrier(0);  // one token tile at a time: the sums of all of them would not fit the registers
