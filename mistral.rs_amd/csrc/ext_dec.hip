@@ -18,6 +18,12 @@
 
 #include "dec_gemv.cuh"
 
+// a uniform value that the kernel does not write, by the scalar unit (a pointer out of the argument block is a vector load otherwise); MRS_KEEP_S: it has arrived (arguments: read with the
+// others and not behind the first branch)
+#ifndef MRS_SLOAD32
+#define MRS_SLOAD32(p) (*(const __attribute__((address_space(4))) uint32_t *)(size_t)(p))
+#define MRS_KEEP_S(x) asm volatile("" ::"s"(x))
+#endif
 #ifndef MRS_WAIT_VMCNT0
 #define MRS_WAIT_VMCNT0() asm volatile("s_waitcnt vmcnt(0)" ::: "memory")
 #endif
@@ -328,27 +334,42 @@ __device__ __forceinline__ float attn4_probs(const float (&val)[2], const bool (
   ps = ps + dpp_f<0x128>(ps);               // lane ^ 8
   return ps + __shfl_xor(ps, 16, 64);
 }
-// o += P V over the block's tokens, dims dim0 + 4 (lane / 4) + v of head lane % 4
-template <class CT, int ND>
-__device__ __forceinline__ void attn4_values(const char *v_s, const float *p_s, int b, int ctx, int dim0, int lane, f4v (&o)[ND]) {
-  const bool tail = (b + 1) * 32 > ctx;  // slots past the context may hold NaNs
+// o += P V over the block's tokens, dims dim0 + 4 (lane / 4) + v of head lane % 4.  The operands leave LDS all at once, ahead of the chain (eight tokens at a time it stood
+// still for a read every eight products: 0.52 us per block)
+template <int ND> struct Attn4V { int4 v[ND][4]; };
+template <int ND>
+__device__ __forceinline__ void attn4_read_values(const char *v_s, int b, int ctx, int dim0, int lane, Attn4V<ND> &x) {
 #pragma unroll
-  for (int c = 0; c < 4; ++c) {
-    const float4 p0 = *(const float4 *)(p_s + (lane & 3) * A4_P + 8 * c), p1 = *(const float4 *)(p_s + (lane & 3) * A4_P + 8 * c + 4);
-    float vf[ND][8];
+  for (int n = 0; n < ND; ++n)
 #pragma unroll
-    for (int n = 0; n < ND; ++n) {
-      int4 raw = attn4_read_v(v_s, dim0 + 64 * n + lane, c);
-      if (tail) {
-        int *d = (int *)&raw;
+    for (int c = 0; c < 4; ++c) x.v[n][c] = attn4_read_v(v_s, dim0 + 64 * n + lane, c);
+  if ((b + 1) * 32 > ctx) {  // slots past the context may hold NaNs
+#pragma unroll
+    for (int n = 0; n < ND; ++n)
+#pragma unroll
+      for (int c = 0; c < 4; ++c) {
+        int *d = (int *)&x.v[n][c];
 #pragma unroll
         for (int u = 0; u < 4; ++u) {
           const int left = ctx - (b * 32 + c * 8 + 2 * u);  // a dword holds two tokens
           d[u] = left > 1 ? d[u] : left == 1 ? d[u] & 0xffff : 0;
         }
       }
-      unpack16<CT>(raw, vf[n]);
-    }
+  }
+}
+struct Attn4P { float4 p[8]; };
+__device__ __forceinline__ void attn4_read_probs(const float *p_s, int lane, Attn4P &x) {
+#pragma unroll
+  for (int i = 0; i < 8; ++i) x.p[i] = *(const float4 *)(p_s + (lane & 3) * A4_P + 4 * i);
+}
+template <class CT, int ND>
+__device__ __forceinline__ void attn4_values(const Attn4V<ND> &x, const Attn4P &pr, f4v (&o)[ND]) {
+#pragma unroll
+  for (int c = 0; c < 4; ++c) {
+    float vf[ND][8];
+#pragma unroll
+    for (int n = 0; n < ND; ++n) unpack16<CT>(x.v[n][c], vf[n]);
+    const float4 p0 = pr.p[2 * c], p1 = pr.p[2 * c + 1];
     const float pb[8] = {p0.x, p0.y, p0.z, p0.w, p1.x, p1.y, p1.z, p1.w};
 #pragma unroll
     for (int j = 0; j < 8; ++j)
@@ -393,18 +414,23 @@ __device__ __forceinline__ void attn4_merge(const Attn2Args &a, int kvh, int seq
       }
     const float w = fast_exp_ref(m - dec2::wave_max_all(m)), lw = l * w;  // split j's in lane j
     float s_all = 0.f, a0 = 0.f, a1 = 0.f;
+    auto add = [&](int g, int k) {
+      const float wj = dec2::rlf(w, g * MB + k), lwj = dec2::rlf(lw, g * MB + k);
+      const float t0 = __uint_as_float(r[g][k].x) * wj, t1 = __uint_as_float(r[g][k].y) * wj;
+      s_all = s_all + lwj;
+      a0 = a0 + t0; a1 = a1 + t1;
+    };
 #pragma unroll
-    for (int g = 0; g < 4; ++g)
-      if (g * MB < ns) {
+    for (int g = 0; g < 4; ++g) {
+      if ((g + 1) * MB <= ns) {  // all of them: no branch between one split and the next
+#pragma unroll
+        for (int k = 0; k < MB; ++k) add(g, k);
+      } else if (g * MB < ns) {
 #pragma unroll
         for (int k = 0; k < MB; ++k)
-          if (g * MB + k < ns) {
-            const float wj = dec2::rlf(w, g * MB + k), lwj = dec2::rlf(lw, g * MB + k);
-            const float t0 = __uint_as_float(r[g][k].x) * wj, t1 = __uint_as_float(r[g][k].y) * wj;
-            s_all = s_all + lwj;
-            a0 = a0 + t0; a1 = a1 + t1;
-          }
+          if (g * MB + k < ns) add(g, k);
       }
+    }
     const float inv = 1.0f / s_all;
     *(float2 *)&o_s[wave + 4 * i][2 * lane] = make_float2(a0 * inv, a1 * inv);
   }
@@ -437,8 +463,9 @@ __global__ void __launch_bounds__(256, 3) dec_attn4_kernel(const Attn2Args a) {
   const int tid = tid_opaque(), lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int kvh = blockIdx.x, seq = blockIdx.y, split0 = blockIdx.z * SPW, split = split0 + wave / HG, head0 = kvh * G + wave % HG * 4;
   // the page index does not depend on the context length: both scalar loads leave together
-  const unsigned page = t.block_tables[(size_t)seq * t.max_blocks_per_seq + min(split, t.max_blocks_per_seq - 1)];
-  const int ctx = (int)t.context_lens[seq], ns = (ctx + 31) / 32;
+  const unsigned page = MRS_SLOAD32(t.block_tables + (size_t)seq * t.max_blocks_per_seq + min(split, t.max_blocks_per_seq - 1));
+  const int ctx = (int)MRS_SLOAD32(t.context_lens + seq), ns = (ctx + 31) / 32;
+  MRS_KEEP_S(page); MRS_KEEP_S(t.k_cache); MRS_KEEP_S(t.kv_block_stride); MRS_KEEP_S(t.kv_head_stride); MRS_KEEP_S(t.window);
   if (split0 >= ns) return;  // workgroup-uniform: no split of this sequence lands here
   if (split < ns) {
     const int lo = t.window > 0 && ctx > t.window ? ctx - t.window : 0;
@@ -453,10 +480,15 @@ __global__ void __launch_bounds__(256, 3) dec_attn4_kernel(const Attn2Args a) {
       MRS_WAVE_SYNC();
       float val[2]; bool ok[2];
       m = attn4_scores<CT>(t, kr, q_s[wave], split, ctx, lo, lane, val, ok);
-      l = attn4_probs(val, ok, m, p_s[wave], lane);
       MRS_WAIT_VMCNT0();  // the values have landed
       MRS_WAVE_SYNC();
-      attn4_values<CT, 2>(v_s[wave], p_s[wave], split, ctx, 0, lane, o);
+      Attn4V<2> vals;
+      Attn4P probs;
+      attn4_read_values<2>(v_s[wave], split, ctx, 0, lane, vals);
+      l = attn4_probs(val, ok, m, p_s[wave], lane);
+      MRS_WAVE_SYNC();
+      attn4_read_probs(p_s[wave], lane, probs);
+      attn4_values<CT, 2>(vals, probs, o);
     }
     attn4_publish_o<TICKET>(t, seq, head0, split, 0, lane, o[0]);
     attn4_publish_o<TICKET>(t, seq, head0, split, 64, lane, o[1]);
@@ -479,8 +511,10 @@ __global__ void __launch_bounds__(256, 2) dec_attn4_long_kernel(const Attn2Args 
   const int tid = tid_opaque(), lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), hd = lane & 3;
   const int kvh = blockIdx.x, seq = blockIdx.y, split = blockIdx.z;
   const uint32_t *bt = t.block_tables + (size_t)seq * t.max_blocks_per_seq;
-  unsigned page = bt[min(split * t.bpw + wave, t.max_blocks_per_seq - 1)];
-  const int ctx = (int)t.context_lens[seq], nblk = (ctx + 31) / 32, ns = (nblk + t.bpw - 1) / t.bpw;
+  unsigned page = MRS_SLOAD32(bt + min(split * t.bpw + wave, t.max_blocks_per_seq - 1));
+  const int ctx = (int)MRS_SLOAD32(t.context_lens + seq);
+  MRS_KEEP_S(page); MRS_KEEP_S(t.k_cache); MRS_KEEP_S(t.kv_block_stride); MRS_KEEP_S(t.kv_head_stride); MRS_KEEP_S(t.window);
+  const int nblk = (ctx + 31) / 32, ns = (nblk + t.bpw - 1) / t.bpw;
   if (split >= ns) return;  // workgroup-uniform
   const int b0 = split * t.bpw, b1 = min(b0 + t.bpw, nblk), lo = t.window > 0 && ctx > t.window ? ctx - t.window : 0;
   const int pv_hg = G == 8 ? wave >> 1 : 0, pv_dim = (wave & 1) * 64;  // P . V: the wave's group of heads and dims
@@ -495,7 +529,7 @@ __global__ void __launch_bounds__(256, 2) dec_attn4_long_kernel(const Attn2Args 
     attn_load_k(t, base_of(page), kr, b0 + wave < b1 ? KV_BLOCK_BYTES : 0);
     if (wave < HG) attn4_stage_q(t, seq, kvh * G + wave * 4, q_s[wave], lane);
     if (b0 + wave < b1) attn4_stage_v(t, base_of(page), v_dyn + wave * A4_V, lane);
-    page = bt[min(b0 + 4 + wave, b1 - 1)];
+    page = MRS_SLOAD32(bt + min(b0 + 4 + wave, b1 - 1));
     __syncthreads();
     for (int g0 = b0, it = 0; g0 < b1; g0 += 4, ++it) {
       const int b = g0 + wave, nb = min(4, b1 - g0);
@@ -513,7 +547,7 @@ __global__ void __launch_bounds__(256, 2) dec_attn4_long_kernel(const Attn2Args 
       if (g0 + 4 < b1) {
         attn_load_k(t, next, kr, b + 4 < b1 ? KV_BLOCK_BYTES : 0);
         if (b + 4 < b1) attn4_stage_v(t, next, v_dyn + ((it + 1) & 1) * 4 * A4_V + wave * A4_V, lane);
-        page = bt[min(b + 8, b1 - 1)];
+        page = MRS_SLOAD32(bt + min(b + 8, b1 - 1));
       }
       if (b < b1) {
 #pragma unroll
@@ -529,17 +563,37 @@ __global__ void __launch_bounds__(256, 2) dec_attn4_long_kernel(const Attn2Args 
         for (int w = 0; w < nb; ++w) m_run[h] = fmaxf(m_run[h], mx_s[it & 1][w][h * 4 + hd]);
       __syncthreads();  // B: the probabilities
       if (pv) {
-        for (int w = 0; w < nb; ++w) {
-          const float mn = fmaxf(m_pv, mx_s[it & 1][w][pv_hg * 4 + hd]), ps = ps_s[w][pv_hg * 4 + hd];
-          if (g0 + w == b0) {
-            l = ps;
-          } else {
-            const float alpha = fast_exp_ref(m_pv - mn);
-            l = l * alpha + ps;
-            o[0] = o[0] * alpha;
-          }
+        const char *v_g = v_dyn + (it & 1) * 4 * A4_V;
+        Attn4V<1> vals[2];
+        Attn4P probs[2];
+        auto read = [&](int w) {
+          attn4_read_values<1>(v_g + w * A4_V, g0 + w, ctx, pv_dim, lane, vals[w & 1]);
+          attn4_read_probs(p_s[w][pv_hg], lane, probs[w & 1]);
+        };
+        read(0);
+        // the four blocks' corrections first: their exponentials run side by side, and between the blocks' chains of products stands one multiplication
+        float mxw[4], psw[4], alpha[4];
+#pragma unroll
+        for (int w = 0; w < 4; ++w) { mxw[w] = w < nb ? mx_s[it & 1][w][pv_hg * 4 + hd] : -FLT_MAX; psw[w] = ps_s[w][pv_hg * 4 + hd]; }
+#pragma unroll
+        for (int w = 0; w < 4; ++w) {
+          const float mn = fmaxf(m_pv, mxw[w]);
+          alpha[w] = fast_exp_ref(m_pv - mn);
           m_pv = mn;
-          attn4_values<CT, 1>(v_dyn + (it & 1) * 4 * A4_V + w * A4_V, p_s[w][pv_hg], g0 + w, ctx, pv_dim, lane, o);
+        }
+#pragma unroll
+        for (int w = 0; w < 4; ++w) MRS_OPAQUE_TID(alpha[w]);  // here, not where they are used
+#pragma unroll
+        for (int w = 0; w < 4; ++w) {
+          if (w >= nb) break;  // wave-uniform
+          if (w + 1 < nb) read(w + 1);
+          if (g0 + w == b0) {
+            l = psw[w];
+          } else {
+            l = l * alpha[w] + psw[w];
+            o[0] = o[0] * alpha[w];
+          }
+          attn4_values<CT, 1>(vals[w & 1], probs[w & 1], o);
         }
       }
     }

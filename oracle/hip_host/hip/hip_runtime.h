@@ -475,6 +475,8 @@ static inline void hiphost_buffer_load_lds(__amdgpu_buffer_rsrc_t r, char *dst, 
 #define MRS_LDS_FRAG(TYPE, P, ADDR, OFF) (*(const TYPE *)((P) + (ADDR) + (OFF)))
 #define MRS_WAIT_VMCNT0() ((void)0)                                     /* product code: s_waitcnt vmcnt(0) */
 #define MRS_WAIT_VMCNT(N) ((void)0)                                     /* product code: s_waitcnt vmcnt(N) */
+#define MRS_SLOAD32(p) (*(p))                                           /* product code: a scalar load */
+#define MRS_KEEP_S(x) ((void)(x))
 #define MRS_OPAQUE(V) ((void)0)                                         /* product code: an empty asm that hides the value from the optimizer */
 #define MRS_KEEP_BRANCH() ((void)0)
 #define __builtin_amdgcn_fence(ORDER, SCOPE) ((void)0)                  /* one workgroup runs at a time: nothing to order */
