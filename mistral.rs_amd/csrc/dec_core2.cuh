@@ -142,12 +142,38 @@ __device__ __forceinline__ Act act_view(char *smem, int K, int ncols, int mode) 
   return Act{smem, (const float *)d, (const int *)(d + (size_t)ncols * Sp * dw * 4), K, S, dw, (S + 3) / 4, CQ, Sp};
 }
 
-// quantize N superblocks at once: lane l holds elements 4 l .. 4 l + 3 of each (v[n], superblock sb[n], live[n] wave-uniform) -> column c of the image.
-// Every step is a loop over n so that the N reduction chains interleave (one chain alone is ~100 dependent instructions).
+// quantize N = 1, 2 or 4 superblocks at once: lane l holds elements 4 l .. 4 l + 3 of each (v[n], superblock sb[n], live[n] wave-uniform) -> column c of the image.
 // Quantizers: candle BlockQ8K::from_float (amax with its sign, iscale = -128 / max, q = min(127, round(iscale x)), d = 1 / iscale, the FIRST
 // element of largest magnitude wins) and quantize_row_q8_0 (d = amax / 127, q = round(x / d), d kept as f16) -- oracle/ggml_oracle.c.
+// A launch that quantizes its own rows is bound by the vector instructions of this function (four cycles each, two waves per SIMD, 256 workgroups that all do the same): the largest
+// magnitudes of the N superblocks are reduced together, superblock n in the lanes n of N, so that reduction, both divisions and the stores of scales and run sums happen once for all.
+// us, a reduction and two divisions per superblock / this: 4096 x 14336 from f32, Q4_K 12.6 / 11.7, Q6_K 13.7 / 13.1; 28672 x 4096 behind a norm 15.25 / 15.1.
+template <int N> __device__ __forceinline__ float lane_merge(const float (&a)[N], int lane) {  // lane l: the largest of superblock l % N over the lane's quad
+  if constexpr (N == 4) {
+    const bool o1 = (lane & 1) != 0, o2 = (lane & 2) != 0;
+    const float b0 = fmaxf(o1 ? a[1] : a[0], dppf<0xB1>(o1 ? a[0] : a[1])), b1 = fmaxf(o1 ? a[3] : a[2], dppf<0xB1>(o1 ? a[2] : a[3]));
+    return fmaxf(o2 ? b1 : b0, dppf<0x4E>(o2 ? b0 : b1));
+  } else {
+    float b;
+    if constexpr (N == 2) { const bool o1 = (lane & 1) != 0; b = fmaxf(o1 ? a[1] : a[0], dppf<0xB1>(o1 ? a[0] : a[1])); }
+    else b = fmaxf(a[0], dppf<0xB1>(a[0]));
+    return fmaxf(b, dppf<0x4E>(b));
+  }
+}
+__device__ __forceinline__ float max_rows(float v) {  // the largest of a lane's column over the wave's four rows of 16 lanes
+  const unsigned u = __float_as_uint(v);
+  const auto s = __builtin_amdgcn_permlane16_swap(u, u, false, false);
+  const unsigned w = __float_as_uint(fmaxf(__uint_as_float(s[0]), __uint_as_float(s[1])));
+  const auto t = __builtin_amdgcn_permlane32_swap(w, w, false, false);
+  return fmaxf(__uint_as_float(t[0]), __uint_as_float(t[1]));
+}
+// four values as the bytes of a dword (their low bytes)
+__device__ __forceinline__ int pack4(int q0, int q1, int q2, int q3) {
+  return (int)(__builtin_amdgcn_perm((unsigned)q1, (unsigned)q0, 0x0c0c0400u) | __builtin_amdgcn_perm((unsigned)q3, (unsigned)q2, 0x04000c0cu));
+}
 template <int N>
 __device__ __forceinline__ void quantize_multi(const float4 (&v)[N], const int (&sb)[N], const bool (&live)[N], int c, int mode, char *img, int K, int ncols) {
+  static_assert(N == 1 || N == 2 || N == 4, "a superblock per lane of N");
   const int lane = lane_opaque(), S = K / 256, dw = act_dw(mode), Cs = (S + 3) / 4, CQ = act_cq(K), Sp = act_sp(K);
   char *q0p = img + (size_t)c * 4 * CQ;
   float *d0p = (float *)(img + (size_t)ncols * 4 * CQ) + (size_t)c * Sp * dw;
@@ -155,16 +181,32 @@ __device__ __forceinline__ void quantize_multi(const float4 (&v)[N], const int (
   int qo[N];
 #pragma unroll
   for (int n = 0; n < N; ++n) { const int sbn = live[n] ? sb[n] : 0, p = chunk_of(sbn, Cs); qo[n] = p * CQ + (sbn - p * Cs) * 256; }
+  // the lane's superblock: n = lane % N
+  const int mine = lane & (N - 1);
+  int sbl = sb[0];
+  bool livel = live[0];
+#pragma unroll
+  for (int n = 1; n < N; ++n) { sbl = mine == n ? sb[n] : sbl; livel = mine == n ? live[n] : livel; }
   if (mode == ACT_Q8K) {
-    float amax[N], mx[N];
+    float hi4[N], lo4[N], a[N];
+#pragma unroll
+    for (int n = 0; n < N; ++n) {
+      hi4[n] = fmaxf(fmaxf(v[n].x, v[n].y), fmaxf(v[n].z, v[n].w)); lo4[n] = fminf(fminf(v[n].x, v[n].y), fminf(v[n].z, v[n].w));
+      a[n] = fmaxf(hi4[n], -lo4[n]);
+    }
+    float am = lane_merge<N>(a, lane);
+    am = fmaxf(am, dppf<0x124>(am));
+    am = fmaxf(am, dppf<0x128>(am));
+    am = max_rows(am);
+    // the sign of the first element with the largest magnitude decides iscale; only when +amax and -amax both occur does the order matter
+    float amax[N];
+    unsigned neg = 0;
     bool tie = false;
 #pragma unroll
     for (int n = 0; n < N; ++n) {
-      const float hi4 = fmaxf(fmaxf(v[n].x, v[n].y), fmaxf(v[n].z, v[n].w)), lo4 = fminf(fminf(v[n].x, v[n].y), fminf(v[n].z, v[n].w));
-      amax[n] = wave_max_all(fmaxf(hi4, -lo4));
-      // the sign of the first element with the largest magnitude decides iscale; only when +amax and -amax both occur does the order matter
-      const unsigned long long bp = __ballot(hi4 == amax[n]), bn = __ballot(lo4 == -amax[n]);
-      mx[n] = bn == 0 ? amax[n] : -amax[n];
+      amax[n] = rlf(am, n);
+      const unsigned long long bp = __ballot(hi4[n] == amax[n]), bn = __ballot(lo4[n] == -amax[n]);
+      neg |= bn == 0 ? 0u : 1u << n;
       tie = tie || (bp != 0 && bn != 0 && amax[n] != 0.f);
     }
     if (tie) {  // wave-uniform, rare: the exact first-index search
@@ -174,40 +216,50 @@ __device__ __forceinline__ void quantize_multi(const float4 (&v)[N], const int (
         const int first = wave_min_all(lane * 4 + cand);
         const int sl = (first >> 2) & 63, comp = first & 3;
         const float m1 = rlf(comp == 0 ? v[n].x : (comp == 1 ? v[n].y : (comp == 2 ? v[n].z : v[n].w)), sl);
-        mx[n] = amax[n] != 0.f ? m1 : mx[n];
+        neg = (neg & ~(1u << n)) | (m1 < 0.f ? 1u << n : 0u);
       }
     }
+    const float mx = ((neg >> mine) & 1u) ? -am : am;
+    const bool nz = am != 0.f;
+    const float iscale = nz ? -128.f / mx : 0.f;  // all-zero block: every quant 0, d = 0
+    const float dd = nz ? 1.0f / iscale : 0.f;
+    int packed[N], sum[N];
 #pragma unroll
     for (int n = 0; n < N; ++n) {
-      const bool nz = amax[n] != 0.f;
-      const float iscale = nz ? -128.f / mx[n] : 0.f;  // all-zero block: every quant 0, d = 0
-      const int q0 = (int)fminf(127.f, round_away(iscale * v[n].x)), q1 = (int)fminf(127.f, round_away(iscale * v[n].y));
-      const int q2 = (int)fminf(127.f, round_away(iscale * v[n].z)), q3 = (int)fminf(127.f, round_away(iscale * v[n].w));
-      const float dd = nz ? 1.0f / iscale : 0.f;
-      const int packed = (q0 & 0xff) | ((q1 & 0xff) << 8) | ((q2 & 0xff) << 16) | ((q3 & 0xff) << 24);
-      int sum = dot4(packed, 0x01010101, 0);
-      sum += dppi<0xB1>(sum);
-      sum += dppi<0x4E>(sum);  // 4 lanes = one run of 16
-      if (live[n]) {
-        *(int *)(q0p + qo[n] + lane * 4) = packed;
-        if ((lane & 3) == 0) b0p[(size_t)sb[n] * ACT_BS + (lane >> 2)] = sum;
-        if (lane == 0) d0p[(size_t)sb[n] * dw] = dd;
-      }
+      const float is = rlf(iscale, n);
+      // min(127, round away from zero): the conversion truncates
+      auto q = [&](float x) { const float y = is * x; return (int)fminf(127.f, y + copysignf(0.49999997f, y)); };
+      packed[n] = pack4(q(v[n].x), q(v[n].y), q(v[n].z), q(v[n].w));
+      sum[n] = dot4(packed[n], 0x01010101, 0);
+      if (live[n]) *(int *)(q0p + qo[n] + lane * 4) = packed[n];
     }
+    // 4 lanes = one run of 16: lane l gets the sum of run l / 4 of its superblock
+    int s;
+    if constexpr (N == 4) {
+      const bool o1 = (lane & 1) != 0, o2 = (lane & 2) != 0;
+      const int s0 = (o1 ? sum[1] : sum[0]) + dppi<0xB1>(o1 ? sum[0] : sum[1]), s1 = (o1 ? sum[3] : sum[2]) + dppi<0xB1>(o1 ? sum[2] : sum[3]);
+      s = (o2 ? s1 : s0) + dppi<0x4E>(o2 ? s0 : s1);
+    } else {
+      if constexpr (N == 2) { const bool o1 = (lane & 1) != 0; s = (o1 ? sum[1] : sum[0]) + dppi<0xB1>(o1 ? sum[0] : sum[1]); }
+      else s = sum[0] + dppi<0xB1>(sum[0]);
+      s += dppi<0x4E>(s);
+    }
+    if ((lane & 3) < N && livel) b0p[(size_t)sbl * ACT_BS + (lane >> 2)] = s;
+    if (lane < N && livel) d0p[(size_t)sbl * dw] = dd;
   } else {
+    float a[N];
+#pragma unroll
+    for (int n = 0; n < N; ++n) a[n] = fmaxf(fmaxf(fabsf(v[n].x), fabsf(v[n].y)), fmaxf(fabsf(v[n].z), fabsf(v[n].w)));
+    float am = lane_merge<N>(a, lane);
+    am = fmaxf(am, dppf<0x1B>(dppf<0x141>(am)));  // lane ^ 4: 8 lanes = one block of 32
+    const float dq = am / 127.0f, id = dq != 0.f ? 1.0f / dq : 0.0f;
 #pragma unroll
     for (int n = 0; n < N; ++n) {
-      float amax = fmaxf(fmaxf(fabsf(v[n].x), fabsf(v[n].y)), fmaxf(fabsf(v[n].z), fabsf(v[n].w)));
-      amax = fmaxf(amax, dppf<0xB1>(amax));
-      amax = fmaxf(amax, dppf<0x4E>(amax));
-      amax = fmaxf(amax, dppf<0x141>(amax));  // 8 lanes = one block of 32
-      const float dq = amax / 127.0f, id = dq != 0.f ? 1.0f / dq : 0.0f;
-      const int q0 = (int)round_away(v[n].x * id), q1 = (int)round_away(v[n].y * id), q2 = (int)round_away(v[n].z * id), q3 = (int)round_away(v[n].w * id);
-      if (live[n]) {
-        *(int *)(q0p + qo[n] + lane * 4) = (q0 & 0xff) | ((q1 & 0xff) << 8) | ((q2 & 0xff) << 16) | ((q3 & 0xff) << 24);
-        if ((lane & 7) == 0) d0p[(size_t)sb[n] * dw + (lane >> 3)] = half_bits_to_float(float_to_half_bits(dq));
-      }
+      const float idn = N == 1 ? id : n == 0 ? dppf<0x00>(id) : n == 1 ? dppf<0x55>(id) : n == 2 ? dppf<0xAA>(id) : dppf<0xFF>(id);
+      auto q = [&](float x) { const float y = x * idn; return (int)(y + copysignf(0.49999997f, y)); };
+      if (live[n]) *(int *)(q0p + qo[n] + lane * 4) = pack4(q(v[n].x), q(v[n].y), q(v[n].z), q(v[n].w));
     }
+    if ((lane & 7) < N && livel) d0p[(size_t)sbl * dw + (lane >> 3)] = half_bits_to_float(float_to_half_bits(dq));
   }
 }
 __device__ __forceinline__ void quantize_sb(float4 v, int sb, int c, int mode, char *img, int K, int ncols) {

@@ -388,11 +388,18 @@ static hiphost_u32x2 permlane32_swap(unsigned a, unsigned b) {
   const unsigned ao = exchange(a, lane ^ 32), bo = exchange(b, lane ^ 32);
   return lane >= 32 ? hiphost_u32x2{bo, b} : hiphost_u32x2{a, ao};
 }
+// v_permlane16_swap_b32: the odd rows of 16 lanes of the first operand against the even rows of the second
+static hiphost_u32x2 permlane16_swap(unsigned a, unsigned b) {
+  const int lane = linear_tid() & (WAVE - 1);
+  const unsigned ao = exchange(a, lane ^ 16), bo = exchange(b, lane ^ 16);
+  return (lane & 16) ? hiphost_u32x2{bo, b} : hiphost_u32x2{a, ao};
+}
 }  // namespace hiphost
 #define __builtin_amdgcn_mfma_i32_16x16x64_i8(A, B, C, CBSZ, ABID, BLGP) hiphost::mfma_16x16x64_i8((A), (B), (C))
 #define __builtin_amdgcn_mfma_i32_16x16x32_i8(A, B, C, CBSZ, ABID, BLGP) hiphost::mfma_16x16x32_i8((A), (B), (C))
 #define __builtin_amdgcn_mfma_f32_16x16x32_f16(A, B, C, CBSZ, ABID, BLGP) hiphost::mfma_16x16x32_f16((A), (B), (C))
 #define __builtin_amdgcn_permlane32_swap(A, B, FI, BC) hiphost::permlane32_swap((A), (B))
+#define __builtin_amdgcn_permlane16_swap(A, B, FI, BC) hiphost::permlane16_swap((A), (B))
 // buffer resource: base + byte range; raw_buffer_load returns zeros out of range (as the hardware's bounds check does)
 struct __amdgpu_buffer_rsrc_t { const char *base; unsigned bytes; };
 static inline __amdgpu_buffer_rsrc_t hiphost_make_rsrc(void *p, int bytes) { return __amdgpu_buffer_rsrc_t{(const char *)p, (unsigned)bytes}; }
