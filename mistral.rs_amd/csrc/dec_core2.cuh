@@ -31,6 +31,12 @@
 #include <type_traits>
 #include <utility>
 
+// a uniform value that the kernel does not write, by the scalar unit (a pointer out of the argument block is a vector load otherwise); MRS_KEEP_S: it has arrived (arguments: read with the
+// others and not behind the first branch)
+#ifndef MRS_SLOAD32
+#define MRS_SLOAD32(p) (*(const __attribute__((address_space(4))) uint32_t *)(size_t)(p))
+#define MRS_KEEP_S(x) asm volatile("" ::"s"(x))
+#endif
 #ifndef MRS_WAVE_SYNC
 #define MRS_WAVE_SYNC() __builtin_amdgcn_wave_barrier()
 #endif

@@ -291,6 +291,136 @@ __global__ void __launch_bounds__(NT) dec_gemv_kernel(const GemvArgs a) {
   } else gemv_phase<NCOLS, EPI, TMASK, RING2>(a, smem, red, &ctr, nullptr);
 }
 
+// ---- Two waves per unit: rows of one column into the residual stream whose launch has units for half of a workgroup's waves at most (4096 rows on 256 CUs).
+// stream() gave such a unit to one wave: four waves of eight streamed, a ring of four tiles each, which stood still while they quantized 14336 values of activations; then one wave per SIMD
+// multiplied 14 tiles behind one another.  Here both waves of a unit stream half of its tiles (or the tiles of one of the token's two experts each: PAIR_TOP2), all of them or seven at a time
+// in registers, and the halves' sums meet in LDS: the second wave goes on with its terms from the first's sum, so the order of the sums is the row's.  A wave that requests more than the
+// CU's share of the memory can take is blocked in the issue, and everyone waits for it at the barrier: the tiles are requested a few at a time, between the steps of the quantization, the
+// last of them behind the barrier.  One tile in front of it, two and one between (rows of 13 and 14 tiles per unit), us: Q4_K 4096 x 14336 10.4 (in front all seven 12.2, two 10.7; behind
+// the barrier all but two 11.3); shorter rows two, two and one: Q6_K 3072 x 8192 6.9 (with one in front 7.3).
+// us, stream() / this: Q4_K 4096 x 14336 11.6 / 10.4, 4096 x 11008 9.3 / 7.8, 4096 x 7168 7.1 / 6.3, Q5_K 4096 x 14336 12.2 / 10.8, Q6_K 13.1 / 11.6, 3072 x 8192 7.9 / 6.9, Q8_0 14.2 / 12.4; Q4_K 4096 x 4096 from
+// an image 4.8 / 4.2; two experts of 4096 x 14336 Q4_K 22.4 / 17.7, Q6_K 23.8 / 20.9, Q8_0 25.8 / 22.1, of 2048 x 8192 Q4_K 11.1 / 9.6.
+constexpr int PAIR_RING = 7;  // tiles of a wave (TOP2: twice)
+enum : int { PAIR_F32 = 0, PAIR_IMG = 1, PAIR_TOP2 = 2 };
+template <int TYPE, int R, int SRC>
+__global__ void __launch_bounds__(NT) dec_gemv_pair_kernel(const GemvArgs a) {
+  extern __shared__ __attribute__((aligned(16))) char smem[];
+  __shared__ float hand_s[NW / 2][64];
+  using TL = Tile<TYPE>;
+  constexpr bool TOP2 = SRC == PAIR_TOP2;
+  constexpr int NCI = TOP2 ? 2 : 1, mode = TYPE == T_Q8_0 ? ACT_Q80 : ACT_Q8K;
+  constexpr unsigned tileb = tile_bytes(TYPE);
+  const int tid = tid_opaque(), lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), half = wave >> 2;
+  const int K = a.K, S = K / 256, Cs = (S + 3) / 4, bx = (int)blockIdx.x;
+  const int u0 = bx * a.ubase[0] + min(bx, a.urem[0]), u = u0 + (wave & 3);
+  const bool has = u < u0 + a.ubase[0] + (bx < a.urem[0] ? 1 : 0);
+  const int p = (lane >> 2) & 3, c = lane & 3, row = u * 4 + (lane >> 4), nrows = a.nrows[0];
+  // the rows of activations first
+  const float *x1 = TOP2 ? a.x + a.ldx : a.x;
+  const size_t img_bytes = act_bytes(K, 1);
+  ActRegs<1> xa = act_issue_all<1>(SRC == PAIR_IMG ? a.x_img : (const void *)a.x, SRC == PAIR_IMG ? (unsigned)img_bytes : (unsigned)K * 4u, nullptr, K, wave), xb;
+  if constexpr (TOP2) xb = act_issue_all<1>(x1, (unsigned)K * 4u, nullptr, K, wave);
+  const float res = a.out[min(row, nrows - 1)];
+  const int e = TOP2 ? (int)MRS_SLOAD32(a.expert_sel + half) : 0;
+  const float w0 = TOP2 ? a.acc_scale[0] : a.acc_scale ? *a.acc_scale : 1.0f, w1 = TOP2 ? a.acc_scale[1] : 0.f;
+  // tiles t0 .. t0 + nt - 1 of the unit: both halves of its rows' tiles, or all of the expert's
+  const int nA = (Cs + 1) / 2, t0 = TOP2 || half == 0 ? 0 : nA, nt = !has ? 0 : TOP2 ? Cs : half == 0 ? nA : Cs - nA;
+  const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc((void *)a.m[0].base, (short)0, (int)a.m[0].bytes, 0x00020000);
+  const unsigned base = ((unsigned)(e * ((nrows + 3) / 4) + u) * (unsigned)Cs + (unsigned)t0) * tileb;
+  constexpr unsigned DEAD = 0xF0000000u;  // beyond every tensor: zeros, no traffic, and every wave's count of requests stays the same
+  typename TL::Raw ring[R];
+  auto request = [&](int i) { ring[i % R] = TL::load(rs, i < nt ? base + (unsigned)i * tileb : DEAD, lane); };
+  auto requests = [&](int from, int to) {
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int i = from; i < to; ++i) request(i);
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  auto quantize = [&](const ActRegs<1> &x, int col, int j0) {  // superblocks wave + 8 j of the column, j = j0 .. j0 + 3
+    if (wave + 8 * j0 >= S) return;  // wave-uniform
+    float4 v[4]; int sb[4]; bool live[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) { sb[i] = wave + 8 * (j0 + i); live[i] = j0 + i < NPX && sb[i] < S; v[i] = as_f4(x.xv[0][j0 + i < NPX ? j0 + i : 0]); }
+    quantize_multi<4>(v, sb, live, col, mode, smem, K, NCI);
+  };
+  constexpr int P0 = R == PAIR_RING ? 1 : 2, P1 = R < P0 + 2 ? R : P0 + 2, P2 = R < P1 + 1 ? R : P1 + 1, P3 = R < 6 ? R : 6, P4 = R;
+  MRS_TL2(a, 0);
+  __syncthreads();  // every wave's rows are requested
+  requests(0, P0);
+  MRS_TL2(a, 1);
+  if constexpr (SRC == PAIR_IMG) {
+    requests(P0, R);
+    img_finish_all<1>(smem, xa, a.x_img, img_bytes, wave);
+  } else {
+    quantize(xa, 0, 0);
+    requests(P0, P1);
+    quantize(xa, 0, 4);
+    requests(P1, P2);
+    if constexpr (TOP2) {
+      quantize(xb, 1, 0);
+      requests(P2, P3);
+      quantize(xb, 1, 4);
+      requests(P3, P4);
+    }
+  }
+  MRS_TL2(a, 2);
+  __syncthreads();
+  if constexpr (SRC != PAIR_IMG) requests(TOP2 ? P4 : P2, R);
+  MRS_TL2(a, 3);
+  const Act act = act_view(smem, K, NCI, mode);
+  const int qo = p * act.CQ + c * 64;
+  auto term = [&](int i) -> float {  // T of the lane's superblock in tile t0 + i
+    float T[1];
+    const int ts = min(t0 + i, Cs - 1);
+    TL::template term<1>(ring[i % R], p * Cs + ts, qo + ts * 256, c, act, TOP2 ? half : 0, T);
+    return T[0];
+  };
+  auto live = [&](int i) { return i < nt && p * Cs + t0 + i < S; };
+  auto row_sum = [&](float acc) {  // ((c0 + c1) + c2) + c3 in the chunk-3 quad of every row
+    float s = dppf<0x124>(acc) + acc;
+    s = dppf<0x124>(s) + acc;
+    return dppf<0x124>(s) + acc;
+  };
+  const bool own = has && (lane & 15) == owner_off(Geo{}) && row < nrows;
+  float acc = 0.f;
+  if constexpr (TOP2) {
+#pragma unroll
+    for (int i = 0; i < 2 * R; ++i) {
+      const float T = term(i);
+      acc = i == 0 ? (live(0) ? T : 0.f) : live(i) ? acc + T : acc;
+      if (i < R) request(i + R);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    const float tot = row_sum(acc);
+    if (half == 0) hand_s[wave & 3][lane] = tot;
+    __syncthreads();
+    if (half == 1 && own) {
+      const float h1 = res * a.resid_scale + hand_s[wave & 3][lane] * w0;
+      a.out[row] = h1 * 1.0f + tot * w1;
+    }
+  } else {
+    float T[R];
+#pragma unroll
+    for (int i = 0; i < R; ++i) T[i] = term(i);
+    auto chain = [&](bool first) {
+#pragma unroll
+      for (int i = 0; i < R; ++i) acc = first && i == 0 ? (live(0) ? T[0] : 0.f) : live(i) ? acc + T[i] : acc;
+    };
+    if (half == 0) { chain(true); hand_s[wave][lane] = acc; }
+    __syncthreads();
+    if (half == 1) {
+      acc = hand_s[wave & 3][lane];
+      chain(false);
+      const float tot = row_sum(acc);
+      if (own) a.out[row] = res * a.resid_scale + tot * w0;
+    }
+  }
+  MRS_TL2(a, 14);
+}
+// tiles per unit that it takes: an image's rows of 3 and 4 (a wave then has two), f32 rows of 7 .. 14 (4 .. 7 in registers; longer rows do not fit the prologue's seven pieces either), two
+// experts' rows of 8 .. 14.  Other counts and launches with more units per workgroup are stream()'s
+__host__ inline bool pair_ring_ok(int src, int Cs) { return src == PAIR_IMG ? Cs == 3 || Cs == 4 : src == PAIR_F32 ? Cs >= 7 && Cs <= 2 * PAIR_RING : Cs > PAIR_RING && Cs <= 2 * PAIR_RING; }
+int pair_launch(int type, int src, int grid, size_t lds, const GemvArgs &a, hipStream_t s);
 
 // launch one GEMV phase with NCOLS activation columns (ext_dec_gemv.hip, one definition per NCOLS)
 template <int NCOLS> int gemv_launch(int epi, int tmask, bool ring2, int grid, size_t lds, const GemvArgs &a, hipStream_t s);

@@ -18,12 +18,6 @@
 
 #include "dec_gemv.cuh"
 
-// a uniform value that the kernel does not write, by the scalar unit (a pointer out of the argument block is a vector load otherwise); MRS_KEEP_S: it has arrived (arguments: read with the
-// others and not behind the first branch)
-#ifndef MRS_SLOAD32
-#define MRS_SLOAD32(p) (*(const __attribute__((address_space(4))) uint32_t *)(size_t)(p))
-#define MRS_KEEP_S(x) asm volatile("" ::"s"(x))
-#endif
 #ifndef MRS_WAIT_VMCNT0
 #define MRS_WAIT_VMCNT0() asm volatile("s_waitcnt vmcnt(0)" ::: "memory")
 #endif
@@ -735,6 +729,11 @@ template <int EPI> struct Launch {
     if (a.upe < 1) a.upe = 1;
     size_t lds = (act_bytes(a.K, NCI) + 15) & ~(size_t)15;
     if (lds > LDS_IMG_MAX) return -2;
+    if constexpr (NCOLS == 1 && (EPI == EPI_RESID || EPI == EPI_RESID2)) {  // units for half of the waves: two waves per unit (dec_gemv_pair_kernel)
+      const int src = EPI == EPI_RESID2 ? PAIR_TOP2 : a.x_img ? PAIR_IMG : PAIR_F32;
+      const bool plain = EPI == EPI_RESID2 ? !a.x_img : !a.expert_sel;
+      if (plain && !a.norm_w && a.ubase[0] + (a.urem[0] > 0) <= NW / 2 && pair_ring_ok(src, g.Cs)) return pair_launch(a.m[0].type, src, grid, lds, a, s);
+    }
     int tmask = 0;
     for (int i = 0; i < (EPI == EPI_QKV ? 3 : 1); ++i) tmask |= tmask_of(a.m[i].type);
     // ring depth: 2 tiles per wave when every wave of a workgroup streams (>= 8 units per workgroup), the format's 4 otherwise (dec_core2.cuh stream() RING2)

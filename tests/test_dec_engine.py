@@ -82,6 +82,31 @@ def test_proj_gpu(oracle, dev, tname, n, k, b, mode):
     check_proj(oracle, GpuBackend(dev), tname, n, k, b, mode, seed=n + k)
 
 
+# Launches with units for at most half of a workgroup's waves: two waves per unit, each with half of its tiles (7 .. 14 tiles of an f32 row, three and four of an image; the other counts take
+# the other kernel), rows that are not a multiple of four, a short last chunk, workgroups of one and of two units
+PAIRS = [("Q4_K", 6, 6656, None), ("Q4_K", 9, 14336, None), ("Q4_K", 4, 14080, None), ("Q4_K", 3, 9216, None), ("Q4_K", 5, 6144, None), ("Q5_K", 7, 11008, None), ("Q6_K", 5, 13824, None), ("Q6_K", 4, 8192, None),
+         ("Q6_K", 6, 10240, None), ("Q8_0", 6, 9728, None), ("Q8_0", 3, 14336, None), ("Q4_K", 13, 4096, "img"), ("Q8_0", 10, 3072, "img"), ("Q6_K", 7, 2816, "img"), ("Q5_K", 5, 3840, "img"),
+         ("Q4_K", 1030, 2304, "img")]
+
+
+def check_pairs(O, be, tname, n, k, img):
+    if img:
+        check_image_proj(O, be, tname, n, k, 1, False)
+    else:
+        check_proj(O, be, tname, n, k, 1, 1, seed=n + k)
+
+
+@pytest.mark.parametrize("tname,n,k,img", PAIRS)
+def test_two_waves_per_unit_host_emulation(oracle, tname, n, k, img):
+    check_pairs(oracle, HostBackend(), tname, n, k, img)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("tname,n,k,img", PAIRS + [("Q5_K", 4096, 11008, None), ("Q8_0", 4095, 14336, None), ("Q6_K", 3072, 8192, None), ("Q4_K", 2050, 4096, "img")])
+def test_two_waves_per_unit_gpu(oracle, dev, tname, n, k, img):
+    check_pairs(oracle, GpuBackend(dev), tname, n, k, img)
+
+
 def check_norm_proj(O, be, tname, n, k, b):
     """RMSNorm fused into the prologue (candle's x / sqrt(mean + eps) * w): bit-equal to the engine-order restatement (same expression, the
     kernel's summation tree); against candle's in-order sum a 1-ulp difference of the norm can move single quants by one step, so that bar
@@ -644,7 +669,8 @@ def check_proj_top2(O, be, tname, n, k, experts, sels):
     np.testing.assert_array_equal(one.numpy(), two.numpy())
 
 
-@pytest.mark.parametrize("tname,n,k,experts,sels", [("Q4_K", 80, 512, 4, [3, 1]), ("Q6_K", 32, 768, 3, [0, 2]), ("Q4_K", 16, 1024, 2, [1, 1])])
+@pytest.mark.parametrize("tname,n,k,experts,sels", [("Q4_K", 80, 512, 4, [3, 1]), ("Q6_K", 32, 768, 3, [0, 2]), ("Q4_K", 16, 1024, 2, [1, 1]), ("Q4_K", 8, 8192, 2, [1, 0]),
+                                                          ("Q6_K", 4, 14336, 2, [0, 1]), ("Q8_0", 4, 14336, 2, [1, 1]), ("Q5_K", 12, 11008, 2, [1, 0])])
 def test_proj_top2_host_emulation(oracle, tname, n, k, experts, sels):
     check_proj_top2(oracle, HostBackend(), tname, n, k, experts, sels)
 
