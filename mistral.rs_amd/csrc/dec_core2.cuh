@@ -177,22 +177,22 @@ __device__ __forceinline__ float max_rows(float v) {  // the largest of a lane's
 __device__ __forceinline__ int pack4(int q0, int q1, int q2, int q3) {
   return (int)(__builtin_amdgcn_perm((unsigned)q1, (unsigned)q0, 0x0c0c0400u) | __builtin_amdgcn_perm((unsigned)q3, (unsigned)q2, 0x04000c0cu));
 }
-template <int N>
-__device__ __forceinline__ void quantize_multi(const float4 (&v)[N], const int (&sb)[N], const bool (&live)[N], int c, int mode, char *img, int K, int ncols) {
+template <int N>  // superblock n -> column col[n] of the image
+__device__ __forceinline__ void quantize_multi(const float4 (&v)[N], const int (&sb)[N], const bool (&live)[N], const int (&col)[N], int mode, char *img, int K, int ncols) {
   static_assert(N == 1 || N == 2 || N == 4, "a superblock per lane of N");
   const int lane = lane_opaque(), S = K / 256, dw = act_dw(mode), Cs = (S + 3) / 4, CQ = act_cq(K), Sp = act_sp(K);
-  char *q0p = img + (size_t)c * 4 * CQ;
-  float *d0p = (float *)(img + (size_t)ncols * 4 * CQ) + (size_t)c * Sp * dw;
-  int *b0p = (int *)(img + (size_t)ncols * 4 * CQ + (size_t)ncols * Sp * dw * 4) + (size_t)c * Sp * ACT_BS;
+  char *q0p = img;
+  float *d0p = (float *)(img + (size_t)ncols * 4 * CQ);
+  int *b0p = (int *)(img + (size_t)ncols * 4 * CQ + (size_t)ncols * Sp * dw * 4);
   int qo[N];
 #pragma unroll
-  for (int n = 0; n < N; ++n) { const int sbn = live[n] ? sb[n] : 0, p = chunk_of(sbn, Cs); qo[n] = p * CQ + (sbn - p * Cs) * 256; }
+  for (int n = 0; n < N; ++n) { const int sbn = live[n] ? sb[n] : 0, p = chunk_of(sbn, Cs); qo[n] = (col[n] * 4 + p) * CQ + (sbn - p * Cs) * 256; }
   // the lane's superblock: n = lane % N
   const int mine = lane & (N - 1);
-  int sbl = sb[0];
+  int sbl = col[0] * Sp + sb[0];
   bool livel = live[0];
 #pragma unroll
-  for (int n = 1; n < N; ++n) { sbl = mine == n ? sb[n] : sbl; livel = mine == n ? live[n] : livel; }
+  for (int n = 1; n < N; ++n) { sbl = mine == n ? col[n] * Sp + sb[n] : sbl; livel = mine == n ? live[n] : livel; }
   if (mode == ACT_Q8K) {
     float hi4[N], lo4[N], a[N];
 #pragma unroll
@@ -268,6 +268,13 @@ __device__ __forceinline__ void quantize_multi(const float4 (&v)[N], const int (
     if ((lane & 7) < N && livel) d0p[(size_t)sbl * dw + (lane >> 3)] = half_bits_to_float(float_to_half_bits(dq));
   }
 }
+template <int N>
+__device__ __forceinline__ void quantize_multi(const float4 (&v)[N], const int (&sb)[N], const bool (&live)[N], int c, int mode, char *img, int K, int ncols) {
+  int col[N];
+#pragma unroll
+  for (int n = 0; n < N; ++n) col[n] = c;
+  quantize_multi<N>(v, sb, live, col, mode, img, K, ncols);
+}
 __device__ __forceinline__ void quantize_sb(float4 v, int sb, int c, int mode, char *img, int K, int ncols) {
   const float4 va[1] = {v}; const int sa[1] = {sb}; const bool la[1] = {true};
   quantize_multi<1>(va, sa, la, c, mode, img, K, ncols);
@@ -288,6 +295,7 @@ __device__ __forceinline__ float4 norm4(float4 v, float4 w4, float nm, float inv
 // and the other columns of a batch take plain loads.
 constexpr int NPX = 7, NPW = 4;
 template <int VW> struct ActRegs { v4u xv[VW][NPX]; v4u wv[VW][NPW]; };
+template <> struct ActRegs<0> {};
 // xbytes: bytes of the row (K * 4), or of a pre-quantized image when the same registers carry one (img_finish_all) -- ONE producer of the register set for both
 // cases: a struct assigned from two different calls under a run-time branch is demoted to scratch memory by hipcc (round 4's 48-byte frame)
 template <int VW> __device__ __forceinline__ ActRegs<VW> act_issue_all(const void *x, unsigned xbytes, const float *nw, int K, int q) {
@@ -385,6 +393,27 @@ __device__ __forceinline__ void act_quantize_all(char *img, const float *red, co
       }
     }
   }
+}
+// two columns of up to 4096 values behind a norm: a wave's two superblocks of each in one quantizer call
+__device__ __forceinline__ void act_quantize_two(char *img, const float *red, const ActRegs<1> &pre, const ActRegs<1> &pre1, const float *__restrict__ nw, float eps, int K, int mode, int q) {
+  float4 v[4]; int sb[4], col[4]; bool live[4];
+#pragma unroll
+  for (int c = 0; c < 2; ++c) {
+    float nm = 1.0f, inv = 1.0f;
+    if (nw) {
+      const float *r = red + c * 8;
+      nm = sqrtf((((r[0] + r[1]) + (r[2] + r[3])) + ((r[4] + r[5]) + (r[6] + r[7]))) / (float)K + eps);
+      inv = 1.0f / nm;
+    }
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      const int n = 2 * c + j;
+      sb[n] = q + 8 * j; live[n] = sb[n] * 256 < K; col[n] = c;
+      const float4 x = as_f4((c ? pre1 : pre).xv[0][j]);
+      v[n] = nw ? norm4(x, as_f4(pre.wv[0][j]), nm, inv) : x;
+    }
+  }
+  quantize_multi<4>(v, sb, live, col, mode, img, K, 2);
 }
 // all 8 waves of a workgroup as participants, both halves with the barrier in between (the prompt path's quantizer kernel)
 template <int NCOLS>
@@ -617,7 +646,7 @@ template <int TYPE, int NCOLS, int C0> struct TermCols {
 //     share: a wave that requests more is blocked in the issue and cannot do anything else);
 //   * an out-of-range ("dead") buffer load still costs its 16 cycles in the CU's one texture addresser: a pass of dead requests of 8 waves is ~0.5 us;
 //   * nothing can be multiplied before the activation prologue is done, and the prologue's workgroup barrier waits for the SLOWEST wave's blocked issue.
-// Hence: (1) the activation row is requested first, ONE tile per wave next, the sum of squares and its barrier run while those fly, then the rest of the ring, then
+// Hence: (1) the activation row is requested first, ONE tile per wave next, the sum of squares and its barrier run while those fly, then a second tile, then
 // the quantization and the publishing barrier; (2) the ring is NS = 4 tiles; (3) no dead requests in the common case: passes whose NS re-requests are all live run in
 // a loop, the last tiles are computed by straight-line tails that request nothing (or only the r < NS live ones that are left + NS - r dead).
 struct Job {
@@ -745,9 +774,14 @@ __device__ __forceinline__ void stream(const Job &jb, int K, int ncols_img, int 
   MRS_TL2(jb, 1);
   // (publishing the image BEFORE the rest of the ring is requested -- tried for the short launches, round 5 -- made qkv 0.9 us slower in the graph: the requests that
   // would have overlapped the quantization arithmetic then queue behind it)
+  // two tiles in front of the quantization, the others behind it: a wave that requests all of its ring is blocked in the issue while the others wait for its part of the image.  q / k / v of
+  // 6144 x 4096, us, four in front / two: Q8_0 9.4 / 8.8, Q4_K 7.9 / 7.9, two columns 12.5 / 11.6, gate / up of two columns 19.5 / 18.9 (one in front 8.6, 8.25, 12.0, 19.6)
+  constexpr int RA = NS < 2 ? NS : 2;
 #pragma unroll
-  for (int i = 1; i < NS; ++i) issue(ring[i], meta[i], auxv[i]);
+  for (int i = 1; i < RA; ++i) issue(ring[i], meta[i], auxv[i]);
   stage(2, wave);  // normalise + quantize (or copy the image) into LDS
+#pragma unroll
+  for (int i = RA; i < NS; ++i) issue(ring[i], meta[i], auxv[i]);
   MRS_TL2(jb, 2);
   __syncthreads();  // B
   MRS_TL2(jb, 3);

@@ -103,16 +103,34 @@ __device__ __forceinline__ void gemv_phase(const GemvArgs &a, char *smem, float 
   // normalised / quantized.  ONE producer of the register set for both cases (act_issue_all): a struct assigned from two different calls under a run-time branch is
   // demoted to scratch memory by hipcc.
   ActRegs<1> pre;
+  // two columns: the second's row in registers too, requested with the first's (plain loads of it in the sum of squares and in the quantization were two more round trips; us of two columns
+  // behind a norm, so / this, the rings as they were / this with the ring's last tiles behind the quantization: q / k / v of 6144 x 4096 Q4_K 13.0 / 11.9 / 10.9, Q8_0 14.1 / 11.4 in all, gate / up of 28672 x 4096
+  // Q4_K 20.4 / 18.7 / 18.1, Q8_0 26.6 / 24.9 in all)
+  constexpr bool TWO = NCOLS == 2;
+  ActRegs<TWO ? 1 : 0> pre1;
   const size_t img_bytes = act_bytes(K, NCI);
   const bool from_img = a.x_img != nullptr;
   const void *xsrc = from_img ? a.x_img : (const void *)a.x;
   const unsigned xbytes = from_img ? (unsigned)img_bytes : (unsigned)K * 4u;
   const float *nw_eff = from_img ? nullptr : a.norm_w;
   auto stage = [&](int st, int q) {
-    if (st == 0) pre = act_issue_all<1>(xsrc, xbytes, nw_eff, K, q);
-    else if (st == 1) act_sumsq_all<NCI, 1>(red, pre, a.x, a.ldx, nw_eff, K, q);  // (an image has no norm weight: nothing to do)
-    else if (from_img) img_finish_all<1>(smem, pre, a.x_img, img_bytes, q);
-    else act_quantize_all<NCI, 1>(smem, red, pre, a.x, a.ldx, a.norm_w, a.eps, K, mode, q);
+    if (st == 0) {
+      pre = act_issue_all<1>(xsrc, xbytes, nw_eff, K, q);
+      if constexpr (TWO) pre1 = act_issue_all<1>(a.x + a.ldx, from_img ? 0u : (unsigned)K * 4u, nullptr, K, q);
+    } else if (st == 1) {  // (an image has no norm weight: nothing to do)
+      act_sumsq_all<TWO ? 1 : NCI, 1>(red, pre, a.x, a.ldx, nw_eff, K, q);
+      if constexpr (TWO) act_sumsq_all<1, 1>(red + 8, pre1, a.x + a.ldx, a.ldx, nw_eff, K, q);
+    } else if (from_img) img_finish_all<1>(smem, pre, a.x_img, img_bytes, q);
+    else if (TWO && K <= 4096) {
+      if constexpr (TWO) act_quantize_two(smem, red, pre, pre1, a.norm_w, a.eps, K, mode, q);
+    } else {
+      act_quantize_all<TWO ? 1 : NCI, 1>(smem, red, pre, a.x, a.ldx, a.norm_w, a.eps, K, mode, q, 0, NCI);
+      if constexpr (TWO) {
+#pragma unroll
+        for (int j = 0; j < NPW; ++j) pre1.wv[0][j] = pre.wv[0][j];
+        act_quantize_all<1, 1>(smem, red + 8, pre1, a.x + a.ldx, a.ldx, a.norm_w, a.eps, K, mode, q, 1, NCI);
+      }
+    }
   };
   const bool sbar = nw_eff != nullptr;
   constexpr bool AUX_RING = NCOLS == 1;  // epilogue operands travel with the tiles (latency-bound small batches) or are loaded by the epilogue
@@ -194,7 +212,7 @@ __device__ __forceinline__ void gemv_phase(const GemvArgs &a, char *smem, float 
     // positions and KV slots: a handful of scalars, loaded before anything else; the RoPE factors travel with the record (owner lanes of the pair's two rows)
     int posv[NCOLS], slotv[NCOLS];  // slots are block * block_size + offset of a cache that fits 32-bit indexing per layer (checked by the launcher)
 #pragma unroll
-    for (int c = 0; c < NCOLS; ++c) { posv[c] = a.positions[c]; slotv[c] = mi == 0 ? 0 : (int)a.slot_mapping[c]; }
+    for (int c = 0; c < NCOLS; ++c) { posv[c] = (int)MRS_SLOAD32(a.positions + c); slotv[c] = mi == 0 ? 0 : (int)MRS_SLOAD32(a.slot_mapping + c); }
     auto load_aux = [&](int row) {  // RoPE factors of the row's pair for every column; identity for v and unrotated dims (x*1 - y*0 = x exactly).  Unconditional loads.
       AuxV<NCOLS> v;
       const int pair_i = (row & (a.head_dim - 1)) >> 1;
@@ -244,18 +262,20 @@ __device__ __forceinline__ void gemv_phase(const GemvArgs &a, char *smem, float 
           } else {
             const int slot = slotv[c];
             if (slot >= 0) {
+              // wave-uniform: the page (64 bits, scalar); a lane's place in it fits 32 bits
               const unsigned blk = (unsigned)slot >> a.bs_shift, off = (unsigned)slot & (unsigned)(a.block_size - 1);
-              uint16_t *kc = (uint16_t *)a.k_cache, *vc = (uint16_t *)a.v_cache;
+              const size_t page = (size_t)blk * ((size_t)a.num_kv_heads * (unsigned)a.head_dim * (unsigned)a.block_size);
+              uint16_t *kc = (uint16_t *)a.k_cache + page, *vc = (uint16_t *)a.v_cache + page;
               const uint16_t xb = a.kv_f16 ? float_to_half_bits(x) : float_to_bf16_bits(x), yb = a.kv_f16 ? float_to_half_bits(y) : float_to_bf16_bits(y);
               if (mi == 1) {
-                const int X = a.cache_x;
-                const size_t hb = ((size_t)blk * a.num_kv_heads + head) * (size_t)(a.head_dim >> a.x_shift);
-                if (wr0) kc[(hb + ((unsigned)d0 >> a.x_shift)) * a.block_size * X + off * X + ((unsigned)d0 & (unsigned)(X - 1))] = xb;
-                if (wr1) kc[(hb + ((unsigned)d1 >> a.x_shift)) * a.block_size * X + off * X + ((unsigned)d1 & (unsigned)(X - 1))] = yb;
+                const unsigned X = (unsigned)a.cache_x, hb = (unsigned)head << (a.hd_shift - a.x_shift);
+                auto at = [&](int d) { return (((hb + ((unsigned)d >> a.x_shift)) << a.bs_shift) + off) * X + ((unsigned)d & (X - 1)); };
+                if (wr0) kc[at(d0)] = xb;
+                if (wr1) kc[at(d1)] = yb;
               } else {
-                const size_t o = (((size_t)blk * a.num_kv_heads + head) * a.head_dim + dd) * a.block_size + off;
+                const unsigned o = ((((unsigned)head << a.hd_shift) + (unsigned)dd) << a.bs_shift) + off;
                 if (wr0) vc[o] = xb;
-                if (wr1) vc[o + a.block_size] = yb;
+                if (wr1) vc[o + (unsigned)a.block_size] = yb;
               }
             }
           }

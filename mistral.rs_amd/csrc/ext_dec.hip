@@ -10,6 +10,7 @@
 // Every GEMV phase is the same kernel body: request the activation vector, request the first weight records, run the activation prologue (norm + quantize),
 // stream the workgroup's units, apply the phase's epilogue per finished row.  Arithmetic and f32 order: header of dec_core2.cuh.
 #include "dec_attn.cuh"
+#include <limits.h>
 #include <stdio.h>
 #include <stdlib.h>
 #include <math.h>
@@ -699,17 +700,41 @@ template <int EPI> struct Launch {
     const int upr = g.R * a.rgpu;  // rows per unit
     int grid = 0;
     if (EPI == EPI_QKV) {
-      // workgroups per tensor in proportion to its bytes (a workgroup streams one tensor), at least one each
-      double bytes[3]; double tot = 0; int want = 0;
+      // Workgroups per tensor (a workgroup streams one).  A unit is a wave's, a CU has four SIMDs: five to eight units of a workgroup take as long as eight, four as long as one.  So: the lowest
+      // cost C = (units of a SIMD) x (bytes of a tile) that all tensors can be held to, then fewer units per SIMD for the values and the keys (which write pages besides) where that fits,
+      // and what is left to the fullest workgroups.  Larger launches, of more than eight units per workgroup, wait for the memory: workgroups in proportion to a tensor's bytes.  q / k / v of 6144 x 4096, us, workgroups in proportion to the bytes / this (128, 64, 64): Q4_K 7.15 / 7.0, with Q6_K values 8.7 / 8.15,
+      // Q8_0 8.65 / 8.55, two columns 10.5 / 9.7, 11.4 / 10.6, 11.0 / 10.2.
+      int want = 0, tb[3], per[3], wgs[3];
       for (int i = 0; i < 3; ++i) {
         if (a.nrows[i] % upr) return -3;
         a.units[i] = a.nrows[i] / upr;
-        bytes[i] = (double)a.units[i] * a.rgpu * g.TPC * (double)rec_bytes(a.m[i].type, g); tot += bytes[i]; want += a.units[i];
+        tb[i] = (int)rec_bytes(a.m[i].type, g); want += a.units[i];
       }
-      const int G = want < 256 ? want : 256;
-      int wgs[3], used = 0;
-      for (int i = 0; i < 3; ++i) { wgs[i] = std::max(1, std::min(a.units[i], (int)(G * bytes[i] / tot + 0.5))); used += wgs[i]; }
-      while (used > G) { int big = 0; for (int i = 1; i < 3; ++i) if (wgs[i] > wgs[big]) big = i; if (wgs[big] <= 1) break; --wgs[big]; --used; }
+      if (want <= 256) {
+        for (int i = 0; i < 3; ++i) wgs[i] = a.units[i];
+      } else if (want > 8 * 256) {
+        double tot = 0;
+        int used = 0;
+        for (int i = 0; i < 3; ++i) tot += (double)a.units[i] * tb[i];
+        for (int i = 0; i < 3; ++i) { wgs[i] = std::max(1, std::min(a.units[i], (int)(256 * ((double)a.units[i] * tb[i] / tot) + 0.5))); used += wgs[i]; }
+        while (used > 256) { int big = 0; for (int i = 1; i < 3; ++i) if (wgs[i] > wgs[big]) big = i; --wgs[big]; --used; }
+      } else {
+        auto need = [&](int i, int n) { return (a.units[i] + 4 * n - 1) / (4 * n); };  // workgroups of tensor i with n units per SIMD
+        auto used = [&] { return wgs[0] + wgs[1] + wgs[2]; };
+        for (int C = std::max(tb[0], std::max(tb[1], tb[2]));;) {
+          int next = INT_MAX;
+          for (int i = 0; i < 3; ++i) { per[i] = C / tb[i]; wgs[i] = need(i, per[i]); next = std::min(next, (per[i] + 1) * tb[i]); }
+          if (used() <= 256) break;
+          C = next;
+        }
+        for (int i = 2; i >= 0; --i)
+          while (per[i] > 1 && used() - wgs[i] + need(i, per[i] - 1) <= 256) wgs[i] = need(i, --per[i]);
+        while (used() < 256) {
+          int full = 0;
+          for (int i = 1; i < 3; ++i) if ((long long)a.units[i] * tb[i] * wgs[full] > (long long)a.units[full] * tb[full] * wgs[i]) full = i;
+          ++wgs[full];
+        }
+      }
       a.wg0[0] = 0; for (int i = 0; i < 3; ++i) a.wg0[i + 1] = a.wg0[i] + wgs[i];
       grid = a.wg0[3];
     } else {

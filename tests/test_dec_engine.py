@@ -240,6 +240,22 @@ def test_qkv_gpu(oracle, dev, tq, tv, heads, kvh, hd, k, b, kvd):
     check_qkv(oracle, GpuBackend(dev), tq, tv, heads, kvh, hd, k, b, kvd)
 
 
+# two columns from registers (up to 4096 values in one quantizer call, longer rows column by column), and workgroups per tensor by the units of a SIMD (more than 256 units, at most 8 x 256) or by bytes
+QKV_SPLITS = [("Q4_K", "Q6_K", 8, 1, 128, 256, 1, 1), ("Q8_0", "Q8_0", 9, 1, 128, 256, 2, 0), ("Q4_K", "Q6_K", 2, 1, 64, 4352, 2, 1), ("Q8_0", "Q8_0", 2, 1, 64, 4096, 2, 1),
+              ("Q5_K", "Q6_K", 2, 1, 64, 3840, 2, 0)]
+
+
+@pytest.mark.parametrize("tq,tv,heads,kvh,hd,k,b,kvd", QKV_SPLITS)
+def test_qkv_columns_and_splits_host_emulation(oracle, tq, tv, heads, kvh, hd, k, b, kvd):
+    check_qkv(oracle, HostBackend(), tq, tv, heads, kvh, hd, k, b, kvd)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("tq,tv,heads,kvh,hd,k,b,kvd", QKV_SPLITS + [("Q4_K", "Q6_K", 64, 8, 128, 512, 1, 1), ("Q4_K", "Q4_K", 48, 8, 128, 512, 2, 0), ("Q6_K", "Q6_K", 63, 1, 128, 256, 1, 1)])
+def test_qkv_columns_and_splits_gpu(oracle, dev, tq, tv, heads, kvh, hd, k, b, kvd):
+    check_qkv(oracle, GpuBackend(dev), tq, tv, heads, kvh, hd, k, b, kvd)
+
+
 ACT_IMG = [C.c_void_p, C.c_int, C.c_void_p, C.c_float, C.c_int, C.c_int, C.c_int, C.c_void_p, C.c_void_p]
 PROJ_IMG_ = [C.POINTER(Mat), C.c_int, C.c_void_p, C.c_void_p, C.c_int, C.c_int, C.c_float, C.c_int, C.c_void_p]
 GLU_IMG = [C.POINTER(Mat), C.POINTER(Mat), C.c_int, C.c_void_p, C.c_int, C.c_void_p, C.c_int, C.c_int, C.c_void_p]
