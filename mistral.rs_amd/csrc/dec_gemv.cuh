@@ -311,24 +311,26 @@ __global__ void __launch_bounds__(NT) dec_gemv_kernel(const GemvArgs a) {
   } else gemv_phase<NCOLS, EPI, TMASK, RING2>(a, smem, red, &ctr, nullptr);
 }
 
-// ---- Two waves per unit: rows of one column into the residual stream whose launch has units for half of a workgroup's waves at most (4096 rows on 256 CUs).
+// ---- Two waves per unit: rows of one column (or two, from an image) into the residual stream whose launch has units for half of a workgroup's waves at most (4096 rows on 256 CUs).
 // stream() gave such a unit to one wave: four waves of eight streamed, a ring of four tiles each, which stood still while they quantized 14336 values of activations; then one wave per SIMD
 // multiplied 14 tiles behind one another.  Here both waves of a unit stream half of its tiles (or the tiles of one of the token's two experts each: PAIR_TOP2), all of them or seven at a time
 // in registers, and the halves' sums meet in LDS: the second wave goes on with its terms from the first's sum, so the order of the sums is the row's.  A wave that requests more than the
 // CU's share of the memory can take is blocked in the issue, and everyone waits for it at the barrier: the tiles are requested a few at a time, between the steps of the quantization, the
-// last of them behind the barrier.  One tile in front of it, two and one between (rows of 13 and 14 tiles per unit), us: Q4_K 4096 x 14336 10.4 (in front all seven 12.2, two 10.7; behind
+// last of them behind the barrier, one in front of each product.  One tile in front of it, two and one between (rows of 13 and 14 tiles per unit), us: Q4_K 4096 x 14336 10.4 (in front all seven 12.2, two 10.7; behind
 // the barrier all but two 11.3); shorter rows two, two and one: Q6_K 3072 x 8192 6.9 (with one in front 7.3).
-// us, stream() / this: Q4_K 4096 x 14336 11.6 / 10.4, 4096 x 11008 9.3 / 7.8, 4096 x 7168 7.1 / 6.3, Q5_K 4096 x 14336 12.2 / 10.8, Q6_K 13.1 / 11.6, 3072 x 8192 7.9 / 6.9, Q8_0 14.2 / 12.4; Q4_K 4096 x 4096 from
-// an image 4.8 / 4.2; two experts of 4096 x 14336 Q4_K 22.4 / 17.7, Q6_K 23.8 / 20.9, Q8_0 25.8 / 22.1, of 2048 x 8192 Q4_K 11.1 / 9.6.
+// us, stream() / this: Q4_K 4096 x 14336 11.6 / 10.2, 4096 x 11008 9.3 / 7.8, 4096 x 7168 7.1 / 6.3, Q5_K 4096 x 14336 12.2 / 10.8, Q6_K 13.1 / 11.3, 3072 x 8192 7.9 / 6.9, Q8_0 14.2 / 12.3; Q4_K 4096 x 4096 from
+// an image 4.8 / 4.1; two columns from an image Q4_K 4096 x 4096 5.95 / 4.55, 4096 x 14336 11.5 / 10.8, 4096 x 11008 9.8 / 7.95, Q6_K 4096 x 14336 13.0 / 11.2, 3072 x 8192 8.8 / 6.9, Q8_0 4096 x 14336 14.1 / 12.5 (all of the
+// image's tiles in front of the barrier 12.1, 9.5, 14.4, 8.0, 14.6); two experts of 4096 x 14336 Q4_K 22.4 / 17.7, Q6_K 23.8 / 20.9, Q8_0 25.8 / 22.1, of 2048 x 8192 Q4_K 11.1 / 9.6.
 constexpr int PAIR_RING = 7;  // tiles of a wave (TOP2: twice)
 enum : int { PAIR_F32 = 0, PAIR_IMG = 1, PAIR_TOP2 = 2 };
-template <int TYPE, int R, int SRC>
+template <int TYPE, int R, int SRC, int NC = 1>  // NC columns: 2 from an image
 __global__ void __launch_bounds__(NT) dec_gemv_pair_kernel(const GemvArgs a) {
   extern __shared__ __attribute__((aligned(16))) char smem[];
-  __shared__ float hand_s[NW / 2][64];
+  __shared__ float hand_s[NW / 2][NC][64];
   using TL = Tile<TYPE>;
   constexpr bool TOP2 = SRC == PAIR_TOP2;
-  constexpr int NCI = TOP2 ? 2 : 1, mode = TYPE == T_Q8_0 ? ACT_Q80 : ACT_Q8K;
+  static_assert(NC == 1 || SRC == PAIR_IMG, "rows of f32: one column");
+  constexpr int NCI = TOP2 ? 2 : NC, mode = TYPE == T_Q8_0 ? ACT_Q80 : ACT_Q8K;
   constexpr unsigned tileb = tile_bytes(TYPE);
   const int tid = tid_opaque(), lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), half = wave >> 2;
   const int K = a.K, S = K / 256, Cs = (S + 3) / 4, bx = (int)blockIdx.x;
@@ -337,10 +339,12 @@ __global__ void __launch_bounds__(NT) dec_gemv_pair_kernel(const GemvArgs a) {
   const int p = (lane >> 2) & 3, c = lane & 3, row = u * 4 + (lane >> 4), nrows = a.nrows[0];
   // the rows of activations first
   const float *x1 = TOP2 ? a.x + a.ldx : a.x;
-  const size_t img_bytes = act_bytes(K, 1);
+  const size_t img_bytes = act_bytes(K, NC);
   ActRegs<1> xa = act_issue_all<1>(SRC == PAIR_IMG ? a.x_img : (const void *)a.x, SRC == PAIR_IMG ? (unsigned)img_bytes : (unsigned)K * 4u, nullptr, K, wave), xb;
   if constexpr (TOP2) xb = act_issue_all<1>(x1, (unsigned)K * 4u, nullptr, K, wave);
-  const float res = a.out[min(row, nrows - 1)];
+  float res[NC];
+#pragma unroll
+  for (int k = 0; k < NC; ++k) res[k] = a.out[(size_t)k * a.out_stride + min(row, nrows - 1)];
   const int e = TOP2 ? (int)MRS_SLOAD32(a.expert_sel + half) : 0;
   const float w0 = TOP2 ? a.acc_scale[0] : a.acc_scale ? *a.acc_scale : 1.0f, w1 = TOP2 ? a.acc_scale[1] : 0.f;
   // tiles t0 .. t0 + nt - 1 of the unit: both halves of its rows' tiles, or all of the expert's
@@ -363,13 +367,13 @@ __global__ void __launch_bounds__(NT) dec_gemv_pair_kernel(const GemvArgs a) {
     for (int i = 0; i < 4; ++i) { sb[i] = wave + 8 * (j0 + i); live[i] = j0 + i < NPX && sb[i] < S; v[i] = as_f4(x.xv[0][j0 + i < NPX ? j0 + i : 0]); }
     quantize_multi<4>(v, sb, live, col, mode, smem, K, NCI);
   };
-  constexpr int P0 = R == PAIR_RING ? 1 : 2, P1 = R < P0 + 2 ? R : P0 + 2, P2 = R < P1 + 1 ? R : P1 + 1, P3 = R < 6 ? R : 6, P4 = R;
+  constexpr int P0 = R == PAIR_RING ? 1 : 2, P1 = R < P0 + 2 ? R : P0 + 2, P2 = R < P1 + 1 ? R : P1 + 1, P3 = R < 6 ? R : 6, P4 = R, PI = 2;
   MRS_TL2(a, 0);
   __syncthreads();  // every wave's rows are requested
   requests(0, P0);
   MRS_TL2(a, 1);
   if constexpr (SRC == PAIR_IMG) {
-    requests(P0, R);
+    requests(P0, PI);
     img_finish_all<1>(smem, xa, a.x_img, img_bytes, wave);
   } else {
     quantize(xa, 0, 0);
@@ -385,15 +389,14 @@ __global__ void __launch_bounds__(NT) dec_gemv_pair_kernel(const GemvArgs a) {
   }
   MRS_TL2(a, 2);
   __syncthreads();
-  if constexpr (SRC != PAIR_IMG) requests(TOP2 ? P4 : P2, R);
+  constexpr int BEFORE = TOP2 ? P4 : SRC == PAIR_IMG ? PI : P2;  // tiles requested in front of the barrier
+  if constexpr (TOP2) requests(BEFORE, R);
   MRS_TL2(a, 3);
   const Act act = act_view(smem, K, NCI, mode);
   const int qo = p * act.CQ + c * 64;
-  auto term = [&](int i) -> float {  // T of the lane's superblock in tile t0 + i
-    float T[1];
+  auto term = [&](int i, float(&T)[NC]) {  // T of the lane's superblock in tile t0 + i
     const int ts = min(t0 + i, Cs - 1);
-    TL::template term<1>(ring[i % R], p * Cs + ts, qo + ts * 256, c, act, TOP2 ? half : 0, T);
-    return T[0];
+    TL::template term<NC>(ring[i % R], p * Cs + ts, qo + ts * 256, c, act, TOP2 ? half : 0, T);
   };
   auto live = [&](int i) { return i < nt && p * Cs + t0 + i < S; };
   auto row_sum = [&](float acc) {  // ((c0 + c1) + c2) + c3 in the chunk-3 quad of every row
@@ -402,45 +405,59 @@ __global__ void __launch_bounds__(NT) dec_gemv_pair_kernel(const GemvArgs a) {
     return dppf<0x124>(s) + acc;
   };
   const bool own = has && (lane & 15) == owner_off(Geo{}) && row < nrows;
-  float acc = 0.f;
   if constexpr (TOP2) {
+    float acc = 0.f;
 #pragma unroll
     for (int i = 0; i < 2 * R; ++i) {
-      const float T = term(i);
-      acc = i == 0 ? (live(0) ? T : 0.f) : live(i) ? acc + T : acc;
+      float T[1];
+      term(i, T);
+      acc = i == 0 ? (live(0) ? T[0] : 0.f) : live(i) ? acc + T[0] : acc;
       if (i < R) request(i + R);
       __builtin_amdgcn_sched_barrier(0);
     }
     const float tot = row_sum(acc);
-    if (half == 0) hand_s[wave & 3][lane] = tot;
+    if (half == 0) hand_s[wave & 3][0][lane] = tot;
     __syncthreads();
     if (half == 1 && own) {
-      const float h1 = res * a.resid_scale + hand_s[wave & 3][lane] * w0;
+      const float h1 = res[0] * a.resid_scale + hand_s[wave & 3][0][lane] * w0;
       a.out[row] = h1 * 1.0f + tot * w1;
     }
   } else {
-    float T[R];
+    float T[R][NC], acc[NC];
 #pragma unroll
-    for (int i = 0; i < R; ++i) T[i] = term(i);
+    for (int i = 0; i < R; ++i) {
+      if (BEFORE + i < R) requests(BEFORE + i, BEFORE + i + 1);
+      term(i, T[i]);
+    }
     auto chain = [&](bool first) {
 #pragma unroll
-      for (int i = 0; i < R; ++i) acc = first && i == 0 ? (live(0) ? T[0] : 0.f) : live(i) ? acc + T[i] : acc;
+      for (int i = 0; i < R; ++i)
+#pragma unroll
+        for (int k = 0; k < NC; ++k) acc[k] = first && i == 0 ? (live(0) ? T[0][k] : 0.f) : live(i) ? acc[k] + T[i][k] : acc[k];
     };
-    if (half == 0) { chain(true); hand_s[wave][lane] = acc; }
+    if (half == 0) {
+      chain(true);
+#pragma unroll
+      for (int k = 0; k < NC; ++k) hand_s[wave][k][lane] = acc[k];
+    }
     __syncthreads();
     if (half == 1) {
-      acc = hand_s[wave & 3][lane];
+#pragma unroll
+      for (int k = 0; k < NC; ++k) acc[k] = hand_s[wave & 3][k][lane];
       chain(false);
-      const float tot = row_sum(acc);
-      if (own) a.out[row] = res * a.resid_scale + tot * w0;
+#pragma unroll
+      for (int k = 0; k < NC; ++k) {
+        const float tot = row_sum(acc[k]);
+        if (own) a.out[(size_t)k * a.out_stride + row] = res[k] * a.resid_scale + tot * w0;
+      }
     }
   }
   MRS_TL2(a, 14);
 }
-// tiles per unit that it takes: an image's rows of 3 and 4 (a wave then has two), f32 rows of 7 .. 14 (4 .. 7 in registers; longer rows do not fit the prologue's seven pieces either), two
+// tiles per unit that it takes: an image's rows of 3 and 4 (a wave then has two) and two columns' of 7 .. 14, f32 rows of 7 .. 14 (4 .. 7 in registers; longer rows do not fit the prologue's seven pieces either), two
 // experts' rows of 8 .. 14.  Other counts and launches with more units per workgroup are stream()'s
-__host__ inline bool pair_ring_ok(int src, int Cs) { return src == PAIR_IMG ? Cs == 3 || Cs == 4 : src == PAIR_F32 ? Cs >= 7 && Cs <= 2 * PAIR_RING : Cs > PAIR_RING && Cs <= 2 * PAIR_RING; }
-int pair_launch(int type, int src, int grid, size_t lds, const GemvArgs &a, hipStream_t s);
+__host__ inline bool pair_ring_ok(int src, int ncols, int Cs) { return src == PAIR_IMG ? Cs == 3 || Cs == 4 || (ncols == 2 && Cs >= 7 && Cs <= 2 * PAIR_RING) : src == PAIR_F32 ? Cs >= 7 && Cs <= 2 * PAIR_RING : Cs > PAIR_RING && Cs <= 2 * PAIR_RING; }
+template <int NCOLS> int pair_launch(int type, int src, int grid, size_t lds, const GemvArgs &a, hipStream_t s);  // 1 or 2 columns (ext_dec_gemv.hip)
 
 // launch one GEMV phase with NCOLS activation columns (ext_dec_gemv.hip, one definition per NCOLS)
 template <int NCOLS> int gemv_launch(int epi, int tmask, bool ring2, int grid, size_t lds, const GemvArgs &a, hipStream_t s);

@@ -754,10 +754,10 @@ template <int EPI> struct Launch {
     if (a.upe < 1) a.upe = 1;
     size_t lds = (act_bytes(a.K, NCI) + 15) & ~(size_t)15;
     if (lds > LDS_IMG_MAX) return -2;
-    if constexpr (NCOLS == 1 && (EPI == EPI_RESID || EPI == EPI_RESID2)) {  // units for half of the waves: two waves per unit (dec_gemv_pair_kernel)
+    if constexpr (NCOLS <= 2 && (EPI == EPI_RESID || EPI == EPI_RESID2)) {  // units for half of the waves: two waves per unit (dec_gemv_pair_kernel)
       const int src = EPI == EPI_RESID2 ? PAIR_TOP2 : a.x_img ? PAIR_IMG : PAIR_F32;
-      const bool plain = EPI == EPI_RESID2 ? !a.x_img : !a.expert_sel;
-      if (plain && !a.norm_w && a.ubase[0] + (a.urem[0] > 0) <= NW / 2 && pair_ring_ok(src, g.Cs)) return pair_launch(a.m[0].type, src, grid, lds, a, s);
+      const bool plain = EPI == EPI_RESID2 ? !a.x_img : !a.expert_sel && (NCOLS == 1 || a.x_img);
+      if (plain && !a.norm_w && a.ubase[0] + (a.urem[0] > 0) <= NW / 2 && pair_ring_ok(src, NCOLS, g.Cs)) return pair_launch<NCOLS>(a.m[0].type, src, grid, lds, a, s);
     }
     int tmask = 0;
     for (int i = 0; i < (EPI == EPI_QKV ? 3 : 1); ++i) tmask |= tmask_of(a.m[i].type);

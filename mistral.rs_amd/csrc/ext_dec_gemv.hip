@@ -42,20 +42,21 @@ template <> int gemv_launch<MRS_DEC_NC>(int epi, int tmask, bool ring2, int grid
   default: return -1;
   }
 }
-#if MRS_DEC_NC == 1
-template <int TYPE, int R, int SRC> static void pair_go(int grid, size_t lds, const GemvArgs &a, hipStream_t s) {
-  hipLaunchKernelGGL((dec_gemv_pair_kernel<TYPE, R, SRC>), dim3(grid), dim3(NT), lds, s, a);
+#if MRS_DEC_NC <= 2
+template <int TYPE, int R, int SRC> static int pair_go(int grid, size_t lds, const GemvArgs &a, hipStream_t s) {
+  hipLaunchKernelGGL((dec_gemv_pair_kernel<TYPE, R, SRC, MRS_DEC_NC>), dim3(grid), dim3(NT), lds, s, a);
+  return 0;
 }
 template <int TYPE> static int pair_typed(int src, int grid, size_t lds, const GemvArgs &a, hipStream_t s) {
   const int Cs = geo_for(a.K).Cs;
-  if (src == PAIR_IMG) pair_go<TYPE, 2, PAIR_IMG>(grid, lds, a, s);
-  else if (src == PAIR_TOP2) pair_go<TYPE, PAIR_RING, PAIR_TOP2>(grid, lds, a, s);
-  else if (Cs <= 8) pair_go<TYPE, 4, PAIR_F32>(grid, lds, a, s);
-  else if (Cs <= 12) pair_go<TYPE, 6, PAIR_F32>(grid, lds, a, s);
-  else pair_go<TYPE, PAIR_RING, PAIR_F32>(grid, lds, a, s);
-  return 0;
+  constexpr int LONG = MRS_DEC_NC == 1 ? PAIR_F32 : PAIR_IMG;
+  if (src == PAIR_IMG && Cs <= 4) return pair_go<TYPE, 2, PAIR_IMG>(grid, lds, a, s);
+#if MRS_DEC_NC == 1
+  if (src == PAIR_TOP2) return pair_go<TYPE, PAIR_RING, PAIR_TOP2>(grid, lds, a, s);
+#endif
+  return Cs <= 8 ? pair_go<TYPE, 4, LONG>(grid, lds, a, s) : Cs <= 12 ? pair_go<TYPE, 6, LONG>(grid, lds, a, s) : pair_go<TYPE, PAIR_RING, LONG>(grid, lds, a, s);
 }
-int pair_launch(int type, int src, int grid, size_t lds, const GemvArgs &a, hipStream_t s) {
+template <> int pair_launch<MRS_DEC_NC>(int type, int src, int grid, size_t lds, const GemvArgs &a, hipStream_t s) {
   switch (type) {
   case T_Q4_K: return pair_typed<T_Q4_K>(src, grid, lds, a, s);
   case T_Q5_K: return pair_typed<T_Q5_K>(src, grid, lds, a, s);

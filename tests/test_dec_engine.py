@@ -86,12 +86,12 @@ def test_proj_gpu(oracle, dev, tname, n, k, b, mode):
 # the other kernel), rows that are not a multiple of four, a short last chunk, workgroups of one and of two units
 PAIRS = [("Q4_K", 6, 6656, None), ("Q4_K", 9, 14336, None), ("Q4_K", 4, 14080, None), ("Q4_K", 3, 9216, None), ("Q4_K", 5, 6144, None), ("Q5_K", 7, 11008, None), ("Q6_K", 5, 13824, None), ("Q6_K", 4, 8192, None),
          ("Q6_K", 6, 10240, None), ("Q8_0", 6, 9728, None), ("Q8_0", 3, 14336, None), ("Q4_K", 13, 4096, "img"), ("Q8_0", 10, 3072, "img"), ("Q6_K", 7, 2816, "img"), ("Q5_K", 5, 3840, "img"),
-         ("Q4_K", 1030, 2304, "img")]
+         ("Q4_K", 1030, 2304, "img"), ("Q4_K", 6, 14336, "img2"), ("Q6_K", 5, 11008, "img2"), ("Q8_0", 7, 7168, "img2"), ("Q5_K", 3, 9216, "img2"), ("Q6_K", 13, 4096, "img2")]
 
 
 def check_pairs(O, be, tname, n, k, img):
     if img:
-        check_image_proj(O, be, tname, n, k, 1, False)
+        check_image_proj(O, be, tname, n, k, 2 if img == "img2" else 1, False)
     else:
         check_proj(O, be, tname, n, k, 1, 1, seed=n + k)
 
@@ -102,7 +102,7 @@ def test_two_waves_per_unit_host_emulation(oracle, tname, n, k, img):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("tname,n,k,img", PAIRS + [("Q5_K", 4096, 11008, None), ("Q8_0", 4095, 14336, None), ("Q6_K", 3072, 8192, None), ("Q4_K", 2050, 4096, "img")])
+@pytest.mark.parametrize("tname,n,k,img", PAIRS + [("Q5_K", 4096, 11008, None), ("Q8_0", 4095, 14336, None), ("Q6_K", 3072, 8192, None), ("Q4_K", 2050, 4096, "img"), ("Q6_K", 4095, 14336, "img2"), ("Q8_0", 2050, 4096, "img2")])
 def test_two_waves_per_unit_gpu(oracle, dev, tname, n, k, img):
     check_pairs(oracle, GpuBackend(dev), tname, n, k, img)
 
