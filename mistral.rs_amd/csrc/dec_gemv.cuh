@@ -318,7 +318,7 @@ __global__ void __launch_bounds__(NT) dec_gemv_kernel(const GemvArgs a) {
 // CU's share of the memory can take is blocked in the issue, and everyone waits for it at the barrier: the tiles are requested a few at a time, between the steps of the quantization, the
 // last of them behind the barrier, one in front of each product.  One tile in front of it, two and one between (rows of 13 and 14 tiles per unit), us: Q4_K 4096 x 14336 10.4 (in front all seven 12.2, two 10.7; behind
 // the barrier all but two 11.3); shorter rows two, two and one: Q6_K 3072 x 8192 6.9 (with one in front 7.3).
-// us, stream() / this: Q4_K 4096 x 14336 11.6 / 10.2, 4096 x 11008 9.3 / 7.8, 4096 x 7168 7.1 / 6.3, Q5_K 4096 x 14336 12.2 / 10.8, Q6_K 13.1 / 11.3, 3072 x 8192 7.9 / 6.9, Q8_0 14.2 / 12.3; Q4_K 4096 x 4096 from
+// us, stream() / this: Q4_K 4096 x 14336 11.6 / 10.2, 4096 x 11008 9.3 / 7.8, 4096 x 7168 7.1 / 6.3, Q5_K 4096 x 14336 12.2 / 10.8, Q6_K 13.1 / 11.3, 3072 x 8192 7.9 / 6.9, Q8_0 14.2 / 12.3, rows of 4096 and 3072 (two tiles of a wave): Q8_0 4096 x 4096 5.7 / 5.1, Q4_K 3072 x 3072 4.8 / 4.2; Q4_K 4096 x 4096 from
 // an image 4.8 / 4.1; two columns from an image Q4_K 4096 x 4096 5.95 / 4.55, 4096 x 14336 11.5 / 10.8, 4096 x 11008 9.8 / 7.95, Q6_K 4096 x 14336 13.0 / 11.2, 3072 x 8192 8.8 / 6.9, Q8_0 4096 x 14336 14.1 / 12.5 (all of the
 // image's tiles in front of the barrier 12.1, 9.5, 14.4, 8.0, 14.6); two experts of 4096 x 14336 Q4_K 22.4 / 17.7, Q6_K 23.8 / 20.9, Q8_0 25.8 / 22.1, of 2048 x 8192 Q4_K 11.1 / 9.6.
 constexpr int PAIR_RING = 7;  // tiles of a wave (TOP2: twice)
@@ -454,9 +454,9 @@ __global__ void __launch_bounds__(NT) dec_gemv_pair_kernel(const GemvArgs a) {
   }
   MRS_TL2(a, 14);
 }
-// tiles per unit that it takes: an image's rows of 3 and 4 (a wave then has two) and two columns' of 7 .. 14, f32 rows of 7 .. 14 (4 .. 7 in registers; longer rows do not fit the prologue's seven pieces either), two
+// tiles per unit that it takes: an image's rows of 3 and 4 (a wave then has two) and two columns' of 7 .. 14, f32 rows of 3, 4 and 7 .. 14 (2, 4 .. 7 in registers; longer rows do not fit the prologue's seven pieces either), two
 // experts' rows of 8 .. 14.  Other counts and launches with more units per workgroup are stream()'s
-__host__ inline bool pair_ring_ok(int src, int ncols, int Cs) { return src == PAIR_IMG ? Cs == 3 || Cs == 4 || (ncols == 2 && Cs >= 7 && Cs <= 2 * PAIR_RING) : src == PAIR_F32 ? Cs >= 7 && Cs <= 2 * PAIR_RING : Cs > PAIR_RING && Cs <= 2 * PAIR_RING; }
+__host__ inline bool pair_ring_ok(int src, int ncols, int Cs) { return src == PAIR_IMG ? Cs == 3 || Cs == 4 || (ncols == 2 && Cs >= 7 && Cs <= 2 * PAIR_RING) : src == PAIR_F32 ? Cs == 3 || Cs == 4 || (Cs >= 7 && Cs <= 2 * PAIR_RING) : Cs > PAIR_RING && Cs <= 2 * PAIR_RING; }
 template <int NCOLS> int pair_launch(int type, int src, int grid, size_t lds, const GemvArgs &a, hipStream_t s);  // 1 or 2 columns (ext_dec_gemv.hip)
 
 // launch one GEMV phase with NCOLS activation columns (ext_dec_gemv.hip, one definition per NCOLS)

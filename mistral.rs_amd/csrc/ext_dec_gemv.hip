@@ -54,6 +54,9 @@ template <int TYPE> static int pair_typed(int src, int grid, size_t lds, const G
 #if MRS_DEC_NC == 1
   if (src == PAIR_TOP2) return pair_go<TYPE, PAIR_RING, PAIR_TOP2>(grid, lds, a, s);
 #endif
+#if MRS_DEC_NC == 1
+  if (Cs <= 4) return pair_go<TYPE, 2, PAIR_F32>(grid, lds, a, s);
+#endif
   return Cs <= 8 ? pair_go<TYPE, 4, LONG>(grid, lds, a, s) : Cs <= 12 ? pair_go<TYPE, 6, LONG>(grid, lds, a, s) : pair_go<TYPE, PAIR_RING, LONG>(grid, lds, a, s);
 }
 template <> int pair_launch<MRS_DEC_NC>(int type, int src, int grid, size_t lds, const GemvArgs &a, hipStream_t s) {

@@ -82,11 +82,11 @@ def test_proj_gpu(oracle, dev, tname, n, k, b, mode):
     check_proj(oracle, GpuBackend(dev), tname, n, k, b, mode, seed=n + k)
 
 
-# Launches with units for at most half of a workgroup's waves: two waves per unit, each with half of its tiles (7 .. 14 tiles of an f32 row, three and four of an image; the other counts take
+# Launches with units for at most half of a workgroup's waves: two waves per unit, each with half of its tiles (3, 4 and 7 .. 14 tiles of an f32 row, three and four of an image; the other counts take
 # the other kernel), rows that are not a multiple of four, a short last chunk, workgroups of one and of two units
 PAIRS = [("Q4_K", 6, 6656, None), ("Q4_K", 9, 14336, None), ("Q4_K", 4, 14080, None), ("Q4_K", 3, 9216, None), ("Q4_K", 5, 6144, None), ("Q5_K", 7, 11008, None), ("Q6_K", 5, 13824, None), ("Q6_K", 4, 8192, None),
          ("Q6_K", 6, 10240, None), ("Q8_0", 6, 9728, None), ("Q8_0", 3, 14336, None), ("Q4_K", 13, 4096, "img"), ("Q8_0", 10, 3072, "img"), ("Q6_K", 7, 2816, "img"), ("Q5_K", 5, 3840, "img"),
-         ("Q4_K", 1030, 2304, "img"), ("Q4_K", 6, 14336, "img2"), ("Q6_K", 5, 11008, "img2"), ("Q8_0", 7, 7168, "img2"), ("Q5_K", 3, 9216, "img2"), ("Q6_K", 13, 4096, "img2")]
+         ("Q4_K", 1030, 2304, "img"), ("Q4_K", 6, 14336, "img2"), ("Q6_K", 5, 11008, "img2"), ("Q8_0", 7, 7168, "img2"), ("Q5_K", 3, 9216, "img2"), ("Q6_K", 13, 4096, "img2"), ("Q8_0", 13, 4096, None), ("Q4_K", 6, 3072, None), ("Q5_K", 5, 2816, None)]
 
 
 def check_pairs(O, be, tname, n, k, img):
