@@ -772,8 +772,6 @@ __device__ __forceinline__ void stream(const Job &jb, int K, int ncols_img, int 
   stage(1, wave);  // squares, wave sums -- while the first tile of every wave is in flight
   if (sbar) __syncthreads();  // S
   MRS_TL2(jb, 1);
-  // (publishing the image BEFORE the rest of the ring is requested -- tried for the short launches, round 5 -- made qkv 0.9 us slower in the graph: the requests that
-  // would have overlapped the quantization arithmetic then queue behind it)
   // two tiles in front of the quantization, the others behind it: a wave that requests all of its ring is blocked in the issue while the others wait for its part of the image.  q / k / v of
   // 6144 x 4096, us, four in front / two: Q8_0 9.4 / 8.8, Q4_K 7.9 / 7.9, two columns 12.5 / 11.6, gate / up of two columns 19.5 / 18.9 (one in front 8.6, 8.25, 12.0, 19.6)
   constexpr int RA = NS < 2 ? NS : 2;

@@ -459,7 +459,7 @@ class Llama {
     static const int mm_min_b = [] { const char *e = getenv("MRS_DEC_MM"); if (e && atoi(e) == 0) return 1 << 30; const char *m = getenv("MRS_DEC_MM_MIN_B"); return m ? atoi(m) : 3; }();  // 8B Q4_K_M at 1500 tokens, us per step of two sequences, here / vector ALU: 2297 / 2356; they stay there (the same bits, 2.5 %)
     const bool mmb = imgb && b >= mm_min_b;
     // Two columns of a hidden-sized row: the GEMVs' own prologue hides most of its work behind the weight requests, an image launch in front of them cannot (8B Q4_K_M, image +
-    // GEMV / GEMV alone: q / k / v 4.5 + 10.9 / 15.3 us, gate / up 4.5 + 17.4 / 21.1, lm_head 4.5 + 69.2 / 73.0, and a launch less each); rows of the FFN width keep the image
+    // GEMV / GEMV alone: q / k / v 4.5 + 10.9 / 15.3 us, gate / up 4.5 + 17.4 / 21.1, lm_head 4.5 + 69.2 / 73.0, and a launch less each; alone 10.5 and 18.1 since both rows are held in registers); rows of the FFN width keep the image
     // (o_proj and down_proj of the two columns together 9.8 us, 14.3 without), and longer hidden rows too (two layers of 8192, whole step at 1500 tokens, image / prologue: 335 / 341).
     const bool imgn = imgb && (b >= 3 || mmb || d > 4096);
     auto qi_of = [](const std::unique_ptr<GgufMatMul> &l) -> const void * { return l && l->get_qtensor() ? l->get_qtensor()->qi : nullptr; };
